@@ -460,7 +460,7 @@ def bench_cutce(ct, torch, steps, warmup, logits_cache=True):
     chunks = -(-(-(-config.vocab // 256)) // 4)
     per_kernel_bytes = {
         "cutce_merge_kernel": chunks * active * 12 + 8 * active + 8 * config.rows,
-        "cutce_pack_rows_kernel": 2 * active * config.hidden * 2,
+        "cutce_rows_kernel": 2 * active * config.hidden * 2,
     }
     if logits_cache:
         per_kernel_bytes["cutce_dlogits_cached_kernel"] = (-(-active // 256) * 256) * config.vocab * 6

@@ -143,6 +143,7 @@ SYMBOLS = {
     "ct_attn_bwd": (c_int32, [c_void_p, POINTER(AttnBwdArgs)]),
     "ct_attn_delta": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32]),
     "ct_cutce_fwd_workspace_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_fwd_workspace_min_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_bwd_workspace_min_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_bwd_workspace_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_logits_cache_bytes": (c_size_t, [POINTER(CutceShape)]),

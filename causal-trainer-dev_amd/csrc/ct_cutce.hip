@@ -29,7 +29,7 @@
 namespace ct {
 
 constexpr int kBK = kGemmBK;
-constexpr int kTilesPerChunk = 4;  // vocab tiles per stats work unit
+constexpr int kComputeUnits = 256;    // of an MI355X; sizes of work units are chosen by it
 #ifndef CT_CUTCE_SWEEP
 #define CT_CUTCE_SWEEP 1
 #endif
@@ -131,61 +131,143 @@ struct XcdUnits {
   }
 };
 
+// The head as the GEMM kernels read it: column v of row n at base[n * ld + v - col0]. Either the
+// caller's tensor (ld = V) or, where its rows are not 16-byte aligned (V % 8 != 0), an aligned copy
+// of the columns col0 .. in the workspace ("panel", cutce_panel_kernel), padded with zero columns to
+// whole tiles.
+struct HeadView {
+  const bf16* base;
+  long ld;
+  int col0;
+  bool aligned, padded;
+};
+
 struct CutceParams {
   const bf16* hidden;
-  const bf16* head;
+  HeadView head;
   const int* targets;
   const float* weights;
   int N, d, V, n_pad;
   int* idx;
   CutceHeader* header;
-  bool hidden_aligned, head_aligned;
+  bool hidden_aligned;
+
+  // columns of the head that a tile at v0 may read, relative to the view
+  CT_DEVICE int head_cols(int v0) const { return head.padded ? v0 - head.col0 + kGemmTile : V - head.col0; }
 };
 
 // ---------------------------------------------------------------------------
-// index: stable compaction of active rows
+// index: stable compaction of active rows (and, for the backward, their constants)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void cutce_index_kernel(const float* weights, int N, int n_pad,
-                                                           int compact, int* idx,
-                                                           CutceHeader* header) {
-  __shared__ int wave_total[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
-  if (!compact) {
-    for (int i = tid; i < n_pad; i += blockDim.x) idx[i] = i < N ? i : 0;
-    if (tid == 0) {
-      header->n_act = N;
-      header->counter = 0;
-    }
-    reset_unit_counters(header);
-    reset_dlogits_counters(header);
-    return;
+// Per-slot constants of the backward: (w dy, lse log2 e, target), zeros / -1 past the active rows.
+struct CutceRowParams {
+  float* fac;
+  float* lse2;
+  int* tgt;
+};
+
+// Workgroup b places the rows 1024 b .. 1024 b + 1023; it counts the active rows in front of them
+// by itself (N floats, from L2 for all but the first reader), so no workgroup waits for another: one
+// pass of latency instead of one per 1024 rows (27 -> 5 us at N = 16384).
+template <bool BACKWARD>
+__global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, int compact, const float* lse,
+                                                           const float* dy, CutceRowParams rp) {
+  __shared__ int wave_total[16], wave_first[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int begin = blockIdx.x * 1024, i = begin + tid;
+  const bool last = blockIdx.x == gridDim.x - 1;
+  if (last) {
+    reset_unit_counters(p.header);
+    reset_dlogits_counters(p.header);
   }
-  int carry = 0;
-  for (int base = 0; base < N; base += blockDim.x) {
-    const int i = base + tid;
-    const bool active = i < N && weights[i] != 0.f;
+  const float w = i < p.N ? p.weights[i] : 0.f;
+  const bool active = w != 0.f;
+  int slot = i, total = p.N, filler = 0;
+  bool placed = i < p.N;
+  if (compact) {
+    int count = 0, first = p.N;  // active rows of this wavefront's share in front of `begin`
+    for (int base = 0; base < begin; base += 1024) {
+      const unsigned long long ballot = __ballot(p.weights[base + tid] != 0.f);
+      if (ballot) first = min(first, base + wave * 64 + __ffsll(ballot) - 1);
+      count += __popcll(ballot);
+    }
     const unsigned long long ballot = __ballot(active);
-    const int before = __popcll(ballot & ((1ull << lane) - 1ull));
+    if (ballot) first = min(first, begin + wave * 64 + __ffsll(ballot) - 1);
+    if (lane == 0) {
+      wave_total[wave] = count;
+      wave_first[wave] = first;
+    }
+    __syncthreads();
+    int before = 0;
+    filler = p.N;
+    for (int k = 0; k < 16; ++k) {
+      before += wave_total[k];
+      filler = min(filler, wave_first[k]);
+    }
+    filler = filler < p.N ? filler : 0;  // keeps gathers past the end on a live row
+    __syncthreads();
     if (lane == 0) wave_total[wave] = __popcll(ballot);
     __syncthreads();
-    int offset = 0, all = 0;
-    for (int k = 0; k < nwaves; ++k) {
-      if (k < wave) offset += wave_total[k];
-      all += wave_total[k];
+    total = before;
+    for (int k = 0; k < 16; ++k) {
+      if (k < wave) before += wave_total[k];
+      total += wave_total[k];
     }
-    if (active) idx[carry + offset + before] = i;
-    carry += all;
-    __syncthreads();
+    slot = before + __popcll(ballot & ((1ull << lane) - 1ull));
+    placed = active;
   }
-  __syncthreads();
-  const int filler = carry > 0 ? idx[0] : 0;  // keeps gathers past the end on a live row
-  for (int i = carry + tid; i < n_pad; i += blockDim.x) idx[i] = filler;
+  if (placed) {
+    p.idx[slot] = i;
+    if constexpr (BACKWARD) {
+      rp.fac[slot] = active ? w * dy[0] : 0.f;
+      rp.lse2[slot] = active ? lse[i] * kLog2e : __builtin_inff();
+      rp.tgt[slot] = active ? p.targets[i] : -1;
+    }
+  }
+  if (!last) return;
+  for (int k = total + tid; k < p.n_pad; k += 1024) {
+    p.idx[k] = filler;
+    if constexpr (BACKWARD) {
+      rp.fac[k] = 0.f;
+      rp.lse2[k] = __builtin_inff();
+      rp.tgt[k] = -1;
+    }
+  }
   if (tid == 0) {
-    header->n_act = carry;
-    header->counter = 0;
+    p.header->n_act = total;
+    p.header->counter = 0;
   }
-  reset_unit_counters(header);
-  reset_dlogits_counters(header);
+}
+
+// ---------------------------------------------------------------------------
+// panel: an aligned, zero-padded copy of `cols` (a multiple of 256) columns of the head
+// ---------------------------------------------------------------------------
+// With V % 8 != 0 the rows of the head start at addresses that are multiples of 2 bytes only, and
+// the asynchronous copies of the GEMM loop move aligned 16-byte chunks. One pass over the head
+// (2 bytes read and written per element) makes them usable: the guarded loop that loads such
+// rows element by element runs at 20-90 TFLOP/s against the pipelined one's 600-1300.
+constexpr int kPanelRows = 4;
+__global__ __launch_bounds__(256) void cutce_panel_kernel(const bf16* head, int V, int d, int col0, int cols,
+                                                          bf16* panel, CutceHeader* header) {
+  // (the statistics kernel that follows starts from fresh work counters)
+  if (header && blockIdx.x == 0 && blockIdx.y == 0) reset_unit_counters(header);
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (c >= cols) return;
+  const int row0 = blockIdx.y * kPanelRows;
+  const int left = V - (col0 + c);
+  const bf16* src = head + (size_t)row0 * V + col0 + c;
+  bf16* dst = panel + (size_t)row0 * cols + c;
+  bf16x8 v[kPanelRows];
+  if (left >= 8) {
+#pragma unroll
+    for (int r = 0; r < kPanelRows; ++r) __builtin_memcpy(&v[r], src + (size_t)r * V, 16);
+  } else {
+    for (int r = 0; r < kPanelRows; ++r)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[r][e] = e < left ? src[(size_t)r * V + e] : (bf16)0.f;
+  }
+#pragma unroll
+  for (int r = 0; r < kPanelRows; ++r) store_global16(dst + (size_t)r * cols, as_u32x4(v[r]));
 }
 
 // ---------------------------------------------------------------------------
@@ -199,8 +281,8 @@ CT_DEVICE void merge_stats(float& m, float& s, float m_o, float s_o) {
 }
 
 template <bool CACHE>
-__global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* part, int chunks,
-                                                          float* cache) {
+__global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
+                                                          int tiles_per_chunk, float* cache) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
@@ -215,6 +297,7 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
   units.init(p.header->xcd_counter[0], chunks, active_blocks, kSweepUnits);
   int chunk, rb;
   while (units.next(chunk, rb, &unit_s)) {
+    chunk += chunk0;
     const int n0 = rb * kGemmTile;
     const int my_slot = n0 + tid;
     const int active = my_slot < n_act && p.weights[p.idx[my_slot]] != 0.f;
@@ -238,11 +321,11 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
     KcLoader B;
     B.init(p.hidden, p.d, p.idx, n0, n_act, p.d, p.hidden_aligned, true, true);
 
-    const int vt_end = min((chunk + 1) * kTilesPerChunk, vocab_tiles);
-    for (int vt = chunk * kTilesPerChunk; vt < vt_end; ++vt) {
+    const int vt_end = min((chunk + 1) * tiles_per_chunk, vocab_tiles);
+    for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = vt * kGemmTile;
       McLoader A;
-      A.init(p.head, p.V, nullptr, v0, p.V, p.d, p.head_aligned);
+      A.init(p.head.base, p.head.ld, nullptr, v0 - p.head.col0, p.head_cols(v0), p.d, p.head.aligned, true);
       GemmAcc acc;
       acc.clear();
       gemm_tile(A, B, 0, p.d, smem, acc);
@@ -419,60 +502,27 @@ __global__ __launch_bounds__(64) void cutce_finalize_kernel(const double* block_
 // ---------------------------------------------------------------------------
 // backward
 // ---------------------------------------------------------------------------
-// dHidden rows of ignored tokens are exactly zero.
-__global__ __launch_bounds__(256) void cutce_zero_rows_kernel(const float* weights, int N, int d,
-                                                              bf16* dhidden) {
-  const int row = blockIdx.x;
-  if (row >= N || weights[row] != 0.f) return;
-  u32x4* dst = reinterpret_cast<u32x4*>(dhidden + (size_t)row * d);
-  for (int c = threadIdx.x; c < d / 8; c += 256) dst[c] = u32x4{0u, 0u, 0u, 0u};
-}
-
-// packed[slot] = hidden[idx[slot]] for the slots of every started 256-slot block. The head
-// gradient contracts over slots; with the rows packed its operand tiles are plain strided
-// copies instead of a gather through idx at every step. (idx repeats the first active row
-// past n_act, so the padding rows hold finite values; their G^T entries are zero.)
-__global__ __launch_bounds__(256) void cutce_pack_rows_kernel(CutceParams p, bf16* packed) {
-  const int slot = blockIdx.x;
+// Row work in front of the gradients, one wavefront per row: dHidden rows of ignored tokens are
+// exactly zero, and (packed != nullptr) packed[slot] = hidden[idx[slot]] for the slots of every started
+// 256-slot block. The head gradient contracts over slots; with the rows packed its operand tiles
+// are plain strided copies instead of a gather through idx at every step. (idx repeats the first
+// active row past n_act, so the padding rows hold finite values; their G^T entries are zero.)
+__global__ __launch_bounds__(256) void cutce_rows_kernel(CutceParams p, bf16* packed, bf16* dhidden) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row < p.N && p.weights[row] == 0.f) {
+    u32x4* dst = reinterpret_cast<u32x4*>(dhidden + (size_t)row * p.d);
+    for (int c = lane; c < p.d / 8; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
+  }
   const int n_act = p.header->n_act;
-  if (slot >= (n_act + kGemmTile - 1) / kGemmTile * kGemmTile) return;
-  const bf16* src = p.hidden + (size_t)p.idx[slot] * p.d;
-  bf16* dst = packed + (size_t)slot * p.d;
+  if (!packed || row >= (n_act + kGemmTile - 1) / kGemmTile * kGemmTile) return;
+  const bf16* src = p.hidden + (size_t)p.idx[row] * p.d;
+  bf16* dst = packed + (size_t)row * p.d;
   if (p.hidden_aligned) {
-    for (int c = threadIdx.x; c < p.d / 8; c += 256)
+    for (int c = lane; c < p.d / 8; c += 64)
       reinterpret_cast<u32x4*>(dst)[c] = reinterpret_cast<const u32x4*>(src)[c];
   } else {
-    for (int c = threadIdx.x; c < p.d; c += 256) dst[c] = src[c];
+    for (int c = lane; c < p.d; c += 64) dst[c] = src[c];
   }
-}
-
-// Per-slot constants of the backward: (w dy, lse log2 e, target), zeros / -1 past the active rows.
-struct CutceRowParams {
-  float* fac;
-  float* lse2;
-  int* tgt;
-};
-
-__global__ __launch_bounds__(256) void cutce_rowparams_kernel(CutceParams p, const float* lse,
-                                                              const float* dy, CutceRowParams rp) {
-  const int slot = blockIdx.x * 256 + threadIdx.x;
-  if (slot >= p.n_pad) return;
-  // A slot without weight gets factor 0 and lse = +inf: exp2(x - inf) is exactly 0 for every finite
-  // logit, so the gradient formula gives 0 for it without a per-element test.
-  float f = 0.f, l2 = __builtin_inff();
-  int t = -1;
-  if (slot < p.header->n_act) {
-    const int row = p.idx[slot];
-    const float wr = p.weights[row];
-    if (wr != 0.f) {
-      f = wr * dy[0];
-      l2 = lse[row] * kLog2e;
-      t = p.targets[row];
-    }
-  }
-  rp.fac[slot] = f;
-  rp.lse2[slot] = l2;
-  rp.tgt[slot] = t;
 }
 
 CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
@@ -481,9 +531,10 @@ CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
 
 // G^T[v - slab0][slot], logits recomputed (transposed tile as in the statistics kernel: rows =
 // vocabulary, lanes = row slots). Persistent like the statistics kernel and with its unit order:
-// a unit is kTilesPerChunk vocabulary tiles of the slab times one block of 256 active rows.
+// a unit is tiles_per_chunk vocabulary tiles of the slab times one block of 256 active rows.
 __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
-                                                            int slab0, int slab_tiles, bf16* G) {
+                                                            int slab0, int slab_tiles, int tiles_per_chunk,
+                                                            bf16* G) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
@@ -493,7 +544,7 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
   // the two GEMM kernels that follow start from fresh work counters
   if (blockIdx.x == 0) reset_unit_counters(p.header);
   const int active_blocks = (n_act + kGemmTile - 1) / kGemmTile;  // G^T columns past them are never read
-  const int chunks = (slab_tiles + kTilesPerChunk - 1) / kTilesPerChunk;
+  const int chunks = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk;
   XcdUnits units;
   units.init(p.header->xcd_counter[2], chunks, active_blocks, kSweepUnits);
   int chunk, rb;
@@ -507,11 +558,11 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
     const i32x4 tgt = *reinterpret_cast<const i32x4*>(rp.tgt + slot4);
     KcLoader B;
     B.init(p.hidden, p.d, p.idx, n0, n_act, p.d, p.hidden_aligned, true, true);
-    const int vt_end = min((chunk + 1) * kTilesPerChunk, slab_tiles);
-    for (int vt = chunk * kTilesPerChunk; vt < vt_end; ++vt) {
+    const int vt_end = min((chunk + 1) * tiles_per_chunk, slab_tiles);
+    for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = slab0 + vt * kGemmTile;
       McLoader A;
-      A.init(p.head, p.V, nullptr, v0, p.V, p.d, p.head_aligned);
+      A.init(p.head.base, p.head.ld, nullptr, v0 - p.head.col0, p.head_cols(v0), p.d, p.head.aligned, true);
       GemmAcc acc;
       acc.clear();
       gemm_tile(A, B, 0, p.d, smem, acc);
@@ -552,17 +603,20 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
 // owns 8 slots and walks kDlogitsRows vocabulary rows with them, so the per-slot constants
 // (factor, lse, target: 96 bytes per thread) are loaded once per kDlogitsRows * 32 bytes of
 // logits and all of a thread's logits loads are in flight together.
-// grid = (slab rows / kDlogitsRows, ceil(n_pad / 2048)).
+// One thread per (8 vocabulary rows, 8 slots) pair, the slots fastest: at least 32 consecutive lanes
+// (n_pad >= 256) read along a row, and no lane idles however few rows there are.
 constexpr int kDlogitsRows = 8;
 __global__ __launch_bounds__(256) void cutce_dlogits_cached_kernel(CutceParams p, CutceRowParams rp,
                                                                    const float* cache, int slab0,
-                                                                   bf16* G) {
-  const int vrel0 = blockIdx.x * kDlogitsRows;
-  const int slot0 = (blockIdx.y * 256 + threadIdx.x) * 8;
+                                                                   int slab_rows, bf16* G) {
+  const int groups = p.n_pad / 8;  // slot groups per vocabulary row
+  const long index = (long)blockIdx.x * 256 + threadIdx.x;
+  const int vrel0 = (int)(index / groups) * kDlogitsRows;
+  const int slot0 = (int)(index % groups) * 8;
   // the two GEMM kernels that follow start from fresh work counters
-  if (blockIdx.x == 0 && blockIdx.y == 0) reset_unit_counters(p.header);
+  if (blockIdx.x == 0) reset_unit_counters(p.header);
   const int n_act = p.header->n_act;
-  if (slot0 >= (n_act + kGemmTile - 1) / kGemmTile * kGemmTile) return;
+  if (vrel0 >= slab_rows || slot0 >= (n_act + kGemmTile - 1) / kGemmTile * kGemmTile) return;
   const f32x4 f0 = *reinterpret_cast<const f32x4*>(rp.fac + slot0);
   const f32x4 f1 = *reinterpret_cast<const f32x4*>(rp.fac + slot0 + 4);
   const f32x4 l0 = *reinterpret_cast<const f32x4*>(rp.lse2 + slot0);
@@ -590,10 +644,56 @@ __global__ __launch_bounds__(256) void cutce_dlogits_cached_kernel(CutceParams p
   }
 }
 
+// How the two gradient GEMMs of a slab are cut along their contraction. With few rows (or a small
+// vocabulary) there are few 256 x 256 output tiles and long contractions: 16 tiles of 32003 terms at
+// N = 999, d = 1024, half a millisecond on 16 of 256 compute units. A cut tile leaves f32 partial sums
+// [part][rows][columns] that cutce_reduce_kernel adds in part order (deterministic). The number of
+// parts is chosen on the device, where the number of active rows is known; the host only
+// provides room for them.
+struct CutceSplits {
+  float* hidden_sums;    // [parts][active row blocks * 256][d]
+  float* head_sums;      // [parts][d][slab_width]
+  size_t hidden_room;    // floats in hidden_sums
+  int head_most;         // parts that head_sums has room for
+  int all_tiles;         // of the whole vocabulary
+  bool with_head;
+};
+
+// Lengths in units of 128 terms of one tile (about 2 us): a compute unit's fair share of all of the
+// work is total / 256, and tiles much longer than that are cut down to it. Partial sums cost 512 KB of
+// traffic per part and tile (about 0.1 us of the device's bandwidth), so with little work the parts
+// stay longer: at length t the last tile ends after 2 t us and the sums of total / t parts take
+// 0.1 total / t us, least at t = sqrt(0.05 total).
+__host__ __device__ inline float part_length(int row_blocks, int d, int tiles, bool with_head) {
+  const float col_blocks = (float)((d + kGemmTile - 1) / kGemmTile);
+  const float total = (with_head ? 4.f : 2.f) * (float)row_blocks * col_blocks * (float)tiles;
+  const float share = total / kComputeUnits, least = __builtin_sqrtf(0.05f * total);
+  return share > least ? share : least;
+}
+__host__ __device__ inline int whole_parts(float parts) { return parts < 1.5f ? 1 : parts > 64.f ? 64 : (int)(parts + 0.5f); }
+
+CT_DEVICE int hidden_parts(const CutceSplits& sp, int n_act, int d, int slab_tiles) {
+  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+  if (row_blocks == 0) return 1;
+  const int parts = whole_parts(2.f * slab_tiles / part_length(row_blocks, d, slab_tiles, sp.with_head));
+  const size_t fit = sp.hidden_room / ((size_t)row_blocks * kGemmTile * d);
+  return uniform(fit < (size_t)parts ? (fit > 1 ? (int)fit : 1) : parts);
+}
+// A slab's dHead is cut as the whole vocabulary's is, whatever the slab: dHead is bit for bit the same
+// for every workspace. (dHidden adds over slabs anyway.)
+CT_DEVICE int head_parts(const CutceSplits& sp, int n_act, int d) {
+  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+  if (row_blocks == 0) return 1;
+  return uniform(min(whole_parts(2.f * row_blocks / part_length(row_blocks, d, sp.all_tiles, true)), sp.head_most));
+}
+
+// First of the 128-term groups of part `split`.
+CT_DEVICE int split_begin(int groups, int split, int splits) { return (int)((long)groups * split / splits); }
+
 // dHidden[idx[slot], n] (+)= sum_v G^T[v, slot] head[n, slab0 + v]: the workgroup's share of the
 // units, pulled from counter set 0.
 CT_DEVICE void dhidden_units(const CutceParams& p, const bf16* G, int slab0, int slab_width, int mode,
-                             float* dh_acc, bf16* dhidden, const lds_addr smem) {
+                             float* dh_acc, bf16* dhidden, const CutceSplits& sp, const lds_addr smem) {
   // mode: 0 = single slab (store bf16), 1 = first slab (store f32), 2 = middle
   // slab (add f32), 3 = last slab (add, store bf16)
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
@@ -603,21 +703,39 @@ CT_DEVICE void dhidden_units(const CutceParams& p, const bf16* G, int slab0, int
   __shared__ int unit_s;
   // the dlogits kernel of the next vocabulary slab starts from fresh work counters
   if (blockIdx.x == 0) reset_dlogits_counters(p.header);
-  // units: (row block, column block) over the started row blocks
+  // Terms of the contraction: the whole slab where the head is padded, else up to the end of the
+  // vocabulary; the last k_width % 128 of them apart, since nothing past a row's end may be read.
+  const int k_width = p.head.padded ? slab_width : min(slab_width, p.V - slab0);
+  const int groups = k_width / 128;
+  const int parts = hidden_parts(sp, n_act, p.d, slab_width / kGemmTile);
+  const size_t part_rows = (size_t)((n_act + kGemmTile - 1) / kGemmTile) * kGemmTile;
+  // units: (row block, (split, column block)) over the started row blocks
   XcdUnits units;
-  units.init(p.header->xcd_counter[0], (n_act + kGemmTile - 1) / kGemmTile, col_blocks);
-  int rb, cb;
-  while (units.next(rb, cb, &unit_s)) {
+  units.init(p.header->xcd_counter[0], (n_act + kGemmTile - 1) / kGemmTile, col_blocks * parts);
+  int rb, cbs;
+  while (units.next(rb, cbs, &unit_s)) {
+    const int split = cbs / col_blocks, cb = cbs % col_blocks;
     const int n0 = rb * kGemmTile, c0 = cb * kGemmTile;
+    const int k_begin = split_begin(groups, split, parts) * 128;
+    const int k_mid = split_begin(groups, split + 1, parts) * 128;
+    // (G^T is zero from the vocabulary's end to the end of the slab)
+    const int k_end = split == parts - 1 && k_mid < k_width ? min(k_mid + 128, slab_width) : k_mid;
     McLoader A;
     A.init(G, p.n_pad, nullptr, n0, p.n_pad, slab_width, true);
-    // (rows of B interleaved: lane j owns the 4 consecutive columns c0 + wn + 4 j + nb)
+    // (rows of B interleaved: lane j owns the 4 consecutive columns c0 + wn + 4 j + nb; rows past d
+    // are copies of the first, their columns are not stored)
     KcLoader B;
-    B.init(p.head + slab0, p.V, nullptr, c0, p.d, min(slab_width, p.V - slab0), p.head_aligned,
-           false, true);
+    B.init(p.head.base + (slab0 - p.head.col0), p.head.ld, nullptr, c0, p.d, k_mid, p.head.aligned, true, true);
     GemmAcc acc;
     acc.clear();
-    gemm_tile(A, B, 0, slab_width, smem, acc);
+    for (int part = 0; part < 2; ++part) {
+      if (part == 1) {
+        if (k_mid == k_end) break;
+        B.alias_invalid_k(k_width);
+        if (!B.fast) B.alias_k = false;  // the guarded loop zero fills by itself
+      }
+      gemm_tile(A, B, part ? k_mid : k_begin, part ? k_end : k_mid, smem, acc);
+    }
 
     const int col = c0 + wn + 4 * j;  // hidden sizes are multiples of 128: col < d implies col + 3 < d
 #pragma unroll
@@ -626,8 +744,12 @@ CT_DEVICE void dhidden_units(const CutceParams& p, const bf16* G, int slab0, int
       for (int r = 0; r < 16; ++r) {
         const int slot = n0 + wm + 32 * i + acc_row(r, half);
         if (slot >= n_act || col >= p.d) continue;
-        const long row = p.idx[slot];
         f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
+        if (parts > 1) {
+          *reinterpret_cast<f32x4*>(sp.hidden_sums + (split * part_rows + slot) * p.d + col) = val;
+          continue;
+        }
+        const long row = p.idx[slot];
         f32x4* a = reinterpret_cast<f32x4*>(dh_acc + (size_t)slot * p.d + col);
         if (mode >= 2) val += *a;
         if (mode == 1 || mode == 2) *a = val;
@@ -643,66 +765,71 @@ CT_DEVICE void dhidden_units(const CutceParams& p, const bf16* G, int slab0, int
 
 __global__ __launch_bounds__(256) void cutce_dhidden_kernel(CutceParams p, const bf16* G,
                                                             int slab0, int slab_width, int mode,
-                                                            float* dh_acc, bf16* dhidden) {
+                                                            float* dh_acc, bf16* dhidden, CutceSplits sp) {
   extern __shared__ __align__(16) char smem_raw[];
-  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, lds_address_of(smem_raw));
+  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, sp, lds_address_of(smem_raw));
+}
+
+// Four consecutive columns of a row of dHead; the rows of an odd vocabulary start at any multiple
+// of 2 bytes, which an ordinary store may.
+CT_DEVICE void store_dhead4(bf16* dst, int left, f32x4 val) {
+  bf16x4 out;
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
+  if (left >= 4) {
+    __builtin_memcpy(dst, &out, 8);
+  } else {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+      if (nb < left) dst[nb] = out[nb];
+  }
 }
 
 // dHead[m, slab0 + v] = sum_slot packed[slot, m] G^T[v, slot], packed[slot] = hidden[idx[slot]]:
 // the workgroup's share of the units, pulled from counter set 1.
 CT_DEVICE void dhead_units(const CutceParams& p, const bf16* packed, const bf16* G, int slab0,
-                           int slab_tiles, bf16* dhead, const lds_addr smem) {
+                           int slab_tiles, bf16* dhead, const CutceSplits& sp, const lds_addr smem) {
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
   const int m_blocks = (p.d + kGemmTile - 1) / kGemmTile;
   const int n_act = p.header->n_act;
   // 4 contraction steps at a time; slots n_act .. k_end-1 are valid memory: G^T holds zeros
   // there (the dlogits kernels write whole 256-slot blocks) and the packed rows are finite.
-  const int k_end = min(p.n_pad, (n_act + 4 * kBK - 1) / (4 * kBK) * (4 * kBK));
+  const int groups = min(p.n_pad, (n_act + 4 * kBK - 1) / (4 * kBK) * (4 * kBK)) / (4 * kBK);
+  const int slab_width = slab_tiles * kGemmTile;
   __shared__ int unit_s;
-  // units: (vocabulary tile of the slab, hidden column block)
+  // units: (vocabulary tile of the slab, (split, hidden column block))
   XcdUnits units;
-  units.init(p.header->xcd_counter[1], slab_tiles, m_blocks);
-  int vt, mb;
-  while (units.next(vt, mb, &unit_s)) {
+  const int parts = head_parts(sp, n_act, p.d);
+  units.init(p.header->xcd_counter[1], slab_tiles, m_blocks * parts);
+  int vt, mbs;
+  while (units.next(vt, mbs, &unit_s)) {
+    const int split = mbs / m_blocks, mb = mbs % m_blocks;
     const int m0 = mb * kGemmTile, v0 = vt * kGemmTile;  // v0 relative to the slab
-    McLoader A;
-    A.init(packed, p.d, nullptr, m0, p.d, k_end, true);
+    const int k_begin = split_begin(groups, split, parts) * 128, k_end = split_begin(groups, split + 1, parts) * 128;
+    McLoader A;  // (columns past d are copies, their rows of dHead are not stored)
+    A.init(packed, p.d, nullptr, m0, p.d, k_end, true, true);
     // (rows of B interleaved: lane j owns the 4 consecutive vocabulary ids v .. v + 3)
     KcLoader B;
-    B.init(G, p.n_pad, nullptr, v0, slab_tiles * kGemmTile, k_end, true, false, true);
+    B.init(G, p.n_pad, nullptr, v0, slab_width, k_end, true, false, true);
     GemmAcc acc;
     acc.clear();
-    gemm_tile(A, B, 0, k_end, smem, acc);
+    gemm_tile(A, B, k_begin, k_end, smem, acc);
 
     const int v = slab0 + v0 + wn + 4 * j;
-    const bool vector_store = (p.V % 4 == 0) && ((reinterpret_cast<uintptr_t>(dhead) & 7u) == 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm + 32 * i + acc_row(r, half);
         if (m >= p.d) continue;
-        bf16* dst = dhead + (size_t)m * p.V + v;
-        if (vector_store && v + 3 < p.V) {
-          bf16x4 out;
-#pragma unroll
-          for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)acc.c[i][nb][r];
-          *reinterpret_cast<bf16x4*>(dst) = out;
-        } else {
-#pragma unroll
-          for (int nb = 0; nb < 4; ++nb)
-            if (v + nb < p.V) dst[nb] = (bf16)acc.c[i][nb][r];
-        }
+        const f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
+        if (parts > 1)
+          *reinterpret_cast<f32x4*>(sp.head_sums + ((size_t)split * p.d + m) * slab_width + (v - slab0)) = val;
+        else
+          store_dhead4(dhead + (size_t)m * p.V + v, p.V - v, val);
       }
   }
-}
-
-__global__ __launch_bounds__(256) void cutce_dhead_kernel(CutceParams p, const bf16* packed,
-                                                          const bf16* G, int slab0, int slab_tiles,
-                                                          bf16* dhead) {
-  extern __shared__ __align__(16) char smem_raw[];
-  dhead_units(p, packed, G, slab0, slab_tiles, dhead, lds_address_of(smem_raw));
 }
 
 // Both gradients of a slab in one launch. The hidden gradient has few, long units (45 x 16 at
@@ -713,11 +840,55 @@ __global__ __launch_bounds__(256) void cutce_dhead_kernel(CutceParams p, const b
 __global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, const bf16* packed,
                                                          const bf16* G, int slab0, int slab_width,
                                                          int slab_tiles, int mode, float* dh_acc,
-                                                         bf16* dhidden, bf16* dhead) {
+                                                         bf16* dhidden, bf16* dhead, CutceSplits sp) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
-  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, smem);
-  dhead_units(p, packed, G, slab0, slab_tiles, dhead, smem);
+  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, sp, smem);
+  dhead_units(p, packed, G, slab0, slab_tiles, dhead, sp, smem);
+}
+
+// Adds the partial sums of cut tiles, a thread 4 columns of a row at a time: first those of dHidden's
+// active rows, then those of the slab's part of dHead. Nothing to do for a gradient that was not cut.
+__global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, int slab0, int slab_width, int mode,
+                                                           float* dh_acc, bf16* dhidden, bf16* dhead,
+                                                           CutceSplits sp) {
+  const int n_act = p.header->n_act;
+  const long first = (long)blockIdx.x * 256 + threadIdx.x, stride = (long)gridDim.x * 256;
+  const int parts_h = hidden_parts(sp, n_act, p.d, slab_width / kGemmTile);
+  if (parts_h > 1) {
+    const int quads = p.d / 4;
+    const size_t part_size = (size_t)((n_act + kGemmTile - 1) / kGemmTile) * kGemmTile * p.d;
+    for (long index = first; index < (long)n_act * quads; index += stride) {
+      const int slot = (int)(index / quads), col = (int)(index % quads) * 4;
+      const float* src = sp.hidden_sums + (size_t)slot * p.d + col;
+      f32x4 val = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+      for (int s = 1; s < parts_h; ++s) val += *reinterpret_cast<const f32x4*>(src + s * part_size);
+      f32x4* a = reinterpret_cast<f32x4*>(dh_acc + (size_t)slot * p.d + col);
+      if (mode >= 2) val += *a;
+      if (mode == 1 || mode == 2) {
+        *a = val;
+      } else {
+        bf16x4 out;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
+        *reinterpret_cast<bf16x4*>(dhidden + (size_t)p.idx[slot] * p.d + col) = out;
+      }
+    }
+  }
+  if (!sp.with_head) return;
+  const int parts_w = head_parts(sp, n_act, p.d);
+  if (parts_w <= 1) return;
+  const int width = min(slab_width, (p.V - slab0 + 3) & ~3);
+  const int quads = width / 4;
+  for (long index = first; index < (long)p.d * quads; index += stride) {
+    const int m = (int)(index / quads), v = (int)(index % quads) * 4;
+    const float* src = sp.head_sums + (size_t)m * slab_width + v;
+    f32x4 val = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+    for (int s = 1; s < parts_w; ++s) val += *reinterpret_cast<const f32x4*>(src + (size_t)s * p.d * slab_width);
+    store_dhead4(dhead + (size_t)m * p.V + slab0 + v, p.V - slab0 - v, val);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -727,12 +898,33 @@ static size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 static int padded_rows(int N) { return (int)align_up((size_t)N, kGemmTile); }
 static int vocab_tile_count(int V) { return (V + kGemmTile - 1) / kGemmTile; }
-static int stats_chunks(int V) {
-  return (vocab_tile_count(V) + kTilesPerChunk - 1) / kTilesPerChunk;
+
+// Vocabulary tiles per work unit of the two projection kernels. Four keep a unit's hidden rows in use
+// for four tiles and leave a quarter of the partial statistics; with fewer than two units per compute
+// unit that costs more than it gives (the last round, or the only one, is longer), so short problems
+// take units of two tiles or one.
+static int tiles_per_chunk(int tiles, int row_blocks) {
+  for (int t = 4; t > 1; t /= 2)
+    if ((long)((tiles + t - 1) / t) * row_blocks >= 2 * kComputeUnits) return t;
+  return 1;
+}
+static int stats_chunks(const ct_cutce_shape& s) {
+  const int tiles = vocab_tile_count(s.vocab);
+  const int t = tiles_per_chunk(tiles, padded_rows(s.rows) / kGemmTile);
+  return (tiles + t - 1) / t;
 }
 
+// Heads whose rows do not all start on 16 bytes go through an aligned copy (cutce_panel_kernel).
+static bool needs_panel(const ct_cutce_shape& s) { return s.vocab % 8 != 0; }
+static size_t panel_tile_bytes(const ct_cutce_shape& s) { return (size_t)s.hidden * kGemmTile * sizeof(bf16); }
+// bytes of the panel of the whole vocabulary, 0 if none is needed
+static size_t full_panel_bytes(const ct_cutce_shape& s) {
+  return needs_panel(s) ? panel_tile_bytes(s) * vocab_tile_count(s.vocab) : 0;
+}
+
+// Workspace of the forward: `base` bytes it cannot do without, then as much of the panel as fits.
 struct FwdLayout {
-  size_t header, idx, part, sums, total;
+  size_t header, idx, part, sums, base, total;
 };
 static FwdLayout fwd_layout(const ct_cutce_shape& s) {
   const int n_pad = padded_rows(s.rows);
@@ -740,13 +932,29 @@ static FwdLayout fwd_layout(const ct_cutce_shape& s) {
   L.header = 0;
   L.idx = align_up(sizeof(CutceHeader), 256);
   L.part = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
-  L.sums = L.part + align_up((size_t)stats_chunks(s.vocab) * n_pad * 3 * sizeof(float), 256);
-  L.total = L.sums + align_up((size_t)(n_pad / kMergeSlots) * 2 * sizeof(double), 256);
+  L.sums = L.part + align_up((size_t)stats_chunks(s) * n_pad * 3 * sizeof(float), 256);
+  L.base = L.sums + align_up((size_t)(n_pad / kMergeSlots) * 2 * sizeof(double), 256);
+  L.total = L.base + full_panel_bytes(s);
   return L;
 }
 
+// Room for the partial sums (see CutceSplits). The bytes that the parts of dHidden take, and the number
+// of parts of dHead, are largest with every row active (times 4/3: a number of parts is rounded).
+static size_t hidden_sums_bytes(const ct_cutce_shape& s, int slab_tiles, bool with_head) {
+  const int row_blocks = padded_rows(s.rows) / kGemmTile;
+  const double parts = 2.0 * slab_tiles / part_length(row_blocks, s.hidden, slab_tiles, with_head);
+  const double least = 1.5 / row_blocks;  // with fewer not even a single row block is cut
+  return parts < least ? 0 : align_up((size_t)(1.34 * parts * padded_rows(s.rows) * s.hidden * sizeof(float)), 256);
+}
+static int most_head_parts(const ct_cutce_shape& s) {
+  const int row_blocks = padded_rows(s.rows) / kGemmTile;
+  return whole_parts(2.f * row_blocks / part_length(row_blocks, s.hidden, vocab_tile_count(s.vocab), true));
+}
+
 struct BwdLayout {
-  size_t header, idx, rowparams, packed, g, acc, total;
+  size_t header, idx, rowparams, packed, panel, g, head_sums, acc, hidden_sums, total;
+  size_t hidden_sums_bytes;
+  int head_most;
   int slab_cols;  // multiple of 256
   int slabs;
 };
@@ -755,8 +963,25 @@ static size_t bwd_fixed_bytes(int n_pad, int d) {
   return align_up(sizeof(CutceHeader), 256) + 4 * align_up((size_t)n_pad * sizeof(int), 256) +
          align_up((size_t)n_pad * d * sizeof(bf16), 256);
 }
-// Largest slab that fits in `bytes` (0 if even one tile column does not).
-static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes) {
+// What one tile column of a slab takes: its part of G^T, without a panel in the logits cache of the
+// panel, and the partial sums of dHead if that is cut.
+struct BwdTileBytes {
+  size_t g, panel, head_sums;
+  size_t all() const { return g + panel + head_sums; }
+};
+static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, bool panel_in_cache, bool with_head) {
+  const int parts = with_head ? most_head_parts(s) : 1;
+  return BwdTileBytes{(size_t)padded_rows(s.rows) * kGemmTile * sizeof(bf16),
+                      needs_panel(s) && !panel_in_cache ? panel_tile_bytes(s) : 0,
+                      parts > 1 ? (size_t)parts * s.hidden * kGemmTile * sizeof(float) : 0};
+}
+static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
+  return align_up((size_t)padded_rows(s.rows) * s.hidden * sizeof(float), 256);
+}
+// The whole vocabulary as one slab if that fits in `bytes`, else the largest slab that does
+// (slab_cols = 0 if even one tile column does not). The partial sums of a cut dHidden come last: as
+// many parts as fit behind one slab, with several slabs in up to half of what is left for slabs.
+static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_in_cache, bool with_head) {
   const int n_pad = padded_rows(s.rows);
   const int tiles = vocab_tile_count(s.vocab);
   BwdLayout L = {};
@@ -764,22 +989,32 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes) {
   L.idx = align_up(sizeof(CutceHeader), 256);
   L.rowparams = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
   L.packed = L.rowparams + 3 * align_up((size_t)n_pad * sizeof(int), 256);
-  L.g = bwd_fixed_bytes(n_pad, s.hidden);
-  const size_t per_tile = (size_t)n_pad * kGemmTile * sizeof(bf16);
-  const size_t acc_bytes = align_up((size_t)n_pad * s.hidden * sizeof(float), 256);
-  if (bytes >= L.g + per_tile * tiles) {
-    L.slab_cols = tiles * kGemmTile;
-    L.slabs = 1;
-    L.acc = 0;
-    L.total = L.g + per_tile * tiles;
-    return L;
+  L.panel = bwd_fixed_bytes(n_pad, s.hidden);
+  const BwdTileBytes tile = bwd_tile_bytes(s, panel_in_cache, with_head);
+  const size_t per_tile = tile.all(), acc_bytes = bwd_acc_bytes(s);
+  size_t fit = tiles, room;
+  L.head_most = with_head ? most_head_parts(s) : 1;
+  if (bytes < L.panel + per_tile * tiles) {
+    if (bytes < L.panel + acc_bytes + per_tile) return L;
+    room = bytes - L.panel - acc_bytes;
+    fit = room / per_tile;
+    for (size_t fewer = fit; fewer > fit / 2; fewer -= (fewer + 7) / 8) {
+      if (per_tile * fewer + hidden_sums_bytes(s, (int)fewer, with_head) > room) continue;
+      fit = fewer;
+      break;
+    }
+  } else {
+    room = bytes - L.panel;
   }
-  if (bytes < L.g + acc_bytes + per_tile) return L;  // slab_cols == 0
-  const size_t fit = (bytes - L.g - acc_bytes) / per_tile;
+  const size_t want = hidden_sums_bytes(s, (int)fit, with_head), spare = (room - per_tile * fit) / 256 * 256;
+  L.hidden_sums_bytes = want < spare ? want : spare;
   L.slab_cols = (int)fit * kGemmTile;
   L.slabs = (tiles + (int)fit - 1) / (int)fit;
-  L.acc = L.g + per_tile * fit;
-  L.total = L.acc + acc_bytes;
+  L.g = L.panel + tile.panel * fit;
+  L.head_sums = L.g + tile.g * fit;
+  L.acc = L.head_sums + tile.head_sums * fit;
+  L.hidden_sums = L.acc + (L.slabs > 1 ? acc_bytes : 0);
+  L.total = L.hidden_sums + L.hidden_sums_bytes;
   return L;
 }
 
@@ -812,37 +1047,45 @@ static int device_cu_count() {
 
 using namespace ct;
 
+static bool valid_sizes(const ct_cutce_shape* s) { return s && s->rows > 0 && s->hidden > 0 && s->vocab > 0; }
+
 extern "C" size_t ct_cutce_fwd_workspace_bytes(const ct_cutce_shape* shape) {
-  if (!shape || shape->rows <= 0 || shape->vocab <= 0) return 0;
-  return fwd_layout(*shape).total;
+  return valid_sizes(shape) ? fwd_layout(*shape).total : 0;
 }
 
+extern "C" size_t ct_cutce_fwd_workspace_min_bytes(const ct_cutce_shape* shape) {
+  return valid_sizes(shape) ? fwd_layout(*shape).base : 0;
+}
+
+namespace ct {
+static size_t logits_bytes(const ct_cutce_shape& s) {
+  return (size_t)padded_rows(s.rows) * vocab_tile_count(s.vocab) * kGemmTile * sizeof(float);
+}
+}  // namespace ct
+
 extern "C" size_t ct_cutce_logits_cache_bytes(const ct_cutce_shape* shape) {
-  if (!shape || shape->rows <= 0 || shape->vocab <= 0) return 0;
-  return (size_t)padded_rows(shape->rows) * vocab_tile_count(shape->vocab) * kGemmTile * sizeof(float);
+  return valid_sizes(shape) ? logits_bytes(*shape) + full_panel_bytes(*shape) : 0;
 }
 
 extern "C" size_t ct_cutce_bwd_workspace_bytes(const ct_cutce_shape* shape) {
-  if (!shape || shape->rows <= 0 || shape->vocab <= 0) return 0;
-  const int n_pad = padded_rows(shape->rows);
-  return bwd_fixed_bytes(n_pad, shape->hidden) +
-         (size_t)n_pad * vocab_tile_count(shape->vocab) * kGemmTile * sizeof(bf16);
+  if (!valid_sizes(shape)) return 0;
+  const size_t trained = bwd_layout(*shape, ~(size_t)0, false, true).total;
+  const size_t frozen = bwd_layout(*shape, ~(size_t)0, false, false).total;
+  return trained > frozen ? trained : frozen;
 }
 
 extern "C" size_t ct_cutce_bwd_workspace_min_bytes(const ct_cutce_shape* shape) {
-  if (!shape || shape->rows <= 0 || shape->vocab <= 0) return 0;
-  const int n_pad = padded_rows(shape->rows);
-  if (vocab_tile_count(shape->vocab) == 1) return ct_cutce_bwd_workspace_bytes(shape);
-  return bwd_fixed_bytes(n_pad, shape->hidden) +
-         align_up((size_t)n_pad * shape->hidden * sizeof(float), 256) +
-         (size_t)n_pad * kGemmTile * sizeof(bf16);
+  if (!valid_sizes(shape)) return 0;
+  const size_t fixed =
+      bwd_fixed_bytes(padded_rows(shape->rows), shape->hidden) + bwd_tile_bytes(*shape, false, true).all();
+  return vocab_tile_count(shape->vocab) == 1 ? fixed : fixed + bwd_acc_bytes(*shape);
 }
 
 static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, const int32_t* targets,
                                const float* weights, const ct_cutce_shape& s, char* ws) {
   CutceParams p;
   p.hidden = reinterpret_cast<const bf16*>(hidden);
-  p.head = reinterpret_cast<const bf16*>(head);
+  p.head = HeadView{reinterpret_cast<const bf16*>(head), s.vocab, 0, is_aligned16(head) && s.vocab % 8 == 0, false};
   p.targets = targets;
   p.weights = weights;
   p.N = s.rows;
@@ -852,8 +1095,20 @@ static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, con
   p.header = reinterpret_cast<CutceHeader*>(ws);
   p.idx = reinterpret_cast<int*>(ws + align_up(sizeof(CutceHeader), 256));
   p.hidden_aligned = is_aligned16(hidden);
-  p.head_aligned = is_aligned16(head) && (s.vocab % 8 == 0);
   return p;
+}
+
+// Fills `panel` with the tile columns tile0 .. tile0 + tiles - 1 of the head.
+static int launch_panel(hipStream_t stream, const bf16* head, const ct_cutce_shape& s, int tile0, int tiles, bf16* panel,
+                        CutceHeader* counters_to_reset) {
+  const int cols = tiles * kGemmTile;
+  LaunchScope scope("cutce_panel_kernel", stream);
+  hipLaunchKernelGGL(cutce_panel_kernel, dim3((cols + 2047) / 2048, s.hidden / kPanelRows), dim3(256), 0, stream, head,
+                     s.vocab, s.hidden, tile0 * kGemmTile, cols, panel, counters_to_reset);
+  return scope.done();
+}
+static HeadView panel_view(const bf16* panel, int tile0, int tiles) {
+  return HeadView{panel, (long)tiles * kGemmTile, tile0 * kGemmTile, true, true};
 }
 
 // Shared body of ct_cutce_fwd and ct_cutce_fwd_noalloc: `ws` / `ws_bytes` is the workspace to use
@@ -866,8 +1121,8 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   int rc = validate_cutce(fn, a->shape);
   if (rc) return rc;
   const FwdLayout L = fwd_layout(a->shape);
-  if (ws_bytes < L.total)
-    return fail(CT_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu bytes", fn, ws_bytes, L.total);
+  if (ws_bytes < L.base)
+    return fail(CT_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu bytes", fn, ws_bytes, L.base);
   CT_REQUIRE(is_aligned16(ws_), "%s: workspace must be 16-byte aligned", fn);
   if (a->logits_cache) {
     CT_REQUIRE(is_aligned16(a->logits_cache), "%s: logits cache must be 16-byte aligned", fn);
@@ -880,26 +1135,49 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, ws);
   float* part = reinterpret_cast<float*>(ws + L.part);
   double* sums = reinterpret_cast<double*>(ws + L.sums);
-  const int chunks = stats_chunks(p.V);
-  const int row_blocks = p.n_pad / kGemmTile;
+  const int chunks = stats_chunks(a->shape), row_blocks = p.n_pad / kGemmTile, tiles = vocab_tile_count(p.V);
+  const int per_chunk = tiles_per_chunk(tiles, row_blocks);
+  const bf16* head = p.head.base;
 
   LaunchScope scope1("cutce_index_kernel", stream);
-  hipLaunchKernelGGL(cutce_index_kernel, dim3(1), dim3(1024), 0, stream, p.weights, p.N, p.n_pad,
-                     a->sparse_compaction ? 1 : 0, p.idx, p.header);
+  hipLaunchKernelGGL(cutce_index_kernel<false>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p,
+                     a->sparse_compaction ? 1 : 0, nullptr, nullptr, CutceRowParams{});
   if ((rc = scope1.done())) return rc;
 
+  // The panel of a head with unaligned rows: at the end of the logits cache, where the backward finds
+  // it again, or in what the workspace has behind its fixed part, a number of chunks at a time.
+  bf16* panel = nullptr;
+  int chunks_per_pass = chunks;
+  if (needs_panel(a->shape)) {
+    if (a->logits_cache) {
+      panel = reinterpret_cast<bf16*>(static_cast<char*>(a->logits_cache) + logits_bytes(a->shape));
+    } else {
+      const size_t chunk_bytes = panel_tile_bytes(a->shape) * per_chunk;
+      const size_t fit = ws_bytes >= L.total ? (size_t)chunks : (ws_bytes - L.base) / chunk_bytes;
+      if (fit) panel = reinterpret_cast<bf16*>(ws + L.base);
+      if (fit) chunks_per_pass = (int)(fit < (size_t)chunks ? fit : (size_t)chunks);
+    }
+  }
   const size_t smem = GemmSmem::kBytes;
   if ((rc = set_smem(cutce_stats_kernel<false>, smem, fn))) return rc;
   if ((rc = set_smem(cutce_stats_kernel<true>, smem, fn))) return rc;
-  const int persistent = min(device_cu_count(), chunks * row_blocks);
-  LaunchScope scope2("cutce_stats_kernel", stream);
-  if (a->logits_cache)
-    hipLaunchKernelGGL(cutce_stats_kernel<true>, dim3(persistent), dim3(256), smem, stream, p, part,
-                       chunks, static_cast<float*>(a->logits_cache));
-  else
-    hipLaunchKernelGGL(cutce_stats_kernel<false>, dim3(persistent), dim3(256), smem, stream, p, part,
-                       chunks, static_cast<float*>(nullptr));
-  if ((rc = scope2.done())) return rc;
+  for (int chunk0 = 0; chunk0 < chunks; chunk0 += chunks_per_pass) {
+    const int pass_chunks = min(chunks_per_pass, chunks - chunk0);
+    if (panel) {
+      const int tile0 = chunk0 * per_chunk, pass_tiles = min(pass_chunks * per_chunk, tiles - tile0);
+      if ((rc = launch_panel(stream, head, a->shape, tile0, pass_tiles, panel, p.header))) return rc;
+      p.head = panel_view(panel, tile0, pass_tiles);
+    }
+    const int persistent = min(device_cu_count(), pass_chunks * row_blocks);
+    LaunchScope scope2("cutce_stats_kernel", stream);
+    if (a->logits_cache)
+      hipLaunchKernelGGL(cutce_stats_kernel<true>, dim3(persistent), dim3(256), smem, stream, p, part, chunk0,
+                         pass_chunks, per_chunk, static_cast<float*>(a->logits_cache));
+    else
+      hipLaunchKernelGGL(cutce_stats_kernel<false>, dim3(persistent), dim3(256), smem, stream, p, part, chunk0,
+                         pass_chunks, per_chunk, static_cast<float*>(nullptr));
+    if ((rc = scope2.done())) return rc;
+  }
 
   const int merge_blocks = p.n_pad / kMergeSlots;
   LaunchScope scope3("cutce_merge_kernel", stream);
@@ -938,7 +1216,7 @@ extern "C" int32_t ct_cutce_fwd_noalloc(void* stream, const ct_cutce_fwd_args* a
   CT_REQUIRE(a, "ct_cutce_fwd_noalloc: null args");
   int rc = validate_cutce("ct_cutce_fwd_noalloc", a->shape);
   if (rc) return rc;
-  const size_t need = fwd_layout(a->shape).total;
+  const size_t need = fwd_layout(a->shape).base;  // (a panel, if one is needed, takes what is left)
   if (need > kNoAllocScratchBytes)
     return fail(CT_UNSUPPORTED,
                 "ct_cutce_fwd_noalloc: rows=%d, vocab=%d need %zu bytes of scratch, the static "
@@ -975,7 +1253,7 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   if (rc) return rc;
   CT_REQUIRE(is_aligned16(a->workspace) && is_aligned16(a->dhidden),
              "ct_cutce_bwd: workspace and dhidden must be 16-byte aligned");
-  const BwdLayout L = bwd_layout(a->shape, a->workspace_bytes);
+  const BwdLayout L = bwd_layout(a->shape, a->workspace_bytes, a->logits_cache != nullptr, a->dhead != nullptr);
   if (L.slab_cols == 0)
     return fail(CT_WORKSPACE_TOO_SMALL, "ct_cutce_bwd: workspace %zu < %zu bytes",
                 a->workspace_bytes, ct_cutce_bwd_workspace_min_bytes(&a->shape));
@@ -1002,62 +1280,77 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   const size_t smem = GemmSmem::kBytes;
   if ((rc = set_smem(cutce_dlogits_kernel, smem, "ct_cutce_bwd"))) return rc;
   if ((rc = set_smem(cutce_dhidden_kernel, smem, "ct_cutce_bwd"))) return rc;
-  if ((rc = set_smem(cutce_dhead_kernel, smem, "ct_cutce_bwd"))) return rc;
   if ((rc = set_smem(cutce_grads_kernel, smem, "ct_cutce_bwd"))) return rc;
 
   LaunchScope scope5("cutce_index_kernel", stream);
-  hipLaunchKernelGGL(cutce_index_kernel, dim3(1), dim3(1024), 0, stream, p.weights, p.N, p.n_pad,
-                     a->sparse_compaction ? 1 : 0, p.idx, p.header);
+  hipLaunchKernelGGL(cutce_index_kernel<true>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p,
+                     a->sparse_compaction ? 1 : 0, a->lse, a->dy, rp);
   if ((rc = scope5.done())) return rc;
-  LaunchScope scope6("cutce_zero_rows_kernel", stream);
-  hipLaunchKernelGGL(cutce_zero_rows_kernel, dim3(p.N), dim3(256), 0, stream, p.weights, p.N, p.d,
-                     dhidden);
+  bf16* packed = dhead ? reinterpret_cast<bf16*>(ws + L.packed) : nullptr;
+  LaunchScope scope6("cutce_rows_kernel", stream);
+  hipLaunchKernelGGL(cutce_rows_kernel, dim3(p.n_pad / 4), dim3(256), 0, stream, p, packed, dhidden);
   if ((rc = scope6.done())) return rc;
-  LaunchScope scope10("cutce_rowparams_kernel", stream);
-  hipLaunchKernelGGL(cutce_rowparams_kernel, dim3(row_blocks), dim3(256), 0, stream, p, a->lse, a->dy,
-                     rp);
-  if ((rc = scope10.done())) return rc;
 
   const int cus = device_cu_count();
-  bf16* packed = reinterpret_cast<bf16*>(ws + L.packed);
-  if (dhead) {
-    LaunchScope scope12("cutce_pack_rows_kernel", stream);
-    hipLaunchKernelGGL(cutce_pack_rows_kernel, dim3(p.n_pad), dim3(256), 0, stream, p, packed);
-    if ((rc = scope12.done())) return rc;
-  }
-
   const int tiles = vocab_tile_count(p.V);
   const int tiles_per_slab = L.slab_cols / kGemmTile;
+  const bf16* head = p.head.base;
+  bf16* panel = nullptr;
+  if (needs_panel(a->shape)) {
+    if (cache) {  // the forward left it there
+      p.head = panel_view(reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(cache) + logits_bytes(a->shape)), 0, tiles);
+    } else {
+      panel = reinterpret_cast<bf16*>(ws + L.panel);
+    }
+  }
   for (int s = 0; s < L.slabs; ++s) {
     const int slab0 = s * L.slab_cols;
     const int slab_tiles = min(tiles_per_slab, tiles - s * tiles_per_slab);
     const int slab_width = slab_tiles * kGemmTile;
+    if (panel) {
+      if ((rc = launch_panel(stream, head, a->shape, s * tiles_per_slab, slab_tiles, panel, nullptr))) return rc;
+      p.head = panel_view(panel, s * tiles_per_slab, slab_tiles);
+    }
     if (cache) {
       LaunchScope scope11("cutce_dlogits_cached_kernel", stream);
-      hipLaunchKernelGGL(cutce_dlogits_cached_kernel, dim3(slab_width / kDlogitsRows, (p.n_pad + 2047) / 2048),
-                         dim3(256), 0, stream, p, rp, cache, slab0, G);
+      const long threads = (long)(slab_width / kDlogitsRows) * (p.n_pad / 8);
+      hipLaunchKernelGGL(cutce_dlogits_cached_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p, rp,
+                         cache, slab0, slab_width, G);
       if ((rc = scope11.done())) return rc;
     } else {
       LaunchScope scope7("cutce_dlogits_kernel", stream);
-      const int dl_units = ((slab_tiles + kTilesPerChunk - 1) / kTilesPerChunk) * row_blocks;
+      const int per_chunk = tiles_per_chunk(slab_tiles, row_blocks);
+      const int dl_units = ((slab_tiles + per_chunk - 1) / per_chunk) * row_blocks;
       hipLaunchKernelGGL(cutce_dlogits_kernel, dim3(min(cus, dl_units)), dim3(256), smem, stream,
-                         p, rp, slab0, slab_tiles, G);
+                         p, rp, slab0, slab_tiles, per_chunk, G);
       if ((rc = scope7.done())) return rc;
     }
     const int mode = L.slabs == 1 ? 0 : (s == 0 ? 1 : (s == L.slabs - 1 ? 3 : 2));
-    const int col_blocks = (p.d + kGemmTile - 1) / kGemmTile;
+    CutceSplits sp;
+    sp.hidden_sums = reinterpret_cast<float*>(ws + L.hidden_sums);
+    sp.head_sums = reinterpret_cast<float*>(ws + L.head_sums);
+    sp.hidden_room = L.hidden_sums_bytes / sizeof(float);
+    sp.head_most = L.head_most;
+    sp.all_tiles = tiles;
+    sp.with_head = dhead != nullptr;
     if (dhead) {
       // both gradients in one launch: the head-gradient units fill the hidden gradient's tail
       LaunchScope scope8("cutce_grads_kernel", stream);
-      const int units = max(row_blocks * col_blocks, col_blocks * slab_tiles);
-      hipLaunchKernelGGL(cutce_grads_kernel, dim3(min(cus, units)), dim3(256), smem, stream, p, packed, G,
-                         slab0, slab_width, slab_tiles, mode, dh_acc, dhidden, dhead);
+      hipLaunchKernelGGL(cutce_grads_kernel, dim3(cus), dim3(256), smem, stream, p, packed,
+                         G, slab0, slab_width, slab_tiles, mode, dh_acc, dhidden, dhead, sp);
       if ((rc = scope8.done())) return rc;
     } else {
       LaunchScope scope8("cutce_dhidden_kernel", stream);
-      hipLaunchKernelGGL(cutce_dhidden_kernel, dim3(min(cus, row_blocks * col_blocks)), dim3(256), smem,
-                         stream, p, G, slab0, slab_width, mode, dh_acc, dhidden);
+      hipLaunchKernelGGL(cutce_dhidden_kernel, dim3(cus), dim3(256), smem,
+                         stream, p, G, slab0, slab_width, mode, dh_acc, dhidden, sp);
       if ((rc = scope8.done())) return rc;
+    }
+    if (sp.hidden_room || sp.head_most > 1) {
+      LaunchScope scope9("cutce_reduce_kernel", stream);
+      const long quads = max((long)p.n_pad * p.d, sp.head_most > 1 ? (long)p.d * slab_width : 0) / 4;
+      hipLaunchKernelGGL(cutce_reduce_kernel, dim3((unsigned)min((quads + 255) / 256, (long)cus * 8)), dim3(256), 0, stream, p,
+                         slab0, slab_width, mode, dh_acc, dhidden, dhead, sp);
+      if ((rc = scope9.done())) return rc;
     }
   }
   return CT_OK;

@@ -62,6 +62,7 @@ struct KcLoader {
   u32x4 regs[NCH];
   int chunk, k_valid, row_mask;
   bool fast;
+  bool alias_k;  // k >= k_valid (a multiple of 8) reads the row's first chunk: see alias_invalid_k()
 
   // rows m0 .. m0+255 of `base_` (leading dimension ld elements), optionally
   // gathered through row_index. Rows >= rows_valid read as zero, or, with
@@ -75,6 +76,7 @@ struct KcLoader {
                       bool interleave_rows = false) {
     const int t = threadIdx.x;
     k_valid = k_valid_;
+    alias_k = false;
     const bool gathered = row_index != nullptr;
     base = reinterpret_cast<const char*>(gathered ? base_ : base_ + (size_t)m0 * ld);
     row_mask = 0;
@@ -92,10 +94,24 @@ struct KcLoader {
     }
     fast = aligned && (alias_invalid_rows || m0 + kGemmTile <= rows_valid) && k_valid % kGemmBK == 0;
   }
+  // For the last steps of a contraction that ends inside a step: from here on terms k >= k_valid are
+  // read as the first terms of their row, so the copies stay inside the rows and the pipelined
+  // loop serves (for callers whose other operand is zero there).
+  CT_DEVICE void alias_invalid_k(int k_valid_) {
+    k_valid = k_valid_;
+    alias_k = true;
+  }
   // copies N0 .. N1-1 of the thread's NCH 16-byte slots
   template <int N0 = 0, int N1 = NCH>
   CT_DEVICE void dma(int k0, lds_addr tile) const {
     const int wave = uniform(threadIdx.x >> 6);
+    if (alias_k) {  // uniform
+      const bool inside = k0 + chunk * 8 < k_valid;
+#pragma unroll
+      for (int n = N0; n < N1; ++n)
+        dma16_s(base, inside ? voff[n] + (unsigned)k0 * 2u : voff[n] - (unsigned)chunk * 16u, tile + (n * 256 + wave * 64) * 16);
+      return;
+    }
     const char* p = base + (size_t)k0 * 2;
 #pragma unroll
     for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
@@ -137,21 +153,25 @@ struct McLoader {
   bool fast;
 
   // columns m0 .. m0+255 of `base_`; contraction rows optionally gathered.
-  // Columns >= cols_valid and rows >= k_valid read as zero.
+  // Columns >= cols_valid and rows >= k_valid read as zero, or, with alias_invalid_cols (then m0 and
+  // cols_valid are multiples of 8), the columns as a copy of the tile's first 8 (for callers that
+  // discard what they get from them): a ragged last tile then takes the pipelined loop too.
   CT_DEVICE void init(const bf16* base_, long ld_, const int* row_index_, int m0, int cols_valid,
-                      int k_valid_, bool aligned) {
+                      int k_valid_, bool aligned, bool alias_invalid_cols = false) {
     const int t = threadIdx.x;
     base = reinterpret_cast<const char*>(base_ + m0);
     row_index = row_index_;
     ld = ld_;
     k_valid = k_valid_;
     cols_left = cols_valid - m0;
-    fast = aligned && m0 + kGemmTile <= cols_valid && k_valid % kGemmBK == 0;
+    alias_invalid_cols = alias_invalid_cols && aligned;
+    fast = aligned && (alias_invalid_cols || m0 + kGemmTile <= cols_valid) && k_valid % kGemmBK == 0;
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
       const int r = t / CPR + 8 * n;
-      const int c = ((t % CPR) ^ swizzle<CPR>(r)) * 8;
+      int c = ((t % CPR) ^ swizzle<CPR>(r)) * 8;
       col[n & 1] = c;
+      if (alias_invalid_cols && c >= cols_left) c = 0;
       voff[n] = (unsigned)(((row_index ? 0 : (long)r * ld) + c) * 2);
     }
   }
@@ -327,7 +347,7 @@ CT_DEVICE void gemm_tile(ALoader& A, BLoader& B, int k_begin, int k_end, lds_add
     wait_vmcnt((min(steps, 3) - 1) * kLoadsPerStep);
     workgroup_barrier();
     if constexpr (std::is_same<ALoader, McLoader>::value && std::is_same<BLoader, KcLoader>::value) {
-      if (steps % 4 == 0 && !A.row_index) {  // uniform
+      if (steps % 4 == 0 && !A.row_index && !B.alias_k) {  // uniform
         gemm_loop_scheduled(A, B, k_begin, steps, smem, afo, bfo, wm, wn, acc);
         return;
       }

@@ -382,18 +382,25 @@ typedef struct ct_cutce_shape {
   int32_t vocab;  /* V > 0 */
 } ct_cutce_shape;
 
-/* Bytes of workspace ct_cutce_fwd needs. */
+/* Preferred and smallest workspace for ct_cutce_fwd. The two differ where vocab is no multiple of
+ * 8: the kernels then read the head through an aligned copy of its columns (2 bytes per element),
+ * made in the workspace behind its fixed part as many columns at a time as fit, or in the logits
+ * cache if there is one; with no room for it the projection runs in a slower guarded loop. Same
+ * results in each case. */
 size_t ct_cutce_fwd_workspace_bytes(const ct_cutce_shape* shape);
+size_t ct_cutce_fwd_workspace_min_bytes(const ct_cutce_shape* shape);
 /*
  * Smallest and preferred workspace for ct_cutce_bwd. With the preferred size
- * the whole vocabulary is processed as one slab; with less, the vocabulary
- * is walked in slabs and dHidden is accumulated in f32 in the workspace.
+ * the whole vocabulary is processed as one slab, and gradient tiles with long
+ * contractions may be cut into parts that leave f32 partial sums; with less, the
+ * vocabulary is walked in slabs and dHidden is accumulated in f32 in the workspace.
  */
 size_t ct_cutce_bwd_workspace_min_bytes(const ct_cutce_shape* shape);
 size_t ct_cutce_bwd_workspace_bytes(const ct_cutce_shape* shape);
 /*
  * Bytes of the optional logits cache (f32, vocabulary-major, rows and
- * vocabulary padded to 256). When the caller lends one to ct_cutce_fwd and
+ * vocabulary padded to 256; where vocab is no multiple of 8 also the aligned copy
+ * of the head that both directions read). When the caller lends one to ct_cutce_fwd and
  * hands the same buffer to ct_cutce_bwd, the backward forms its bf16 dlogits
  * from the cached f32 logits instead of repeating the projection: 3 GEMMs per
  * step instead of 4 (the reference runs 5, src/kernels/cut_cross_entropy.py:258,
@@ -437,7 +444,7 @@ int32_t ct_cutce_fwd(void* stream, const ct_cutce_fwd_args* args);
  * kernels as ct_cutce_fwd, but args->workspace / workspace_bytes are ignored:
  * the workspace is a static device array inside the library,
  * ct_cutce_fwd_noalloc_max_bytes() (32 MiB) per GPU, held until the process
- * ends. Shapes whose ct_cutce_fwd_workspace_bytes() exceeds that are rejected
+ * ends. Shapes whose ct_cutce_fwd_workspace_min_bytes() exceeds that are rejected
  * with CT_UNSUPPORTED before any launch (N = 16384, V = 128256 needs 25 MB and
  * fits). The call makes no hipMalloc / hipFree and no allocating library call.
  * All calls on one GPU share the array: calls that overlap on one GPU (two

@@ -332,3 +332,38 @@ def test_benchmark_shape(ct, gpu, cache):
     g = ((weights * dy)[:, None] * (prob - onehot.float())).to(torch.bfloat16).float()
     dw_ref = hidden.float().T @ g
     assert relative_l2(dhead[:, cols], dw_ref) <= GRAD_RTOL
+
+
+@pytest.mark.parametrize("rows,width,vocab", [
+    (1, 128, 7),          # smaller than any tile, one term in the last group
+    (70, 1408, 1016),     # aligned rows, a ragged last tile, half a hidden tile; both gradients cut
+    (999, 256, 4099),     # unaligned rows: the panel; dHidden cut
+    (2817, 384, 264),     # many rows, two vocabulary tiles: dHead cut
+    (513, 128, 33025),    # units of several vocabulary tiles, one column in the last
+])
+def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
+    """Sizes at the edges of the panel, of the tiles and of the parts the gradient contractions are cut
+    into; the forward gives the same bits whatever part of the panel its workspace holds."""
+
+    import ctypes
+
+    case = _case(rows + vocab, rows, width, vocab)
+    for cache in (False, True):
+        print("case", rows, width, vocab, cache, flush=True)
+        _check(_gpu(ct, gpu, *case, 0.37, compaction=True, cache=cache), *case, 0.37)
+    lib, shape = ct._lib.load(), ct._lib.CutceShape(rows, width, vocab)
+    least = lib.ct_cutce_fwd_workspace_min_bytes(ctypes.byref(shape))
+    full = lib.ct_cutce_fwd_workspace_bytes(ctypes.byref(shape))
+    assert (full > least) == (vocab % 8 != 0)
+    hidden, head, targets, weights = (t.to(gpu) for t in case)
+    results = []
+    for size in (full, (least + full) // 2, least):     # all of the panel, some of it, the guarded loop
+        out = torch.full((rows + 2,), float("nan"), device=gpu)
+        workspace = torch.empty(size, dtype=torch.uint8, device=gpu)
+        args = ct._lib.CutceFwdArgs(
+            hidden=hidden.data_ptr(), head=head.data_ptr(), targets=targets.data_ptr(), weights=weights.data_ptr(),
+            nll_sum=out[0:].data_ptr(), weight_sum=out[1:].data_ptr(), lse=out[2:].data_ptr(),
+            workspace=workspace.data_ptr(), workspace_bytes=size, shape=shape, sparse_compaction=1)
+        ct._lib.check(lib.ct_cutce_fwd(ct._lib.current_stream(), args))
+        results.append(out.cpu())
+    assert all(torch.equal(r, results[0]) for r in results[1:]) and torch.isfinite(results[0]).all()
