@@ -21,6 +21,7 @@
 // The cache is vocabulary-major [vocab, rows] like G^T: in the transposed tile
 // the GEMMs produce, the lanes of a wavefront run along the rows, so both are
 // written with contiguous stores.
+#include <atomic>
 #include <mutex>
 
 #include "ct_error.h"
@@ -30,10 +31,6 @@ namespace ct {
 
 constexpr int kBK = kGemmBK;
 constexpr int kComputeUnits = 256;    // of an MI355X; sizes of work units are chosen by it
-#ifndef CT_CUTCE_SWEEP
-#define CT_CUTCE_SWEEP 1
-#endif
-constexpr bool kSweepUnits = CT_CUTCE_SWEEP != 0;  // unit order of the two projection kernels
 constexpr float kNegInfF = -__builtin_inff();
 
 struct CutceHeader {
@@ -56,30 +53,43 @@ CT_DEVICE void reset_dlogits_counters(CutceHeader* header) {
 
 // Work order of the persistent GEMM kernels. A unit is a pair (a, b) of operand tile indices,
 // a < a_count, b < b_count; every unit is one 256 x 256 GEMM tile (or a run of them) that
-// reads tile a of one operand and tile b of the other. Each XCD has its own L2, so the
-// workgroups of one XCD should work at the same time on units that share operands: the
-// (a, b) grid is walked in blocks of kA x kB = 32 units (the 32 compute units of an XCD: 4 + 8
-// operand tiles feed 32 GEMM tiles), the sequence of blocks is cut into 8 equal ranges, and an
-// XCD takes the units of its range through its own counter. Indices that fall outside the
-// grid (ragged edges) are skipped. An XCD that runs dry helps the next one.
+// reads tile a of one operand and tile b of the other. A workgroup asks for its next unit when the
+// GEMM of the last one is done (request), so that the counter's answer travels behind the epilogue.
 //
-// Sweep mode (the two projection kernels, a = vocabulary chunk, b = row block): XCD x owns the
+// Plain order, up to kPlainRounds units per workgroup: the grid is walked with a as the slow index, the
+// first unit of a workgroup is its own number, the others come from one counter. Within a round
+// every XCD gets 32 consecutive units, which share operands. (Short problems have no use for the orders
+// below: counters of XCDs that own nothing, indices that fall outside ragged grids and rounds of
+// asking the other XCDs cost 10-20 us a launch.)
+//
+// Each XCD has its own L2, so in large problems the workgroups of one XCD should work at the same time
+// on units that share operands. Blocks: the (a, b) grid is walked in blocks of kA x kB = 32 units (the
+// 32 compute units of an XCD: 4 + 8 operand tiles feed 32 GEMM tiles), the sequence of blocks is cut
+// into 8 equal ranges, and an XCD takes the units of its range through its own counter. Indices that
+// fall outside the grid (ragged edges) are skipped. An XCD that runs dry helps the next one.
+//
+// Sweep (the two projection kernels, a = vocabulary chunk, b = row block): XCD x owns the
 // row blocks x, x + 8, ... and walks (a, its row blocks) with a as the slow index, so all eight
 // XCDs are on the same few vocabulary chunks at the same time. The head is the large operand
 // (1 GB against 0.1 GB of hidden rows): with every XCD on the same chunk it leaves HBM about once
 // per pass, and the other XCDs find it in the memory-side cache; in block mode each XCD streams
 // its own range of the vocabulary and the head is read from HBM once per 8 row blocks.
-struct XcdUnits {
+constexpr int kPlainRounds = 8;
+struct UnitQueue {
   static constexpr int kA = 4, kB = 8, kXcds = 8;
+  enum Order { kPlain, kBlocks, kSweep };
   int* counters;
-  int a_count, b_count, b_groups, padded_total, per_xcd, my_xcd;
+  int a_count, b_count, total, b_groups, padded_total, per_xcd, my_xcd;
   int helping;  // how many XCDs further the counter in use belongs to
-  bool sweep;
-  CT_DEVICE void init(int* counters_, int a_count_, int b_count_, bool sweep_ = false) {
-    sweep = sweep_;
+  Order order;
+  bool requested, started;
+  int pending;  // of thread 0: the counter's answer
+  CT_DEVICE void init(int* counters_, int a_count_, int b_count_, Order large) {
     counters = counters_;
     a_count = a_count_;
     b_count = b_count_;
+    total = a_count * b_count;
+    order = total <= kPlainRounds * (int)gridDim.x ? kPlain : large;
     b_groups = (b_count + kB - 1) / kB;
     padded_total = ((a_count + kA - 1) / kA) * b_groups * kA * kB;
     per_xcd = (padded_total + kXcds - 1) / kXcds;
@@ -87,47 +97,62 @@ struct XcdUnits {
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id));
     my_xcd = (int)(xcc_id & 7u);
     helping = 0;
+    requested = started = false;
+  }
+  CT_DEVICE void request() {
+    if (threadIdx.x == 0) pending = atomicAdd(counters + (order == kPlain ? 0 : (my_xcd + helping) % kXcds), 1);
+    requested = true;
+  }
+  // The answer, for all threads of the workgroup (contains barriers).
+  CT_DEVICE int receive(int* lds_slot) {
+    if (!requested) request();
+    requested = false;
+    if (threadIdx.x == 0) *lds_slot = pending;
+    __syncthreads();
+    const int answer = uniform(*lds_slot);  // scalar from here on: unit indices feed scalar address arithmetic
+    __syncthreads();
+    return answer;
+  }
+  CT_DEVICE int next_plain(int* lds_slot) {
+    const int n = gridDim.x;
+    const int i = started ? n + receive(lds_slot) : (int)blockIdx.x;
+    started = true;
+    const int round = i / n * n;
+    if (round + n > total || n % kXcds) return i;
+    return round + (i - round) % kXcds * (n / kXcds) + (i - round) / kXcds;
   }
   // Called by all threads of the workgroup (contains barriers); false when nothing is left.
-  CT_DEVICE bool next_sweep(int& a, int& b, int* lds_slot) {
+  CT_DEVICE bool next(int& a, int& b, int* lds_slot) {
+    if (order == kPlain) {
+      const int i = next_plain(lds_slot);
+      a = i / b_count;
+      b = i % b_count;
+      return i < total;
+    }
     while (helping < kXcds) {
       const int x = (my_xcd + helping) % kXcds;
-      const int mine = x < b_count ? (b_count - x + kXcds - 1) / kXcds : 0;  // row blocks of XCD x
-      if (threadIdx.x == 0) *lds_slot = mine ? atomicAdd(&counters[x], 1) : 0;
-      __syncthreads();
-      const int local = uniform(*lds_slot);  // scalar from here on: unit indices feed scalar address arithmetic
-      __syncthreads();
-      if (mine && local < a_count * mine) {
-        a = local / mine;
-        b = x + kXcds * (local % mine);
-        return true;
+      if (order == kSweep) {
+        const int mine = x < b_count ? (b_count - x + kXcds - 1) / kXcds : 0;  // row blocks of XCD x
+        const int local = receive(lds_slot);
+        if (local < a_count * mine) {
+          a = local / mine;
+          b = x + kXcds * (local % mine);
+          return true;
+        }
+      } else {
+        const int local = receive(lds_slot);
+        const int index = x * per_xcd + local;
+        if (local < per_xcd && index < padded_total) {
+          const int in_block = index % (kA * kB), block = index / (kA * kB);
+          a = (block / b_groups) * kA + in_block / kB;
+          b = (block % b_groups) * kB + in_block % kB;
+          if (a < a_count && b < b_count) return true;
+          continue;
+        }
       }
       ++helping;
     }
     return false;
-  }
-  CT_DEVICE bool next(int& a, int& b, int* lds_slot) {
-    if (sweep) return next_sweep(a, b, lds_slot);
-    for (;;) {
-      int index = -1;
-      while (helping < kXcds) {
-        const int x = (my_xcd + helping) % kXcds;
-        if (threadIdx.x == 0) *lds_slot = atomicAdd(&counters[x], 1);
-        __syncthreads();
-        const int local = uniform(*lds_slot);  // scalar from here on: unit indices feed scalar address arithmetic
-        __syncthreads();
-        if (local < per_xcd && x * per_xcd + local < padded_total) {
-          index = x * per_xcd + local;
-          break;
-        }
-        ++helping;
-      }
-      if (index < 0) return false;
-      const int in_block = index % (kA * kB), block = index / (kA * kB);
-      a = (block / b_groups) * kA + in_block / kB;
-      b = (block % b_groups) * kB + in_block % kB;
-      if (a < a_count && b < b_count) return true;
-    }
   }
 };
 
@@ -135,11 +160,14 @@ struct XcdUnits {
 // caller's tensor (ld = V) or, where its rows are not 16-byte aligned (V % 8 != 0), an aligned copy
 // of the columns col0 .. in the workspace ("panel", cutce_panel_kernel), padded with zero columns to
 // whole tiles.
+// An aligned head whose vocabulary is no multiple of 128 has the columns from the last such multiple
+// on a second time in `tail` [d][128], padded with zeros, for the contraction over the vocabulary.
 struct HeadView {
   const bf16* base;
+  const bf16* tail;
   long ld;
   int col0;
-  bool aligned, padded;
+  bool padded;
 };
 
 struct CutceParams {
@@ -148,11 +176,15 @@ struct CutceParams {
   const int* targets;
   const float* weights;
   int N, d, V, n_pad;
-  int* idx;
+  int compact;
+  int* idx;            // [n_pad] row of each slot
+  int* slot_target;    // [n_pad] forward: target of each slot, -1 for a row without weight
+  int* block_active;   // [n_pad / 256] forward: whether a block of slots has a row with weight
   CutceHeader* header;
   bool hidden_aligned;
 
   // columns of the head that a tile at v0 may read, relative to the view
+  CT_DEVICE const int* gather() const { return compact ? idx : nullptr; }  // (slots are rows otherwise)
   CT_DEVICE int head_cols(int v0) const { return head.padded ? v0 - head.col0 + kGemmTile : V - head.col0; }
 };
 
@@ -170,8 +202,8 @@ struct CutceRowParams {
 // by itself (N floats, from L2 for all but the first reader), so no workgroup waits for another: one
 // pass of latency instead of one per 1024 rows (27 -> 5 us at N = 16384).
 template <bool BACKWARD>
-__global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, int compact, const float* lse,
-                                                           const float* dy, CutceRowParams rp) {
+__global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, const float* lse, const float* dy,
+                                                           CutceRowParams rp) {
   __shared__ int wave_total[16], wave_first[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int begin = blockIdx.x * 1024, i = begin + tid;
@@ -184,7 +216,7 @@ __global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, int co
   const bool active = w != 0.f;
   int slot = i, total = p.N, filler = 0;
   bool placed = i < p.N;
-  if (compact) {
+  if (p.compact) {
     int count = 0, first = p.N;  // active rows of this wavefront's share in front of `begin`
     for (int base = 0; base < begin; base += 1024) {
       const unsigned long long ballot = __ballot(p.weights[base + tid] != 0.f);
@@ -216,8 +248,17 @@ __global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, int co
     slot = before + __popcll(ballot & ((1ull << lane) - 1ull));
     placed = active;
   }
+  if constexpr (!BACKWARD) {
+    const unsigned long long ballot = __ballot(active);
+    __syncthreads();
+    if (lane == 0) wave_first[wave] = ballot != 0;
+    __syncthreads();
+    const int* any = wave_first + (wave & ~3);
+    if (lane == 0 && (wave & 3) == 0 && i < p.n_pad) p.block_active[i / kGemmTile] = p.compact || any[0] || any[1] || any[2] || any[3];
+  }
   if (placed) {
     p.idx[slot] = i;
+    if constexpr (!BACKWARD) p.slot_target[slot] = active ? p.targets[i] : -1;
     if constexpr (BACKWARD) {
       rp.fac[slot] = active ? w * dy[0] : 0.f;
       rp.lse2[slot] = active ? lse[i] * kLog2e : __builtin_inff();
@@ -227,6 +268,7 @@ __global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, int co
   if (!last) return;
   for (int k = total + tid; k < p.n_pad; k += 1024) {
     p.idx[k] = filler;
+    if constexpr (!BACKWARD) p.slot_target[k] = -1;
     if constexpr (BACKWARD) {
       rp.fac[k] = 0.f;
       rp.lse2[k] = __builtin_inff();
@@ -280,7 +322,7 @@ CT_DEVICE void merge_stats(float& m, float& s, float m_o, float s_o) {
   m = m_new;
 }
 
-template <bool CACHE>
+template <bool CACHE, bool GUARDED>
 __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
                                                           int tiles_per_chunk, float* cache) {
   extern __shared__ __align__(16) char smem_raw[];
@@ -293,24 +335,17 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
 
   // units: (vocabulary chunk, row block)
   const int active_blocks = (n_act + kGemmTile - 1) / kGemmTile;
-  XcdUnits units;
-  units.init(p.header->xcd_counter[0], chunks, active_blocks, kSweepUnits);
+  UnitQueue units;
+  units.init(p.header->xcd_counter[0], chunks, active_blocks, UnitQueue::kSweep);
   int chunk, rb;
   while (units.next(chunk, rb, &unit_s)) {
     chunk += chunk0;
     const int n0 = rb * kGemmTile;
-    const int my_slot = n0 + tid;
-    const int active = my_slot < n_act && p.weights[p.idx[my_slot]] != 0.f;
-    if (!__syncthreads_or(active)) continue;  // no row of this block carries weight
+    if (!p.block_active[rb]) continue;  // no row of this block carries weight
 
     // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
     // n0 + wn + 4 j + nb, so a lane owns 4 consecutive slots.
-    int tgt[4];
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int slot = n0 + wn + 4 * j + nb;
-      tgt[nb] = slot < n_act ? p.targets[p.idx[slot]] : -1;
-    }
+    const i32x4 tgt = *reinterpret_cast<const i32x4*>(p.slot_target + n0 + wn + 4 * j);
     float m2[4], sum[4], tl[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
@@ -319,16 +354,17 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
       tl[nb] = 0.f;
     }
     KcLoader B;
-    B.init(p.hidden, p.d, p.idx, n0, n_act, p.d, p.hidden_aligned, true, true);
+    B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
 
     const int vt_end = min((chunk + 1) * tiles_per_chunk, vocab_tiles);
     for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = vt * kGemmTile;
       McLoader A;
-      A.init(p.head.base, p.head.ld, nullptr, v0 - p.head.col0, p.head_cols(v0), p.d, p.head.aligned, true);
+      A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
       GemmAcc acc;
       acc.clear();
-      gemm_tile(A, B, 0, p.d, smem, acc);
+      gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
+      if (vt + 1 == vt_end) units.request();
 
       const int vbase = v0 + wm + 4 * half;  // vocab id of (i, r) = vbase + 32 i + 8 (r/4) + r%4
       const bool ragged = v0 + kGemmTile > p.V;
@@ -507,8 +543,15 @@ __global__ __launch_bounds__(64) void cutce_finalize_kernel(const double* block_
 // 256-slot block. The head gradient contracts over slots; with the rows packed its operand tiles
 // are plain strided copies instead of a gather through idx at every step. (idx repeats the first
 // active row past n_act, so the padding rows hold finite values; their G^T entries are zero.)
-__global__ __launch_bounds__(256) void cutce_rows_kernel(CutceParams p, bf16* packed, bf16* dhidden) {
+// (tail != nullptr) Also row n < d of HeadView::tail.
+__global__ __launch_bounds__(256) void cutce_rows_kernel(CutceParams p, bf16* packed, bf16* dhidden, bf16* tail) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (tail && row < p.d && lane < 16) {
+    const int v = p.V / 128 * 128 + lane * 8;
+    u32x4 chunk = {0u, 0u, 0u, 0u};
+    if (v < p.V) chunk = load_global16(p.head.base + (size_t)row * p.V + v);
+    store_global16(tail + (size_t)row * 128 + lane * 8, chunk);
+  }
   if (row < p.N && p.weights[row] == 0.f) {
     u32x4* dst = reinterpret_cast<u32x4*>(dhidden + (size_t)row * p.d);
     for (int c = lane; c < p.d / 8; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
@@ -532,6 +575,7 @@ CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
 // G^T[v - slab0][slot], logits recomputed (transposed tile as in the statistics kernel: rows =
 // vocabulary, lanes = row slots). Persistent like the statistics kernel and with its unit order:
 // a unit is tiles_per_chunk vocabulary tiles of the slab times one block of 256 active rows.
+template <bool GUARDED>
 __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
                                                             int slab0, int slab_tiles, int tiles_per_chunk,
                                                             bf16* G) {
@@ -545,8 +589,8 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
   if (blockIdx.x == 0) reset_unit_counters(p.header);
   const int active_blocks = (n_act + kGemmTile - 1) / kGemmTile;  // G^T columns past them are never read
   const int chunks = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk;
-  XcdUnits units;
-  units.init(p.header->xcd_counter[2], chunks, active_blocks, kSweepUnits);
+  UnitQueue units;
+  units.init(p.header->xcd_counter[2], chunks, active_blocks, UnitQueue::kSweep);
   int chunk, rb;
   while (units.next(chunk, rb, &unit_s)) {
     const int n0 = rb * kGemmTile;
@@ -557,15 +601,16 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
     const f32x4 lse2 = *reinterpret_cast<const f32x4*>(rp.lse2 + slot4);
     const i32x4 tgt = *reinterpret_cast<const i32x4*>(rp.tgt + slot4);
     KcLoader B;
-    B.init(p.hidden, p.d, p.idx, n0, n_act, p.d, p.hidden_aligned, true, true);
+    B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
     const int vt_end = min((chunk + 1) * tiles_per_chunk, slab_tiles);
     for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = slab0 + vt * kGemmTile;
       McLoader A;
-      A.init(p.head.base, p.head.ld, nullptr, v0 - p.head.col0, p.head_cols(v0), p.d, p.head.aligned, true);
+      A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
       GemmAcc acc;
       acc.clear();
-      gemm_tile(A, B, 0, p.d, smem, acc);
+      gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
+      if (vt + 1 == vt_end) units.request();
 
       bf16* origin = G + (size_t)(v0 - slab0 + uniform(wm)) * p.n_pad + n0 + uniform(wn);
       const unsigned lane_off = (unsigned)(4 * half * p.n_pad + 4 * j) * 2u;  // bytes
@@ -690,84 +735,81 @@ CT_DEVICE int head_parts(const CutceSplits& sp, int n_act, int d) {
 // First of the 128-term groups of part `split`.
 CT_DEVICE int split_begin(int groups, int split, int splits) { return (int)((long)groups * split / splits); }
 
-// dHidden[idx[slot], n] (+)= sum_v G^T[v, slot] head[n, slab0 + v]: the workgroup's share of the
-// units, pulled from counter set 0.
-CT_DEVICE void dhidden_units(const CutceParams& p, const bf16* G, int slab0, int slab_width, int mode,
-                             float* dh_acc, bf16* dhidden, const CutceSplits& sp, const lds_addr smem) {
-  // mode: 0 = single slab (store bf16), 1 = first slab (store f32), 2 = middle
-  // slab (add f32), 3 = last slab (add, store bf16)
+// One slab of the vocabulary, as the gradient kernels see it.
+struct CutceSlab {
+  const bf16* G;       // G^T [width][n_pad]
+  const bf16* packed;  // [n_pad][d]
+  int first, width;    // vocabulary ids first .. first + width - 1, width a multiple of 256
+  int mode;            // 0 = single slab (store bf16), 1 = first slab (store f32), 2 = middle
+                       // slab (add f32), 3 = last slab (add, store bf16)
+  float* dh_acc;
+  bf16* dhidden;
+  bf16* dhead;
+};
+
+// dHidden[idx[slot], n] (+)= sum_v G^T[v, slot] head[n, first + v] of row block rb, column block cb and
+// part `split` of the contraction.
+template <bool GUARDED>
+CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int rb, int cb, int split,
+                            int parts, int n_act, UnitQueue& units, const lds_addr smem) {
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
-  const int col_blocks = (p.d + kGemmTile - 1) / kGemmTile;
-  const int n_act = p.header->n_act;
-  __shared__ int unit_s;
-  // the dlogits kernel of the next vocabulary slab starts from fresh work counters
-  if (blockIdx.x == 0) reset_dlogits_counters(p.header);
   // Terms of the contraction: the whole slab where the head is padded, else up to the end of the
-  // vocabulary; the last k_width % 128 of them apart, since nothing past a row's end may be read.
-  const int k_width = p.head.padded ? slab_width : min(slab_width, p.V - slab0);
+  // vocabulary; the last k_width % 128 of them from the tail, since nothing past a row's end may be
+  // read (G^T is zero from the vocabulary's end to the end of the slab).
+  const int k_width = p.head.padded ? sl.width : min(sl.width, p.V - sl.first);
   const int groups = k_width / 128;
-  const int parts = hidden_parts(sp, n_act, p.d, slab_width / kGemmTile);
-  const size_t part_rows = (size_t)((n_act + kGemmTile - 1) / kGemmTile) * kGemmTile;
-  // units: (row block, (split, column block)) over the started row blocks
-  XcdUnits units;
-  units.init(p.header->xcd_counter[0], (n_act + kGemmTile - 1) / kGemmTile, col_blocks * parts);
-  int rb, cbs;
-  while (units.next(rb, cbs, &unit_s)) {
-    const int split = cbs / col_blocks, cb = cbs % col_blocks;
-    const int n0 = rb * kGemmTile, c0 = cb * kGemmTile;
-    const int k_begin = split_begin(groups, split, parts) * 128;
-    const int k_mid = split_begin(groups, split + 1, parts) * 128;
-    // (G^T is zero from the vocabulary's end to the end of the slab)
-    const int k_end = split == parts - 1 && k_mid < k_width ? min(k_mid + 128, slab_width) : k_mid;
-    McLoader A;
-    A.init(G, p.n_pad, nullptr, n0, p.n_pad, slab_width, true);
-    // (rows of B interleaved: lane j owns the 4 consecutive columns c0 + wn + 4 j + nb; rows past d
-    // are copies of the first, their columns are not stored)
+  const int n0 = rb * kGemmTile, c0 = cb * kGemmTile;
+  const int k_begin = split_begin(groups, split, parts) * 128, k_mid = split_begin(groups, split + 1, parts) * 128;
+  const bool with_tail = split == parts - 1 && k_mid < k_width;
+  McLoader A;
+  A.init(sl.G, p.n_pad, n0, p.n_pad, sl.width);
+  GemmAcc acc;
+  acc.clear();
+  // (rows of B interleaved: lane j owns the 4 consecutive columns c0 + wn + 4 j + nb; rows past d
+  // are copies of the first, their columns are not stored)
+  const bf16* head = p.head.base + (sl.first - p.head.col0);
+  if constexpr (GUARDED) {
     KcLoader B;
-    B.init(p.head.base + (slab0 - p.head.col0), p.head.ld, nullptr, c0, p.d, k_mid, p.head.aligned, true, true);
-    GemmAcc acc;
-    acc.clear();
-    for (int part = 0; part < 2; ++part) {
-      if (part == 1) {
-        if (k_mid == k_end) break;
-        B.alias_invalid_k(k_width);
-        if (!B.fast) B.alias_k = false;  // the guarded loop zero fills by itself
-      }
-      gemm_tile(A, B, part ? k_mid : k_begin, part ? k_end : k_mid, smem, acc);
+    B.init(head, p.head.ld, nullptr, c0, p.d, k_width, true);
+    gemm_tile<true>(A, B, k_begin, with_tail ? k_width : k_mid, smem, acc);
+  } else {
+#pragma nounroll
+    for (int part = 0; part <= (int)with_tail; ++part) {
+      KcLoader B;
+      B.init(part ? p.head.tail - k_mid : head, part ? 128 : p.head.ld, nullptr, c0, p.d, k_width, true);
+      gemm_tile<false>(A, B, part ? k_mid : k_begin, part ? k_mid + 128 : k_mid, smem, acc);
     }
-
-    const int col = c0 + wn + 4 * j;  // hidden sizes are multiples of 128: col < d implies col + 3 < d
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int slot = n0 + wm + 32 * i + acc_row(r, half);
-        if (slot >= n_act || col >= p.d) continue;
-        f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
-        if (parts > 1) {
-          *reinterpret_cast<f32x4*>(sp.hidden_sums + (split * part_rows + slot) * p.d + col) = val;
-          continue;
-        }
-        const long row = p.idx[slot];
-        f32x4* a = reinterpret_cast<f32x4*>(dh_acc + (size_t)slot * p.d + col);
-        if (mode >= 2) val += *a;
-        if (mode == 1 || mode == 2) *a = val;
-        if (mode == 0 || mode == 3) {
-          bf16x4 out;
-#pragma unroll
-          for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-          *reinterpret_cast<bf16x4*>(dhidden + row * p.d + col) = out;
-        }
-      }
   }
-}
+  units.request();
 
-__global__ __launch_bounds__(256) void cutce_dhidden_kernel(CutceParams p, const bf16* G,
-                                                            int slab0, int slab_width, int mode,
-                                                            float* dh_acc, bf16* dhidden, CutceSplits sp) {
-  extern __shared__ __align__(16) char smem_raw[];
-  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, sp, lds_address_of(smem_raw));
+  const int col = c0 + wn + 4 * j;  // hidden sizes are multiples of 128: col < d implies col + 3 < d
+  // f32 to the partial sums or to the sum over slabs (adding what is there from the second slab on),
+  // bf16 to dHidden from the only or the last slab. (The flags are made opaque at every element: one copy
+  // of the 64 stores that branches, instead of a copy for every combination.)
+  float* f32_out = parts > 1 ? sp.hidden_sums + (size_t)split * ((n_act + kGemmTile - 1) / kGemmTile * kGemmTile) * p.d
+                             : sl.dh_acc;
+  const int flags_all = uniform(parts > 1 ? 1 : (sl.mode == 1 || sl.mode == 2 ? 1 : 0) | (sl.mode >= 2 ? 2 : 0));
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int slot = n0 + wm + 32 * i + acc_row(r, half);
+      if (slot >= n_act || col >= p.d) continue;
+      f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
+      int flags = flags_all;
+      asm volatile("" : "+s"(flags));
+      f32x4* a = reinterpret_cast<f32x4*>(f32_out + (size_t)slot * p.d + col);
+      if (flags & 2) val += *a;
+      if (flags & 1) {
+        *a = val;
+      } else {
+        bf16x4 out;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
+        *reinterpret_cast<bf16x4*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col) = out;
+      }
+    }
 }
 
 // Four consecutive columns of a row of dHead; the rows of an odd vocabulary start at any multiple
@@ -785,76 +827,98 @@ CT_DEVICE void store_dhead4(bf16* dst, int left, f32x4 val) {
   }
 }
 
-// dHead[m, slab0 + v] = sum_slot packed[slot, m] G^T[v, slot], packed[slot] = hidden[idx[slot]]:
-// the workgroup's share of the units, pulled from counter set 1.
-CT_DEVICE void dhead_units(const CutceParams& p, const bf16* packed, const bf16* G, int slab0,
-                           int slab_tiles, bf16* dhead, const CutceSplits& sp, const lds_addr smem) {
+// dHead[m, first + v] = sum_slot packed[slot, m] G^T[v, slot], packed[slot] = hidden[idx[slot]], of
+// vocabulary tile vt, hidden column block mb and part `split` of the contraction.
+template <bool GUARDED>
+CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int vt, int mb, int split,
+                          int parts, int n_act, UnitQueue& units, const lds_addr smem) {
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
-  const int m_blocks = (p.d + kGemmTile - 1) / kGemmTile;
-  const int n_act = p.header->n_act;
   // 4 contraction steps at a time; slots n_act .. k_end-1 are valid memory: G^T holds zeros
   // there (the dlogits kernels write whole 256-slot blocks) and the packed rows are finite.
   const int groups = min(p.n_pad, (n_act + 4 * kBK - 1) / (4 * kBK) * (4 * kBK)) / (4 * kBK);
-  const int slab_width = slab_tiles * kGemmTile;
-  __shared__ int unit_s;
-  // units: (vocabulary tile of the slab, (split, hidden column block))
-  XcdUnits units;
-  const int parts = head_parts(sp, n_act, p.d);
-  units.init(p.header->xcd_counter[1], slab_tiles, m_blocks * parts);
-  int vt, mbs;
-  while (units.next(vt, mbs, &unit_s)) {
-    const int split = mbs / m_blocks, mb = mbs % m_blocks;
-    const int m0 = mb * kGemmTile, v0 = vt * kGemmTile;  // v0 relative to the slab
-    const int k_begin = split_begin(groups, split, parts) * 128, k_end = split_begin(groups, split + 1, parts) * 128;
-    McLoader A;  // (columns past d are copies, their rows of dHead are not stored)
-    A.init(packed, p.d, nullptr, m0, p.d, k_end, true, true);
-    // (rows of B interleaved: lane j owns the 4 consecutive vocabulary ids v .. v + 3)
-    KcLoader B;
-    B.init(G, p.n_pad, nullptr, v0, slab_width, k_end, true, false, true);
-    GemmAcc acc;
-    acc.clear();
-    gemm_tile(A, B, k_begin, k_end, smem, acc);
+  const int m0 = mb * kGemmTile, v0 = vt * kGemmTile;  // v0 relative to the slab
+  const int k_begin = split_begin(groups, split, parts) * 128, k_end = split_begin(groups, split + 1, parts) * 128;
+  McLoader A;  // (columns past d are copies, their rows of dHead are not stored)
+  A.init(sl.packed, p.d, m0, p.d, k_end);
+  // (rows of B interleaved: lane j owns the 4 consecutive vocabulary ids v .. v + 3)
+  KcLoader B;
+  B.init(sl.G, p.n_pad, nullptr, v0, sl.width, k_end, true);
+  GemmAcc acc;
+  acc.clear();
+  gemm_tile<GUARDED>(A, B, k_begin, k_end, smem, acc);
+  units.request();
 
-    const int v = slab0 + v0 + wn + 4 * j;
+  const int v = sl.first + v0 + wn + 4 * j;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm + 32 * i + acc_row(r, half);
-        if (m >= p.d) continue;
-        const f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
-        if (parts > 1)
-          *reinterpret_cast<f32x4*>(sp.head_sums + ((size_t)split * p.d + m) * slab_width + (v - slab0)) = val;
-        else
-          store_dhead4(dhead + (size_t)m * p.V + v, p.V - v, val);
-      }
-  }
+    for (int r = 0; r < 16; ++r) {
+      const int m = m0 + wm + 32 * i + acc_row(r, half);
+      if (m >= p.d) continue;
+      const f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
+      int to_sums = uniform(parts > 1);
+      asm volatile("" : "+s"(to_sums));
+      if (to_sums)
+        *reinterpret_cast<f32x4*>(sp.head_sums + ((size_t)split * p.d + m) * sl.width + (v - sl.first)) = val;
+      else
+        store_dhead4(sl.dhead + (size_t)m * p.V + v, p.V - v, val);
+    }
 }
 
-// Both gradients of a slab in one launch. The hidden gradient has few, long units (45 x 16 at
-// N = 16384, d = 4096: 2.8 per compute unit, so its last round leaves a sixth of the device idle);
-// a workgroup that finds no hidden-gradient unit left goes on to the head-gradient units, which
-// are many and short, and the idle tail of the first fills with work of the second. The two
-// read the same G^T and write different tensors: neither waits for the other.
-__global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, const bf16* packed,
-                                                         const bf16* G, int slab0, int slab_width,
-                                                         int slab_tiles, int mode, float* dh_acc,
-                                                         bf16* dhidden, bf16* dhead, CutceSplits sp) {
+// Both gradients of a slab in one launch (HEAD = false: the head is frozen). The hidden gradient has few,
+// long units (45 x 16 at N = 16384, d = 4096: 2.8 per compute unit, so its last round leaves a sixth of the
+// device idle); a workgroup that finds no hidden-gradient unit left goes on to the head-gradient
+// units, which are many and short, and the idle tail of the first fills with work of the second. The
+// two read the same G^T and write different tensors: neither waits for the other.
+template <bool HEAD, bool GUARDED>
+__global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
-  dhidden_units(p, G, slab0, slab_width, mode, dh_acc, dhidden, sp, smem);
-  dhead_units(p, packed, G, slab0, slab_tiles, dhead, sp, smem);
+  __shared__ int unit_s;
+  const int n_act = p.header->n_act;
+  // the dlogits kernel of the next vocabulary slab starts from fresh work counters
+  if (blockIdx.x == 0) reset_dlogits_counters(p.header);
+  const int col_blocks = (p.d + kGemmTile - 1) / kGemmTile, slab_tiles = sl.width / kGemmTile;
+  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+  const int parts_h = hidden_parts(sp, n_act, p.d, slab_tiles);
+  const int parts_w = HEAD ? head_parts(sp, n_act, p.d) : 1;
+  const int total_h = row_blocks * col_blocks * parts_h, total_w = HEAD ? slab_tiles * col_blocks * parts_w : 0;
+  // Short problems walk one list, the longer units first; large ones the hidden gradient's grid (row
+  // block, (part, column block)) and then the head gradient's (vocabulary tile, (part, column block)).
+  const bool one_list = total_h + total_w <= kPlainRounds * (int)gridDim.x;
+  UnitQueue units;
+  bool in_head = false;
+  if (one_list) units.init(p.header->xcd_counter[0], total_h + total_w, 1, UnitQueue::kPlain);
+  else units.init(p.header->xcd_counter[0], row_blocks, col_blocks * parts_h, UnitQueue::kBlocks);
+  for (;;) {
+    int a, b;
+    if (!units.next(a, b, &unit_s)) {
+      if (one_list || in_head || !HEAD) break;
+      in_head = true;
+      units.init(p.header->xcd_counter[1], slab_tiles, col_blocks * parts_w, UnitQueue::kBlocks);
+      continue;
+    }
+    if (one_list) {
+      in_head = a >= total_h;
+      const int index = in_head ? a - total_h : a, width = col_blocks * (in_head ? parts_w : parts_h);
+      a = index / width;
+      b = index % width;
+    }
+    if (!in_head) {
+      dhidden_unit<GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
+    } else if constexpr (HEAD) {
+      dhead_unit<GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_w, n_act, units, smem);
+    }
+  }
 }
 
 // Adds the partial sums of cut tiles, a thread 4 columns of a row at a time: first those of dHidden's
 // active rows, then those of the slab's part of dHead. Nothing to do for a gradient that was not cut.
-__global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, int slab0, int slab_width, int mode,
-                                                           float* dh_acc, bf16* dhidden, bf16* dhead,
-                                                           CutceSplits sp) {
+__global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
   const int n_act = p.header->n_act;
   const long first = (long)blockIdx.x * 256 + threadIdx.x, stride = (long)gridDim.x * 256;
-  const int parts_h = hidden_parts(sp, n_act, p.d, slab_width / kGemmTile);
+  const int parts_h = hidden_parts(sp, n_act, p.d, sl.width / kGemmTile);
   if (parts_h > 1) {
     const int quads = p.d / 4;
     const size_t part_size = (size_t)((n_act + kGemmTile - 1) / kGemmTile) * kGemmTile * p.d;
@@ -864,30 +928,30 @@ __global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, int sl
       f32x4 val = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll 4
       for (int s = 1; s < parts_h; ++s) val += *reinterpret_cast<const f32x4*>(src + s * part_size);
-      f32x4* a = reinterpret_cast<f32x4*>(dh_acc + (size_t)slot * p.d + col);
-      if (mode >= 2) val += *a;
-      if (mode == 1 || mode == 2) {
+      f32x4* a = reinterpret_cast<f32x4*>(sl.dh_acc + (size_t)slot * p.d + col);
+      if (sl.mode >= 2) val += *a;
+      if (sl.mode == 1 || sl.mode == 2) {
         *a = val;
       } else {
         bf16x4 out;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-        *reinterpret_cast<bf16x4*>(dhidden + (size_t)p.idx[slot] * p.d + col) = out;
+        *reinterpret_cast<bf16x4*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col) = out;
       }
     }
   }
   if (!sp.with_head) return;
   const int parts_w = head_parts(sp, n_act, p.d);
   if (parts_w <= 1) return;
-  const int width = min(slab_width, (p.V - slab0 + 3) & ~3);
+  const int width = min(sl.width, (p.V - sl.first + 3) & ~3);
   const int quads = width / 4;
   for (long index = first; index < (long)p.d * quads; index += stride) {
     const int m = (int)(index / quads), v = (int)(index % quads) * 4;
-    const float* src = sp.head_sums + (size_t)m * slab_width + v;
+    const float* src = sp.head_sums + (size_t)m * sl.width + v;
     f32x4 val = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll 4
-    for (int s = 1; s < parts_w; ++s) val += *reinterpret_cast<const f32x4*>(src + (size_t)s * p.d * slab_width);
-    store_dhead4(dhead + (size_t)m * p.V + slab0 + v, p.V - slab0 - v, val);
+    for (int s = 1; s < parts_w; ++s) val += *reinterpret_cast<const f32x4*>(src + (size_t)s * p.d * sl.width);
+    store_dhead4(sl.dhead + (size_t)m * p.V + sl.first + v, p.V - sl.first - v, val);
   }
 }
 
@@ -900,13 +964,11 @@ static int padded_rows(int N) { return (int)align_up((size_t)N, kGemmTile); }
 static int vocab_tile_count(int V) { return (V + kGemmTile - 1) / kGemmTile; }
 
 // Vocabulary tiles per work unit of the two projection kernels. Four keep a unit's hidden rows in use
-// for four tiles and leave a quarter of the partial statistics; with fewer than two units per compute
-// unit that costs more than it gives (the last round, or the only one, is longer), so short problems
-// take units of two tiles or one.
+// for four tiles and leave a quarter of the partial statistics; short problems take units of two
+// tiles or one, which end together (263 tiles x 8 row blocks in units of four are 2.06 rounds: three).
 static int tiles_per_chunk(int tiles, int row_blocks) {
-  for (int t = 4; t > 1; t /= 2)
-    if ((long)((tiles + t - 1) / t) * row_blocks >= 2 * kComputeUnits) return t;
-  return 1;
+  const long units = (long)tiles * row_blocks;
+  return units <= kPlainRounds * kComputeUnits ? 1 : units <= 2 * kPlainRounds * kComputeUnits ? 2 : 4;
 }
 static int stats_chunks(const ct_cutce_shape& s) {
   const int tiles = vocab_tile_count(s.vocab);
@@ -924,14 +986,16 @@ static size_t full_panel_bytes(const ct_cutce_shape& s) {
 
 // Workspace of the forward: `base` bytes it cannot do without, then as much of the panel as fits.
 struct FwdLayout {
-  size_t header, idx, part, sums, base, total;
+  size_t header, idx, target, active, part, sums, base, total;
 };
 static FwdLayout fwd_layout(const ct_cutce_shape& s) {
   const int n_pad = padded_rows(s.rows);
   FwdLayout L;
   L.header = 0;
   L.idx = align_up(sizeof(CutceHeader), 256);
-  L.part = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
+  L.target = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
+  L.active = L.target + align_up((size_t)n_pad * sizeof(int), 256);
+  L.part = L.active + align_up((size_t)(n_pad / kGemmTile) * sizeof(int), 256);
   L.sums = L.part + align_up((size_t)stats_chunks(s) * n_pad * 3 * sizeof(float), 256);
   L.base = L.sums + align_up((size_t)(n_pad / kMergeSlots) * 2 * sizeof(double), 256);
   L.total = L.base + full_panel_bytes(s);
@@ -952,16 +1016,16 @@ static int most_head_parts(const ct_cutce_shape& s) {
 }
 
 struct BwdLayout {
-  size_t header, idx, rowparams, packed, panel, g, head_sums, acc, hidden_sums, total;
+  size_t header, idx, rowparams, packed, tail, panel, g, head_sums, acc, hidden_sums, total;
   size_t hidden_sums_bytes;
   int head_most;
   int slab_cols;  // multiple of 256
   int slabs;
 };
-// header, idx, 3 row parameter arrays, packed hidden rows
+// header, idx, 3 row parameter arrays, packed hidden rows, tail of the head
 static size_t bwd_fixed_bytes(int n_pad, int d) {
   return align_up(sizeof(CutceHeader), 256) + 4 * align_up((size_t)n_pad * sizeof(int), 256) +
-         align_up((size_t)n_pad * d * sizeof(bf16), 256);
+         align_up((size_t)n_pad * d * sizeof(bf16), 256) + (size_t)d * 128 * sizeof(bf16);
 }
 // What one tile column of a slab takes: its part of G^T, without a panel in the logits cache of the
 // panel, and the partial sums of dHead if that is cut.
@@ -990,6 +1054,7 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_in
   L.rowparams = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
   L.packed = L.rowparams + 3 * align_up((size_t)n_pad * sizeof(int), 256);
   L.panel = bwd_fixed_bytes(n_pad, s.hidden);
+  L.tail = L.panel - (size_t)s.hidden * 128 * sizeof(bf16);
   const BwdTileBytes tile = bwd_tile_bytes(s, panel_in_cache, with_head);
   const size_t per_tile = tile.all(), acc_bytes = bwd_acc_bytes(s);
   size_t fit = tiles, room;
@@ -1028,19 +1093,29 @@ static int validate_cutce(const char* fn, const ct_cutce_shape& s) {
 
 static bool is_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <class K>
-static int set_smem(K kernel, size_t bytes, const char* what) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e != hipSuccess) return fail(CT_LAUNCH_FAILED, "%s: %s", what, hipGetErrorString(e));
+// The GEMM kernels need more than the default 64 KB of LDS; each says so once per device.
+template <class... Kernels>
+static int allow_gemm_lds(const char* fn, std::atomic<unsigned>& done, Kernels... kernels) {
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 32) device = -1;
+  if (device >= 0 && (done.load(std::memory_order_acquire) >> device & 1u)) return CT_OK;
+  for (const void* kernel : {reinterpret_cast<const void*>(kernels)...}) {
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GemmSmem::kBytes);
+    if (e != hipSuccess) return fail(CT_LAUNCH_FAILED, "%s: %s", fn, hipGetErrorString(e));
+  }
+  if (device >= 0) done.fetch_or(1u << device, std::memory_order_release);
   return CT_OK;
 }
 
+// Compute units of the current device, asked for once per device.
 static int device_cu_count() {
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  return cus > 0 ? cus : 256;
+  static std::atomic<int> known[32];
+  int device = 0, cus = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 32) return kComputeUnits;
+  if ((cus = known[device].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) cus = kComputeUnits;
+  known[device].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
 }  // namespace ct
@@ -1082,10 +1157,11 @@ extern "C" size_t ct_cutce_bwd_workspace_min_bytes(const ct_cutce_shape* shape) 
 }
 
 static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, const int32_t* targets,
-                               const float* weights, const ct_cutce_shape& s, char* ws) {
-  CutceParams p;
+                               const float* weights, const ct_cutce_shape& s, int compact, char* ws) {
+  CutceParams p = {};
   p.hidden = reinterpret_cast<const bf16*>(hidden);
-  p.head = HeadView{reinterpret_cast<const bf16*>(head), s.vocab, 0, is_aligned16(head) && s.vocab % 8 == 0, false};
+  p.head = HeadView{reinterpret_cast<const bf16*>(head), nullptr, s.vocab, 0, false};
+  p.compact = compact ? 1 : 0;
   p.targets = targets;
   p.weights = weights;
   p.N = s.rows;
@@ -1108,7 +1184,7 @@ static int launch_panel(hipStream_t stream, const bf16* head, const ct_cutce_sha
   return scope.done();
 }
 static HeadView panel_view(const bf16* panel, int tile0, int tiles) {
-  return HeadView{panel, (long)tiles * kGemmTile, tile0 * kGemmTile, true, true};
+  return HeadView{panel, nullptr, (long)tiles * kGemmTile, tile0 * kGemmTile, true};
 }
 
 // Shared body of ct_cutce_fwd and ct_cutce_fwd_noalloc: `ws` / `ws_bytes` is the workspace to use
@@ -1132,7 +1208,7 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   }
   hipStream_t stream = (hipStream_t)stream_;
   char* ws = static_cast<char*>(ws_);
-  CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, ws);
+  CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, a->sparse_compaction, ws);
   float* part = reinterpret_cast<float*>(ws + L.part);
   double* sums = reinterpret_cast<double*>(ws + L.sums);
   const int chunks = stats_chunks(a->shape), row_blocks = p.n_pad / kGemmTile, tiles = vocab_tile_count(p.V);
@@ -1140,8 +1216,10 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   const bf16* head = p.head.base;
 
   LaunchScope scope1("cutce_index_kernel", stream);
-  hipLaunchKernelGGL(cutce_index_kernel<false>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p,
-                     a->sparse_compaction ? 1 : 0, nullptr, nullptr, CutceRowParams{});
+  p.slot_target = reinterpret_cast<int*>(ws + L.target);
+  p.block_active = reinterpret_cast<int*>(ws + L.active);
+  hipLaunchKernelGGL(cutce_index_kernel<false>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p, nullptr, nullptr,
+                     CutceRowParams{});
   if ((rc = scope1.done())) return rc;
 
   // The panel of a head with unaligned rows: at the end of the logits cache, where the backward finds
@@ -1159,8 +1237,13 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     }
   }
   const size_t smem = GemmSmem::kBytes;
-  if ((rc = set_smem(cutce_stats_kernel<false>, smem, fn))) return rc;
-  if ((rc = set_smem(cutce_stats_kernel<true>, smem, fn))) return rc;
+  static std::atomic<unsigned> lds_allowed{0};
+  if ((rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<false, false>, cutce_stats_kernel<true, false>,
+                           cutce_stats_kernel<false, true>, cutce_stats_kernel<true, true>)))
+    return rc;
+  const bool guarded = !p.hidden_aligned || (!panel && !(is_aligned16(head) && p.V % 8 == 0));
+  const auto stats = a->logits_cache ? (guarded ? cutce_stats_kernel<true, true> : cutce_stats_kernel<true, false>)
+                                     : (guarded ? cutce_stats_kernel<false, true> : cutce_stats_kernel<false, false>);
   for (int chunk0 = 0; chunk0 < chunks; chunk0 += chunks_per_pass) {
     const int pass_chunks = min(chunks_per_pass, chunks - chunk0);
     if (panel) {
@@ -1170,12 +1253,8 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     }
     const int persistent = min(device_cu_count(), pass_chunks * row_blocks);
     LaunchScope scope2("cutce_stats_kernel", stream);
-    if (a->logits_cache)
-      hipLaunchKernelGGL(cutce_stats_kernel<true>, dim3(persistent), dim3(256), smem, stream, p, part, chunk0,
-                         pass_chunks, per_chunk, static_cast<float*>(a->logits_cache));
-    else
-      hipLaunchKernelGGL(cutce_stats_kernel<false>, dim3(persistent), dim3(256), smem, stream, p, part, chunk0,
-                         pass_chunks, per_chunk, static_cast<float*>(nullptr));
+    hipLaunchKernelGGL(stats, dim3(persistent), dim3(256), smem, stream, p, part, chunk0, pass_chunks, per_chunk,
+                       static_cast<float*>(a->logits_cache));
     if ((rc = scope2.done())) return rc;
   }
 
@@ -1259,7 +1338,7 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
                 a->workspace_bytes, ct_cutce_bwd_workspace_min_bytes(&a->shape));
   hipStream_t stream = (hipStream_t)stream_;
   char* ws = static_cast<char*>(a->workspace);
-  CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, ws);
+  CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, a->sparse_compaction, ws);
   bf16* G = reinterpret_cast<bf16*>(ws + L.g);
   float* dh_acc = L.slabs > 1 ? reinterpret_cast<float*>(ws + L.acc) : nullptr;
   bf16* dhidden = reinterpret_cast<bf16*>(a->dhidden);
@@ -1278,23 +1357,28 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   rp.lse2 = reinterpret_cast<float*>(ws + L.rowparams + params_stride);
   rp.tgt = reinterpret_cast<int*>(ws + L.rowparams + 2 * params_stride);
   const size_t smem = GemmSmem::kBytes;
-  if ((rc = set_smem(cutce_dlogits_kernel, smem, "ct_cutce_bwd"))) return rc;
-  if ((rc = set_smem(cutce_dhidden_kernel, smem, "ct_cutce_bwd"))) return rc;
-  if ((rc = set_smem(cutce_grads_kernel, smem, "ct_cutce_bwd"))) return rc;
+  static std::atomic<unsigned> lds_allowed{0};
+  if ((rc = allow_gemm_lds("ct_cutce_bwd", lds_allowed, cutce_dlogits_kernel<false>, cutce_dlogits_kernel<true>,
+                           cutce_grads_kernel<false, false>, cutce_grads_kernel<true, false>, cutce_grads_kernel<false, true>,
+                           cutce_grads_kernel<true, true>)))
+    return rc;
 
   LaunchScope scope5("cutce_index_kernel", stream);
-  hipLaunchKernelGGL(cutce_index_kernel<true>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p,
-                     a->sparse_compaction ? 1 : 0, a->lse, a->dy, rp);
+  hipLaunchKernelGGL(cutce_index_kernel<true>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p, a->lse, a->dy, rp);
   if ((rc = scope5.done())) return rc;
   bf16* packed = dhead ? reinterpret_cast<bf16*>(ws + L.packed) : nullptr;
   LaunchScope scope6("cutce_rows_kernel", stream);
-  hipLaunchKernelGGL(cutce_rows_kernel, dim3(p.n_pad / 4), dim3(256), 0, stream, p, packed, dhidden);
+  const bool head_aligned = is_aligned16(a->head) && p.V % 8 == 0;
+  bf16* tail = head_aligned && p.V % 128 ? reinterpret_cast<bf16*>(ws + L.tail) : nullptr;
+  hipLaunchKernelGGL(cutce_rows_kernel, dim3(max(p.n_pad, tail ? p.d : 0) / 4), dim3(256), 0, stream, p, packed, dhidden,
+                     tail);
   if ((rc = scope6.done())) return rc;
 
   const int cus = device_cu_count();
   const int tiles = vocab_tile_count(p.V);
   const int tiles_per_slab = L.slab_cols / kGemmTile;
   const bf16* head = p.head.base;
+  p.head.tail = tail;
   bf16* panel = nullptr;
   if (needs_panel(a->shape)) {
     if (cache) {  // the forward left it there
@@ -1303,6 +1387,11 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
       panel = reinterpret_cast<bf16*>(ws + L.panel);
     }
   }
+  // (an unaligned head with a multiple of 8 columns has no panel)
+  const bool guarded_head = !needs_panel(a->shape) && !head_aligned;
+  const bool guarded_logits = guarded_head || !p.hidden_aligned;
+  const auto grads = dhead ? (guarded_head ? cutce_grads_kernel<true, true> : cutce_grads_kernel<true, false>)
+                           : (guarded_head ? cutce_grads_kernel<false, true> : cutce_grads_kernel<false, false>);
   for (int s = 0; s < L.slabs; ++s) {
     const int slab0 = s * L.slab_cols;
     const int slab_tiles = min(tiles_per_slab, tiles - s * tiles_per_slab);
@@ -1321,11 +1410,12 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
       LaunchScope scope7("cutce_dlogits_kernel", stream);
       const int per_chunk = tiles_per_chunk(slab_tiles, row_blocks);
       const int dl_units = ((slab_tiles + per_chunk - 1) / per_chunk) * row_blocks;
-      hipLaunchKernelGGL(cutce_dlogits_kernel, dim3(min(cus, dl_units)), dim3(256), smem, stream,
-                         p, rp, slab0, slab_tiles, per_chunk, G);
+      hipLaunchKernelGGL(guarded_logits ? cutce_dlogits_kernel<true> : cutce_dlogits_kernel<false>, dim3(min(cus, dl_units)),
+                         dim3(256), smem, stream, p, rp, slab0, slab_tiles, per_chunk, G);
       if ((rc = scope7.done())) return rc;
     }
     const int mode = L.slabs == 1 ? 0 : (s == 0 ? 1 : (s == L.slabs - 1 ? 3 : 2));
+    const CutceSlab slab = {G, packed, slab0, slab_width, mode, dh_acc, dhidden, dhead};
     CutceSplits sp;
     sp.hidden_sums = reinterpret_cast<float*>(ws + L.hidden_sums);
     sp.head_sums = reinterpret_cast<float*>(ws + L.head_sums);
@@ -1333,23 +1423,14 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
     sp.head_most = L.head_most;
     sp.all_tiles = tiles;
     sp.with_head = dhead != nullptr;
-    if (dhead) {
-      // both gradients in one launch: the head-gradient units fill the hidden gradient's tail
-      LaunchScope scope8("cutce_grads_kernel", stream);
-      hipLaunchKernelGGL(cutce_grads_kernel, dim3(cus), dim3(256), smem, stream, p, packed,
-                         G, slab0, slab_width, slab_tiles, mode, dh_acc, dhidden, dhead, sp);
-      if ((rc = scope8.done())) return rc;
-    } else {
-      LaunchScope scope8("cutce_dhidden_kernel", stream);
-      hipLaunchKernelGGL(cutce_dhidden_kernel, dim3(cus), dim3(256), smem,
-                         stream, p, G, slab0, slab_width, mode, dh_acc, dhidden, sp);
-      if ((rc = scope8.done())) return rc;
-    }
+    LaunchScope scope8(dhead ? "cutce_grads_kernel" : "cutce_dhidden_kernel", stream);
+    hipLaunchKernelGGL(grads, dim3(cus), dim3(256), smem, stream, p, slab, sp);
+    if ((rc = scope8.done())) return rc;
     if (sp.hidden_room || sp.head_most > 1) {
       LaunchScope scope9("cutce_reduce_kernel", stream);
       const long quads = max((long)p.n_pad * p.d, sp.head_most > 1 ? (long)p.d * slab_width : 0) / 4;
       hipLaunchKernelGGL(cutce_reduce_kernel, dim3((unsigned)min((quads + 255) / 256, (long)cus * 8)), dim3(256), 0, stream, p,
-                         slab0, slab_width, mode, dh_acc, dhidden, dhead, sp);
+                         slab, sp);
       if ((rc = scope9.done())) return rc;
     }
   }

@@ -12,21 +12,18 @@
 //   McLoader  "m-contiguous": matrix rows are the contraction index, the M
 //             (or N) index is contiguous. LDS tile [BK][256], fragments read
 //             with transposed LDS reads.
-// Rows can be addressed through an index list (gather).
+// The rows of a k-contiguous operand can be addressed through an index list (gather).
 //
-// Two main loops share the loaders:
-//   pipelined  every row / column / k of the tile is in range and 16-byte
-//              aligned: tiles are copied global -> LDS asynchronously, three
-//              steps ahead, into a ring of 4 LDS stages; MFMA fragments are
-//              double buffered in registers so that LDS reads of the next
-//              half step overlap the 16 MFMAs of the current one; one
-//              barrier per step.
-//   guarded    anything ragged or unaligned: element-wise guarded loads that
-//              zero fill, staged through registers, 2 LDS stages.
-// The choice is uniform over the workgroup.
+// Two main loops share the loaders; a kernel is compiled for one of them (GUARDED), because both in
+// one kernel cost it registers, spills and instruction cache:
+//   pipelined  operands 16-byte aligned, contraction a multiple of 128: tiles are copied global ->
+//              LDS asynchronously, three steps ahead, into a ring of 4 LDS stages; MFMA fragments
+//              are double buffered in registers so that LDS reads of the next half step overlap
+//              the 16 MFMAs of the current one; one barrier per step (gen_gemm_asm.py). Rows or
+//              columns of a tile past the end of the matrix are copies of valid ones.
+//   guarded    unaligned operands: element-wise guarded loads that zero fill, staged through
+//              registers, 2 LDS stages.
 #pragma once
-
-#include <type_traits>
 
 #include "ct_common.hip.h"
 #include "ct_gemm_asm.inc"
@@ -60,26 +57,20 @@ struct KcLoader {
   const char* base;    // uniform
   unsigned voff[NCH];
   u32x4 regs[NCH];
-  int chunk, k_valid, row_mask;
-  bool fast;
-  bool alias_k;  // k >= k_valid (a multiple of 8) reads the row's first chunk: see alias_invalid_k()
+  int chunk, k_valid;
 
   // rows m0 .. m0+255 of `base_` (leading dimension ld elements), optionally
-  // gathered through row_index. Rows >= rows_valid read as zero, or, with
-  // alias_invalid_rows, as a copy of the first row (for callers that discard
-  // those rows); k >= k_valid reads as zero.
+  // gathered through row_index. Rows >= rows_valid are copies of the first row (callers discard
+  // what they get from them); the guarded loop reads k >= k_valid as zero.
   // With interleave_rows, tile row 128 w + 32 nb + j holds matrix row m0 + 128 w + 4 j + nb:
   // in the accumulator layout lane j of a wavefront then owns 4 consecutive matrix rows (its
   // column blocks nb = 0..3), which an epilogue can store with one 8- or 16-byte access.
   CT_DEVICE void init(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid,
-                      int k_valid_, bool aligned, bool alias_invalid_rows,
-                      bool interleave_rows = false) {
+                      int k_valid_, bool interleave_rows = false) {
     const int t = threadIdx.x;
     k_valid = k_valid_;
-    alias_k = false;
     const bool gathered = row_index != nullptr;
     base = reinterpret_cast<const char*>(gathered ? base_ : base_ + (size_t)m0 * ld);
-    row_mask = 0;
     const int r0 = t / CPR;
     chunk = (t % CPR) ^ swizzle<CPR>(r0);  // rows r0 + 64 n share the swizzle
 #pragma unroll
@@ -88,30 +79,14 @@ struct KcLoader {
       const int r = interleave_rows ? ((tile_row & 128) | ((tile_row & 31) << 2) | ((tile_row >> 5) & 3))
                                     : tile_row;
       const bool ok = m0 + r < rows_valid;
-      if (ok || alias_invalid_rows) row_mask |= 1 << n;
       const long src = gathered ? row_index[ok ? m0 + r : 0] : (ok ? r : 0);
       voff[n] = (unsigned)((src * ld + chunk * 8) * 2);
     }
-    fast = aligned && (alias_invalid_rows || m0 + kGemmTile <= rows_valid) && k_valid % kGemmBK == 0;
-  }
-  // For the last steps of a contraction that ends inside a step: from here on terms k >= k_valid are
-  // read as the first terms of their row, so the copies stay inside the rows and the pipelined
-  // loop serves (for callers whose other operand is zero there).
-  CT_DEVICE void alias_invalid_k(int k_valid_) {
-    k_valid = k_valid_;
-    alias_k = true;
   }
   // copies N0 .. N1-1 of the thread's NCH 16-byte slots
   template <int N0 = 0, int N1 = NCH>
   CT_DEVICE void dma(int k0, lds_addr tile) const {
     const int wave = uniform(threadIdx.x >> 6);
-    if (alias_k) {  // uniform
-      const bool inside = k0 + chunk * 8 < k_valid;
-#pragma unroll
-      for (int n = N0; n < N1; ++n)
-        dma16_s(base, inside ? voff[n] + (unsigned)k0 * 2u : voff[n] - (unsigned)chunk * 16u, tile + (n * 256 + wave * 64) * 16);
-      return;
-    }
     const char* p = base + (size_t)k0 * 2;
 #pragma unroll
     for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
@@ -121,8 +96,7 @@ struct KcLoader {
     const int count = min(max(k_valid - k, 0), 8);
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      const bool ok = (row_mask >> n) & 1;
-      regs[n] = (ok && count) ? load_chunk_guarded(reinterpret_cast<const bf16*>(
+      regs[n] = count ? load_chunk_guarded(reinterpret_cast<const bf16*>(
                                                        base + (size_t)k0 * 2 + voff[n]),
                                                    count)
                               : u32x4{0u, 0u, 0u, 0u};
@@ -144,66 +118,37 @@ struct McLoader {
   static constexpr int CPR = kGemmTile / 8;  // 32
   static constexpr int NCH = 4;
   const char* base;  // uniform: column m0 of row 0
-  const int* row_index;
   long ld;
   unsigned voff[NCH];
   u32x4 regs[NCH];
   int col[2];  // first column of the chunk fetched in even / odd passes
   int cols_left, k_valid;
-  bool fast;
 
-  // columns m0 .. m0+255 of `base_`; contraction rows optionally gathered.
-  // Columns >= cols_valid and rows >= k_valid read as zero, or, with alias_invalid_cols (then m0 and
-  // cols_valid are multiples of 8), the columns as a copy of the tile's first 8 (for callers that
-  // discard what they get from them): a ragged last tile then takes the pipelined loop too.
-  CT_DEVICE void init(const bf16* base_, long ld_, const int* row_index_, int m0, int cols_valid,
-                      int k_valid_, bool aligned, bool alias_invalid_cols = false) {
+  // columns m0 .. m0+255 of `base_`. The guarded loop reads columns >= cols_valid and rows >= k_valid
+  // as zero; the pipelined one, where cols_valid is a multiple of 8, such columns as copies of the
+  // tile's first 8 (callers discard what they get from them).
+  CT_DEVICE void init(const bf16* base_, long ld_, int m0, int cols_valid, int k_valid_) {
     const int t = threadIdx.x;
     base = reinterpret_cast<const char*>(base_ + m0);
-    row_index = row_index_;
     ld = ld_;
     k_valid = k_valid_;
     cols_left = cols_valid - m0;
-    alias_invalid_cols = alias_invalid_cols && aligned;
-    fast = aligned && (alias_invalid_cols || m0 + kGemmTile <= cols_valid) && k_valid % kGemmBK == 0;
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
       const int r = t / CPR + 8 * n;
       int c = ((t % CPR) ^ swizzle<CPR>(r)) * 8;
       col[n & 1] = c;
-      if (alias_invalid_cols && c >= cols_left) c = 0;
-      voff[n] = (unsigned)(((row_index ? 0 : (long)r * ld) + c) * 2);
+      if (c >= cols_left) c = 0;
+      voff[n] = (unsigned)(((long)r * ld + c) * 2);
     }
   }
   // copies N0 .. N1-1 of the thread's NCH 16-byte slots (N0 even, N1 = N0 + 2 or NCH)
   template <int N0 = 0, int N1 = NCH>
   CT_DEVICE void dma(int k0, lds_addr tile) const {
     const int wave = uniform(threadIdx.x >> 6);
-    if (row_index) {
-      // A wavefront covers rows k0 + 2 wave + {0, 1} + 8 n: read the two row indices
-      // with scalar loads (tracked by lgkmcnt, so they do not force the copies
-      // still in flight to drain the way a vector load would).
-      typedef int i32x2 __attribute__((ext_vector_type(2)));
-      const int* ip = row_index + k0 + 2 * wave + 8 * N0;
-      const bool upper = lane_id() >= 32;
+    const char* p = base + (size_t)k0 * ld * 2;
 #pragma unroll
-      for (int n = N0; n < N1; n += 2) {
-        i32x2 p0, p1;
-        asm volatile(
-            "s_load_dwordx2 %0, %2, 0x0\n\ts_load_dwordx2 %1, %2, 0x20\n\ts_waitcnt lgkmcnt(0)"
-            : "=&s"(p0), "=&s"(p1)
-            : "s"(ip + 8 * (n - N0))
-            : "memory");
-        dma16(base + (size_t)(upper ? p0[1] : p0[0]) * ld * 2 + voff[n],
-              tile + (n * 256 + wave * 64) * 16);
-        dma16(base + (size_t)(upper ? p1[1] : p1[0]) * ld * 2 + voff[n + 1],
-              tile + ((n + 1) * 256 + wave * 64) * 16);
-      }
-    } else {
-      const char* p = base + (size_t)k0 * ld * 2;
-#pragma unroll
-      for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
-    }
+    for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
   }
   CT_DEVICE void fetch(int k0) {
     const int r0 = (int)threadIdx.x / CPR;
@@ -212,9 +157,7 @@ struct McLoader {
       const int k = k0 + r0 + 8 * n;
       const int count = min(max(cols_left - col[n & 1], 0), 8);
       if (k < k_valid && count) {
-        const size_t src = row_index ? (size_t)row_index[k] : (size_t)k0;
-        regs[n] = load_chunk_guarded(reinterpret_cast<const bf16*>(base + src * ld * 2 + voff[n]),
-                                     count);
+        regs[n] = load_chunk_guarded(reinterpret_cast<const bf16*>(base + (size_t)k0 * ld * 2 + voff[n]), count);
       } else {
         regs[n] = u32x4{0u, 0u, 0u, 0u};
       }
@@ -261,33 +204,14 @@ CT_DEVICE void mfma_block(const GemmFrags& f, GemmAcc& acc) {
     for (int jn = 0; jn < 4; ++jn) acc.c[i][jn] = mfma32(f.a[i], f.b[jn], acc.c[i][jn]);
 }
 
-template <int I0, int I1>
-CT_DEVICE void mfma_rows(const GemmFrags& f, GemmAcc& acc) {
-#pragma unroll
-  for (int i = I0; i < I1; ++i)
-#pragma unroll
-    for (int jn = 0; jn < 4; ++jn) acc.c[i][jn] = mfma32(f.a[i], f.b[jn], acc.c[i][jn]);
-}
-
-// s_waitcnt vmcnt(N) for N in {0, 8, 12, 16} (expcnt / lgkmcnt left at "no wait").
-CT_DEVICE void wait_vmcnt(int outstanding) {
-  if (outstanding >= 16)
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (1 << 14));  // vmcnt = 16
-  else if (outstanding >= 12)
-    __builtin_amdgcn_s_waitcnt(0x0F70 | 12);
-  else if (outstanding >= 8)
-    __builtin_amdgcn_s_waitcnt(0x0F70 | 8);
-  else
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-}
-CT_DEVICE void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0) only
+// s_waitcnt vmcnt(16) (expcnt / lgkmcnt left at "no wait")
+CT_DEVICE void wait_vmcnt16() { __builtin_amdgcn_s_waitcnt(0x0F70 | (1 << 14)); }
 // Execution barrier without the memory fence of __syncthreads() (which would wait for
 // every copy in flight); callers order their own LDS traffic with the waits above.
 CT_DEVICE void workgroup_barrier() { __builtin_amdgcn_s_barrier(); }
 
 // The pipelined main loop with a fixed instruction order (see gen_gemm_asm.py), for an
-// m-contiguous A without row gather, a k-contiguous B and a step count that is a positive
-// multiple of 4. Entered with the copies of steps 0..2 issued and step 0 landed for every
+// m-contiguous A, a k-contiguous B and a step count that is a positive multiple of 4. Entered with the copies of steps 0..2 issued and step 0 landed for every
 // wavefront; returns with nothing in flight and the LDS tiles free.
 CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned long long b = (unsigned long long)(uintptr_t)p;
@@ -322,91 +246,55 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader& A, const KcLoader& B, int k_b
                : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
 }
 
-// acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T. Must be called by
-// all 256 threads; ends with the LDS tiles free for reuse.
-template <class ALoader, class BLoader>
-CT_DEVICE void gemm_tile(ALoader& A, BLoader& B, int k_begin, int k_end, lds_addr smem,
-                         GemmAcc& acc) {
+// acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T (k_end - k_begin a multiple of 128
+// unless GUARDED). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
+template <bool GUARDED>
+CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_addr smem, GemmAcc& acc) {
   constexpr int BK = kGemmBK, kTile = GemmSmem::kTileBytes, kStage = GemmSmem::kStageBytes;
-  constexpr int kRing = GemmSmem::kStages * kStage;
-  constexpr int kLoadsPerStep = ALoader::NCH + BLoader::NCH;  // 8 per thread
-  static_assert(kLoadsPerStep == 8, "wait_vmcnt assumes 8 copies per thread per step");
   const int w = threadIdx.x >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
   if (k_begin >= k_end) return;
-  const typename ALoader::FragOffsets afo(smem);
-  const typename BLoader::FragOffsets bfo(smem);
-  const int steps = (k_end - k_begin + BK - 1) / BK;
-
-  if (A.fast && B.fast) {
+  const McLoader::FragOffsets afo(smem);
+  const KcLoader::FragOffsets bfo(smem);
+  if constexpr (!GUARDED) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
-    for (int i = 0; i < 3 && i < steps; ++i) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
       A.dma(k_begin + i * BK, smem + i * kStage);
       B.dma(k_begin + i * BK, smem + i * kStage + kTile);
     }
-    wait_vmcnt((min(steps, 3) - 1) * kLoadsPerStep);
+    static_assert(McLoader::NCH + KcLoader::NCH == 8, "the wait leaves the copies of two steps in flight");
+    wait_vmcnt16();
     workgroup_barrier();
-    if constexpr (std::is_same<ALoader, McLoader>::value && std::is_same<BLoader, KcLoader>::value) {
-      if (steps % 4 == 0 && !A.row_index && !B.alias_k) {  // uniform
-        gemm_loop_scheduled(A, B, k_begin, steps, smem, afo, bfo, wm, wn, acc);
-        return;
+    gemm_loop_scheduled(A, B, k_begin, (k_end - k_begin) / BK, smem, afo, bfo, wm, wn, acc);
+  } else {
+    A.fetch(k_begin);
+    B.fetch(k_begin);
+    A.commit(smem);
+    B.commit(smem + kTile);
+    __syncthreads();
+    int cur = 0, nxt = kStage;
+    for (int k0 = k_begin; k0 < k_end; k0 += BK) {
+      const bool more = k0 + BK < k_end;
+      if (more) {
+        A.fetch(k0 + BK);
+        B.fetch(k0 + BK);
       }
-    }
-    GemmFrags f0, f1;
-    load_frags<ALoader, BLoader>(f0, 0, afo, bfo, 0, wm, wn);
-    int stage = 0;
-    for (int k = 0; k < steps; ++k) {
-      // The copies of step k+3 go into the stage read during step k-1 (free since the
-      // last barrier); the B half is issued between the MFMAs so that a shorter burst of
-      // copies stalls the matrix pipe.
-      const int dst = (stage + 3 * kStage) & (kRing - 1);
-      const int k_next = k_begin + (k + 3) * BK;
-      const bool more = k + 3 < steps;
-      load_frags<ALoader, BLoader>(f1, stage, afo, bfo, 1, wm, wn);
-      mfma_rows<0, 1>(f0, acc);
-      if (more) A.dma(k_next, smem + dst);
-      mfma_rows<1, 3>(f0, acc);
-      if (more) B.dma(k_next, smem + dst + kTile);
-      mfma_rows<3, 4>(f0, acc);
-      // step k+1 must have landed: at most the copies of steps k+2, k+3 may be in flight
-      wait_vmcnt(min(max(steps - k - 2, 0), 2) * kLoadsPerStep);
-      wait_lds();  // our reads of this stage are done before anyone recycles it
-      workgroup_barrier();
-      stage = (stage + kStage) & (kRing - 1);
-      if (k + 1 < steps) load_frags<ALoader, BLoader>(f0, stage, afo, bfo, 0, wm, wn);
-      mfma_rows<0, 4>(f1, acc);
-    }
-    wait_lds();
-    __syncthreads();
-    return;
-  }
-
-  A.fetch(k_begin);
-  B.fetch(k_begin);
-  A.commit(smem);
-  B.commit(smem + kTile);
-  __syncthreads();
-  int cur = 0, nxt = kStage;
-  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-    const bool more = k0 + BK < k_end;
-    if (more) {
-      A.fetch(k0 + BK);
-      B.fetch(k0 + BK);
-    }
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      GemmFrags f;
-      load_frags<ALoader, BLoader>(f, cur, afo, bfo, ks, wm, wn);
-      mfma_block(f, acc);
+      for (int ks = 0; ks < BK / 16; ++ks) {
+        GemmFrags f;
+        load_frags<McLoader, KcLoader>(f, cur, afo, bfo, ks, wm, wn);
+        mfma_block(f, acc);
+      }
+      if (more) {
+        A.commit(smem + nxt);
+        B.commit(smem + nxt + kTile);
+      }
+      __syncthreads();
+      const int tmp = cur;
+      cur = nxt;
+      nxt = tmp;
     }
-    if (more) {
-      A.commit(smem + nxt);
-      B.commit(smem + nxt + kTile);
-    }
-    __syncthreads();
-    const int tmp = cur;
-    cur = nxt;
-    nxt = tmp;
   }
 }
 
