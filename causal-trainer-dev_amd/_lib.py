@@ -12,6 +12,7 @@ from pathlib import Path
 
 PACKAGE_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = PACKAGE_DIR / "libct_hotpath.so"
+NATIVE_PATH = PACKAGE_DIR / "_native.so"
 
 CT_OK = 0
 CT_INVALID_ARGUMENT = -1
@@ -154,6 +155,7 @@ SYMBOLS = {
 }
 
 _library = None
+_native = None
 
 
 def load() -> ctypes.CDLL:
@@ -180,6 +182,26 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"libct_hotpath ABI {version} does not match binding ABI {ABI_VERSION}")
     _library = library
     return library
+
+
+def native():
+    """The extension module with the torch side of the operators (csrc/ct_torch.cc)."""
+
+    global _native
+    if _native is None:
+        load()
+        if not NATIVE_PATH.exists():
+            raise RuntimeError(
+                f"{NATIVE_PATH} is missing: build it with `python {PACKAGE_DIR / 'build.py'}`. "
+                "There is no fallback implementation."
+            )
+        import torch  # noqa: F401  (its libraries are what the module links)
+
+        from . import _native as module
+
+        module.set_error_class(CtError)
+        _native = module
+    return _native
 
 
 def check(status: int) -> None:

@@ -1,8 +1,9 @@
-"""Build recipe for libct_hotpath.so (HIP, gfx950 only).
+"""Build recipe for libct_hotpath.so (HIP, gfx950 only) and _native.so (its torch side, host code).
 
 Run ``python causal-trainer-dev_amd/build.py`` (or call :func:`build`) on any
-machine with hipcc; no GPU is needed to compile. The shared library is placed
-next to this file and is what :mod:`_lib` loads through ctypes.
+machine with hipcc; no GPU is needed to compile. The libraries are placed
+next to this file: libct_hotpath.so is what :mod:`_lib` loads through ctypes and what
+_native.so links, _native.so the extension module the torch operators call.
 """
 
 from __future__ import annotations
@@ -17,6 +18,7 @@ from pathlib import Path
 PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC = PACKAGE_DIR / "csrc"
 LIBRARY = PACKAGE_DIR / "libct_hotpath.so"
+NATIVE = PACKAGE_DIR / "_native.so"
 SOURCES = ("ct_error.hip", "ct_attn.hip", "ct_cutce.hip", "ct_prep.hip", "ct_layer.hip", "ct_logits_ce.hip")
 
 # -packed-fp32-ops is switched off on purpose: hipcc must not form packed FP32
@@ -63,14 +65,47 @@ def build(verbose: bool = False, extra_flags: tuple[str, ...] = ()) -> Path:
             print(" ".join(cmd), flush=True)
         _run(cmd)
 
-    with ThreadPoolExecutor(max_workers=min(4, len(sources))) as pool:
+    native_object = build_dir / "ct_torch.o"
+    with ThreadPoolExecutor(max_workers=4) as pool:
+        native = pool.submit(_compile_native, native_object, verbose)
         list(pool.map(compile_one, zip(sources, objects)))
-    link = [compiler, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc",
+        native.result()
+    link = [compiler, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-Wl,-soname,libct_hotpath.so",
             *map(str, objects), "-o", str(LIBRARY)]
     if verbose:
         print(" ".join(link), flush=True)
     _run(link)
+    _link_native(native_object, verbose)
     return LIBRARY
+
+
+def _torch_paths():
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    return root / "include", root / "lib"
+
+
+def _compile_native(obj: Path, verbose: bool) -> None:
+    import sysconfig
+
+    include, _ = _torch_paths()
+    cmd = ["g++", "-c", str(CSRC / "ct_torch.cc"), "-o", str(obj), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+           "-DTORCH_EXTENSION_NAME=_native", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-Wno-attributes",
+           f"-I{include}", f"-I{include / 'torch/csrc/api/include'}", "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    _run(cmd)
+
+
+def _link_native(obj: Path, verbose: bool) -> None:
+    _, lib = _torch_paths()
+    cmd = ["g++", "-shared", str(obj), "-o", str(NATIVE), str(LIBRARY), "-Wl,-rpath,$ORIGIN", f"-L{lib}",
+           f"-Wl,-rpath,{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    _run(cmd)
 
 
 if __name__ == "__main__":

@@ -35,6 +35,7 @@ keeps the single full-vocabulary slab.
 
 from __future__ import annotations
 
+import functools
 
 import torch
 
@@ -76,25 +77,8 @@ def cutce_forward(hidden, head, targets, weights, *, sparse_compaction: bool = F
     the forward fills for ``cutce_backward``.
     """
 
-    lib = _lib.load()
-    rows, width = hidden.shape
-    shape = _shape_struct(rows, width, head.shape[1])
-    device = hidden.device
-    workspace = torch.empty(lib.ct_cutce_fwd_workspace_bytes(shape), dtype=torch.uint8, device=device)
-    scalars = torch.empty(2, dtype=torch.float32, device=device)
-    lse = torch.empty(rows, dtype=torch.float32, device=device)
-    args = _lib.CutceFwdArgs(
-        hidden=hidden.data_ptr(), head=head.data_ptr(), targets=targets.data_ptr(),
-        weights=weights.data_ptr(), nll_sum=scalars[0:].data_ptr(),
-        weight_sum=scalars[1:].data_ptr(), lse=lse.data_ptr(),
-        workspace=workspace.data_ptr(), workspace_bytes=workspace.numel(),
-        shape=shape, sparse_compaction=int(bool(sparse_compaction)),
-        logits_cache=_lib.pointer(logits_cache),
-        logits_cache_bytes=0 if logits_cache is None else logits_cache.numel(),
-    )
-    with torch.cuda.device(device):
-        _lib.check(lib.ct_cutce_fwd(_lib.current_stream(), args))
-    return scalars[0], scalars[1], lse
+    return _lib.native().cutce_forward(hidden.detach(), head.detach(), targets, weights, bool(sparse_compaction),
+                                       logits_cache, -1)
 
 
 def cutce_backward(hidden, head, targets, weights, lse, dy, *, sparse_compaction: bool = False,
@@ -106,62 +90,39 @@ def cutce_backward(hidden, head, targets, weights, lse, dy, *, sparse_compaction
     to recompute the logits.
     """
 
-    lib = _lib.load()
-    rows, width = hidden.shape
-    shape = _shape_struct(rows, width, head.shape[1])
-    device = hidden.device
-    if workspace_bytes is None:
-        workspace_bytes = lib.ct_cutce_bwd_workspace_bytes(shape)
-    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
-    dhidden = torch.empty_like(hidden)
-    dhead = torch.empty_like(head) if lm_head_trainable else None
-    dy = dy.to(device=device, dtype=torch.float32).reshape(1).contiguous()
-    args = _lib.CutceBwdArgs(
-        hidden=hidden.data_ptr(), head=head.data_ptr(), targets=targets.data_ptr(),
-        weights=weights.data_ptr(), lse=lse.data_ptr(), dy=dy.data_ptr(),
-        dhidden=dhidden.data_ptr(), dhead=_lib.pointer(dhead),
-        workspace=workspace.data_ptr(), workspace_bytes=workspace.numel(),
-        shape=shape, sparse_compaction=int(bool(sparse_compaction)),
-        logits_cache=_lib.pointer(logits_cache),
-        logits_cache_bytes=0 if logits_cache is None else logits_cache.numel(),
-    )
-    with torch.cuda.device(device):
-        _lib.check(lib.ct_cutce_bwd(_lib.current_stream(), args))
-    return dhidden, dhead
+    dy = dy.to(device=hidden.device, dtype=torch.float32).reshape(1).contiguous()
+    return _lib.native().cutce_backward(
+        hidden.detach(), head.detach(), targets, weights, lse, dy, bool(sparse_compaction), bool(lm_head_trainable),
+        -1 if workspace_bytes is None else int(workspace_bytes), logits_cache)
 
 
-class _CutCE(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, hidden, head, targets, weights, lm_head_trainable, sparse_compaction,
-                logits_cache, local_chunk_size):
-        cache = None
-        ctx.workspace_bytes = backward_workspace_bytes(hidden.shape[0], hidden.shape[1], head.shape[1],
-                                                       local_chunk_size)
-        if logits_cache and not local_chunk_size and (hidden.requires_grad or head.requires_grad):
-            size = logits_cache_bytes(hidden.shape[0], hidden.shape[1], head.shape[1])
-            if size <= LOGITS_CACHE_LIMIT_BYTES:
-                cache = torch.empty(size, dtype=torch.uint8, device=hidden.device)
-        nll_sum, weight_sum, lse = cutce_forward(hidden, head, targets, weights,
-                                                 sparse_compaction=sparse_compaction,
-                                                 logits_cache=cache)
-        # The reference's residual (:587-593) plus, when it fits, the f32 logits cache.
-        ctx.save_for_backward(hidden, head, targets, weights, lse)
-        ctx.logits_cache = cache
-        ctx.lm_head_trainable = lm_head_trainable
-        ctx.sparse_compaction = sparse_compaction
-        ctx.mark_non_differentiable(weight_sum)
-        return nll_sum, weight_sum
+@functools.lru_cache(maxsize=256)
+def _workspaces(rows: int, hidden: int, vocab: int, local_chunk_size: int):
+    """(forward, backward) workspace sizes; -1 leaves the choice to the library."""
 
-    @staticmethod
-    def backward(ctx, nll_cotangent, _weight_cotangent):
-        hidden, head, targets, weights, lse = ctx.saved_tensors
-        dhidden, dhead = cutce_backward(
-            hidden, head, targets, weights, lse, nll_cotangent,
-            sparse_compaction=ctx.sparse_compaction, lm_head_trainable=ctx.lm_head_trainable,
-            logits_cache=ctx.logits_cache, workspace_bytes=ctx.workspace_bytes,
-        )
-        ctx.logits_cache = None
-        return dhidden, dhead, None, None, None, None, None, None
+    if local_chunk_size <= 0:
+        return -1, -1
+    backward = backward_workspace_bytes(rows, hidden, vocab, local_chunk_size)
+    lib, shape = _lib.load(), _shape_struct(rows, hidden, vocab)
+    # (the forward's part that may be smaller, an aligned copy of the head, keeps to the same bound)
+    forward = max(lib.ct_cutce_fwd_workspace_min_bytes(shape), min(lib.ct_cutce_fwd_workspace_bytes(shape), backward))
+    return int(forward), int(backward)
+
+
+def _cut(hidden, head, targets, weights, trainable, compaction, cache, chunk):
+    """The operator on plain arguments (what the native side checks), None for any other."""
+
+    try:
+        if targets.shape != weights.shape or hidden.shape[:-1] != targets.shape:
+            return None
+        rows, width, vocab = targets.numel(), hidden.shape[-1], head.shape[1]
+        if rows == 0 or width == 0 or vocab == 0:
+            return None
+        sizes = (-1, -1) if chunk == 0 else _workspaces(rows, width, vocab, chunk)
+        return _lib.native().cut_ce(hidden, head, targets, weights, bool(trainable), bool(compaction),
+                                    bool(cache) and chunk == 0, LOGITS_CACHE_LIMIT_BYTES, *sizes)
+    except (AttributeError, IndexError, TypeError):
+        return None     # (something is wrong with the arguments: the validation says what)
 
 
 def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weights, *, mesh=None,
@@ -181,6 +142,11 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
     each, about 0.4 ms per GB on this part); its gradient comes back as ``[V, d]``.
     """
 
+    if mesh is None and head_layout == "dv" and type(local_chunk_size) is int and local_chunk_size >= 0:
+        out = _cut(hidden_states, lm_head_kernel, targets, weights, lm_head_trainable, sparse_compaction, logits_cache,
+                   local_chunk_size)
+        if out is not None:
+            return out
     if head_layout not in ("dv", "vd"):
         raise ValueError("head_layout must be 'dv' ([hidden, vocab]) or 'vd' ([vocab, hidden])")
     if head_layout == "vd":
@@ -222,12 +188,11 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
                          + ", ".join(sharded_rows))
     if active:
         raise ValueError(f"this build runs on one GPU; mesh axes larger than 1: {active}")
-    width = hidden_states.shape[-1]
-    return _CutCE.apply(
-        hidden_states.reshape(-1, width).contiguous(), lm_head_kernel.contiguous(),
-        targets.reshape(-1).contiguous(), weights.reshape(-1).contiguous(),
-        bool(lm_head_trainable), bool(sparse_compaction), bool(logits_cache), local_chunk_size,
-    )
+    out = _cut(hidden_states.contiguous(), lm_head_kernel.contiguous(), targets.contiguous(), weights.contiguous(),
+               lm_head_trainable, sparse_compaction, logits_cache, local_chunk_size)
+    if out is None:
+        raise RuntimeError("Cut cross-entropy is available only for dense tensors on one ROCm GPU")
+    return out
 
 
 __all__ = ["LOGITS_CACHE_LIMIT_BYTES", "backward_workspace_bytes", "cutce_backward", "cutce_forward", "logits_cache_bytes",

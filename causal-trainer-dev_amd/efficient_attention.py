@@ -21,6 +21,7 @@ read per-tile bounds from ``AttentionMetadata.tile_bounds``.
 
 from __future__ import annotations
 
+import functools
 import math
 from typing import NamedTuple
 
@@ -60,17 +61,6 @@ def _as_device_int32(value, name: str) -> torch.Tensor:
     return tensor.contiguous()
 
 
-def _block_summary(segments: torch.Tensor, ends: torch.Tensor | None, block: int) -> torch.Tensor:
-    batch, sequence = segments.shape
-    width = 3 if ends is not None else 2
-    out = torch.empty((batch, sequence // block, width), dtype=torch.int32, device=segments.device)
-    lib = _lib.load()
-    _lib.check(lib.ct_attn_block_summary(_lib.current_stream(), segments.data_ptr(),
-                                         _lib.pointer(ends), batch, sequence, block,
-                                         out.data_ptr()))
-    return out
-
-
 def prepare_attention_metadata(canonical_segment_ids, *, mesh, profile,
                                attention_end=None) -> AttentionMetadata:
     """Build per-tile summaries once, immediately before the decoder loop."""
@@ -97,14 +87,7 @@ def prepare_attention_metadata(canonical_segment_ids, *, mesh, profile,
         if ends.shape != segments.shape:
             raise ValueError("attention_end must match canonical_segment_ids")
 
-    lib = _lib.load()
-    bounds = torch.empty(lib.ct_attn_meta_bytes(batch, sequence) // 4, dtype=torch.int32,
-                         device=segments.device)
-    with torch.cuda.device(segments.device):
-        _lib.check(lib.ct_attn_prepare(_lib.current_stream(), segments.data_ptr(),
-                                       _lib.pointer(ends), batch, sequence, bounds.data_ptr()))
-        q_summary = _block_summary(segments, ends, block_q)
-        kv_summary = _block_summary(segments, None, outer)
+    bounds, q_summary, kv_summary = _lib.native().attention_metadata(segments, ends, block_q, outer)
     return AttentionMetadata(
         query_segment_ids=segments,
         kv_segment_ids=segments,
@@ -161,28 +144,6 @@ def _python_scalar(scale) -> float:
     return number
 
 
-def _attn_forward(query, key, value, metadata, scale):
-    batch, sequence, q_heads, head_dim = query.shape
-    out = torch.empty_like(query)
-    lse = torch.empty((batch, sequence, q_heads), dtype=torch.float32, device=query.device)
-    args = _lib.AttnFwdArgs(
-        q=query.data_ptr(), k=key.data_ptr(), v=value.data_ptr(),
-        segment_ids=metadata.query_segment_ids.data_ptr(),
-        attention_end=_lib.pointer(metadata.attention_end),
-        tile_meta=metadata.tile_bounds.data_ptr(),
-        out=out.data_ptr(), lse=lse.data_ptr(),
-        batch=batch, seq=sequence, q_heads=q_heads, kv_heads=key.shape[2], head_dim=head_dim,
-        scale=scale,
-    )
-    with torch.cuda.device(query.device):
-        _lib.check(_lib.load().ct_attn_fwd(_lib.current_stream(), args))
-    return out, lse
-
-
-# Left to itself (dq_form=None) the backward offers the library the larger workspace of the
-# stored-dS form for rows of up to 4096 positions, if that is at most 4 GiB.
-_FROM_DS_UP_TO_SEQ = 4096
-_FROM_DS_WORKSPACE_CAP = 4 << 30
 _DKV_KERNELS = {None: 0, "narrow": _lib.ATTN_BWD_DKV_NARROW, "wide": _lib.ATTN_BWD_DKV_WIDE}
 _DQ_FORMS = {None: 0, "recompute": _lib.ATTN_BWD_DQ_RECOMPUTE, "from_ds": _lib.ATTN_BWD_DQ_FROM_DS}
 
@@ -199,89 +160,34 @@ class BackwardWorkspace:
     run on one stream, one after the other."""
 
     def __init__(self):
-        self._buffer = None
-        self._built_for = None
-
-    def _acquire(self, nbytes, device, key):
-        if self._buffer is None or self._buffer.numel() < nbytes or self._buffer.device != device:
-            self._buffer = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            self._built_for = None
-        return self._buffer, self._built_for == key
-
-    def _built(self, key):
-        self._built_for = key
+        self._kept = _lib.native().KeptWorkspace()
 
 
-def _attn_backward(query, key, value, metadata, out, lse, dout, scale, with_delta=False, dkv_kernel=None,
-                   dq_form=None, workspace_bytes=None, kept=None):
-    batch, sequence, q_heads, head_dim = query.shape
-    lib = _lib.load()
-    dq = torch.empty_like(query)
-    dk = torch.empty_like(key)
-    dv = torch.empty_like(value)
-    delta = torch.empty_like(lse)
-    shape = (batch, sequence, query.shape[2], key.shape[2], head_dim)
-    if workspace_bytes is None:
-        stored = int(lib.ct_attn_bwd_workspace_bytes_from_ds(*shape, int(metadata.attention_end is not None)))
-        if dq_form == "from_ds":
-            workspace_bytes = stored
-            if workspace_bytes == 0:
-                raise ValueError("dq_form='from_ds' is not available for this shape (dS blocks of one KV head "
-                                 "exceed 64 GiB)")
-        elif dq_form is None and sequence <= _FROM_DS_UP_TO_SEQ and 0 < stored <= _FROM_DS_WORKSPACE_CAP:
-            # the library then takes the stored-dS form, which is the faster one at such rows
-            workspace_bytes = stored
-        else:
-            workspace_bytes = int(lib.ct_attn_bwd_workspace_bytes(*shape))
-    variant = _DKV_KERNELS[dkv_kernel] | _DQ_FORMS[dq_form]
-    if kept is None:
-        workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=query.device)
-    else:
-        # (the version counter of the metadata tensor changes when it is written in place)
-        built_for = (metadata.tile_bounds.data_ptr(), metadata.tile_bounds._version, shape, variant,
-                     workspace_bytes, float(scale))
-        workspace, list_kept = kept._acquire(workspace_bytes, query.device, built_for)
-        if list_kept:
-            variant |= _lib.ATTN_BWD_WORK_LIST_KEPT
-    args = _lib.AttnBwdArgs(
-        q=query.data_ptr(), k=key.data_ptr(), v=value.data_ptr(),
-        segment_ids=metadata.query_segment_ids.data_ptr(),
-        attention_end=_lib.pointer(metadata.attention_end),
-        tile_meta=metadata.tile_bounds.data_ptr(),
-        out=out.data_ptr(), lse=lse.data_ptr(), dout=dout.data_ptr(),
-        dq=dq.data_ptr(), dk=dk.data_ptr(), dv=dv.data_ptr(), delta=delta.data_ptr(),
-        workspace=workspace.data_ptr(), workspace_bytes=workspace_bytes,
-        batch=batch, seq=sequence, q_heads=q_heads, kv_heads=key.shape[2], head_dim=head_dim,
-        scale=scale, variant=variant,
-    )
-    with torch.cuda.device(query.device):
-        _lib.check(lib.ct_attn_bwd(_lib.current_stream(), args))
-    if kept is not None:
-        kept._built(built_for)
-    if with_delta:
-        return dq, dk, dv, delta.view(batch, q_heads, sequence)
-    return dq, dk, dv
+def _kept(workspace):
+    return None if workspace is None else workspace._kept
 
 
-class _EfficientAttention(torch.autograd.Function):
-    """Custom VJP with the reference's residual (q, k, v, metadata, O, LSE) (:1831-1863)."""
+@functools.lru_cache(maxsize=1024)
+def _plain_profile(query_shape, key_shape, profile, has_end):
+    """(summary granularity of queries, of keys) for shapes that pass validation on one device."""
 
-    @staticmethod
-    def forward(ctx, query, key, value, metadata, scale, backward_workspace=None):
-        out, lse = _attn_forward(query, key, value, metadata, scale)
-        ctx.save_for_backward(query, key, value, out, lse)
-        ctx.attention_metadata = metadata
-        ctx.scale = scale
-        ctx.backward_workspace = backward_workspace
-        return out
+    if profile is None:
+        profile = resolve_attention_profile(query_shape, key_shape, None, has_attention_end=has_end)
+    validate_attention_profile(profile, query_shape, key_shape, None)
+    return int(profile.block_q), int(profile.block_kv_outer)
 
-    @staticmethod
-    def backward(ctx, output_cotangent):
-        query, key, value, out, lse = ctx.saved_tensors
-        dout = output_cotangent.to(torch.bfloat16).contiguous()
-        dq, dk, dv = _attn_backward(query, key, value, ctx.attention_metadata, out, lse, dout, ctx.scale,
-                                    kept=ctx.backward_workspace)
-        return dq, dk, dv, None, None, None
+
+def _attend(query, key, value, metadata, profile, scale, workspace):
+    """The operator on plain arguments (what the native side checks), None for any other."""
+
+    if not isinstance(metadata, AttentionMetadata) or not (profile is None or isinstance(profile, AttentionKernelProfile)):
+        return None
+    try:
+        blocks = _plain_profile(query.shape, key.shape, profile, metadata.attention_end is not None)
+        return _lib.native().attention(query, key, value, *metadata[:6], *blocks,
+                                       query.shape[-1] ** -0.5 if scale is None else scale, _kept(workspace))
+    except (AttributeError, IndexError, TypeError, ValueError):
+        return None     # (something is wrong with the arguments: the validation says what)
 
 
 def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None, scale=None,
@@ -294,6 +200,10 @@ def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None,
     a model that share ``metadata`` share the scratch buffer of the backward and the work list in it.
     """
 
+    if mesh is None and causal is True and (scale is None or type(scale) in (float, int)):
+        out = _attend(query, key, value, metadata, profile, scale, backward_workspace)
+        if out is not None:
+            return out
     if not isinstance(causal, bool):
         raise TypeError("causal must be a compile-time bool")
     if not causal:
@@ -322,16 +232,22 @@ def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None,
     validate_attention_profile(resolved_profile, query_shape, key_shape, mesh)
     _validate_metadata(metadata, query_shape, resolved_profile)
     resolved_scale = default_attention_scale(query_shape[-1]) if scale is None else _python_scalar(scale)
-    return _EfficientAttention.apply(
-        query.contiguous(), key.contiguous(), value.contiguous(), metadata, resolved_scale, backward_workspace
-    )
+    metadata = metadata._replace(**{name: tensor.contiguous() for name, tensor in metadata._asdict().items()
+                                    if tensor is not None})
+    out = _attend(query.contiguous(), key.contiguous(), value.contiguous(), metadata, resolved_profile,
+                  resolved_scale, backward_workspace)
+    if out is None:
+        raise RuntimeError("efficient_attention is available only for dense tensors on one ROCm GPU")
+    return out
 
 
 def attention_forward_with_lse(query, key, value, metadata, *, scale=None):
     """Forward only, returning ``(O, LSE)``: the residual pair the custom VJP saves."""
 
     resolved = default_attention_scale(query.shape[-1]) if scale is None else float(scale)
-    return _attn_forward(query.contiguous(), key.contiguous(), value.contiguous(), metadata, resolved)
+    return _lib.native().attention_forward(
+        query.contiguous().detach(), key.contiguous().detach(), value.contiguous().detach(), metadata.query_segment_ids,
+        metadata.attention_end, metadata.tile_bounds, resolved)
 
 
 def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=None, with_delta=False,
@@ -348,8 +264,14 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     buffer, and with it the dK/dV work list, from one call to the next."""
 
     resolved = default_attention_scale(query.shape[-1]) if scale is None else float(scale)
-    return _attn_backward(query, key, value, metadata, out, lse, dout.contiguous(), resolved, with_delta,
-                          dkv_kernel, dq_form, workspace_bytes, workspace)
+    dq, dk, dv, delta = _lib.native().attention_backward(
+        query.detach(), key.detach(), value.detach(), metadata.query_segment_ids, metadata.attention_end,
+        metadata.tile_bounds, out.detach(), lse, dout.contiguous(), resolved, _DKV_KERNELS[dkv_kernel] | _DQ_FORMS[dq_form],
+        -1 if workspace_bytes is None else int(workspace_bytes), _kept(workspace))
+    if with_delta:
+        batch, sequence, q_heads, _ = query.shape
+        return dq, dk, dv, delta.view(batch, q_heads, sequence)
+    return dq, dk, dv
 
 
 __all__ = [

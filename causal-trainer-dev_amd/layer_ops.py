@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .prep import _int32, canonicalize_segment_ids
+from .prep import _int32, _nonzero, canonicalize_segment_ids
 
 _STYLES = {"gpt-j": 0, "gpt-neox": 1}
 
@@ -22,19 +22,14 @@ def _make_position_ids_precanonicalized(attention_mask, segment_ids) -> torch.Te
     mask = torch.as_tensor(attention_mask)
     if mask.ndim != 2:
         raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
-    valid = _int32(mask != 0, "attention_mask")
+    valid = _nonzero(mask, "attention_mask")
     segments = torch.as_tensor(segment_ids)
     if tuple(segments.shape) != tuple(valid.shape):
         raise ValueError(f"segment_ids must have shape {tuple(valid.shape)}, got {tuple(segments.shape)}")
     segments = _int32(segments, "segment_ids")
-    batch, sequence = valid.shape
-    out = torch.empty_like(valid)
-    if batch == 0 or sequence == 0:
-        return out
-    with torch.cuda.device(valid.device):
-        _lib.check(_lib.load().ct_position_ids(_lib.current_stream(), valid.data_ptr(), segments.data_ptr(),
-                                               batch, sequence, out.data_ptr()))
-    return out
+    if valid.numel() == 0:
+        return torch.empty_like(valid)
+    return _lib.native().position_ids(valid, segments)
 
 
 def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
@@ -60,42 +55,11 @@ def rotary_cos_sin(position_ids, inv_freq, dtype=torch.bfloat16):
     positions = _int32(positions, "position_ids")
     frequencies = frequencies.to(device=positions.device, dtype=torch.float32).contiguous()
     batch, sequence = positions.shape
-    pairs = frequencies.shape[0]
-    cosine = torch.empty((batch, sequence, pairs), dtype=torch.bfloat16, device=positions.device)
-    sine = torch.empty_like(cosine)
-    if batch * sequence:
-        with torch.cuda.device(positions.device):
-            _lib.check(_lib.load().ct_rotary_cos_sin(
-                _lib.current_stream(), positions.data_ptr(), frequencies.data_ptr(), batch * sequence, pairs,
-                cosine.data_ptr(), sine.data_ptr()))
-    return cosine, sine
-
-
-def _rotate(query, key, cosine, sine, style: int, inverse: bool, q_scale: float):
-    batch, sequence, q_heads, head_dim = query.shape
-    q_out, k_out = torch.empty_like(query), torch.empty_like(key)
-    args = _lib.RotaryArgs(
-        q_in=query.data_ptr(), k_in=key.data_ptr(), q_out=q_out.data_ptr(), k_out=k_out.data_ptr(),
-        cosine=cosine.data_ptr(), sine=sine.data_ptr(), tokens=batch * sequence,
-        q_heads=q_heads, kv_heads=key.shape[2], head_dim=head_dim, rotary_pairs=cosine.shape[-1],
-        rope_style=style, inverse=1 if inverse else 0, q_scale=float(q_scale))
-    with torch.cuda.device(query.device):
-        _lib.check(_lib.load().ct_apply_rotary(_lib.current_stream(), args))
-    return q_out, k_out
-
-
-class _ApplyRotary(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, query, key, cosine, sine, style, q_scale):
-        ctx.save_for_backward(cosine, sine)
-        ctx.style, ctx.q_scale = style, q_scale
-        return _rotate(query, key, cosine, sine, style, False, q_scale)
-
-    @staticmethod
-    def backward(ctx, dq, dk):
-        cosine, sine = ctx.saved_tensors
-        dq_in, dk_in = _rotate(dq.contiguous(), dk.contiguous(), cosine, sine, ctx.style, True, ctx.q_scale)
-        return dq_in, dk_in, None, None, None, None
+    if batch * sequence == 0:
+        shape = (batch, sequence, frequencies.shape[0])
+        return (torch.empty(shape, dtype=torch.bfloat16, device=positions.device),
+                torch.empty(shape, dtype=torch.bfloat16, device=positions.device))
+    return _lib.native().rotary_tables(positions, frequencies)
 
 
 def apply_rotary_cos_sin(query, key, cosine, sine, *, rope_style: str = "gpt-j", q_scale: float = 1.0):
@@ -105,6 +69,13 @@ def apply_rotary_cos_sin(query, key, cosine, sine, *, rope_style: str = "gpt-j",
     operator's bf16 pre-scale of Q in the same pass; call the attention operator with scale 1 then.
     """
 
+    if rope_style in _STYLES and type(q_scale) in (float, int):
+        try:
+            rotated = _lib.native().apply_rotary(query, key, cosine, sine, _STYLES[rope_style], q_scale)
+        except TypeError:
+            rotated = None      # (something is wrong with the arguments: the validation says what)
+        if rotated is not None:
+            return rotated
     if query.ndim != 4 or key.ndim != 4:
         raise ValueError("query and key must have shape [batch, sequence, heads, head_dim]")
     if query.shape[:2] != key.shape[:2] or query.shape[-1] != key.shape[-1]:
@@ -126,8 +97,13 @@ def apply_rotary_cos_sin(query, key, cosine, sine, *, rope_style: str = "gpt-j",
         raise ValueError("the MI355X path rotates bfloat16 query and key only")
     cosine = cosine.to(torch.bfloat16).contiguous()
     sine = sine.to(torch.bfloat16).contiguous()
-    return _ApplyRotary.apply(query.contiguous(), key.contiguous(), cosine, sine, _STYLES[rope_style],
-                              float(q_scale))
+    if query.numel() == 0 or key.numel() == 0:
+        raise _lib.CtError(_lib.CT_INVALID_ARGUMENT, "ct_apply_rotary: dimensions must be positive")
+    rotated = _lib.native().apply_rotary(query.contiguous(), key.contiguous(), cosine, sine, _STYLES[rope_style],
+                                         float(q_scale))
+    if rotated is None:
+        raise RuntimeError("query, key and the tables must be dense tensors on one ROCm GPU")
+    return rotated
 
 
 def apply_rotary_embedding(query, key, position_ids, inv_freq, *, rope_style: str = "gpt-j"):
@@ -137,38 +113,16 @@ def apply_rotary_embedding(query, key, position_ids, inv_freq, *, rope_style: st
     return apply_rotary_cos_sin(query, key, cosine, sine, rope_style=rope_style)
 
 
-class _RmsNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, scale, eps):
-        hidden = x.shape[-1]
-        x2 = x.reshape(-1, hidden)
-        y = torch.empty_like(x2)
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.load().ct_rms_norm_fwd(_lib.current_stream(), x2.data_ptr(), scale.data_ptr(), eps,
-                                                   x2.shape[0], hidden, y.data_ptr(), None))
-        ctx.save_for_backward(x2, scale)
-        ctx.eps, ctx.shape = eps, x.shape
-        return y.reshape(x.shape)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x2, scale = ctx.saved_tensors
-        hidden = x2.shape[-1]
-        lib = _lib.load()
-        dy2 = dy.contiguous().reshape(-1, hidden)
-        dx = torch.empty_like(x2)
-        dscale = torch.empty(hidden, dtype=torch.float32, device=x2.device)
-        workspace = torch.empty(lib.ct_rms_norm_bwd_workspace_bytes(hidden), dtype=torch.uint8, device=x2.device)
-        with torch.cuda.device(x2.device):
-            _lib.check(lib.ct_rms_norm_bwd(_lib.current_stream(), x2.data_ptr(), scale.data_ptr(), dy2.data_ptr(),
-                                           ctx.eps, x2.shape[0], hidden, dx.data_ptr(), dscale.data_ptr(),
-                                           workspace.data_ptr(), workspace.numel()))
-        return dx.reshape(ctx.shape), dscale.to(scale.dtype), None
-
-
 def rms_norm(x, scale, eps: float, compute_dtype=torch.bfloat16) -> torch.Tensor:
     """RMS normalisation over the last axis with f32 statistics and a learned scale."""
 
+    if compute_dtype == torch.bfloat16:
+        try:
+            y = _lib.native().rms_norm(x, scale, eps)
+        except TypeError:
+            y = None    # (something is wrong with the arguments: the validation says what)
+        if y is not None:
+            return y
     if compute_dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
         raise ValueError("the MI355X path normalises bfloat16 activations with a bfloat16 compute dtype")
     if not x.is_cuda:
@@ -177,7 +131,7 @@ def rms_norm(x, scale, eps: float, compute_dtype=torch.bfloat16) -> torch.Tensor
         raise ValueError(f"scale must have shape ({x.shape[-1]},), got {tuple(scale.shape)}")
     if x.numel() == 0:
         return torch.empty_like(x)
-    return _RmsNorm.apply(x.contiguous(), scale.to(device=x.device, dtype=torch.bfloat16).contiguous(), float(eps))
+    return _lib.native().rms_norm(x.contiguous(), scale.to(device=x.device, dtype=torch.bfloat16).contiguous(), float(eps))
 
 
 __all__ = ["make_position_ids", "rotary_cos_sin", "apply_rotary_cos_sin", "apply_rotary_embedding", "rms_norm"]

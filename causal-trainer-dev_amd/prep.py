@@ -24,27 +24,29 @@ def _int32(tensor, name: str, shape=None) -> torch.Tensor:
     return tensor.to(torch.int32).contiguous()
 
 
+def _nonzero(tensor, name: str) -> torch.Tensor:
+    """A mask for the kernels that read "not zero" as set: int32 as it is, anything else compared first."""
+
+    tensor = torch.as_tensor(tensor)
+    return _int32(tensor if tensor.dtype == torch.int32 else tensor != 0, name)
+
+
 def canonicalize_segment_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     """One-based ids of contiguous valid runs, zero for padding (int32 ``[batch, sequence]``)."""
 
     mask = torch.as_tensor(attention_mask)
     if mask.ndim != 2:
         raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
-    valid = _int32(mask != 0, "attention_mask")
+    valid = _nonzero(mask, "attention_mask")
     labels = None
     if segment_ids is not None:
         labels = torch.as_tensor(segment_ids)
         if tuple(labels.shape) != tuple(valid.shape):
             raise ValueError(f"segment_ids must have shape {tuple(valid.shape)}, got {tuple(labels.shape)}")
         labels = _int32(labels, "segment_ids")
-    batch, sequence = valid.shape
-    out = torch.empty_like(valid)
-    if batch == 0 or sequence == 0:
-        return out
-    with torch.cuda.device(valid.device):
-        _lib.check(_lib.load().ct_canonicalize_segment_ids(
-            _lib.current_stream(), valid.data_ptr(), _lib.pointer(labels), batch, sequence, out.data_ptr()))
-    return out
+    if valid.numel() == 0:
+        return torch.empty_like(valid)
+    return _lib.native().canonical_ids(valid, labels)
 
 
 def shifted_targets_and_weights(input_ids, attention_mask, segment_ids=None, assistant_mask=None,
@@ -65,7 +67,7 @@ def shifted_targets_and_weights(input_ids, attention_mask, segment_ids=None, ass
         assistant = torch.as_tensor(assistant_mask)
         if tuple(assistant.shape) != tuple(shape):
             raise ValueError(f"assistant_mask must have shape {tuple(shape)}, got {tuple(assistant.shape)}")
-        assistant_t = _int32(assistant != 0, "assistant_mask")
+        assistant_t = _nonzero(assistant, "assistant_mask")
     loss_t = None
     if loss_mask is not None:
         loss_t = torch.as_tensor(loss_mask)
@@ -75,26 +77,10 @@ def shifted_targets_and_weights(input_ids, attention_mask, segment_ids=None, ass
     batch, sequence = shape
     if sequence < 2:
         raise ValueError("input_ids needs at least two positions to form a prediction edge")
-    lib = _lib.load()
-    targets = torch.empty((batch, sequence - 1), dtype=torch.int32, device=tokens.device)
-    weights = torch.empty((batch, sequence - 1), dtype=torch.float32, device=tokens.device)
-    scratch = None
-    if segment_t is not None:
-        if mask_t is None:          # every token valid
-            mask_t = torch.ones_like(tokens)
-        scratch = torch.empty(lib.ct_shifted_targets_scratch_bytes(batch, sequence), dtype=torch.uint8,
-                              device=tokens.device)
-    args = _lib.ShiftedTargetsArgs(
-        input_ids=tokens.data_ptr(), attention_mask=_lib.pointer(mask_t),
-        segment_ids=_lib.pointer(segment_t), assistant_mask=_lib.pointer(assistant_t),
-        loss_mask=_lib.pointer(loss_t), labels=_lib.pointer(label_t),
-        targets=targets.data_ptr(), weights=weights.data_ptr(),
-        scratch=_lib.pointer(scratch), scratch_bytes=0 if scratch is None else scratch.numel(),
-        batch=batch, seq=sequence, ignore_index=int(ignore_index),
-    )
-    with torch.cuda.device(tokens.device):
-        _lib.check(lib.ct_shifted_targets_and_weights(_lib.current_stream(), args))
-    return targets, weights
+    if batch == 0:
+        raise _lib.CtError(_lib.CT_INVALID_ARGUMENT, "ct_shifted_targets_and_weights: batch and sequence must be positive, "
+                           f"got [{batch}, {sequence}]")
+    return _lib.native().shifted_targets(tokens, mask_t, segment_t, assistant_t, loss_t, label_t, int(ignore_index))
 
 
 __all__ = ["canonicalize_segment_ids", "shifted_targets_and_weights"]
