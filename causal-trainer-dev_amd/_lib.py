@@ -122,6 +122,7 @@ SYMBOLS = {
     "ct_abi_version": (c_int32, []),
     "ct_calibration_copy": (c_int32, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "ct_canonicalize_segment_ids": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
+    "ct_segment_positions": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "ct_shifted_targets_scratch_bytes": (c_size_t, [c_int32, c_int32]),
     "ct_shifted_targets_and_weights": (c_int32, [c_void_p, POINTER(ShiftedTargetsArgs)]),
     "ct_position_ids": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
@@ -138,6 +139,8 @@ SYMBOLS = {
     "ct_attn_bwd_workspace_bytes": (c_size_t, [c_int32, c_int32, c_int32, c_int32, c_int32]),
     "ct_attn_bwd_workspace_bytes_from_ds": (c_size_t, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "ct_attn_prepare": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
+    "ct_attn_prepare_summaries": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p,
+                                            c_int32, c_void_p, c_int32, c_void_p]),
     "ct_attn_block_summary": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                         c_void_p]),
     "ct_attn_fwd": (c_int32, [c_void_p, POINTER(AttnFwdArgs)]),

@@ -14,286 +14,334 @@
 namespace ct {
 
 // ---------------------------------------------------------------------------
-// Tile bounds. One workgroup per batch row; phase 1 summarises every
-// 32-position block, phase 2 turns the summaries into visit ranges.
+// Tile bounds, in three launches: the summary of every 32-position block; from a row's summaries, what
+// each block has to visit; from those ranges, the work-sorted schedules, the dS offsets and the bins.
+//
+// All of it is latency: the searches and the ranking are quadratic in a row's blocks, and one
+// workgroup per row for everything took 43 us at S = 4096 and 0.6 ms at S = 32768 (its LDS pipe). Now
+// 32 lanes read a block's ids, 16 lanes share the search of a block in a workgroup per 64 blocks, and
+// every schedule has a workgroup of its own, with as many lanes per tile as there are threads for.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void attn_prepare_kernel(const int* seg, const int* end, int S,
-                                                            int* meta, int* sched_all,
-                                                            int* global_scratch) {
-  // [nrb][3]: min_nz, max_id, end_max; later schedule_ints(nrb) work counts. In LDS when the
-  // row fits, else this batch row's part of the scratch region (3 * nrb ints per row).
-  extern __shared__ int lds_meta_shared[];
-  const int b = blockIdx.x;
-  int* lds_meta = global_scratch ? global_scratch + (size_t)b * 3 * (S / 32) : lds_meta_shared;
-  const int nrb = S / 32, nt = S / kKeyTile;
-  const int* segb = seg + (size_t)b * S;
-  const int* endb = end ? end + (size_t)b * S : nullptr;
-  int* mb = meta + (size_t)b * nrb * kMetaW;
-  int* sched = sched_all + (size_t)b * schedule_ints(nrb);
 
-  for (int rb = threadIdx.x; rb < nrb; rb += blockDim.x) {
-    int min_nz = INT_MAX, max_id = 0, end_min = INT_MAX, end_max = -1;
-    const int first_id = segb[rb * 32];
-    bool same = true;
-    for (int i = 0; i < 32; ++i) {
-      const int pos = rb * 32 + i;
-      const int id = segb[pos];
-      same &= (id == first_id);
-      if (id != 0) {
-        min_nz = min(min_nz, id);
-        max_id = max(max_id, id);
-        const int e = endb ? endb[pos] : pos;
-        end_min = min(end_min, e);
-        end_max = max(end_max, e);
-      }
-    }
-    if (max_id == 0) min_nz = 0;  // reference: all-padding block -> (0, 0)
-    int* m = mb + rb * kMetaW;
-    m[kMinNz] = min_nz;
+// Lanes that share one of n work items of a workgroup of `threads` (a power of two, at most 64).
+CT_DEVICE int lanes_per_item(int n, int threads) {
+  int lanes = 1;
+  while (lanes < 64 && lanes * 2 * n <= threads) lanes *= 2;
+  return lanes;
+}
+CT_DEVICE int min_over(int v, int lanes) {
+  for (int off = lanes / 2; off > 0; off /= 2) v = min(v, __shfl_xor(v, off, 64));
+  return v;
+}
+CT_DEVICE int max_over(int v, int lanes) {
+  for (int off = lanes / 2; off > 0; off /= 2) v = max(v, __shfl_xor(v, off, 64));
+  return v;
+}
+CT_DEVICE int sum_over(int v, int lanes) {
+  for (int off = lanes / 2; off > 0; off /= 2) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// grid (ceil(S / 1024), B): 32 consecutive lanes per block
+__global__ __launch_bounds__(1024) void attn_blocks_kernel(const int* seg, const int* end, int S, int* meta) {
+  const int b = blockIdx.y, pos = blockIdx.x * 1024 + threadIdx.x;
+  if (pos >= S) return;  // (S % 128 == 0: whole wavefronts)
+  const int id = seg[(size_t)b * S + pos], e = end ? end[(size_t)b * S + pos] : pos;
+  const bool counts = id != 0;
+  const int low = min_over(counts ? id : INT_MAX, 32), high = max_over(counts ? id : INT_MIN, 32);
+  const int end_min = min_over(counts ? e : INT_MAX, 32), end_max = max_over(counts ? e : -1, 32);
+  const int zeros = 32 - __popcll(__ballot(counts) >> (threadIdx.x & 32) & 0xffffffffull);
+  if (pos % 32 == 0) {
+    const int max_id = max(high, 0);
+    int* m = meta + ((size_t)b * (S / 32) + pos / 32) * kMetaW;
+    m[kMinNz] = max_id == 0 ? 0 : low;  // reference: all-padding block -> (0, 0)
     m[kMaxId] = max_id;
-    m[kUniform] = (same && first_id != 0) ? first_id : 0;
+    m[kUniform] = zeros == 0 && low == high ? low : 0;
     m[kEndMin] = end_min;
     m[kEndMax] = end_max;
-    m[9] = 0;
     m[10] = 0;
     m[11] = 0;
-    lds_meta[rb * 3 + 0] = min_nz;
-    lds_meta[rb * 3 + 1] = max_id;
-    lds_meta[rb * 3 + 2] = end_max;
   }
-  __threadfence();
-  __syncthreads();
+}
 
-  for (int rb = threadIdx.x; rb < nrb; rb += blockDim.x) {
-    const int my_min = lds_meta[rb * 3 + 0], my_max = lds_meta[rb * 3 + 1],
-              my_end = lds_meta[rb * 3 + 2];
-    // As queries: which 64-key tiles?
-    int kv_first = INT_MAX, kv_last = -1;
+// Block summaries in the reference's format (ct_attn_block_summary); `block` = 0: none.
+struct SummaryOut {
+  int* out;
+  int block, width;  // width 3: with the largest visible end
+};
+
+// grid (ceil(nrb / 64), B): 16 lanes per block search what it has to visit; the workgroups of a row also
+// write its block summaries.
+__global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, bool in_lds, SummaryOut queries,
+                                                           SummaryOut keys) {
+  extern __shared__ __align__(16) int lds_rows[];  // [3][nrb]: min_nz, max_id, end_max of the row's blocks
+  const int b = blockIdx.y, nrb = S / 32, nt = S / kKeyTile;
+  int* mb = meta + (size_t)b * nrb * kMetaW;
+  if (in_lds) {
+    for (int i = threadIdx.x; i < nrb; i += 1024) {
+      lds_rows[i] = mb[i * kMetaW + kMinNz];
+      lds_rows[nrb + i] = mb[i * kMetaW + kMaxId];
+      lds_rows[2 * nrb + i] = mb[i * kMetaW + kEndMax];
+    }
+    __syncthreads();
+  }
+  auto min_nz = [&](int i) { return in_lds ? lds_rows[i] : mb[i * kMetaW + kMinNz]; };
+  auto max_id = [&](int i) { return in_lds ? lds_rows[nrb + i] : mb[i * kMetaW + kMaxId]; };
+  auto end_max = [&](int i) { return in_lds ? lds_rows[2 * nrb + i] : mb[i * kMetaW + kEndMax]; };
+
+  constexpr int kLanes = 16;
+  const int lane = threadIdx.x % kLanes, rb = blockIdx.x * (1024 / kLanes) + threadIdx.x / kLanes;
+  if (rb < nrb) {
+    const int my_min = min_nz(rb), my_max = max_id(rb), my_end = end_max(rb);
+    int kv_first = INT_MAX, kv_last = -1, q_first = INT_MAX, q_last = -1;
     if (my_min != 0) {
+      // As queries: which 64-key tiles?
       const int t_hi = min(my_end / kKeyTile, nt - 1);
-      for (int t = 0; t <= t_hi; ++t) {
-        const int a_min = lds_meta[(2 * t) * 3], c_min = lds_meta[(2 * t + 1) * 3];
+      for (int t = lane; t <= t_hi; t += kLanes) {
+        const int a_min = min_nz(2 * t), c_min = min_nz(2 * t + 1);
         const int k_min = a_min == 0 ? c_min : (c_min == 0 ? a_min : min(a_min, c_min));
-        const int k_max = max(lds_meta[(2 * t) * 3 + 1], lds_meta[(2 * t + 1) * 3 + 1]);
+        const int k_max = max(max_id(2 * t), max_id(2 * t + 1));
         if (blocks_interact(my_min, my_max, my_end, k_min, k_max, t * kKeyTile)) {
           kv_first = min(kv_first, t);
           kv_last = t;
         }
       }
-    }
-    // As keys: which 32-row query blocks?
-    int q_first = INT_MAX, q_last = -1;
-    if (my_min != 0) {
-      for (int qb = 0; qb < nrb; ++qb) {
-        if (blocks_interact(lds_meta[qb * 3], lds_meta[qb * 3 + 1], lds_meta[qb * 3 + 2], my_min,
-                            my_max, rb * 32)) {
+      // As keys: which 32-row query blocks?
+      for (int qb = lane; qb < nrb; qb += kLanes) {
+        if (blocks_interact(min_nz(qb), max_id(qb), end_max(qb), my_min, my_max, rb * 32)) {
           q_first = min(q_first, qb);
           q_last = qb;
         }
       }
     }
-    int* m = mb + rb * kMetaW;
-    m[kKvFirst] = kv_first;
-    m[kKvLast] = kv_last;
-    m[kQFirst] = q_first;
-    m[kQLast] = q_last;
-  }
-  __threadfence();  // the table and (for long rows) the scratch arrays are re-read through global memory
-  __syncthreads();
-
-  // Where the dS blocks of each key block start (kDsOff): exclusive prefix sum of the lengths of
-  // the query-block ranges. Every thread sums a contiguous run of row blocks, the runs are
-  // scanned across the workgroup, and each thread then walks its run again.
-  {
-    __shared__ long long scan_buf[1024];
-    const int per = (nrb + (int)blockDim.x - 1) / (int)blockDim.x;
-    const int lo = min(nrb, (int)threadIdx.x * per), hi = min(nrb, lo + per);
-    auto pairs_of = [&](int rb) {
-      const int* m = mb + rb * kMetaW;
-      return m[kQLast] >= m[kQFirst] ? (long long)(m[kQLast] - m[kQFirst] + 1) : 0ll;
-    };
-    long long local = 0;
-    for (int rb = lo; rb < hi; ++rb) local += pairs_of(rb);
-    scan_buf[threadIdx.x] = local;
-    __syncthreads();
-    for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-      const long long below = (int)threadIdx.x >= off ? scan_buf[threadIdx.x - off] : 0ll;
-      __syncthreads();
-      scan_buf[threadIdx.x] += below;
-      __syncthreads();
-    }
-    long long run = scan_buf[threadIdx.x] - local;
-    for (int rb = lo; rb < hi; ++rb) {
-      mb[rb * kMetaW + kDsOff] = (int)min(run, (long long)INT_MAX);
-      run += pairs_of(rb);
+    kv_first = min_over(kv_first, kLanes);
+    kv_last = max_over(kv_last, kLanes);
+    q_first = min_over(q_first, kLanes);
+    q_last = max_over(q_last, kLanes);
+    if (lane == 0) {
+      int* m = mb + rb * kMetaW;
+      m[kKvFirst] = kv_first;
+      m[kKvLast] = kv_last;
+      m[kQFirst] = q_first;
+      m[kQLast] = q_last;
     }
   }
 
-  // Phase 3: amount of work per tile, for the four schedules, into LDS (the
-  // summaries are no longer needed): [0, nrb) query tiles of 1 row block,
-  // then tiles of 2, of 4, then 128-key tiles.
-  int* work = lds_meta;
-  const int off2 = nrb, off4 = nrb + nrb / 2, offk = nrb + nrb / 2 + nrb / 4;
-  for (int i = threadIdx.x; i < nrb; i += blockDim.x) {
-    const int* m = mb + i * kMetaW;
-    work[i] = m[kKvLast] >= m[kKvFirst] ? m[kKvLast] - m[kKvFirst] + 1 : 0;
-  }
-  for (int pb = 2; pb <= 4; pb *= 2) {
-    int* dst = work + (pb == 2 ? off2 : off4);
-    for (int i = threadIdx.x; i < nrb / pb; i += blockDim.x) {
-      int first = INT_MAX, last = -1;
-      for (int k = 0; k < pb; ++k) {
-        const int* m = mb + (i * pb + k) * kMetaW;
-        first = min(first, m[kKvFirst]);
-        last = max(last, m[kKvLast]);
+  for (int side = 0; side < 2; ++side) {
+    const SummaryOut& summary = side ? keys : queries;
+    if (!summary.block) continue;
+    const int per = summary.block / 32, count = S / summary.block, groups = 1024 / kLanes;
+    for (int i = blockIdx.x * groups + threadIdx.x / kLanes; i < count; i += gridDim.x * groups) {
+      int low = INT_MAX, high = 0, last = 0;
+      for (int k = i * per + lane; k < (i + 1) * per; k += kLanes) {
+        if (min_nz(k) != 0) low = min(low, min_nz(k));
+        high = max(high, max_id(k));
+        last = max(last, end_max(k));
       }
-      dst[i] = last >= first ? last - first + 1 : 0;
-    }
-  }
-  for (int i = threadIdx.x; i < nrb / 4; i += blockDim.x) {
-    int first = INT_MAX, last = -1;
-    for (int k = 0; k < 4; ++k) {
-      const int* m = mb + (i * 4 + k) * kMetaW;
-      first = min(first, m[kQFirst]);
-      last = max(last, m[kQLast]);
-    }
-    work[offk + i] = last >= first ? last - first + 1 : 0;
-  }
-  const int off8 = 2 * nrb, n8 = (nrb + 7) / 8;
-  for (int i = threadIdx.x; i < n8; i += blockDim.x) {
-    int first = INT_MAX, last = -1;
-    for (int k = 0; k < 8 && i * 8 + k < nrb; ++k) {
-      const int* m = mb + (i * 8 + k) * kMetaW;
-      first = min(first, m[kKvFirst]);
-      last = max(last, m[kKvLast]);
-    }
-    work[off8 + i] = last >= first ? last - first + 1 : 0;
-  }
-  __threadfence();
-  __syncthreads();
-
-  // Phase 4: rank sort (descending work, ties by index) -> schedules.
-  const int counts[5] = {nrb, nrb / 2, nrb / 4, nrb / 4, n8};
-  const int offsets[5] = {0, off2, off4, offk, off8};
-  for (int sidx = 0; sidx < 5; ++sidx) {
-    const int n = counts[sidx];
-    const int* wk = work + offsets[sidx];
-    int* out = sched + offsets[sidx];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int wi = wk[i];
-      int rank = 0;
-      for (int k = 0; k < n; ++k) {
-        const int wv = wk[k];
-        rank += (wv > wi) || (wv == wi && k < i);
+      low = min_over(low, kLanes);
+      high = max_over(high, kLanes);
+      last = max_over(last, kLanes);
+      if (lane == 0) {
+        int* out = summary.out + ((size_t)b * count + i) * summary.width;
+        out[0] = high == 0 ? 0 : low;
+        out[1] = high;
+        if (summary.width == 3) out[2] = last;
       }
-      out[rank] = i;
     }
+  }
+}
+
+// Number of the tiles in front of tile i when they are ordered by decreasing work, ties by index;
+// shared by `lanes` lanes (w 16-byte aligned).
+CT_DEVICE int rank_of(const int* w, int n, int i, int lanes) {
+  const int wi = w[i], lane = threadIdx.x % lanes;
+  int rank = 0;
+  auto count = [&](int wv, int k) { rank += (wv > wi) || (wv == wi && k < i); };
+  for (int q = lane; q < n / 4; q += lanes) {
+    const int4 v = reinterpret_cast<const int4*>(w)[q];
+    count(v.x, 4 * q);
+    count(v.y, 4 * q + 1);
+    count(v.z, 4 * q + 2);
+    count(v.w, 4 * q + 3);
+  }
+  for (int k = n / 4 * 4 + lane; k < n; k += lanes) count(w[k], k);
+  return sum_over(rank, lanes);
+}
+// Tiles between the first and the last that row blocks first .. end - 1 have to visit (`from`: kKvFirst or
+// kQFirst, followed by the last).
+CT_DEVICE int visit_span(const int* mb, int first_block, int end_block, int from) {
+  int first = INT_MAX, last = -1;
+  for (int k = first_block; k < end_block; ++k) {
+    first = min(first, mb[k * kMetaW + from]);
+    last = max(last, mb[k * kMetaW + from + 1]);
+  }
+  return last >= first ? last - first + 1 : 0;
+}
+
+// One of the five schedules of a batch row: query tiles of 1, 2, 4 row blocks, 128-key tiles, query
+// tiles of 8.
+CT_DEVICE void build_schedule(int job, const int* mb, int nrb, int* sched, int* work) {
+  const int pb = job == 3 ? 4 : job == 4 ? 8 : 1 << job, n = job == 4 ? (nrb + 7) / 8 : nrb / pb;
+  for (int i = threadIdx.x; i < n; i += 1024)
+    work[i] = visit_span(mb, i * pb, min(nrb, (i + 1) * pb), job == 3 ? kQFirst : kKvFirst);
+  __syncthreads();
+  const int lanes = lanes_per_item(n, 1024);
+  int* out = sched + (job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, pb));
+  for (int i = threadIdx.x / lanes; i < n; i += 1024 / lanes) {
+    const int rank = rank_of(work, n, i, lanes);
+    if (threadIdx.x % lanes == 0) out[rank] = i;
+  }
+}
+
+// Where the dS blocks of each key block of a row start (kDsOff): exclusive prefix sum of the lengths of
+// the query-block ranges. Every thread sums a contiguous run of row blocks, the runs are
+// scanned across the workgroup, and each thread then walks its run again.
+CT_DEVICE void build_ds_offsets(int* mb, int nrb) {
+  __shared__ long long wave_sum[16];
+  const int per = (nrb + 1023) / 1024, lane = threadIdx.x & 63;
+  const int lo = min(nrb, (int)threadIdx.x * per), hi = min(nrb, lo + per);
+  long long local = 0;
+  for (int rb = lo; rb < hi; ++rb) local += visit_span(mb, rb, rb + 1, kQFirst);
+  long long incl = local;
+  for (int off = 1; off < 64; off <<= 1) {
+    const long long below = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += below;
+  }
+  if (lane == 63) wave_sum[threadIdx.x >> 6] = incl;
+  __syncthreads();
+  long long run = incl - local;
+  for (int k = 0; k < (int)threadIdx.x >> 6; ++k) run += wave_sum[k];
+  for (int rb = lo; rb < hi; ++rb) {
+    mb[rb * kMetaW + kDsOff] = (int)min(run, (long long)INT_MAX);
+    run += visit_span(mb, rb, rb + 1, kQFirst);
   }
 }
 
 // Packs the query tiles of the whole batch into kBins bins of near equal work
-// (longest processing time first). One workgroup per tile size (2, 4, 8 row blocks);
-// the greedy pass runs on one wavefront, lane j keeping the load of bin j.
-__global__ __launch_bounds__(1024) void attn_bins_kernel(int* meta, int B, int S,
-                                                         int* global_scratch) {
-  // work[n], order[n], bin_of[n]: in LDS when they fit, else this workgroup's third of the
-  // scratch region (3 * B * tiles(2) ints per workgroup)
-  extern __shared__ int lds_bins_shared[];
-  __shared__ int counts[kBins];
+// (longest processing time first: the heaviest tile left goes to the least loaded bin, ties to the
+// lowest bin), by one workgroup per tile size pb (2, 4, 8 row blocks). lds_bins: 3 ints per tile.
+//
+// The greedy pass is serial, but up to kBins of its steps can be taken together: with the bins ranked
+// by load, the next tiles go to the bins of rank 0, 1, 2, ... until one of those just filled would
+// again be the least loaded. Lane j of one wavefront keeps the load of bin j; a round of up to 32
+// tiles takes about as long as one tile did by a butterfly of 64-bit shuffles (157 -> 20 us for the
+// 256 tiles of four rows of 4096), with the same bins.
+CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
+  __shared__ int start[kBins + 1];
   const int nrb = S / 32;
-  const int pb = 2 << blockIdx.x;
   const int tpr = bin_tiles_per_row(nrb, pb), n = B * tpr;
-  int* lds_bins = global_scratch
-                      ? global_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2)
-                      : lds_bins_shared;
   int* work = lds_bins;
   int* order = lds_bins + n;
-  int* bin_of = lds_bins + 2 * n;
+  int* place = lds_bins + 2 * n;  // first the work in rank order, then (position in its bin) * kBins + bin
   int* region = meta + bin_region_offset(B, nrb, pb);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+  for (int i = threadIdx.x; i < n; i += 1024) {
     const int b = i / tpr, qt = i % tpr;
     const int* mb = meta + (size_t)b * nrb * kMetaW;
-    int first = INT_MAX, last = -1;
-    for (int k = 0; k < pb && qt * pb + k < nrb; ++k) {
-      first = min(first, mb[(qt * pb + k) * kMetaW + kKvFirst]);
-      last = max(last, mb[(qt * pb + k) * kMetaW + kKvLast]);
-    }
     // a tile without keys still costs a launch of the prologue; +3 ~ prologue and store
-    work[i] = (last >= first ? last - first + 1 : 0) + 3;
+    work[i] = visit_span(mb, qt * pb, min(nrb, (qt + 1) * pb), kKvFirst) + 3;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int wi = work[i];
-    int rank = 0;
-    for (int k = 0; k < n; ++k) {
-      const int wv = work[k];
-      rank += (wv > wi) || (wv == wi && k < i);
+  const int lanes = lanes_per_item(n, 1024);
+  for (int i = threadIdx.x / lanes; i < n; i += 1024 / lanes) {
+    const int rank = rank_of(work, n, i, lanes);
+    if (threadIdx.x % lanes == 0) {
+      order[rank] = i;
+      place[rank] = work[i];
     }
-    order[rank] = i;
   }
   __syncthreads();
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    int load = lane < kBins ? 0 : INT_MAX;
-    for (int r = 0; r < n; ++r) {
-      // argmin over lanes (ties to the lowest bin): reduce (load, lane) keys
-      long long key = ((long long)load << 8) | lane;
-      for (int off = 32; off > 0; off >>= 1) {
-        const long long other = __shfl_xor(key, off, 64);
-        key = other < key ? other : key;
+    int load = lane < kBins ? 0 : INT_MAX, count = 0;
+    for (int r = 0; r < n;) {
+      // rank of this lane's bin by (load, bin)
+      int rank = lane < kBins ? 0 : lane;
+#pragma unroll
+      for (int j = 0; j < kBins; ++j) {
+        const int other = __builtin_amdgcn_readlane(load, j);
+        if (lane < kBins) rank += other < load || (other == load && j < lane);
       }
-      const int target = (int)(key & 0xff);
-      const int item = order[r];
-      if (lane == target) {
-        load += work[item];
-        bin_of[r] = target;
+      const bool offered = lane < kBins && r + rank < n;
+      const int filled = offered ? load + place[r + rank] : INT_MAX;
+      // in rank order: the load of the bin of rank k, and the least load among those filled before it
+      const int by_rank = __builtin_amdgcn_ds_permute(rank * 4, load);
+      int least = __builtin_amdgcn_ds_permute(rank * 4, filled);
+      for (int off = 1; off < kBins; off <<= 1) {
+        const int below = __shfl_up(least, off, 64);
+        if (lane >= off) least = min(least, below);
       }
+      least = __shfl_up(least, 1, 64);
+      if (lane == 0) least = INT_MAX;
+      const unsigned long long stop = __ballot(lane >= kBins || r + lane >= n || least <= by_rank);
+      const int taken = __ffsll(stop) - 1;  // at least one: least is INT_MAX at rank 0
+      if (lane < kBins && rank < taken) {
+        load = filled;
+        place[r + rank] = count * kBins + lane;
+        ++count;
+      }
+      r += taken;
+    }
+    if (lane < kBins) {
+      int incl = count;
+      for (int off = 1; off < kBins; off <<= 1) {
+        const int below = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += below;
+      }
+      start[lane] = incl - count;
+      if (lane == kBins - 1) start[kBins] = incl;
     }
   }
   __syncthreads();
-  // offsets by counting, then a stable scatter in rank order (heaviest first inside a bin)
-  if (threadIdx.x < kBins) {
-    int count = 0;
-    for (int r = 0; r < n; ++r) count += bin_of[r] == (int)threadIdx.x;
-    counts[threadIdx.x] = count;
+  // in rank order inside a bin: heaviest first
+  if (threadIdx.x <= kBins) region[threadIdx.x] = start[threadIdx.x];
+  for (int r = threadIdx.x; r < n; r += 1024)
+    region[kBins + 1 + start[place[r] % kBins] + place[r] / kBins] = order[r];
+}
+
+// grid: the bins' three workgroups (they take longest), then six per batch row: its schedules and dS
+// offsets. Working arrays in LDS when they fit, else in the scratch region of the metadata buffer.
+__global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, int S, int* sched_all, int* row_scratch,
+                                                              int* bins_scratch) {
+  extern __shared__ __align__(16) int lds_work[];
+  const int nrb = S / 32;
+  if (blockIdx.x < 3) {
+    const int pb = 2 << blockIdx.x;
+    build_bins(meta, B, S, pb, bins_scratch ? bins_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2) : lds_work);
+    return;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int j = 0; j < kBins; ++j) {
-      region[j] = run;
-      run += counts[j];
-    }
-    region[kBins] = run;
-  }
-  __syncthreads();
-  if (threadIdx.x < kBins) {
-    int pos = region[threadIdx.x];
-    for (int r = 0; r < n; ++r)
-      if (bin_of[r] == (int)threadIdx.x) region[kBins + 1 + pos++] = order[r];
+  const int b = (blockIdx.x - 3) / 6, job = (blockIdx.x - 3) % 6;
+  int* mb = meta + (size_t)b * nrb * kMetaW;
+  if (job == 5) {
+    build_ds_offsets(mb, nrb);
+  } else {
+    const int offset = job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, job == 4 ? 8 : 1 << job);
+    build_schedule(job, mb, nrb, sched_all + (size_t)b * schedule_ints(nrb),
+                   row_scratch ? row_scratch + (size_t)b * 3 * nrb + offset : lds_work);
   }
 }
 
-__global__ void attn_block_summary_kernel(const int* seg, const int* end, int S, int block,
-                                          int nblocks, int width, int* out) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+// One wavefront per block.
+__global__ __launch_bounds__(256) void attn_block_summary_kernel(const int* seg, const int* end, int block,
+                                                                 int nblocks, int width, int* out) {
+  const int gid = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (gid >= nblocks) return;
-  const int per_row = S / block;
-  const int b = gid / per_row, blk = gid % per_row;
-  const int* segb = seg + (size_t)b * S + (size_t)blk * block;
-  int min_nz = INT_MAX, max_id = 0, end_max = 0;
-  for (int i = 0; i < block; ++i) {
-    const int id = segb[i];
+  const size_t first = (size_t)gid * block;
+  int low = INT_MAX, high = 0, last = 0;
+  for (int i = lane; i < block; i += 64) {
+    const int id = seg[first + i];
     if (id != 0) {
-      min_nz = min(min_nz, id);
-      max_id = max(max_id, id);
+      low = min(low, id);
+      high = max(high, id);
+      if (end) last = max(last, end[first + i]);
     }
-    if (end) end_max = max(end_max, id != 0 ? end[(size_t)b * S + (size_t)blk * block + i] : 0);
   }
-  if (max_id == 0) min_nz = 0;
-  out[(size_t)gid * width + 0] = min_nz;
-  out[(size_t)gid * width + 1] = max_id;
-  if (end) out[(size_t)gid * width + 2] = end_max;
+  low = min_over(low, 64);
+  high = max_over(high, 64);
+  last = max_over(last, 64);
+  if (lane != 0) return;
+  out[(size_t)gid * width + 0] = high == 0 ? 0 : low;
+  out[(size_t)gid * width + 1] = high;
+  if (end) out[(size_t)gid * width + 2] = last;
 }
 
 static float round_to_bf16(float x) {
@@ -532,11 +580,10 @@ extern "C" size_t ct_attn_bwd_workspace_bytes_from_ds(int32_t batch, int32_t seq
   return plan.spill ? plan.total : 0;
 }
 
-extern "C" int32_t ct_attn_prepare(void* stream, const int32_t* segment_ids,
-                                   const int32_t* attention_end, int32_t batch, int32_t seq,
-                                   int32_t* tile_meta) {
-  CT_REQUIRE(segment_ids && tile_meta, "ct_attn_prepare: null pointer");
-  int rc = validate_shape("ct_attn_prepare", batch, seq, 1, 1, 128);
+static int32_t prepare_on(const char* fn, void* stream, const int32_t* segment_ids, const int32_t* attention_end,
+                          int32_t batch, int32_t seq, int32_t* tile_meta, SummaryOut queries, SummaryOut keys) {
+  CT_REQUIRE(segment_ids && tile_meta, "%s: null pointer", fn);
+  int rc = validate_shape(fn, batch, seq, 1, 1, 128);
   if (rc) return rc;
   const int nrb = seq / 32;
   // working arrays: LDS when they fit, else the scratch region after the table
@@ -547,30 +594,42 @@ extern "C" int32_t ct_attn_prepare(void* stream, const int32_t* segment_ids,
     scratch += (size_t)batch * 3 * nrb;
   }
   int* bins_scratch = bins_fit_lds(batch, nrb) ? nullptr : scratch;
-  const size_t smem = prepare_scratch ? 0 : (size_t)nrb * 3 * sizeof(int);
-  {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prepare_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       kPrepareLdsRowBlocks * 3 * 4);
-    if (e != hipSuccess) return fail(CT_LAUNCH_FAILED, "ct_attn_prepare: %s", hipGetErrorString(e));
-  }
-  const int threads = nrb >= 1024 ? 1024 : ((nrb + 63) / 64) * 64;
-  LaunchScope scope5("attn_prepare_kernel", (hipStream_t)stream);
-  hipLaunchKernelGGL(attn_prepare_kernel, dim3(batch), dim3(threads), smem, (hipStream_t)stream,
-                     segment_ids, attention_end, seq, tile_meta,
-                     tile_meta + (size_t)batch * nrb * kMetaW, prepare_scratch);
-  rc = scope5.done();
-  if (rc) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  LaunchScope scope5("attn_blocks_kernel", st);
+  hipLaunchKernelGGL(attn_blocks_kernel, dim3((seq + 1023) / 1024, batch), dim3(1024), 0, st, segment_ids, attention_end, seq,
+                     tile_meta);
+  if ((rc = scope5.done())) return rc;
+  CT_ENSURE_LDS(fn, &attn_ranges_kernel, kPrepareLdsRowBlocks * 3 * 4);
+  LaunchScope scope6("attn_ranges_kernel", st);
+  hipLaunchKernelGGL(attn_ranges_kernel, dim3((nrb + 63) / 64, batch), dim3(1024),
+                     prepare_scratch ? 0 : (size_t)nrb * 3 * sizeof(int), st, tile_meta, seq, prepare_scratch == nullptr,
+                     queries, keys);
+  if ((rc = scope6.done())) return rc;
   const size_t bins_smem = bins_scratch ? 0 : (size_t)3 * batch * bin_tiles_per_row(nrb, 2) * sizeof(int);
-  {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bins_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBinsLdsInts * 4);
-    if (e != hipSuccess) return fail(CT_LAUNCH_FAILED, "ct_attn_prepare: %s", hipGetErrorString(e));
-  }
-  LaunchScope scope8("attn_bins_kernel", (hipStream_t)stream);
-  hipLaunchKernelGGL(attn_bins_kernel, dim3(3), dim3(1024), bins_smem, (hipStream_t)stream, tile_meta,
-                     batch, seq, bins_scratch);
+  const size_t row_smem = prepare_scratch ? 0 : (size_t)nrb * sizeof(int);
+  CT_ENSURE_LDS(fn, &attn_schedules_kernel, kBinsLdsInts * 4);
+  LaunchScope scope8("attn_schedules_kernel", st);
+  hipLaunchKernelGGL(attn_schedules_kernel, dim3(3 + 6 * batch), dim3(1024), bins_smem > row_smem ? bins_smem : row_smem, st,
+                     tile_meta, batch, seq, tile_meta + (size_t)batch * nrb * kMetaW, prepare_scratch, bins_scratch);
   return scope8.done();
+}
+
+extern "C" int32_t ct_attn_prepare(void* stream, const int32_t* segment_ids,
+                                   const int32_t* attention_end, int32_t batch, int32_t seq,
+                                   int32_t* tile_meta) {
+  return prepare_on("ct_attn_prepare", stream, segment_ids, attention_end, batch, seq, tile_meta, SummaryOut{}, SummaryOut{});
+}
+
+extern "C" int32_t ct_attn_prepare_summaries(void* stream, const int32_t* segment_ids, const int32_t* attention_end,
+                                             int32_t batch, int32_t seq, int32_t* tile_meta, int32_t block_q,
+                                             int32_t* q_summary, int32_t block_kv, int32_t* kv_summary) {
+  CT_REQUIRE(q_summary && kv_summary, "ct_attn_prepare_summaries: null pointer");
+  CT_REQUIRE(block_q > 0 && block_q % 32 == 0 && block_kv > 0 && block_kv % 32 == 0 && seq > 0 && seq % block_q == 0 &&
+                 seq % block_kv == 0,
+             "ct_attn_prepare_summaries: blocks %d and %d must be multiples of 32 that divide the sequence %d", block_q,
+             block_kv, seq);
+  return prepare_on("ct_attn_prepare_summaries", stream, segment_ids, attention_end, batch, seq, tile_meta,
+                    SummaryOut{q_summary, block_q, attention_end ? 3 : 2}, SummaryOut{kv_summary, block_kv, 2});
 }
 
 extern "C" int32_t ct_attn_block_summary(void* stream, const int32_t* segment_ids,
@@ -582,8 +641,8 @@ extern "C" int32_t ct_attn_block_summary(void* stream, const int32_t* segment_id
              block);
   const int nblocks = batch * (seq / block);
   LaunchScope scope6("attn_block_summary_kernel", (hipStream_t)stream);
-  hipLaunchKernelGGL(attn_block_summary_kernel, dim3((nblocks + 127) / 128), dim3(128), 0,
-                     (hipStream_t)stream, segment_ids, attention_end, seq, block, nblocks,
+  hipLaunchKernelGGL(attn_block_summary_kernel, dim3((nblocks + 3) / 4), dim3(256), 0,
+                     (hipStream_t)stream, segment_ids, attention_end, block, nblocks,
                      attention_end ? 3 : 2, out);
   return scope6.done();
 }

@@ -93,7 +93,7 @@ __host__ __device__ inline size_t bin_region_offset(int B, int nrb, int pb) {
 // query tiles in the batch) use a scratch region at the end of the caller's metadata buffer
 // instead, so the buffer is only longer for the shapes that need it.
 constexpr int kPrepareLdsRowBlocks = 8192;              // 96 KB of LDS
-constexpr int kBinsLdsInts = (160 * 1024 - 1024) / 4;   // what attn_bins_kernel may take
+constexpr int kBinsLdsInts = (160 * 1024 - 1024) / 4;   // what attn_schedules_kernel may take
 __host__ __device__ inline size_t meta_table_ints(int B, int nrb) {
   return bin_region_offset(B, nrb, 8) + bin_region_ints(B, nrb, 8);
 }

@@ -9,62 +9,70 @@
 
 namespace ct {
 
-// One workgroup per batch row. ids[s] = number of run starts in [0, s] where position s is
-// valid, else 0; a run starts at a valid position whose predecessor is invalid or carries a
-// different label (position 0 compares its label with itself, as the reference does).
-// VALID_IS_ONE: a position is valid iff mask == 1 (the loss path), else iff mask != 0.
-template <bool VALID_IS_ONE>
-__global__ __launch_bounds__(1024) void canonicalize_kernel(const int* mask, const int* labels,
-                                                            int S, int* out) {
-  __shared__ int wave_sums[16];
-  __shared__ int carry_s;
+// One workgroup per batch row, kScanPer consecutive positions per thread and pass. A run starts at a
+// valid position (mask != 0) whose predecessor is invalid or carries a different label (position 0
+// compares its label with itself, as the reference does).
+// POSITIONS = false: out[s] = number of run starts in [0, s] where s is valid, else 0;
+// POSITIONS = true:  out[s] = s - the latest run start where s is valid, else 0.
+// The time is that of the passes' chains (load, scan in the wavefront, exchange, store): 4096 positions
+// take one pass.
+constexpr int kScanPer = 4;
+template <bool POSITIONS>
+__global__ __launch_bounds__(1024) void segment_scan_kernel(const int* mask, const int* labels, int S, int* out) {
+  __shared__ int wave_total[2][16];
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nwaves = blockDim.x >> 6;
-  const int* mrow = mask ? mask + (size_t)b * S : nullptr;
+  const int* mrow = mask + (size_t)b * S;
   const int* lrow = labels ? labels + (size_t)b * S : nullptr;
   int* orow = out + (size_t)b * S;
-  auto valid_at = [&](int s) {
-    if (!mrow) return true;
-    return VALID_IS_ONE ? mrow[s] == 1 : mrow[s] != 0;
-  };
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (int base = 0; base < S; base += blockDim.x) {
-    const int s = base + tid;
-    bool valid = false, start = false;
-    if (s < S) {
-      valid = valid_at(s);
-      const bool prev_valid = s > 0 && valid_at(s - 1);
-      const int label = lrow ? lrow[s] : 0;
-      const int prev_label = lrow ? lrow[s > 0 ? s - 1 : 0] : 0;
-      start = valid && (!prev_valid || label != prev_label);
+  int carry = 0;  // of the passes before: run starts so far / the latest start
+  for (int base = 0, pass = 0; base < S; base += blockDim.x * kScanPer, ++pass) {
+    const int s0 = base + tid * kScanPer;
+    int m[kScanPer + 1], l[kScanPer + 1];
+#pragma unroll
+    for (int k = 0; k <= kScanPer; ++k) {
+      const int s = s0 + k - 1;
+      const bool in = s >= 0 && s < S;
+      m[k] = in ? mrow[s] : 0;
+      l[k] = lrow && in ? lrow[s] : 0;
     }
-    // inclusive scan of `start` over the workgroup
-    int incl = start ? 1 : 0;
+    int run[kScanPer], mine = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+      const bool start = m[k + 1] != 0 && (m[k] == 0 || l[k + 1] != l[k]);
+      mine = POSITIONS ? max(mine, start ? s0 + k : 0) : mine + start;
+      run[k] = mine;
+    }
+    int incl = mine;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int other = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += other;
+      if (lane >= off) incl = POSITIONS ? max(incl, other) : incl + other;
     }
-    if (lane == 63) wave_sums[wave] = incl;
+    int* total = wave_total[pass & 1];  // (two of them: one barrier per pass)
+    if (lane == 63) total[wave] = incl;
     __syncthreads();
-    int before = carry_s;
-    for (int k = 0; k < wave; ++k) before += wave_sums[k];
-    if (s < S) orow[s] = valid ? before + incl : 0;
-    __syncthreads();
-    if (tid == 0) {
-      int total = carry_s;
-      for (int k = 0; k < nwaves; ++k) total += wave_sums[k];
-      carry_s = total;
+    int before = carry;
+    for (int k = 0; k < nwaves; ++k) {
+      if (k < wave) before = POSITIONS ? max(before, total[k]) : before + total[k];
+      carry = POSITIONS ? max(carry, total[k]) : carry + total[k];
     }
-    __syncthreads();
+    const int left = __shfl_up(incl, 1, 64);
+    if (lane) before = POSITIONS ? max(before, left) : before + left;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+      const int value = POSITIONS ? s0 + k - max(before, run[k]) : before + run[k];
+      if (s0 + k < S) orow[s0 + k] = m[k + 1] != 0 ? value : 0;
+    }
   }
 }
 
 // targets[b, s] = labels[b, s + 1] where the weight is positive, else 0;
 // weights[b, s] = valid edge * assistant[s + 1] * loss_mask[s + 1]  (f32 products in that order).
+// Two neighbours lie in the same canonical run iff both are valid (mask == 1 here, not != 0:
+// src/training/losses.py:52) and carry the same label, so no run ids are needed.
 __global__ __launch_bounds__(256) void shifted_targets_kernel(
-    const int* input_ids, const int* labels, const int* mask, const int* canonical,
+    const int* input_ids, const int* labels, const int* mask, const int* segments,
     const int* assistant, const float* loss_mask, int ignore_index, int B, int S, int* targets,
     float* weights) {
   const long gid = (long)blockIdx.x * 256 + threadIdx.x;
@@ -76,7 +84,7 @@ __global__ __launch_bounds__(256) void shifted_targets_kernel(
   const int target = lab[next];
   bool valid = target != ignore_index;
   if (mask) valid = valid && mask[here] == 1 && mask[next] == 1;
-  if (canonical) valid = valid && canonical[here] == canonical[next] && canonical[next] != 0;
+  if (segments) valid = valid && segments[here] == segments[next];
   float w = valid ? 1.f : 0.f;
   if (assistant) w *= (assistant[next] != 0) ? 1.f : 0.f;
   if (loss_mask) w *= loss_mask[next];
@@ -90,6 +98,15 @@ static int check_dims(const char* fn, int batch, int seq) {
   return CT_OK;
 }
 
+template <bool POSITIONS>
+static int launch_segment_scan(hipStream_t stream, const char* name, const int* mask, const int* labels, int batch, int seq,
+                               int* out) {
+  const int needed = (seq + kScanPer - 1) / kScanPer, threads = needed >= 1024 ? 1024 : ((needed + 63) / 64) * 64;
+  LaunchScope scope(name, stream);
+  hipLaunchKernelGGL((segment_scan_kernel<POSITIONS>), dim3(batch), dim3(threads), 0, stream, mask, labels, seq, out);
+  return scope.done();
+}
+
 }  // namespace ct
 
 using namespace ct;
@@ -100,16 +117,23 @@ extern "C" int32_t ct_canonicalize_segment_ids(void* stream, const int32_t* atte
   CT_REQUIRE(attention_mask && canonical_ids, "ct_canonicalize_segment_ids: null pointer");
   int rc = check_dims("ct_canonicalize_segment_ids", batch, seq);
   if (rc) return rc;
-  const int threads = seq >= 1024 ? 1024 : ((seq + 63) / 64) * 64;
-  LaunchScope scope("canonicalize_kernel", (hipStream_t)stream);
-  hipLaunchKernelGGL((canonicalize_kernel<false>), dim3(batch), dim3(threads), 0, (hipStream_t)stream,
-                     attention_mask, segment_ids, seq, canonical_ids);
-  return scope.done();
+  return launch_segment_scan<false>((hipStream_t)stream, "canonicalize_kernel", attention_mask, segment_ids, batch, seq,
+                                    canonical_ids);
+}
+
+extern "C" int32_t ct_segment_positions(void* stream, const int32_t* attention_mask, const int32_t* segment_ids,
+                                        int32_t batch, int32_t seq, int32_t* position_ids) {
+  CT_REQUIRE(attention_mask && position_ids, "ct_segment_positions: null pointer");
+  int rc = check_dims("ct_segment_positions", batch, seq);
+  if (rc) return rc;
+  return launch_segment_scan<true>((hipStream_t)stream, "segment_positions_kernel", attention_mask, segment_ids, batch, seq,
+                                   position_ids);
 }
 
 extern "C" size_t ct_shifted_targets_scratch_bytes(int32_t batch, int32_t seq) {
-  if (batch <= 0 || seq <= 0) return 0;
-  return (size_t)batch * seq * sizeof(int32_t);
+  (void)batch;
+  (void)seq;
+  return 0;  // (the kernel compares neighbours and needs none)
 }
 
 extern "C" int32_t ct_shifted_targets_and_weights(void* stream_, const ct_shifted_targets_args* a) {
@@ -120,23 +144,10 @@ extern "C" int32_t ct_shifted_targets_and_weights(void* stream_, const ct_shifte
   CT_REQUIRE(a->seq >= 2, "ct_shifted_targets_and_weights: sequence length %d leaves no prediction edge",
              a->seq);
   hipStream_t stream = (hipStream_t)stream_;
-  int* canonical = nullptr;
-  if (a->segment_ids) {
-    CT_REQUIRE(a->scratch && a->scratch_bytes >= ct_shifted_targets_scratch_bytes(a->batch, a->seq),
-               "ct_shifted_targets_and_weights: scratch of %zu bytes needed with segment ids",
-               ct_shifted_targets_scratch_bytes(a->batch, a->seq));
-    canonical = static_cast<int*>(a->scratch);
-    const int threads = a->seq >= 1024 ? 1024 : ((a->seq + 63) / 64) * 64;
-    LaunchScope scope1("canonicalize_kernel", stream);
-    // validity for the loss is "mask == 1" (src/training/losses.py:52), not "mask != 0"
-    hipLaunchKernelGGL((canonicalize_kernel<true>), dim3(a->batch), dim3(threads), 0, stream,
-                       a->attention_mask, a->segment_ids, a->seq, canonical);
-    if ((rc = scope1.done())) return rc;
-  }
   const long total = (long)a->batch * (a->seq - 1);
   LaunchScope scope2("shifted_targets_kernel", stream);
   hipLaunchKernelGGL(shifted_targets_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
-                     a->input_ids, a->labels, a->attention_mask, canonical, a->assistant_mask,
+                     a->input_ids, a->labels, a->attention_mask, a->segment_ids, a->assistant_mask,
                      a->loss_mask, a->ignore_index, a->batch, a->seq, a->targets, a->weights);
   return scope2.done();
 }

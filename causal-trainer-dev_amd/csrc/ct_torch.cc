@@ -579,13 +579,14 @@ MaybeTensor canonical_ids(const Tensor& mask, const MaybeTensor& labels) {
   return out;
 }
 
-MaybeTensor position_ids(const Tensor& mask, const Tensor& canonical) {
-  if (!plain(mask, at::kInt, 2) || !plain(canonical, at::kInt, 2) || mask.numel() == 0 || canonical.sizes() != mask.sizes())
+// positions inside the runs of (mask, labels)
+MaybeTensor segment_positions(const Tensor& mask, const MaybeTensor& labels) {
+  if (!plain(mask, at::kInt, 2) || mask.numel() == 0 || (labels && (!plain(*labels, at::kInt, 2) || labels->sizes() != mask.sizes())))
     return std::nullopt;
   const c10::DeviceGuard guard(mask.device());
   Tensor out = ints(mask.sizes(), mask);
-  check(ct_position_ids(current_stream(), ptr<int32_t>(mask), ptr<int32_t>(canonical), (int32_t)mask.size(0),
-                        (int32_t)mask.size(1), ptr<int32_t>(out)));
+  check(ct_segment_positions(current_stream(), ptr<int32_t>(mask), ptr<int32_t>(labels), (int32_t)mask.size(0),
+                             (int32_t)mask.size(1), ptr<int32_t>(out)));
   return out;
 }
 
@@ -613,7 +614,7 @@ std::optional<std::tuple<Tensor, Tensor>> shifted_targets(const Tensor& tokens, 
   if (loss_mask && (!plain(*loss_mask, at::kFloat, 2) || loss_mask->sizes() != tokens.sizes())) return std::nullopt;
   const c10::DeviceGuard guard(tokens.device());
   const int64_t batch = tokens.size(0), seq = tokens.size(1);
-  Tensor targets = ints({batch, seq - 1}, tokens), weights = floats({batch, seq - 1}, tokens), work, all_valid;
+  Tensor targets = ints({batch, seq - 1}, tokens), weights = floats({batch, seq - 1}, tokens);
   ct_shifted_targets_args a = {};
   a.input_ids = ptr<int32_t>(tokens);
   a.attention_mask = ptr<int32_t>(mask);
@@ -623,15 +624,6 @@ std::optional<std::tuple<Tensor, Tensor>> shifted_targets(const Tensor& tokens, 
   a.labels = ptr<int32_t>(labels);
   a.targets = ptr<int32_t>(targets);
   a.weights = ptr<float>(weights);
-  if (segments) {
-    if (!mask) {  // every token valid
-      all_valid = at::ones_like(tokens);
-      a.attention_mask = ptr<int32_t>(all_valid);
-    }
-    a.scratch_bytes = ct_shifted_targets_scratch_bytes((int32_t)batch, (int32_t)seq);
-    work = scratch(a.scratch_bytes, tokens);
-    a.scratch = work.data_ptr();
-  }
   a.batch = (int32_t)batch;
   a.seq = (int32_t)seq;
   a.ignore_index = (int32_t)ignore_index;
@@ -647,6 +639,11 @@ std::tuple<Tensor, Tensor, Tensor> attention_metadata(const Tensor& segments, co
   Tensor bounds = ints({(int64_t)(ct_attn_meta_bytes(batch, seq) / 4)}, segments);
   Tensor q_summary = ints({batch, seq / block_q, ends ? 3 : 2}, segments), kv_summary = ints({batch, seq / block_kv, 2}, segments);
   void* stream = current_stream();
+  if (block_q % 32 == 0 && block_kv % 32 == 0) {
+    check(ct_attn_prepare_summaries(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, ptr<int32_t>(bounds),
+                                    (int32_t)block_q, ptr<int32_t>(q_summary), (int32_t)block_kv, ptr<int32_t>(kv_summary)));
+    return {bounds, q_summary, kv_summary};
+  }
   check(ct_attn_prepare(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, ptr<int32_t>(bounds)));
   check(ct_attn_block_summary(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, (int32_t)block_q,
                               ptr<int32_t>(q_summary)));
@@ -679,7 +676,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("cutce_forward", &cutce_forward);
   m.def("cutce_backward", &cutce_backward);
   m.def("canonical_ids", &canonical_ids);
-  m.def("position_ids", &position_ids);
+  m.def("segment_positions", &segment_positions);
   m.def("rotary_tables", &rotary_tables);
   m.def("shifted_targets", &shifted_targets);
   m.def("attention_metadata", &attention_metadata);

@@ -13,23 +13,9 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .prep import _int32, _nonzero, canonicalize_segment_ids
+from .prep import _int32, _mask_and_labels
 
 _STYLES = {"gpt-j": 0, "gpt-neox": 1}
-
-
-def _make_position_ids_precanonicalized(attention_mask, segment_ids) -> torch.Tensor:
-    mask = torch.as_tensor(attention_mask)
-    if mask.ndim != 2:
-        raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
-    valid = _nonzero(mask, "attention_mask")
-    segments = torch.as_tensor(segment_ids)
-    if tuple(segments.shape) != tuple(valid.shape):
-        raise ValueError(f"segment_ids must have shape {tuple(valid.shape)}, got {tuple(segments.shape)}")
-    segments = _int32(segments, "segment_ids")
-    if valid.numel() == 0:
-        return torch.empty_like(valid)
-    return _lib.native().position_ids(valid, segments)
 
 
 def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
@@ -38,7 +24,10 @@ def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     mask = torch.as_tensor(attention_mask)
     if mask.ndim != 2:
         raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
-    return _make_position_ids_precanonicalized(mask, canonicalize_segment_ids(mask, segment_ids))
+    valid, labels = _mask_and_labels(mask, segment_ids)
+    if valid.numel() == 0:
+        return torch.empty_like(valid)
+    return _lib.native().segment_positions(valid, labels)
 
 
 def rotary_cos_sin(position_ids, inv_freq, dtype=torch.bfloat16):

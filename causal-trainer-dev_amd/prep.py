@@ -21,7 +21,7 @@ def _int32(tensor, name: str, shape=None) -> torch.Tensor:
         raise RuntimeError(f"{name} must live on a ROCm GPU")
     if shape is not None and tuple(tensor.shape) != tuple(shape):
         raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(tensor.shape)}")
-    return tensor.to(torch.int32).contiguous()
+    return tensor.contiguous() if tensor.dtype == torch.int32 else tensor.to(torch.int32).contiguous()
 
 
 def _nonzero(tensor, name: str) -> torch.Tensor:
@@ -31,19 +31,23 @@ def _nonzero(tensor, name: str) -> torch.Tensor:
     return _int32(tensor if tensor.dtype == torch.int32 else tensor != 0, name)
 
 
+def _mask_and_labels(mask, segment_ids):
+    valid = _nonzero(mask, "attention_mask")
+    if segment_ids is None:
+        return valid, None
+    labels = torch.as_tensor(segment_ids)
+    if labels.shape != valid.shape:
+        raise ValueError(f"segment_ids must have shape {tuple(valid.shape)}, got {tuple(labels.shape)}")
+    return valid, _int32(labels, "segment_ids")
+
+
 def canonicalize_segment_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     """One-based ids of contiguous valid runs, zero for padding (int32 ``[batch, sequence]``)."""
 
     mask = torch.as_tensor(attention_mask)
     if mask.ndim != 2:
         raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
-    valid = _nonzero(mask, "attention_mask")
-    labels = None
-    if segment_ids is not None:
-        labels = torch.as_tensor(segment_ids)
-        if tuple(labels.shape) != tuple(valid.shape):
-            raise ValueError(f"segment_ids must have shape {tuple(valid.shape)}, got {tuple(labels.shape)}")
-        labels = _int32(labels, "segment_ids")
+    valid, labels = _mask_and_labels(mask, segment_ids)
     if valid.numel() == 0:
         return torch.empty_like(valid)
     return _lib.native().canonical_ids(valid, labels)

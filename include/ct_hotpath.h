@@ -101,6 +101,16 @@ int32_t ct_attn_block_summary(void* stream, const int32_t* segment_ids,
                               const int32_t* attention_end, int32_t batch, int32_t seq,
                               int32_t block, int32_t* out);
 
+/*
+ * ct_attn_prepare and the block summaries of both sides (ct_attn_block_summary at block_q with
+ * attention_end, and at block_kv without) in the same launches: what prepare_attention_metadata
+ * returns. Both blocks are multiples of 32 that divide seq.
+ */
+int32_t ct_attn_prepare_summaries(void* stream, const int32_t* segment_ids,
+                                  const int32_t* attention_end, int32_t batch, int32_t seq,
+                                  int32_t* tile_meta, int32_t block_q, int32_t* q_summary,
+                                  int32_t block_kv, int32_t* kv_summary);
+
 typedef struct ct_attn_fwd_args {
   const uint16_t* q;            /* bf16 [batch, seq, q_heads, head_dim] */
   const uint16_t* k;            /* bf16 [batch, seq, kv_heads, head_dim] */
@@ -231,6 +241,14 @@ int32_t ct_canonicalize_segment_ids(void* stream, const int32_t* attention_mask,
                                     const int32_t* segment_ids, int32_t batch, int32_t seq,
                                     int32_t* canonical_ids);
 
+/*
+ * position_ids[b, s] = distance of s from the start of its valid run (the runs of
+ * ct_canonicalize_segment_ids), 0 where attention_mask[b, s] == 0: make_position_ids
+ * (src/modeling/rotary.py:63-79) in one pass, without the canonical ids in between.
+ */
+int32_t ct_segment_positions(void* stream, const int32_t* attention_mask, const int32_t* segment_ids,
+                             int32_t batch, int32_t seq, int32_t* position_ids);
+
 typedef struct ct_shifted_targets_args {
   const int32_t* input_ids;       /* int32 [batch, seq] */
   const int32_t* attention_mask;  /* int32 [batch, seq] or NULL (all valid); valid iff == 1 */
@@ -240,7 +258,7 @@ typedef struct ct_shifted_targets_args {
   const int32_t* labels;          /* int32 [batch, seq] or NULL (= input_ids) */
   int32_t* targets;               /* int32 out [batch, seq - 1]; 0 where the weight is not > 0 */
   float* weights;                 /* f32 out [batch, seq - 1] */
-  void* scratch;                  /* ct_shifted_targets_scratch_bytes(), only read with segment_ids */
+  void* scratch;                  /* ct_shifted_targets_scratch_bytes(), now 0: not read */
   size_t scratch_bytes;
   int32_t batch, seq;
   int32_t ignore_index;           /* the reference default is -100 */
