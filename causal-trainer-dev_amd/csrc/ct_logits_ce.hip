@@ -24,17 +24,26 @@ constexpr float kNegInfinity = -__builtin_inff();
 template <class T>
 __device__ __forceinline__ float to_f32(T v) { return (float)v; }
 
-// (m, s): running maximum (log2 domain) and sum of exp2(x log2e - m)
-__device__ __forceinline__ void online_add(float& m, float& s, const float* x, int n) {
-  float cm = kNegInfinity;
-  for (int e = 0; e < n; ++e) cm = fmaxf(cm, x[e]);
+// (m, s): running maximum (log2 domain) and sum of exp2(x log2e - m). The exponents are at most 0, so the
+// bare instruction serves: what it flushes to 0 is below 2^-126 of the sum.
+template <int N>
+__device__ __forceinline__ void online_add(float& m, float& s, const float* x) {
+  float cm = x[0];
+#pragma unroll
+  for (int e = 1; e < N; ++e) cm = fmaxf(cm, x[e]);
   cm *= kLog2eF;
   if (cm > m) {
-    s *= exp2f(m - cm);  // m = -inf: s is 0 and stays 0
+    s *= __builtin_amdgcn_exp2f(m - cm);  // m = -inf: s is 0 and stays 0
     m = cm;
   }
   if (m == kNegInfinity) return;  // only -inf so far
-  for (int e = 0; e < n; ++e) s += exp2f(fmaf(x[e], kLog2eF, -m));
+  float t = 0.f;
+#pragma unroll
+  for (int e = 0; e < N; e += 2) {
+    s += __builtin_amdgcn_exp2f(fmaf(x[e], kLog2eF, -m));
+    if (e + 1 < N) t += __builtin_amdgcn_exp2f(fmaf(x[e + 1], kLog2eF, -m));
+  }
+  s += t;
 }
 __device__ __forceinline__ void online_merge(float& m, float& s, float mo, float so) {
   const float mn = fmaxf(m, mo);
@@ -43,15 +52,44 @@ __device__ __forceinline__ void online_merge(float& m, float& s, float mo, float
   m = mn;
 }
 
+// A row as 16-byte chunks: `head` elements in front of the first aligned address (rows of an odd
+// vocabulary start anywhere), `chunks` chunks, the rest behind them.
+template <class T>
+struct RowChunks {
+  static constexpr int kPer = 16 / sizeof(T);  // elements per chunk
+  int head, chunks;
+  __device__ RowChunks(const T* x, int vocab) {
+    const int off = (int)(reinterpret_cast<uintptr_t>(x) & 15u) / (int)sizeof(T);
+    head = off ? min(vocab, kPer - off) : 0;
+    chunks = (vocab - head) / kPer;
+  }
+};
+template <class T>
+__device__ __forceinline__ void widen(u32x4 raw, float* v) {
+  if constexpr (sizeof(T) == 2) {
+    const bf16x8 b = __builtin_bit_cast(bf16x8, raw);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)b[e];
+  } else {
+    const f32x4 f = __builtin_bit_cast(f32x4, raw);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = f[e];
+  }
+}
+
 // One workgroup per row. valid = target != ignore_index && weight != 0; invalid rows cost no
 // traffic and give loss = lse = 0. A target outside [0, vocab) on a valid row contributes a
 // target logit of 0, as the reference's masked lookup does.
-template <class T>
-__global__ __launch_bounds__(256) void sparse_ce_fwd_kernel(const T* logits, const int* targets,
-                                                            const float* weights, int vocab,
-                                                            int ignore_index, bool vector_ok,
-                                                            float* loss, float* lse) {
-  __shared__ float wm[4], ws[4];
+// Bound by memory: a thread has kUnroll chunks in flight. Aligned or not, a row is read in whole chunks
+// (element by element, as before, the rows of an odd vocabulary ran at 2.2 TB/s).
+constexpr int kUnroll = 4;
+template <class T, int THREADS>
+__global__ __launch_bounds__(THREADS) void sparse_ce_fwd_kernel(const T* logits, const int* targets,
+                                                                const float* weights, int vocab,
+                                                                int ignore_index,
+                                                                float* loss, float* lse) {
+  constexpr int kWaves = THREADS / 64;
+  __shared__ float wm[kWaves], ws[kWaves];
   const long row = blockIdx.x;
   const int tid = threadIdx.x;
   const int target = targets[row];
@@ -65,28 +103,29 @@ __global__ __launch_bounds__(256) void sparse_ce_fwd_kernel(const T* logits, con
   }
   const T* x = logits + (size_t)row * vocab;
   float m = kNegInfinity, s = 0.f;
-  constexpr int kPer = 16 / sizeof(T);  // elements per 16-byte access
-  int done = 0;
-  if (vector_ok) {
-    const int chunks = vocab / kPer;
-    for (int c = tid; c < chunks; c += 256) {
-      float v[kPer];
-      if constexpr (sizeof(T) == 2) {
-        const bf16x8 raw = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x + (size_t)c * kPer));
+  const RowChunks<T> rc(x, vocab);
+  constexpr int kPer = RowChunks<T>::kPer;
+  const u32x4* body = reinterpret_cast<const u32x4*>(x + rc.head);
+  int c = tid;
+  for (; c + (kUnroll - 1) * THREADS < rc.chunks; c += kUnroll * THREADS) {
+    u32x4 raw[kUnroll];
 #pragma unroll
-        for (int e = 0; e < kPer; ++e) v[e] = (float)raw[e];
-      } else {
-        const f32x4 raw = *reinterpret_cast<const f32x4*>(x + (size_t)c * kPer);
+    for (int u = 0; u < kUnroll; ++u) raw[u] = body[c + u * THREADS];
+    float v[kUnroll * kPer];
 #pragma unroll
-        for (int e = 0; e < kPer; ++e) v[e] = raw[e];
-      }
-      online_add(m, s, v, kPer);
-    }
-    done = chunks * kPer;
+    for (int u = 0; u < kUnroll; ++u) widen<T>(raw[u], v + u * kPer);
+    online_add<kUnroll * kPer>(m, s, v);
   }
-  for (int i = done + tid; i < vocab; i += 256) {
-    const float v = to_f32(x[i]);
-    online_add(m, s, &v, 1);
+  for (; c < rc.chunks; c += THREADS) {
+    float v[kPer];
+    widen<T>(body[c], v);
+    online_add<kPer>(m, s, v);
+  }
+  // the elements in front of and behind the chunks: fewer than 2 kPer
+  const int behind = rc.head + rc.chunks * kPer, loose = rc.head + vocab - behind;
+  if (tid < loose) {
+    const float v = to_f32(x[tid < rc.head ? tid : behind + tid - rc.head]);
+    online_add<1>(m, s, &v);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -99,7 +138,7 @@ __global__ __launch_bounds__(256) void sparse_ce_fwd_kernel(const T* logits, con
   }
   __syncthreads();
   if (tid == 0) {
-    for (int k = 1; k < 4; ++k) online_merge(m, s, wm[k], ws[k]);
+    for (int k = 1; k < kWaves; ++k) online_merge(m, s, wm[k], ws[k]);
     const float row_lse = logf(s) + m * kLn2F;
     const float target_logit = (target >= 0 && target < vocab) ? to_f32(x[target]) : 0.f;
     lse[row] = row_lse;
@@ -107,13 +146,15 @@ __global__ __launch_bounds__(256) void sparse_ce_fwd_kernel(const T* logits, con
   }
 }
 
-// grid = (rows, column chunks of 256 * kPer * kIter elements).
+// grid = (rows, parts of kCeBwdChunks chunks of a row).
 // dlogits = w dy (exp(x - lse) - onehot) on valid rows, 0 elsewhere, in the logits dtype.
-template <class T>
+// STREAM: the tensors are too large to be found in a cache again, so reads and writes bypass it.
+constexpr int kCeBwdChunks = 256 * 2 * kUnroll;
+template <class T, bool STREAM>
 __global__ __launch_bounds__(256) void sparse_ce_bwd_kernel(const T* logits, const float* lse,
                                                             const int* targets, const float* weights,
                                                             const float* dy, int vocab, int ignore_index,
-                                                            bool vector_ok, int chunk_elems, T* dlogits) {
+                                                            bool same_alignment, T* dlogits) {
   const long row = blockIdx.x;
   const int tid = threadIdx.x;
   const int target = targets[row];
@@ -123,46 +164,64 @@ __global__ __launch_bounds__(256) void sparse_ce_bwd_kernel(const T* logits, con
   const float lse2 = valid ? lse[row] * kLog2eF : 0.f;
   const T* x = logits + (size_t)row * vocab;
   T* g = dlogits + (size_t)row * vocab;
-  constexpr int kPer = 16 / sizeof(T);
-  const int begin = blockIdx.y * chunk_elems, end = min(vocab, begin + chunk_elems);
+  constexpr int kPer = RowChunks<T>::kPer;
   auto grad = [&](float v, int index) {
-    if (!valid) return 0.f;
     return factor * (exp2f(fmaf(v, kLog2eF, -lse2)) - (index == target ? 1.f : 0.f));
   };
-  int done = begin;
-  if (vector_ok) {  // begin is a multiple of kPer
-    const int chunks = (end - begin) / kPer;
-    for (int c = tid; c < chunks; c += 256) {
-      const int i0 = begin + c * kPer;
-      if constexpr (sizeof(T) == 2) {
-        bf16x8 out;
-        if (valid) {
-          const bf16x8 raw = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x + i0));
+  // (chunks are aligned in dlogits, where they are written; logits aligned another way are read unaligned)
+  const RowChunks<T> rc(g, vocab);
+  const int first = blockIdx.y * kCeBwdChunks, last = min(rc.chunks, first + kCeBwdChunks);
+  auto load = [&](int c) {
+    const T* at = x + rc.head + (size_t)c * kPer;
+    u32x4 raw;
+    if (!same_alignment) __builtin_memcpy(&raw, at, 16);
+    else if (STREAM) raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(at));
+    else raw = *reinterpret_cast<const u32x4*>(at);
+    return raw;
+  };
+  auto store = [&](int c, u32x4 out) {
+    u32x4* at = reinterpret_cast<u32x4*>(g + rc.head + (size_t)c * kPer);
+    if (STREAM) __builtin_nontemporal_store(out, at);
+    else *at = out;
+  };
+  auto gradients = [&](u32x4 raw, int c) {
+    float v[kPer];
+    widen<T>(raw, v);
+    const int i0 = rc.head + c * kPer;
+    if constexpr (sizeof(T) == 2) {
+      bf16x8 out;
 #pragma unroll
-          for (int e = 0; e < kPer; ++e) out[e] = (bf16)grad((float)raw[e], i0 + e);
-        } else {
+      for (int e = 0; e < kPer; ++e) out[e] = (bf16)grad(v[e], i0 + e);
+      return __builtin_bit_cast(u32x4, out);
+    } else {
+      f32x4 out;
 #pragma unroll
-          for (int e = 0; e < kPer; ++e) out[e] = (bf16)0.f;
-        }
-        *reinterpret_cast<u32x4*>(g + i0) = __builtin_bit_cast(u32x4, out);
-      } else {
-        f32x4 out = {0.f, 0.f, 0.f, 0.f};
-        if (valid) {
-          const f32x4 raw = *reinterpret_cast<const f32x4*>(x + i0);
-#pragma unroll
-          for (int e = 0; e < kPer; ++e) out[e] = grad(raw[e], i0 + e);
-        }
-        *reinterpret_cast<f32x4*>(g + i0) = out;
-      }
+      for (int e = 0; e < kPer; ++e) out[e] = grad(v[e], i0 + e);
+      return __builtin_bit_cast(u32x4, out);
     }
-    done = begin + chunks * kPer;
+  };
+  if (!valid) {
+    for (int c = first + tid; c < last; c += 256) store(c, u32x4{0u, 0u, 0u, 0u});
+  } else {
+    int c = first + tid;
+    for (; c + (kUnroll - 1) * 256 < last; c += kUnroll * 256) {
+      u32x4 raw[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) raw[u] = load(c + u * 256);
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) store(c + u * 256, gradients(raw[u], c + u * 256));
+    }
+    for (; c < last; c += 256) store(c, gradients(load(c), c));
   }
-  for (int i = done + tid; i < end; i += 256) g[i] = (T)grad(valid ? to_f32(x[i]) : 0.f, i);
+  const int behind = rc.head + rc.chunks * kPer, loose = rc.head + vocab - behind;
+  if (blockIdx.y == 0 && tid < loose) {
+    const int i = tid < rc.head ? tid : behind + tid - rc.head;
+    g[i] = (T)(valid ? grad(to_f32(x[i]), i) : 0.f);
+  }
 }
 
-constexpr int kCeBwdChunk = 256 * 8 * 8;  // elements of a row per workgroup (a multiple of 8)
-
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// Logits larger than the memory-side cache (256 MB) are not found there by the backward.
+constexpr size_t kStreamBytes = (size_t)384 << 20;
 
 static int check_ce(const char* fn, const ct_sparse_ce_args* a) {
   CT_REQUIRE(a, "%s: null args", fn);
@@ -171,6 +230,8 @@ static int check_ce(const char* fn, const ct_sparse_ce_args* a) {
   CT_REQUIRE(a->logits_dtype == CT_DTYPE_BF16 || a->logits_dtype == CT_DTYPE_F32,
              "%s: logits must be bfloat16 or float32", fn);
   CT_REQUIRE(a->rows <= 0x7fffffffLL, "%s: at most 2^31 - 1 rows", fn);
+  CT_REQUIRE(reinterpret_cast<uintptr_t>(a->logits) % (a->logits_dtype == CT_DTYPE_BF16 ? 2 : 4) == 0,
+             "%s: logits must be aligned to their element size", fn);
   return CT_OK;
 }
 
@@ -183,17 +244,17 @@ extern "C" int32_t ct_sparse_ce_fwd(void* stream_, const ct_sparse_ce_args* a, f
   if (rc) return rc;
   CT_REQUIRE(loss && lse, "ct_sparse_ce_fwd: null output");
   hipStream_t stream = (hipStream_t)stream_;
-  const size_t elem = a->logits_dtype == CT_DTYPE_BF16 ? 2 : 4;
-  const bool vector_ok = aligned16(a->logits) && ((size_t)a->vocab * elem) % 16 == 0;
   LaunchScope scope("sparse_ce_fwd_kernel", stream);
+  // few rows leave compute units without a workgroup: then a row gets four times the threads
+  const bool wide = a->rows <= 512 && a->vocab >= 8192;
+  const auto launch = [&](auto kernel, auto* logits) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)a->rows), dim3(wide ? 1024 : 256), 0, stream, logits, a->targets, a->weights,
+                       a->vocab, a->ignore_index, loss, lse);
+  };
   if (a->logits_dtype == CT_DTYPE_BF16)
-    hipLaunchKernelGGL((sparse_ce_fwd_kernel<bf16>), dim3((unsigned)a->rows), dim3(256), 0, stream,
-                       static_cast<const bf16*>(a->logits), a->targets, a->weights, a->vocab,
-                       a->ignore_index, vector_ok, loss, lse);
+    launch(wide ? sparse_ce_fwd_kernel<bf16, 1024> : sparse_ce_fwd_kernel<bf16, 256>, static_cast<const bf16*>(a->logits));
   else
-    hipLaunchKernelGGL((sparse_ce_fwd_kernel<float>), dim3((unsigned)a->rows), dim3(256), 0, stream,
-                       static_cast<const float*>(a->logits), a->targets, a->weights, a->vocab,
-                       a->ignore_index, vector_ok, loss, lse);
+    launch(wide ? sparse_ce_fwd_kernel<float, 1024> : sparse_ce_fwd_kernel<float, 256>, static_cast<const float*>(a->logits));
   return scope.done();
 }
 
@@ -204,16 +265,19 @@ extern "C" int32_t ct_sparse_ce_bwd(void* stream_, const ct_sparse_ce_args* a, c
   CT_REQUIRE(lse && dy && dlogits, "ct_sparse_ce_bwd: null pointer");
   hipStream_t stream = (hipStream_t)stream_;
   const size_t elem = a->logits_dtype == CT_DTYPE_BF16 ? 2 : 4;
-  const bool vector_ok = aligned16(a->logits) && aligned16(dlogits) && ((size_t)a->vocab * elem) % 16 == 0;
-  const dim3 grid((unsigned)a->rows, (unsigned)((a->vocab + kCeBwdChunk - 1) / kCeBwdChunk));
+  CT_REQUIRE(reinterpret_cast<uintptr_t>(dlogits) % elem == 0, "ct_sparse_ce_bwd: dlogits must be aligned to its element size");
+  const bool same = ((reinterpret_cast<uintptr_t>(a->logits) ^ reinterpret_cast<uintptr_t>(dlogits)) & 15u) == 0;
+  const bool stream_through = (size_t)a->rows * a->vocab * elem > kStreamBytes;
+  const int chunks = (int)(a->vocab * elem / 16);
+  const dim3 grid((unsigned)a->rows, (unsigned)(chunks > kCeBwdChunks ? (chunks + kCeBwdChunks - 1) / kCeBwdChunks : 1));
   LaunchScope scope("sparse_ce_bwd_kernel", stream);
+  const auto launch = [&](auto kernel, auto* out) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<decltype(out)>(const_cast<void*>(a->logits)), lse, a->targets,
+                       a->weights, dy, a->vocab, a->ignore_index, same, out);
+  };
   if (a->logits_dtype == CT_DTYPE_BF16)
-    hipLaunchKernelGGL((sparse_ce_bwd_kernel<bf16>), grid, dim3(256), 0, stream,
-                       static_cast<const bf16*>(a->logits), lse, a->targets, a->weights, dy, a->vocab,
-                       a->ignore_index, vector_ok, kCeBwdChunk, static_cast<bf16*>(dlogits));
+    launch(stream_through ? sparse_ce_bwd_kernel<bf16, true> : sparse_ce_bwd_kernel<bf16, false>, static_cast<bf16*>(dlogits));
   else
-    hipLaunchKernelGGL((sparse_ce_bwd_kernel<float>), grid, dim3(256), 0, stream,
-                       static_cast<const float*>(a->logits), lse, a->targets, a->weights, dy, a->vocab,
-                       a->ignore_index, vector_ok, kCeBwdChunk, static_cast<float*>(dlogits));
+    launch(stream_through ? sparse_ce_bwd_kernel<float, true> : sparse_ce_bwd_kernel<float, false>, static_cast<float*>(dlogits));
   return scope.done();
 }

@@ -104,3 +104,27 @@ def test_argument_errors(ct, gpu):
     out = ct.pallas_fused_sparse_cross_entropy(logits[:, :0], torch.zeros((2, 0), device=gpu),
                                                torch.zeros((2, 0), device=gpu))
     assert out.shape == (2, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab,offset", [(6, 8197, 1), (6, 8197, 3), (3, 5, 2), (700, 2061, 1)])
+def test_rows_at_any_alignment(ct, gpu, dtype, rows, vocab, offset):
+    """Rows that start between 16-byte addresses, and logits aligned differently from their gradient:
+    the loss and the gradient of an aligned copy up to f32 summation order."""
+
+    logits, targets, weights = _case(np.random.default_rng(vocab + offset), rows, vocab, dtype, scale=2.0)
+    storage = torch.empty(rows * vocab + offset, dtype=dtype, device=gpu)
+    x = storage[offset:].view(1, rows, vocab)
+    x.copy_(logits[None])
+    cot = torch.ones(rows)
+    loss, grad = _run(ct, gpu, logits, targets, weights, cot)
+    moved = x.detach().requires_grad_(True)
+    assert moved.data_ptr() % 16 == offset * moved.element_size()
+    got = ct.pallas_fused_sparse_cross_entropy(moved, targets.to(gpu)[None], weights.to(gpu)[None], mesh=None)
+    got.backward(cot.to(gpu)[None])
+    torch.testing.assert_close(got[0].detach().cpu(), loss, rtol=1e-5, atol=1e-5)
+    # the gradients differ by what the last bits of lse make of them: 2^-22 relative on a probability
+    unit = 2.0 ** -7 if dtype == torch.bfloat16 else 1e-5
+    assert bool(((moved.grad[0].cpu().float() - grad.float()).abs() <= unit * grad.float().abs() + 1e-7).all())
+    want = cutce_ref.pallas_sparse_cross_entropy(logits, targets, weights)[0]
+    torch.testing.assert_close(loss, want, rtol=1e-5, atol=1e-5)
