@@ -14,13 +14,12 @@ namespace ct {
 
 typedef __bf16 bf16;
 typedef bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 __device__ __forceinline__ u32x4 as_u32x4(bf16x8 v) { return __builtin_bit_cast(u32x4, v); }
-__device__ __forceinline__ bf16x4 as_bf16x4(u32x2 v) { return __builtin_bit_cast(bf16x4, v); }
 
 // One workgroup per batch row. A run starts at a valid position whose canonical id differs
 // from its predecessor's or whose predecessor's id is 0 (position 0: predecessor id 0);
@@ -84,97 +83,92 @@ __device__ __forceinline__ bf16 scaled(bf16 v, float s, bool on) {
   return on ? (bf16)((float)v * s) : v;
 }
 
-// One thread per 16-byte chunk (8 channels) of a (token, head) row; Q heads first, then K
-// heads. ADJACENT: pairs (2i, 2i+1), a chunk holds 4 pairs. Otherwise pairs (i, i + R/2): the
-// threads of the first half of the rotated channels also handle the partner chunk, those of
-// the second half do nothing. Channels past the rotated ones are copied (and scaled).
+// Rotary embedding in 16-byte chunks. A work item is one chunk (8 channels) of a head, Q heads first,
+// then K heads, for TOKENS consecutive tokens. ADJACENT: pairs (2i, 2i+1), a chunk holds 4 pairs. Otherwise
+// pairs (i, i + R/2): the item of a rotated chunk in the first half also handles the partner chunk, and
+// the chunks of the second half are no items. Channels past the rotated ones are copied (and scaled).
 // forward: out = bf16(bf16(R x) * s); inverse: out = bf16(R^T bf16(x * s)). The rotation is
 // evaluated in f32 from the bf16 operands and rounded once.
-template <bool ADJACENT>
-__device__ __forceinline__ void apply_rotary_chunk(const ct_rotary_args& a, long t, int h, int c);
-
-// One workgroup per token walks the (head, chunk) pairs of that token: no 64-bit index
-// arithmetic per chunk, and the token's cos / sin row is shared by the whole workgroup.
-template <bool ADJACENT>
-__global__ __launch_bounds__(256) void apply_rotary_kernel(ct_rotary_args a) {
-  const int cpr = a.head_dim / 8;  // chunks per head row
-  const int heads = a.q_heads + a.kv_heads;
-  const long t = blockIdx.x;
-  for (unsigned item = threadIdx.x; item < (unsigned)(heads * cpr); item += 256)
-    apply_rotary_chunk<ADJACENT>(a, t, (int)(item / (unsigned)cpr), (int)(item % (unsigned)cpr));
-}
-
-template <bool ADJACENT>
-__device__ __forceinline__ void apply_rotary_chunk(const ct_rotary_args& a, long t, int h, int c) {
-  const bool is_q = h < a.q_heads;
-  const uint16_t* in = is_q ? a.q_in : a.k_in;
-  uint16_t* out = is_q ? a.q_out : a.k_out;
-  const size_t row = is_q ? ((size_t)t * a.q_heads + h) : ((size_t)t * a.kv_heads + (h - a.q_heads));
-  const size_t base = row * a.head_dim;
-  const bool scale_on = is_q && a.q_scale != 1.0f;
-  const float s = (float)(bf16)a.q_scale;  // the scale is rounded to bf16 first
+//
+// Bound by memory (each row read and written once, no 64-bit index arithmetic per chunk: a workgroup
+// belongs to its tokens). With two tokens the rows of both are requested before the first is worked on,
+// and head and chunk are found once for both; the size of a workgroup leaves no lane without an item
+// where that is possible, and the second halves of rotated heads no longer idle. At 16384 tokens of 32 + 8
+// heads of 128: adjacent pairs, 64 channels 65.5 -> 61.7 us (5.5 TB/s), halves 99.9 -> 74.5, halves of 128
+// channels 85.6 -> 61.2 (one token: 62.6, 78.9, 60.2; four: 65.4, 76.7, 63.2).
+constexpr int kRotaryTokens = 2;
+template <bool ADJACENT, int TOKENS>
+__global__ __launch_bounds__(512) void apply_rotary_kernel(ct_rotary_args a, int items_per_head, int items) {
   const int rot_chunks = a.rotary_pairs / 4;  // rotary_dim / 8
+  const int half_chunks = rot_chunks / 2;
+  const float s = (float)(bf16)a.q_scale;  // the scale is rounded to bf16 first
   const float sign = a.inverse ? -1.f : 1.f;
-
-  if (c >= rot_chunks) {
-    bf16x8 v = as_bf16x8(*reinterpret_cast<const u32x4*>(in + base + c * 8));
+  const long t0 = (long)blockIdx.x * TOKENS;
+  const int valid = a.tokens - t0 < TOKENS ? (int)(a.tokens - t0) : TOKENS;
+  for (unsigned item = threadIdx.x; item < (unsigned)items; item += blockDim.x) {
+    const int h = (int)(item / (unsigned)items_per_head);
+    int c = (int)(item % (unsigned)items_per_head);
+    if (!ADJACENT && c >= half_chunks) c += half_chunks;  // past the rotated channels
+    const bool is_q = h < a.q_heads, rotated = c < rot_chunks;
+    const size_t stride = (size_t)(is_q ? a.q_heads : a.kv_heads) * a.head_dim;  // of a token
+    const size_t at = t0 * stride + (size_t)(is_q ? h : h - a.q_heads) * a.head_dim + c * 8;
+    const uint16_t* in = (is_q ? a.q_in : a.k_in) + at;
+    uint16_t* out = (is_q ? a.q_out : a.k_out) + at;
+    const bool scale_on = is_q && a.q_scale != 1.0f;
+    u32x4 x1[TOKENS], x2[TOKENS], cv[TOKENS], sv[TOKENS];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = scaled(v[e], s, scale_on);
-    *reinterpret_cast<u32x4*>(out + base + c * 8) = as_u32x4(v);
-    return;
-  }
-  const bf16* cs = reinterpret_cast<const bf16*>(a.cosine) + (size_t)t * a.rotary_pairs;
-  const bf16* sn = reinterpret_cast<const bf16*>(a.sine) + (size_t)t * a.rotary_pairs;
-  if constexpr (ADJACENT) {
-    bf16x8 v = as_bf16x8(*reinterpret_cast<const u32x4*>(in + base + c * 8));
-    const bf16x4 cv = as_bf16x4(*reinterpret_cast<const u32x2*>(cs + c * 4));
-    const bf16x4 sv = as_bf16x4(*reinterpret_cast<const u32x2*>(sn + c * 4));
-    bf16x8 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bf16 even = v[2 * i], odd = v[2 * i + 1];
-      if (a.inverse) {
-        even = scaled(even, s, scale_on);
-        odd = scaled(odd, s, scale_on);
+    for (int k = 0; k < TOKENS; ++k) {
+      const int t = min(k, valid - 1);
+      x1[k] = *reinterpret_cast<const u32x4*>(in + t * stride);
+      if (!rotated) continue;
+      const uint16_t* cs = a.cosine + (t0 + t) * a.rotary_pairs;
+      const uint16_t* sn = a.sine + (t0 + t) * a.rotary_pairs;
+      if constexpr (ADJACENT) {
+        const u32x2 c2 = *reinterpret_cast<const u32x2*>(cs + c * 4), s2 = *reinterpret_cast<const u32x2*>(sn + c * 4);
+        cv[k] = u32x4{c2[0], c2[1], 0, 0};
+        sv[k] = u32x4{s2[0], s2[1], 0, 0};
+      } else {
+        x2[k] = *reinterpret_cast<const u32x4*>(in + t * stride + half_chunks * 8);
+        cv[k] = *reinterpret_cast<const u32x4*>(cs + c * 8);
+        sv[k] = *reinterpret_cast<const u32x4*>(sn + c * 8);
       }
-      const float co = (float)cv[i], si = sign * (float)sv[i];
-      bf16 oe = (bf16)((float)even * co - (float)odd * si);
-      bf16 oo = (bf16)((float)odd * co + (float)even * si);
-      if (!a.inverse) {
-        oe = scaled(oe, s, scale_on);
-        oo = scaled(oo, s, scale_on);
-      }
-      o[2 * i] = oe;
-      o[2 * i + 1] = oo;
     }
-    *reinterpret_cast<u32x4*>(out + base + c * 8) = as_u32x4(o);
-  } else {
-    const int half_chunks = rot_chunks / 2;
-    if (c >= half_chunks) return;  // written by the thread of the partner chunk
-    bf16x8 first = as_bf16x8(*reinterpret_cast<const u32x4*>(in + base + c * 8));
-    bf16x8 second = as_bf16x8(*reinterpret_cast<const u32x4*>(in + base + (c + half_chunks) * 8));
-    const bf16x8 cv = as_bf16x8(*reinterpret_cast<const u32x4*>(cs + c * 8));
-    const bf16x8 sv = as_bf16x8(*reinterpret_cast<const u32x4*>(sn + c * 8));
-    bf16x8 o1, o2;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      bf16 x1 = first[i], x2 = second[i];
-      if (a.inverse) {
-        x1 = scaled(x1, s, scale_on);
-        x2 = scaled(x2, s, scale_on);
+    for (int k = 0; k < TOKENS; ++k) {
+      if (k >= valid) break;
+      bf16x8 v = as_bf16x8(x1[k]), o;
+      if (!rotated) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = scaled(v[e], s, scale_on);
+      } else {
+        const bf16x8 co8 = as_bf16x8(cv[k]), si8 = as_bf16x8(sv[k]);
+        bf16x8 second = ADJACENT ? v : as_bf16x8(x2[k]), o2;
+#pragma unroll
+        for (int i = 0; i < (ADJACENT ? 4 : 8); ++i) {
+          bf16 p = ADJACENT ? v[2 * i] : v[i], q = ADJACENT ? v[2 * i + 1] : second[i];
+          if (a.inverse) {
+            p = scaled(p, s, scale_on);
+            q = scaled(q, s, scale_on);
+          }
+          const float co = (float)co8[i], si = sign * (float)si8[i];
+          bf16 rp = (bf16)((float)p * co - (float)q * si);
+          bf16 rq = (bf16)((float)q * co + (float)p * si);
+          if (!a.inverse) {
+            rp = scaled(rp, s, scale_on);
+            rq = scaled(rq, s, scale_on);
+          }
+          if constexpr (ADJACENT) {
+            o[2 * i] = rp;
+            o[2 * i + 1] = rq;
+          } else {
+            o[i] = rp;
+            o2[i] = rq;
+          }
+        }
+        if constexpr (!ADJACENT) *reinterpret_cast<u32x4*>(out + k * stride + half_chunks * 8) = as_u32x4(o2);
       }
-      const float co = (float)cv[i], si = sign * (float)sv[i];
-      bf16 r1 = (bf16)((float)x1 * co - (float)x2 * si);
-      bf16 r2 = (bf16)((float)x2 * co + (float)x1 * si);
-      if (!a.inverse) {
-        r1 = scaled(r1, s, scale_on);
-        r2 = scaled(r2, s, scale_on);
-      }
-      o1[i] = r1;
-      o2[i] = r2;
+      *reinterpret_cast<u32x4*>(out + k * stride) = as_u32x4(o);
     }
-    *reinterpret_cast<u32x4*>(out + base + c * 8) = as_u32x4(o1);
-    *reinterpret_cast<u32x4*>(out + base + (c + half_chunks) * 8) = as_u32x4(o2);
   }
 }
 
@@ -252,108 +246,163 @@ __global__ __launch_bounds__(256) void rms_norm_fwd_kernel(const uint16_t* x, co
   }
 }
 
-// The same for d = 512 NCH with the row held in registers: every load of the row is in flight
+// The same for d <= 512 NCH with the row held in registers: every load of the row is in flight
 // at once and x is read from memory exactly once.
 template <int NCH>
 __global__ __launch_bounds__(256) void rms_norm_fwd_rows_kernel(const uint16_t* x, const uint16_t* scale,
-                                                                float eps, long rows, uint16_t* y,
+                                                                float eps, long rows, int d, uint16_t* y,
                                                                 float* rstd) {
-  constexpr int d = 512 * NCH;
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, chunks = d / 8;
   const uint16_t* xr = x + (size_t)row * d;
-  bf16x8 v[NCH];
+  u32x4 v[NCH];
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) v[i] = as_bf16x8(*reinterpret_cast<const u32x4*>(xr + (lane + 64 * i) * 8));
+  for (int i = 0; i < NCH; ++i)
+    v[i] = i < NCH - 1 || lane + 64 * i < chunks ? *reinterpret_cast<const u32x4*>(xr + (lane + 64 * i) * 8) : u32x4{0, 0, 0, 0};
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += (float)v[i][e] * (float)v[i][e];
+    for (int e = 0; e < 8; ++e) ss += (float)as_bf16x8(v[i])[e] * (float)as_bf16x8(v[i])[e];
   ss = wave_sum(ss);
   const float r = 1.0f / sqrtf(ss / (float)d + eps);
   if (rstd && lane == 0) rstd[row] = r;
   uint16_t* yr = y + (size_t)row * d;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
+    if (i == NCH - 1 && lane + 64 * i >= chunks) break;
     const bf16x8 w = as_bf16x8(*reinterpret_cast<const u32x4*>(scale + (lane + 64 * i) * 8));
     bf16x8 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)(bf16)((float)v[i][e] * r) * (float)w[e]);
+    for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)(bf16)((float)as_bf16x8(v[i])[e] * r) * (float)w[e]);
     *reinterpret_cast<u32x4*>(yr + (lane + 64 * i) * 8) = as_u32x4(o);
   }
 }
 
 // Backward of y = bf16(xhat) * w, xhat = x r: with g = dy w (f32),
-//   dx = r (g - xhat mean(g xhat)),   dscale = sum over rows of dy bf16(xhat).
-// Wavefront `wv` of the launch takes rows wv, wv + W, ... and keeps its share of dscale in
-// registers (NCH chunks of 8 channels per lane, d = 512 NCH); it leaves one f32 partial row
-// which rms_norm_dscale_kernel adds up in wavefront order.
-template <int NCH>
+//   dx = r (g - xhat mean(g xhat)) = r (g - xhat r mean(g x)),   dscale = sum over rows of dy bf16(xhat).
+// WAVES wavefronts share a row (NCH chunks of 8 channels per lane, d <= 512 WAVES NCH), a workgroup takes
+// 4 / WAVES rows at a time and keeps its share of dscale in registers; it leaves one f32 partial row that
+// rms_norm_dscale_kernel adds up in workgroup order.
+//
+// Bound by memory: 6 bytes per element. With one wavefront per row and up to 320 registers the loads of a
+// row waited for the two reductions of the row before (102 us at [16384, 4096]), and every wavefront
+// left a partial row (32 MB written and read again). Sharing a row keeps a lane at 2 chunks, which leaves
+// registers to load the next row ahead; both sums of a row travel in one reduction; hidden sizes
+// that are not 512 times a power of two take the same kernel with the last chunk masked.
+template <int WAVES, int NCH>
 __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const uint16_t* x, const uint16_t* scale,
-                                                           const uint16_t* dy, float eps, long rows,
+                                                           const uint16_t* dy, float eps, long rows, int d,
                                                            uint16_t* dx, float* partial) {
-  constexpr int d = 512 * NCH;
-  const int lane = threadIdx.x & 63;
-  const long wv = (long)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (long)gridDim.x * 4;
+  constexpr int kRows = 4 / WAVES;  // rows a workgroup works on at a time
+  __shared__ float exch[2][4][2];
+  extern __shared__ float sums[];   // [kRows - 1][d] where several rows end in one partial row
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = wave % WAVES, chunks = d / 8;
   float acc[NCH][8];
+  u32x4 w[NCH], xn[NCH], gn[NCH];
+  int col[NCH];  // of chunk i, -1 past the row's end (only the last can be)
 #pragma unroll
-  for (int i = 0; i < NCH; ++i)
+  for (int i = 0; i < NCH; ++i) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
-  bf16x8 w[NCH];
-#pragma unroll
-  for (int i = 0; i < NCH; ++i)
-    w[i] = as_bf16x8(*reinterpret_cast<const u32x4*>(scale + (lane + 64 * i) * 8));
-
-  for (long row = wv; row < rows; row += waves) {
-    const uint16_t* xr = x + (size_t)row * d;
-    const uint16_t* gr = dy + (size_t)row * d;
-    bf16x8 xv[NCH], gv[NCH];
-    float ss = 0.f;
+    const int c = lane + 64 * (part + WAVES * i);
+    col[i] = c < chunks ? c * 8 : -1;
+    w[i] = col[i] >= 0 ? *reinterpret_cast<const u32x4*>(scale + col[i]) : u32x4{0, 0, 0, 0};
+  }
+  auto fetch = [&](long row) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      xv[i] = as_bf16x8(*reinterpret_cast<const u32x4*>(xr + (lane + 64 * i) * 8));
-      gv[i] = as_bf16x8(*reinterpret_cast<const u32x4*>(gr + (lane + 64 * i) * 8));
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += (float)xv[i][e] * (float)xv[i][e];
+      const bool in = row < rows && col[i] >= 0;
+      xn[i] = in ? *reinterpret_cast<const u32x4*>(x + (size_t)row * d + col[i]) : u32x4{0, 0, 0, 0};
+      gn[i] = in ? *reinterpret_cast<const u32x4*>(dy + (size_t)row * d + col[i]) : u32x4{0, 0, 0, 0};
     }
-    ss = wave_sum(ss);
-    const float r = 1.0f / sqrtf(ss / (float)d + eps);
-    float dot = 0.f;
+  };
+  const long stride = (long)gridDim.x * kRows;
+  long row = (long)blockIdx.x * kRows + wave / WAVES;
+  fetch(row);
+  // (all wavefronts of a workgroup take the same number of turns: the barrier below is uniform)
+  for (long base = (long)blockIdx.x * kRows, turn = 0; base < rows; base += stride, row += stride, ++turn) {
+    u32x4 xv[NCH], gv[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      xv[i] = xn[i];
+      gv[i] = gn[i];
+    }
+    fetch(row + stride);
+    float ss = 0.f, dot = 0.f;
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float xhat = (float)xv[i][e] * r;
-        dot += (float)gv[i][e] * (float)w[i][e] * xhat;
-        acc[i][e] += (float)gv[i][e] * (float)(bf16)xhat;
+        const float xf = (float)as_bf16x8(xv[i])[e];
+        ss += xf * xf;
+        dot += (float)as_bf16x8(gv[i])[e] * (float)as_bf16x8(w[i])[e] * xf;
       }
-    dot = wave_sum(dot) / (float)d;
-    uint16_t* dr = dx + (size_t)row * d;
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      bf16x8 o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float xhat = (float)xv[i][e] * r;
-        o[e] = (bf16)(r * ((float)gv[i][e] * (float)w[i][e] - xhat * dot));
+    ss = wave_sum(ss);
+    dot = wave_sum(dot);
+    if constexpr (WAVES > 1) {
+      float (*e)[2] = exch[turn & 1];  // (two of them: one barrier per turn)
+      if (lane == 0) {
+        e[wave][0] = ss;
+        e[wave][1] = dot;
       }
-      *reinterpret_cast<u32x4*>(dr + (lane + 64 * i) * 8) = as_u32x4(o);
+      __syncthreads();
+      ss = dot = 0.f;
+#pragma unroll
+      for (int k = 0; k < WAVES; ++k) {
+        ss += e[wave / WAVES * WAVES + k][0];
+        dot += e[wave / WAVES * WAVES + k][1];
+      }
+    }
+    const float r = 1.0f / sqrtf(ss / (float)d + eps);
+    const float mean = dot * r / (float)d;
+    if (row < rows) {
+      uint16_t* dr = dx + (size_t)row * d;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        if (col[i] < 0) continue;
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float xhat = (float)as_bf16x8(xv[i])[e] * r, g = (float)as_bf16x8(gv[i])[e];
+          acc[i][e] += g * (float)(bf16)xhat;
+          o[e] = (bf16)(r * (g * (float)as_bf16x8(w[i])[e] - xhat * mean));
+        }
+        *reinterpret_cast<u32x4*>(dr + col[i]) = as_u32x4(o);
+      }
     }
   }
-  float* prow = partial + (size_t)wv * d;
+  // the workgroup's row groups, in order
+  float* prow = partial + (size_t)blockIdx.x * d;
+  if constexpr (kRows > 1) {
+    if (wave >= WAVES) {
+      float* mine = sums + (size_t)(wave / WAVES - 1) * d;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+        if (col[i] >= 0)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) mine[col[i] + e] = acc[i][e];
+    }
+    __syncthreads();
+    if (wave >= WAVES) return;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (col[i] >= 0)
+#pragma unroll
+        for (int k = 0; k < kRows - 1; ++k)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[i][e] += sums[(size_t)k * d + col[i] + e];
+  }
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) prow[(lane + 64 * i) * 8 + e] = acc[i][e];
+    if (col[i] >= 0) {
+      *reinterpret_cast<f32x4*>(prow + col[i]) = f32x4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+      *reinterpret_cast<f32x4*>(prow + col[i] + 4) = f32x4{acc[i][4], acc[i][5], acc[i][6], acc[i][7]};
+    }
 }
 
-// dscale[col] = sum of the wavefronts' partial rows in a fixed order: thread (c, g) adds the rows
-// of sixteenth g for column 64 blockIdx.x + c (four independent chains, joined in order), then the
-// sixteen group sums are added in order.
-// Any hidden size that is a multiple of 8: the row is walked three times (sum of squares, the
+// Hidden sizes past 8192: the row is walked three times (sum of squares, the
 // dot product, dx; the repeats are served from cache) and the wavefront's dscale sums live in its
 // row of `partial` instead of registers (a lane only ever touches its own columns of it).
 __global__ __launch_bounds__(256) void rms_norm_bwd_any_kernel(const uint16_t* x, const uint16_t* scale,
@@ -402,33 +451,41 @@ __global__ __launch_bounds__(256) void rms_norm_bwd_any_kernel(const uint16_t* x
   }
 }
 
-__global__ __launch_bounds__(1024) void rms_norm_dscale_kernel(const float* partial, int waves, int d,
-                                                               float* dscale) {
-  __shared__ float group[16][64];
-  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int col = blockIdx.x * 64 + c;
-  const int per = waves / 16;  // a multiple of 4
+// dscale[col] = sum of the partial rows in a fixed order: thread (c, g) adds the rows g, g + 32, ... for
+// column 32 blockIdx.x + c (four independent chains, joined in order), then the 32 group sums are added
+// in order. Exactly one of the two outputs is given.
+__global__ __launch_bounds__(1024) void rms_norm_dscale_kernel(const float* partial, int count, int d,
+                                                               float* dscale, bf16* dscale_rounded) {
+  __shared__ float group[32][33];
+  const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int col = blockIdx.x * 32 + c;
   float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
   if (col < d) {
-    const float* p = partial + (size_t)g * per * d + col;
-    for (int i = 0; i < per; i += 4) {
+    const float* p = partial + col;
+    int i = g;
+    for (; i + 96 < count; i += 128) {
       s0 += p[(size_t)i * d];
-      s1 += p[(size_t)(i + 1) * d];
-      s2 += p[(size_t)(i + 2) * d];
-      s3 += p[(size_t)(i + 3) * d];
+      s1 += p[(size_t)(i + 32) * d];
+      s2 += p[(size_t)(i + 64) * d];
+      s3 += p[(size_t)(i + 96) * d];
     }
+    for (; i < count; i += 32) s0 += p[(size_t)i * d];
   }
   group[g][c] = (s0 + s1) + (s2 + s3);
   __syncthreads();
   if (g == 0 && col < d) {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) s += group[k][c];
-    dscale[col] = s;
+    for (int k = 0; k < 32; ++k) s += group[k][c];
+    if (dscale) dscale[col] = s;
+    else dscale_rounded[col] = (bf16)s;
   }
 }
 
-constexpr int kNormBwdBlocks = 512;  // 2048 wavefronts, 8 per compute unit
+// Partial rows of dscale: three workgroups per compute unit, as many as the registers of a shared row
+// leave room for (the walking kernel writes one per wavefront).
+constexpr int kNormBwdBlocks = 768;
+constexpr int kNormBwdAnyBlocks = 512;
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -492,12 +549,20 @@ extern "C" int32_t ct_apply_rotary(void* stream, const ct_rotary_args* a) {
       hipLaunchKernelGGL((apply_rotary_rows_kernel<false>), grid, dim3(256), 0, (hipStream_t)stream, *a);
     return scope.done();
   }
-  if (a->rope_style == CT_ROPE_GPT_J)
-    hipLaunchKernelGGL((apply_rotary_kernel<true>), dim3((unsigned)a->tokens), dim3(256), 0,
-                       (hipStream_t)stream, *a);
-  else
-    hipLaunchKernelGGL((apply_rotary_kernel<false>), dim3((unsigned)a->tokens), dim3(256), 0,
-                       (hipStream_t)stream, *a);
+  const bool adjacent = a->rope_style == CT_ROPE_GPT_J;
+  const int per_head = a->head_dim / 8 - (adjacent ? 0 : a->rotary_pairs / 8), items = (a->q_heads + a->kv_heads) * per_head;
+  // as many threads as leave the fewest idle in the last round (640 items: 320), the most of those
+  int threads = 64;
+  for (int n = 128; n <= 512; n += 64)
+    if ((items + n - 1) / n * n <= (items + threads - 1) / threads * threads) threads = n;
+  // several tokens a workgroup once every compute unit has 8 workgroups of them
+  const int tokens = a->tokens >= 256 * 8 * kRotaryTokens ? kRotaryTokens : 1;
+  const dim3 grid((unsigned)((a->tokens + tokens - 1) / tokens)), block(threads);
+  hipStream_t st = (hipStream_t)stream;
+  if (adjacent && tokens == 1) hipLaunchKernelGGL((apply_rotary_kernel<true, 1>), grid, block, 0, st, *a, per_head, items);
+  else if (adjacent) hipLaunchKernelGGL((apply_rotary_kernel<true, kRotaryTokens>), grid, block, 0, st, *a, per_head, items);
+  else if (tokens == 1) hipLaunchKernelGGL((apply_rotary_kernel<false, 1>), grid, block, 0, st, *a, per_head, items);
+  else hipLaunchKernelGGL((apply_rotary_kernel<false, kRotaryTokens>), grid, block, 0, st, *a, per_head, items);
   return scope.done();
 }
 
@@ -512,27 +577,32 @@ extern "C" int32_t ct_rms_norm_fwd(void* stream, const uint16_t* x, const uint16
   LaunchScope scope("rms_norm_fwd_kernel", (hipStream_t)stream);
   const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
   hipStream_t st = (hipStream_t)stream;
-  switch (hidden % 512 == 0 ? hidden / 512 : 0) {
-    case 1: hipLaunchKernelGGL((rms_norm_fwd_rows_kernel<1>), grid, block, 0, st, x, scale, eps, (long)rows, y, rstd); break;
-    case 2: hipLaunchKernelGGL((rms_norm_fwd_rows_kernel<2>), grid, block, 0, st, x, scale, eps, (long)rows, y, rstd); break;
-    case 4: hipLaunchKernelGGL((rms_norm_fwd_rows_kernel<4>), grid, block, 0, st, x, scale, eps, (long)rows, y, rstd); break;
-    case 8: hipLaunchKernelGGL((rms_norm_fwd_rows_kernel<8>), grid, block, 0, st, x, scale, eps, (long)rows, y, rstd); break;
-    case 16: hipLaunchKernelGGL((rms_norm_fwd_rows_kernel<16>), grid, block, 0, st, x, scale, eps, (long)rows, y, rstd); break;
-    default: hipLaunchKernelGGL(rms_norm_fwd_kernel, grid, block, 0, st, x, scale, eps, (long)rows, hidden, y, rstd);
+  const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, x, scale, eps, (long)rows, hidden, y, rstd); };
+  switch (int chunks = (hidden + 511) / 512; chunks) {
+    case 1: launch(rms_norm_fwd_rows_kernel<1>); break;
+    case 2: launch(rms_norm_fwd_rows_kernel<2>); break;
+    case 3: launch(rms_norm_fwd_rows_kernel<3>); break;
+    case 4: launch(rms_norm_fwd_rows_kernel<4>); break;
+    case 5: launch(rms_norm_fwd_rows_kernel<5>); break;
+    case 6: launch(rms_norm_fwd_rows_kernel<6>); break;
+    case 7: launch(rms_norm_fwd_rows_kernel<7>); break;
+    case 8: launch(rms_norm_fwd_rows_kernel<8>); break;
+    case 10: launch(rms_norm_fwd_rows_kernel<10>); break;
+    case 16: launch(rms_norm_fwd_rows_kernel<16>); break;
+    default: launch(rms_norm_fwd_kernel);
   }
   return scope.done();
 }
 
 extern "C" size_t ct_rms_norm_bwd_workspace_bytes(int32_t hidden) {
   if (hidden <= 0) return 0;
-  return (size_t)kNormBwdBlocks * 4 * hidden * sizeof(float);
+  return (size_t)(hidden <= 8192 ? kNormBwdBlocks : kNormBwdAnyBlocks * 4) * hidden * sizeof(float);
 }
 
-extern "C" int32_t ct_rms_norm_bwd(void* stream_, const uint16_t* x, const uint16_t* scale,
-                                   const uint16_t* dy, float eps, int64_t rows, int32_t hidden,
-                                   uint16_t* dx, float* dscale, void* workspace,
-                                   size_t workspace_bytes) {
-  CT_REQUIRE(x && scale && dy && dx && dscale && workspace, "ct_rms_norm_bwd: null pointer");
+static int32_t rms_norm_bwd_on(void* stream_, const uint16_t* x, const uint16_t* scale, const uint16_t* dy, float eps,
+                               int64_t rows, int32_t hidden, uint16_t* dx, float* dscale, uint16_t* dscale_rounded,
+                               void* workspace, size_t workspace_bytes) {
+  CT_REQUIRE(x && scale && dy && dx && (dscale || dscale_rounded) && workspace, "ct_rms_norm_bwd: null pointer");
   CT_REQUIRE(rows > 0, "ct_rms_norm_bwd: rows must be positive");
   CT_REQUIRE(hidden > 0 && hidden % 8 == 0, "ct_rms_norm_bwd: hidden size must be a multiple of 8, got %d", hidden);
   CT_REQUIRE(aligned16(x) && aligned16(scale) && aligned16(dy) && aligned16(dx) && aligned16(workspace),
@@ -542,23 +612,46 @@ extern "C" int32_t ct_rms_norm_bwd(void* stream_, const uint16_t* x, const uint1
                 ct_rms_norm_bwd_workspace_bytes(hidden));
   hipStream_t stream = (hipStream_t)stream_;
   float* partial = static_cast<float*>(workspace);
+  int count;  // partial rows
   LaunchScope scope("rms_norm_bwd_kernel", stream);
-  const dim3 grid(kNormBwdBlocks), block(256);
-  // rows held in registers for 512 * {1, 2, 4, 8, 16}; any other multiple of 8 walks the row
-  const bool in_registers = hidden == 512 || hidden == 1024 || hidden == 2048 || hidden == 4096 || hidden == 8192;
-  switch (in_registers ? hidden / 512 : 0) {
-    case 0: hipLaunchKernelGGL(rms_norm_bwd_any_kernel, grid, block, 0, stream, x, scale, dy, eps, (long)rows, hidden, dx, partial); break;
-    case 1: hipLaunchKernelGGL((rms_norm_bwd_kernel<1>), grid, block, 0, stream, x, scale, dy, eps, (long)rows, dx, partial); break;
-    case 2: hipLaunchKernelGGL((rms_norm_bwd_kernel<2>), grid, block, 0, stream, x, scale, dy, eps, (long)rows, dx, partial); break;
-    case 4: hipLaunchKernelGGL((rms_norm_bwd_kernel<4>), grid, block, 0, stream, x, scale, dy, eps, (long)rows, dx, partial); break;
-    case 8: hipLaunchKernelGGL((rms_norm_bwd_kernel<8>), grid, block, 0, stream, x, scale, dy, eps, (long)rows, dx, partial); break;
-    default: hipLaunchKernelGGL((rms_norm_bwd_kernel<16>), grid, block, 0, stream, x, scale, dy, eps, (long)rows, dx, partial); break;
+  if (hidden > 8192) {
+    hipLaunchKernelGGL(rms_norm_bwd_any_kernel, dim3(kNormBwdAnyBlocks), dim3(256), 0, stream, x, scale, dy, eps, (long)rows,
+                       hidden, dx, partial);
+    count = kNormBwdAnyBlocks * 4;
+  } else {
+    // wavefronts that share a row: the fewest that keep a lane at 2 chunks (3 or 4 past 4096)
+    const int waves = hidden <= 1024 ? 1 : hidden <= 2048 ? 2 : 4, at_a_time = 4 / waves;
+    const int64_t groups = (rows + at_a_time - 1) / at_a_time;
+    count = groups < kNormBwdBlocks ? (int)groups : kNormBwdBlocks;
+    const size_t smem = (size_t)(at_a_time - 1) * hidden * sizeof(float);
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(count), dim3(256), smem, stream, x, scale, dy, eps, (long)rows, hidden, dx, partial);
+    };
+    switch (int chunks = (hidden + 512 * waves - 1) / (512 * waves); 8 * waves + chunks) {
+      case 9: launch(rms_norm_bwd_kernel<1, 1>); break;
+      case 10: launch(rms_norm_bwd_kernel<1, 2>); break;
+      case 18: launch(rms_norm_bwd_kernel<2, 2>); break;
+      case 34: launch(rms_norm_bwd_kernel<4, 2>); break;
+      case 35: launch(rms_norm_bwd_kernel<4, 3>); break;
+      default: launch(rms_norm_bwd_kernel<4, 4>); break;
+    }
   }
   int rc = scope.done();
   if (rc) return rc;
   LaunchScope scope2("rms_norm_dscale_kernel", stream);
-  static_assert(kNormBwdBlocks * 4 % 64 == 0, "dscale kernel splits the partial rows 16 x 4 ways");
-  hipLaunchKernelGGL(rms_norm_dscale_kernel, dim3((hidden + 63) / 64), dim3(1024), 0, stream, partial,
-                     kNormBwdBlocks * 4, hidden, dscale);
+  hipLaunchKernelGGL(rms_norm_dscale_kernel, dim3((hidden + 31) / 32), dim3(1024), 0, stream, partial, count, hidden, dscale,
+                     reinterpret_cast<bf16*>(dscale_rounded));
   return scope2.done();
+}
+
+extern "C" int32_t ct_rms_norm_bwd(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy, float eps,
+                                   int64_t rows, int32_t hidden, uint16_t* dx, float* dscale, void* workspace,
+                                   size_t workspace_bytes) {
+  return rms_norm_bwd_on(stream, x, scale, dy, eps, rows, hidden, dx, dscale, nullptr, workspace, workspace_bytes);
+}
+
+extern "C" int32_t ct_rms_norm_bwd_rounded(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
+                                           float eps, int64_t rows, int32_t hidden, uint16_t* dx, uint16_t* dscale,
+                                           void* workspace, size_t workspace_bytes) {
+  return rms_norm_bwd_on(stream, x, scale, dy, eps, rows, hidden, dx, nullptr, dscale, workspace, workspace_bytes);
 }

@@ -290,12 +290,12 @@ struct RmsNormNode : Node {
     const c10::DeviceGuard guard(X.device());
     const int64_t hidden = X.size(-1), rows = X.numel() / hidden;
     const Tensor dy = gradient(grads[0], X.sizes(), at::kBFloat16, X);
-    Tensor dx = fresh(X), dscale = floats({hidden}, X);
+    Tensor dx = fresh(X), dscale = fresh(W);
     const size_t bytes = ct_rms_norm_bwd_workspace_bytes((int32_t)hidden);
     Tensor workspace = scratch(bytes, X);
-    check(ct_rms_norm_bwd(current_stream(), bits(X), bits(W), bits(dy), (float)eps, rows, (int32_t)hidden, bits(dx),
-                          ptr<float>(dscale), workspace.data_ptr(), bytes));
-    return {dx, dscale.to(W.scalar_type())};
+    check(ct_rms_norm_bwd_rounded(current_stream(), bits(X), bits(W), bits(dy), (float)eps, rows, (int32_t)hidden, bits(dx),
+                                  bits(dscale), workspace.data_ptr(), bytes));
+    return {dx, dscale};
   }
   void release_variables() override {
     x.reset_data();

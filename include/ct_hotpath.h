@@ -340,13 +340,18 @@ size_t ct_rms_norm_bwd_workspace_bytes(int32_t hidden);
 
 /*
  * Gradients of ct_rms_norm_fwd: dx bf16 [rows, hidden], dscale f32 [hidden]
- * (summed over rows in a fixed order). hidden % 8 == 0 (512 * {1, 2, 4, 8, 16}
- * keeps the row in registers; other sizes walk it three times).
+ * (summed over rows in a fixed order). hidden % 8 == 0 (up to 8192 the row is
+ * kept in registers; larger ones walk it three times).
  * Replaces: the autodiff transpose of rms_norm (src/modeling/architecture.py:155-162).
  */
 int32_t ct_rms_norm_bwd(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
                         float eps, int64_t rows, int32_t hidden, uint16_t* dx, float* dscale,
                         void* workspace, size_t workspace_bytes);
+
+/* The same with dscale rounded to bf16 (the gradient of a bf16 scale). */
+int32_t ct_rms_norm_bwd_rounded(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
+                                float eps, int64_t rows, int32_t hidden, uint16_t* dx, uint16_t* dscale,
+                                void* workspace, size_t workspace_bytes);
 
 /* ------------------------------------------------------------------------
  * Sparse cross-entropy on materialised logits (the non-fused loss backend)

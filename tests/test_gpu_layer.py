@@ -219,3 +219,19 @@ def test_rms_norm_gradients_match_oracle(ct, gpu, rows, hidden):
     with pytest.raises((RuntimeError, ValueError), match="multiple of 8"):
         bad = torch.ones((2, 132), dtype=torch.bfloat16, device=gpu, requires_grad=True)
         ct.rms_norm(bad, torch.ones(132, dtype=torch.bfloat16, device=gpu), 1e-6).sum().backward()
+
+
+@pytest.mark.parametrize("rows,hidden", [(300, 1032), (513, 2048), (41, 2056), (90, 4104), (33, 6152), (7, 8184)])
+def test_rms_norm_rows_shared_by_wavefronts(ct, gpu, rows, hidden):
+    """Hidden sizes at both ends of what 1, 2 and 4 wavefronts share, with masked last chunks and row
+    counts that leave some of a workgroup's places empty."""
+
+    test_rms_norm_forward_matches_oracle(ct, gpu, rows, hidden)
+    test_rms_norm_gradients_match_oracle(ct, gpu, rows, hidden)
+
+
+@pytest.mark.parametrize("style", ["gpt-j", "gpt-neox"])
+def test_rotary_of_two_tokens_per_workgroup(ct, gpu, style):
+    """Many tokens, an odd number of them: the last workgroup has one."""
+
+    test_rotary_matches_oracle(ct, gpu, style, (1, 4097, 3, 1, 64, 32))
