@@ -4,6 +4,7 @@
 
 #include "ct_attn_bwd_kernels.hip.h"
 #include "ct_attn_dkv_wide.hip.h"
+#include "ct_attn_fwd_split.hip.h"
 #include "ct_attn_kernels.hip.h"
 #include "ct_error.h"
 
@@ -403,22 +404,66 @@ static int ensure_lds(const char* fn, const void* kernel, size_t bytes, std::ato
     if (rc_) return rc_;                                                                  \
   } while (0)
 
+// Workgroups that share a work bin of a (head slice, KV head) group. A workgroup fills a compute
+// unit, so groups x 32 bins fill the 256 units whole times exactly when the groups come in eights;
+// the fewest members that make (groups x members) a multiple of 8 do the same for every other count.
+static int fwd_members(int groups) { return groups % 8 == 0 ? 1 : groups % 4 == 0 ? 2 : groups % 2 == 0 ? 4 : 8; }
+
 template <int D, int HS>
 static int launch_fwd(hipStream_t stream, const AttnParams& p) {
   const size_t smem = VkStage<D>::kTotalBytes;
   CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_kernel<D, HS>), smem);
-  const int grid = (p.Hq / HS) * kBins;  // (head slice, KV head) groups x work bins
+  const int groups = p.Hq / HS;  // (head slice, KV head)
+  const int grid = groups * kBins * fwd_members(groups);
   LaunchScope scope1("attn_fwd_kernel", stream);
   hipLaunchKernelGGL((attn_fwd_kernel<D, HS>), dim3(grid), dim3(kFwdWaves * 64), smem, stream, p);
   return scope1.done();
 }
 
+template <int D, int HS, int KS, int KB, int SUB>
+static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
+  const size_t smem = SplitStage<D, KS, KB, SUB>::kTotalBytes;
+  CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_split_kernel<D, HS, KS, KB, SUB>), smem);
+  const int grid = (p.Hq / HS) * p.B * bin_tiles_per_row(p.S / 32, 4 / KS / HS);
+  LaunchScope scope("attn_fwd_split_kernel", stream);
+  hipLaunchKernelGGL((attn_fwd_split_kernel<D, HS, KS, KB, SUB>), dim3(grid), dim3(256), smem, stream, p);
+  return scope.done();
+}
+template <int D, int KS, int KB, int SUB>
+static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
+  const int hs = heads_per_group(p.Hq, p.Hkv);
+  if constexpr (KS == 1)
+    if (hs == 4) return launch_fwd_split<D, 4, KS, KB, SUB>(stream, p);
+  if constexpr (KS <= 2)
+    if (hs >= 2) return launch_fwd_split<D, 2, KS, KB, SUB>(stream, p);
+  return launch_fwd_split<D, 1, KS, KB, SUB>(stream, p);
+}
+
+// By the row blocks of the launch (32 query rows of one head: one wavefront's work; the device has
+// 1024 SIMDs). Few of them leave SIMDs idle while the longest row's chain of steps runs: its keys
+// are then shared by wavefronts. Where the lines lie was measured over row lengths 128 to 26496 and
+// documents from 36 positions to the whole row:
+//   head dimension 64: sharing by four wins up to 512 row blocks (half a wavefront per SIMD), sharing
+//     by two up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47 us).
+//   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920, 106 against 102 us
+//     at 2048). Above, the large launch's interleaved loop is ahead where rows see 8 key tiles or more
+//     (229 against 242 us), and is behind where they see few (61 against 46 us), which is certain
+//     only for short rows: the line at 20 key tiles per row is where whole-row documents cost 4 %.
 template <int D>
 static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
-  switch (heads_per_group(p.Hq, p.Hkv)) {
-    case 4: return launch_fwd<D, 4>(stream, p);
-    case 2: return launch_fwd<D, 2>(stream, p);
-    default: return launch_fwd<D, 1>(stream, p);
+  const long blocks = (long)p.B * p.Hq * (p.S / 32);
+  if constexpr (D == 64) {
+    if (blocks <= 512) return launch_fwd_split<D, 4, 1, 1>(stream, p);
+    if (blocks < 7168) return launch_fwd_split<D, 2, 1, 1>(stream, p);
+    return launch_fwd_split<D, 1, 1, 2>(stream, p);
+  } else {
+    if (blocks < 2048) return launch_fwd_split<D, 2, 1, 1>(stream, p);
+    if (p.S <= 20 * kKeyTile) return launch_fwd_split<D, 1, 2, 1>(stream, p);
+    switch (heads_per_group(p.Hq, p.Hkv)) {
+      case 4: return launch_fwd<D, 4>(stream, p);
+      case 2: return launch_fwd<D, 2>(stream, p);
+      default: return launch_fwd<D, 1>(stream, p);
+    }
   }
 }
 

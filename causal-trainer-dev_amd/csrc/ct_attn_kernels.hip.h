@@ -509,10 +509,9 @@ CT_DEVICE void dq_acc_half_128(const TrFragOffsets<16, KSlots::kAccum>& to, bf16
 // ---------------------------------------------------------------------------
 // Forward
 //
-// One workgroup of 8 wavefronts per compute unit (wavefronts w and w + 4 share a SIMD), each with
-// 32 query rows of one head. Two forms of the key-tile loop:
-//
-// D = 128, interleaved (attn_fwd_item). Per key tile t a wavefront has three pieces of work: the
+// Head dimension 128, large launches (the others: ct_attn_fwd_split.hip.h). One workgroup of 8
+// wavefronts per compute unit (wavefronts w and w + 4 share a SIMD), each with 32 query rows of one
+// head. Per key tile t a wavefront has three pieces of work: the
 // softmax arithmetic of tile t (vector ALU), O += V(t-1)^T P(t-1)^T and S(t+1)^T = K(t+1) Q^T
 // (32 MFMAs). They are independent of each other, so the arithmetic is issued between the MFMAs
 // of the same wavefront (three asm statements per tile, see gen_attn_asm.py): about five vector
@@ -526,26 +525,6 @@ CT_DEVICE void dq_acc_half_128(const TrFragOffsets<16, KSlots::kAccum>& to, bf16
 // the buffer that the step before has finished with, and awaited at its end, in front of the one
 // workgroup barrier per step. Segment ids of the key tiles go through a ring of 4 slots (tile t
 // in slot t % 4, copied together with its K rows, read in the step of tile t).
-//
-// Other head sizes, phased (attn_fwd_item_phased):
-// One workgroup of 8 wavefronts per compute unit: wavefronts w and w + 4 share
-// a SIMD. Per key tile a wavefront alternates between a VALU phase (softmax of
-// the tile's scores) and an MFMA phase (O += V^T P of this tile, then the
-// scores of the next tile). Wavefronts 4..7 (the "late" group) run half a step
-// behind wavefronts 0..3 (they pass one extra barrier before the loop, the
-// others one after it), and a workgroup barrier closes every phase, so on each
-// SIMD one wavefront is in its VALU phase while the other one is in its MFMA
-// phase and the two pipes overlap.
-//
-// Global phase numbering: the early group runs VALU phase t in phase 2t and
-// MFMA phase t in phase 2t + 1; the late group one phase later. LDS holds 2
-// stages; stage s = V rows of tile s and K rows of tile s + 1, exactly the
-// operands of MFMA phase s, read in phases 2s + 1 and 2s + 2. The copies for
-// stage t + 1 replace stage t - 1 and are issued at the start of phase 2t + 1
-// (early group: on entering MFMA phase t; late group: on entering VALU phase
-// t) and awaited at the end of phase 2t + 2, one barrier before the first read.
-// Segment ids of the key tiles go through a ring of 4 slots (tile t in slot
-// t % 4, copied together with stage t - 1, read in phases 2t and 2t + 1).
 // ---------------------------------------------------------------------------
 constexpr int kFwdWaves = 8;
 constexpr float kRescaleSlack = 8.f;
@@ -585,11 +564,6 @@ struct VkFetcher {
     dma.issue(kbase + (size_t)tile * kKeyTile * row_stride_bytes, stage + VkStage<D>::kK);
     if (threadIdx.x < 16)  // 64 ids = 16 lanes x 16 bytes, linear layout
       dma16_s(segb + tile * kKeyTile, threadIdx.x * 16, lds0 + VkStage<D>::seg_slot(tile));
-  }
-  // stage s: V(s), K(s + 1); tiles past `last` are skipped
-  CT_DEVICE void issue_stage(int s, int last, lds_addr stage, lds_addr lds0) const {
-    if (s <= last) issue_v(s, stage);
-    if (s + 1 <= last) issue_k(s + 1, stage, lds0);
   }
   // Stage s = V(s), K(s + 2) as the operands of a statement that issues this wavefront's copies
   // itself. A K tile past `last` is replaced by tile `last` (copied to where nothing reads it):
@@ -676,207 +650,6 @@ struct FwdAhead {
   }
 };
 
-// One query tile (kFwdWaves / HS row blocks x HS heads of one KV head), start to finish. `ahead`
-// holds what this tile read ahead on entry and what tile (batch row next_b, tile next_qt) did on
-// return. The request is unconditional (the last tile of a workgroup names itself again): a
-// conditional one would keep the old Q registers alive through the whole tile.
-template <int D, int HS>
-CT_DEVICE void attn_fwd_item_phased(const AttnParams& p, FwdAhead<D, HS>& ahead, int next_b,
-                             int next_qt, int kvh, int slice, const lds_addr lds0,
-                             const RowFragOffsets<D / 8>& ro,
-                             const TrFragOffsets<D / 8, KSlots::kAccum>& to) {
-  constexpr int kStage = VkStage<D>::kBytes;
-  const QueryTileContext<D, HS, kFwdWaves> ctx(p, ahead.b, kvh, slice, ahead.qt, ahead.bounds, ahead.seg_q,
-                                                ahead.end_q);
-
-  const int l = lane_id(), half = l >> 5, w = threadIdx.x >> 6;
-  const bool late = uniform(w) >= kFwdWaves / 2;
-  const size_t q_row_stride = (size_t)p.Hq * D;
-  const size_t kv_row_stride = (size_t)p.Hkv * D;
-
-
-  f32x16 oacc[D / 32];
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db) oacc[db] = zero16();
-  float m_run = kNegInf;  // softmax reference (a recent running max), log2 domain
-  float l_run = 0.f;      // this lane's share of the running sum (f32: the LSE is held to 1e-3)
-
-  const VkFetcher<D> fetch(ctx.kbase, ctx.vbase, ctx.segb, kv_row_stride);
-  int t = ctx.first;
-  const int last = ctx.last;
-  KeyTileBounds kb = {0, 0, 0}, nb = {0, 0, 0};  // bounds of tiles t and t + 1
-  f32x16 s[2];
-  bool visit = false;
-  if (t <= last) {
-    fetch.issue_k(t, lds0 + kStage, lds0);  // stage first - 1 (buffer 1): only its K half
-    fetch.issue_stage(t, last, lds0, lds0);  // stage first -> buffer 0
-    kb = key_tile_bounds(ctx.meta_b, t);
-    if (t + 1 <= last) nb = key_tile_bounds(ctx.meta_b, t + 1);
-    visit = ctx.wave_visits(kb, t);
-  }
-  // the next tile's bounds: scalar loads behind this tile's first copies; nothing here uses them
-  ahead.request_bounds(p, next_b, kvh, slice, next_qt);
-  // (the Q rows are touched only now: the first copies above needed nothing but the bounds)
-  bf16x8 qf[D / 16];
-  ahead.q_rows.to_fragments(lds0 + (VkStage<D>::kStorePatches + w * VkStage<D>::kStorePatchBytes), qf);
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) qf[ks] = scale_bf16x8(qf[ks], p.scale);
-  dma_wait_all();
-  __syncthreads();
-  if (visit) scores_t<D>(kStage + VkStage<D>::kK, ro, qf, s);
-  if (late) __builtin_amdgcn_s_barrier();
-
-  // The VALU phase of tile t: masks, running maximum and sum, probabilities as bf16 fragments.
-  auto softmax_phase = [&](bf16x8* pf) {
-    if (visit) {
-      float mx = kNegInf;
-      {
-        // What the summaries leave open for this tile. A key tile with one shared id X turns
-        // the id test into a per-query predicate (seg_q == X), which folds into the visible-end
-        // bound; only a key tile that mixes ids needs the per-key comparison.
-        const int k_uniform = uniform(kb.uniform);
-        const bool mixed_keys = k_uniform == 0;
-        const bool need_seg = ctx.mine.uniform == 0 || ctx.mine.uniform != k_uniform;
-        const bool need_causal = t * kKeyTile + kKeyTile - 1 > ctx.mine.end_min;
-        if (need_seg || need_causal) {
-          const int seg_cmp = ctx.row_valid() ? ctx.seg_q : -1;
-          int last_rel = ctx.end_q - t * kKeyTile - 4 * half;
-          if (mixed_keys) {
-            mask_scores_t<true, true>(lds0 + VkStage<D>::seg_slot(t), seg_cmp, last_rel, s);
-          } else {
-            if (seg_cmp != k_uniform) last_rel = -1;  // no key of this tile is visible
-            mask_scores_t<false, true>(lds0, seg_cmp, last_rel, s);
-          }
-        }
-      }
-#pragma unroll
-      for (int kbk = 0; kbk < 2; ++kbk)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kbk][r]);
-      mx = pair_max(mx) * kLog2e;
-      // The running reference m_run only follows the true maximum when that has grown by
-      // more than kRescaleSlack (log2 units): probabilities are then at most 2^slack, well
-      // inside bf16 / f32 range, the normalisation by the row sum is unchanged, and the
-      // accumulator is rescaled on few tiles instead of most.
-      if (__any(mx > m_run + kRescaleSlack)) {
-        const float m_new = fmaxf(m_run, mx);
-        const float m_use = (m_new == kNegInf) ? 0.f : m_new;
-        const float alpha = exp2_fast(m_run - m_use);  // m_run = -inf -> 0
-        l_run *= alpha;
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
-        m_run = m_new;
-      }
-      const float m_use = (m_run == kNegInf) ? 0.f : m_run;
-      float psum = 0.f;
-#pragma unroll
-      for (int kbk = 0; kbk < 2; ++kbk)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          s[kbk][r] = exp2_fast(fmaf(s[kbk][r], kLog2e, -m_use));
-          psum += s[kbk][r];
-        }
-      l_run += psum;
-#pragma unroll
-      for (int step4 = 0; step4 < 4; ++step4) pf[step4] = pack_acc8(s[step4 >> 1], step4 & 1);
-    }
-  };
-  // O^T += V^T P^T for the tile in buffer CUR
-  auto pv_phase = [&](auto stage_tag, const bf16x8* pf) {
-    constexpr int CUR = decltype(stage_tag)::value;
-    if constexpr (D == 128) {
-      pv_sequence_128<CUR * kStage + VkStage<D>::kV>(to, pf, oacc);
-    } else {
-#pragma unroll
-      for (int step4 = 0; step4 < 4; ++step4)
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-          oacc[db] = mfma32(to.load(CUR * kStage + VkStage<D>::kV, step4, db), pf[step4], oacc[db]);
-    }
-  };
-
-  // One step = VALU phase + MFMA phase of tile t < last; CUR is the buffer of stage t.
-  auto step = [&](auto stage_tag) {
-    constexpr int CUR = decltype(stage_tag)::value;
-    const lds_addr next_stage = lds0 + (CUR ^ 1) * kStage;
-    // ---- VALU phase ----
-    if (late) fetch.issue_stage(t + 1, last, next_stage, lds0);
-    // bounds of tile t + 2: requested now, first needed one step from now
-    KeyTileBounds nnb = nb;
-    if (t + 2 <= last) nnb = key_tile_bounds(ctx.meta_b, t + 2);
-    bf16x8 pf[4];
-    softmax_phase(pf);
-    if (!late) dma_wait_all();  // stage t, issued one step ago
-    __builtin_amdgcn_s_barrier();
-    // ---- MFMA phase ----
-    if (!late) fetch.issue_stage(t + 1, last, next_stage, lds0);
-    const bool visit_next = ctx.wave_visits(nb, t + 1);
-    if (visit) pv_phase(stage_tag, pf);
-    if constexpr (D == 128) {
-      if (visit_next) qk_sequence_128<CUR * kStage + VkStage<D>::kK>(ro, qf, s);
-    } else {
-      if (visit_next) scores_t<D>(CUR * kStage + VkStage<D>::kK, ro, qf, s);
-    }
-    if (late) dma_wait_all();  // stage t + 1, issued at the start of this step
-    __builtin_amdgcn_s_barrier();
-    visit = visit_next;
-    kb = nb;
-    nb = nnb;
-    ++t;
-  };
-  const bool any_tile = t <= last;
-  while (t < last) {
-    step(std::integral_constant<int, 0>{});
-    if (t >= last) break;
-    step(std::integral_constant<int, 1>{});
-  }
-  // The step of the last tile: nothing to fetch and no scores to form, so the Q registers are
-  // free, and no later wait of this tile is a wait for memory: the next tile's rows are requested
-  // behind the last such wait and land under the PV product, the stores of O and the next
-  // tile's first copies. (One call site for every path: several would meet in register copies
-  // that wait for the loads.)
-  bf16x8 pf[4];
-  if (any_tile) {
-    softmax_phase(pf);
-    if (!late) dma_wait_all();  // stage t, issued one step ago
-    __builtin_amdgcn_s_barrier();
-  }
-  ahead.request_rows(p, kvh, slice);
-  if (any_tile) {
-    if (visit) {
-      if (((last - ctx.first) & 1) == 0)
-        pv_phase(std::integral_constant<int, 0>{}, pf);
-      else
-        pv_phase(std::integral_constant<int, 1>{}, pf);
-    }
-    __builtin_amdgcn_s_barrier();
-  }
-  if (!late) __builtin_amdgcn_s_barrier();
-  // Every copy of this tile has been waited for by the wavefronts that issued it, so only LDS
-  // traffic has to settle before the stages become store patches (a wait for memory here would
-  // wait for the next tile's loads).
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-
-  const float l_tot = pair_sum(l_run);
-  const bool has = l_tot > 0.f;
-  const float inv = has ? 1.f / l_tot : 0.f;
-  if (ctx.active) {
-    const int le = lane_id_here();
-    const size_t stat = ((size_t)ctx.work.b * p.S + ctx.work.rb * 32 + (le & 31)) * p.Hq + ctx.work.h;
-    if (le < 32) p.lse[stat] = has ? (__logf(l_tot) + m_run * kLn2) : 0.f;
-    const lds_addr patch = lds0 + w * 32 * D * 2;
-    bf16* obase = p.out + (((size_t)ctx.work.b * p.S + ctx.work.rb * 32) * p.Hq + ctx.work.h) * D;
-    store_rows_t<D>(oacc, inv, patch, obase, q_row_stride);
-  }
-  // The store patches overlap the stages of the next item: its copies may start once every
-  // wavefront has read its patch back (LDS reads only; the global stores stay in flight).
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-}
-
 // store_rows_t for the accumulator in a[0:63] (D = 128), one 32-column block in registers at a time.
 CT_DEVICE void fwd_store_rows(float row_scale, lds_addr patch, bf16* gbase, size_t row_stride) {
   constexpr int D = 128, CPR = D / 8;
@@ -910,7 +683,10 @@ CT_DEVICE void fwd_store_rows(float row_scale, lds_addr patch, bf16* gbase, size
   Patch::to_global(patch, l, gbase, row_stride);
 }
 
-// One query tile, interleaved form (D = 128). Arguments as attn_fwd_item_phased.
+// One query tile (kFwdWaves / HS row blocks x HS heads of one KV head), start to finish. `ahead`
+// holds what this tile read ahead on entry and what tile (batch row next_b, tile next_qt) did on
+// return. The request is unconditional (the last tile of a workgroup names itself again): a
+// conditional one would keep the old Q registers alive through the whole tile.
 template <int D, int HS>
 CT_DEVICE void attn_fwd_item(const AttnParams& p, FwdAhead<D, HS>& ahead, int next_b,
                              int next_qt, bool more, int kvh, int slice, const lds_addr lds0,
@@ -1241,10 +1017,11 @@ CT_DEVICE void attn_fwd_item(const AttnParams& p, FwdAhead<D, HS>& ahead, int ne
   }
 }
 
-// Workgroup (group, bin): walks the query tiles of one work bin for one
+// Workgroup (group, bin, member): walks its share of the query tiles of one work bin for one
 // (head slice, KV head) group. The group is the fast index, so with 8 groups a
 // group stays on one XCD (workgroup ids are dealt round robin to the 8 XCDs)
-// and its K/V rows stay in that XCD's L2.
+// and its K/V rows stay in that XCD's L2. A bin's tiles come in order of falling work and are dealt
+// to the bin's members back and forth, which keeps the members' sums together.
 template <int D, int HS>
 __global__ __launch_bounds__(kFwdWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 attn_fwd_kernel(AttnParams p) {
@@ -1256,25 +1033,31 @@ attn_fwd_kernel(AttnParams p) {
   const int nrb = p.S / 32;
   const int slices = (p.Hq / p.Hkv) / HS;
   const int groups = slices * p.Hkv;
-  const int group = blockIdx.x % groups, bin = blockIdx.x / groups;
+  const int group = blockIdx.x % groups, rest = blockIdx.x / groups;
+  const int bin = rest % kBins, member = rest / kBins, members = gridDim.x / (groups * kBins);
   const int kvh = group % p.Hkv, slice = group / p.Hkv;
   const MetaPtr region = meta_const(p.meta + bin_region_offset(p.B, nrb, PB));
   const int tpr = bin_tiles_per_row(nrb, PB);
   const int it_end = uniform(region[bin + 1]);
-  int it = uniform(region[bin]);
+  int it = uniform(region[bin]) + member;
   if (it >= it_end) return;
+  // to the next tile: alternately the two distances of the back and forth walk (both `members`
+  // apart on average; 1 when a bin has one workgroup)
+  int ahead_by = 2 * (members - member) - 1;
   FwdAhead<D, HS> ahead;
   {
     const int item = uniform(region[kBins + 1 + it]);
     ahead.request_bounds(p, item / tpr, kvh, slice, item % tpr);
     ahead.request_rows(p, kvh, slice);
   }
-  for (; it < it_end; ++it) {
-    const int next_item = uniform(region[kBins + 1 + min(it + 1, it_end - 1)]);
-    if constexpr (D == 128)
-      attn_fwd_item<D, HS>(p, ahead, next_item / tpr, next_item % tpr, it + 1 < it_end, kvh, slice, lds0, ro, to);
-    else
-      attn_fwd_item_phased<D, HS>(p, ahead, next_item / tpr, next_item % tpr, kvh, slice, lds0, ro, to);
+  for (;;) {
+    const int next = it + ahead_by;
+    const bool more = next < it_end;
+    const int next_item = uniform(region[kBins + 1 + (more ? next : it)]);
+    attn_fwd_item<D, HS>(p, ahead, next_item / tpr, next_item % tpr, more, kvh, slice, lds0, ro, to);
+    if (!more) break;
+    it = next;
+    ahead_by = 2 * members - ahead_by;
   }
 }
 

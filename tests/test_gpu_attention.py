@@ -260,6 +260,49 @@ def test_kept_work_list(ct, gpu, form):
     assert built == [True, False, False, True, False], launches
 
 
+@pytest.mark.parametrize("shape", [
+    # batch, seq, Hq, Hkv, D: both sides of each size at which the forward changes its form (row blocks of 32
+    # queries per head over the launch: 512 and 7168 for D = 64, 2048 for D = 128; 1280 positions for D = 128)
+    (1, 1024, 16, 8, 64), (9, 128, 15, 5, 64), (2, 384, 48, 6, 64), (7, 1024, 30, 5, 64), (7, 1024, 32, 8, 64),
+    (8, 1024, 28, 14, 64), (8, 1024, 28, 28, 64), (2, 1024, 30, 10, 128), (1, 1920, 32, 4, 128), (2, 1024, 32, 4, 128),
+    (2, 1280, 26, 13, 128), (2, 1280, 26, 26, 128),
+    # 12, 2 and 3 workgroup groups: 2, 4 and 8 workgroups walk a work bin of the large form
+    (2, 1408, 24, 12, 128), (24, 1408, 2, 2, 128), (16, 1408, 3, 3, 128)],
+    ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_forms_of_the_forward(ct, gpu, shape, with_ends):
+    """O and LSE of sampled batch rows and KV heads in every form of the forward; the same bits on every call."""
+
+    batch, seq, q_heads, kv_heads, dim = shape
+    rng = np.random.default_rng(batch * seq + q_heads)
+    generator = torch.Generator().manual_seed(seq)
+    q, k, v = (torch.randn((batch, seq, heads, dim), generator=generator).to(torch.bfloat16)
+               for heads in (q_heads, kv_heads, kv_heads))
+    ids = _layout(rng, batch, seq, holes=True, max_len=seq)
+    ids[0] = 1                                        # one document over a whole row: the longest chain of steps
+    ids[-1, seq // 2:] = 0
+    ends = _random_ends(rng, ids, 9) if with_ends else None
+    profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=with_ends)
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile,
+                                             attention_end=None if ends is None else torch.from_numpy(ends).to(gpu))
+    inputs = [t.to(gpu) for t in (q, k, v)]
+    out, lse = ct.attention_forward_with_lse(*inputs, metadata, scale=0.1)
+    again = ct.attention_forward_with_lse(*inputs, metadata, scale=0.1)
+    assert torch.equal(out, again[0]) and torch.equal(lse, again[1])
+    out, lse = out.cpu(), lse.cpu()
+    group = q_heads // kv_heads
+    for row in sorted({0, batch // 2, batch - 1}):
+        allowed = ref.allowed_from_canonical(ids[row:row + 1], None if ends is None else ends[row:row + 1])
+        head = int(rng.integers(kv_heads))
+        heads = slice(head * group, (head + 1) * group)
+        out_ref, lse_ref = ref.efficient_forward(q[row:row + 1, :, heads], k[row:row + 1, :, head:head + 1],
+                                                 v[row:row + 1, :, head:head + 1], allowed, scale=0.1)
+        assert float((out[row:row + 1, :, heads].float() - out_ref.float()).abs().max()) <= O_ATOL
+        assert float((lse[row:row + 1, :, heads] - lse_ref).abs().max()) <= LSE_ATOL
+        pad = torch.from_numpy(ids[row] == 0)
+        assert (out[row, pad] == 0).all() and (lse[row, pad] == 0).all()
+
+
 @pytest.mark.parametrize("scale", [0.0, 1e-37, -0.09, 1.0])
 @pytest.mark.parametrize("dim", [64, 128])
 def test_any_finite_scale(ct, gpu, bwd_variant, scale, dim):
