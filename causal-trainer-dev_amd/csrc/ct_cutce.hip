@@ -23,6 +23,7 @@
 // written with contiguous stores.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "ct_error.h"
 #include "ct_gemm.hip.h"
@@ -322,6 +323,18 @@ CT_DEVICE void merge_stats(float& m, float& s, float m_o, float s_o) {
   m = m_new;
 }
 
+// The rows of a wavefront's tile in the order of its accumulators (0..3, 8..11, ...; lanes of the other half
+// are 4 rows on), as a scalar address that advances. The stride is opaque: as a loop invariant its
+// 64 multiples are formed in front of the persistent loop and spilled.
+struct TileRows {
+  char* row;
+  int stride;  // bytes
+  CT_DEVICE TileRows(void* origin, int stride_) : row(reinterpret_cast<char*>(origin)), stride(uniform(stride_)) {
+    asm volatile("" : "+s"(stride));
+  }
+  CT_DEVICE void advance(int r) { row += (long)stride * ((r & 3) == 3 ? 5 : 1); }
+};
+
 template <bool CACHE, bool GUARDED>
 __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
                                                           int tiles_per_chunk, float* cache) {
@@ -374,43 +387,50 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
         // a 32-bit lane offset, so the stores need no per-store vector address arithmetic.
         float* origin = cache + (size_t)(v0 + uniform(wm)) * p.n_pad + n0 + uniform(wn);
         const unsigned lane_off = (unsigned)(4 * half * p.n_pad + 4 * j) * 4u;  // bytes
+        TileRows rows(origin, p.n_pad * 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            float* row = origin + (size_t)(32 * i + 8 * (r >> 2) + (r & 3)) * p.n_pad;
-            const f32x4 quad = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
-            store_global16_s<0>(row, lane_off, quad);
+            store_global16_s<0>(rows.row, lane_off, acc.quad(i, r));
+            rows.advance(r);
           }
       }
+      // (The limit is opaque in each pass over the tile and so is the result of every 16 elements: 64
+      // comparison masks kept for the next pass, or values whose use is put off past a branch, do
+      // not fit and spill, and a reload waits for the stores of the logits cache.)
+      const auto fold = [&](auto ragged_tile) {
+        const auto each = [&](int nb, float& result, auto&& f) {
+          int limit = p.V - vbase;
+          if (ragged_tile.value) asm volatile("" : "+v"(limit));
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        float tmax = kNegInfF;
+          for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            if (ragged && vbase + 32 * i + 8 * (r >> 2) + (r & 3) >= p.V) acc.c[i][nb][r] = kNegInfF;
-            tmax = fmaxf(tmax, acc.c[i][nb][r]);
+            for (int r = 0; r < 16; ++r) {
+              const int row = 32 * i + acc_row(r, 0);
+              const float x = acc.value(i, nb, r);
+              f(row, ragged_tile.value && row >= limit ? kNegInfF : x);
+            }
+            asm volatile("" : "+v"(result));
           }
-        const int rel = tgt[nb] - (v0 + wm);
-        if (__any(rel >= 0 && rel < 128)) {
+        };
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (vbase + 32 * i + 8 * (r >> 2) + (r & 3) == tgt[nb]) tl[nb] += acc.c[i][nb][r];
+        for (int nb = 0; nb < 4; ++nb) {
+          float tmax = kNegInfF;
+          each(nb, tmax, [&](int, float x) { tmax = fmaxf(tmax, x); });
+          const int rel = tgt[nb] - (v0 + wm);
+          if (__any(rel >= 0 && rel < 128))
+            each(nb, tl[nb], [&](int row, float x) { tl[nb] += vbase + row == tgt[nb] ? x : 0.f; });
+          const float m_new = fmaxf(m2[nb], tmax * kLog2e);
+          const float m_use = (m_new == kNegInfF) ? 0.f : m_new;
+          float add = 0.f;
+          each(nb, add, [&](int, float x) { add += exp2_fast(x * kLog2e - m_use); });
+          sum[nb] = sum[nb] * exp2_fast(m2[nb] - m_use) + add;
+          m2[nb] = m_new;
         }
-        const float m_new = fmaxf(m2[nb], tmax * kLog2e);
-        const float m_use = (m_new == kNegInfF) ? 0.f : m_new;
-        float add = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) add += exp2_fast(acc.c[i][nb][r] * kLog2e - m_use);
-        sum[nb] = sum[nb] * exp2_fast(m2[nb] - m_use) + add;
-        m2[nb] = m_new;
-      }
+      };
+      if (ragged) fold(std::true_type{});
+      else fold(std::false_type{});
     }
 
     // lanes l and l^32 hold the same rows; then the two wavefronts with equal wn.
@@ -621,25 +641,34 @@ __global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, Cutce
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) target_here |= (unsigned)(tgt[nb] - (v0 + wm)) < 128u;
       const bool plain = v0 + kGemmTile <= p.V && !__any(target_here);
+      TileRows rows(origin, p.n_pad * 2);
+      if (plain) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int vrel = 32 * i + 8 * (r >> 2) + (r & 3);
-          const int v = v0 + wm + 4 * half + vrel;
-          bf16x4 quad;
-          if (plain) {
+          for (int r = 0; r < 16; ++r) {
+            const f32x4 x = acc.quad(i, r);
+            bf16x4 quad;
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-              quad[nb] = (bf16)(fac[nb] * exp2_fast(acc.c[i][nb][r] * kLog2e - lse2[nb]));
-          } else {
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-              quad[nb] = (bf16)((fac[nb] != 0.f && v < p.V)
-                                    ? dlogit(acc.c[i][nb][r], fac[nb], lse2[nb], tgt[nb], v) : 0.f);
+            for (int nb = 0; nb < 4; ++nb) quad[nb] = (bf16)(fac[nb] * exp2_fast(x[nb] * kLog2e - lse2[nb]));
+            store_global8_s<0>(rows.row, lane_off, quad);
+            rows.advance(r);
           }
-          store_global8_s<0>(origin + (size_t)vrel * p.n_pad, lane_off, quad);
-        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int v = v0 + wm + 32 * i + acc_row(r, half);
+            const f32x4 x = acc.quad(i, r);
+            bf16x4 quad;
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+              quad[nb] = (bf16)((fac[nb] != 0.f && v < p.V) ? dlogit(x[nb], fac[nb], lse2[nb], tgt[nb], v) : 0.f);
+            store_global8_s<0>(rows.row, lane_off, quad);
+            rows.advance(r);
+          }
+      }
     }
   }
 }
@@ -783,31 +812,62 @@ CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const Cut
   }
   units.request();
 
-  const int col = c0 + wn + 4 * j;  // hidden sizes are multiples of 128: col < d implies col + 3 < d
-  // f32 to the partial sums or to the sum over slabs (adding what is there from the second slab on),
-  // bf16 to dHidden from the only or the last slab. (The flags are made opaque at every element: one copy
-  // of the 64 stores that branches, instead of a copy for every combination.)
-  float* f32_out = parts > 1 ? sp.hidden_sums + (size_t)split * ((n_act + kGemmTile - 1) / kGemmTile * kGemmTile) * p.d
-                             : sl.dh_acc;
-  const int flags_all = uniform(parts > 1 ? 1 : (sl.mode == 1 || sl.mode == 2 ? 1 : 0) | (sl.mode >= 2 ? 2 : 0));
+  // To the partial sums or the sum over slabs in f32 (adding what is there from the second slab on), from
+  // the only or the last slab to dHidden in bf16. Addresses are a wave-uniform row plus one 32-bit lane
+  // offset: formed per element they spill, and a reload waits for every store in front of it (all GEMM
+  // epilogues in this form, forward and backward at N = 16384, d = 4096, V = 128256: 31.2 -> 29.5 ms;
+  // at N = 999, d = 1024, V = 32003: 447 -> 356 us). Both f32 buffers have rows to the end of the block.
+  const int row0 = n0 + uniform(wm), col0 = c0 + uniform(wn);
+  if (col0 >= p.d) return;  // hidden sizes are multiples of 128: all of the wavefront's columns or none
+  if (parts > 1 || sl.mode != 0) {
+    float* origin = (parts > 1 ? sp.hidden_sums + (size_t)split * ((n_act + kGemmTile - 1) / kGemmTile * kGemmTile) * p.d
+                               : sl.dh_acc) + (size_t)row0 * p.d + col0;
+    const unsigned lane_off = (unsigned)(4 * half * p.d + 4 * j) * 4u;  // bytes
+    TileRows rows(origin, p.d * 4);
+    if (parts > 1 || sl.mode == 1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const f32x4 val = acc.quad(i, r);
+          store_global16_s<0>(rows.row, lane_off, val);
+          rows.advance(r);
+        }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        *reinterpret_cast<f32x4*>(rows.row + lane_off) += acc.quad(i, r);
+        rows.advance(r);
+      }
+    if (sl.mode == 2) return;
+    for (int r = 0; r < 64; ++r) {
+      const int slot = row0 + 32 * (r >> 4) + acc_row(r & 15, half);
+      if (slot >= n_act) continue;
+      const f32x4 val = *reinterpret_cast<const f32x4*>(sl.dh_acc + (size_t)slot * p.d + col0 + 4 * j);
+      bf16x4 out;
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
+      *reinterpret_cast<bf16x4*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col0 + 4 * j) = out;
+    }
+    return;
+  }
+  bf16* columns = sl.dhidden + col0 + 4 * j;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int slot = n0 + wm + 32 * i + acc_row(r, half);
-      if (slot >= n_act || col >= p.d) continue;
-      f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
-      int flags = flags_all;
-      asm volatile("" : "+s"(flags));
-      f32x4* a = reinterpret_cast<f32x4*>(f32_out + (size_t)slot * p.d + col);
-      if (flags & 2) val += *a;
-      if (flags & 1) {
-        *a = val;
-      } else {
+    for (int q = 0; q < 4; ++q) {
+      const int slot = row0 + 32 * i + 8 * q + 4 * half;
+      const i32x4 to = *reinterpret_cast<const i32x4*>(p.idx + slot);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 val = acc.quad(i, 4 * q + e);
         bf16x4 out;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-        *reinterpret_cast<bf16x4*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col) = out;
+        if (slot + e < n_act) *reinterpret_cast<bf16x4*>(columns + (size_t)to[e] * p.d) = out;
       }
     }
 }
@@ -849,21 +909,53 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
   gemm_tile<GUARDED>(A, B, k_begin, k_end, smem, acc);
   units.request();
 
-  const int v = sl.first + v0 + wn + 4 * j;
+  const int row0 = m0 + uniform(wm), col0 = v0 + uniform(wn);
+  if (row0 >= p.d) return;  // hidden sizes are multiples of 128: all of the wavefront's rows or none
+  if (parts > 1) {
+    float* origin = sp.head_sums + ((size_t)split * p.d + row0) * sl.width + col0;
+    const unsigned lane_off = (unsigned)(4 * half * sl.width + 4 * j) * 4u;  // bytes
+    TileRows rows(origin, sl.width * 4);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = m0 + wm + 32 * i + acc_row(r, half);
-      if (m >= p.d) continue;
-      const f32x4 val = {acc.c[i][0][r], acc.c[i][1][r], acc.c[i][2][r], acc.c[i][3][r]};
-      int to_sums = uniform(parts > 1);
-      asm volatile("" : "+s"(to_sums));
-      if (to_sums)
-        *reinterpret_cast<f32x4*>(sp.head_sums + ((size_t)split * p.d + m) * sl.width + (v - sl.first)) = val;
-      else
-        store_dhead4(sl.dhead + (size_t)m * p.V + v, p.V - v, val);
-    }
+      for (int r = 0; r < 16; ++r) {
+        const f32x4 val = acc.quad(i, r);
+        store_global16_s<0>(rows.row, lane_off, val);
+        rows.advance(r);
+      }
+    return;
+  }
+  // The rows of an odd vocabulary start at any multiple of 2 bytes, which an ordinary store may.
+  const int left = p.V - (sl.first + col0 + 4 * j);
+  bf16* origin = sl.dhead + (size_t)row0 * p.V + sl.first + col0;
+  const unsigned lane_off = (unsigned)(4 * half * p.V + 4 * j) * 2u;  // bytes
+  if (left >= 4) {
+    TileRows rows(origin, p.V * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const f32x4 val = acc.quad(i, r);
+        bf16x4 out;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
+        store_global8_s<0>(rows.row, lane_off, out);
+        rows.advance(r);
+      }
+  } else {
+#pragma unroll
+    for (int nb = 0; nb < 3; ++nb)
+      if (nb < left) {
+        TileRows rows(origin, p.V * 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            reinterpret_cast<bf16*>(rows.row + lane_off)[nb] = (bf16)acc.value(i, nb, r);
+            rows.advance(r);
+          }
+      }
+  }
 }
 
 // Both gradients of a slab in one launch (HEAD = false: the head is frozen). The hidden gradient has few,

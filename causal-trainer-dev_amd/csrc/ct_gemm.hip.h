@@ -181,6 +181,22 @@ struct GemmAcc {
 #pragma unroll
       for (int b = 0; b < 4; ++b) c[a][b] = zero16();
   }
+  // Wait states between the compiler's last MFMA and value(), whose read it does not see.
+  CT_DEVICE void settle() {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) asm volatile("" : "+a"(c[a][b]));
+    asm volatile("s_nop 15\n\ts_nop 7");
+  }
+  // An element, read where the call stands. (An epilogue's branches otherwise have the reads and what
+  // is computed from them moved in front of the branch, where 256 of them do not fit and spill.)
+  CT_DEVICE float value(int i, int nb, int r) const {
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(c[i][nb][r]));
+    return v;
+  }
+  CT_DEVICE f32x4 quad(int i, int r) const { return f32x4{value(i, 0, r), value(i, 1, r), value(i, 2, r), value(i, 3, r)}; }
 };
 
 struct GemmFrags {
@@ -295,6 +311,7 @@ CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_a
       cur = nxt;
       nxt = tmp;
     }
+    acc.settle();
   }
 }
 
