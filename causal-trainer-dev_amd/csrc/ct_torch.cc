@@ -57,7 +57,8 @@ inline uint16_t* bits(const Tensor& t) { return ptr<uint16_t>(t); }
 
 inline bool plain(const Tensor& t, at::ScalarType dtype, int64_t dim) {
   return t.defined() && t.is_cuda() && t.scalar_type() == dtype && t.dim() == dim && t.is_contiguous() &&
-         t.layout() == at::kStrided && !t.is_neg() && !t.is_conj();
+         t.layout() == at::kStrided && !t.is_neg() && !t.is_conj() &&
+         !t._fw_grad(0).defined();  // (the operators have no forward-mode derivative: refused, not dropped)
 }
 inline Tensor scratch(size_t bytes, const Tensor& like) {
   return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte).requires_grad(false));

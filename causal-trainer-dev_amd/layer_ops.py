@@ -120,7 +120,10 @@ def rms_norm(x, scale, eps: float, compute_dtype=torch.bfloat16) -> torch.Tensor
         raise ValueError(f"scale must have shape ({x.shape[-1]},), got {tuple(scale.shape)}")
     if x.numel() == 0:
         return torch.empty_like(x)
-    return _lib.native().rms_norm(x.contiguous(), scale.to(device=x.device, dtype=torch.bfloat16).contiguous(), float(eps))
+    y = _lib.native().rms_norm(x.contiguous(), scale.to(device=x.device, dtype=torch.bfloat16).contiguous(), float(eps))
+    if y is None:
+        raise RuntimeError("x and scale must be dense tensors on one ROCm GPU")
+    return y
 
 
 __all__ = ["make_position_ids", "rotary_cos_sin", "apply_rotary_cos_sin", "apply_rotary_embedding", "rms_norm"]

@@ -119,6 +119,20 @@ def test_weight_patterns(ct, gpu, pattern):
         assert not with_c[3].any() and not with_c[4].any()
 
 
+def test_forward_mode_is_refused(ct, gpu):
+    """The operators have no forward-mode derivative: a dual input raises instead of losing its tangent."""
+
+    from torch.autograd import forward_ad
+    hidden, head, targets, weights = _case(7, 64, 128, 300)
+    x = hidden.reshape(1, 64, 128).to(gpu)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(RuntimeError):
+            ct.pallas_cut_linear_cross_entropy(dual, head.to(gpu), targets.reshape(1, 64).to(gpu), weights.reshape(1, 64).to(gpu))
+        with pytest.raises(RuntimeError):
+            ct.rms_norm(dual, torch.ones(128, dtype=torch.bfloat16, device=gpu), 1e-6)
+
+
 def test_head_layout_vocab_major(ct, gpu):
     """The operator with the head given as [V, d] (a checkpoint's layout): the same loss and hidden
     gradient as with [d, V], bit for bit (the kernels see the same transposed copy), and the head's
