@@ -119,6 +119,20 @@ def test_weight_patterns(ct, gpu, pattern):
         assert not with_c[3].any() and not with_c[4].any()
 
 
+def test_small_hidden_large_logits_match_with_and_without_cache(ct, gpu):
+    """Where the operator does without the logits cache (hidden <= 640, logits beyond 256 MB) the results
+    are those of the recomputing form: the same f32 logits of the same products."""
+
+    hidden, head, targets, weights = _case(9, 1100, 128, 65537)
+    arguments = (targets.reshape(2, 550).to(gpu), weights.reshape(2, 550).to(gpu))
+    outcomes = []
+    for cache in (True, False):
+        x, w = hidden.reshape(2, 550, 128).to(gpu).requires_grad_(True), head.to(gpu).requires_grad_(True)
+        nll, _ = ct.pallas_cut_linear_cross_entropy(x, w, *arguments, logits_cache=cache)
+        outcomes.append((nll.detach(), *torch.autograd.grad(nll, (x, w))))
+    assert all(torch.equal(a, b) for a, b in zip(*outcomes))
+
+
 def test_forward_mode_is_refused(ct, gpu):
     """The operators have no forward-mode derivative: a dual input raises instead of losing its tangent."""
 
