@@ -122,6 +122,7 @@ SYMBOLS = {
     "ct_abi_version": (c_int32, []),
     "ct_calibration_copy": (c_int32, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "ct_canonicalize_segment_ids": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
+    "ct_transpose16": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "ct_segment_positions": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "ct_shifted_targets_scratch_bytes": (c_size_t, [c_int32, c_int32]),
     "ct_shifted_targets_and_weights": (c_int32, [c_void_p, POINTER(ShiftedTargetsArgs)]),

@@ -515,14 +515,14 @@ struct CutCeNode : Node {
   SavedVariable hidden, head, targets, weights;
   Tensor lse;
   MaybeTensor cache;
-  bool compaction = false, trainable = true;
+  bool compaction = false, trainable = true, vocab_major = false;
   int64_t workspace_bytes = -1;
   variable_list apply(variable_list&& grads) override {
     const Tensor X = hidden.unpack(), W = head.unpack(), T = targets.unpack(), w = weights.unpack();
     const Tensor dy = gradient(grads[0], {}, at::kFloat, X);
     const MaybeTensor logits = std::exchange(cache, std::nullopt);
     auto [dx, dw] = cutce_backward(X, W, T, w, lse, dy, compaction, trainable, workspace_bytes, logits);
-    return {dx, dw ? *dw : Tensor()};
+    return {dx, !dw ? Tensor() : vocab_major ? dw->t() : *dw};
   }
   void release_variables() override {
     hidden.reset_data();
@@ -542,32 +542,42 @@ struct CutCeNode : Node {
 // 512: 120 / 124; 130 x 76000, 512: 180 / 188; 1000 x 32003, 512: 225 / 224.
 bool cache_pays(const ct_cutce_shape& shape, size_t bytes) { return shape.hidden > 640 || bytes <= ((size_t)256 << 20); }
 
+// vocab_major: head is [V, d]; the kernels get a transposed copy, the gradient goes back as a view of theirs.
 std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Tensor& head, const Tensor& targets,
                                                  const Tensor& weights, bool trainable, bool compaction, bool use_cache,
-                                                 int64_t cache_limit, int64_t forward_bytes, int64_t backward_bytes) {
+                                                 int64_t cache_limit, int64_t forward_bytes, int64_t backward_bytes,
+                                                 bool vocab_major) {
   if (!plain(hidden, at::kBFloat16, 3) || !plain(head, at::kBFloat16, 2) || !plain(targets, at::kInt, 2) ||
       !plain(weights, at::kFloat, 2) || hidden.numel() == 0 || head.numel() == 0 || hidden.size(2) % 128 ||
-      head.size(0) != hidden.size(2) || targets.sizes() != hidden.sizes().slice(0, 2) || weights.sizes() != targets.sizes() ||
-      head.device() != hidden.device() || targets.device() != hidden.device() || weights.device() != hidden.device())
+      head.size(vocab_major ? 1 : 0) != hidden.size(2) || targets.sizes() != hidden.sizes().slice(0, 2) ||
+      weights.sizes() != targets.sizes() || head.device() != hidden.device() || targets.device() != hidden.device() ||
+      weights.device() != hidden.device())
     return std::nullopt;
   const bool graph = needs_graph({hidden, head});
-  MaybeTensor cache;
-  if (use_cache && (hidden.requires_grad() || head.requires_grad())) {
-    const ct_cutce_shape shape = cut_shape(hidden, head);
-    const size_t bytes = ct_cutce_logits_cache_bytes(&shape);
-    if ((int64_t)bytes <= cache_limit && graph && cache_pays(shape, bytes)) cache = scratch(bytes, hidden);
+  Tensor columns = head;  // [d, V]
+  if (vocab_major) {
+    const c10::DeviceGuard guard(head.device());
+    columns = at::empty({head.size(1), head.size(0)}, head.options().requires_grad(false));
+    check(ct_transpose16(current_stream(), bits(head), (int32_t)head.size(0), (int32_t)head.size(1), bits(columns)));
   }
-  auto [nll, weight_sum, lse] = cutce_forward(hidden, head, targets, weights, compaction, cache, forward_bytes);
+  MaybeTensor cache;
+  if (use_cache && graph) {
+    const ct_cutce_shape shape = cut_shape(hidden, columns);
+    const size_t bytes = ct_cutce_logits_cache_bytes(&shape);
+    if ((int64_t)bytes <= cache_limit && cache_pays(shape, bytes)) cache = scratch(bytes, hidden);
+  }
+  auto [nll, weight_sum, lse] = cutce_forward(hidden, columns, targets, weights, compaction, cache, forward_bytes);
   if (graph) {
     auto node = graph_node<CutCeNode>({hidden, head});
     node->hidden = SavedVariable(hidden, false);
-    node->head = SavedVariable(head, false);
+    node->head = SavedVariable(columns, false);
     node->targets = SavedVariable(targets, false);
     node->weights = SavedVariable(weights, false);
     node->lse = lse;
     node->cache = cache;
     node->compaction = compaction;
     node->trainable = trainable;
+    node->vocab_major = vocab_major;
     node->workspace_bytes = backward_bytes;
     torch::autograd::set_history(nll, node);
   }

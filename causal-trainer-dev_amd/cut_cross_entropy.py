@@ -110,18 +110,18 @@ def _workspaces(rows: int, hidden: int, vocab: int, local_chunk_size: int):
     return int(forward), int(backward)
 
 
-def _cut(hidden, head, targets, weights, trainable, compaction, cache, chunk):
+def _cut(hidden, head, targets, weights, trainable, compaction, cache, chunk, layout):
     """The operator on plain arguments (what the native side checks), None for any other."""
 
     try:
         if targets.shape != weights.shape or hidden.shape[:-1] != targets.shape:
             return None
-        rows, width, vocab = targets.numel(), hidden.shape[-1], head.shape[1]
+        rows, width, vocab = targets.numel(), hidden.shape[-1], head.shape[layout == "dv"]
         if rows == 0 or width == 0 or vocab == 0:
             return None
         sizes = (-1, -1) if chunk == 0 else _workspaces(rows, width, vocab, chunk)
         return _lib.native().cut_ce(hidden, head, targets, weights, bool(trainable), bool(compaction),
-                                    bool(cache) and chunk == 0, LOGITS_CACHE_LIMIT_BYTES, *sizes)
+                                    bool(cache) and chunk == 0, LOGITS_CACHE_LIMIT_BYTES, *sizes, layout == "vd")
     except (AttributeError, IndexError, TypeError):
         return None     # (something is wrong with the arguments: the validation says what)
 
@@ -139,13 +139,13 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
     ``head_layout="vd"``: lm_head_kernel is ``[V, d]`` (a checkpoint's ``[out, in]`` layout, which the
     reference transposes once at load, src/causal_trainer/checkpointing/huggingface.py:1-6). The
     kernels read ``[d, V]`` with the vocabulary contiguous, so this layout costs a transposing copy
-    of the head per call and one of its gradient in the backward (2 B read + 2 B written per element
-    each, about 0.4 ms per GB on this part); its gradient comes back as ``[V, d]``.
+    of the head per call (2 B read + 2 B written per element); its gradient comes back as ``[V, d]``, a view
+    of the kernels' ``[d, V]``.
     """
 
-    if mesh is None and head_layout == "dv" and type(local_chunk_size) is int and local_chunk_size >= 0:
+    if mesh is None and head_layout in ("dv", "vd") and type(local_chunk_size) is int and local_chunk_size >= 0:
         out = _cut(hidden_states, lm_head_kernel, targets, weights, lm_head_trainable, sparse_compaction, logits_cache,
-                   local_chunk_size)
+                   local_chunk_size, head_layout)
         if out is not None:
             return out
     if head_layout not in ("dv", "vd"):
@@ -153,7 +153,7 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
     if head_layout == "vd":
         if lm_head_kernel.ndim != 2:
             raise ValueError("lm_head_kernel must have shape [vocab, hidden]")
-        lm_head_kernel = lm_head_kernel.t()   # (made contiguous below; autograd transposes the gradient back)
+        lm_head_kernel = lm_head_kernel.t()   # (a head that is not dense: made contiguous below)
 
     local_chunk_size = _integer(local_chunk_size, "local_chunk_size must be a static non-negative integer")
     if local_chunk_size < 0:
@@ -190,7 +190,7 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
     if active:
         raise ValueError(f"this build runs on one GPU; mesh axes larger than 1: {active}")
     out = _cut(hidden_states.contiguous(), lm_head_kernel.contiguous(), targets.contiguous(), weights.contiguous(),
-               lm_head_trainable, sparse_compaction, logits_cache, local_chunk_size)
+               lm_head_trainable, sparse_compaction, logits_cache, local_chunk_size, "dv")
     if out is None:
         raise RuntimeError("Cut cross-entropy is available only for dense tensors on one ROCm GPU")
     return out

@@ -249,6 +249,11 @@ int32_t ct_canonicalize_segment_ids(void* stream, const int32_t* attention_mask,
 int32_t ct_segment_positions(void* stream, const int32_t* attention_mask, const int32_t* segment_ids,
                              int32_t batch, int32_t seq, int32_t* position_ids);
 
+/* dst [cols][rows] = the transpose of src [rows][cols], 16-bit elements: a head in a checkpoint's [vocab, hidden]
+ * layout as the cut cross-entropy takes it (the reference transposes at load,
+ * src/causal_trainer/checkpointing/huggingface.py:1-6). */
+int32_t ct_transpose16(void* stream, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst);
+
 typedef struct ct_shifted_targets_args {
   const int32_t* input_ids;       /* int32 [batch, seq] */
   const int32_t* attention_mask;  /* int32 [batch, seq] or NULL (all valid); valid iff == 1 */

@@ -119,6 +119,17 @@ def test_weight_patterns(ct, gpu, pattern):
         assert not with_c[3].any() and not with_c[4].any()
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 128), (63, 128), (64, 64), (65, 200), (137, 77), (700, 384)])
+def test_transpose16(ct, gpu, rows, cols):
+    """The transposed copy of a [vocab, hidden] head: whole tiles, ragged ones, rows at odd addresses."""
+
+    source = torch.randint(-2 ** 15, 2 ** 15, (rows, cols), dtype=torch.int16, device=gpu)
+    copy = torch.empty((cols, rows), dtype=torch.int16, device=gpu)
+    ct._lib.check(ct._lib.load().ct_transpose16(torch.cuda.current_stream().cuda_stream, source.data_ptr(), rows, cols,
+                                                copy.data_ptr()))
+    assert torch.equal(copy, source.t())
+
+
 def test_small_hidden_large_logits_match_with_and_without_cache(ct, gpu):
     """Where the operator does without the logits cache (hidden <= 640, logits beyond 256 MB) the results
     are those of the recomputing form: the same f32 logits of the same products."""
