@@ -545,9 +545,7 @@ static int launch_delta(hipStream_t stream, const bf16* out, const bf16* dout, f
 template <int D>
 static int launch_schedule(hipStream_t stream, const AttnParams& p, int kvh_side_by_side) {
   LaunchScope scope7("attn_dkv_schedule_kernel", stream);
-  hipLaunchKernelGGL(attn_dkv_schedule_kernel, dim3(1), dim3(1024), 0, stream, p.meta, p.B, p.S,
-                     kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
-                     p.dkv_entries, p.dq_counters, kDqCounters);
+  hipLaunchKernelGGL(attn_dkv_schedule_kernel, dim3(1), dim3(1024), 0, stream, p, kvh_side_by_side);
   return scope7.done();
 }
 
@@ -568,19 +566,25 @@ static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool 
   return launch_dkv_reduce<D>(stream, p);
 }
 
-// Stored-dS form: row statistics; the work list; then per pass of KV heads the dK/dV kernel, which
+// Stored-dS form: row statistics and the work list; then per pass of KV heads the dK/dV kernel, which
 // leaves its dS blocks in the region, and dQ as a product over those blocks; the sum of split chunks.
+// (That sum at the end of the last dQ launch instead: dQ 17 -> 29 us at [2, 1024], 210 -> 221 us at [4, 4096],
+// against the 4.5 and 22 us of its own launch.)
 template <int D>
 static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pass, bool wide, bool list_kept) {
-  {
-    const long tiles = (long)p.B * p.Hq * (p.S / (D == 128 ? 64 : 128));
+  const long tiles = (long)p.B * p.Hq * (p.S / (D == 128 ? 64 : 128));
+  const unsigned stats_groups = (unsigned)(tiles < 8192 ? tiles : 8192);
+  int rc;
+  if (list_kept) {
     LaunchScope scope("attn_bwd_stats_kernel", stream);
-    hipLaunchKernelGGL((attn_bwd_stats_kernel<D>), dim3((unsigned)(tiles < 8192 ? tiles : 8192)), dim3(256), 0,
-                       stream, p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale(p.scale));
-    int rc = scope.done();
-    if (rc) return rc;
+    hipLaunchKernelGGL((attn_bwd_stats_kernel<D>), dim3(stats_groups), dim3(256), 0, stream, p, exponent_scale(p.scale));
+    rc = scope.done();
+  } else {
+    LaunchScope scope("attn_dkv_schedule_kernel", stream);  // (the list and the statistics)
+    hipLaunchKernelGGL((attn_bwd_setup_kernel<D>), dim3(1 + (stats_groups + 3) / 4), dim3(1024), 0, stream, p, kvh_per_pass,
+                       exponent_scale(p.scale));
+    rc = scope.done();
   }
-  int rc = list_kept ? 0 : launch_schedule<D>(stream, p, kvh_per_pass);
   if (rc) return rc;
   for (int base = 0; base < p.Hkv; base += kvh_per_pass) {
     p.kvh_base = base;

@@ -381,12 +381,9 @@ CT_DEVICE int dkv_split_count(int items, int target) {
 
 // Builds the dK/dV work list (one workgroup of 1024 threads): chunk target from
 // the total amount of work, chunk count per tile, entries bucketed by
-// decreasing work.
-__global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(const int* meta, int B, int S,
-                                                                 int Hkv, int g, int max_entries,
-                                                                 int max_partials, int* header,
-                                                                 int2* entries, int* zeroed,
-                                                                 int zeroed_count) {
+// decreasing work. Clears the dQ kernel's work counters.
+CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int max_entries, int max_partials, int* header,
+                            int2* entries, int* zeroed, int zeroed_count) {
   for (int i = threadIdx.x; i < zeroed_count; i += 1024) zeroed[i] = 0;  // dQ's work counters
   __shared__ long long red[16];  // one value per wavefront
   __shared__ int hist[256];
@@ -511,6 +508,25 @@ __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(const int* meta
     }
     __syncthreads();
   }
+}
+
+__global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, int kvh_side_by_side) {
+  dkv_schedule(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
+               p.dkv_entries, p.dq_counters, kDqCounters);
+}
+
+// The work list and, in the other workgroups, the row statistics: two independent passes in one launch. The
+// list is one workgroup's chain of barriers (7 us at [2, 1024], the statistics 4 us), so the shorter of the
+// two costs nothing.
+template <int D>
+__global__ __launch_bounds__(1024) void attn_bwd_setup_kernel(AttnParams p, int kvh_side_by_side, float exponent_scale) {
+  if (blockIdx.x == 0) {
+    dkv_schedule(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
+                 p.dkv_entries, p.dq_counters, kDqCounters);
+    return;
+  }
+  bwd_stats_tiles<D>(p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale,
+                     (blockIdx.x - 1) * 4 + (threadIdx.x >> 8), (gridDim.x - 1) * 4, threadIdx.x & 255);
 }
 
 // f32 partial sums of one chunk of a split key tile.

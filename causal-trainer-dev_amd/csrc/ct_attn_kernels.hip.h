@@ -1112,18 +1112,16 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* out, const 
 // workgroups take the heads of the same positions, so the rows in flight at a time are one
 // contiguous stretch of `out` and `dout`.
 template <int D>
-__global__ __launch_bounds__(256) void attn_bwd_stats_kernel(const bf16* out, const bf16* dout,
-                                                             const float* lse, float* neg_delta,
-                                                             float* neg_lse_scaled, int B, int S,
-                                                             int Hq, float exponent_scale) {
+CT_DEVICE void bwd_stats_tiles(const bf16* out, const bf16* dout, const float* lse, float* neg_delta, float* neg_lse_scaled,
+                               int B, int S, int Hq, float exponent_scale, long first, long stride, int tid) {
   constexpr int LPR = D / 8;          // lanes per row
   constexpr int RPP = 256 / LPR;      // rows per pass of the workgroup
   constexpr int kUnroll = 4;
   constexpr int kTile = kUnroll * RPP;  // 64 (D = 128) or 128 (D = 64) positions: divides S
   const int tiles_per_row = S / kTile;
   const long tiles = (long)B * tiles_per_row * Hq;
-  const int r0 = threadIdx.x / LPR, chunk = threadIdx.x % LPR;
-  for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+  const int r0 = tid / LPR, chunk = tid % LPR;
+  for (long tile = first; tile < tiles; tile += stride) {
     const int h = (int)(tile % Hq);
     const long rest = tile / Hq;
     const int st = (int)(rest % tiles_per_row), b = (int)(rest / tiles_per_row);
@@ -1151,6 +1149,12 @@ __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(const bf16* out, co
       }
     }
   }
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void attn_bwd_stats_kernel(AttnParams p, float exponent_scale) {
+  bwd_stats_tiles<D>(p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale, blockIdx.x, gridDim.x,
+                     threadIdx.x);
 }
 
 }  // namespace ct
