@@ -525,9 +525,8 @@ static int launch_dkv(hipStream_t stream, const AttnParams& p, bool wide) {
 
 template <int D>
 static int launch_dkv_reduce(hipStream_t stream, const AttnParams& p) {
-  const int grid = p.dkv_max_entries * p.Hkv;
   LaunchScope scope9("attn_dkv_reduce_kernel", stream);
-  hipLaunchKernelGGL((attn_dkv_reduce_kernel<D>), dim3(grid), dim3(256), 4 * 32 * D * 2, stream, p);
+  hipLaunchKernelGGL((attn_dkv_reduce_kernel<D>), dim3(kReduceGroups), dim3(256), 0, stream, p);
   return scope9.done();
 }
 
@@ -568,8 +567,6 @@ static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool 
 
 // Stored-dS form: row statistics and the work list; then per pass of KV heads the dK/dV kernel, which
 // leaves its dS blocks in the region, and dQ as a product over those blocks; the sum of split chunks.
-// (That sum at the end of the last dQ launch instead: dQ 17 -> 29 us at [2, 1024], 210 -> 221 us at [4, 4096],
-// against the 4.5 and 22 us of its own launch.)
 template <int D>
 static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pass, bool wide, bool list_kept) {
   const long tiles = (long)p.B * p.Hq * (p.S / (D == 128 ? 64 : 128));

@@ -542,53 +542,84 @@ CT_DEVICE size_t dkv_partial_offset(int slot, int Hkv, int kvh, int wave) {
 }
 
 // Adds the chunks of every split key tile in chunk order (fixed order: the result does not
-// depend on timing) and writes dK, dV. One workgroup per (entry, KV head); only the entry of
-// chunk 0 of a split tile has work.
+// depend on timing) and writes dK, dV. Bound by the partials' bytes (64 or 128 KB a chunk, from the memory-side
+// cache), so the work is spread thin: a wavefront takes 32 keys x 32 columns of one tensor, four chunks
+// of which it has in flight, and every workgroup finds the split tiles in the work list by itself (a few
+// hundred entries). One workgroup per tile and KV head walked up to 32 chunks on a few dozen compute units:
+// [1, 7424, 6/1 heads of 64] 52 -> 12 us, [1, 2432, 16/4 of 64] 25 -> 7, [4, 4096, 32/8 of 128] 22 -> 15,
+// [2, 2432, 16/16 of 128] 19 -> 14, [4, 4224, 8/1 of 128] 25 -> 16.
+constexpr int kReduceGroups = 1024;
 template <int D>
 __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
-  extern __shared__ __align__(16) char smem_raw[];
-  const lds_addr lds0 = lds_address_of(smem_raw);
-  const int l = lane_id(), w = threadIdx.x >> 6;
+  constexpr int kMaxSplitTiles = kDkvSlots + 8;  // dkv_layout: at most half of max_partials <= 2 (kDkvSlots + 2)
+  constexpr int kPieces = 2 * 4 * (D / 32);      // (tensor, wavefront of the dK/dV kernel, 32 columns)
+  __shared__ int2 split[kMaxSplitTiles];
+  __shared__ int wave_count[4];
+  __shared__ __align__(16) bf16 patches[4][32 * 32];
+  const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
-  const int kvh = blockIdx.x % p.Hkv, entry = blockIdx.x / p.Hkv;
   // This is the last kernel of a backward call: it leaves the dQ kernel's work counters at zero,
   // so that a later call on the same workspace can keep the work list and skip the kernel that
   // builds it (and clears the counters).
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < kDqCounters; i += blockDim.x) p.dq_counters[i] = 0;
-  if (entry >= uniform(p.dkv_header[0])) return;
-  const int2 work_entry = p.dkv_entries[entry];
-  const int tile = uniform(work_entry.x), packed = uniform(work_entry.y);
-  const int chunk = packed & 255, nsplit = (packed >> 8) & 255, slot0 = (unsigned)packed >> 16;
-  if (chunk != 0 || nsplit <= 1) return;
-  const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
-  f32x16 dkacc[D / 32], dvacc[D / 32];
+  const int entries = uniform(p.dkv_header[0]);
+  int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
+  for (int base = 0; base < entries; base += 256) {
+    const int i = base + threadIdx.x;
+    const int2 entry = i < entries ? p.dkv_entries[i] : make_int2(0, 0);
+    const bool mine = (entry.y & 255) == 0 && ((entry.y >> 8) & 255) > 1;  // chunk 0 of several
+    const unsigned long long ballot = __ballot(mine);
+    if (l == 0) wave_count[w] = __popcll(ballot);
+    __syncthreads();
+    int at = tiles + __popcll(ballot & ((1ull << l) - 1ull));
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
-    dkacc[db] = zero16();
-    dvacc[db] = zero16();
+    for (int k = 0; k < 4; ++k) {
+      if (k < w) at += wave_count[k];
+      tiles += wave_count[k];
+    }
+    if (mine && at < kMaxSplitTiles) split[at] = entry;
+    __syncthreads();
   }
-  for (int c = 0; c < nsplit; ++c) {
-    const float* src = p.dkv_partials + dkv_partial_offset<D>(slot0 + c, p.Hkv, kvh, w) + l * 4;
+  tiles = uniform(min(tiles, kMaxSplitTiles));
+  for (int item = blockIdx.x * 4 + w; item < tiles * p.Hkv * kPieces; item += gridDim.x * 4) {
+    const int piece = item % kPieces, kvh = item / kPieces % p.Hkv;
+    const int2 entry = split[item / kPieces / p.Hkv];
+    const int tile = uniform(entry.x), nsplit = uniform((entry.y >> 8) & 255), slot0 = uniform((unsigned)entry.y >> 16);
+    const int db = piece % (D / 32), keys = piece / (D / 32) % 4, tensor = piece / (D / 32) / 4;
+    const float* src = p.dkv_partials + dkv_partial_offset<D>(slot0, p.Hkv, kvh, keys) + tensor * DkvPartial<D>::kPerTensor +
+                       db * 1024 + l * 4;
+    const size_t chunk_stride = (size_t)p.Hkv * DkvPartial<D>::kPerChunk;
+    f32x4 sum[4] = {};
+    for (int c = 0; c < nsplit; c += 4) {
+      f32x4 v[4][4];
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(src + (db * 4 + q4) * 256);
-        const f32x4 cv = *reinterpret_cast<const f32x4*>(src + DkvPartial<D>::kPerTensor + (db * 4 + q4) * 256);
+        for (int q = 0; q < 4; ++q)
+          v[k][q] = c + k < nsplit ? *reinterpret_cast<const f32x4*>(src + (c + k) * chunk_stride + q * 256) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          dkacc[db][4 * q4 + e] += a[e];
-          dvacc[db][4 * q4 + e] += cv[e];
-        }
-      }
+      for (int k = 0; k < 4; ++k)
+        if (c + k < nsplit)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[q] += v[k][q];
+    }
+    // lane (j, half) holds column j of the keys 8 q + 4 half + e: through LDS to rows of 64 bytes
+    bf16* patch = patches[w];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) patch[(8 * q + 4 * half + e) * 32 + j] = (bf16)sum[q][e];
+    __builtin_amdgcn_wave_barrier();
+    const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
+    bf16* out = (tensor ? p.dv : p.dk) + (((size_t)b * p.S + (kt * 4 + keys) * 32) * p.Hkv + kvh) * D + db * 32;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int row = (l >> 2) + 16 * n, chunk = (l & 3) * 8;
+      store_global16(out + (size_t)row * p.Hkv * D + chunk, *reinterpret_cast<const u32x4*>(patch + row * 32 + chunk));
+    }
   }
-  const lds_addr patch = lds0 + w * 32 * D * 2;
-  const size_t kv_row_stride = (size_t)p.Hkv * D;
-  const size_t out_off = (((size_t)b * p.S + (kt * 4 + w) * 32) * p.Hkv + kvh) * D;
-  store_rows<D>(dkacc, patch, p.dk + out_off, kv_row_stride);
-  __builtin_amdgcn_wave_barrier();
-  store_rows<D>(dvacc, patch, p.dv + out_off, kv_row_stride);
 }
 
 // Byte address of the dS block (key block rb with table entries ds_off / q_first, query block qb)
