@@ -273,7 +273,9 @@ CT_DEVICE void qdo_fetch(const TileDma<kQueryTile, D / 8>& dma, const AttnParams
                       : which == 1 ? reinterpret_cast<const char*>(p.delta + head_major)
                       : which == 2 ? reinterpret_cast<const char*>(p.seg + row_major)
                                    : reinterpret_cast<const char*>(p.end + row_major);
-    const unsigned lane = threadIdx.x & 63;
+    // (head dimension 64, at its register limit: an offset kept for the loop is spilled, and its reload
+    // waits for the copies)
+    const unsigned lane = D == 64 ? (unsigned)lane_id_here() : threadIdx.x & 63;
     if (lane < 8) dma16_s(src, lane * 16, stage + QdoStage<D>::kLse + which * (kQueryTile * 4));
   }
 }
@@ -632,8 +634,12 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
 
 // SPILL: every (key block, query block) step also stores its bf16 dS block to the dS region, for
 // attn_dq_blocks_kernel.
+//
+// Head dimension 64 is held to 168 registers, three workgroups per compute unit (LDS has room for four): its steps are
+// short and the vector ALU waits between the matrix instructions. With 177 registers and two workgroups:
+// [2, 15616, 12/2 heads of 64] 544 -> 445 us, [1, 7424, 6/1] 95 -> 80.
 template <int D, bool SPILL>
-__global__ __launch_bounds__(256, 2) void attn_dkv_kernel(AttnParams p) {
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr lds0 = lds_address_of(smem_raw);
   constexpr int kStage = QdoStage<D>::kBytes;
