@@ -496,7 +496,8 @@ __global__ __launch_bounds__(kMergeSlots * kMergeParts) void cutce_merge_kernel(
   }
   float m = kNegInfF, s = 0.f, t = 0.f;
   if (wr != 0.f) {
-    for (int c = piece; c < chunks; c += kMergeParts) {
+#pragma unroll 4
+    for (int c = piece; c < chunks; c += kMergeParts) {  // (several chunks' loads in flight)
       const float* e = part + ((size_t)c * p.n_pad + slot) * 3;
       merge_stats(m, s, e[0], e[1]);
       t += e[2];
