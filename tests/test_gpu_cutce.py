@@ -144,6 +144,29 @@ def test_small_hidden_large_logits_match_with_and_without_cache(ct, gpu):
     assert all(torch.equal(a, b) for a, b in zip(*outcomes))
 
 
+@pytest.mark.parametrize("ignored", [0.0, 0.4, 1.0])
+def test_operator_leaves_ignored_rows_out(ct, gpu, ignored):
+    """The operator's results do not depend on sparse_compaction, and agree with the full-logits oracle."""
+
+    hidden, head, targets, weights = _case(13, 300, 128, 501)
+    targets = targets.clamp(min=0)     # (rows that _case ignores count here)
+    weights = torch.where(torch.rand(300, generator=torch.Generator().manual_seed(3)) < ignored, 0.0, 1.0)
+    arguments = (targets.reshape(1, 300).to(gpu), weights.reshape(1, 300).to(gpu))
+    outcomes = []
+    for compaction in (False, True):
+        x, w = hidden.reshape(1, 300, 128).to(gpu).requires_grad_(True), head.to(gpu).requires_grad_(True)
+        nll, total = ct.pallas_cut_linear_cross_entropy(x, w, *arguments, sparse_compaction=compaction)
+        outcomes.append((nll.detach(), total, *torch.autograd.grad(nll, (x, w))))
+    assert all(torch.equal(a, b) for a, b in zip(*outcomes))
+    assert float(outcomes[0][1]) == float(weights.sum())
+    if ignored < 1:
+        _, dh_pure, dw_pure = ref.full_logits_loss_and_grads(hidden, head, targets, weights, 1.0)
+        assert relative_l2(outcomes[0][2].cpu().reshape(300, 128), dh_pure) <= GRAD_RTOL
+        assert relative_l2(outcomes[0][3].cpu(), dw_pure) <= GRAD_RTOL
+    else:
+        assert not outcomes[0][2].any() and not outcomes[0][3].any() and float(outcomes[0][0]) == 0
+
+
 def test_forward_mode_is_refused(ct, gpu):
     """The operators have no forward-mode derivative: a dual input raises instead of losing its tangent."""
 
