@@ -196,6 +196,8 @@ def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None,
 
     query ``[B, S, Hq, D]``, key / value ``[B, S, Hkv, D]``, all bf16 on a ROCm
     device; returns ``[B, S, Hq, D]`` bf16. Gradients flow to query, key, value.
+    Its backward takes dQ from stored dS blocks (up to 4 GiB of scratch) where that is the faster form: rows of up to
+    4096 positions, longer ones at head dimension 128 or with few query rows.
     ``backward_workspace`` (this build's addition, a :class:`BackwardWorkspace`) lets the layers of
     a model that share ``metadata`` share the scratch buffer of the backward and the work list in it.
     """

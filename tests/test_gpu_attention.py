@@ -260,6 +260,31 @@ def test_kept_work_list(ct, gpu, form):
     assert built == [True, False, False, True, False], launches
 
 
+@pytest.mark.parametrize("shape,form", [
+    ((1, 4224, 2, 1, 128), "from_ds"), ((1, 4096, 14, 2, 64), "from_ds"), ((1, 4224, 2, 1, 64), "from_ds"),
+    ((1, 4224, 12, 4, 64), "recompute"), ((1, 8192, 6, 2, 64), "from_ds"), ((1, 8320, 2, 2, 64), "recompute")],
+    ids=lambda v: v if isinstance(v, str) else "S%d_Hq%d_Hkv%d_D%d" % v[1:])
+def test_form_of_the_operators_backward(ct, gpu, shape, form):
+    """Both sides of the sizes at which the operator asks for another form of its backward: its gradients are
+    those of the form that the rule names, bit for bit, and both forms agree."""
+
+    batch, seq, q_heads, kv_heads, dim = shape
+    ids = _layout(np.random.default_rng(seq), batch, seq, max_len=900)
+    generator = torch.Generator().manual_seed(q_heads)
+    q, k, v, dout = (torch.randn((batch, seq, heads, dim), generator=generator).to(torch.bfloat16).to(gpu)
+                     for heads in (q_heads, kv_heads, kv_heads, q_heads))
+    profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=False)
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile)
+    inputs = tuple(t.clone().requires_grad_(True) for t in (q, k, v))
+    gradients = torch.autograd.grad(ct.efficient_attention(*inputs, metadata, profile=profile), inputs, dout)
+    out, lse = ct.attention_forward_with_lse(q, k, v, metadata, scale=dim ** -0.5)
+    results = {f: ct.attention_backward(q, k, v, metadata, out, lse, dout, scale=dim ** -0.5, dq_form=f)
+               for f in ("recompute", "from_ds")}
+    assert all(torch.equal(a, b) for a, b in zip(gradients, results[form]))
+    for a, b in zip(results["recompute"], results["from_ds"]):
+        assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
+
+
 @pytest.mark.parametrize("shape", [
     # batch, seq, Hq, Hkv, D: both sides of each size at which the forward changes its form (row blocks of 32
     # queries per head over the launch: 512 and 7168 for D = 64, 2048 for D = 128; 1280 positions for D = 128)
