@@ -441,7 +441,9 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   for (int t = tid; t < ntiles; t += 1024) local += items_of(t);
   const long long total = block_sum(local);
   long long want = (total * Hkv + kDkvSlots - 1) / kDkvSlots;  // one compute slot's fair share
-  int target = (int)min((long long)INT_MAX / 2, max((long long)kDkvMinChunk, want));
+  const long long pairs = (long long)ntiles * Hkv;  // (key tile, KV head)
+  const int least = pairs <= kDkvSlots / 16 ? kDkvMinChunk / 4 : pairs <= kDkvSlots / 2 ? kDkvMinChunk / 2 : kDkvMinChunk;
+  int target = (int)min((long long)INT_MAX / 2, max((long long)least, want));
 
   // Entry and partial-slot counts for this target; coarsen the target if they overflow the
   // space the host reserved (cannot happen for target >= want, kept as a guard).

@@ -128,7 +128,12 @@ __host__ __device__ inline size_t meta_total_ints(int B, int nrb) {
 // the partial sums.
 // ---------------------------------------------------------------------------
 constexpr int kDkvSlots = 512;     // workgroups resident at once on the device (2 per CU)
-constexpr int kDkvMinChunk = 16;   // items
+// Fewest items (steps of one query block) of a chunk: a step takes 1 us, a chunk's sums 64 or 128 KB written
+// and read. With fewer (key tile, KV head) pairs than compute units chunks are half as long, with
+// hardly any a quarter: the chain of steps is then what the launch waits for. Backward, us, with 16 / 8 / 4:
+// [2, 1024, 8/8 heads of 64] (128 pairs) 49 / 45 / 48, [4, 768, 12/4 of 128] (96) 65 / 58 / 62, [2, 512, 2/1 of 128] (8)
+// 57 / 50 / 46, [1, 384, 4/1 of 64] (3) 43 / 39 / 36; [6, 2176, 4/4 of 128] (408) 68 / 73 / 78.
+constexpr int kDkvMinChunk = 16;
 constexpr int kDkvMaxSplit = 32;
 constexpr int kDkvKeys = 128;      // keys per dK/dV tile
 
