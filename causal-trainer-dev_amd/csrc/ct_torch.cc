@@ -45,6 +45,15 @@ inline void check(int status) {
 
 inline void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// Whether the current stream is being captured into a graph.
+inline bool capturing() {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &status) == hipSuccess)
+    return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // (the default stream while another one is captured)
+  return true;
+}
+
 template <class T>
 inline T* ptr(const Tensor& t) {
   return static_cast<T*>(t.data_ptr());
@@ -97,11 +106,14 @@ inline bool needs_graph(std::initializer_list<Tensor> inputs) {
 // attention
 // ---------------------------------------------------------------------------------------------
 
-// Scratch of the attention backward kept from call to call (BackwardWorkspace in Python).
+// Scratch of the attention backward kept from call to call (BackwardWorkspace in Python), and what the
+// dK/dV work list in it was built from. The metadata tensor is held, not remembered by its address: an
+// address goes to the next batch's metadata as soon as the last one's are dropped. Writes to it in place
+// show in its version counter (inference tensors have none: their list is built on every call).
 struct KeptWorkspace {
   Tensor buffer;
-  bool built = false;
-  std::tuple<void*, uint32_t, std::vector<int64_t>, int, size_t, float> built_for;
+  Tensor listed;  // undefined: no list
+  std::tuple<uint32_t, std::vector<int64_t>, int, size_t, float> listed_for;
 };
 
 struct AttnShape {
@@ -170,20 +182,22 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
     }
   }
   Tensor dq = fresh(q), dk = fresh(k), dv = fresh(v), delta = fresh(lse), workspace;
+  // (A graph keeps the addresses it was captured with and runs its kernels out of order with later calls:
+  // it gets scratch of its own, from its own pool, and builds its own lists.)
+  if (kept && capturing()) kept = nullptr;
   if (kept) {
-    // (the version counter of the metadata tensor changes when it is written in place)
-    const uint32_t version = bounds.is_inference() ? 0 : bounds.unsafeGetTensorImpl()->version_counter().current_version();
-    auto wanted = std::make_tuple(bounds.data_ptr(), version,
+    const bool versioned = !bounds.is_inference();
+    auto wanted = std::make_tuple(versioned ? bounds.unsafeGetTensorImpl()->version_counter().current_version() : 0u,
                                   std::vector<int64_t>{s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim}, variant, bytes,
                                   (float)scale);
     if (!kept->buffer.defined() || (size_t)kept->buffer.numel() < bytes || kept->buffer.device() != q.device()) {
       kept->buffer = scratch(bytes, q);
-      kept->built = false;
+      kept->listed.reset();
     }
     workspace = kept->buffer;
-    if (kept->built && kept->built_for == wanted) variant |= CT_ATTN_BWD_WORK_LIST_KEPT;
-    kept->built = false;  // (until the call below has been made)
-    kept->built_for = std::move(wanted);
+    if (versioned && kept->listed.is_same(bounds) && kept->listed_for == wanted) variant |= CT_ATTN_BWD_WORK_LIST_KEPT;
+    kept->listed.reset();  // (until the call below has been made)
+    kept->listed_for = std::move(wanted);
   } else {
     workspace = scratch(bytes, q);
   }
@@ -211,7 +225,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
   a.scale = (float)scale;
   a.variant = variant;
   check(ct_attn_bwd(current_stream(), &a));
-  if (kept) kept->built = true;
+  if (kept) kept->listed = bounds;
   return {dq, dk, dv, delta};
 }
 
@@ -668,9 +682,10 @@ std::optional<std::tuple<Tensor, Tensor>> shifted_targets(const Tensor& tokens, 
   return std::make_tuple(targets, weights);
 }
 
-// (tile bounds, query summary, key summary); segment ids and ends already int32, contiguous, on the GPU
-std::tuple<Tensor, Tensor, Tensor> attention_metadata(const Tensor& segments, const MaybeTensor& ends, int64_t block_q,
-                                                      int64_t block_kv) {
+// (tile bounds, query summary, key summary, whether a graph's replays will write them); segment ids and ends
+// already int32, contiguous, on the GPU
+std::tuple<Tensor, Tensor, Tensor, bool> attention_metadata(const Tensor& segments, const MaybeTensor& ends,
+                                                            int64_t block_q, int64_t block_kv) {
   const c10::DeviceGuard guard(segments.device());
   const int32_t batch = (int32_t)segments.size(0), seq = (int32_t)segments.size(1);
   Tensor bounds = ints({(int64_t)(ct_attn_meta_bytes(batch, seq) / 4)}, segments);
@@ -679,13 +694,13 @@ std::tuple<Tensor, Tensor, Tensor> attention_metadata(const Tensor& segments, co
   if (block_q % 32 == 0 && block_kv % 32 == 0) {
     check(ct_attn_prepare_summaries(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, ptr<int32_t>(bounds),
                                     (int32_t)block_q, ptr<int32_t>(q_summary), (int32_t)block_kv, ptr<int32_t>(kv_summary)));
-    return {bounds, q_summary, kv_summary};
+    return {bounds, q_summary, kv_summary, capturing()};
   }
   check(ct_attn_prepare(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, ptr<int32_t>(bounds)));
   check(ct_attn_block_summary(stream, ptr<int32_t>(segments), ptr<int32_t>(ends), batch, seq, (int32_t)block_q,
                               ptr<int32_t>(q_summary)));
   check(ct_attn_block_summary(stream, ptr<int32_t>(segments), nullptr, batch, seq, (int32_t)block_kv, ptr<int32_t>(kv_summary)));
-  return {bounds, q_summary, kv_summary};
+  return {bounds, q_summary, kv_summary, capturing()};
 }
 
 }  // namespace

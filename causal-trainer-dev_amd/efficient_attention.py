@@ -87,7 +87,9 @@ def prepare_attention_metadata(canonical_segment_ids, *, mesh, profile,
         if ends.shape != segments.shape:
             raise ValueError("attention_end must match canonical_segment_ids")
 
-    bounds, q_summary, kv_summary = _lib.native().attention_metadata(segments, ends, block_q, outer)
+    bounds, q_summary, kv_summary, captured = _lib.native().attention_metadata(segments, ends, block_q, outer)
+    if captured:
+        bounds.written_by_replays = True    # (see _kept)
     return AttentionMetadata(
         query_segment_ids=segments,
         kv_segment_ids=segments,
@@ -157,14 +159,18 @@ class BackwardWorkspace:
     ``efficient_attention(..., backward_workspace=...)``): the first call builds the list, later
     calls with the same metadata, shape and form tell the library to keep it
     (``CT_ATTN_BWD_WORK_LIST_KEPT``), which saves a launch per call. The calls that share one must
-    run on one stream, one after the other."""
+    run on one stream, one after the other. The object holds the metadata tensor its list was built
+    from. Inside a graph capture, and for metadata prepared in one (every replay writes them again,
+    unseen), it is left out: such calls take scratch of their own and build their own list."""
 
     def __init__(self):
         self._kept = _lib.native().KeptWorkspace()
 
 
-def _kept(workspace):
-    return None if workspace is None else workspace._kept
+def _kept(workspace, metadata):
+    if workspace is None or getattr(metadata.tile_bounds, "written_by_replays", False):
+        return None
+    return workspace._kept
 
 
 @functools.lru_cache(maxsize=1024)
@@ -185,7 +191,7 @@ def _attend(query, key, value, metadata, profile, scale, workspace):
     try:
         blocks = _plain_profile(query.shape, key.shape, profile, metadata.attention_end is not None)
         return _lib.native().attention(query, key, value, *metadata[:6], *blocks,
-                                       query.shape[-1] ** -0.5 if scale is None else scale, _kept(workspace))
+                                       query.shape[-1] ** -0.5 if scale is None else scale, _kept(workspace, metadata))
     except (AttributeError, IndexError, TypeError, ValueError):
         return None     # (something is wrong with the arguments: the validation says what)
 
@@ -269,7 +275,7 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     dq, dk, dv, delta = _lib.native().attention_backward(
         query.detach(), key.detach(), value.detach(), metadata.query_segment_ids, metadata.attention_end,
         metadata.tile_bounds, out.detach(), lse, dout.contiguous(), resolved, _DKV_KERNELS[dkv_kernel] | _DQ_FORMS[dq_form],
-        -1 if workspace_bytes is None else int(workspace_bytes), _kept(workspace))
+        -1 if workspace_bytes is None else int(workspace_bytes), _kept(workspace, metadata))
     if with_delta:
         batch, sequence, q_heads, _ = query.shape
         return dq, dk, dv, delta.view(batch, q_heads, sequence)

@@ -260,6 +260,77 @@ def test_kept_work_list(ct, gpu, form):
     assert built == [True, False, False, True, False], launches
 
 
+def _kept_list_layers(ct, gpu):
+    """A layer's backward with a shared workspace and without one: ``layer(metadata, kept)`` runs both and compares."""
+
+    batch, seq, q_heads, kv_heads, dim = 2, 1024, 4, 2, 128
+    rng = np.random.default_rng(5)
+    layouts = [torch.from_numpy(_layout(rng, batch, seq, max_len=longest)).to(gpu) for longest in (900, 100, 400, 60)]
+    q, dout = (_bf16(rng.standard_normal((batch, seq, q_heads, dim))).to(gpu) for _ in range(2))
+    k, v = (_bf16(rng.standard_normal((batch, seq, kv_heads, dim))).to(gpu) for _ in range(2))
+    profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=False)
+
+    def prepare(ids):
+        return ct.prepare_attention_metadata(ids, mesh=None, profile=profile)
+
+    def backward(metadata, kept):
+        out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+        return ct.attention_backward(q, k, v, metadata, out, lse, dout, workspace=kept)
+
+    def layer(metadata, kept):
+        torch.cuda.synchronize()
+        for got, want in zip(backward(metadata, kept), backward(metadata, None)):
+            assert torch.equal(got, want)
+
+    return layouts, prepare, backward, layer
+
+
+def test_kept_work_list_of_dropped_metadata(ct, gpu):
+    """A program that drops a batch's metadata before it makes the next one's gets the same memory again, were it
+    not held: the list of the batch before must not be taken for the new one's."""
+
+    layouts, prepare, _, layer = _kept_list_layers(ct, gpu)
+    kept, address = ct.BackwardWorkspace(), None
+    for ids in layouts:
+        metadata = prepare(ids)
+        assert metadata.tile_bounds.data_ptr() != address     # (still the workspace's)
+        address = metadata.tile_bounds.data_ptr()
+        layer(metadata, kept)
+        layer(metadata, kept)
+        del metadata
+    with torch.inference_mode():      # no version counter that would tell of writes
+        metadata = prepare(layouts[0].clone())
+        layer(metadata, kept)
+        metadata.tile_bounds.copy_(prepare(layouts[1]).tile_bounds)
+        metadata.query_segment_ids.copy_(layouts[1])
+        layer(metadata, kept)
+
+
+def test_kept_work_list_and_graphs(ct, gpu):
+    """Metadata that a graph's replays write are never taken for those a list was built from, and a captured
+    backward keeps clear of the shared buffer and its list."""
+
+    layouts, prepare, backward, layer = _kept_list_layers(ct, gpu)
+    kept = ct.BackwardWorkspace()
+    static = layouts[0].clone()
+    eager = prepare(layouts[0])
+    layer(eager, kept)                      # (a list is there)
+    preparation, step = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(preparation):
+        replayed = prepare(static)
+    with torch.cuda.graph(step):
+        captured = backward(eager, kept)
+    for ids in layouts:
+        static.copy_(ids)
+        preparation.replay()
+        layer(replayed, kept)
+        layer(prepare(ids), kept)           # (another list in the shared buffer)
+        step.replay()
+        torch.cuda.synchronize()
+        for got, want in zip(captured, backward(eager, None)):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("shape,form", [
     ((1, 4224, 2, 1, 128), "from_ds"), ((1, 4096, 14, 2, 64), "from_ds"), ((1, 4224, 2, 1, 64), "from_ds"),
     ((1, 4224, 12, 4, 64), "recompute"), ((1, 8192, 6, 2, 64), "from_ds"), ((1, 8320, 2, 2, 64), "recompute")],
