@@ -1184,6 +1184,22 @@ static int validate_cutce(const char* fn, const ct_cutce_shape& s) {
   return CT_OK;
 }
 
+// The GEMM loop addresses the 256 rows of a k-contiguous tile by 32-bit byte offsets (KcLoader::voff).
+// Rows in place are offsets from the tile's first row, so it is their stride that is limited ...
+constexpr int kMaxRowStride = 1 << 23;  // elements: 255 rows of 2 bytes each stay below 4 GiB
+// ... and gathered rows are offsets from the tensor's first.
+static bool gather_reaches(const ct_cutce_shape& s) {
+  return (size_t)s.rows * (size_t)s.hidden * sizeof(bf16) <= (size_t)1 << 32;
+}
+// The gradients read such tiles of the head (stride: its padded vocabulary) and, for dHead, of G^T
+// (stride: its padded rows).
+static int validate_cutce_strides(const char* fn, const ct_cutce_shape& s, bool with_head) {
+  if (vocab_tile_count(s.vocab) > kMaxRowStride / kGemmTile || (with_head && s.rows > kMaxRowStride))
+    return fail(CT_UNSUPPORTED, "%s: a vocabulary of more than 2^23 (got %d), or dHead over more than 2^23 rows (got %d)",
+                fn, s.vocab, s.rows);
+  return CT_OK;
+}
+
 static bool is_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // The GEMM kernels need more than the default 64 KB of LDS; each says so once per device.
@@ -1254,7 +1270,7 @@ static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, con
   CutceParams p = {};
   p.hidden = reinterpret_cast<const bf16*>(hidden);
   p.head = HeadView{reinterpret_cast<const bf16*>(head), nullptr, s.vocab, 0, false};
-  p.compact = compact ? 1 : 0;
+  p.compact = compact && gather_reaches(s);  // (rows in place give the same results)
   p.targets = targets;
   p.weights = weights;
   p.N = s.rows;
@@ -1422,6 +1438,7 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
                  a->workspace,
              "ct_cutce_bwd: null pointer");
   int rc = validate_cutce("ct_cutce_bwd", a->shape);
+  if (!rc) rc = validate_cutce_strides("ct_cutce_bwd", a->shape, a->dhead != nullptr);
   if (rc) return rc;
   CT_REQUIRE(is_aligned16(a->workspace) && is_aligned16(a->dhidden),
              "ct_cutce_bwd: workspace and dhidden must be 16-byte aligned");

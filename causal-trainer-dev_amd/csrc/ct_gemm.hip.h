@@ -50,7 +50,7 @@ struct GemmSmem {
 // In both loaders thread t owns the 16-byte LDS slots t + 256 n of the tile
 // (n < 4): slot P holds physical chunk P % CPR of row P / CPR, i.e. logical
 // chunk (P % CPR) ^ swizzle(row); voff[n] is the byte offset of that chunk
-// from `base` at k = 0.
+// from `base` at k = 0 (32 bits: the host checks sizes and strides against it).
 struct KcLoader {
   static constexpr int CPR = kGemmBK / 8;  // 4
   static constexpr int NCH = 4;

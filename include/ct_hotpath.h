@@ -451,7 +451,8 @@ typedef struct ct_cutce_fwd_args {
   void* workspace;
   size_t workspace_bytes;
   ct_cutce_shape shape;
-  int32_t sparse_compaction; /* gather active rows first (same results) */
+  int32_t sparse_compaction; /* gather active rows first (same results; rows of a hidden tensor of
+                              * more than 4 GiB stay in place, where the gather does not reach) */
   void* logits_cache;        /* NULL, or ct_cutce_logits_cache_bytes() of device memory to fill */
   size_t logits_cache_bytes;
 } ct_cutce_fwd_args;

@@ -167,6 +167,37 @@ def test_operator_leaves_ignored_rows_out(ct, gpu, ignored):
         assert not outcomes[0][2].any() and not outcomes[0][3].any() and float(outcomes[0][0]) == 0
 
 
+@pytest.mark.parametrize("cache", [False, True], ids=["recompute", "cache"])
+def test_hidden_states_beyond_4_gib(ct, gpu, cache):
+    """Active rows on both sides of the 4 GiB that a 32-bit offset reaches (row 262144 at this width)."""
+
+    rows, width, vocab = 262144 + 300, 8192, 40
+    line = (1 << 32) // (2 * width)
+    active = torch.cat([torch.arange(5), torch.arange(1000, line, 1000), torch.arange(line - 40, line + 150, 3),
+                        torch.tensor([rows - 1])])
+    hidden, head, targets, _ = _case(31, active.numel(), width, vocab, hidden_scale=0.5)
+    targets, weights = targets.clamp(min=0), torch.linspace(0.5, 1.5, active.numel())
+    x = torch.zeros((4, rows // 4, width), dtype=torch.bfloat16, device=gpu)
+    at = active.to(gpu)
+    x.view(rows, width)[at] = hidden.to(gpu)
+    all_targets = torch.full((rows,), -100, dtype=torch.int32, device=gpu)
+    all_weights = torch.zeros(rows, device=gpu)
+    all_targets[at], all_weights[at] = targets.to(gpu), weights.to(gpu)
+    x.requires_grad_(True)
+    w = head.to(gpu).requires_grad_(True)
+    nll, total = ct.pallas_cut_linear_cross_entropy(x, w, all_targets.view(4, -1), all_weights.view(4, -1),
+                                                    sparse_compaction=True, logits_cache=cache)
+    dx, dw = torch.autograd.grad(nll, (x, w))
+    nll_ref, weight_ref, _ = ref.cut_forward(hidden, head, targets, weights)
+    assert float(nll.detach()) == pytest.approx(float(nll_ref), rel=LOSS_RTOL)
+    assert float(total) == pytest.approx(float(weight_ref), rel=1e-6)
+    _, dh_pure, dw_pure = ref.full_logits_loss_and_grads(hidden, head, targets, weights, 1.0)
+    dx = dx.view(rows, width)
+    assert torch.equal(dx.any(dim=1).nonzero().flatten(), at)
+    assert relative_l2(dx[at].cpu(), dh_pure) <= GRAD_RTOL
+    assert relative_l2(dw.cpu(), dw_pure) <= GRAD_RTOL
+
+
 def test_forward_mode_is_refused(ct, gpu):
     """The operators have no forward-mode derivative: a dual input raises instead of losing its tangent."""
 

@@ -84,6 +84,22 @@ def test_argument_validation_happens_before_any_launch(ct):
     assert library.ct_cutce_fwd(None, ctypes.byref(cargs)) == ct._lib.CT_WORKSPACE_TOO_SMALL
 
 
+def test_cutce_backward_refuses_strides_beyond_its_32_bit_offsets(ct):
+    """Tiles of 256 rows, 2 bytes an element: a stride of 2^23 is the last whose offsets stay below 4 GiB. In reach,
+    the call gets as far as its workspace."""
+
+    library = ct._lib.load()
+    args = ct._lib.CutceBwdArgs(workspace_bytes=16)
+    for field in ("hidden", "head", "targets", "weights", "lse", "dy", "dhidden", "workspace"):
+        setattr(args, field, 4096)       # never dereferenced: validation fails first
+    for rows, vocab, dhead, status in (
+            (10, 1 << 23, 4096, ct._lib.CT_WORKSPACE_TOO_SMALL), (10, (1 << 23) + 1, 4096, ct._lib.CT_UNSUPPORTED),
+            (10, (1 << 23) + 1, None, ct._lib.CT_UNSUPPORTED), (1 << 23, 50, 4096, ct._lib.CT_WORKSPACE_TOO_SMALL),
+            ((1 << 23) + 1, 50, 4096, ct._lib.CT_UNSUPPORTED), ((1 << 23) + 1, 50, None, ct._lib.CT_WORKSPACE_TOO_SMALL)):
+        args.shape, args.dhead = ct._lib.CutceShape(rows, 128, vocab), dhead
+        assert library.ct_cutce_bwd(None, ctypes.byref(args)) == status, (rows, vocab, dhead, library.ct_last_error())
+
+
 def test_profile_resolution_matches_reference_tiers(ct):
     # tests/kernels/test_efficient_attention.py:226-249: S=4096, 32 heads, tp=4 -> h8, q256, kv 512/256
     profile = ct.resolve_attention_profile((4, 4096, 32, 128), (4, 4096, 1, 128), {"tp": 4})
