@@ -250,17 +250,17 @@ int operator_form(const AttnShape& s, bool with_ends) {
 }
 
 struct AttentionNode : Node {
-  SavedVariable q, k, v, out;
-  Tensor lse, segments, bounds;
+  SavedVariable q, k, v, out, lse;
+  Tensor segments, bounds;
   MaybeTensor ends;
   double scale = 0;
   std::shared_ptr<KeptWorkspace> kept;
 
   variable_list apply(variable_list&& grads) override {
     const auto self = shared_from_this();
-    const Tensor Q = q.unpack(), K = k.unpack(), V = v.unpack(), O = out.unpack(self);
+    const Tensor Q = q.unpack(), K = k.unpack(), V = v.unpack(), O = out.unpack(self), L = lse.unpack();
     auto [dq, dk, dv, delta] =
-        attention_backward(Q, K, V, segments, ends, bounds, O, lse, gradient(grads[0], O.sizes(), at::kBFloat16, O), scale,
+        attention_backward(Q, K, V, segments, ends, bounds, O, L, gradient(grads[0], O.sizes(), at::kBFloat16, O), scale,
                            operator_form(attn_shape(Q, K), ends && ends->defined()), -1, kept.get());
     return {dq, dk, dv};
   }
@@ -269,7 +269,7 @@ struct AttentionNode : Node {
     k.reset_data();
     v.reset_data();
     out.reset_data();
-    lse.reset();
+    lse.reset_data();
   }
   std::string name() const override { return "EfficientAttentionBackward"; }
 };
@@ -301,7 +301,7 @@ MaybeTensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
     node->q = SavedVariable(q, false);
     node->k = SavedVariable(k, false);
     node->v = SavedVariable(v, false);
-    node->lse = lse;
+    node->lse = SavedVariable(lse, false);
     node->segments = query_ids;
     node->ends = ends;
     node->bounds = *bounds;
@@ -438,22 +438,21 @@ ct_sparse_ce_args sparse_args(const Tensor& logits, const Tensor& targets, const
 }
 
 struct SparseCeNode : Node {
-  SavedVariable logits, targets, weights;
-  Tensor lse;
+  SavedVariable logits, targets, weights, lse;
   variable_list apply(variable_list&& grads) override {
-    const Tensor X = logits.unpack(), T = targets.unpack(), W = weights.unpack();
+    const Tensor X = logits.unpack(), T = targets.unpack(), W = weights.unpack(), L = lse.unpack();
     const c10::DeviceGuard guard(X.device());
     const Tensor dy = gradient(grads[0], T.sizes(), at::kFloat, X);
     Tensor dlogits = fresh(X);
     const ct_sparse_ce_args a = sparse_args(X, T, W);
-    check(ct_sparse_ce_bwd(current_stream(), &a, ptr<float>(lse), ptr<float>(dy), dlogits.data_ptr()));
+    check(ct_sparse_ce_bwd(current_stream(), &a, ptr<float>(L), ptr<float>(dy), dlogits.data_ptr()));
     return {dlogits};
   }
   void release_variables() override {
     logits.reset_data();
     targets.reset_data();
     weights.reset_data();
-    lse.reset();
+    lse.reset_data();
   }
   std::string name() const override { return "SparseCrossEntropyBackward"; }
 };
@@ -472,7 +471,7 @@ MaybeTensor sparse_ce(const Tensor& logits, const Tensor& targets, const Tensor&
     node->logits = SavedVariable(logits, false);
     node->targets = SavedVariable(targets, false);
     node->weights = SavedVariable(weights, false);
-    node->lse = lse;
+    node->lse = SavedVariable(lse, false);
     torch::autograd::set_history(loss, node);
   }
   return loss;
@@ -545,16 +544,15 @@ std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tenso
 // The reference's residual (src/causal_trainer/kernels/cut_cross_entropy.py:587-593) plus, when it
 // fits, the f32 logits cache, which the first backward gives back.
 struct CutCeNode : Node {
-  SavedVariable hidden, head, targets, weights;
-  Tensor lse;
+  SavedVariable hidden, head, targets, weights, lse;
   MaybeTensor cache;
   bool compaction = false, trainable = true, vocab_major = false;
   int64_t workspace_bytes = -1;
   variable_list apply(variable_list&& grads) override {
-    const Tensor X = hidden.unpack(), W = head.unpack(), T = targets.unpack(), w = weights.unpack();
+    const Tensor X = hidden.unpack(), W = head.unpack(), T = targets.unpack(), w = weights.unpack(), L = lse.unpack();
     const Tensor dy = gradient(grads[0], {}, at::kFloat, X);
     const MaybeTensor logits = std::exchange(cache, std::nullopt);
-    auto [dx, dw] = cutce_backward(X, W, T, w, lse, dy, compaction, trainable, workspace_bytes, logits);
+    auto [dx, dw] = cutce_backward(X, W, T, w, L, dy, compaction, trainable, workspace_bytes, logits);
     return {dx, !dw ? Tensor() : vocab_major ? dw->t() : *dw};
   }
   void release_variables() override {
@@ -562,7 +560,7 @@ struct CutCeNode : Node {
     head.reset_data();
     targets.reset_data();
     weights.reset_data();
-    lse.reset();
+    lse.reset_data();
     cache.reset();
   }
   std::string name() const override { return "CutCrossEntropyBackward"; }
@@ -606,7 +604,7 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
     node->head = SavedVariable(columns, false);
     node->targets = SavedVariable(targets, false);
     node->weights = SavedVariable(weights, false);
-    node->lse = lse;
+    node->lse = SavedVariable(lse, false);
     node->cache = cache;
     node->compaction = compaction;
     node->trainable = trainable;
