@@ -11,6 +11,7 @@
 // or normalises, and calls again.
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -42,6 +43,31 @@ struct StatusError : std::exception {
 inline void check(int status) {
   if (status != CT_OK) throw StatusError(status);
 }
+
+py::handle error_class;  // CtError of _lib.py, kept for the life of the process
+// Makes `e` the current Python error (the caller holds the GIL).
+void set_python_error(const StatusError& e) {
+  if (!error_class) return PyErr_SetString(PyExc_RuntimeError, e.what());
+  py::object error = error_class(e.status, e.message);
+  PyErr_SetObject(error_class.ptr(), error.ptr());
+}
+
+// A node whose library errors reach the caller of the backward as CtError: autograd hands on Python
+// errors as they are and any other exception as a plain RuntimeError.
+struct OperatorNode : Node {
+  virtual variable_list differentiate(variable_list&& grads) = 0;
+  variable_list apply(variable_list&& grads) final {
+    try {
+      return differentiate(std::move(grads));
+    } catch (const StatusError& e) {
+      py::gil_scoped_acquire gil;
+      set_python_error(e);
+      python_error raised;
+      raised.persist();  // (this thread's Python state may end with the GIL's release)
+      throw raised;
+    }
+  }
+};
 
 inline void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
@@ -249,14 +275,14 @@ int operator_form(const AttnShape& s, bool with_ends) {
   return bytes > 0 && bytes <= kFromDsWorkspaceCap ? CT_ATTN_BWD_DQ_FROM_DS : 0;
 }
 
-struct AttentionNode : Node {
+struct AttentionNode : OperatorNode {
   SavedVariable q, k, v, out, lse;
   Tensor segments, bounds;
   MaybeTensor ends;
   double scale = 0;
   std::shared_ptr<KeptWorkspace> kept;
 
-  variable_list apply(variable_list&& grads) override {
+  variable_list differentiate(variable_list&& grads) override {
     const auto self = shared_from_this();
     const Tensor Q = q.unpack(), K = k.unpack(), V = v.unpack(), O = out.unpack(self), L = lse.unpack();
     auto [dq, dk, dv, delta] =
@@ -316,10 +342,10 @@ MaybeTensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
 // ---------------------------------------------------------------------------------------------
 // RMS norm and rotary embedding
 // ---------------------------------------------------------------------------------------------
-struct RmsNormNode : Node {
+struct RmsNormNode : OperatorNode {
   SavedVariable x, scale;
   double eps = 0;
-  variable_list apply(variable_list&& grads) override {
+  variable_list differentiate(variable_list&& grads) override {
     const Tensor X = x.unpack(), W = scale.unpack();
     const c10::DeviceGuard guard(X.device());
     const int64_t hidden = X.size(-1), rows = X.numel() / hidden;
@@ -380,12 +406,12 @@ std::tuple<Tensor, Tensor> rotate(const Tensor& q, const Tensor& k, const Tensor
   return {q_out, k_out};
 }
 
-struct RotaryNode : Node {
+struct RotaryNode : OperatorNode {
   SavedVariable cosine, sine;
   std::vector<int64_t> q_shape, k_shape;
   int style = 0;
   double q_scale = 1;
-  variable_list apply(variable_list&& grads) override {
+  variable_list differentiate(variable_list&& grads) override {
     const Tensor C = cosine.unpack(), S = sine.unpack();
     const Tensor dq = gradient(grads[0], q_shape, at::kBFloat16, C), dk = gradient(grads[1], k_shape, at::kBFloat16, C);
     auto [q, k] = rotate(dq, dk, C, S, style, true, q_scale);
@@ -437,9 +463,9 @@ ct_sparse_ce_args sparse_args(const Tensor& logits, const Tensor& targets, const
   return a;
 }
 
-struct SparseCeNode : Node {
+struct SparseCeNode : OperatorNode {
   SavedVariable logits, targets, weights, lse;
-  variable_list apply(variable_list&& grads) override {
+  variable_list differentiate(variable_list&& grads) override {
     const Tensor X = logits.unpack(), T = targets.unpack(), W = weights.unpack(), L = lse.unpack();
     const c10::DeviceGuard guard(X.device());
     const Tensor dy = gradient(grads[0], T.sizes(), at::kFloat, X);
@@ -543,12 +569,12 @@ std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tenso
 
 // The reference's residual (src/causal_trainer/kernels/cut_cross_entropy.py:587-593) plus, when it
 // fits, the f32 logits cache, which the first backward gives back.
-struct CutCeNode : Node {
+struct CutCeNode : OperatorNode {
   SavedVariable hidden, head, targets, weights, lse;
   MaybeTensor cache;
   bool compaction = false, trainable = true, vocab_major = false;
   int64_t workspace_bytes = -1;
-  variable_list apply(variable_list&& grads) override {
+  variable_list differentiate(variable_list&& grads) override {
     const Tensor X = hidden.unpack(), W = head.unpack(), T = targets.unpack(), w = weights.unpack(), L = lse.unpack();
     const Tensor dy = gradient(grads[0], {}, at::kFloat, X);
     const MaybeTensor logits = std::exchange(cache, std::nullopt);
@@ -704,15 +730,12 @@ std::tuple<Tensor, Tensor, Tensor, bool> attention_metadata(const Tensor& segmen
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  static py::handle error_class;  // CtError of _lib.py, kept for the life of the process
   m.def("set_error_class", [](py::object cls) { error_class = cls.release(); });
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);
     } catch (const StatusError& e) {
-      if (!error_class) return PyErr_SetString(PyExc_RuntimeError, e.what());
-      py::object error = error_class(e.status, e.message);
-      PyErr_SetObject(error_class.ptr(), error.ptr());
+      set_python_error(e);
     }
   });
   py::class_<KeptWorkspace, std::shared_ptr<KeptWorkspace>>(m, "KeptWorkspace").def(py::init<>());

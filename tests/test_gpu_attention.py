@@ -537,6 +537,23 @@ def test_custom_vjp_through_autograd(ct, gpu):
         ct.efficient_attention(q, k, v, metadata, profile=ct.AttentionKernelProfile(4, 128, 128, 128))
 
 
+def test_library_errors_of_a_backward_are_ct_errors(ct, gpu):
+    """What the library refuses inside a backward (here a cotangent that is not 16-byte aligned) reaches the caller with
+    its status, and the next backward runs."""
+
+    generator = torch.Generator(device=gpu).manual_seed(3)
+    q, k, v, dout = (torch.randn((1, 128, 2, 64), generator=generator, device=gpu).to(torch.bfloat16) for _ in range(4))
+    inputs = tuple(t.requires_grad_(True) for t in (q, k, v))
+    ids = torch.ones((1, 128), dtype=torch.int32, device=gpu)
+    metadata = ct.prepare_attention_metadata(ids, mesh=None, profile=ct.resolve_attention_profile(q.shape, k.shape, None))
+    shifted = torch.empty(dout.numel() + 1, dtype=torch.bfloat16, device=gpu)[1:].view(dout.shape).copy_(dout)
+    out = ct.efficient_attention(*inputs, metadata)
+    with pytest.raises(ct._lib.CtError, match="16-byte aligned") as raised:
+        torch.autograd.grad(out, inputs, shifted, retain_graph=True)
+    assert raised.value.status == ct._lib.CT_INVALID_ARGUMENT and "16-byte aligned" in raised.value.message
+    assert all(g.isfinite().all() for g in torch.autograd.grad(out, inputs, dout))
+
+
 def test_metadata_matches_oracle_bit_exact(ct, gpu):
     rng = np.random.default_rng(51)
     # known answers of the reference first (tests/kernels/test_efficient_attention.py:446-480)
