@@ -179,19 +179,23 @@ std::tuple<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, c
 constexpr int64_t kFromDsUpToSeq = 4096;
 constexpr size_t kFromDsWorkspaceCap = (size_t)4 << 30;
 
-// variant: CT_ATTN_BWD_* values; workspace_bytes < 0: what the library asks for the form
+// variant: CT_ATTN_BWD_* values; workspace_bytes < 0: what the library asks for the form. A stored-dS form that
+// the caller did not pin (no form in `variant`, or form_is_free) gives way to the recomputing one, which needs
+// little scratch, where the device has no room for its blocks.
 std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, const Tensor& k, const Tensor& v,
                                                               const Tensor& segments, const MaybeTensor& ends,
                                                               const Tensor& bounds, const Tensor& out, const Tensor& lse,
                                                               const Tensor& dout, double scale, int variant,
-                                                              int64_t workspace_bytes, KeptWorkspace* kept) {
+                                                              int64_t workspace_bytes, KeptWorkspace* kept,
+                                                              bool form_is_free) {
   const c10::DeviceGuard guard(q.device());
   const AttnShape s = attn_shape(q, k);
+  const int form = variant & 0xf0;
+  const size_t least = ct_attn_bwd_workspace_bytes(s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim);
   size_t bytes;
   if (workspace_bytes >= 0) {
     bytes = (size_t)workspace_bytes;
   } else {
-    const int form = variant & 0xf0;
     const size_t stored = form == CT_ATTN_BWD_DQ_RECOMPUTE || (form == 0 && s.seq > kFromDsUpToSeq)
                               ? 0
                               : ct_attn_bwd_workspace_bytes_from_ds(s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim,
@@ -201,31 +205,39 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
         throw py::value_error("dq_form='from_ds' is not available for this shape (dS blocks of one KV head "
                               "exceed 64 GiB)");
       bytes = stored;
-    } else if (stored > 0 && stored <= kFromDsWorkspaceCap) {
-      bytes = stored;
     } else {
-      bytes = ct_attn_bwd_workspace_bytes(s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim);
+      bytes = stored > 0 && stored <= kFromDsWorkspaceCap ? stored : least;
     }
   }
   Tensor dq = fresh(q), dk = fresh(k), dv = fresh(v), delta = fresh(lse), workspace;
   // (A graph keeps the addresses it was captured with and runs its kernels out of order with later calls:
   // it gets scratch of its own, from its own pool, and builds its own lists.)
   if (kept && capturing()) kept = nullptr;
+  const auto take = [&](size_t size) {
+    if (!kept) return scratch(size, q);
+    if (!kept->buffer.defined() || (size_t)kept->buffer.numel() < size || kept->buffer.device() != q.device()) {
+      kept->listed.reset();
+      kept->buffer.reset();
+      kept->buffer = scratch(size, q);
+    }
+    return kept->buffer;
+  };
+  try {
+    workspace = take(bytes);
+  } catch (const c10::OutOfMemoryError&) {
+    if (workspace_bytes >= 0 || bytes <= least || (form != 0 && !form_is_free)) throw;
+    variant &= ~CT_ATTN_BWD_DQ_FROM_DS;
+    bytes = least;
+    workspace = take(bytes);
+  }
   if (kept) {
     const bool versioned = !bounds.is_inference();
     auto wanted = std::make_tuple(versioned ? bounds.unsafeGetTensorImpl()->version_counter().current_version() : 0u,
                                   std::vector<int64_t>{s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim}, variant, bytes,
                                   (float)scale);
-    if (!kept->buffer.defined() || (size_t)kept->buffer.numel() < bytes || kept->buffer.device() != q.device()) {
-      kept->buffer = scratch(bytes, q);
-      kept->listed.reset();
-    }
-    workspace = kept->buffer;
     if (versioned && kept->listed.is_same(bounds) && kept->listed_for == wanted) variant |= CT_ATTN_BWD_WORK_LIST_KEPT;
     kept->listed.reset();  // (until the call below has been made)
     kept->listed_for = std::move(wanted);
-  } else {
-    workspace = scratch(bytes, q);
   }
   ct_attn_bwd_args a = {};
   a.q = bits(q);
@@ -287,7 +299,7 @@ struct AttentionNode : OperatorNode {
     const Tensor Q = q.unpack(), K = k.unpack(), V = v.unpack(), O = out.unpack(self), L = lse.unpack();
     auto [dq, dk, dv, delta] =
         attention_backward(Q, K, V, segments, ends, bounds, O, L, gradient(grads[0], O.sizes(), at::kBFloat16, O), scale,
-                           operator_form(attn_shape(Q, K), ends && ends->defined()), -1, kept.get());
+                           operator_form(attn_shape(Q, K), ends && ends->defined()), -1, kept.get(), true);
     return {dq, dk, dv};
   }
   void release_variables() override {

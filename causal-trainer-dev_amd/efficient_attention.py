@@ -202,8 +202,8 @@ def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None,
 
     query ``[B, S, Hq, D]``, key / value ``[B, S, Hkv, D]``, all bf16 on a ROCm
     device; returns ``[B, S, Hq, D]`` bf16. Gradients flow to query, key, value.
-    Its backward takes dQ from stored dS blocks (up to 4 GiB of scratch) where that is the faster form: rows of up to
-    4096 positions, longer ones at head dimension 128 or with few query rows.
+    Its backward takes dQ from stored dS blocks (up to 4 GiB of scratch): rows of up to 4096 positions, longer ones at
+    head dimension 128 or with few query rows. Where the device has no room for the blocks it recomputes instead.
     ``backward_workspace`` (this build's addition, a :class:`BackwardWorkspace`) lets the layers of
     a model that share ``metadata`` share the scratch buffer of the backward and the work list in it.
     """
@@ -275,7 +275,7 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     dq, dk, dv, delta = _lib.native().attention_backward(
         query.detach(), key.detach(), value.detach(), metadata.query_segment_ids, metadata.attention_end,
         metadata.tile_bounds, out.detach(), lse, dout.contiguous(), resolved, _DKV_KERNELS[dkv_kernel] | _DQ_FORMS[dq_form],
-        -1 if workspace_bytes is None else int(workspace_bytes), _kept(workspace, metadata))
+        -1 if workspace_bytes is None else int(workspace_bytes), _kept(workspace, metadata), False)
     if with_delta:
         batch, sequence, q_heads, _ = query.shape
         return dq, dk, dv, delta.view(batch, q_heads, sequence)

@@ -356,6 +356,41 @@ def test_form_of_the_operators_backward(ct, gpu, shape, form):
         assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
 
 
+@pytest.mark.parametrize("seq,q_heads", [(8192, 8), (4096, 32)])
+def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
+    """The operator's own choice of the stored-dS form gives way to the recomputing form where the allocator has no room
+    for the blocks (here: a limit set on it), bit for bit; the form that a caller pinned raises."""
+
+    generator = torch.Generator(device=gpu).manual_seed(seq)
+    q, k, v, dout = (torch.randn((1, seq, heads, 128), generator=generator, device=gpu).to(torch.bfloat16)
+                     for heads in (q_heads, 8, 8, q_heads))
+    ids = torch.from_numpy(_layout(np.random.default_rng(seq), 1, seq, max_len=2000)).to(gpu)
+    metadata = ct.prepare_attention_metadata(ids, mesh=None, profile=ct.resolve_attention_profile(q.shape, k.shape, None))
+    out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+    expected = ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="recompute")
+    library = ct._lib.load()
+    room = 384 << 20
+    assert library.ct_attn_bwd_workspace_bytes(1, seq, q_heads, 8, 128) < room // 2
+    assert room < library.ct_attn_bwd_workspace_bytes_from_ds(1, seq, q_heads, 8, 128, 0)
+    inputs = tuple(t.requires_grad_(True) for t in (q, k, v))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+    try:
+        for kept in (None, ct.BackwardWorkspace()):
+            for _ in range(2):
+                got = torch.autograd.grad(ct.efficient_attention(*inputs, metadata, backward_workspace=kept), inputs, dout)
+                assert all(torch.equal(a, b) for a, b in zip(got, expected))
+        if seq <= 4096:       # (left open, the same choice is the library's)
+            got = ct.attention_backward(q, k, v, metadata, out, lse, dout)
+            assert all(torch.equal(a, b) for a, b in zip(got, expected))
+        with pytest.raises(torch.OutOfMemoryError):
+            ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="from_ds")
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 @pytest.mark.parametrize("shape", [
     # batch, seq, Hq, Hkv, D: both sides of each size at which the forward changes its form (row blocks of 32
     # queries per head over the launch: 512 and 7168 for D = 64, 2048 for D = 128; 1280 positions for D = 128)
