@@ -19,6 +19,7 @@
 
 #include <cmath>
 #include <exception>
+#include <mutex>
 #include <optional>
 #include <tuple>
 
@@ -137,6 +138,7 @@ inline bool needs_graph(std::initializer_list<Tensor> inputs) {
 // address goes to the next batch's metadata as soon as the last one's are dropped. Writes to it in place
 // show in its version counter (inference tensors have none: their list is built on every call).
 struct KeptWorkspace {
+  std::mutex mutex;  // held while a call chooses, launches and records
   Tensor buffer;
   Tensor listed;  // undefined: no list
   std::tuple<uint32_t, std::vector<int64_t>, int, size_t, float> listed_for;
@@ -213,6 +215,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
   // (A graph keeps the addresses it was captured with and runs its kernels out of order with later calls:
   // it gets scratch of its own, from its own pool, and builds its own lists.)
   if (kept && capturing()) kept = nullptr;
+  const std::unique_lock<std::mutex> lock = kept ? std::unique_lock<std::mutex>(kept->mutex) : std::unique_lock<std::mutex>();
   const auto take = [&](size_t size) {
     if (!kept) return scratch(size, q);
     if (!kept->buffer.defined() || (size_t)kept->buffer.numel() < size || kept->buffer.device() != q.device()) {
@@ -751,18 +754,20 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     }
   });
   py::class_<KeptWorkspace, std::shared_ptr<KeptWorkspace>>(m, "KeptWorkspace").def(py::init<>());
-  m.def("attention", &attention);
-  m.def("attention_forward", &attention_forward);
-  m.def("attention_backward", &attention_backward);
-  m.def("rms_norm", &rms_norm);
-  m.def("apply_rotary", &apply_rotary);
-  m.def("sparse_ce", &sparse_ce);
-  m.def("cut_ce", &cut_ce);
-  m.def("cutce_forward", &cutce_forward);
-  m.def("cutce_backward", &cutce_backward);
-  m.def("canonical_ids", &canonical_ids);
-  m.def("segment_positions", &segment_positions);
-  m.def("rotary_tables", &rotary_tables);
-  m.def("shifted_targets", &shifted_targets);
-  m.def("attention_metadata", &attention_metadata);
+  // The GIL is only needed to convert arguments and results: allocations and launches may block.
+  const auto def = [&m](const char* name, auto function) { m.def(name, function, py::call_guard<py::gil_scoped_release>()); };
+  def("attention", &attention);
+  def("attention_forward", &attention_forward);
+  def("attention_backward", &attention_backward);
+  def("rms_norm", &rms_norm);
+  def("apply_rotary", &apply_rotary);
+  def("sparse_ce", &sparse_ce);
+  def("cut_ce", &cut_ce);
+  def("cutce_forward", &cutce_forward);
+  def("cutce_backward", &cutce_backward);
+  def("canonical_ids", &canonical_ids);
+  def("segment_positions", &segment_positions);
+  def("rotary_tables", &rotary_tables);
+  def("shifted_targets", &shifted_targets);
+  def("attention_metadata", &attention_metadata);
 }

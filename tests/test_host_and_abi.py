@@ -2,6 +2,8 @@
 
 import ctypes
 import re
+import sys
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -98,6 +100,33 @@ def test_cutce_backward_refuses_strides_beyond_its_32_bit_offsets(ct):
             ((1 << 23) + 1, 50, 4096, ct._lib.CT_UNSUPPORTED), ((1 << 23) + 1, 50, None, ct._lib.CT_WORKSPACE_TOO_SMALL)):
         args.shape, args.dhead = ct._lib.CutceShape(rows, 128, vocab), dhead
         assert library.ct_cutce_bwd(None, ctypes.byref(args)) == status, (rows, vocab, dhead, library.ct_last_error())
+
+
+def test_native_operators_let_other_threads_run(ct):
+    """The native functions give the GIL up while they work: with Python's own switching as good as off, a waiting
+    thread still gets its turn (after a few dozen calls; a call that keeps the GIL never lets it in)."""
+
+    native, x = ct._lib.native(), torch.zeros(2, 128)
+    go, ran, interval = threading.Lock(), [], sys.getswitchinterval()
+    go.acquire()
+
+    def other():
+        go.acquire()
+        ran.append(True)
+
+    thread = threading.Thread(target=other)
+    thread.start()
+    sys.setswitchinterval(1000)
+    try:
+        go.release()
+        for _ in range(1_000_000):
+            if ran:
+                break
+            assert native.rms_norm(x, x, 1e-6) is None     # (not on a GPU: the wrapper's validation would say so)
+        assert ran
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
 
 
 def test_profile_resolution_matches_reference_tiers(ct):
