@@ -3,11 +3,13 @@
 Run ``python causal-trainer-dev_amd/build.py`` (or call :func:`build`) on any
 machine with hipcc; no GPU is needed to compile. The libraries are placed
 next to this file: libct_hotpath.so is what :mod:`_lib` loads through ctypes and what
-_native.so links, _native.so the extension module the torch operators call.
+_native.so links, _native.so the extension module the torch operators call. The first needs
+nothing but hipcc; the second also g++ and torch, and is left out where torch is not installed.
 """
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -50,7 +52,7 @@ def _run(cmd: list[str]) -> None:
 
 
 def build(verbose: bool = False, extra_flags: tuple[str, ...] = ()) -> Path:
-    """Compile every HIP source and link libct_hotpath.so. Always recompiles."""
+    """Compile every HIP source and link libct_hotpath.so, then _native.so. Always recompiles."""
 
     compiler = hipcc()
     build_dir = PACKAGE_DIR / "build"
@@ -66,15 +68,19 @@ def build(verbose: bool = False, extra_flags: tuple[str, ...] = ()) -> Path:
         _run(cmd)
 
     native_object = build_dir / "ct_torch.o"
+    with_torch = importlib.util.find_spec("torch") is not None
     with ThreadPoolExecutor(max_workers=4) as pool:
-        native = pool.submit(_compile_native, native_object, verbose)
+        native = pool.submit(_compile_native, native_object, verbose) if with_torch else None
         list(pool.map(compile_one, zip(sources, objects)))
-        native.result()
     link = [compiler, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-Wl,-soname,libct_hotpath.so",
             *map(str, objects), "-o", str(LIBRARY)]
     if verbose:
         print(" ".join(link), flush=True)
     _run(link)
+    if native is None:
+        print(f"torch is not installed: {NATIVE.name}, which the torch operators need, is not built", file=sys.stderr)
+        return LIBRARY
+    native.result()
     _link_native(native_object, verbose)
     return LIBRARY
 

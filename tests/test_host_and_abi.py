@@ -1,6 +1,7 @@
 """CPU-only checks of the host-side mirror and of the C ABI surface (no compute calls)."""
 
 import ctypes
+import importlib.util
 import re
 import sys
 import threading
@@ -100,6 +101,36 @@ def test_cutce_backward_refuses_strides_beyond_its_32_bit_offsets(ct):
             ((1 << 23) + 1, 50, 4096, ct._lib.CT_UNSUPPORTED), ((1 << 23) + 1, 50, None, ct._lib.CT_WORKSPACE_TOO_SMALL)):
         args.shape, args.dhead = ct._lib.CutceShape(rows, 128, vocab), dhead
         assert library.ct_cutce_bwd(None, ctypes.byref(args)) == status, (rows, vocab, dhead, library.ct_last_error())
+
+
+@pytest.mark.parametrize("torch_side", ["absent", "broken", "there"])
+def test_library_is_linked_whatever_becomes_of_the_torch_side(monkeypatch, tmp_path, torch_side):
+    """libct_hotpath.so needs hipcc only: it is linked without torch, and before a torch side that fails to compile
+    (which is still an error)."""
+
+    spec = importlib.util.spec_from_file_location("build_recipe", ROOT / "causal-trainer-dev_amd" / "build.py")
+    recipe = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(recipe)
+    made = []
+
+    def run(command):
+        output = Path(command[command.index("-o") + 1]).name
+        if torch_side == "broken" and output == "ct_torch.o":
+            raise RuntimeError("no g++")
+        made.append(output)
+
+    monkeypatch.setattr(recipe, "PACKAGE_DIR", tmp_path)
+    monkeypatch.setattr(recipe, "hipcc", lambda: "hipcc")
+    monkeypatch.setattr(recipe, "_run", run)
+    monkeypatch.setattr(recipe.importlib.util, "find_spec", lambda name: None if torch_side == "absent" else spec)
+    if torch_side == "broken":
+        with pytest.raises(RuntimeError, match="no g"):
+            recipe.build()
+    else:
+        assert recipe.build() == recipe.LIBRARY
+    objects = {Path(name).stem + ".o" for name in recipe.SOURCES} | ({"ct_torch.o"} if torch_side == "there" else set())
+    assert set(made[:len(objects)]) == objects
+    assert made[len(objects):] == ["libct_hotpath.so"] + (["_native.so"] if torch_side == "there" else [])
 
 
 def test_native_operators_let_other_threads_run(ct):
