@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .prep import _int32, _mask_and_labels
+from .prep import _dense, _int32, _mask_and_labels
 
 _STYLES = {"gpt-j": 0, "gpt-neox": 1}
 
@@ -27,7 +27,7 @@ def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     valid, labels = _mask_and_labels(mask, segment_ids)
     if valid.numel() == 0:
         return torch.empty_like(valid)
-    return _lib.native().segment_positions(valid, labels)
+    return _dense(_lib.native().segment_positions(valid, labels), "attention_mask and segment_ids")
 
 
 def rotary_cos_sin(position_ids, inv_freq, dtype=torch.bfloat16):
@@ -48,7 +48,7 @@ def rotary_cos_sin(position_ids, inv_freq, dtype=torch.bfloat16):
         shape = (batch, sequence, frequencies.shape[0])
         return (torch.empty(shape, dtype=torch.bfloat16, device=positions.device),
                 torch.empty(shape, dtype=torch.bfloat16, device=positions.device))
-    return _lib.native().rotary_tables(positions, frequencies)
+    return _dense(_lib.native().rotary_tables(positions, frequencies), "position_ids and inv_freq")
 
 
 def apply_rotary_cos_sin(query, key, cosine, sine, *, rope_style: str = "gpt-j", q_scale: float = 1.0):

@@ -31,6 +31,14 @@ def _nonzero(tensor, name: str) -> torch.Tensor:
     return _int32(tensor if tensor.dtype == torch.int32 else tensor != 0, name)
 
 
+def _dense(result, names: str):
+    """What the native side returned, an error if it did not take the arguments."""
+
+    if result is None:
+        raise RuntimeError(f"{names} must be dense tensors on one ROCm GPU, without forward-mode tangents")
+    return result
+
+
 def _mask_and_labels(mask, segment_ids):
     valid = _nonzero(mask, "attention_mask")
     if segment_ids is None:
@@ -50,7 +58,7 @@ def canonicalize_segment_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     valid, labels = _mask_and_labels(mask, segment_ids)
     if valid.numel() == 0:
         return torch.empty_like(valid)
-    return _lib.native().canonical_ids(valid, labels)
+    return _dense(_lib.native().canonical_ids(valid, labels), "attention_mask and segment_ids")
 
 
 def shifted_targets_and_weights(input_ids, attention_mask, segment_ids=None, assistant_mask=None,
@@ -84,7 +92,8 @@ def shifted_targets_and_weights(input_ids, attention_mask, segment_ids=None, ass
     if batch == 0:
         raise _lib.CtError(_lib.CT_INVALID_ARGUMENT, "ct_shifted_targets_and_weights: batch and sequence must be positive, "
                            f"got [{batch}, {sequence}]")
-    return _lib.native().shifted_targets(tokens, mask_t, segment_t, assistant_t, loss_t, label_t, int(ignore_index))
+    return _dense(_lib.native().shifted_targets(tokens, mask_t, segment_t, assistant_t, loss_t, label_t, int(ignore_index)),
+                  "input_ids and the masks")
 
 
 __all__ = ["canonicalize_segment_ids", "shifted_targets_and_weights"]

@@ -110,3 +110,23 @@ def test_prepared_targets_feed_the_loss_unchanged(ct, gpu):
     flat = weights.reshape(-1).cpu()
     assert float(weight_sum) == float(flat.sum())
     assert ((lse.cpu() == 0) == (flat == 0)).all()
+
+
+def test_arguments_that_the_native_side_does_not_take_are_named(ct, gpu):
+    """What passes the wrappers' checks and is still no dense tensor of the GPU raises with its name (and is never
+    handed to a kernel)."""
+
+    tokens = torch.arange(8, dtype=torch.int32, device=gpu).view(2, 4)
+    with pytest.raises(RuntimeError, match="input_ids and the masks must be dense"):
+        ct.shifted_targets_and_weights(tokens, None, loss_mask=torch.ones(2, 4))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(torch.ones(4, device=gpu), torch.ones(4, device=gpu))
+        with pytest.raises(RuntimeError, match="position_ids and inv_freq must be dense"):
+            ct.rotary_cos_sin(tokens, dual)
+    refusing = type("Native", (), {name: staticmethod(lambda *arguments: None)
+                                   for name in ("canonical_ids", "segment_positions")})
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(ct._lib, "native", lambda: refusing)
+        for function in (ct.canonicalize_segment_ids, ct.make_position_ids):
+            with pytest.raises(RuntimeError, match="attention_mask and segment_ids must be dense"):
+                function(tokens)
