@@ -153,19 +153,23 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, boo
 }
 
 // Number of the tiles in front of tile i when they are ordered by decreasing work, ties by index;
-// shared by `lanes` lanes (w 16-byte aligned).
+// shared by `lanes` lanes. Read in 16-byte quads from the first multiple of 16 bytes on: the arrays in LDS start
+// at one, those in the metadata buffer's scratch region (rows beyond 262144 positions, many tiles) anywhere.
 CT_DEVICE int rank_of(const int* w, int n, int i, int lanes) {
   const int wi = w[i], lane = threadIdx.x % lanes;
+  const int head = min(n, (int)(-(uintptr_t)w / sizeof(int) % 4)), quads = (n - head) / 4;
   int rank = 0;
   auto count = [&](int wv, int k) { rank += (wv > wi) || (wv == wi && k < i); };
-  for (int q = lane; q < n / 4; q += lanes) {
-    const int4 v = reinterpret_cast<const int4*>(w)[q];
-    count(v.x, 4 * q);
-    count(v.y, 4 * q + 1);
-    count(v.z, 4 * q + 2);
-    count(v.w, 4 * q + 3);
+  for (int k = lane; k < head; k += lanes) count(w[k], k);
+  for (int q = lane; q < quads; q += lanes) {
+    const int4 v = reinterpret_cast<const int4*>(w + head)[q];
+    const int k = head + 4 * q;
+    count(v.x, k);
+    count(v.y, k + 1);
+    count(v.z, k + 2);
+    count(v.w, k + 3);
   }
-  for (int k = n / 4 * 4 + lane; k < n; k += lanes) count(w[k], k);
+  for (int k = head + 4 * quads + lane; k < n; k += lanes) count(w[k], k);
   return sum_over(rank, lanes);
 }
 // Tiles between the first and the last that row blocks first .. end - 1 have to visit (`from`: kKvFirst or

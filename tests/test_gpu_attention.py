@@ -846,6 +846,44 @@ def test_million_token_sequence(ct, gpu):
                               ends[:, window] - window.start, dim ** -0.5)
 
 
+@pytest.mark.parametrize("batch,seq", [(2, 262144 + 384), (1, 262144 + 128), (40, 32768), (2, 640)])
+def test_schedules_are_the_stable_order_by_work(ct, gpu, batch, seq):
+    """All five schedules of every row and the order inside the bins, with working arrays in LDS (the last shape) and in
+    the scratch region, where rows of a length like these start them at any multiple of 4 bytes."""
+
+    rng = np.random.default_rng(seq)
+    ids = np.cumsum(rng.random((batch, seq)) < 0.002, axis=1).astype(np.int32) + 1
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None,
+                                             profile=ct.AttentionKernelProfile(1, 128, 128, 128))
+    blocks = seq // 32
+    flat = metadata.tile_bounds.cpu().numpy()
+    bounds = ct.tile_bounds_table(metadata).cpu().numpy()
+
+    def work(row, tile_blocks, column):
+        tiles = (blocks + tile_blocks - 1) // tile_blocks
+        first, last = np.full(tiles * tile_blocks, 2 ** 31 - 1), np.full(tiles * tile_blocks, -1)
+        first[:blocks], last[:blocks] = bounds[row, :, column], bounds[row, :, column + 1]
+        first, last = first.reshape(tiles, -1).min(1), last.reshape(tiles, -1).max(1)
+        return np.where(last >= first, last - first + 1, 0)
+
+    cursor = batch * blocks * 12
+    for row in range(batch):
+        for tile_blocks, column in ((1, 5), (2, 5), (4, 5), (4, 7), (8, 5)):
+            expected = np.argsort(-work(row, tile_blocks, column), kind="stable")
+            np.testing.assert_array_equal(flat[cursor:cursor + expected.size], expected)
+            cursor += expected.size
+        cursor = batch * blocks * 12 + (row + 1) * (2 * blocks + blocks // 4)
+    for tile_blocks in (2, 4, 8):
+        spans = np.concatenate([work(row, tile_blocks, 5) for row in range(batch)])
+        ranks = np.empty(spans.size, np.int64)
+        ranks[np.argsort(-spans, kind="stable")] = np.arange(spans.size)
+        offsets, items = flat[cursor:cursor + 33], flat[cursor + 33:cursor + 33 + spans.size]
+        np.testing.assert_array_equal(np.sort(items), np.arange(spans.size))
+        for start, stop in zip(offsets[:-1], offsets[1:]):
+            assert (np.diff(ranks[items[start:stop]]) > 0).all()
+        cursor += 33 + spans.size
+
+
 def _longest_segment(ids):
     """(batch row, start, stop) of the longest run of one nonzero id."""
 
