@@ -194,11 +194,6 @@ __host__ inline size_t ds_bytes_per_kv_head(int B, int S, int Hq, int Hkv, bool 
   return (size_t)(Hq / Hkv) * B * ds_row_blocks(S, has_end) * kDsBlockBytes;
 }
 
-// Longest row for which the backward takes the stored-dS form by itself when the caller's
-// workspace has room for it (measured 1-3 % faster than recomputing at 4096-token packed rows,
-// 15 % slower at 32768).
-constexpr int kFromDsUpToSeq = 4096;
-
 struct BwdPlan {
   DkvLayout L;
   bool spill;         // dS goes through the region, dQ from stored blocks

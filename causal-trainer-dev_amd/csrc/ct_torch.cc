@@ -176,9 +176,8 @@ std::tuple<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, c
 }
 
 // Left to itself (neither form nor size given) the backward offers the library the larger workspace of
-// the stored-dS form for rows of up to 4096 positions, if that is at most 4 GiB: the library then
-// takes that form, which is the faster one at such rows.
-constexpr int64_t kFromDsUpToSeq = 4096;
+// the stored-dS form for rows of up to CT_ATTN_FROM_DS_UP_TO_SEQ positions, if that is at most 4 GiB: the library
+// then takes that form.
 constexpr size_t kFromDsWorkspaceCap = (size_t)4 << 30;
 
 // variant: CT_ATTN_BWD_* values; workspace_bytes < 0: what the library asks for the form. A stored-dS form that
@@ -198,7 +197,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
   if (workspace_bytes >= 0) {
     bytes = (size_t)workspace_bytes;
   } else {
-    const size_t stored = form == CT_ATTN_BWD_DQ_RECOMPUTE || (form == 0 && s.seq > kFromDsUpToSeq)
+    const size_t stored = form == CT_ATTN_BWD_DQ_RECOMPUTE || (form == 0 && s.seq > CT_ATTN_FROM_DS_UP_TO_SEQ)
                               ? 0
                               : ct_attn_bwd_workspace_bytes_from_ds(s.batch, s.seq, s.q_heads, s.kv_heads, s.head_dim,
                                                                     ends && ends->defined());
@@ -270,19 +269,18 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
   return {dq, dk, dv, delta};
 }
 
-// The reference's residual (q, k, v, metadata, O, LSE) (src/causal_trainer/kernels/efficient_attention.py:1831-1863)
 // The form of the backward that the operator asks for. Left open, the library takes dQ from stored dS blocks at
-// rows of up to 4096 positions; longer ones ask for that form where it is the faster one and its workspace is at
-// most 4 GiB. It saves the two products that the recomputing dQ kernel repeats and pays 2 KB written and read
-// per block. Measured over rows of 4224 to 25600 positions with documents from 16 positions to the whole row,
-// recomputing / stored:
+// rows of up to 4096 positions (what that gains and loses: beside the flag in ct_hotpath.h); longer ones ask for
+// that form where it is the faster one and its workspace is at most 4 GiB. It saves the two products that the
+// recomputing dQ kernel repeats and pays 2 KB written and read per block. Measured over rows of 4224 to 25600
+// positions with documents from 16 positions to the whole row, recomputing / stored:
 //   head dimension 128: 0.98 to 1.39, below 1 only by noise, at every length whose blocks fit
 //     ([1, 7424, 6/1 heads] 297 / 254 us, [2, 8192, 8/8] 107 / 90, [1, 16384, 8/8] 174 / 144, [1, 25600, 4/4] 448 / 389).
 //   head dimension 64: a block's products are half as long and its traffic the same. Launches of few row blocks (32
 //     query rows of one head) gain, 0.99 to 1.18 up to 1400 of them ([1, 7424, 6/1] 189 / 167); with 2048 whole-row
 //     documents lose (0.84 at [1, 16384, 4/1]), with 4096 most long ones (0.75 to 0.91).
 int operator_form(const AttnShape& s, bool with_ends) {
-  if (s.seq <= 4096) return 0;
+  if (s.seq <= CT_ATTN_FROM_DS_UP_TO_SEQ) return 0;
   const bool pays = s.head_dim == 128 ? s.seq <= 32768
                                       : s.seq <= 8192 && (int64_t)s.batch * s.q_heads * (s.seq / 32) <= 1536;
   if (!pays) return 0;
@@ -290,6 +288,7 @@ int operator_form(const AttnShape& s, bool with_ends) {
   return bytes > 0 && bytes <= kFromDsWorkspaceCap ? CT_ATTN_BWD_DQ_FROM_DS : 0;
 }
 
+// The reference's residual (q, k, v, metadata, O, LSE) (src/causal_trainer/kernels/efficient_attention.py:1831-1863)
 struct AttentionNode : OperatorNode {
   SavedVariable q, k, v, out, lse;
   Tensor segments, bounds;

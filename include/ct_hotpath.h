@@ -148,12 +148,19 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * reference's _local_attention_dq, src/kernels/efficient_attention.py:985-1267); FROM_DS = the
  * dK/dV kernel (NARROW) stores its bf16 dS blocks in the workspace and dQ is the product of those
  * blocks with K: 14 D instead of 18 D executed flops per pair for 4 bytes of HBM traffic per
- * pair and head; measured 1-3 % faster than RECOMPUTE on packed 4096-token rows and 15 % slower
- * on 32768-token rows; needs ct_attn_bwd_workspace_bytes_from_ds. Left open (0): FROM_DS for
- * rows of at most 4096 positions if the caller's workspace holds the dS blocks of all KV heads
+ * pair and head; needs ct_attn_bwd_workspace_bytes_from_ds. Left open (0): FROM_DS for
+ * rows of at most CT_ATTN_FROM_DS_UP_TO_SEQ positions if the caller's workspace holds the dS blocks of all KV heads
  * (workspace_bytes >= ct_attn_bwd_workspace_bytes_from_ds and that size is the one-pass size),
  * else RECOMPUTE: a caller chooses by the workspace it offers. All give the same results within
- * the operator's tolerances (not bitwise: summation orders differ). */
+ * the operator's tolerances (not bitwise: summation orders differ).
+ * Measured, backward in us, RECOMPUTE / FROM_DS. Head dimension 128: [4, 4096, 32/8 heads] with documents of
+ * 64..4096 positions 703 / 670, whole rows 1831 / 1731; 0.96 to 1.18 times over rows of 1024 to 4096; [1, 32768, 64/8]
+ * 26405 / 26749 and whole rows 52877 / 61723 (eight passes), [1, 32768, 8/2] 3631 / 3082.
+ * Head dimension 64 at up to 4096 positions: 0.98 to 1.14 times for launches of up to 2048 row blocks (32 query rows
+ * of one head); beyond, ahead with short documents only ([4, 4096, 16/4], 8192 row blocks: documents of 16..128
+ * positions 105 / 92, of 64..4096 246 / 276, whole rows 550 / 715). The line looks at the row length alone: a caller
+ * with such launches offers the small workspace, or asks for RECOMPUTE. */
+#define CT_ATTN_FROM_DS_UP_TO_SEQ 4096
 #define CT_ATTN_BWD_DKV_NARROW 1
 #define CT_ATTN_BWD_DKV_WIDE 2
 #define CT_ATTN_BWD_DQ_RECOMPUTE 0x10
@@ -163,8 +170,9 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * (same tile_meta, shape, variant and workspace size) can keep the list. With this flag the call
  * does not build it: the head of `workspace` must be as the previous ct_attn_bwd call on this
  * workspace left it (every call leaves the list in place and the work counters of the dQ kernel at
- * zero). One launch and 0.01 ms less per call; anything else in the workspace may be overwritten
- * between the calls. */
+ * zero). Saves a launch and 0.01 ms per call of the recomputing form, and in the stored-dS form the list's share of
+ * the launch that also forms the row statistics (up to 7 us of small launches); anything else in the workspace
+ * may be overwritten between the calls. */
 #define CT_ATTN_BWD_WORK_LIST_KEPT 0x100
 
 typedef struct ct_attn_bwd_args {
