@@ -578,6 +578,9 @@ extern "C" int32_t ct_rms_norm_fwd(void* stream, const uint16_t* x, const uint16
   const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
   hipStream_t st = (hipStream_t)stream;
   const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, x, scale, eps, (long)rows, hidden, y, rstd); };
+  // Rows in registers up to 4096 channels and around the two larger sizes that models have, 5120 and 8192 (an instance
+  // per 512 channels); rows of 4104 to 4608, 5128 to 7680 and more than 8192 are walked twice, the second
+  // time from cache.
   switch (int chunks = (hidden + 511) / 512; chunks) {
     case 1: launch(rms_norm_fwd_rows_kernel<1>); break;
     case 2: launch(rms_norm_fwd_rows_kernel<2>); break;
