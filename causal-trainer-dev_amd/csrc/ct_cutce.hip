@@ -335,64 +335,66 @@ struct TileRows {
   CT_DEVICE void advance(int r) { row += (long)stride * ((r & 3) == 3 ? 5 : 1); }
 };
 
-template <bool CACHE, bool GUARDED>
-__global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
-                                                          int tiles_per_chunk, float* cache) {
+template <int NB, bool CACHE, bool GUARDED>
+__global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
+                                                                    int tiles_per_chunk, float* cache) {
+  constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
-  const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
-  const int vocab_tiles = (p.V + kGemmTile - 1) / kGemmTile;
+  const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
+  const int vocab_tiles = (p.V + kTile - 1) / kTile;
   const int n_act = p.header->n_act;
 
   // units: (vocabulary chunk, row block)
-  const int active_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+  const int active_blocks = (n_act + kTile - 1) / kTile;
   UnitQueue units;
   units.init(p.header->xcd_counter[0], chunks, active_blocks, UnitQueue::kSweep);
   int chunk, rb;
   while (units.next(chunk, rb, &unit_s)) {
     chunk += chunk0;
-    const int n0 = rb * kGemmTile;
-    if (!p.block_active[rb]) continue;  // no row of this block carries weight
+    const int n0 = rb * kTile;
+    if (!p.block_active[n0 / kGemmTile]) continue;  // no row of this block carries weight
 
     // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
-    // n0 + wn + 4 j + nb, so a lane owns 4 consecutive slots.
-    const i32x4 tgt = *reinterpret_cast<const i32x4*>(p.slot_target + n0 + wn + 4 * j);
-    float m2[4], sum[4], tl[4];
+    // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
+    typedef int LaneInts __attribute__((ext_vector_type(NB)));
+    const LaneInts tgt = *reinterpret_cast<const LaneInts*>(p.slot_target + n0 + wn + NB * j);
+    float m2[NB], sum[NB], tl[NB];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
       m2[nb] = kNegInfF;
       sum[nb] = 0.f;
       tl[nb] = 0.f;
     }
-    KcLoader B;
+    KcLoader<NB> B;
     B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
 
     const int vt_end = min((chunk + 1) * tiles_per_chunk, vocab_tiles);
     for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
-      const int v0 = vt * kGemmTile;
-      McLoader A;
+      const int v0 = vt * kTile;
+      McLoader<NB> A;
       A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
-      GemmAcc acc;
+      GemmAcc<NB> acc;
       acc.clear();
       gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
       if (vt + 1 == vt_end) units.request();
 
       const int vbase = v0 + wm + 4 * half;  // vocab id of (i, r) = vbase + 32 i + 8 (r/4) + r%4
-      const bool ragged = v0 + kGemmTile > p.V;
+      const bool ragged = v0 + kTile > p.V;
       if constexpr (CACHE) {
-        // cache^T[v][slot]: a lane stores its 4 consecutive slots with one 16-byte access, 32
-        // lanes = 512 contiguous bytes. Address = wave-uniform tile origin + uniform row offset +
+        // cache^T[v][slot]: a lane stores its NB consecutive slots with one access, 32
+        // lanes = NB * 128 contiguous bytes. Address = wave-uniform tile origin + uniform row offset +
         // a 32-bit lane offset, so the stores need no per-store vector address arithmetic.
         float* origin = cache + (size_t)(v0 + uniform(wm)) * p.n_pad + n0 + uniform(wn);
-        const unsigned lane_off = (unsigned)(4 * half * p.n_pad + 4 * j) * 4u;  // bytes
+        const unsigned lane_off = (unsigned)(4 * half * p.n_pad + NB * j) * 4u;  // bytes
         TileRows rows(origin, p.n_pad * 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            store_global16_s<0>(rows.row, lane_off, acc.quad(i, r));
+            store_lane(rows.row, lane_off, acc.lane(i, r));
             rows.advance(r);
           }
       }
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
           int limit = p.V - vbase;
           if (ragged_tile.value) asm volatile("" : "+v"(limit));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
+          for (int i = 0; i < NB; ++i) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
               const int row = 32 * i + acc_row(r, 0);
@@ -415,11 +417,11 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
           }
         };
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
           float tmax = kNegInfF;
           each(nb, tmax, [&](int, float x) { tmax = fmaxf(tmax, x); });
           const int rel = tgt[nb] - (v0 + wm);
-          if (__any(rel >= 0 && rel < 128))
+          if (__any(rel >= 0 && rel < kWave))
             each(nb, tl[nb], [&](int row, float x) { tl[nb] += vbase + row == tgt[nb] ? x : 0.f; });
           const float m_new = fmaxf(m2[nb], tmax * kLog2e);
           const float m_use = (m_new == kNegInfF) ? 0.f : m_new;
@@ -435,15 +437,15 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
 
     // lanes l and l^32 hold the same rows; then the two wavefronts with equal wn.
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
       merge_stats(m2[nb], sum[nb], xor32(m2[nb]), xor32(sum[nb]));
       tl[nb] += xor32(tl[nb]);
     }
-    float* exch = reinterpret_cast<float*>(smem_raw);  // [2 wn][128 rows][3]
+    float* exch = reinterpret_cast<float*>(smem_raw);  // [2 wn][kWave rows][3]
     if (wm != 0 && half == 0) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        float* e = exch + ((w & 1) * 128 + 32 * nb + j) * 3;
+      for (int nb = 0; nb < NB; ++nb) {
+        float* e = exch + ((w & 1) * kWave + 32 * nb + j) * 3;
         e[0] = m2[nb];
         e[1] = sum[nb];
         e[2] = tl[nb];
@@ -452,11 +454,11 @@ __global__ __launch_bounds__(256) void cutce_stats_kernel(CutceParams p, float* 
     __syncthreads();
     if (wm == 0 && half == 0) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const float* e = exch + ((w & 1) * 128 + 32 * nb + j) * 3;
+      for (int nb = 0; nb < NB; ++nb) {
+        const float* e = exch + ((w & 1) * kWave + 32 * nb + j) * 3;
         merge_stats(m2[nb], sum[nb], e[0], e[1]);
         tl[nb] += e[2];
-        float* out = part + ((size_t)chunk * p.n_pad + n0 + wn + 4 * j + nb) * 3;
+        float* out = part + ((size_t)chunk * p.n_pad + n0 + wn + NB * j + nb) * 3;
         out[0] = m2[nb];
         out[1] = sum[nb];
         out[2] = tl[nb];
@@ -596,77 +598,78 @@ CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
 // G^T[v - slab0][slot], logits recomputed (transposed tile as in the statistics kernel: rows =
 // vocabulary, lanes = row slots). Persistent like the statistics kernel and with its unit order:
 // a unit is tiles_per_chunk vocabulary tiles of the slab times one block of 256 active rows.
-template <bool GUARDED>
-__global__ __launch_bounds__(256) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
-                                                            int slab0, int slab_tiles, int tiles_per_chunk,
-                                                            bf16* G) {
+template <int NB, bool GUARDED>
+__global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
+                                                                      int slab0, int slab_tiles, int tiles_per_chunk,
+                                                                      bf16* G) {
+  constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
+  typedef float LaneFloats __attribute__((ext_vector_type(NB)));
+  typedef int LaneInts __attribute__((ext_vector_type(NB)));
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
-  const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
+  const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
   const int n_act = p.header->n_act;
   // the two GEMM kernels that follow start from fresh work counters
   if (blockIdx.x == 0) reset_unit_counters(p.header);
-  const int active_blocks = (n_act + kGemmTile - 1) / kGemmTile;  // G^T columns past them are never read
+  const int active_blocks = (n_act + kTile - 1) / kTile;  // G^T columns past them are never used
   const int chunks = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk;
   UnitQueue units;
   units.init(p.header->xcd_counter[2], chunks, active_blocks, UnitQueue::kSweep);
   int chunk, rb;
   while (units.next(chunk, rb, &unit_s)) {
-    const int n0 = rb * kGemmTile;
+    const int n0 = rb * kTile;
     // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
-    // n0 + wn + 4 j + nb, so a lane owns 4 consecutive slots of G^T and stores them together.
-    const int slot4 = n0 + wn + 4 * j;
-    const f32x4 fac = *reinterpret_cast<const f32x4*>(rp.fac + slot4);
-    const f32x4 lse2 = *reinterpret_cast<const f32x4*>(rp.lse2 + slot4);
-    const i32x4 tgt = *reinterpret_cast<const i32x4*>(rp.tgt + slot4);
-    KcLoader B;
+    // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
+    const int slot = n0 + wn + NB * j;
+    const LaneFloats fac = *reinterpret_cast<const LaneFloats*>(rp.fac + slot);
+    const LaneFloats lse2 = *reinterpret_cast<const LaneFloats*>(rp.lse2 + slot);
+    const LaneInts tgt = *reinterpret_cast<const LaneInts*>(rp.tgt + slot);
+    KcLoader<NB> B;
     B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
     const int vt_end = min((chunk + 1) * tiles_per_chunk, slab_tiles);
     for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
-      const int v0 = slab0 + vt * kGemmTile;
-      McLoader A;
+      const int v0 = slab0 + vt * kTile;
+      McLoader<NB> A;
       A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
-      GemmAcc acc;
+      GemmAcc<NB> acc;
       acc.clear();
       gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
       if (vt + 1 == vt_end) units.request();
 
       bf16* origin = G + (size_t)(v0 - slab0 + uniform(wm)) * p.n_pad + n0 + uniform(wn);
-      const unsigned lane_off = (unsigned)(4 * half * p.n_pad + 4 * j) * 2u;  // bytes
+      const unsigned lane_off = (unsigned)(4 * half * p.n_pad + NB * j) * 2u;  // bytes
       // Most tiles hold no target of the wavefront's rows and lie inside the vocabulary: there the
       // gradient is factor * softmax, three instructions per element. (Slots without weight have
       // factor 0 and lse = +inf.)
       bool target_here = false;
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) target_here |= (unsigned)(tgt[nb] - (v0 + wm)) < 128u;
-      const bool plain = v0 + kGemmTile <= p.V && !__any(target_here);
+      for (int nb = 0; nb < NB; ++nb) target_here |= (unsigned)(tgt[nb] - (v0 + wm)) < (unsigned)kWave;
+      const bool plain = v0 + kTile <= p.V && !__any(target_here);
       TileRows rows(origin, p.n_pad * 2);
       if (plain) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const f32x4 x = acc.quad(i, r);
-            bf16x4 quad;
+            LaneFloats x = acc.lane(i, r);
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) quad[nb] = (bf16)(fac[nb] * exp2_fast(x[nb] * kLog2e - lse2[nb]));
-            store_global8_s<0>(rows.row, lane_off, quad);
+            for (int nb = 0; nb < NB; ++nb) x[nb] = fac[nb] * exp2_fast(x[nb] * kLog2e - lse2[nb]);
+            store_lane(rows.row, lane_off, to_bf16(x));
             rows.advance(r);
           }
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int v = v0 + wm + 32 * i + acc_row(r, half);
-            const f32x4 x = acc.quad(i, r);
-            bf16x4 quad;
+            LaneFloats x = acc.lane(i, r);
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-              quad[nb] = (bf16)((fac[nb] != 0.f && v < p.V) ? dlogit(x[nb], fac[nb], lse2[nb], tgt[nb], v) : 0.f);
-            store_global8_s<0>(rows.row, lane_off, quad);
+            for (int nb = 0; nb < NB; ++nb)
+              x[nb] = (fac[nb] != 0.f && v < p.V) ? dlogit(x[nb], fac[nb], lse2[nb], tgt[nb], v) : 0.f;
+            store_lane(rows.row, lane_off, to_bf16(x));
             rows.advance(r);
           }
       }
@@ -726,40 +729,44 @@ __global__ __launch_bounds__(256) void cutce_dlogits_cached_kernel(CutceParams p
 // parts is chosen on the device, where the number of active rows is known; the host only
 // provides room for them.
 struct CutceSplits {
-  float* hidden_sums;    // [parts][active row blocks * 256][d]
+  float* hidden_sums;    // [parts][active row blocks * tile][d]
   float* head_sums;      // [parts][d][slab_width]
   size_t hidden_room;    // floats in hidden_sums
   int head_most;         // parts that head_sums has room for
-  int all_tiles;         // of the whole vocabulary
+  int tile;              // 256 or 128: the output tile's sides
+  int vocab;             // columns of the whole vocabulary, padded to 256
   bool with_head;
 };
 
-// Lengths in units of 128 terms of one tile (about 2 us): a compute unit's fair share of all of the
-// work is total / 256, and tiles much longer than that are cut down to it. Partial sums cost 512 KB of
-// traffic per part and tile (about 0.1 us of the device's bandwidth), so with little work the parts
-// stay longer: at length t the last tile ends after 2 t us and the sums of total / t parts take
-// 0.1 total / t us, least at t = sqrt(0.05 total).
-__host__ __device__ inline float part_length(int row_blocks, int d, int tiles, bool with_head) {
-  const float col_blocks = (float)((d + kGemmTile - 1) / kGemmTile);
-  const float total = (with_head ? 4.f : 2.f) * (float)row_blocks * col_blocks * (float)tiles;
-  const float share = total / kComputeUnits, least = __builtin_sqrtf(0.05f * total);
+// Lengths in units of 128 terms of one tile: a workgroup's fair share of all of the work is total / slots, and
+// tiles much longer than that are cut down to it. Partial sums cost 8 bytes of traffic per part and
+// element, so with little work the parts stay longer: at length t the last tile ends after t units and the
+// sums take total / t parts, least where t is the square root of total times the price of a part in units
+// (256 x 256: 0.1 us of the device's bandwidth against 2 us a unit; 128 x 128: 0.026 against 1).
+__host__ __device__ inline float part_length(int tile, int row_blocks, int d, int vocab, bool with_head) {
+  const float col_blocks = (float)((d + tile - 1) / tile);
+  const float groups = (float)row_blocks * col_blocks * (float)(vocab / 128);
+  const float total = (with_head ? 2.f : 1.f) * groups;
+  const float share = total / (float)(tile == kGemmTile ? kComputeUnits : 2 * kComputeUnits);
+  const float least = __builtin_sqrtf((tile == kGemmTile ? 0.05f : 0.026f) * total);
   return share > least ? share : least;
 }
 __host__ __device__ inline int whole_parts(float parts) { return parts < 1.5f ? 1 : parts > 64.f ? 64 : (int)(parts + 0.5f); }
 
-CT_DEVICE int hidden_parts(const CutceSplits& sp, int n_act, int d, int slab_tiles) {
-  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+CT_DEVICE int hidden_parts(const CutceSplits& sp, int tile, int n_act, int d, int slab_width) {
+  const int row_blocks = (n_act + tile - 1) / tile;
   if (row_blocks == 0) return 1;
-  const int parts = whole_parts(2.f * slab_tiles / part_length(row_blocks, d, slab_tiles, sp.with_head));
-  const size_t fit = sp.hidden_room / ((size_t)row_blocks * kGemmTile * d);
+  const int parts = whole_parts((float)(slab_width / 128) / part_length(tile, row_blocks, d, slab_width, sp.with_head));
+  const size_t fit = sp.hidden_room / ((size_t)row_blocks * tile * d);
   return uniform(fit < (size_t)parts ? (fit > 1 ? (int)fit : 1) : parts);
 }
 // A slab's dHead is cut as the whole vocabulary's is, whatever the slab: dHead is bit for bit the same
 // for every workspace. (dHidden adds over slabs anyway.)
-CT_DEVICE int head_parts(const CutceSplits& sp, int n_act, int d) {
-  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
+CT_DEVICE int head_parts(const CutceSplits& sp, int tile, int n_act, int d) {
+  const int row_blocks = (n_act + tile - 1) / tile;
   if (row_blocks == 0) return 1;
-  return uniform(min(whole_parts(2.f * row_blocks / part_length(row_blocks, d, sp.all_tiles, true)), sp.head_most));
+  const float groups = (float)(row_blocks * (tile / 128));
+  return uniform(min(whole_parts(groups / part_length(tile, row_blocks, d, sp.vocab, true)), sp.head_most));
 }
 
 // First of the 128-term groups of part `split`.
@@ -779,34 +786,35 @@ struct CutceSlab {
 
 // dHidden[idx[slot], n] (+)= sum_v G^T[v, slot] head[n, first + v] of row block rb, column block cb and
 // part `split` of the contraction.
-template <bool GUARDED>
+template <int NB, bool GUARDED>
 CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int rb, int cb, int split,
                             int parts, int n_act, UnitQueue& units, const lds_addr smem) {
+  constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
-  const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
+  const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
   // Terms of the contraction: the whole slab where the head is padded, else up to the end of the
   // vocabulary; the last k_width % 128 of them from the tail, since nothing past a row's end may be
   // read (G^T is zero from the vocabulary's end to the end of the slab).
   const int k_width = p.head.padded ? sl.width : min(sl.width, p.V - sl.first);
   const int groups = k_width / 128;
-  const int n0 = rb * kGemmTile, c0 = cb * kGemmTile;
+  const int n0 = rb * kTile, c0 = cb * kTile;
   const int k_begin = split_begin(groups, split, parts) * 128, k_mid = split_begin(groups, split + 1, parts) * 128;
   const bool with_tail = split == parts - 1 && k_mid < k_width;
-  McLoader A;
+  McLoader<NB> A;
   A.init(sl.G, p.n_pad, n0, p.n_pad, sl.width);
-  GemmAcc acc;
+  GemmAcc<NB> acc;
   acc.clear();
-  // (rows of B interleaved: lane j owns the 4 consecutive columns c0 + wn + 4 j + nb; rows past d
+  // (rows of B interleaved: lane j owns the NB consecutive columns c0 + wn + NB j + nb; rows past d
   // are copies of the first, their columns are not stored)
   const bf16* head = p.head.base + (sl.first - p.head.col0);
   if constexpr (GUARDED) {
-    KcLoader B;
+    KcLoader<NB> B;
     B.init(head, p.head.ld, nullptr, c0, p.d, k_width, true);
     gemm_tile<true>(A, B, k_begin, with_tail ? k_width : k_mid, smem, acc);
   } else {
 #pragma nounroll
     for (int part = 0; part <= (int)with_tail; ++part) {
-      KcLoader B;
+      KcLoader<NB> B;
       B.init(part ? p.head.tail - k_mid : head, part ? 128 : p.head.ld, nullptr, c0, p.d, k_width, true);
       gemm_tile<false>(A, B, part ? k_mid : k_begin, part ? k_mid + 128 : k_mid, smem, acc);
     }
@@ -818,57 +826,52 @@ CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const Cut
   // offset: formed per element they spill, and a reload waits for every store in front of it (all GEMM
   // epilogues in this form, forward and backward at N = 999, d = 1024, V = 32003: 447 -> 356 us; at N = 16384,
   // d = 4096, V = 128256 part of the 1.6 % that the pass gained in all). Both f32 buffers have rows to the end of the block.
+  typedef typename GemmAcc<NB>::Lane LaneFloats;
+  typedef decltype(to_bf16(LaneFloats{})) LaneBf16;
   const int row0 = n0 + uniform(wm), col0 = c0 + uniform(wn);
   if (col0 >= p.d) return;  // hidden sizes are multiples of 128: all of the wavefront's columns or none
   if (parts > 1 || sl.mode != 0) {
-    float* origin = (parts > 1 ? sp.hidden_sums + (size_t)split * ((n_act + kGemmTile - 1) / kGemmTile * kGemmTile) * p.d
+    float* origin = (parts > 1 ? sp.hidden_sums + (size_t)split * ((n_act + kTile - 1) / kTile * kTile) * p.d
                                : sl.dh_acc) + (size_t)row0 * p.d + col0;
-    const unsigned lane_off = (unsigned)(4 * half * p.d + 4 * j) * 4u;  // bytes
+    const unsigned lane_off = (unsigned)(4 * half * p.d + NB * j) * 4u;  // bytes
     TileRows rows(origin, p.d * 4);
     if (parts > 1 || sl.mode == 1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const f32x4 val = acc.quad(i, r);
-          store_global16_s<0>(rows.row, lane_off, val);
+          store_lane(rows.row, lane_off, acc.lane(i, r));
           rows.advance(r);
         }
       return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        *reinterpret_cast<f32x4*>(rows.row + lane_off) += acc.quad(i, r);
+        *reinterpret_cast<LaneFloats*>(rows.row + lane_off) += acc.lane(i, r);
         rows.advance(r);
       }
     if (sl.mode == 2) return;
-    for (int r = 0; r < 64; ++r) {
+    for (int r = 0; r < 16 * NB; ++r) {
       const int slot = row0 + 32 * (r >> 4) + acc_row(r & 15, half);
       if (slot >= n_act) continue;
-      const f32x4 val = *reinterpret_cast<const f32x4*>(sl.dh_acc + (size_t)slot * p.d + col0 + 4 * j);
-      bf16x4 out;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-      *reinterpret_cast<bf16x4*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col0 + 4 * j) = out;
+      const LaneFloats val = *reinterpret_cast<const LaneFloats*>(sl.dh_acc + (size_t)slot * p.d + col0 + NB * j);
+      *reinterpret_cast<LaneBf16*>(sl.dhidden + (size_t)p.idx[slot] * p.d + col0 + NB * j) = to_bf16(val);
     }
     return;
   }
-  bf16* columns = sl.dhidden + col0 + 4 * j;
+  bf16* columns = sl.dhidden + col0 + NB * j;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int slot = row0 + 32 * i + 8 * q + 4 * half;
       const i32x4 to = *reinterpret_cast<const i32x4*>(p.idx + slot);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const f32x4 val = acc.quad(i, 4 * q + e);
-        bf16x4 out;
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-        if (slot + e < n_act) *reinterpret_cast<bf16x4*>(columns + (size_t)to[e] * p.d) = out;
+        const LaneBf16 out = to_bf16(acc.lane(i, 4 * q + e));
+        if (slot + e < n_act) *reinterpret_cast<LaneBf16*>(columns + (size_t)to[e] * p.d) = out;
       }
     }
 }
@@ -890,22 +893,23 @@ CT_DEVICE void store_dhead4(bf16* dst, int left, f32x4 val) {
 
 // dHead[m, first + v] = sum_slot packed[slot, m] G^T[v, slot], packed[slot] = hidden[idx[slot]], of
 // vocabulary tile vt, hidden column block mb and part `split` of the contraction.
-template <bool GUARDED>
+template <int NB, bool GUARDED>
 CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int vt, int mb, int split,
                           int parts, int n_act, UnitQueue& units, const lds_addr smem) {
+  constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
-  const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
+  const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
   // 4 contraction steps at a time; slots n_act .. k_end-1 are valid memory: G^T holds zeros
-  // there (the dlogits kernels write whole 256-slot blocks) and the packed rows are finite.
+  // there (the dlogits kernels write whole blocks of at least 128 slots) and the packed rows are finite.
   const int groups = min(p.n_pad, (n_act + 4 * kBK - 1) / (4 * kBK) * (4 * kBK)) / (4 * kBK);
-  const int m0 = mb * kGemmTile, v0 = vt * kGemmTile;  // v0 relative to the slab
+  const int m0 = mb * kTile, v0 = vt * kTile;  // v0 relative to the slab
   const int k_begin = split_begin(groups, split, parts) * 128, k_end = split_begin(groups, split + 1, parts) * 128;
-  McLoader A;  // (columns past d are copies, their rows of dHead are not stored)
+  McLoader<NB> A;  // (columns past d are copies, their rows of dHead are not stored)
   A.init(sl.packed, p.d, m0, p.d, k_end);
-  // (rows of B interleaved: lane j owns the 4 consecutive vocabulary ids v .. v + 3)
-  KcLoader B;
+  // (rows of B interleaved: lane j owns NB consecutive vocabulary ids)
+  KcLoader<NB> B;
   B.init(sl.G, p.n_pad, nullptr, v0, sl.width, k_end, true);
-  GemmAcc acc;
+  GemmAcc<NB> acc;
   acc.clear();
   gemm_tile<GUARDED>(A, B, k_begin, k_end, smem, acc);
   units.request();
@@ -914,42 +918,37 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
   if (row0 >= p.d) return;  // hidden sizes are multiples of 128: all of the wavefront's rows or none
   if (parts > 1) {
     float* origin = sp.head_sums + ((size_t)split * p.d + row0) * sl.width + col0;
-    const unsigned lane_off = (unsigned)(4 * half * sl.width + 4 * j) * 4u;  // bytes
+    const unsigned lane_off = (unsigned)(4 * half * sl.width + NB * j) * 4u;  // bytes
     TileRows rows(origin, sl.width * 4);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const f32x4 val = acc.quad(i, r);
-        store_global16_s<0>(rows.row, lane_off, val);
+        store_lane(rows.row, lane_off, acc.lane(i, r));
         rows.advance(r);
       }
     return;
   }
   // The rows of an odd vocabulary start at any multiple of 2 bytes, which an ordinary store may.
-  const int left = p.V - (sl.first + col0 + 4 * j);
+  const int left = p.V - (sl.first + col0 + NB * j);
   bf16* origin = sl.dhead + (size_t)row0 * p.V + sl.first + col0;
-  const unsigned lane_off = (unsigned)(4 * half * p.V + 4 * j) * 2u;  // bytes
-  if (left >= 4) {
+  const unsigned lane_off = (unsigned)(4 * half * p.V + NB * j) * 2u;  // bytes
+  if (left >= NB) {
     TileRows rows(origin, p.V * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const f32x4 val = acc.quad(i, r);
-        bf16x4 out;
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) out[nb] = (bf16)val[nb];
-        store_global8_s<0>(rows.row, lane_off, out);
+        store_lane(rows.row, lane_off, to_bf16(acc.lane(i, r)));
         rows.advance(r);
       }
   } else {
 #pragma unroll
-    for (int nb = 0; nb < 3; ++nb)
+    for (int nb = 0; nb < NB - 1; ++nb)
       if (nb < left) {
         TileRows rows(origin, p.V * 2);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             reinterpret_cast<bf16*>(rows.row + lane_off)[nb] = (bf16)acc.value(i, nb, r);
@@ -964,18 +963,19 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
 // device idle); a workgroup that finds no hidden-gradient unit left goes on to the head-gradient
 // units, which are many and short, and the idle tail of the first fills with work of the second. The
 // two read the same G^T and write different tensors: neither waits for the other.
-template <bool HEAD, bool GUARDED>
-__global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
+template <int NB, bool HEAD, bool GUARDED>
+__global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
+  constexpr int kTile = GemmShape<NB>::kTile;
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
   const int n_act = p.header->n_act;
   // the dlogits kernel of the next vocabulary slab starts from fresh work counters
   if (blockIdx.x == 0) reset_dlogits_counters(p.header);
-  const int col_blocks = (p.d + kGemmTile - 1) / kGemmTile, slab_tiles = sl.width / kGemmTile;
-  const int row_blocks = (n_act + kGemmTile - 1) / kGemmTile;
-  const int parts_h = hidden_parts(sp, n_act, p.d, slab_tiles);
-  const int parts_w = HEAD ? head_parts(sp, n_act, p.d) : 1;
+  const int col_blocks = (p.d + kTile - 1) / kTile, slab_tiles = sl.width / kTile;
+  const int row_blocks = (n_act + kTile - 1) / kTile;
+  const int parts_h = hidden_parts(sp, kTile, n_act, p.d, sl.width);
+  const int parts_w = HEAD ? head_parts(sp, kTile, n_act, p.d) : 1;
   const int total_h = row_blocks * col_blocks * parts_h, total_w = HEAD ? slab_tiles * col_blocks * parts_w : 0;
   // Short problems walk one list, the longer units first; large ones the hidden gradient's grid (row
   // block, (part, column block)) and then the head gradient's (vocabulary tile, (part, column block)).
@@ -999,9 +999,9 @@ __global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, CutceSl
       b = index % width;
     }
     if (!in_head) {
-      dhidden_unit<GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
+      dhidden_unit<NB, GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
     } else if constexpr (HEAD) {
-      dhead_unit<GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_w, n_act, units, smem);
+      dhead_unit<NB, GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_w, n_act, units, smem);
     }
   }
 }
@@ -1011,10 +1011,10 @@ __global__ __launch_bounds__(256) void cutce_grads_kernel(CutceParams p, CutceSl
 __global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
   const int n_act = p.header->n_act;
   const long first = (long)blockIdx.x * 256 + threadIdx.x, stride = (long)gridDim.x * 256;
-  const int parts_h = hidden_parts(sp, n_act, p.d, sl.width / kGemmTile);
+  const int parts_h = hidden_parts(sp, sp.tile, n_act, p.d, sl.width);
   if (parts_h > 1) {
     const int quads = p.d / 4;
-    const size_t part_size = (size_t)((n_act + kGemmTile - 1) / kGemmTile) * kGemmTile * p.d;
+    const size_t part_size = (size_t)((n_act + sp.tile - 1) / sp.tile) * sp.tile * p.d;
     for (long index = first; index < (long)n_act * quads; index += stride) {
       const int slot = (int)(index / quads), col = (int)(index % quads) * 4;
       const float* src = sp.hidden_sums + (size_t)slot * p.d + col;
@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, CutceS
     }
   }
   if (!sp.with_head) return;
-  const int parts_w = head_parts(sp, n_act, p.d);
+  const int parts_w = head_parts(sp, sp.tile, n_act, p.d);
   if (parts_w <= 1) return;
   const int width = min(sl.width, (p.V - sl.first + 3) & ~3);
   const int quads = width / 4;
@@ -1063,10 +1063,40 @@ static int tiles_per_chunk(int tiles, int row_blocks) {
   const long units = (long)tiles * row_blocks;
   return units <= kPlainRounds * kComputeUnits ? 1 : units <= 2 * kPlainRounds * kComputeUnits ? 2 : 4;
 }
-static int stats_chunks(const ct_cutce_shape& s) {
-  const int tiles = vocab_tile_count(s.vocab);
-  const int t = tiles_per_chunk(tiles, padded_rows(s.rows) / kGemmTile);
-  return (tiles + t - 1) / t;
+
+// The output tile of the GEMM kernels, 256 or 128. The large one does twice the work per byte that reaches LDS
+// (a compute unit's 64 bytes a clock keep up with no more than the small tile's MFMAs); the small one gives
+// short problems four times the workgroups, a quarter of the epilogue per wavefront and, up to one tile per
+// compute unit, half the time per step. Measured (us, large / small; statistics kernel and dlogits kernel):
+// 32 to 64 large tiles 500 x 4000, d = 512: 25 / 12 and 26 / 14, d = 6144: 99 / 48 and 100 / 51; 96 large =
+// 376 small tiles 1000 x 6000, d = 512: 23 / 16 and 26 / 18, d = 2048: 44 / 36 and 45 / 40; 500 small tiles
+// 250 x 32000, d = 2048: 49 / 52 and 48 / 58; 704, 4000 x 2800: 53 / 62 and 54 / 69.
+constexpr int kMostSmallTiles = 448;
+static int projection_tile(int rows, int tiles) {
+  return (long)((rows + 127) / 128) * (2 * tiles) <= kMostSmallTiles ? 128 : kGemmTile;
+}
+// The gradients cut long contractions, so the large tile fills the device too, at the price of more partial sums.
+// By the groups of 128 terms of all small tiles (with the reduction; large / small): 384 of them 300 x 776, d = 1024:
+// 23 / 15; 1024, 500 x 4000, d = 512: 25 / 20; 2048, 500 x 8000: 28 / 26; 3072, 1000 x 6000: 31 / 33; 4096,
+// 500 x 4000, d = 2048: 36 / 40.
+constexpr int kMostSmallGroups = 1536;
+static int gradient_tile(const ct_cutce_shape& s) {
+  const long groups = 2L * ((s.rows + 127) / 128) * (s.hidden / 128) * (2 * vocab_tile_count(s.vocab));
+  return groups <= kMostSmallGroups ? 128 : kGemmTile;
+}
+
+// The statistics kernel's units: `chunks` of `per_chunk` tiles of `tile` columns.
+struct StatsUnits {
+  int tile, tiles, per_chunk, chunks;
+};
+static StatsUnits stats_units(const ct_cutce_shape& s) {
+  const int tiles = vocab_tile_count(s.vocab), row_blocks = padded_rows(s.rows) / kGemmTile;
+  if (projection_tile(s.rows, tiles) != kGemmTile) {
+    const int small = (s.vocab + 127) / 128;
+    return {128, small, 1, small};
+  }
+  const int t = tiles_per_chunk(tiles, row_blocks);
+  return {kGemmTile, tiles, t, (tiles + t - 1) / t};
 }
 
 // Heads whose rows do not all start on 16 bytes go through an aligned copy (cutce_panel_kernel).
@@ -1089,7 +1119,7 @@ static FwdLayout fwd_layout(const ct_cutce_shape& s) {
   L.target = L.idx + align_up((size_t)n_pad * sizeof(int), 256);
   L.active = L.target + align_up((size_t)n_pad * sizeof(int), 256);
   L.part = L.active + align_up((size_t)(n_pad / kGemmTile) * sizeof(int), 256);
-  L.sums = L.part + align_up((size_t)stats_chunks(s) * n_pad * 3 * sizeof(float), 256);
+  L.sums = L.part + align_up((size_t)stats_units(s).chunks * n_pad * 3 * sizeof(float), 256);
   L.base = L.sums + align_up((size_t)(n_pad / kMergeSlots) * 2 * sizeof(double), 256);
   L.total = L.base + full_panel_bytes(s);
   return L;
@@ -1097,15 +1127,26 @@ static FwdLayout fwd_layout(const ct_cutce_shape& s) {
 
 // Room for the partial sums (see CutceSplits). The bytes that the parts of dHidden take, and the number
 // of parts of dHead, are largest with every row active (times 4/3: a number of parts is rounded).
-static size_t hidden_sums_bytes(const ct_cutce_shape& s, int slab_tiles, bool with_head) {
-  const int row_blocks = padded_rows(s.rows) / kGemmTile;
-  const double parts = 2.0 * slab_tiles / part_length(row_blocks, s.hidden, slab_tiles, with_head);
+// Short problems get the room of both tiles: the large one cuts them into more parts, and a caller's bound on
+// the workspace that is a share of the preferred size (local_chunk_size) stays what it was.
+static size_t hidden_sums_bytes(const ct_cutce_shape& s, int tile, int slab_tiles, bool with_head) {
+  const int row_blocks = (s.rows + tile - 1) / tile, width = slab_tiles * kGemmTile;
+  const double parts = (double)(width / 128) / part_length(tile, row_blocks, s.hidden, width, with_head);
   const double least = 1.5 / row_blocks;  // with fewer not even a single row block is cut
-  return parts < least ? 0 : align_up((size_t)(1.34 * parts * padded_rows(s.rows) * s.hidden * sizeof(float)), 256);
+  return parts < least ? 0 : align_up((size_t)(1.34 * parts * row_blocks * tile * s.hidden * sizeof(float)), 256);
+}
+static size_t hidden_sums_bytes(const ct_cutce_shape& s, int slab_tiles, bool with_head) {
+  const size_t large = hidden_sums_bytes(s, kGemmTile, slab_tiles, with_head);
+  const size_t chosen = hidden_sums_bytes(s, gradient_tile(s), slab_tiles, with_head);
+  return large > chosen ? large : chosen;
+}
+static int most_head_parts(const ct_cutce_shape& s, int tile) {
+  const int row_blocks = (s.rows + tile - 1) / tile;
+  return whole_parts((float)(row_blocks * (tile / 128)) /
+                     part_length(tile, row_blocks, s.hidden, vocab_tile_count(s.vocab) * kGemmTile, true));
 }
 static int most_head_parts(const ct_cutce_shape& s) {
-  const int row_blocks = padded_rows(s.rows) / kGemmTile;
-  return whole_parts(2.f * row_blocks / part_length(row_blocks, s.hidden, vocab_tile_count(s.vocab), true));
+  return max(most_head_parts(s, kGemmTile), most_head_parts(s, gradient_tile(s)));
 }
 
 struct BwdLayout {
@@ -1209,7 +1250,7 @@ static int allow_gemm_lds(const char* fn, std::atomic<unsigned>& done, Kernels..
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 32) device = -1;
   if (device >= 0 && (done.load(std::memory_order_acquire) >> device & 1u)) return CT_OK;
   for (const void* kernel : {reinterpret_cast<const void*>(kernels)...}) {
-    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GemmSmem::kBytes);
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GemmShape<4>::kBytes);
     if (e != hipSuccess) return fail(CT_LAUNCH_FAILED, "%s: %s", fn, hipGetErrorString(e));
   }
   if (device >= 0) done.fetch_or(1u << device, std::memory_order_release);
@@ -1296,6 +1337,52 @@ static HeadView panel_view(const bf16* panel, int tile0, int tiles) {
   return HeadView{panel, nullptr, (long)tiles * kGemmTile, tile0 * kGemmTile, true};
 }
 
+template <int NB>
+static int launch_stats(const char* fn, hipStream_t stream, const CutceParams& p, bool guarded, float* part, int chunk0,
+                        int chunks, int tiles_per_chunk, float* cache) {
+  static std::atomic<unsigned> lds_allowed{0};
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<NB, false, false>, cutce_stats_kernel<NB, true, false>,
+                                cutce_stats_kernel<NB, false, true>, cutce_stats_kernel<NB, true, true>);
+  if (rc) return rc;
+  const auto kernel = cache ? (guarded ? cutce_stats_kernel<NB, true, true> : cutce_stats_kernel<NB, true, false>)
+                            : (guarded ? cutce_stats_kernel<NB, false, true> : cutce_stats_kernel<NB, false, false>);
+  const int slots = device_cu_count() * GemmShape<NB>::kGroups, units = chunks * ((p.N + 64 * NB - 1) / (64 * NB));
+  LaunchScope scope("cutce_stats_kernel", stream);
+  hipLaunchKernelGGL(kernel, dim3(min(slots, units)), dim3(256), GemmShape<NB>::kBytes, stream, p, part, chunk0, chunks,
+                     tiles_per_chunk, cache);
+  return scope.done();
+}
+
+// slab_tiles: of the kernel's tile size
+template <int NB>
+static int launch_dlogits(const char* fn, hipStream_t stream, const CutceParams& p, const CutceRowParams& rp, bool guarded,
+                          int slab0, int slab_tiles, int tiles_per_chunk, bf16* G) {
+  static std::atomic<unsigned> lds_allowed{0};
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_dlogits_kernel<NB, false>, cutce_dlogits_kernel<NB, true>);
+  if (rc) return rc;
+  const int slots = device_cu_count() * GemmShape<NB>::kGroups;
+  const int units = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk * ((p.N + 64 * NB - 1) / (64 * NB));
+  LaunchScope scope("cutce_dlogits_kernel", stream);
+  hipLaunchKernelGGL((guarded ? cutce_dlogits_kernel<NB, true> : cutce_dlogits_kernel<NB, false>), dim3(min(slots, units)),
+                     dim3(256), GemmShape<NB>::kBytes, stream, p, rp, slab0, slab_tiles, tiles_per_chunk, G);
+  return scope.done();
+}
+
+template <int NB>
+static int launch_grads(const char* fn, hipStream_t stream, const CutceParams& p, const CutceSlab& slab, const CutceSplits& sp,
+                        bool guarded) {
+  static std::atomic<unsigned> lds_allowed{0};
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_grads_kernel<NB, false, false>, cutce_grads_kernel<NB, true, false>,
+                                cutce_grads_kernel<NB, false, true>, cutce_grads_kernel<NB, true, true>);
+  if (rc) return rc;
+  const auto kernel = sp.with_head ? (guarded ? cutce_grads_kernel<NB, true, true> : cutce_grads_kernel<NB, true, false>)
+                                   : (guarded ? cutce_grads_kernel<NB, false, true> : cutce_grads_kernel<NB, false, false>);
+  LaunchScope scope(sp.with_head ? "cutce_grads_kernel" : "cutce_dhidden_kernel", stream);
+  hipLaunchKernelGGL(kernel, dim3(device_cu_count() * GemmShape<NB>::kGroups), dim3(256), GemmShape<NB>::kBytes, stream, p, slab,
+                     sp);
+  return scope.done();
+}
+
 // Shared body of ct_cutce_fwd and ct_cutce_fwd_noalloc: `ws` / `ws_bytes` is the workspace to use
 // (the caller's, or this device's static scratch array), `fn` the name for error texts.
 static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_, size_t ws_bytes,
@@ -1320,8 +1407,6 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, a->sparse_compaction, ws);
   float* part = reinterpret_cast<float*>(ws + L.part);
   double* sums = reinterpret_cast<double*>(ws + L.sums);
-  const int chunks = stats_chunks(a->shape), row_blocks = p.n_pad / kGemmTile, tiles = vocab_tile_count(p.V);
-  const int per_chunk = tiles_per_chunk(tiles, row_blocks);
   const bf16* head = p.head.base;
 
   LaunchScope scope1("cutce_index_kernel", stream);
@@ -1331,46 +1416,39 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
                      CutceRowParams{});
   if ((rc = scope1.done())) return rc;
 
+  const StatsUnits units = stats_units(a->shape);
   // The panel of a head with unaligned rows: at the end of the logits cache, where the backward finds
   // it again, or in what the workspace has behind its fixed part, a number of chunks at a time.
+  const int step_tiles = units.per_chunk, step_chunks = kGemmTile / units.tile;  // 256-column tiles and chunks of a panel step
   bf16* panel = nullptr;
-  int chunks_per_pass = chunks;
+  int chunks_per_pass = units.chunks;
   if (needs_panel(a->shape)) {
     if (a->logits_cache) {
       panel = reinterpret_cast<bf16*>(static_cast<char*>(a->logits_cache) + logits_bytes(a->shape));
     } else {
-      const size_t chunk_bytes = panel_tile_bytes(a->shape) * per_chunk;
-      const size_t fit = ws_bytes >= L.total ? (size_t)chunks : (ws_bytes - L.base) / chunk_bytes;
+      const size_t fit = ws_bytes >= L.total ? (size_t)units.chunks : (ws_bytes - L.base) / (panel_tile_bytes(a->shape) * step_tiles);
       if (fit) panel = reinterpret_cast<bf16*>(ws + L.base);
-      if (fit) chunks_per_pass = (int)(fit < (size_t)chunks ? fit : (size_t)chunks);
+      if (fit) chunks_per_pass = (int)(fit * step_chunks < (size_t)units.chunks ? fit * step_chunks : (size_t)units.chunks);
     }
   }
-  const size_t smem = GemmSmem::kBytes;
-  static std::atomic<unsigned> lds_allowed{0};
-  if ((rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<false, false>, cutce_stats_kernel<true, false>,
-                           cutce_stats_kernel<false, true>, cutce_stats_kernel<true, true>)))
-    return rc;
   const bool guarded = !p.hidden_aligned || (!panel && !(is_aligned16(head) && p.V % 8 == 0));
-  const auto stats = a->logits_cache ? (guarded ? cutce_stats_kernel<true, true> : cutce_stats_kernel<true, false>)
-                                     : (guarded ? cutce_stats_kernel<false, true> : cutce_stats_kernel<false, false>);
-  for (int chunk0 = 0; chunk0 < chunks; chunk0 += chunks_per_pass) {
-    const int pass_chunks = min(chunks_per_pass, chunks - chunk0);
+  for (int chunk0 = 0; chunk0 < units.chunks; chunk0 += chunks_per_pass) {
+    const int pass_chunks = min(chunks_per_pass, units.chunks - chunk0);
     if (panel) {
-      const int tile0 = chunk0 * per_chunk, pass_tiles = min(pass_chunks * per_chunk, tiles - tile0);
+      const int tile0 = chunk0 / step_chunks * step_tiles;
+      const int pass_tiles = min((pass_chunks + step_chunks - 1) / step_chunks * step_tiles, vocab_tile_count(p.V) - tile0);
       if ((rc = launch_panel(stream, head, a->shape, tile0, pass_tiles, panel, p.header))) return rc;
       p.head = panel_view(panel, tile0, pass_tiles);
     }
-    const int persistent = min(device_cu_count(), pass_chunks * row_blocks);
-    LaunchScope scope2("cutce_stats_kernel", stream);
-    hipLaunchKernelGGL(stats, dim3(persistent), dim3(256), smem, stream, p, part, chunk0, pass_chunks, per_chunk,
-                       static_cast<float*>(a->logits_cache));
-    if ((rc = scope2.done())) return rc;
+    const auto launch = units.tile == kGemmTile ? launch_stats<4> : launch_stats<2>;
+    if ((rc = launch(fn, stream, p, guarded, part, chunk0, pass_chunks, units.per_chunk, static_cast<float*>(a->logits_cache))))
+      return rc;
   }
 
   const int merge_blocks = p.n_pad / kMergeSlots;
   LaunchScope scope3("cutce_merge_kernel", stream);
   hipLaunchKernelGGL(cutce_merge_kernel, dim3(merge_blocks), dim3(kMergeSlots * kMergeParts), 0, stream, p, part,
-                     chunks, a->lse, sums);
+                     units.chunks, a->lse, sums);
   if ((rc = scope3.done())) return rc;
   LaunchScope scope4("cutce_finalize_kernel", stream);
   hipLaunchKernelGGL(cutce_finalize_kernel, dim3(1), dim3(64), 0, stream, sums, merge_blocks,
@@ -1466,13 +1544,6 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   rp.fac = reinterpret_cast<float*>(ws + L.rowparams);
   rp.lse2 = reinterpret_cast<float*>(ws + L.rowparams + params_stride);
   rp.tgt = reinterpret_cast<int*>(ws + L.rowparams + 2 * params_stride);
-  const size_t smem = GemmSmem::kBytes;
-  static std::atomic<unsigned> lds_allowed{0};
-  if ((rc = allow_gemm_lds("ct_cutce_bwd", lds_allowed, cutce_dlogits_kernel<false>, cutce_dlogits_kernel<true>,
-                           cutce_grads_kernel<false, false>, cutce_grads_kernel<true, false>, cutce_grads_kernel<false, true>,
-                           cutce_grads_kernel<true, true>)))
-    return rc;
-
   LaunchScope scope5("cutce_index_kernel", stream);
   hipLaunchKernelGGL(cutce_index_kernel<true>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p, a->lse, a->dy, rp);
   if ((rc = scope5.done())) return rc;
@@ -1500,8 +1571,6 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   // (an unaligned head with a multiple of 8 columns has no panel)
   const bool guarded_head = !needs_panel(a->shape) && !head_aligned;
   const bool guarded_logits = guarded_head || !p.hidden_aligned;
-  const auto grads = dhead ? (guarded_head ? cutce_grads_kernel<true, true> : cutce_grads_kernel<true, false>)
-                           : (guarded_head ? cutce_grads_kernel<false, true> : cutce_grads_kernel<false, false>);
   for (int s = 0; s < L.slabs; ++s) {
     const int slab0 = s * L.slab_cols;
     const int slab_tiles = min(tiles_per_slab, tiles - s * tiles_per_slab);
@@ -1517,12 +1586,14 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
                          cache, slab0, slab_width, G);
       if ((rc = scope11.done())) return rc;
     } else {
-      LaunchScope scope7("cutce_dlogits_kernel", stream);
-      const int per_chunk = tiles_per_chunk(slab_tiles, row_blocks);
-      const int dl_units = ((slab_tiles + per_chunk - 1) / per_chunk) * row_blocks;
-      hipLaunchKernelGGL(guarded_logits ? cutce_dlogits_kernel<true> : cutce_dlogits_kernel<false>, dim3(min(cus, dl_units)),
-                         dim3(256), smem, stream, p, rp, slab0, slab_tiles, per_chunk, G);
-      if ((rc = scope7.done())) return rc;
+      if (projection_tile(p.N, slab_tiles) == kGemmTile) {
+        rc = launch_dlogits<4>("ct_cutce_bwd", stream, p, rp, guarded_logits, slab0, slab_tiles,
+                               tiles_per_chunk(slab_tiles, row_blocks), G);
+      } else {  // (an unpadded head has no columns past the vocabulary to read)
+        const int columns = p.head.padded ? slab_width : min(slab_width, p.V - slab0);
+        rc = launch_dlogits<2>("ct_cutce_bwd", stream, p, rp, guarded_logits, slab0, (columns + 127) / 128, 1, G);
+      }
+      if (rc) return rc;
     }
     const int mode = L.slabs == 1 ? 0 : (s == 0 ? 1 : (s == L.slabs - 1 ? 3 : 2));
     const CutceSlab slab = {G, packed, slab0, slab_width, mode, dh_acc, dhidden, dhead};
@@ -1531,11 +1602,11 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
     sp.head_sums = reinterpret_cast<float*>(ws + L.head_sums);
     sp.hidden_room = L.hidden_sums_bytes / sizeof(float);
     sp.head_most = L.head_most;
-    sp.all_tiles = tiles;
+    sp.tile = gradient_tile(a->shape);
+    sp.vocab = tiles * kGemmTile;
     sp.with_head = dhead != nullptr;
-    LaunchScope scope8(dhead ? "cutce_grads_kernel" : "cutce_dhidden_kernel", stream);
-    hipLaunchKernelGGL(grads, dim3(cus), dim3(256), smem, stream, p, slab, sp);
-    if ((rc = scope8.done())) return rc;
+    rc = (sp.tile == kGemmTile ? launch_grads<4> : launch_grads<2>)("ct_cutce_bwd", stream, p, slab, sp, guarded_head);
+    if (rc) return rc;
     if (sp.hidden_room || sp.head_most > 1) {
       LaunchScope scope9("cutce_reduce_kernel", stream);
       const long quads = max((long)p.n_pad * p.d, sp.head_most > 1 ? (long)p.d * slab_width : 0) / 4;

@@ -1,16 +1,16 @@
-// 256 x 256 workgroup-tile bf16 GEMM core for gfx950, used by the cut
-// cross-entropy kernels.
+// Workgroup-tile bf16 GEMM core for gfx950, used by the cut cross-entropy kernels.
 //
-// 4 wavefronts in a 2 x 2 arrangement, 128 x 128 outputs per wavefront held
-// as 4 x 4 mfma32 accumulator blocks (256 f32 registers per lane). The
-// contraction runs in steps of BK = 32.
+// 4 wavefronts in a 2 x 2 arrangement, each with NB x NB mfma32 accumulator blocks. NB = 4: a tile of
+// 256 x 256, 256 f32 registers per lane, one workgroup per compute unit; NB = 2: 128 x 128, 64 registers, two
+// workgroups per compute unit, for problems with few tiles (which one: projection_tile and gradient_tile in
+// ct_cutce.hip). The contraction runs in steps of BK = 32.
 //
 // An operand comes in one of two memory layouts:
 //   KcLoader  "k-contiguous": matrix rows are the M (or N) index, the
-//             contraction index is contiguous. LDS tile [256][BK], MFMA
+//             contraction index is contiguous. LDS tile [64 NB][BK], MFMA
 //             fragments read with ds_read_b128.
 //   McLoader  "m-contiguous": matrix rows are the contraction index, the M
-//             (or N) index is contiguous. LDS tile [BK][256], fragments read
+//             (or N) index is contiguous. LDS tile [BK][64 NB], fragments read
 //             with transposed LDS reads.
 // The rows of a k-contiguous operand can be addressed through an index list (gather).
 //
@@ -19,7 +19,7 @@
 //   pipelined  operands 16-byte aligned, contraction a multiple of 128: tiles are copied global ->
 //              LDS asynchronously, three steps ahead, into a ring of 4 LDS stages; MFMA fragments
 //              are double buffered in registers so that LDS reads of the next half step overlap
-//              the 16 MFMAs of the current one; one barrier per step (gen_gemm_asm.py). Rows or
+//              the current MFMAs; one barrier per step (gen_gemm_asm.py). Rows or
 //              columns of a tile past the end of the matrix are copies of valid ones.
 //   guarded    unaligned operands: element-wise guarded loads that zero fill, staged through
 //              registers, 2 LDS stages.
@@ -30,7 +30,7 @@
 
 namespace ct {
 
-constexpr int kGemmTile = 256;
+constexpr int kGemmTile = 256;  // of the large tile, and what row blocks and vocabulary are padded to
 constexpr int kGemmBK = 32;
 
 CT_DEVICE u32x4 load_chunk_guarded(const bf16* p, int count) {
@@ -40,31 +40,36 @@ CT_DEVICE u32x4 load_chunk_guarded(const bf16* p, int count) {
   return as_u32x4(v);
 }
 
-struct GemmSmem {
-  static constexpr int kTileBytes = kGemmTile * kGemmBK * 2;  // 16 KB
-  static constexpr int kStageBytes = 2 * kTileBytes;          // A tile then B tile
+// A workgroup's tile: 4 wavefronts of NB x NB accumulator blocks.
+template <int NB>
+struct GemmShape {
+  static constexpr int kTile = 64 * NB, kWave = 32 * NB;
+  static constexpr int kTileBytes = kTile * kGemmBK * 2;  // NB = 4: 16 KB
+  static constexpr int kStageBytes = 2 * kTileBytes;      // A tile then B tile
   static constexpr int kStages = 4;
-  static constexpr size_t kBytes = (size_t)kStages * kStageBytes;  // 128 KB
+  static constexpr int kGroups = NB == 4 ? 1 : 2;         // workgroups per compute unit that registers are for
+  static constexpr size_t kBytes = (size_t)kStages * kStageBytes;  // NB = 4: 128 KB
 };
 
 // In both loaders thread t owns the 16-byte LDS slots t + 256 n of the tile
-// (n < 4): slot P holds physical chunk P % CPR of row P / CPR, i.e. logical
+// (n < NB): slot P holds physical chunk P % CPR of row P / CPR, i.e. logical
 // chunk (P % CPR) ^ swizzle(row); voff[n] is the byte offset of that chunk
 // from `base` at k = 0 (32 bits: the host checks sizes and strides against it).
+template <int NB>
 struct KcLoader {
   static constexpr int CPR = kGemmBK / 8;  // 4
-  static constexpr int NCH = 4;
+  static constexpr int NCH = NB;
   const char* base;    // uniform
   unsigned voff[NCH];
   u32x4 regs[NCH];
   int chunk, k_valid;
 
-  // rows m0 .. m0+255 of `base_` (leading dimension ld elements), optionally
+  // rows m0 .. of `base_` (leading dimension ld elements), optionally
   // gathered through row_index. Rows >= rows_valid are copies of the first row (callers discard
   // what they get from them); the guarded loop reads k >= k_valid as zero.
-  // With interleave_rows, tile row 128 w + 32 nb + j holds matrix row m0 + 128 w + 4 j + nb:
-  // in the accumulator layout lane j of a wavefront then owns 4 consecutive matrix rows (its
-  // column blocks nb = 0..3), which an epilogue can store with one 8- or 16-byte access.
+  // With interleave_rows, row 32 nb + j of a wavefront's rows holds matrix row NB j + nb of them:
+  // in the accumulator layout lane j of a wavefront then owns NB consecutive matrix rows (its
+  // column blocks), which an epilogue can store with one access.
   CT_DEVICE void init(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid,
                       int k_valid_, bool interleave_rows = false) {
     const int t = threadIdx.x;
@@ -76,8 +81,8 @@ struct KcLoader {
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
       const int tile_row = r0 + 64 * n;
-      const int r = interleave_rows ? ((tile_row & 128) | ((tile_row & 31) << 2) | ((tile_row >> 5) & 3))
-                                    : tile_row;
+      constexpr int wave_rows = 32 * NB;
+      const int r = interleave_rows ? ((tile_row & wave_rows) | ((tile_row & 31) * NB) | ((tile_row >> 5) % NB)) : tile_row;
       const bool ok = m0 + r < rows_valid;
       const long src = gathered ? row_index[ok ? m0 + r : 0] : (ok ? r : 0);
       voff[n] = (unsigned)((src * ld + chunk * 8) * 2);
@@ -114,9 +119,11 @@ struct KcLoader {
   }
 };
 
+template <int NB>
 struct McLoader {
-  static constexpr int CPR = kGemmTile / 8;  // 32
-  static constexpr int NCH = 4;
+  static constexpr int CPR = 8 * NB;           // 16-byte chunks of a tile row
+  static constexpr int NCH = NB;
+  static constexpr int kRowsPerPass = 256 / CPR;
   const char* base;  // uniform: column m0 of row 0
   long ld;
   unsigned voff[NCH];
@@ -124,7 +131,7 @@ struct McLoader {
   int col[2];  // first column of the chunk fetched in even / odd passes
   int cols_left, k_valid;
 
-  // columns m0 .. m0+255 of `base_`. The guarded loop reads columns >= cols_valid and rows >= k_valid
+  // columns m0 .. of `base_`. The guarded loop reads columns >= cols_valid and rows >= k_valid
   // as zero; the pipelined one, where cols_valid is a multiple of 8, such columns as copies of the
   // tile's first 8 (callers discard what they get from them).
   CT_DEVICE void init(const bf16* base_, long ld_, int m0, int cols_valid, int k_valid_) {
@@ -135,7 +142,7 @@ struct McLoader {
     cols_left = cols_valid - m0;
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      const int r = t / CPR + 8 * n;
+      const int r = t / CPR + kRowsPerPass * n;
       int c = ((t % CPR) ^ swizzle<CPR>(r)) * 8;
       col[n & 1] = c;
       if (c >= cols_left) c = 0;
@@ -154,7 +161,7 @@ struct McLoader {
     const int r0 = (int)threadIdx.x / CPR;
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      const int k = k0 + r0 + 8 * n;
+      const int k = k0 + r0 + kRowsPerPass * n;
       const int count = min(max(cols_left - col[n & 1], 0), 8);
       if (k < k_valid && count) {
         regs[n] = load_chunk_guarded(reinterpret_cast<const bf16*>(base + (size_t)k0 * ld * 2 + voff[n]), count);
@@ -173,20 +180,22 @@ struct McLoader {
   }
 };
 
+template <int NB>
 struct GemmAcc {
-  f32x16 c[4][4];
+  typedef float Lane __attribute__((ext_vector_type(NB)));  // a lane's consecutive elements of a row
+  f32x16 c[NB][NB];
   CT_DEVICE void clear() {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NB; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) c[a][b] = zero16();
+      for (int b = 0; b < NB; ++b) c[a][b] = zero16();
   }
   // Wait states between the compiler's last MFMA and value(), whose read it does not see.
   CT_DEVICE void settle() {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NB; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) asm volatile("" : "+a"(c[a][b]));
+      for (int b = 0; b < NB; ++b) asm volatile("" : "+a"(c[a][b]));
     asm volatile("s_nop 15\n\ts_nop 7");
   }
   // An element, read where the call stands. (An epilogue's branches otherwise have the reads and what
@@ -196,24 +205,40 @@ struct GemmAcc {
     asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(c[i][nb][r]));
     return v;
   }
-  CT_DEVICE f32x4 quad(int i, int r) const { return f32x4{value(i, 0, r), value(i, 1, r), value(i, 2, r), value(i, 3, r)}; }
+  CT_DEVICE Lane lane(int i, int r) const {
+    Lane out;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) out[nb] = value(i, nb, r);
+    return out;
+  }
 };
+
+// Stores of a lane's consecutive elements at a wave-uniform address plus a 32-bit lane offset.
+CT_DEVICE void store_lane(void* row, unsigned lane_offset, f32x4 v) { store_global16_s<0>(row, lane_offset, v); }
+CT_DEVICE void store_lane(void* row, unsigned lane_offset, bf16x4 v) { store_global8_s<0>(row, lane_offset, v); }
+CT_DEVICE void store_lane(void* row, unsigned lane_offset, f32x2 v) {
+  store_global8_s<0>(row, lane_offset, __builtin_bit_cast(bf16x4, v));
+}
+CT_DEVICE void store_lane(void* row, unsigned lane_offset, bf16x2 v) {
+  store_global4_s<0>(row, lane_offset, __builtin_bit_cast(float, v));
+}
+CT_DEVICE bf16x4 to_bf16(f32x4 v) { return bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]}; }
+CT_DEVICE bf16x2 to_bf16(f32x2 v) { return bf16x2{(bf16)v[0], (bf16)v[1]}; }
 
 struct GemmFrags {
   bf16x8 a[4], b[4];
 };
 
-template <class ALoader, class BLoader>
-CT_DEVICE void load_frags(GemmFrags& f, int stage_off, const typename ALoader::FragOffsets& afo,
-                          const typename BLoader::FragOffsets& bfo, int ks, int wm, int wn) {
+CT_DEVICE void load_frags(GemmFrags& f, int stage_off, const McLoader<4>::FragOffsets& afo,
+                          const KcLoader<4>::FragOffsets& bfo, int ks, int wm, int wn) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    f.a[i] = ALoader::frag(stage_off, afo, ks, wm, i);
-    f.b[i] = BLoader::frag(stage_off + GemmSmem::kTileBytes, bfo, ks, wn, i);
+    f.a[i] = McLoader<4>::frag(stage_off, afo, ks, wm, i);
+    f.b[i] = KcLoader<4>::frag(stage_off + GemmShape<4>::kTileBytes, bfo, ks, wn, i);
   }
 }
 
-CT_DEVICE void mfma_block(const GemmFrags& f, GemmAcc& acc) {
+CT_DEVICE void mfma_block(const GemmFrags& f, GemmAcc<4>& acc) {
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -235,9 +260,9 @@ CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
   return ((unsigned long long)hi << 32) | (unsigned long long)lo;
 }
-CT_DEVICE void gemm_loop_scheduled(const McLoader& A, const KcLoader& B, int k_begin, int steps,
-                                   lds_addr smem, const McLoader::FragOffsets& afo,
-                                   const KcLoader::FragOffsets& bfo, int wm, int wn, GemmAcc& acc) {
+CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, int steps,
+                                   lds_addr smem, const McLoader<4>::FragOffsets& afo,
+                                   const KcLoader<4>::FragOffsets& bfo, int wm, int wn, GemmAcc<4>& acc) {
   const int wave = uniform(threadIdx.x >> 6);
   // sources of the copies of step 3
   const unsigned long long src_a =
@@ -247,7 +272,7 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader& A, const KcLoader& B, int k_b
   const unsigned steps_u = (unsigned)uniform(steps);
   const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + wave * 1024));
   const int a_off = (wm / 128) * 256;
-  const int b_off = GemmSmem::kTileBytes + (wn / 32) * KcLoader::FragOffsets::kRowBlockBytes;
+  const int b_off = GemmShape<4>::kTileBytes + (wn / 32) * KcLoader<4>::FragOffsets::kRowBlockBytes;
   asm volatile(CT_GEMM_LOOP
                : "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[0][2]), "+a"(acc.c[0][3]),
                  "+a"(acc.c[1][0]), "+a"(acc.c[1][1]), "+a"(acc.c[1][2]), "+a"(acc.c[1][3]),
@@ -265,13 +290,13 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader& A, const KcLoader& B, int k_b
 // acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T (k_end - k_begin a multiple of 128
 // unless GUARDED). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
 template <bool GUARDED>
-CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_addr smem, GemmAcc& acc) {
-  constexpr int BK = kGemmBK, kTile = GemmSmem::kTileBytes, kStage = GemmSmem::kStageBytes;
+CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
+  constexpr int BK = kGemmBK, kTile = GemmShape<4>::kTileBytes, kStage = GemmShape<4>::kStageBytes;
   const int w = threadIdx.x >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
   if (k_begin >= k_end) return;
-  const McLoader::FragOffsets afo(smem);
-  const KcLoader::FragOffsets bfo(smem);
+  const McLoader<4>::FragOffsets afo(smem);
+  const KcLoader<4>::FragOffsets bfo(smem);
   if constexpr (!GUARDED) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
 #pragma unroll
@@ -279,7 +304,7 @@ CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_a
       A.dma(k_begin + i * BK, smem + i * kStage);
       B.dma(k_begin + i * BK, smem + i * kStage + kTile);
     }
-    static_assert(McLoader::NCH + KcLoader::NCH == 8, "the wait leaves the copies of two steps in flight");
+    static_assert(McLoader<4>::NCH + KcLoader<4>::NCH == 8, "the wait leaves the copies of two steps in flight");
     wait_vmcnt16();
     workgroup_barrier();
     gemm_loop_scheduled(A, B, k_begin, (k_end - k_begin) / BK, smem, afo, bfo, wm, wn, acc);
@@ -299,7 +324,7 @@ CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_a
 #pragma unroll
       for (int ks = 0; ks < BK / 16; ++ks) {
         GemmFrags f;
-        load_frags<McLoader, KcLoader>(f, cur, afo, bfo, ks, wm, wn);
+        load_frags(f, cur, afo, bfo, ks, wm, wn);
         mfma_block(f, acc);
       }
       if (more) {
@@ -310,6 +335,74 @@ CT_DEVICE void gemm_tile(McLoader& A, KcLoader& B, int k_begin, int k_end, lds_a
       const int tmp = cur;
       cur = nxt;
       nxt = tmp;
+    }
+    acc.settle();
+  }
+}
+
+// The same sum for the small tile (NB = 2: 128 x 128, 64 accumulator registers, two workgroups per
+// compute unit), with a fixed order of its own (gen_gemm_asm.py).
+template <bool GUARDED>
+CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
+  typedef GemmShape<2> Shape;
+  typedef RowFragOffsets<KcLoader<2>::CPR> BOffsets;
+  constexpr int kStage = Shape::kStageBytes, kTile = Shape::kTileBytes;
+  if (k_begin >= k_end) return;
+  const int w = uniform(threadIdx.x >> 6), wm = (w >> 1) * Shape::kWave, wn = (w & 1) * Shape::kWave, l = lane_id();
+  // this lane's part of the wavefront's fragments, stage 0
+  lds_addr a_ptr[2][2];
+#pragma unroll
+  for (int second = 0; second < 2; ++second)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = 8 * (l >> 5) + 4 * second + ((l & 15) >> 2), col = wm + 32 * i + 16 * ((l >> 4) & 1) + 4 * (l & 3);
+      a_ptr[second][i] = smem + tile_byte_offset<McLoader<2>::CPR>(row, col >> 3) + (col & 4) * 2;
+    }
+  const BOffsets b_ptr(smem + kTile + (wn / 32) * BOffsets::kRowBlockBytes);
+  if constexpr (!GUARDED) {
+    static_assert(McLoader<2>::NCH + KcLoader<2>::NCH == 4, "the waits count the copies of a step");
+    dma_wait_all();  // nothing of ours may still be in flight when counting copies below
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      A.dma(k_begin + i * kGemmBK, smem + i * kStage);
+      B.dma(k_begin + i * kGemmBK, smem + i * kStage + kTile);
+    }
+    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // step 0 has landed
+    const unsigned long long src_a = uniform64(A.base + (size_t)(k_begin + 3 * kGemmBK) * (size_t)A.ld * 2);
+    const unsigned long long src_b = uniform64(B.base + (size_t)(k_begin + 3 * kGemmBK) * 2);
+    const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
+    const unsigned steps = (unsigned)uniform((k_end - k_begin) / kGemmBK);
+    const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + w * 1024));
+    asm volatile(CT_GEMM_SMALL_LOOP
+                 : "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[1][0]), "+a"(acc.c[1][1])
+                 : "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps), "s"(lds_wave), "v"(a_ptr[0][0]), "v"(a_ptr[0][1]),
+                   "v"(a_ptr[1][0]), "v"(a_ptr[1][1]), "v"(b_ptr.ptr[0]), "v"(b_ptr.ptr[1]), "v"(A.voff[0]), "v"(A.voff[1]),
+                   "v"(B.voff[0]), "v"(B.voff[1])
+                 : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
+  } else {
+#pragma nounroll
+    for (int k0 = k_begin; k0 < k_end; k0 += kGemmBK) {
+      A.fetch(k0);
+      B.fetch(k0);
+      A.commit(smem);
+      B.commit(smem + kTile);
+      __syncthreads();
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 a[2], b[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int off = ks * (16 * McLoader<2>::CPR * 16);
+          const bf16x4_vs lo = lds_load_tr(a_ptr[0][i] + off), hi = lds_load_tr(a_ptr[1][i] + off);
+          a[i] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          b[i] = b_ptr.load(0, i, ks);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc.c[i][j] = mfma32(a[i], b[j], acc.c[i][j]);
+      }
+      __syncthreads();
     }
     acc.settle();
   }

@@ -1,4 +1,4 @@
-"""Generates ct_gemm_asm.inc: the hand-scheduled main loop of the 256 x 256 GEMM tile.
+"""Generates ct_gemm_asm.inc: the hand-scheduled main loops of the 256 x 256 and 128 x 128 GEMM tiles.
 
 One wavefront runs on each SIMD, so whatever the wavefront issues between two MFMAs must fit
 into the 32 cycles the matrix pipe is busy with the first of them, or the pipe drains. A
@@ -133,17 +133,94 @@ def gemm_loop():
     return lines
 
 
+# ---------------------------------------------------------------------------
+# The 128 x 128 tile (2 x 2 blocks per wavefront; ring of 4 LDS stages of 16 KB)
+# ---------------------------------------------------------------------------
+# 8 MFMAs a step are too few to read a step's second half of fragments behind its first, so all fragments
+# of step k + 1 are read, into the other of two register sets, behind the MFMAs of step k:
+#
+#   step k, stage s = k % 4
+#     the fragments of step k have arrived (they were read during step k-1: stage s is free now)
+#     MFMA 0; behind it: this wavefront's copies of step k+1 have landed (vmcnt(8): steps k+2 and
+#       k+3 may stay in flight), barrier
+#     reads of step k+1's fragments behind MFMA 1..6, copies of step k+4 -> stage s behind MFMA 1, 3, 5, 7
+#
+# Fixed registers (clobbers): v[64:95], v[96:127] the two sets, s[40:41] / s[42:43], s44, s45-s46 as above.
+SMALL_STAGE, SMALL_SETS = 16384, (64, 96)
+SMALL_ACC = lambda i, j: "%%%d" % (2 * i + j)
+SMALL_IN = {name: "%%%d" % (4 + k) for k, name in enumerate(
+    ["src_a", "src_b", "stride_a", "steps", "lds_wave", "a00", "a01", "a10", "a11", "b0", "b1", "va0", "va1", "vb0", "vb1"])}
+
+
+def small_frag(register_set, operand, ks, i):
+    return SMALL_SETS[register_set] + 16 * ks + 8 * operand + 4 * i
+
+
+def small_reads(stage, register_set):
+    """the 12 reads of a step's fragments, in the order of their use"""
+    out = []
+    for ks in range(2):
+        for i in range(2):
+            for second in range(2):
+                lo = small_frag(register_set, 0, ks, i) + 2 * second
+                out.append("ds_read_b64_tr_b16 v[%d:%d], %s offset:%d" % (
+                    lo, lo + 1, SMALL_IN["a%d%d" % (second, i)], stage * SMALL_STAGE + ks * 4096))
+            lo = small_frag(register_set, 1, ks, i)
+            out.append("ds_read_b128 v[%d:%d], %s offset:%d" % (
+                lo, lo + 3, SMALL_IN["b%d" % ks], stage * SMALL_STAGE + i * 2048))
+    return out
+
+
+def small_copy(operand, n, stage):
+    return ["s_add_u32 m0, %s, %d" % (SMALL_IN["lds_wave"], stage * SMALL_STAGE + operand * 8192 + n * 4096), "s_nop 0",
+            "global_load_lds_dwordx4 %s, %s" % (SMALL_IN["v%s%d" % ("ab"[operand], n)], ("s[40:41]", "s[42:43]")[operand])]
+
+
+def small_step(u):
+    stage, current, other = u, u & 1, (u + 1) & 1
+    reads = small_reads((u + 1) & 3, other)
+    behind = {m: [] for m in range(8)}
+    behind[0] = [ln.replace(STRIDE_A, SMALL_IN["stride_a"]).replace(STEPS, SMALL_IN["steps"]) for ln in ADVANCE]
+    behind[0] += ["s_waitcnt vmcnt(8)", "s_barrier"]
+    for m in range(1, 7):
+        behind[m] += reads[2 * m - 2:2 * m]
+    for m, (operand, n) in {1: (0, 0), 3: (0, 1), 5: (1, 0), 7: (1, 1)}.items():
+        behind[m] += small_copy(operand, n, stage)
+    lines = ["s_waitcnt lgkmcnt(0)"]
+    for m in range(8):
+        ks, i, j = m >> 2, (m >> 1) & 1, m & 1
+        a, b = small_frag(current, 0, ks, i), small_frag(current, 1, ks, j)
+        lines.append("v_mfma_f32_32x32x16_bf16 %s, v[%d:%d], v[%d:%d], %s" % (
+            SMALL_ACC(i, j), a, a + 3, b, b + 3, SMALL_ACC(i, j)))
+        lines += behind[m]
+    return lines
+
+
+def small_loop():
+    lines = ["s_mov_b64 s[40:41], " + SMALL_IN["src_a"], "s_mov_b64 s[42:43], " + SMALL_IN["src_b"], "s_mov_b32 s44, 4"]
+    lines += small_reads(0, 0)
+    lines.append("ct_gemm_small_loop_%=:")
+    for u in range(4):
+        lines += small_step(u)
+    # (s44 has advanced by 4: the steps done are s44 - 4; the last one read fragments that nobody uses)
+    lines += ["s_sub_u32 s45, s44, 4", "s_cmp_lt_u32 s45, " + SMALL_IN["steps"], "s_cbranch_scc1 ct_gemm_small_loop_%="]
+    lines += ["s_waitcnt vmcnt(0)", "s_waitcnt lgkmcnt(0)", "s_barrier", "s_nop 15", "s_nop 7"]
+    return lines
+
+
 def emit(lines, name):
     body = " \\\n".join('  "%s\\n\\t"' % ln for ln in lines)
     return "#define %s \\\n%s\n" % (name, body)
 
 
-def clobbers():
-    regs = ["v%d" % r for r in range(F0A, HI + 10)] + ["s%d" % r for r in range(40, 47)]
+def clobbers(first, end):
+    regs = ["v%d" % r for r in range(first, end)] + ["s%d" % r for r in range(40, 47)]
     return ", ".join('"%s"' % r for r in regs)
 
 
 if __name__ == "__main__":
     print("// Generated by gen_gemm_asm.py -- do not edit by hand.")
     print(emit(gemm_loop(), "CT_GEMM_LOOP"))
-    print("#define CT_GEMM_LOOP_CLOBBERS %s" % clobbers())
+    print("#define CT_GEMM_LOOP_CLOBBERS %s" % clobbers(F0A, HI + 10))
+    print(emit(small_loop(), "CT_GEMM_SMALL_LOOP"))
+    print("#define CT_GEMM_SMALL_LOOP_CLOBBERS %s" % clobbers(SMALL_SETS[0], SMALL_SETS[1] + 32))

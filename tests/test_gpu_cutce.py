@@ -460,3 +460,28 @@ def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
         ct._lib.check(lib.ct_cutce_fwd(ct._lib.current_stream(), args))
         results.append(out.cpu())
     assert all(torch.equal(r, results[0]) for r in results[1:]) and torch.isfinite(results[0]).all()
+
+
+@pytest.mark.parametrize("rows,width,vocab", [
+    (129, 128, 248),      # both products in 128 x 128 tiles, one column and one row past a tile
+    (1024, 256, 7168),    # 8 x 56 small tiles: the last projection that takes them, gradients in large ones
+    (1025, 256, 6300),    # 9 x 50: the first in large tiles, unaligned rows
+    (897, 640, 1288),     # gradients in small tiles, the last 8 columns from the tail
+    (1025, 1152, 1288),   # small tiles for the projection, large ones for the gradients
+])
+def test_output_tile_sizes(ct, gpu, rows, width, vocab):
+    """Sizes on both sides of the lines between the 128 x 128 and the 256 x 256 tiles, with and without the logits
+    cache and compaction; dHead is the same for every workspace."""
+
+    case = _case(rows + vocab, rows, width, vocab)
+    for cache, compaction in ((False, True), (True, True), (False, False)):
+        print("case", rows, width, vocab, cache, compaction, flush=True)
+        _check(_gpu(ct, gpu, *case, 0.37, compaction=compaction, cache=cache), *case, 0.37)
+    hidden, head, targets, weights = (t.to(gpu) for t in case)
+    dy = torch.tensor(0.37, device=gpu)
+    _, _, lse = ct.cutce_forward(hidden, head, targets, weights, sparse_compaction=True)
+    whole = ct.cutce_backward(hidden, head, targets, weights, lse, dy, sparse_compaction=True)
+    least = ct.cut_cross_entropy.backward_workspace_bytes(rows, width, vocab, 1)
+    slabs = ct.cutce_backward(hidden, head, targets, weights, lse, dy, sparse_compaction=True, workspace_bytes=least)
+    assert torch.equal(whole[1], slabs[1])
+    assert relative_l2(slabs[0].cpu(), whole[0].cpu()) <= GRAD_RTOL
