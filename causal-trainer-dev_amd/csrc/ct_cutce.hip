@@ -1,13 +1,14 @@
 // Projection-fused cut cross-entropy for gfx950: kernels and C ABI.
 //
 // Forward (logits never reach memory):
-//   index    stable list of active rows (weight != 0) -> gather indices
+//   prepare  stable list of active rows (weight != 0) -> gather indices; an aligned copy of a head whose rows are not
 //   stats    persistent GEMM workgroups: logits^T tile = head_tile^T hidden_tile^T,
 //            folded on the fly into per-row running (max, sum exp, target logit)
 //            for one (vocab chunk, row block) unit at a time
-//   merge    combine the vocab chunks per row -> lse, weighted loss, block sums
-//   finalize fixed-order sum of the block sums -> nll_sum, weight_sum
+//   merge    combine the vocab chunks per row -> lse, weighted loss, block sums; the last workgroup adds
+//            those in a fixed order -> nll_sum, weight_sum
 // Backward:
+//   prepare  the same list, the constants of its rows, the active rows packed; the head as above
 //   dlogits  G = w * dy * (exp(logits - lse) - onehot), rounded to bf16, written
 //            vocabulary-major to a workspace slab G^T [vocab slab, rows]
 //   dhidden  dHidden = G head^T
@@ -192,23 +193,14 @@ struct CutceParams {
 // ---------------------------------------------------------------------------
 // index: stable compaction of active rows (and, for the backward, their constants)
 // ---------------------------------------------------------------------------
-// Per-slot constants of the backward: (w dy, lse log2 e, target), zeros / -1 past the active rows.
-struct CutceRowParams {
-  float* fac;
-  float* lse2;
-  int* tgt;
-};
-
-// Workgroup b places the rows 1024 b .. 1024 b + 1023; it counts the active rows in front of them
+// Forward. Workgroup b places the rows 1024 b .. 1024 b + 1023; it counts the active rows in front of them
 // by itself (N floats, from L2 for all but the first reader), so no workgroup waits for another: one
 // pass of latency instead of one per 1024 rows (27 -> 5 us at N = 16384).
-template <bool BACKWARD>
-__global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, const float* lse, const float* dy,
-                                                           CutceRowParams rp) {
+CT_DEVICE void list_rows(const CutceParams& p, int block, int blocks) {
   __shared__ int wave_total[16], wave_first[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int begin = blockIdx.x * 1024, i = begin + tid;
-  const bool last = blockIdx.x == gridDim.x - 1;
+  const int begin = block * 1024, i = begin + tid;
+  const bool last = block == blocks - 1;
   if (last) {
     reset_unit_counters(p.header);
     reset_dlogits_counters(p.header);
@@ -249,32 +241,21 @@ __global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, const 
     slot = before + __popcll(ballot & ((1ull << lane) - 1ull));
     placed = active;
   }
-  if constexpr (!BACKWARD) {
-    const unsigned long long ballot = __ballot(active);
-    __syncthreads();
-    if (lane == 0) wave_first[wave] = ballot != 0;
-    __syncthreads();
-    const int* any = wave_first + (wave & ~3);
-    if (lane == 0 && (wave & 3) == 0 && i < p.n_pad) p.block_active[i / kGemmTile] = p.compact || any[0] || any[1] || any[2] || any[3];
-  }
+  const unsigned long long ballot = __ballot(active);
+  __syncthreads();
+  if (lane == 0) wave_first[wave] = ballot != 0;
+  __syncthreads();
+  const int* any = wave_first + (wave & ~3);
+  if (lane == 0 && (wave & 3) == 0 && i < p.n_pad)
+    p.block_active[i / kGemmTile] = p.compact || any[0] || any[1] || any[2] || any[3];
   if (placed) {
     p.idx[slot] = i;
-    if constexpr (!BACKWARD) p.slot_target[slot] = active ? p.targets[i] : -1;
-    if constexpr (BACKWARD) {
-      rp.fac[slot] = active ? w * dy[0] : 0.f;
-      rp.lse2[slot] = active ? lse[i] * kLog2e : __builtin_inff();
-      rp.tgt[slot] = active ? p.targets[i] : -1;
-    }
+    p.slot_target[slot] = active ? p.targets[i] : -1;
   }
   if (!last) return;
   for (int k = total + tid; k < p.n_pad; k += 1024) {
     p.idx[k] = filler;
-    if constexpr (!BACKWARD) p.slot_target[k] = -1;
-    if constexpr (BACKWARD) {
-      rp.fac[k] = 0.f;
-      rp.lse2[k] = __builtin_inff();
-      rp.tgt[k] = -1;
-    }
+    p.slot_target[k] = -1;
   }
   if (tid == 0) {
     p.header->n_act = total;
@@ -282,35 +263,203 @@ __global__ __launch_bounds__(1024) void cutce_index_kernel(CutceParams p, const 
   }
 }
 
+// Per-slot constants of the backward: (w dy, lse log2 e, target), zeros / -1 past the active rows.
+struct CutceRowParams {
+  float* fac;
+  float* lse2;
+  int* tgt;
+};
+// What the row work of the backward reads and writes beside the list.
+struct CutceRowWork {
+  const float* lse;
+  const float* dy;
+  CutceRowParams rp;
+  bf16* packed;   // [n_pad][d], or null
+  bf16* dhidden;
+};
+
+// Backward. A workgroup of 16 wavefronts places 16 * row_rounds(N) rows and does their row work, a wavefront per
+// row: packed[slot] = hidden[row], and zeros for the dHidden rows of ignored tokens. (The head gradient
+// contracts over slots; with the rows packed its operand tiles are plain strided copies instead of a gather at
+// every step. The slots past the active rows up to the next multiple of 256 hold zeros; their G^T entries
+// are zero or not read.) Every workgroup counts all weights by itself, from L2, and no workgroup waits for
+// another; a wavefront's first row is on its way meanwhile. The list and the row work in two launches took
+// 4.5 + 4.8 us at N = 380, d = 1664, now 5.8, and 9.2 + 40 at N = 16384, d = 4096. One round everywhere makes
+// the counting the longer part (69 us there).
+constexpr int kMostRowRounds = 64;
+__host__ __device__ inline int row_rounds(int rows) { return min((rows + 4095) / 4096, kMostRowRounds); }
+constexpr int kAhead = 8;         // chunks of a row per lane that are read while the weights are counted
+CT_DEVICE void list_and_pack_rows(const CutceParams& p, const CutceRowWork& work, int block, int blocks) {
+  __shared__ int wave_before[16], wave_total[16], wave_first[16], group_count[16], slot_of[16 * kMostRowRounds];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rounds = row_rounds(p.N), rows = 16 * rounds, begin = block * rows, row_chunks = p.d / 8;
+  if (block == 0) {
+    reset_unit_counters(p.header);
+    reset_dlogits_counters(p.header);
+  }
+  const bool ahead = work.packed && p.hidden_aligned;
+  u32x4 chunk[kAhead];
+  const auto row_chunk = [&](int row, int c) {
+    return reinterpret_cast<const u32x4*>(p.hidden + (size_t)min(row, p.N - 1) * p.d)[min(c, row_chunks - 1)];
+  };
+  if (ahead) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(begin + wave, lane + 64 * k);
+  }
+  int before = begin, total = p.N, filler = 0;
+  if (p.compact) {
+    int count_before = 0, count = 0, first = p.N;
+#pragma unroll 4
+    for (int base = 0; base < p.N; base += 1024) {
+      const int i = base + tid;
+      const unsigned long long ballot = __ballot(i < p.N && p.weights[i] != 0.f);
+      const int row0 = base + wave * 64;  // of this wavefront's 64 rows
+      count += __popcll(ballot);
+      const int in_front = min(max(begin - row0, 0), 64);
+      count_before += __popcll(in_front == 64 ? ballot : ballot & ((1ull << in_front) - 1ull));
+      if (ballot) first = min(first, row0 + __ffsll(ballot) - 1);
+    }
+    if (lane == 0) {
+      wave_before[wave] = count_before;
+      wave_total[wave] = count;
+      wave_first[wave] = first;
+    }
+    __syncthreads();
+    before = total = 0;
+    filler = p.N;
+    for (int k = 0; k < 16; ++k) {
+      before += wave_before[k];
+      total += wave_total[k];
+      filler = min(filler, wave_first[k]);
+    }
+    filler = filler < p.N ? filler : 0;  // keeps gathers past the end on a live row
+  }
+  // the list: wavefront g places the g-th 64 rows of the workgroup
+  const int local = wave * 64 + lane, i = begin + local;
+  const bool mine = local < rows && i < p.N;
+  const float w = mine ? p.weights[i] : 0.f;
+  const unsigned long long ballot = __ballot(w != 0.f);
+  if (lane == 0) group_count[wave] = __popcll(ballot);
+  __syncthreads();
+  for (int g = 0; g < wave; ++g) before += p.compact ? group_count[g] : 0;
+  const bool placed = mine && (!p.compact || w != 0.f);
+  const int slot = p.compact ? before + __popcll(ballot & ((1ull << lane) - 1ull)) : i;
+  if (local < rows) slot_of[local] = placed ? slot : -1;
+  if (placed) {
+    p.idx[slot] = i;
+    work.rp.fac[slot] = w != 0.f ? w * work.dy[0] : 0.f;
+    work.rp.lse2[slot] = w != 0.f ? work.lse[i] * kLog2e : __builtin_inff();
+    work.rp.tgt[slot] = w != 0.f ? p.targets[i] : -1;
+  }
+  if (block == 0 && tid == 0) {
+    p.header->n_act = total;
+    p.header->counter = 0;
+  }
+  // the slots past the active rows, shared by the workgroups
+  for (int k = total + block * 1024 + tid; k < p.n_pad; k += blocks * 1024) {
+    p.idx[k] = filler;
+    work.rp.fac[k] = 0.f;
+    work.rp.lse2[k] = __builtin_inff();
+    work.rp.tgt[k] = -1;
+  }
+  __syncthreads();
+  for (int round = 0; round < rounds; ++round) {
+    const int row = begin + 16 * round + wave;
+    if (row >= p.N) break;
+    if (p.weights[row] == 0.f) {
+      u32x4* dst = reinterpret_cast<u32x4*>(work.dhidden + (size_t)row * p.d);
+      for (int c = lane; c < row_chunks; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
+    }
+    const int slot = uniform(slot_of[16 * round + wave]);
+    if (!work.packed || slot < 0) continue;
+    u32x4* dst = reinterpret_cast<u32x4*>(work.packed + (size_t)slot * p.d);
+    if (ahead) {
+      if (round != 0) {
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(row, lane + 64 * k);
+      }
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (lane + 64 * k < row_chunks) dst[lane + 64 * k] = chunk[k];
+#pragma unroll 4
+      for (int c = lane + 64 * kAhead; c < row_chunks; c += 64) dst[c] = row_chunk(row, c);
+    } else {
+      const bf16* from = p.hidden + (size_t)row * p.d;
+      for (int c = lane; c < p.d; c += 64) reinterpret_cast<bf16*>(dst)[c] = from[c];
+    }
+  }
+  if (work.packed) {
+    const int end = (total + kGemmTile - 1) / kGemmTile * kGemmTile;
+    for (int k = total + block * 16 + wave; k < end; k += blocks * 16) {
+      u32x4* dst = reinterpret_cast<u32x4*>(work.packed + (size_t)k * p.d);
+      for (int c = lane; c < p.d / 8; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
-// panel: an aligned, zero-padded copy of `cols` (a multiple of 256) columns of the head
+// The head as the GEMM loop can copy it
 // ---------------------------------------------------------------------------
 // With V % 8 != 0 the rows of the head start at addresses that are multiples of 2 bytes only, and
 // the asynchronous copies of the GEMM loop move aligned 16-byte chunks. One pass over the head
 // (2 bytes read and written per element) makes them usable: the guarded loop that loads such
-// rows element by element runs at 20-90 TFLOP/s against the pipelined one's 600-1300.
-constexpr int kPanelRows = 4;
-__global__ __launch_bounds__(256) void cutce_panel_kernel(const bf16* head, int V, int d, int col0, int cols,
-                                                          bf16* panel, CutceHeader* header) {
-  // (the statistics kernel that follows starts from fresh work counters)
-  if (header && blockIdx.x == 0 && blockIdx.y == 0) reset_unit_counters(header);
-  const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
-  if (c >= cols) return;
-  const int row0 = blockIdx.y * kPanelRows;
-  const int left = V - (col0 + c);
-  const bf16* src = head + (size_t)row0 * V + col0 + c;
-  bf16* dst = panel + (size_t)row0 * cols + c;
-  bf16x8 v[kPanelRows];
-  if (left >= 8) {
+// rows element by element runs at 20-90 TFLOP/s against the pipelined one's 600-1300. The pass needs nothing
+// that the row lists make, so it shares their launch.
+struct HeadCopy {
+  const bf16* head;
+  bf16* panel;  // `cols` (a multiple of 256) columns from col0 on, zero-padded, or null
+  bf16* tail;   // HeadView::tail, or null
+  int col0, cols;
+};
+constexpr int kPanelRows = 4, kPanelColumns = 2048;  // of 256 threads
+__host__ __device__ inline int head_copy_blocks(const HeadCopy& copy, int d) {
+  if (copy.panel) return (copy.cols + kPanelColumns - 1) / kPanelColumns * (d / (4 * kPanelRows));
+  return copy.tail ? (d + 63) / 64 : 0;
+}
+CT_DEVICE void copy_head(const HeadCopy& copy, int V, int d, int block) {
+  const int tid = threadIdx.x;
+  if (copy.panel) {
+    const int col_blocks = (copy.cols + kPanelColumns - 1) / kPanelColumns;
+    const int c = ((block % col_blocks) * 256 + (tid & 255)) * 8, row0 = ((block / col_blocks) * 4 + (tid >> 8)) * kPanelRows;
+    if (c >= copy.cols) return;
+    const int left = V - (copy.col0 + c);
+    const bf16* src = copy.head + (size_t)row0 * V + copy.col0 + c;
+    bf16* dst = copy.panel + (size_t)row0 * copy.cols + c;
+    bf16x8 v[kPanelRows];
+    if (left >= 8) {
 #pragma unroll
-    for (int r = 0; r < kPanelRows; ++r) __builtin_memcpy(&v[r], src + (size_t)r * V, 16);
+      for (int r = 0; r < kPanelRows; ++r) __builtin_memcpy(&v[r], src + (size_t)r * V, 16);
+    } else {
+      for (int r = 0; r < kPanelRows; ++r)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[r][e] = e < left ? src[(size_t)r * V + e] : (bf16)0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < kPanelRows; ++r) store_global16(dst + (size_t)r * copy.cols, as_u32x4(v[r]));
   } else {
-    for (int r = 0; r < kPanelRows; ++r)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[r][e] = e < left ? src[(size_t)r * V + e] : (bf16)0.f;
+    const int row = block * 64 + tid / 16, v = V / 128 * 128 + tid % 16 * 8;
+    if (row >= d) return;
+    u32x4 chunk = {0u, 0u, 0u, 0u};
+    if (v < V) chunk = load_global16(copy.head + (size_t)row * V + v);
+    store_global16(copy.tail + (size_t)row * 128 + tid % 16 * 8, chunk);
   }
-#pragma unroll
-  for (int r = 0; r < kPanelRows; ++r) store_global16(dst + (size_t)r * cols, as_u32x4(v[r]));
+}
+
+// The first list_blocks workgroups make the row list, the others copy the head. A launch that only copies (a
+// further part of the vocabulary) has list_blocks = 0; `reset`: the statistics kernel that follows starts from
+// fresh work counters.
+template <bool BACKWARD>
+__global__ __launch_bounds__(1024) void cutce_prepare_kernel(CutceParams p, CutceRowWork work, HeadCopy copy, int list_blocks,
+                                                             bool reset) {
+  const int block = blockIdx.x;
+  if (block >= list_blocks) {
+    if (reset && block == 0) reset_unit_counters(p.header);
+    copy_head(copy, p.V, p.d, block - list_blocks);
+  } else if constexpr (BACKWARD) {
+    list_and_pack_rows(p, work, block, list_blocks);
+  } else {
+    list_rows(p, block, list_blocks);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -478,9 +627,11 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
 constexpr int kMergeSlots = 32, kMergeParts = 8;
 __global__ __launch_bounds__(kMergeSlots * kMergeParts) void cutce_merge_kernel(CutceParams p, const float* part,
                                                                                 int chunks, float* lse_out,
-                                                                                double* block_sums) {
+                                                                                double* block_sums, float* nll_sum,
+                                                                                float* weight_sum_out) {
   __shared__ float exch[kMergeParts][kMergeSlots][3];
-  __shared__ double red[2][kMergeSlots];
+  __shared__ double red[2][64];
+  __shared__ bool last_s;
   const int tid = threadIdx.x, lane_slot = tid % kMergeSlots, piece = tid / kMergeSlots;
   const int slot = blockIdx.x * kMergeSlots + lane_slot;
   const int n_act = p.header->n_act;
@@ -523,74 +674,39 @@ __global__ __launch_bounds__(kMergeSlots * kMergeParts) void cutce_merge_kernel(
     red[1][lane_slot] = wsum;
   }
   __syncthreads();
-  if (tid == 0) {
-    double loss_sum = 0.0, weight_sum = 0.0;
-    for (int k = 0; k < kMergeSlots; ++k) {  // fixed order
-      loss_sum += red[0][k];
-      weight_sum += red[1][k];
-    }
-    block_sums[2 * blockIdx.x + 0] = loss_sum;
-    block_sums[2 * blockIdx.x + 1] = weight_sum;
+  // The sums of the workgroups are added by the one that ends last, in a fixed order: lane l adds the blocks l,
+  // l + 64, ..., then the lanes are added. They pass through memory by device-scope atomics only, and the answer of
+  // the exchange is what the counter's increment waits for (a fence would write back the L2).
+  const auto bits = reinterpret_cast<unsigned long long*>(block_sums);
+  if (tid < 2) {
+    double sum = 0.0;
+    for (int k = 0; k < kMergeSlots; ++k) sum += red[tid][k];  // fixed order
+    unsigned long long was = __hip_atomic_exchange(bits + 2 * blockIdx.x + tid, __builtin_bit_cast(unsigned long long, sum),
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(was) : : "memory");
+    // (both lanes' exchanges have been answered: they are one instruction of the wavefront)
+    if (tid == 0)
+      last_s = __hip_atomic_fetch_add(&p.header->counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
   }
-}
-
-__global__ __launch_bounds__(64) void cutce_finalize_kernel(const double* block_sums, int blocks,
-                                                            float* nll_sum, float* weight_sum) {
-  // lane l adds the blocks l, l + 64, ... in order, then the lanes are added in order: the
-  // result does not depend on timing
-  __shared__ double red[2][64];
-  double loss = 0.0, wsum = 0.0;
-  for (int b = threadIdx.x; b < blocks; b += 64) {
-    loss += block_sums[2 * b];
-    wsum += block_sums[2 * b + 1];
-  }
-  red[0][threadIdx.x] = loss;
-  red[1][threadIdx.x] = wsum;
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  loss = 0.0;
-  wsum = 0.0;
-  for (int k = 0; k < 64; ++k) {
-    loss += red[0][k];
-    wsum += red[1][k];
-  }
-  *nll_sum = (float)loss;
-  *weight_sum = (float)wsum;
+  if (!last_s || tid >= 64) return;
+  double total[2] = {0.0, 0.0};
+  for (int b = tid; b < (int)gridDim.x; b += 64)
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      total[k] += __builtin_bit_cast(double, __hip_atomic_load(bits + 2 * b + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  red[0][tid] = total[0];
+  red[1][tid] = total[1];
+  __builtin_amdgcn_wave_barrier();
+  if (tid >= 2) return;
+  double sum = 0.0;
+  for (int k = 0; k < 64; ++k) sum += red[tid][k];
+  *(tid ? weight_sum_out : nll_sum) = (float)sum;
 }
 
 // ---------------------------------------------------------------------------
 // backward
 // ---------------------------------------------------------------------------
-// Row work in front of the gradients, one wavefront per row: dHidden rows of ignored tokens are
-// exactly zero, and (packed != nullptr) packed[slot] = hidden[idx[slot]] for the slots of every started
-// 256-slot block. The head gradient contracts over slots; with the rows packed its operand tiles
-// are plain strided copies instead of a gather through idx at every step. (idx repeats the first
-// active row past n_act, so the padding rows hold finite values; their G^T entries are zero.)
-// (tail != nullptr) Also row n < d of HeadView::tail.
-__global__ __launch_bounds__(256) void cutce_rows_kernel(CutceParams p, bf16* packed, bf16* dhidden, bf16* tail) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (tail && row < p.d && lane < 16) {
-    const int v = p.V / 128 * 128 + lane * 8;
-    u32x4 chunk = {0u, 0u, 0u, 0u};
-    if (v < p.V) chunk = load_global16(p.head.base + (size_t)row * p.V + v);
-    store_global16(tail + (size_t)row * 128 + lane * 8, chunk);
-  }
-  if (row < p.N && p.weights[row] == 0.f) {
-    u32x4* dst = reinterpret_cast<u32x4*>(dhidden + (size_t)row * p.d);
-    for (int c = lane; c < p.d / 8; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
-  }
-  const int n_act = p.header->n_act;
-  if (!packed || row >= (n_act + kGemmTile - 1) / kGemmTile * kGemmTile) return;
-  const bf16* src = p.hidden + (size_t)p.idx[row] * p.d;
-  bf16* dst = packed + (size_t)row * p.d;
-  if (p.hidden_aligned) {
-    for (int c = lane; c < p.d / 8; c += 64)
-      reinterpret_cast<u32x4*>(dst)[c] = reinterpret_cast<const u32x4*>(src)[c];
-  } else {
-    for (int c = lane; c < p.d; c += 64) dst[c] = src[c];
-  }
-}
-
 CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
   return fac * (exp2_fast(logit * kLog2e - lse2) - (v == tgt ? 1.f : 0.f));
 }
@@ -1068,10 +1184,11 @@ static int tiles_per_chunk(int tiles, int row_blocks) {
 // (a compute unit's 64 bytes a clock keep up with no more than the small tile's MFMAs); the small one gives
 // short problems four times the workgroups, a quarter of the epilogue per wavefront and, up to one tile per
 // compute unit, half the time per step. Measured (us, large / small; statistics kernel and dlogits kernel):
-// 32 to 64 large tiles 500 x 4000, d = 512: 25 / 12 and 26 / 14, d = 6144: 99 / 48 and 100 / 51; 96 large =
+// 32 large tiles 500 x 4000, d = 512: 25 / 12 and 26 / 14, d = 6144: 99 / 48 and 100 / 51; 96 large =
 // 376 small tiles 1000 x 6000, d = 512: 23 / 16 and 26 / 18, d = 2048: 44 / 36 and 45 / 40; 500 small tiles
-// 250 x 32000, d = 2048: 49 / 52 and 48 / 58; 704, 4000 x 2800: 53 / 62 and 54 / 69.
-constexpr int kMostSmallTiles = 448;
+// 250 x 32000, d = 2048: 49 / 52 and 48 / 58; 414, 380 x 17624, d = 1664: 44 / 45 and 47 / 50; 704, 4000 x 2800:
+// 53 / 62 and 54 / 69.
+constexpr int kMostSmallTiles = 384;
 static int projection_tile(int rows, int tiles) {
   return (long)((rows + 127) / 128) * (2 * tiles) <= kMostSmallTiles ? 128 : kGemmTile;
 }
@@ -1324,14 +1441,18 @@ static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, con
   return p;
 }
 
-// Fills `panel` with the tile columns tile0 .. tile0 + tiles - 1 of the head.
-static int launch_panel(hipStream_t stream, const bf16* head, const ct_cutce_shape& s, int tile0, int tiles, bf16* panel,
-                        CutceHeader* counters_to_reset) {
-  const int cols = tiles * kGemmTile;
-  LaunchScope scope("cutce_panel_kernel", stream);
-  hipLaunchKernelGGL(cutce_panel_kernel, dim3((cols + 2047) / 2048, s.hidden / kPanelRows), dim3(256), 0, stream, head,
-                     s.vocab, s.hidden, tile0 * kGemmTile, cols, panel, counters_to_reset);
+// The row list in `list_blocks` workgroups and a copy of the head (either may be nothing).
+template <bool BACKWARD>
+static int launch_prepare(hipStream_t stream, const CutceParams& p, const CutceRowWork& work, const HeadCopy& copy,
+                          int list_blocks, bool reset) {
+  LaunchScope scope("cutce_prepare_kernel", stream);
+  hipLaunchKernelGGL(cutce_prepare_kernel<BACKWARD>, dim3(list_blocks + head_copy_blocks(copy, p.d)), dim3(1024), 0, stream, p,
+                     work, copy, list_blocks, reset);
   return scope.done();
+}
+// `panel` with the tile columns tile0 .. tile0 + tiles - 1 of the head.
+static HeadCopy panel_copy(const bf16* head, bf16* panel, int tile0, int tiles) {
+  return HeadCopy{head, panel, nullptr, tile0 * kGemmTile, tiles * kGemmTile};
 }
 static HeadView panel_view(const bf16* panel, int tile0, int tiles) {
   return HeadView{panel, nullptr, (long)tiles * kGemmTile, tile0 * kGemmTile, true};
@@ -1409,13 +1530,8 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   double* sums = reinterpret_cast<double*>(ws + L.sums);
   const bf16* head = p.head.base;
 
-  LaunchScope scope1("cutce_index_kernel", stream);
   p.slot_target = reinterpret_cast<int*>(ws + L.target);
   p.block_active = reinterpret_cast<int*>(ws + L.active);
-  hipLaunchKernelGGL(cutce_index_kernel<false>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p, nullptr, nullptr,
-                     CutceRowParams{});
-  if ((rc = scope1.done())) return rc;
-
   const StatsUnits units = stats_units(a->shape);
   // The panel of a head with unaligned rows: at the end of the logits cache, where the backward finds
   // it again, or in what the workspace has behind its fixed part, a number of chunks at a time.
@@ -1434,12 +1550,15 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   const bool guarded = !p.hidden_aligned || (!panel && !(is_aligned16(head) && p.V % 8 == 0));
   for (int chunk0 = 0; chunk0 < units.chunks; chunk0 += chunks_per_pass) {
     const int pass_chunks = min(chunks_per_pass, units.chunks - chunk0);
+    HeadCopy copy = {};
     if (panel) {
       const int tile0 = chunk0 / step_chunks * step_tiles;
       const int pass_tiles = min((pass_chunks + step_chunks - 1) / step_chunks * step_tiles, vocab_tile_count(p.V) - tile0);
-      if ((rc = launch_panel(stream, head, a->shape, tile0, pass_tiles, panel, p.header))) return rc;
+      copy = panel_copy(head, panel, tile0, pass_tiles);
       p.head = panel_view(panel, tile0, pass_tiles);
     }
+    const int list_blocks = chunk0 == 0 ? (p.N + 1023) / 1024 : 0;
+    if ((rc = launch_prepare<false>(stream, p, CutceRowWork{}, copy, list_blocks, list_blocks == 0))) return rc;
     const auto launch = units.tile == kGemmTile ? launch_stats<4> : launch_stats<2>;
     if ((rc = launch(fn, stream, p, guarded, part, chunk0, pass_chunks, units.per_chunk, static_cast<float*>(a->logits_cache))))
       return rc;
@@ -1448,12 +1567,8 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   const int merge_blocks = p.n_pad / kMergeSlots;
   LaunchScope scope3("cutce_merge_kernel", stream);
   hipLaunchKernelGGL(cutce_merge_kernel, dim3(merge_blocks), dim3(kMergeSlots * kMergeParts), 0, stream, p, part,
-                     units.chunks, a->lse, sums);
-  if ((rc = scope3.done())) return rc;
-  LaunchScope scope4("cutce_finalize_kernel", stream);
-  hipLaunchKernelGGL(cutce_finalize_kernel, dim3(1), dim3(64), 0, stream, sums, merge_blocks,
-                     a->nll_sum, a->weight_sum);
-  return scope4.done();
+                     units.chunks, a->lse, sums, a->nll_sum, a->weight_sum);
+  return scope3.done();
 }
 
 extern "C" int32_t ct_cutce_fwd(void* stream, const ct_cutce_fwd_args* a) {
@@ -1544,16 +1659,10 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   rp.fac = reinterpret_cast<float*>(ws + L.rowparams);
   rp.lse2 = reinterpret_cast<float*>(ws + L.rowparams + params_stride);
   rp.tgt = reinterpret_cast<int*>(ws + L.rowparams + 2 * params_stride);
-  LaunchScope scope5("cutce_index_kernel", stream);
-  hipLaunchKernelGGL(cutce_index_kernel<true>, dim3((p.N + 1023) / 1024), dim3(1024), 0, stream, p, a->lse, a->dy, rp);
-  if ((rc = scope5.done())) return rc;
   bf16* packed = dhead ? reinterpret_cast<bf16*>(ws + L.packed) : nullptr;
-  LaunchScope scope6("cutce_rows_kernel", stream);
   const bool head_aligned = is_aligned16(a->head) && p.V % 8 == 0;
   bf16* tail = head_aligned && p.V % 128 ? reinterpret_cast<bf16*>(ws + L.tail) : nullptr;
-  hipLaunchKernelGGL(cutce_rows_kernel, dim3(max(p.n_pad, tail ? p.d : 0) / 4), dim3(256), 0, stream, p, packed, dhidden,
-                     tail);
-  if ((rc = scope6.done())) return rc;
+  const CutceRowWork work = {a->lse, a->dy, rp, packed, dhidden};
 
   const int cus = device_cu_count();
   const int tiles = vocab_tile_count(p.V);
@@ -1575,10 +1684,16 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
     const int slab0 = s * L.slab_cols;
     const int slab_tiles = min(tiles_per_slab, tiles - s * tiles_per_slab);
     const int slab_width = slab_tiles * kGemmTile;
+    HeadCopy copy = {};
     if (panel) {
-      if ((rc = launch_panel(stream, head, a->shape, s * tiles_per_slab, slab_tiles, panel, nullptr))) return rc;
+      copy = panel_copy(head, panel, s * tiles_per_slab, slab_tiles);
       p.head = panel_view(panel, s * tiles_per_slab, slab_tiles);
+    } else if (s == 0) {
+      copy.head = head;
+      copy.tail = tail;
     }
+    const int list_blocks = s == 0 ? (p.N + 16 * row_rounds(p.N) - 1) / (16 * row_rounds(p.N)) : 0;
+    if ((list_blocks || panel) && (rc = launch_prepare<true>(stream, p, work, copy, list_blocks, false))) return rc;
     if (cache) {
       LaunchScope scope11("cutce_dlogits_cached_kernel", stream);
       const long threads = (long)(slab_width / kDlogitsRows) * (p.n_pad / 8);

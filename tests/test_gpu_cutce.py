@@ -464,14 +464,17 @@ def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
 
 @pytest.mark.parametrize("rows,width,vocab", [
     (129, 128, 248),      # both products in 128 x 128 tiles, one column and one row past a tile
-    (1024, 256, 7168),    # 8 x 56 small tiles: the last projection that takes them, gradients in large ones
-    (1025, 256, 6300),    # 9 x 50: the first in large tiles, unaligned rows
+    (50, 4224, 520),      # rows longer than what is read ahead of the list
+    (1024, 256, 6144),    # 8 x 48 small tiles: the last projection that takes them, gradients in large ones
+    (1025, 256, 5500),    # 9 x 44: the first in large tiles, unaligned rows
     (897, 640, 1288),     # gradients in small tiles, the last 8 columns from the tail
     (1025, 1152, 1288),   # small tiles for the projection, large ones for the gradients
+    (4099, 128, 300),     # row lists: two rounds of 16 rows per workgroup, the last one ragged
+    (70001, 128, 130),    # 18 rounds: five wavefronts list rows
 ])
 def test_output_tile_sizes(ct, gpu, rows, width, vocab):
-    """Sizes on both sides of the lines between the 128 x 128 and the 256 x 256 tiles, with and without the logits
-    cache and compaction; dHead is the same for every workspace."""
+    """Sizes on both sides of the lines between the 128 x 128 and the 256 x 256 tiles and between the sizes of the
+    backward's row lists, with and without the logits cache and compaction; dHead is the same for every workspace."""
 
     case = _case(rows + vocab, rows, width, vocab)
     for cache, compaction in ((False, True), (True, True), (False, False)):
