@@ -488,13 +488,38 @@ static int launch_dq(hipStream_t stream, const AttnParams& p) {
   return scope2.done();
 }
 
-template <int D, int HS>
+template <int D, int HS, int KS>
 static int launch_dq_blocks(hipStream_t stream, const AttnParams& p) {
-  const size_t smem = DsStage<D>::kTotalBytes;
-  CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_blocks_kernel<D, HS>), smem);
+  const size_t smem = DsStage<D, KS>::kTotalBytes;
+  CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_blocks_kernel<D, HS, KS>), smem);
+  const int groups = p.Hq / p.Hkv / HS * p.kvh_count;
+  const int grid = KS == 1 ? dq_grid(p, HS) : groups * p.B * bin_tiles_per_row(p.S / 32, kDqbWaves / KS / HS);
   LaunchScope scope("attn_dq_blocks_kernel", stream);
-  hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS>), dim3(dq_grid(p, HS)), dim3(kDqbWaves * 64), smem, stream, p);
+  hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS, KS>), dim3(grid), dim3(kDqbWaves * 64), smem, stream, p);
   return scope.done();
+}
+
+// By the row blocks of the launch (32 query rows of one head). The kernel lives on the bytes it has in flight: in
+// large launches 16 wavefronts per compute unit and work pulling, in small ones the walk of the longest row is the
+// time, two key blocks in flight, and sharing it shortens the walk and puts more of it in flight. Measured
+// (us, one wavefront per row block / two / four), rows with documents of up to the row or images of 1056:
+//   136 row blocks, D = 128: 47 / 24 / 17      432, D = 64: 43 / 23 / 15       608, D = 64: 26 / 14 / 10
+//   1088, D = 64: 43 / 23 / 21 and 22 / 12 / 13, short documents 16 / 7 / 12   1776, D = 128: 44 / 35 / 42
+//   2880, D = 64: 34 / 19 / 29                 8928, D = 64: 248 / 248
+//   3744, D = 128: 124 / 102 / 127, but 2.5 us slower by two with short documents (a compute unit holds one of its
+//   workgroups, of the others two); 7680: 201 / 227
+template <int D>
+static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p) {
+  const long blocks = (long)p.B * p.kvh_count * (p.Hq / p.Hkv) * (p.S / 32);
+  const int hs = heads_per_group(p.Hq, p.Hkv);
+  if (blocks <= 768) return hs == 1 ? launch_dq_blocks<D, 1, 4>(stream, p) : launch_dq_blocks<D, 2, 4>(stream, p);
+  if (blocks <= (D == 64 ? 8192 : 3072))
+    return hs == 4   ? launch_dq_blocks<D, 4, 2>(stream, p)
+           : hs == 2 ? launch_dq_blocks<D, 2, 2>(stream, p)
+                     : launch_dq_blocks<D, 1, 2>(stream, p);
+  return hs == 4   ? launch_dq_blocks<D, 4, 1>(stream, p)
+         : hs == 2 ? launch_dq_blocks<D, 2, 1>(stream, p)
+                   : launch_dq_blocks<D, 1, 1>(stream, p);
 }
 
 // Which dK/dV kernel runs for head dimension 128 when the caller leaves the choice open: the wide
@@ -592,11 +617,7 @@ static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pas
     p.kvh_count = min(kvh_per_pass, p.Hkv - base);
     rc = launch_dkv<D>(stream, p, wide);
     if (rc) return rc;
-    switch (heads_per_group(p.Hq, p.Hkv)) {
-      case 4: rc = launch_dq_blocks<D, 4>(stream, p); break;
-      case 2: rc = launch_dq_blocks<D, 2>(stream, p); break;
-      default: rc = launch_dq_blocks<D, 1>(stream, p); break;
-    }
+    rc = dispatch_dq_blocks<D>(stream, p);
     if (rc) return rc;
   }
   return launch_dkv_reduce<D>(stream, p);

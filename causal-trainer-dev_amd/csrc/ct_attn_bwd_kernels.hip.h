@@ -887,18 +887,27 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
 // reads of one fragment spread over all banks. Three stages: two key blocks are in flight while
 // one is worked on (the kernel lives on bytes in flight; what bounds them is LDS, and with eight
 // wavefronts per K block four fifths of a stage are dS).
+//
+// KS > 1: KS wavefronts share the key blocks of a row block, every KS-th block each (a stage holds the K rows of
+// KS blocks), and add their sums through LDS in a fixed order at the end: for launches of few row blocks, whose
+// time is the walk of the longest row.
 constexpr int kDqbWaves = 8;
-template <int D>
+template <int D, int KS>
 struct DsStage {
   static constexpr int kK = 0;
-  static constexpr int kKBytes = 32 * D * 2;
+  static constexpr int kKBytes = 32 * D * 2;  // of one key block
   static constexpr int kRun = 1024 + 64;
   static constexpr int kPatch = 2 * kRun;
-  static constexpr int kDs = kKBytes;  // [wavefront][kPatch]
-  static constexpr int kBytes = kKBytes + kDqbWaves * kPatch;
+  static constexpr int kDs = KS * kKBytes;  // [wavefront][kPatch]
+  static constexpr int kBytes = kDs + kDqbWaves * kPatch;
   static constexpr int kStages = 3;
-  static constexpr int kTotalBytes =
-      kStages * kBytes > kDqbWaves * 32 * D * 2 ? kStages * kBytes : kDqbWaves * 32 * D * 2;  // >= the store patches
+  static constexpr int kMergeBytes = 64 * (D / 2) * 4;  // the sums that a wavefront hands over
+  static constexpr int kStorePatches = (kDqbWaves - kDqbWaves / KS) * kMergeBytes;
+  static constexpr int kEndBytes = kStorePatches + kDqbWaves / KS * 32 * D * 2;
+  static constexpr int kTotalBytes = kStages * kBytes > kEndBytes ? kStages * kBytes : kEndBytes;
+  // the workgroup's copies of a stage's K rows: by all threads, or by half of them for a small block
+  static constexpr int kCopyThreads = KS * kKBytes >= 8192 ? 512 : 256;
+  typedef TileDma<KS * 32, D / 8, kCopyThreads> KDma;
 };
 
 // Transposed-fragment pointers into a dS block: the B operand of dQ^T += K^T dS^T wants, for
@@ -979,24 +988,25 @@ CT_DEVICE void store_slot_rows_t(const f32x16* acc, float row_scale, lds_addr pa
 }
 
 // s_waitcnt vmcnt(n) for a wave-uniform n that is one of the few values the walk produces.
+template <int MOST>
 CT_DEVICE void wait_all_copies_but(int n) {
-  if (n == 0) __builtin_amdgcn_s_waitcnt(0x0F70);
-  else if (n == 1) __builtin_amdgcn_s_waitcnt(0x0F71);
-  else if (n == 2) __builtin_amdgcn_s_waitcnt(0x0F72);
-  else __builtin_amdgcn_s_waitcnt(0x0F73);
+  if constexpr (MOST == 0) __builtin_amdgcn_s_waitcnt(0x0F70);
+  else if (n >= MOST) __builtin_amdgcn_s_waitcnt(0x0F70 | MOST);
+  else wait_all_copies_but<MOST - 1>(n);
 }
 
-template <int D, int HS>
+template <int D, int HS, int KS>
 CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slice, int qt, const lds_addr lds0,
-                                   const TileDma<32, D / 8, (D == 128 ? 512 : 256)>& kdma,
-                                   const DsFragPtrs& frags, const TrFragOffsets<D / 8, KSlots::kAccum>& tp) {
-  constexpr int PB = kDqbWaves / HS;
-  constexpr int kStage = DsStage<D>::kBytes;
+                                   const typename DsStage<D, KS>::KDma& kdma, const DsFragPtrs& frags,
+                                   const TrFragOffsets<D / 8, KSlots::kAccum>& tp) {
+  using Stage = DsStage<D, KS>;
+  constexpr int kSlots = kDqbWaves / KS, PB = kSlots / HS;
+  constexpr int kStage = Stage::kBytes, kMostCopies = Stage::KDma::kPasses + 2;
   const int nrb = p.S / 32;
   const int g = p.Hq / p.Hkv;
-  const int w = uniform(threadIdx.x >> 6);
-  const int h = kvh * g + slice * HS + (w % HS);
-  int rb = qt * PB + (w / HS);
+  const int w = uniform(threadIdx.x >> 6), slot = w % kSlots, share = w / kSlots;
+  const int h = kvh * g + slice * HS + (slot % HS);
+  int rb = qt * PB + (slot / HS);
   const bool active = rb < nrb;
   if (!active) rb = nrb - 1;
   const int* meta_b = p.meta + (size_t)b * nrb * kMetaW;
@@ -1010,57 +1020,58 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
     first_tile = min(first_tile, uniform(m[kKvFirst]));
     last_tile = max(last_tile, uniform(m[kKvLast]));
   }
-  // the walk is in 32-key blocks (a tile without keys is the pair INT_MAX / -1: converted only
-  // when there is a range, and clamped to the row so that no table entry can lead outside it)
+  // the walk is in steps of KS 32-key blocks (a tile without keys is the pair INT_MAX / -1: converted only
+  // when there is a range, and clamped to the row so that no table entry can lead outside it; rows are whole
+  // numbers of 4 blocks)
   const bool any = first_tile <= last_tile && first_tile >= 0 && last_tile < nrb / 2;
-  const int first = any ? 2 * first_tile : 0;
-  const int last = any ? 2 * last_tile + 1 : -1;
+  const int first = any ? 2 * first_tile / KS : 0;
+  const int last = any ? (2 * last_tile + 1) / KS : -1;
   const char* kbase = reinterpret_cast<const char*>(p.k + ((size_t)b * p.S * p.Hkv + kvh) * D);
   const size_t kv_row_bytes = (size_t)p.Hkv * D * 2;
   const unsigned ds_lane_off = (unsigned)lane_id_here() * 16;
-  const int my_ds = DsStage<D>::kDs + w * DsStage<D>::kPatch;  // this wavefront's block inside a stage
-  // copies of the K rows this wavefront issues per stage (head dimension 64: 256 threads cover the block)
-  const bool copies_k = D == 128 || w < 4;
+  const int my_ds = Stage::kDs + w * Stage::kPatch;  // this wavefront's block inside a stage
+  const bool copies_k = w < Stage::kCopyThreads / 64;
 
   f32x16 dqacc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) dqacc[db] = zero16();
 
-  auto visits = [&](const DsKeyBlockInfo& info, int rbk) {
+  const auto info_of = [&](int t) { return ds_key_block_info(meta_b, t * KS + share); };  // this wavefront's block of step t
+  auto visits = [&](const DsKeyBlockInfo& info, int t) {
     return blocks_interact(mine.min_nz, mine.max_id, mine.end_max, uniform(info.k_min), uniform(info.k_max),
-                           rbk * 32);
+                           (t * KS + share) * 32);
   };
-  // K rows of key block rbk (all wavefronts) and this wavefront's dS block against it; returns the
+  // K rows of step t (all wavefronts) and this wavefront's dS block against its share; returns the
   // number of copy instructions this wavefront issued
-  auto issue = [&](int rbk, const DsKeyBlockInfo& info, lds_addr stage) {
+  auto issue = [&](int t, const DsKeyBlockInfo& info, lds_addr stage) {
     int issued = 0;
     if (copies_k) {
-      kdma.issue(kbase + (size_t)rbk * 32 * kv_row_bytes, stage + DsStage<D>::kK);
-      issued = 1;
+      kdma.issue(kbase + (size_t)t * (KS * 32) * kv_row_bytes, stage + Stage::kK);
+      issued = Stage::KDma::kPasses;
     }
-    if (visits(info, rbk)) {
+    if (visits(info, t)) {
       const char* block = ds_block_address(p, h, b, uniform(info.ds_off), uniform(info.q_first), rb);
       dma16_s(block, ds_lane_off, stage + my_ds);
-      dma16_s(block + 1024, ds_lane_off, stage + (my_ds + DsStage<D>::kRun));
+      dma16_s(block + 1024, ds_lane_off, stage + (my_ds + Stage::kRun));
       issued += 2;
     }
     return issued;
   };
 
-  // info[i]: key block t + i; stage of key block t + i is (stage of t + i) mod 3
+  // cur, next, after: steps t, t + 1, t + 2; the stage of step t + i is (stage of t + i) mod 3
   int t = first;
   DsKeyBlockInfo cur = {}, next = {}, after = {};
-  int pending = 0;  // copy instructions of the youngest key block in flight
+  int pending = 0;  // copy instructions of the youngest step in flight
   if (t <= last) {
-    cur = ds_key_block_info(meta_b, t);
+    cur = info_of(t);
     issue(t, cur, lds0);
     if (t + 1 <= last) {
-      next = ds_key_block_info(meta_b, t + 1);
+      next = info_of(t + 1);
       pending = issue(t + 1, next, lds0 + kStage);
-      if (t + 2 <= last) after = ds_key_block_info(meta_b, t + 2);
+      if (t + 2 <= last) after = info_of(t + 2);
     }
   }
-  wait_all_copies_but(pending);
+  wait_all_copies_but<kMostCopies>(pending);
   __syncthreads();
 
   auto step = [&](auto stage_tag) {
@@ -1070,20 +1081,20 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
     pending = 0;
     if (t + 2 <= last) {
       pending = issue(t + 2, after, lds0 + kFill * kStage);
-      if (t + 3 <= last) later = ds_key_block_info(meta_b, t + 3);
+      if (t + 3 <= last) later = info_of(t + 3);
     }
     if (visits(cur, t)) {
       constexpr int ds_off = CUR * kStage;  // + my_ds, inside the pointers
-      constexpr int k_off = CUR * kStage + DsStage<D>::kK;
+      constexpr int k_off = CUR * kStage + Stage::kK;  // + this wavefront's share, inside the pointers
       const bf16x8 ds0 = frags.load(ds_off, 0), ds1 = frags.load(ds_off, 1);
 #pragma unroll
       for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma32(tp.load(k_off, 0, db), ds0, dqacc[db]);
 #pragma unroll
       for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma32(tp.load(k_off, 1, db), ds1, dqacc[db]);
     }
-    // Copies complete in the order they were issued: all but the ones just issued means key
-    // block t + 1 has landed.
-    wait_all_copies_but(pending);
+    // Copies complete in the order they were issued: all but the ones just issued means step t + 1
+    // has landed.
+    wait_all_copies_but<kMostCopies>(pending);
     __syncthreads();
     cur = next;
     next = after;
@@ -1098,22 +1109,51 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
     step(std::integral_constant<int, 2>{});
   }
 
+  if constexpr (KS > 1) {
+    // (the walk's last barrier is behind every read of the stages)
+    if (share > 0) {
+      const lds_addr sums = lds0 + (w - kSlots) * Stage::kMergeBytes + lane_id_here() * 16;
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd)
+          lds_store<f32x4>(sums + (db * 4 + qd) * 1024,
+                           f32x4{dqacc[db][4 * qd], dqacc[db][4 * qd + 1], dqacc[db][4 * qd + 2], dqacc[db][4 * qd + 3]});
+    }
+    __syncthreads();
+    if (share > 0) return;
+#pragma unroll
+    for (int other = 1; other < KS; ++other) {
+      const lds_addr sums = lds0 + ((other - 1) * kSlots + slot) * Stage::kMergeBytes + lane_id_here() * 16;
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+          const f32x4 o = lds_load<f32x4>(sums + (db * 4 + qd) * 1024);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dqacc[db][4 * qd + e] += o[e];
+        }
+    }
+  }
   if (active) {
-    const lds_addr patch = lds0 + w * 32 * D * 2;
+    const lds_addr patch = lds0 + (Stage::kStorePatches + slot * (32 * D * 2));
     bf16* gbase = p.dq + (((size_t)b * p.S + rb * 32) * p.Hq + h) * D;
     store_slot_rows_t<D>(dqacc, p.scale, patch, gbase, (size_t)p.Hq * D);
   }
-  // the store patches overlap the stages of the next item
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __syncthreads();
+  if constexpr (KS == 1) {
+    // the store patches overlap the stages of the next item
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __syncthreads();
+  }
 }
 
-template <int D, int HS>
+template <int D, int HS, int KS>
 __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
-  constexpr int PB = kDqbWaves / HS;
+  using Stage = DsStage<D, KS>;
+  constexpr int PB = kDqbWaves / KS / HS;
   const int nrb = p.S / 32;
   const int slices = (p.Hq / p.Hkv) / HS;
   const int groups = slices * p.kvh_count;
@@ -1123,10 +1163,15 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
   const int total = p.B * tpr;
   const MetaPtr sched = meta_const(p.sched + query_schedule_offset(nrb, PB));
   const bool dynamic = slices * p.Hkv <= kDqCounters;
-  const TileDma<32, D / 8, (D == 128 ? 512 : 256)> kdma((size_t)p.Hkv * D * 2);
+  const typename Stage::KDma kdma((size_t)p.Hkv * D * 2);
   const int w = threadIdx.x >> 6;
-  const DsFragPtrs frags(lds0 + (DsStage<D>::kDs + w * DsStage<D>::kPatch), lane_id());
-  const TrFragOffsets<D / 8, KSlots::kAccum> tp(lds0);
+  const DsFragPtrs frags(lds0 + (Stage::kDs + w * Stage::kPatch), lane_id());
+  const TrFragOffsets<D / 8, KSlots::kAccum> tp(lds0 + w / (kDqbWaves / KS) * Stage::kKBytes);
+  if constexpr (KS > 1) {  // a workgroup per tile, heaviest first
+    const int b = member % p.B, qt = uniform(sched[(size_t)b * schedule_ints(nrb) + member / p.B]);
+    attn_dq_blocks_item<D, HS, KS>(p, b, kvh, slice, qt, lds0, kdma, frags, tp);
+    return;
+  }
   for (int pull = member;; pull += members) {
     if (dynamic) {
       if (threadIdx.x == 0) next_pull = atomicAdd(&p.dq_counters[slice * p.Hkv + kvh], 1);
@@ -1137,7 +1182,7 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
     if (pull >= total) break;
     const int b = pull % p.B, rank = pull / p.B;
     const int qt = uniform(sched[(size_t)b * schedule_ints(nrb) + rank]);
-    attn_dq_blocks_item<D, HS>(p, b, kvh, slice, qt, lds0, kdma, frags, tp);
+    if constexpr (KS == 1) attn_dq_blocks_item<D, HS, KS>(p, b, kvh, slice, qt, lds0, kdma, frags, tp);
   }
 }
 

@@ -978,3 +978,35 @@ def test_benchmark_shapes(ct, gpu, name, bwd_variant):
         assert ref.relative_l2(dq[b, rows][:, heads], want[2]) <= GRAD_RTOL
         assert ref.relative_l2(dk[b, cols, kvh], want[3]) <= GRAD_RTOL
         assert ref.relative_l2(dv[b, cols, kvh], want[4]) <= GRAD_RTOL
+
+
+@pytest.mark.parametrize("shape", [
+    # batch, seq, Hq, Hkv, D: both sides of the row-block counts (32 query rows of one head) at which the key blocks of
+    # a row are shared by four wavefronts (768), two (3072 for D = 128, 8192 for D = 64) or none, in groups of 1, 2, 4 heads
+    (1, 128, 1, 1, 128), (2, 384, 4, 4, 64), (2, 768, 16, 4, 128), (3, 1024, 8, 4, 64),
+    (1, 896, 28, 28, 128), (2, 1024, 14, 7, 64), (3, 2048, 16, 4, 128), (2, 1920, 68, 17, 64),
+    (1, 2048, 49, 49, 128), (1, 2176, 122, 61, 64), (1, 3200, 84, 21, 64)],
+    ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_forms_of_dq_from_stored_blocks(ct, gpu, shape, with_ends):
+    """dQ from stored dS blocks against the recomputing form in every way of sharing a row's key blocks; rows without
+    keys are zero, and every call gives the same bits."""
+
+    batch, seq, q_heads, kv_heads, dim = shape
+    rng = np.random.default_rng(batch * seq + q_heads)
+    generator = torch.Generator().manual_seed(seq)
+    q, k, v, dout = (torch.randn((batch, seq, heads, dim), generator=generator).to(torch.bfloat16).to(gpu)
+                     for heads in (q_heads, kv_heads, kv_heads, q_heads))
+    ids = _layout(rng, batch, seq, holes=True, max_len=seq)
+    ids[0, :seq - 40] = 1                             # the longest walk, and rows without keys behind it
+    ids[0, seq - 40:] = 0
+    ends = torch.from_numpy(_random_ends(rng, ids, 9)).to(gpu) if with_ends else None
+    profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=with_ends)
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile, attention_end=ends)
+    out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+    expected = ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="recompute")
+    stored = [ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="from_ds") for _ in range(2)]
+    assert all(torch.equal(a, b) for a, b in zip(*stored))
+    assert (stored[0][0][torch.from_numpy(ids).to(gpu) == 0] == 0).all()
+    for a, b in zip(stored[0], expected):
+        assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
