@@ -474,8 +474,11 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   for (int t = tid; t < ntiles; t += 1024) {
     const int items = items_of(t);
     const int ns = dkv_split_count(items, target);
-    const int per = (items + ns - 1) / ns;
-    for (int c = 0; c < ns; ++c) atomicAdd(&hist[bucket_of(max(0, min(per, items - c * per)))], 1);
+    const int per = (items + ns - 1) / ns, full = min(ns, items / max(per, 1));  // chunks of `per` items; then one of
+    const int rest = items - full * per;                                         // the rest, then empty ones
+    if (full > 0) atomicAdd(&hist[bucket_of(per)], full);
+    if (full < ns) atomicAdd(&hist[bucket_of(rest)], 1);
+    if (full + 1 < ns) atomicAdd(&hist[bucket_of(0)], ns - full - 1);
   }
   __syncthreads();
   {
@@ -503,12 +506,15 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
     __syncthreads();
     if (tid == 0) carry += chunk_total;
     if (t < ntiles) {
-      const int per = (items + ns - 1) / ns;
-      for (int c = 0; c < ns; ++c) {
-        const int bk = bucket_of(max(0, min(per, items - c * per)));
-        const int pos = hist[bk] + atomicAdd(&fill[bk], 1);
-        entries[pos] = make_int2(t, c | (ns << 8) | (slot0 << 16));
-      }
+      const int per = (items + ns - 1) / ns, full = min(ns, items / max(per, 1)), rest = items - full * per;
+      const auto place = [&](int begin, int end, int work) {  // chunks begin .. end - 1
+        if (begin >= end) return;
+        const int bk = bucket_of(work), pos = hist[bk] + atomicAdd(&fill[bk], end - begin);
+        for (int c = begin; c < end; ++c) entries[pos + c - begin] = make_int2(t, c | (ns << 8) | (slot0 << 16));
+      };
+      place(0, full, per);
+      place(full, min(full + 1, ns), rest);
+      place(full + 1, ns, 0);
     }
     __syncthreads();
   }
@@ -552,13 +558,15 @@ CT_DEVICE size_t dkv_partial_offset(int slot, int Hkv, int kvh, int wave) {
 // hundred entries). One workgroup per tile and KV head walked up to 32 chunks on a few dozen compute units:
 // [1, 7424, 6/1 heads of 64] 52 -> 12 us, [1, 2432, 16/4 of 64] 25 -> 7, [4, 4096, 32/8 of 128] 22 -> 15,
 // [2, 2432, 16/16 of 128] 19 -> 14, [4, 4224, 8/1 of 128] 25 -> 16.
+// Where there are fewer such pieces than workgroups, the four wavefronts of a workgroup share one, 8 of its rows each,
+// with 16 chunks in flight.
 constexpr int kReduceGroups = 1024;
 template <int D>
 __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
   constexpr int kMaxSplitTiles = kDkvSlots + 8;  // dkv_layout: at most half of max_partials <= 2 (kDkvSlots + 2)
   constexpr int kPieces = 2 * 4 * (D / 32);      // (tensor, wavefront of the dK/dV kernel, 32 columns)
   __shared__ int2 split[kMaxSplitTiles];
-  __shared__ int wave_count[4];
+  __shared__ int wave_count[4][4];
   __shared__ __align__(16) bf16 patches[4][32 * 32];
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
@@ -569,24 +577,37 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
     for (int i = threadIdx.x; i < kDqCounters; i += blockDim.x) p.dq_counters[i] = 0;
   const int entries = uniform(p.dkv_header[0]);
   int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
-  for (int base = 0; base < entries; base += 256) {
-    const int i = base + threadIdx.x;
-    const int2 entry = i < entries ? p.dkv_entries[i] : make_int2(0, 0);
-    const bool mine = (entry.y & 255) == 0 && ((entry.y >> 8) & 255) > 1;  // chunk 0 of several
-    const unsigned long long ballot = __ballot(mine);
-    if (l == 0) wave_count[w] = __popcll(ballot);
-    __syncthreads();
-    int at = tiles + __popcll(ballot & ((1ull << l) - 1ull));
+  for (int base = 0; base < entries; base += 1024) {
+    int2 entry[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k < w) at += wave_count[k];
-      tiles += wave_count[k];
+    for (int n = 0; n < 4; ++n) {
+      const int i = base + n * 256 + threadIdx.x;
+      entry[n] = i < entries ? p.dkv_entries[i] : make_int2(0, 0);
     }
-    if (mine && at < kMaxSplitTiles) split[at] = entry;
+    unsigned long long ballot[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      ballot[n] = __ballot((entry[n].y & 255) == 0 && ((entry[n].y >> 8) & 255) > 1);  // chunk 0 of several
+      if (l == 0) wave_count[n][w] = __popcll(ballot[n]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      if (base + n * 256 >= entries) break;
+      int at = tiles + __popcll(ballot[n] & ((1ull << l) - 1ull));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k < w) at += wave_count[n][k];
+        tiles += wave_count[n][k];
+      }
+      if ((ballot[n] >> l & 1) && at < kMaxSplitTiles) split[at] = entry[n];
+    }
     __syncthreads();
   }
   tiles = uniform(min(tiles, kMaxSplitTiles));
-  for (int item = blockIdx.x * 4 + w; item < tiles * p.Hkv * kPieces; item += gridDim.x * 4) {
+  const int items = tiles * p.Hkv * kPieces;
+  const bool shared = items <= (int)gridDim.x;  // (then a workgroup has one piece at most)
+  for (int item = shared ? blockIdx.x : blockIdx.x * 4 + w; item < items; item += gridDim.x * 4) {
     const int piece = item % kPieces, kvh = item / kPieces % p.Hkv;
     const int2 entry = split[item / kPieces / p.Hkv];
     const int tile = uniform(entry.x), nsplit = uniform((entry.y >> 8) & 255), slot0 = uniform((unsigned)entry.y >> 16);
@@ -594,6 +615,28 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
     const float* src = p.dkv_partials + dkv_partial_offset<D>(slot0, p.Hkv, kvh, keys) + tensor * DkvPartial<D>::kPerTensor +
                        db * 1024 + l * 4;
     const size_t chunk_stride = (size_t)p.Hkv * DkvPartial<D>::kPerChunk;
+    const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
+    bf16* out = (tensor ? p.dv : p.dk) + (((size_t)b * p.S + (kt * 4 + keys) * 32) * p.Hkv + kvh) * D + db * 32;
+    if (shared) {  // keys 8 w .. 8 w + 7 of the piece
+      f32x4 sum = {};
+      for (int c = 0; c < nsplit; c += 16) {
+        f32x4 v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+          v[k] = c + k < nsplit ? *reinterpret_cast<const f32x4*>(src + (c + k) * chunk_stride + w * 256) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+          if (c + k < nsplit) sum += v[k];
+      }
+      bf16* patch = patches[w];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) patch[(4 * half + e) * 32 + j] = (bf16)sum[e];
+      __builtin_amdgcn_wave_barrier();
+      const int row = l >> 2, chunk = (l & 3) * 8;
+      if (row < 8)
+        store_global16(out + (size_t)(8 * w + row) * p.Hkv * D + chunk, *reinterpret_cast<const u32x4*>(patch + row * 32 + chunk));
+      return;
+    }
     f32x4 sum[4] = {};
     for (int c = 0; c < nsplit; c += 4) {
       f32x4 v[4][4];
@@ -616,8 +659,6 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) patch[(8 * q + 4 * half + e) * 32 + j] = (bf16)sum[q][e];
     __builtin_amdgcn_wave_barrier();
-    const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
-    bf16* out = (tensor ? p.dv : p.dk) + (((size_t)b * p.S + (kt * 4 + keys) * 32) * p.Hkv + kvh) * D + db * 32;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const int row = (l >> 2) + 16 * n, chunk = (l & 3) * 8;
