@@ -424,23 +424,23 @@ static int launch_fwd(hipStream_t stream, const AttnParams& p) {
   return scope1.done();
 }
 
-template <int D, int HS, int KS, int KB, int SUB>
+template <int D, int HS, int NW, int KS, int KB, int SUB>
 static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
-  const size_t smem = SplitStage<D, KS, KB, SUB>::kTotalBytes;
-  CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_split_kernel<D, HS, KS, KB, SUB>), smem);
-  const int grid = (p.Hq / HS) * p.B * bin_tiles_per_row(p.S / 32, 4 / KS / HS);
+  const size_t smem = SplitStage<D, NW, KS, KB, SUB>::kTotalBytes;
+  CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_split_kernel<D, HS, NW, KS, KB, SUB>), smem);
+  const int grid = (p.Hq / HS) * p.B * bin_tiles_per_row(p.S / 32, NW / KS / HS);
   LaunchScope scope("attn_fwd_split_kernel", stream);
-  hipLaunchKernelGGL((attn_fwd_split_kernel<D, HS, KS, KB, SUB>), dim3(grid), dim3(256), smem, stream, p);
+  hipLaunchKernelGGL((attn_fwd_split_kernel<D, HS, NW, KS, KB, SUB>), dim3(grid), dim3(NW * 64), smem, stream, p);
   return scope.done();
 }
-template <int D, int KS, int KB, int SUB>
+template <int D, int NW, int KS, int KB, int SUB>
 static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
   const int hs = heads_per_group(p.Hq, p.Hkv);
-  if constexpr (KS == 1)
-    if (hs == 4) return launch_fwd_split<D, 4, KS, KB, SUB>(stream, p);
-  if constexpr (KS <= 2)
-    if (hs >= 2) return launch_fwd_split<D, 2, KS, KB, SUB>(stream, p);
-  return launch_fwd_split<D, 1, KS, KB, SUB>(stream, p);
+  if constexpr (NW / KS >= 4)
+    if (hs == 4) return launch_fwd_split<D, 4, NW, KS, KB, SUB>(stream, p);
+  if constexpr (NW / KS >= 2)
+    if (hs >= 2) return launch_fwd_split<D, 2, NW, KS, KB, SUB>(stream, p);
+  return launch_fwd_split<D, 1, NW, KS, KB, SUB>(stream, p);
 }
 
 // By the row blocks of the launch (32 query rows of one head: one wavefront's work; the device has
@@ -453,16 +453,28 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     at 2048). Above, the large launch's interleaved loop is ahead where rows see 8 key tiles or more
 //     (229 against 242 us), and is behind where they see few (61 against 46 us), which is certain
 //     only for short rows: the line at 20 key tiles per row is where whole-row documents cost 4 %.
+//     Sharing by four takes a compute unit's LDS, so it wins as long as there is a workgroup per compute unit: up to
+//     256 row blocks with one in a workgroup (by two / by four: 33.5 / 22.9 us at 136 with images, 8.9 / 8.5 at 128
+//     short), up to 512 with two (36.9 / 27.6 at 432 with images, 15.1 / 13.6 and, documents up to 300, 12.1 / 11.4 at
+//     512), not for rows that have no chain to share (9.1 / 10.0 at 384 of 384 positions); at 576 with
+//     documents up to 80 it is 9.0 / 15.8.
+//   Calls with visible ends have image blocks, so rows see more: two row blocks by four win there up to 1024 (47.7 /
+//     35.5 at 736, 50.1 / 52.2 at 1104, 52.3 / 48.8 at 1280), at head dimension 64 up to 1280 (31.2 / 25.6 at 736,
+//     38.0 / 30.1 at 1280, 33.1 / 32.9 at 1408); with documents up to 100 they lose (7.8 / 9.9 at 1024).
 template <int D>
 static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   const long blocks = (long)p.B * p.Hq * (p.S / 32);
+  const bool images = p.end != nullptr && p.S >= 2048;
   if constexpr (D == 64) {
-    if (blocks <= 512) return launch_fwd_split<D, 4, 1, 1>(stream, p);
-    if (blocks < 7168) return launch_fwd_split<D, 2, 1, 1>(stream, p);
-    return launch_fwd_split<D, 1, 1, 2>(stream, p);
+    if (blocks <= 512) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
+    if (images && blocks <= 1280) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
+    if (blocks < 7168) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
+    return launch_fwd_split<D, 4, 1, 1, 2>(stream, p);
   } else {
-    if (blocks < 2048) return launch_fwd_split<D, 2, 1, 1>(stream, p);
-    if (p.S <= 20 * kKeyTile) return launch_fwd_split<D, 1, 2, 1>(stream, p);
+    if (blocks <= 256) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
+    if ((blocks <= 512 && p.S > 512) || (images && blocks <= 1024)) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
+    if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
+    if (p.S <= 20 * kKeyTile) return launch_fwd_split<D, 4, 1, 2, 1>(stream, p);
     switch (heads_per_group(p.Hq, p.Hkv)) {
       case 4: return launch_fwd<D, 4>(stream, p);
       case 2: return launch_fwd<D, 2>(stream, p);

@@ -1,16 +1,16 @@
 // Attention forward, several workgroups per compute unit: head dimension 64, and head dimension 128
 // where the launch is small or its rows are short.
 //
-// One workgroup of 4 wavefronts per query tile, launched heaviest tile first and dealt by the
+// One workgroup of NW wavefronts per query tile, launched heaviest tile first and dealt by the
 // hardware. Nothing runs in step across workgroups: what one of them spends on its prologue, its row
 // maxima and its stores is another one's time on the matrix pipe, and no hand-written interleaving is
 // needed. At head dimension 64 the loop is bound by the vector ALU (about 230 instructions and 32
 // exponentials against 16 MFMAs per 64 keys), and 4 wavefronts per SIMD at 103 registers keep it
-// busy; the 8-wavefront workgroup in two half-step-shifted groups that this replaces had 2. Three forms:
+// busy; the 8-wavefront workgroup in two half-step-shifted groups that this replaces had 2. The forms:
 //
 //   KS = 1  a wavefront takes all keys of its 32 query rows
 //   KS = 2  two wavefronts share them, 32 keys each per step: half the chain of steps per row
-//   KS = 4  four share them
+//   KS = 4  four share them; a workgroup has one row block, or with NW = 8 two that share the staged keys
 //
 // For KS > 1 the sums are merged through LDS at the end (in a fixed order). A step stages
 // SUB x KS x KB x 32 keys; a wavefront works on KB x 32 of them at a time, SUB times. 32 at a time
@@ -22,13 +22,15 @@
 //   (2, 4096, 8/8, 64, 4.2)        37.3 -> 20.4  KS = 2     (3, 2944, 24/8, 64, 5.7) 72.7 -> 45.4  KS = 2
 //   (3, 4224, 48/8, 64, 2.3)      121.2 -> 68.9  KS = 1     (8, 4096, 32/8, 64, 32)   796 -> 660   KS = 1
 //   (3, 2560, 8/8, 128, 7.8)       55.3 -> 42.0  KS = 2     (6, 1280, 32/16, 128, 0.4) 61.1 -> 46.2  KS = 1
+// Head dimension 128 by four (KS = 2 -> 4; images of 1056 positions): (1, 2176, 2/2) 33.5 -> 22.9 NW = 4,
+//   (1, 2304, 6/1) 36.9 -> 27.6 and (1, 2944, 8/1) 47.7 -> 35.5 NW = 8.
 #pragma once
 
 #include "ct_attn_kernels.hip.h"
 
 namespace ct {
 
-template <int D, int KS, int KB, int SUB>
+template <int D, int NW, int KS, int KB, int SUB>
 struct SplitStage {
   static constexpr int kKeys = SUB * KS * KB * 32;  // keys per step
   static constexpr int kTileBytes = kKeys * D * 2;
@@ -38,22 +40,22 @@ struct SplitStage {
   static constexpr int kBytes = 2 * kTileBytes + kKeys * 4;
   static constexpr int kTotalBytes = 2 * kBytes;
   static constexpr int kPatchBytes = 32 * D * 2;  // one wavefront's rows, on their way in and out
-  static_assert(4 * kPatchBytes <= kBytes, "the Q rows pass through the second stage");
-  // what a wavefront hands over: O^T and (m, l); two hand over at a time, in front of the store patches
+  static_assert(NW * kPatchBytes <= kBytes, "the Q rows pass through the second stage");
+  // what a wavefront hands over: O^T and (m, l); half of the shares hand over at a time, in front of the store patches
   static constexpr int kMergeBytes = 64 * (D / 2 + 2) * 4;
-  static constexpr int kStorePatches = KS > 1 ? 2 * kMergeBytes : 0;
-  static_assert(kStorePatches + 4 / KS * kPatchBytes <= kTotalBytes, "the merge fits");
+  static constexpr int kStorePatches = NW / KS * (KS / 2) * kMergeBytes;
+  static_assert(kStorePatches + NW / KS * kPatchBytes <= kTotalBytes, "the merge fits");
 };
 
-template <int D, int HS, int KS, int KB, int SUB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : KB == 1 ? 3 : 2))) void
+template <int D, int HS, int NW, int KS, int KB, int SUB>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : KB == 1 ? NW == 4 ? 3 : 2 : 2))) void
 attn_fwd_split_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr lds0 = lds_address_of(smem_raw);
-  using Stage = SplitStage<D, KS, KB, SUB>;
+  using Stage = SplitStage<D, NW, KS, KB, SUB>;
   constexpr bool kSequences = D == 128 && KB == 2;  // the hand-scheduled MFMA sequences
-  constexpr int kSlots = 4 / KS, PB = kSlots / HS;  // row blocks of the workgroup, per head
-  static_assert(PB * HS * KS == 4, "wavefronts = heads x row blocks x key shares");
+  constexpr int kSlots = NW / KS, PB = kSlots / HS;  // row blocks of the workgroup, per head
+  static_assert(PB * HS * KS == NW, "wavefronts = heads x row blocks x key shares");
   const int l = lane_id(), half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int slot = w % kSlots, share = w / kSlots;
   const int nrb = p.S / 32, g = p.Hq / p.Hkv, slices = g / HS, groups = slices * p.Hkv;
@@ -88,7 +90,7 @@ attn_fwd_split_kernel(AttnParams p) {
   int t = any ? first_tile * 64 / Stage::kKeys : 0;
   const int last = any ? (last_tile * 64 + 63) / Stage::kKeys : -1;
 
-  const TileDma<Stage::kKeys, D / 8> dma((size_t)p.Hkv * D * 2);
+  const TileDma<Stage::kKeys, D / 8, NW * 64> dma((size_t)p.Hkv * D * 2);
   const char* kbase = reinterpret_cast<const char*>(p.k + ((size_t)b * p.S * p.Hkv + kvh) * D);
   const char* vbase = reinterpret_cast<const char*>(p.v + ((size_t)b * p.S * p.Hkv + kvh) * D);
   const size_t step_bytes = (size_t)p.Hkv * D * 2 * Stage::kKeys;

@@ -397,6 +397,10 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     (1, 1024, 16, 8, 64), (9, 128, 15, 5, 64), (2, 384, 48, 6, 64), (7, 1024, 30, 5, 64), (7, 1024, 32, 8, 64),
     (8, 1024, 28, 14, 64), (8, 1024, 28, 28, 64), (2, 1024, 30, 10, 128), (1, 1920, 32, 4, 128), (2, 1024, 32, 4, 128),
     (2, 1280, 26, 13, 128), (2, 1280, 26, 26, 128),
+    # keys shared by four at D = 128 (256 and 512 row blocks, rows above 512) and, in calls with ends and rows from 2048
+    # on, in workgroups of two row blocks (1024 for D = 128, 1280 for D = 64)
+    (2, 128, 32, 8, 128), (1, 1152, 8, 4, 128), (2, 1024, 8, 8, 128), (3, 768, 7, 7, 128), (1, 2048, 16, 4, 128),
+    (1, 2176, 16, 2, 128), (2, 2560, 8, 2, 64), (1, 2048, 20, 20, 64), (1, 2688, 16, 16, 64),
     # 12, 2 and 3 workgroup groups: 2, 4 and 8 workgroups walk a work bin of the large form
     (2, 1408, 24, 12, 128), (24, 1408, 2, 2, 128), (16, 1408, 3, 3, 128)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
