@@ -55,8 +55,8 @@ CT_DEVICE void reset_dlogits_counters(CutceHeader* header) {
 
 // Work order of the persistent GEMM kernels. A unit is a pair (a, b) of operand tile indices,
 // a < a_count, b < b_count; every unit is one 256 x 256 GEMM tile (or a run of them) that
-// reads tile a of one operand and tile b of the other. A workgroup asks for its next unit when the
-// GEMM of the last one is done (request), so that the counter's answer travels behind the epilogue.
+// reads tile a of one operand and tile b of the other. A workgroup asks for its next unit ahead (request), so that
+// the counter's answer travels behind an epilogue, or in the projection kernels behind the last GEMM of the unit.
 //
 // Plain order, up to kPlainRounds units per workgroup: the grid is walked with a as the slow index, the
 // first unit of a workgroup is its own number, the others come from one counter. Within a round
@@ -102,7 +102,11 @@ struct UnitQueue {
     requested = started = false;
   }
   CT_DEVICE void request() {
-    if (threadIdx.x == 0) pending = atomicAdd(counters + (order == kPlain ? 0 : (my_xcd + helping) % kXcds), 1);
+    // (an address that is not known to be uniform: for a uniform one the compiler adds once per wavefront and
+    // distributes the answer, for which it waits on the spot)
+    int which = order == kPlain ? 0 : (my_xcd + helping) % kXcds;
+    asm volatile("" : "+v"(which));
+    if (threadIdx.x == 0) pending = atomicAdd(counters + which, 1);
     requested = true;
   }
   // The answer, for all threads of the workgroup (contains barriers).
@@ -484,6 +488,12 @@ struct TileRows {
   CT_DEVICE void advance(int r) { row += (long)stride * ((r & 3) == 3 ? 5 : 1); }
 };
 
+// Bound by the matrix pipe at long contractions; at short ones by what lies between two products, for the large tile
+// has its compute unit to itself. In clocks a tile, 4096 x 32000 at d = 256: product 10.1 k (8.2 k of MFMAs), first
+// copies of the next tile 2.5 k (96 KB at 64 bytes a clock), epilogue 8.5 k, end of a unit 2.4 k; the copies'
+// latency, the cleared accumulators and a second reading of them in the epilogue took 116 us to 104 there, 67 to 65
+// at 900 x 32003, d = 1024, 175 to 162 at 1845 x 67203, d = 512. (Small tiles on two workgroups per compute unit, whose epilogues could
+// fall behind each other's products: 152, 81 and 196, bound by the bytes that reach LDS.)
 template <int NB, bool CACHE, bool GUARDED>
 __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
                                                                     int tiles_per_chunk, float* cache) {
@@ -491,25 +501,45 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr smem = lds_address_of(smem_raw);
   __shared__ int unit_s;
+  __shared__ float exch[2 * kWave * 3];  // [2 wn][kWave rows][3]
   const int tid = threadIdx.x, l = tid & 63, j = l & 31, half = l >> 5, w = tid >> 6;
   const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
   const int vocab_tiles = (p.V + kTile - 1) / kTile;
   const int n_act = p.header->n_act;
 
-  // units: (vocabulary chunk, row block)
+  // units: (vocabulary chunk, row block); row blocks in which no row carries weight are passed over
   const int active_blocks = (n_act + kTile - 1) / kTile;
   UnitQueue units;
   units.init(p.header->xcd_counter[0], chunks, active_blocks, UnitQueue::kSweep);
+  const auto next_unit = [&](int& chunk, int& rb) {
+    while (units.next(chunk, rb, &unit_s))
+      if (p.block_active[rb * kTile / kGemmTile]) return true;
+    return false;
+  };
   int chunk, rb;
-  while (units.next(chunk, rb, &unit_s)) {
-    chunk += chunk0;
-    const int n0 = rb * kTile;
-    if (!p.block_active[n0 / kGemmTile]) continue;  // no row of this block carries weight
-
-    // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
-    // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
-    typedef int LaneInts __attribute__((ext_vector_type(NB)));
-    const LaneInts tgt = *reinterpret_cast<const LaneInts*>(p.slot_target + n0 + wn + NB * j);
+  bool more = next_unit(chunk, rb);
+  McLoader<NB> A;
+  KcLoader<NB> B;
+  GemmTiles<NB, GUARDED, CACHE ? 16 * NB : 0> gemm;
+  // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
+  // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
+  typedef int LaneInts __attribute__((ext_vector_type(NB)));
+  LaneInts next_tgt;
+  // The loaders of a tile and the copies of its first steps. What a new unit loads for its epilogues is waited for
+  // here, where nothing else is in flight: a wait behind the epilogue's stores would be one for them too.
+  const auto begin_tile = [&](int vt, bool new_unit) {
+    if (new_unit) {
+      next_tgt = *reinterpret_cast<const LaneInts*>(p.slot_target + rb * kTile + wn + NB * j);
+      B.init(p.hidden, p.d, p.gather(), rb * kTile, n_act, p.d, true);
+      asm volatile("" : "+v"(next_tgt));
+    }
+    A.init(p.head.base, p.head.ld, vt * kTile - p.head.col0, p.head_cols(vt * kTile), p.d);
+    gemm.begin(A, B, smem);
+  };
+  if (more) begin_tile((chunk0 + chunk) * tiles_per_chunk, true);
+  while (more) {
+    const int n0 = rb * kTile, part_row = chunk0 + chunk;
+    const LaneInts tgt = next_tgt;
     float m2[NB], sum[NB], tl[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -517,18 +547,16 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
       sum[nb] = 0.f;
       tl[nb] = 0.f;
     }
-    KcLoader<NB> B;
-    B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
 
-    const int vt_end = min((chunk + 1) * tiles_per_chunk, vocab_tiles);
-    for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
+    const int vt_end = min((part_row + 1) * tiles_per_chunk, vocab_tiles);
+    for (int vt = part_row * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = vt * kTile;
-      McLoader<NB> A;
-      A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
+      const bool last = vt + 1 == vt_end;
+      if (last) units.request();
       GemmAcc<NB> acc;
-      acc.clear();
-      gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
-      if (vt + 1 == vt_end) units.request();
+      gemm.run(A, B, p.d, smem, acc);
+      if (last) more = next_unit(chunk, rb);
+      if (more) begin_tile(last ? (chunk0 + chunk) * tiles_per_chunk : vt + 1, last);
 
       const int vbase = v0 + wm + 4 * half;  // vocab id of (i, r) = vbase + 32 i + 8 (r/4) + r%4
       const bool ragged = v0 + kTile > p.V;
@@ -547,35 +575,45 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
             rows.advance(r);
           }
       }
-      // (The limit is opaque in each pass over the tile and so is the result of every 16 elements: 64
-      // comparison masks kept for the next pass, or values whose use is put off past a branch, do
-      // not fit and spill, and a reload waits for the stores of the logits cache.)
+      // A column block's 16 NB elements are read once. (The limit is opaque: comparison masks kept for the next
+      // block do not fit and spill, and so is every 16 elements' result, or their use is put off past a branch.)
       const auto fold = [&](auto ragged_tile) {
-        const auto each = [&](int nb, float& result, auto&& f) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          float x[16 * NB];
           int limit = p.V - vbase;
           if (ragged_tile.value) asm volatile("" : "+v"(limit));
+          float tmax = kNegInfF;
 #pragma unroll
           for (int i = 0; i < NB; ++i) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-              const int row = 32 * i + acc_row(r, 0);
-              const float x = acc.value(i, nb, r);
-              f(row, ragged_tile.value && row >= limit ? kNegInfF : x);
+              float& e = x[16 * i + r];
+              e = acc.value(i, nb, r);
+              if (ragged_tile.value && 32 * i + acc_row(r, 0) >= limit) e = kNegInfF;
             }
-            asm volatile("" : "+v"(result));
-          }
-        };
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          float tmax = kNegInfF;
-          each(nb, tmax, [&](int, float x) { tmax = fmaxf(tmax, x); });
+            for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(x[16 * i + r], x[16 * i + r + 1]), tmax);  // (v_max3)
+            asm volatile("" : "+v"(tmax));
+          }
           const int rel = tgt[nb] - (v0 + wm);
-          if (__any(rel >= 0 && rel < kWave))
-            each(nb, tl[nb], [&](int row, float x) { tl[nb] += vbase + row == tgt[nb] ? x : 0.f; });
+          if (__any(rel >= 0 && rel < kWave)) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+#pragma unroll
+              for (int r = 0; r < 16; ++r) tl[nb] += vbase + 32 * i + acc_row(r, 0) == tgt[nb] ? x[16 * i + r] : 0.f;
+              asm volatile("" : "+v"(tl[nb]));
+            }
+          }
           const float m_new = fmaxf(m2[nb], tmax * kLog2e);
           const float m_use = (m_new == kNegInfF) ? 0.f : m_new;
           float add = 0.f;
-          each(nb, add, [&](int, float x) { add += exp2_fast(x * kLog2e - m_use); });
+#pragma unroll
+          for (int i = 0; i < NB; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) add += exp2_fast(x[16 * i + r] * kLog2e - m_use);
+            asm volatile("" : "+v"(add));
+          }
           sum[nb] = sum[nb] * exp2_fast(m2[nb] - m_use) + add;
           m2[nb] = m_new;
         }
@@ -590,7 +628,6 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
       merge_stats(m2[nb], sum[nb], xor32(m2[nb]), xor32(sum[nb]));
       tl[nb] += xor32(tl[nb]);
     }
-    float* exch = reinterpret_cast<float*>(smem_raw);  // [2 wn][kWave rows][3]
     if (wm != 0 && half == 0) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -607,13 +644,13 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
         const float* e = exch + ((w & 1) * kWave + 32 * nb + j) * 3;
         merge_stats(m2[nb], sum[nb], e[0], e[1]);
         tl[nb] += e[2];
-        float* out = part + ((size_t)chunk * p.n_pad + n0 + wn + NB * j + nb) * 3;
+        float* out = part + ((size_t)part_row * p.n_pad + n0 + wn + NB * j + nb) * 3;
         out[0] = m2[nb];
         out[1] = sum[nb];
         out[2] = tl[nb];
       }
     }
-    // the barrier at the top of the loop orders these LDS reads before the next GEMM
+    // (the next unit's GEMM lies between these LDS reads and its writes)
   }
 }
 
@@ -734,37 +771,49 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
   UnitQueue units;
   units.init(p.header->xcd_counter[2], chunks, active_blocks, UnitQueue::kSweep);
   int chunk, rb;
-  while (units.next(chunk, rb, &unit_s)) {
+  bool more = units.next(chunk, rb, &unit_s);
+  McLoader<NB> A;
+  KcLoader<NB> B;
+  GemmTiles<NB, GUARDED, 16 * NB> gemm;
+  // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
+  // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
+  LaneFloats next_fac, next_lse2;
+  LaneInts next_tgt;
+  const auto begin_tile = [&](int vt, bool new_unit) {  // as in the statistics kernel
+    const int v0 = slab0 + vt * kTile;
+    if (new_unit) {
+      const int slot = rb * kTile + wn + NB * j;
+      next_fac = *reinterpret_cast<const LaneFloats*>(rp.fac + slot);
+      next_lse2 = *reinterpret_cast<const LaneFloats*>(rp.lse2 + slot);
+      next_tgt = *reinterpret_cast<const LaneInts*>(rp.tgt + slot);
+      B.init(p.hidden, p.d, p.gather(), rb * kTile, n_act, p.d, true);
+      asm volatile("" : "+v"(next_fac), "+v"(next_lse2), "+v"(next_tgt));
+    }
+    A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
+    gemm.begin(A, B, smem);
+  };
+  if (more) begin_tile(chunk * tiles_per_chunk, true);
+  while (more) {
     const int n0 = rb * kTile;
-    // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
-    // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
-    const int slot = n0 + wn + NB * j;
-    const LaneFloats fac = *reinterpret_cast<const LaneFloats*>(rp.fac + slot);
-    const LaneFloats lse2 = *reinterpret_cast<const LaneFloats*>(rp.lse2 + slot);
-    const LaneInts tgt = *reinterpret_cast<const LaneInts*>(rp.tgt + slot);
-    KcLoader<NB> B;
-    B.init(p.hidden, p.d, p.gather(), n0, n_act, p.d, true);
+    const LaneFloats fac = next_fac, lse2 = next_lse2;
+    const LaneInts tgt = next_tgt;
     const int vt_end = min((chunk + 1) * tiles_per_chunk, slab_tiles);
     for (int vt = chunk * tiles_per_chunk; vt < vt_end; ++vt) {
       const int v0 = slab0 + vt * kTile;
-      McLoader<NB> A;
-      A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
+      const bool last = vt + 1 == vt_end;
+      if (last) units.request();
       GemmAcc<NB> acc;
-      acc.clear();
-      gemm_tile<GUARDED>(A, B, 0, p.d, smem, acc);
-      if (vt + 1 == vt_end) units.request();
+      gemm.run(A, B, p.d, smem, acc);
+      if (last) more = units.next(chunk, rb, &unit_s);
+      if (more) begin_tile(last ? chunk * tiles_per_chunk : vt + 1, last);
 
       bf16* origin = G + (size_t)(v0 - slab0 + uniform(wm)) * p.n_pad + n0 + uniform(wn);
       const unsigned lane_off = (unsigned)(4 * half * p.n_pad + NB * j) * 2u;  // bytes
-      // Most tiles hold no target of the wavefront's rows and lie inside the vocabulary: there the
-      // gradient is factor * softmax, three instructions per element. (Slots without weight have
-      // factor 0 and lse = +inf.)
-      bool target_here = false;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) target_here |= (unsigned)(tgt[nb] - (v0 + wm)) < (unsigned)kWave;
-      const bool plain = v0 + kTile <= p.V && !__any(target_here);
-      TileRows rows(origin, p.n_pad * 2);
-      if (plain) {
+      // factor * softmax, three instructions per element. (Slots without weight have factor 0 and lse = +inf.)
+      const auto store = [&](auto ragged_tile) {
+        TileRows rows(origin, p.n_pad * 2);
+        int limit = p.V - (v0 + wm + 4 * half);
+        if (ragged_tile.value) asm volatile("" : "+v"(limit));
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -772,22 +821,33 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
             LaneFloats x = acc.lane(i, r);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) x[nb] = fac[nb] * exp2_fast(x[nb] * kLog2e - lse2[nb]);
+            if (ragged_tile.value && 32 * i + acc_row(r, 0) >= limit) x = LaneFloats{};
             store_lane(rows.row, lane_off, to_bf16(x));
             rows.advance(r);
           }
-      } else {
+      };
+      if (v0 + kTile > p.V) store(std::true_type{});
+      else store(std::false_type{});
+      // The targets among the wavefront's elements, of which most column blocks have none, are stored a second time:
+      // as a case of every element they cost more than the rest of the epilogue (a tile of 256 x 256 holds one in seven
+      // cases of eight at V = 32000; 4096 rows, d = 256: 155 -> 120 us).
 #pragma unroll
-        for (int i = 0; i < NB; ++i)
+      for (int nb = 0; nb < NB; ++nb) {
+        const int rel = tgt[nb] - (v0 + wm), row = rel - 4 * half;
+        const bool here = (unsigned)rel < (unsigned)kWave && (rel >> 2 & 1) == half;
+        if (!__any(here)) continue;
+        float logit = 0.f;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int v = v0 + wm + 32 * i + acc_row(r, half);
-            LaneFloats x = acc.lane(i, r);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              x[nb] = (fac[nb] != 0.f && v < p.V) ? dlogit(x[nb], fac[nb], lse2[nb], tgt[nb], v) : 0.f;
-            store_lane(rows.row, lane_off, to_bf16(x));
-            rows.advance(r);
+            const float x = acc.value(i, nb, r);
+            logit = row == 32 * i + acc_row(r, 0) ? x : logit;
           }
+          asm volatile("" : "+v"(logit));
+        }
+        if (here && fac[nb] != 0.f)
+          origin[(size_t)rel * p.n_pad + NB * j + nb] = (bf16)(fac[nb] * (exp2_fast(logit * kLog2e - lse2[nb]) - 1.f));
       }
     }
   }
@@ -1184,10 +1244,10 @@ static int tiles_per_chunk(int tiles, int row_blocks) {
 // (a compute unit's 64 bytes a clock keep up with no more than the small tile's MFMAs); the small one gives
 // short problems four times the workgroups, a quarter of the epilogue per wavefront and, up to one tile per
 // compute unit, half the time per step. Measured (us, large / small; statistics kernel and dlogits kernel):
-// 32 large tiles 500 x 4000, d = 512: 25 / 12 and 26 / 14, d = 6144: 99 / 48 and 100 / 51; 96 large =
-// 376 small tiles 1000 x 6000, d = 512: 23 / 16 and 26 / 18, d = 2048: 44 / 36 and 45 / 40; 500 small tiles
-// 250 x 32000, d = 2048: 49 / 52 and 48 / 58; 414, 380 x 17624, d = 1664: 44 / 45 and 47 / 50; 704, 4000 x 2800:
-// 53 / 62 and 54 / 69.
+// 32 large tiles 500 x 4000, d = 512: 19 / 10 and 20 / 11, d = 6144: 98 / 50 and 100 / 51; 96 large =
+// 376 small tiles 1000 x 6000, d = 512: 19 / 17 and 22 / 17, d = 2048: 42 / 40 and 45 / 41; 500 small tiles
+// 250 x 32000, d = 2048: 49 / 56 and 47 / 55; 414, 380 x 17624, d = 1664: 39 / 47 and 41 / 49; 704, 4000 x 2800,
+// d = 1024: 30 / 38 and 34 / 40.
 constexpr int kMostSmallTiles = 384;
 static int projection_tile(int rows, int tiles) {
   return (long)((rows + 127) / 128) * (2 * tiles) <= kMostSmallTiles ? 128 : kGemmTile;

@@ -78,15 +78,21 @@ struct KcLoader {
     base = reinterpret_cast<const char*>(gathered ? base_ : base_ + (size_t)m0 * ld);
     const int r0 = t / CPR;
     chunk = (t % CPR) ^ swizzle<CPR>(r0);  // rows r0 + 64 n share the swizzle
+    int src[NCH];
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
       const int tile_row = r0 + 64 * n;
       constexpr int wave_rows = 32 * NB;
       const int r = interleave_rows ? ((tile_row & wave_rows) | ((tile_row & 31) * NB) | ((tile_row >> 5) % NB)) : tile_row;
       const bool ok = m0 + r < rows_valid;
-      const long src = gathered ? row_index[ok ? m0 + r : 0] : (ok ? r : 0);
-      voff[n] = (unsigned)((src * ld + chunk * 8) * 2);
+      src[n] = gathered ? (ok ? m0 + r : 0) : (ok ? r : 0);
     }
+    if (gathered) {  // (one branch around all of the loads: they travel together)
+#pragma unroll
+      for (int n = 0; n < NCH; ++n) src[n] = row_index[src[n]];
+    }
+#pragma unroll
+    for (int n = 0; n < NCH; ++n) voff[n] = (unsigned)(((long)src[n] * ld + chunk * 8) * 2);
   }
   // copies N0 .. N1-1 of the thread's NCH 16-byte slots
   template <int N0 = 0, int N1 = NCH>
@@ -253,13 +259,16 @@ CT_DEVICE void workgroup_barrier() { __builtin_amdgcn_s_barrier(); }
 
 // The pipelined main loop with a fixed instruction order (see gen_gemm_asm.py), for an
 // m-contiguous A, a k-contiguous B and a step count that is a positive multiple of 4. Entered with the copies of steps 0..2 issued and step 0 landed for every
-// wavefront; returns with nothing in flight and the LDS tiles free.
+// wavefront; returns with nothing in flight and the LDS tiles free. It adds to the accumulators (kAdd) or writes them
+// (kFresh; kFreshBehindStores: at least 51 stores of every wavefront follow the copies of step 2, or these have landed).
+enum class GemmStart { kAdd, kFresh, kFreshBehindStores };
 CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned long long b = (unsigned long long)(uintptr_t)p;
   const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
   const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
   return ((unsigned long long)hi << 32) | (unsigned long long)lo;
 }
+template <GemmStart START>
 CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, int steps,
                                    lds_addr smem, const McLoader<4>::FragOffsets& afo,
                                    const KcLoader<4>::FragOffsets& bfo, int wm, int wn, GemmAcc<4>& acc) {
@@ -273,18 +282,50 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, i
   const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + wave * 1024));
   const int a_off = (wm / 128) * 256;
   const int b_off = GemmShape<4>::kTileBytes + (wn / 32) * KcLoader<4>::FragOffsets::kRowBlockBytes;
-  asm volatile(CT_GEMM_LOOP
-               : "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[0][2]), "+a"(acc.c[0][3]),
-                 "+a"(acc.c[1][0]), "+a"(acc.c[1][1]), "+a"(acc.c[1][2]), "+a"(acc.c[1][3]),
-                 "+a"(acc.c[2][0]), "+a"(acc.c[2][1]), "+a"(acc.c[2][2]), "+a"(acc.c[2][3]),
-                 "+a"(acc.c[3][0]), "+a"(acc.c[3][1]), "+a"(acc.c[3][2]), "+a"(acc.c[3][3])
-               : "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps_u), "s"(lds_wave),
-                 "v"(afo.ptr[0][0] + a_off), "v"(afo.ptr[0][1] + a_off), "v"(afo.ptr[0][2] + a_off),
-                 "v"(afo.ptr[0][3] + a_off), "v"(afo.ptr[1][0] + a_off), "v"(afo.ptr[1][1] + a_off),
-                 "v"(afo.ptr[1][2] + a_off), "v"(afo.ptr[1][3] + a_off), "v"(bfo.ptr[0] + b_off),
-                 "v"(bfo.ptr[1] + b_off), "v"(A.voff[0]), "v"(A.voff[1]), "v"(A.voff[2]),
-                 "v"(A.voff[3]), "v"(B.voff[0]), "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
-               : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
+#define CT_GEMM_ACC(mode) \
+  mode(acc.c[0][0]), mode(acc.c[0][1]), mode(acc.c[0][2]), mode(acc.c[0][3]), mode(acc.c[1][0]), mode(acc.c[1][1]), mode(acc.c[1][2]), mode(acc.c[1][3]), \
+      mode(acc.c[2][0]), mode(acc.c[2][1]), mode(acc.c[2][2]), mode(acc.c[2][3]), mode(acc.c[3][0]), mode(acc.c[3][1]), mode(acc.c[3][2]), mode(acc.c[3][3])
+#define CT_GEMM_IN \
+  "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps_u), "s"(lds_wave), "v"(afo.ptr[0][0] + a_off), \
+      "v"(afo.ptr[0][1] + a_off), "v"(afo.ptr[0][2] + a_off), "v"(afo.ptr[0][3] + a_off), "v"(afo.ptr[1][0] + a_off), \
+      "v"(afo.ptr[1][1] + a_off), "v"(afo.ptr[1][2] + a_off), "v"(afo.ptr[1][3] + a_off), "v"(bfo.ptr[0] + b_off), \
+      "v"(bfo.ptr[1] + b_off), "v"(A.voff[0]), "v"(A.voff[1]), "v"(A.voff[2]), "v"(A.voff[3]), "v"(B.voff[0]), \
+      "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
+  if constexpr (START == GemmStart::kAdd)
+    asm volatile(CT_GEMM_LOOP : CT_GEMM_ACC("+a") : CT_GEMM_IN : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
+  else if constexpr (START == GemmStart::kFresh)
+    asm volatile(CT_GEMM_FRESH_LOOP : CT_GEMM_ACC("=&a") : CT_GEMM_IN : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
+  else
+    asm volatile(CT_GEMM_FRESH_LOOP_BEHIND_STORES : CT_GEMM_ACC("=&a") : CT_GEMM_IN
+                 : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
+#undef CT_GEMM_ACC
+#undef CT_GEMM_IN
+}
+
+// The copies of a tile's first three steps, ahead of gemm_tile_fresh (nothing may be using the LDS stages).
+CT_DEVICE void gemm_copy_ahead(const McLoader<4>& A, const KcLoader<4>& B, lds_addr smem) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    A.dma(i * kGemmBK, smem + i * GemmShape<4>::kStageBytes);
+    B.dma(i * kGemmBK, smem + i * GemmShape<4>::kStageBytes + GemmShape<4>::kTileBytes);
+  }
+}
+
+// acc = A[m-tile, 0:k_end] * B[n-tile, 0:k_end]^T behind gemm_copy_ahead, k_end a positive multiple of 128. STORES:
+// how many stores every wavefront has issued since, 0 or at least 51; `landed`: it waits for all of the copies instead.
+template <int STORES>
+CT_DEVICE void gemm_tile_fresh(const McLoader<4>& A, const KcLoader<4>& B, int k_end, lds_addr smem, GemmAcc<4>& acc, bool landed) {
+  static_assert(STORES == 0 || STORES >= 51, "the waits of the first steps count on it");
+  constexpr GemmStart kStart = STORES ? GemmStart::kFreshBehindStores : GemmStart::kFresh;
+  const int w = threadIdx.x >> 6;
+  const McLoader<4>::FragOffsets afo(smem);
+  const KcLoader<4>::FragOffsets bfo(smem);
+  // step 0's copies: at least 16 + 51 others behind them, or the 16 of steps 1 and 2
+  if (STORES == 0) wait_vmcnt16();
+  else if (landed) dma_wait_all();
+  else asm volatile("s_waitcnt vmcnt(63)" ::: "memory");
+  workgroup_barrier();
+  gemm_loop_scheduled<kStart>(A, B, 0, k_end / kGemmBK, smem, afo, bfo, (w >> 1) * 128, (w & 1) * 128, acc);
 }
 
 // acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T (k_end - k_begin a multiple of 128
@@ -307,7 +348,7 @@ CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end,
     static_assert(McLoader<4>::NCH + KcLoader<4>::NCH == 8, "the wait leaves the copies of two steps in flight");
     wait_vmcnt16();
     workgroup_barrier();
-    gemm_loop_scheduled(A, B, k_begin, (k_end - k_begin) / BK, smem, afo, bfo, wm, wn, acc);
+    gemm_loop_scheduled<GemmStart::kAdd>(A, B, k_begin, (k_end - k_begin) / BK, smem, afo, bfo, wm, wn, acc);
   } else {
     A.fetch(k_begin);
     B.fetch(k_begin);
@@ -407,5 +448,27 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
     acc.settle();
   }
 }
+
+// The tiles of a kernel one after the other: begin() as soon as a tile's loaders are known (the LDS stages are
+// free from the end of the last run() on), run() for its product. In the large tile's pipelined form the copies
+// of its first three steps then travel behind the epilogue of the tile before: with one workgroup on a
+// compute unit nothing else hides them.
+template <int NB, bool GUARDED, int STORES>
+struct GemmTiles {
+  static constexpr bool kAhead = NB == 4 && !GUARDED;
+  bool landed = true;  // the first tile's copies have no stores behind them
+  CT_DEVICE void begin(const McLoader<NB>& A, const KcLoader<NB>& B, lds_addr smem) {
+    if constexpr (kAhead) gemm_copy_ahead(A, B, smem);
+  }
+  CT_DEVICE void run(McLoader<NB>& A, KcLoader<NB>& B, int k_end, lds_addr smem, GemmAcc<NB>& acc) {
+    if constexpr (kAhead) {
+      gemm_tile_fresh<STORES>(A, B, k_end, smem, acc, landed);
+      landed = false;
+    } else {
+      acc.clear();
+      gemm_tile<GUARDED>(A, B, 0, k_end, smem, acc);
+    }
+  }
+};
 
 }  // namespace ct

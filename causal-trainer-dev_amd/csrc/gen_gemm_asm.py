@@ -24,6 +24,13 @@ tile; the body is unrolled over the 4 stages so that every LDS offset is an imme
   source is clamped to the last valid step, which keeps the loop free of branches and the
   vmcnt arithmetic uniform.
 
+CT_GEMM_FRESH_LOOP starts from C = 0 (the first step's first MFMAs take the constant, no accumulator is
+cleared) and its copies of steps 0..2 may be older than an epilogue's stores: vmcnt counts in order, so a
+first iteration of its own waits for no more than the copies it needs. With at least 51 stores behind
+those copies (CT_GEMM_FRESH_LOOP_BEHIND_STORES), vmcnt(63), the largest there is, holds whatever is older
+than the youngest 63: step 1's (8 copies of step 2, the stores, 4 copies of step 3 follow them) and, a step
+later, step 2's; only step 2 waits for the stores, for it needs the copies of step 3 behind them.
+
 Fixed registers (declared as clobbers): v[176:239] fragments, v[240:249] fragment addresses
 + 64 KB, s[40:41] / s[42:43] copy sources of A / B, s44 step counter, s45-s46 temporaries.
 
@@ -64,12 +71,12 @@ def frag_reads(stage, ks):
     return out
 
 
-def mfma(m):
+def mfma(m, from_zero=False):
     ks, r = divmod(m, 16)
     i, j = divmod(r, 4)
     fa, fb = (F0A, F0B) if ks == 0 else (F1A, F1B)
     return "v_mfma_f32_32x32x16_bf16 %s, v[%d:%d], v[%d:%d], %s" % (
-        ACC(i, j), fa + 4 * i, fa + 4 * i + 3, fb + 4 * j, fb + 4 * j + 3, ACC(i, j))
+        ACC(i, j), fa + 4 * i, fa + 4 * i + 3, fb + 4 * j, fb + 4 * j + 3, "0" if from_zero and ks == 0 else ACC(i, j))
 
 
 def copy(operand, n, stage):
@@ -91,7 +98,8 @@ ADVANCE = [
 ]
 
 
-def step(u):
+def step(u, from_zero=False, in_flight=12):
+    """step u % 4 of an iteration; in_flight: how many copies (and stores) may be when step u + 1's have landed"""
     stage, nxt, dst = u, (u + 1) & 3, (u + 3) & 3
     f1 = frag_reads(stage, 1)
     f0n = frag_reads(nxt, 0)
@@ -102,7 +110,7 @@ def step(u):
             behind[m] += f1[key]
     for m, n in {1: 0, 5: 1, 8: 2, 10: 3}.items():
         behind[m] += copy(0, n, dst)
-    behind[12] += ["s_waitcnt vmcnt(12)", "s_waitcnt lgkmcnt(0)", "s_barrier"]
+    behind[12] += ["s_waitcnt vmcnt(%d)" % in_flight, "s_waitcnt lgkmcnt(0)", "s_barrier"]
     # f0 of the next step: a0..a2 are free after MFMA 11, b_j after MFMA 12 + j, a3 after MFMA 15
     for m, keys in {12: ["a0"], 13: ["a1"], 14: ["a2"], 15: ["b0", "b1"], 16: ["b2", "b3"], 17: ["a3"]}.items():
         for key in keys:
@@ -112,22 +120,28 @@ def step(u):
     behind[29] += ADVANCE
     lines = ["s_waitcnt lgkmcnt(0)"]
     for m in range(32):
-        lines.append(mfma(m))
+        lines.append(mfma(m, from_zero))
         lines += behind[m]
     return lines
 
 
-def gemm_loop():
+def gemm_loop(fresh=False, behind_stores=False):
     lines = ["s_mov_b64 s[40:41], " + PTR_A, "s_mov_b64 s[42:43], " + PTR_B, "s_mov_b32 s44, 4"]
     for k in range(10):
         lines.append("v_add_u32 v%d, 0x10000, %%%d" % (HI + k, 21 + k))
     first = frag_reads(0, 0)
     for key in ["a0", "b0", "b1", "b2", "b3", "a1", "a2", "a3"]:
         lines += first[key]
+    if fresh:
+        for u in range(4):
+            lines += step(u, from_zero=u == 0, in_flight=63 if behind_stores and u < 2 else 12)
+        lines += ["s_sub_u32 s45, s44, 4", "s_cmp_lt_u32 s45, " + STEPS, "s_cbranch_scc0 ct_gemm_done_%="]
     lines.append("ct_gemm_loop_%=:")
     for u in range(4):
         lines += step(u)
     lines += ["s_sub_u32 s45, s44, 4", "s_cmp_lt_u32 s45, " + STEPS, "s_cbranch_scc1 ct_gemm_loop_%="]
+    if fresh:
+        lines.append("ct_gemm_done_%=:")
     # drain: nothing in flight, every wavefront done with the LDS tiles, MFMA results readable
     lines += ["s_waitcnt vmcnt(0)", "s_waitcnt lgkmcnt(0)", "s_barrier", "s_nop 15", "s_nop 7"]
     return lines
@@ -221,6 +235,8 @@ def clobbers(first, end):
 if __name__ == "__main__":
     print("// Generated by gen_gemm_asm.py -- do not edit by hand.")
     print(emit(gemm_loop(), "CT_GEMM_LOOP"))
+    print(emit(gemm_loop(fresh=True), "CT_GEMM_FRESH_LOOP"))
+    print(emit(gemm_loop(fresh=True, behind_stores=True), "CT_GEMM_FRESH_LOOP_BEHIND_STORES"))
     print("#define CT_GEMM_LOOP_CLOBBERS %s" % clobbers(F0A, HI + 10))
     print(emit(small_loop(), "CT_GEMM_SMALL_LOOP"))
     print("#define CT_GEMM_SMALL_LOOP_CLOBBERS %s" % clobbers(SMALL_SETS[0], SMALL_SETS[1] + 32))

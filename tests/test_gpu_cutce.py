@@ -488,3 +488,21 @@ def test_output_tile_sizes(ct, gpu, rows, width, vocab):
     slabs = ct.cutce_backward(hidden, head, targets, weights, lse, dy, sparse_compaction=True, workspace_bytes=least)
     assert torch.equal(whole[1], slabs[1])
     assert relative_l2(slabs[0].cpu(), whole[0].cpu()) <= GRAD_RTOL
+
+
+@pytest.mark.parametrize("rows,width,vocab", [
+    (4200, 128, 16380),   # four to five large tiles per workgroup of four steps each, unaligned rows
+    (8500, 128, 20008),   # units of two tiles, the last of one
+    (2100, 640, 16383),   # more steps than a tile's first iteration has
+])
+def test_tiles_one_after_the_other(ct, gpu, rows, width, vocab):
+    """Workgroups that walk several tiles, each of whose first copies travel behind the epilogue of the tile before;
+    the targets crowd the edges of tiles and of the wavefronts' parts of them, several of a wavefront's rows to one."""
+
+    hidden, head, _, weights = _case(rows + vocab, rows, width, vocab)
+    edges = torch.tensor([0, 3, 4, 127, 128, 255, 256, vocab - 257, vocab - 1], dtype=torch.int32)
+    targets = edges[torch.randint(len(edges), (rows,), generator=torch.Generator().manual_seed(rows))]
+    case = (hidden, head, targets, weights)
+    for cache, compaction in ((False, True), (True, True), (False, False)):
+        print("case", rows, width, vocab, cache, compaction, flush=True)
+        _check(_gpu(ct, gpu, *case, 0.37, compaction=compaction, cache=cache), *case, 0.37)
