@@ -1,6 +1,8 @@
 // C ABI of the attention hot path: argument validation and launches.
 #include <atomic>
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "ct_attn_bwd_kernels.hip.h"
 #include "ct_attn_dkv_wide.hip.h"
@@ -30,17 +32,27 @@ CT_DEVICE int lanes_per_item(int n, int threads) {
   while (lanes < 64 && lanes * 2 * n <= threads) lanes *= 2;
   return lanes;
 }
-CT_DEVICE int min_over(int v, int lanes) {
-  for (int off = lanes / 2; off > 0; off /= 2) v = min(v, __shfl_xor(v, off, 64));
+// v over the aligned group of `lanes` lanes (a power of two) that the lane belongs to, for all of them. Up to 16 lanes by
+// lane moves of the vector ALU: a shuffle through LDS costs ten times their latency, and these kernels are nothing else.
+template <class F>
+CT_DEVICE int over_lanes(int v, int lanes, F f) {
+  const auto step = [&](auto control) { v = f(v, __builtin_amdgcn_mov_dpp(v, control.value, 0xf, 0xf, true)); };
+  if (lanes >= 2) step(std::integral_constant<int, 0xb1>{});    // quad_perm 1, 0, 3, 2
+  if (lanes >= 4) step(std::integral_constant<int, 0x4e>{});    // quad_perm 2, 3, 0, 1
+  if (lanes >= 8) step(std::integral_constant<int, 0x141>{});   // the other four of eight, mirrored
+  if (lanes >= 16) step(std::integral_constant<int, 0x140>{});  // the other eight of sixteen
+  if (lanes >= 32) v = f(v, __shfl_xor(v, 16, 64));
+  if (lanes >= 64) v = f(v, __shfl_xor(v, 32, 64));
   return v;
+}
+CT_DEVICE int min_over(int v, int lanes) {
+  return over_lanes(v, lanes, [](int a, int b) { return min(a, b); });
 }
 CT_DEVICE int max_over(int v, int lanes) {
-  for (int off = lanes / 2; off > 0; off /= 2) v = max(v, __shfl_xor(v, off, 64));
-  return v;
+  return over_lanes(v, lanes, [](int a, int b) { return max(a, b); });
 }
 CT_DEVICE int sum_over(int v, int lanes) {
-  for (int off = lanes / 2; off > 0; off /= 2) v += __shfl_xor(v, off, 64);
-  return v;
+  return over_lanes(v, lanes, [](int a, int b) { return a + b; });
 }
 
 // grid (ceil(S / 1024), B): 32 consecutive lanes per block
@@ -152,14 +164,26 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, boo
   }
 }
 
+// The working arrays are in LDS or, for rows beyond 262144 positions and for many tiles, in the metadata buffer's
+// scratch region. In LDS a tile's work and its index are one key, larger for more work and, at the same work, for the lower
+// index (work is below 2^17 there), and a comparison is two instructions. The LDS form
+// is compiled apart: through pointers that may be either, every access waits for the vector memory's counter too.
+template <bool LDS>
+struct TileWork {
+  static constexpr int kIndexBits = 14;
+  static_assert(kPrepareLdsRowBlocks <= 1 << kIndexBits && kBinsLdsInts / 3 <= 1 << kIndexBits, "tiles that the keys tell apart");
+  CT_DEVICE static int pack(int work, int i) { return LDS ? (work << kIndexBits) + (1 << kIndexBits) - 1 - i : work; }
+  CT_DEVICE static int work(int key) { return LDS ? key >> kIndexBits : key; }
+};
 // Number of the tiles in front of tile i when they are ordered by decreasing work, ties by index;
 // shared by `lanes` lanes. Read in 16-byte quads from the first multiple of 16 bytes on: the arrays in LDS start
-// at one, those in the metadata buffer's scratch region (rows beyond 262144 positions, many tiles) anywhere.
+// at one, those in the scratch region anywhere.
+template <bool LDS>
 CT_DEVICE int rank_of(const int* w, int n, int i, int lanes) {
   const int wi = w[i], lane = threadIdx.x % lanes;
-  const int head = min(n, (int)(-(uintptr_t)w / sizeof(int) % 4)), quads = (n - head) / 4;
+  const int head = LDS ? 0 : min(n, (int)(-(uintptr_t)w / sizeof(int) % 4)), quads = (n - head) / 4;
   int rank = 0;
-  auto count = [&](int wv, int k) { rank += (wv > wi) || (wv == wi && k < i); };
+  auto count = [&](int wv, int k) { rank += LDS ? wv > wi : (wv > wi) || (wv == wi && k < i); };
   for (int k = lane; k < head; k += lanes) count(w[k], k);
   for (int q = lane; q < quads; q += lanes) {
     const int4 v = reinterpret_cast<const int4*>(w + head)[q];
@@ -185,15 +209,16 @@ CT_DEVICE int visit_span(const int* mb, int first_block, int end_block, int from
 
 // One of the five schedules of a batch row: query tiles of 1, 2, 4 row blocks, 128-key tiles, query
 // tiles of 8.
+template <bool LDS>
 CT_DEVICE void build_schedule(int job, const int* mb, int nrb, int* sched, int* work) {
   const int pb = job == 3 ? 4 : job == 4 ? 8 : 1 << job, n = job == 4 ? (nrb + 7) / 8 : nrb / pb;
   for (int i = threadIdx.x; i < n; i += 1024)
-    work[i] = visit_span(mb, i * pb, min(nrb, (i + 1) * pb), job == 3 ? kQFirst : kKvFirst);
+    work[i] = TileWork<LDS>::pack(visit_span(mb, i * pb, min(nrb, (i + 1) * pb), job == 3 ? kQFirst : kKvFirst), i);
   __syncthreads();
   const int lanes = lanes_per_item(n, 1024);
   int* out = sched + (job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, pb));
   for (int i = threadIdx.x / lanes; i < n; i += 1024 / lanes) {
-    const int rank = rank_of(work, n, i, lanes);
+    const int rank = rank_of<LDS>(work, n, i, lanes);
     if (threadIdx.x % lanes == 0) out[rank] = i;
   }
 }
@@ -222,16 +247,56 @@ CT_DEVICE void build_ds_offsets(int* mb, int nrb) {
   }
 }
 
+// Lane moves of 32 or 64 bits: the value of the lane that DPP control `CONTROL` names, all ones where it names none or the
+// row of 16 lanes is not in ROWS; lane k's value, as a scalar; the value sent to lane `to`.
+template <int CONTROL, int ROWS>
+CT_DEVICE unsigned moved_lanes(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, CONTROL, ROWS, 0xf, false);
+}
+template <int CONTROL, int ROWS>
+CT_DEVICE unsigned long long moved_lanes(unsigned long long v) {
+  return (unsigned long long)moved_lanes<CONTROL, ROWS>((unsigned)(v >> 32)) << 32 | moved_lanes<CONTROL, ROWS>((unsigned)v);
+}
+// How many of the first 32 lanes hold less. Keys below 2^31: the sign of a difference, of which no scalar register is
+// part (a comparison's mask costs wait states on its way to the sum); lane moves reach the 15 others of a row of 16,
+// and those of the other row once it has changed places.
+template <int ROTATE>
+CT_DEVICE unsigned rotated_below(unsigned other, unsigned v) {
+  return ((unsigned)__builtin_amdgcn_mov_dpp((int)other, 0x120 + ROTATE, 0xf, 0xf, true) - v) >> 31;
+}
+template <int... ROTATE>
+CT_DEVICE int rank_among(unsigned v, std::integer_sequence<int, ROTATE...>) {
+  const unsigned across = (unsigned)__shfl_xor((int)v, 16, 64);
+  return (int)(((across - v) >> 31) + ... + (rotated_below<ROTATE + 1>(v, v) + rotated_below<ROTATE + 1>(across, v)));
+}
+CT_DEVICE int rank_among(unsigned v) { return rank_among(v, std::make_integer_sequence<int, 15>{}); }
+CT_DEVICE int rank_among(unsigned long long v) {
+  int rank = 0;
+  for (int k = 0; k < 32; ++k) {
+    const unsigned low = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, k);
+    const unsigned high = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), k);
+    rank += ((unsigned long long)high << 32 | low) < v;
+  }
+  return rank;
+}
+CT_DEVICE unsigned sent_to(unsigned v, int to) { return (unsigned)__builtin_amdgcn_ds_permute(to * 4, (int)v); }
+CT_DEVICE unsigned long long sent_to(unsigned long long v, int to) {
+  return (unsigned long long)sent_to((unsigned)(v >> 32), to) << 32 | sent_to((unsigned)v, to);
+}
+
 // Packs the query tiles of the whole batch into kBins bins of near equal work
 // (longest processing time first: the heaviest tile left goes to the least loaded bin, ties to the
 // lowest bin), by one workgroup per tile size pb (2, 4, 8 row blocks). lds_bins: 3 ints per tile.
 //
 // The greedy pass is serial, but up to kBins of its steps can be taken together: with the bins ranked
 // by load, the next tiles go to the bins of rank 0, 1, 2, ... until one of those just filled would
-// again be the least loaded. Lane j of one wavefront keeps the load of bin j; a round of up to 32
-// tiles takes about as long as one tile did by a butterfly of 64-bit shuffles (157 -> 20 us for the
-// 256 tiles of four rows of 4096), with the same bins.
+// again be the least loaded. Lane k of one wavefront holds the bin of rank k (its load and number as one key); a round of up
+// to 32 tiles is a chain of some 800 clocks: 32 comparisons for the ranks, one exchange through LDS, a running minimum by lane
+// moves. Nine rounds at four rows of 4096 (256 tiles); with shuffles, unpacked loads and arrays behind generic pointers a
+// round took 2500 and the kernel 15.2 us, now 8.0.
+template <bool LDS>
 CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
+  typedef std::conditional_t<LDS, unsigned, unsigned long long> Key;
   __shared__ int start[kBins + 1];
   const int nrb = S / 32;
   const int tpr = bin_tiles_per_row(nrb, pb), n = B * tpr;
@@ -243,49 +308,52 @@ CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
     const int b = i / tpr, qt = i % tpr;
     const int* mb = meta + (size_t)b * nrb * kMetaW;
     // a tile without keys still costs a launch of the prologue; +3 ~ prologue and store
-    work[i] = visit_span(mb, qt * pb, min(nrb, (qt + 1) * pb), kKvFirst) + 3;
+    work[i] = TileWork<LDS>::pack(visit_span(mb, qt * pb, min(nrb, (qt + 1) * pb), kKvFirst) + 3, i);
   }
   __syncthreads();
   const int lanes = lanes_per_item(n, 1024);
   for (int i = threadIdx.x / lanes; i < n; i += 1024 / lanes) {
-    const int rank = rank_of(work, n, i, lanes);
+    const int rank = rank_of<LDS>(work, n, i, lanes);
     if (threadIdx.x % lanes == 0) {
       order[rank] = i;
-      place[rank] = work[i];
+      place[rank] = TileWork<LDS>::work(work[i]);
     }
   }
   __syncthreads();
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    int load = lane < kBins ? 0 : INT_MAX, count = 0;
+    // of the bin of rank `lane`: load * kBins + bin, and its number of tiles (lanes from kBins on keep out)
+    Key key = lane < kBins ? (Key)lane : ~(Key)0;
+    int count = 0;
     for (int r = 0; r < n;) {
-      // rank of this lane's bin by (load, bin)
-      int rank = lane < kBins ? 0 : lane;
-#pragma unroll
-      for (int j = 0; j < kBins; ++j) {
-        const int other = __builtin_amdgcn_readlane(load, j);
-        if (lane < kBins) rank += other < load || (other == load && j < lane);
-      }
-      const bool offered = lane < kBins && r + rank < n;
-      const int filled = offered ? load + place[r + rank] : INT_MAX;
-      // in rank order: the load of the bin of rank k, and the least load among those filled before it
-      const int by_rank = __builtin_amdgcn_ds_permute(rank * 4, load);
-      int least = __builtin_amdgcn_ds_permute(rank * 4, filled);
-      for (int off = 1; off < kBins; off <<= 1) {
-        const int below = __shfl_up(least, off, 64);
-        if (lane >= off) least = min(least, below);
-      }
-      least = __shfl_up(least, 1, 64);
-      if (lane == 0) least = INT_MAX;
-      const unsigned long long stop = __ballot(lane >= kBins || r + lane >= n || least <= by_rank);
-      const int taken = __ffsll(stop) - 1;  // at least one: least is INT_MAX at rank 0
-      if (lane < kBins && rank < taken) {
-        load = filled;
-        place[r + rank] = count * kBins + lane;
+      const int weight = r + lane < n ? place[r + lane] : 0;
+      const Key filled = key + (Key)weight * kBins;
+      // the least filled bin among those of lower rank
+      Key least = lane < kBins ? filled : ~(Key)0;
+      const auto step = [&](auto control, auto rows) {
+        const Key other = moved_lanes<control.value, rows.value>(least);
+        least = other < least ? other : least;
+      };
+      step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // from 1, 2, 4, 8 lanes below
+      step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+      step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+      step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+      step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // lane 15 to the next sixteen
+      least = moved_lanes<0x138, 0xf>(least);                                          // one lane up
+      const unsigned long long stop = __ballot(lane >= kBins || r + lane >= n || least < key);
+      const int taken = __ffsll(stop) - 1;  // at least one: nothing is below rank 0
+      if (lane < taken) {
+        key = filled;
+        place[r + lane] = count * kBins + (int)(key % kBins);
         ++count;
       }
       r += taken;
+      const int rank = lane < kBins ? rank_among(key) : lane;
+      key = sent_to(key, rank);
+      count = __builtin_amdgcn_ds_permute(rank * 4, count);
     }
+    // back to lane = bin
+    count = __builtin_amdgcn_ds_permute(lane < kBins ? (int)(key % kBins) * 4 : lane * 4, count);
     if (lane < kBins) {
       int incl = count;
       for (int off = 1; off < kBins; off <<= 1) {
@@ -311,7 +379,8 @@ __global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, 
   const int nrb = S / 32;
   if (blockIdx.x < 3) {
     const int pb = 2 << blockIdx.x;
-    build_bins(meta, B, S, pb, bins_scratch ? bins_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2) : lds_work);
+    if (bins_scratch) build_bins<false>(meta, B, S, pb, bins_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2));
+    else build_bins<true>(meta, B, S, pb, lds_work);
     return;
   }
   const int b = (blockIdx.x - 3) / 6, job = (blockIdx.x - 3) % 6;
@@ -320,8 +389,9 @@ __global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, 
     build_ds_offsets(mb, nrb);
   } else {
     const int offset = job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, job == 4 ? 8 : 1 << job);
-    build_schedule(job, mb, nrb, sched_all + (size_t)b * schedule_ints(nrb),
-                   row_scratch ? row_scratch + (size_t)b * 3 * nrb + offset : lds_work);
+    int* sched = sched_all + (size_t)b * schedule_ints(nrb);
+    if (row_scratch) build_schedule<false>(job, mb, nrb, sched, row_scratch + (size_t)b * 3 * nrb + offset);
+    else build_schedule<true>(job, mb, nrb, sched, lds_work);
   }
 }
 

@@ -888,6 +888,38 @@ def test_schedules_are_the_stable_order_by_work(ct, gpu, batch, seq):
         cursor += 33 + spans.size
 
 
+@pytest.mark.parametrize("batch,seq,rate", [(1, 128, 0.01), (2, 1152, 0.02), (4, 4096, 0.002), (3, 8320, 0.0), (1, 262144 + 128, 0.001)])
+def test_work_bins_are_the_greedy_packing(ct, gpu, batch, seq, rate):
+    """Longest tile first onto the least loaded bin, ties to the lowest: fewer tiles than bins, rows of equal and of
+    padded tiles (whose loads tie), many rounds, and arrays in the scratch region (the last shape)."""
+
+    import heapq
+
+    rng = np.random.default_rng(seq)
+    ids = np.cumsum(rng.random((batch, seq)) < rate, axis=1).astype(np.int32) + 1
+    ids[-1, seq // 2:] = 0
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None,
+                                             profile=ct.AttentionKernelProfile(1, 128, 128, 128))
+    blocks = seq // 32
+    flat, bounds = metadata.tile_bounds.cpu().numpy(), ct.tile_bounds_table(metadata).cpu().numpy()
+    cursor = batch * (blocks * 12 + 2 * blocks + blocks // 4)
+    for tile_blocks in (2, 4, 8):
+        tiles = (blocks + tile_blocks - 1) // tile_blocks
+        first, last = np.full((batch, tiles * tile_blocks), 2 ** 31 - 1), np.full((batch, tiles * tile_blocks), -1)
+        first[:, :blocks], last[:, :blocks] = bounds[..., 5], bounds[..., 6]
+        first, last = first.reshape(batch, tiles, -1).min(2), last.reshape(batch, tiles, -1).max(2)
+        work = (np.where(last >= first, last - first + 1, 0) + 3).reshape(-1)
+        bins, heap = [[] for _ in range(32)], [(0, k) for k in range(32)]
+        for item in np.argsort(-work, kind="stable"):
+            load, k = heapq.heappop(heap)
+            bins[k].append(item)
+            heapq.heappush(heap, (load + work[item], k))
+        offsets, items = flat[cursor:cursor + 33], flat[cursor + 33:cursor + 33 + work.size]
+        np.testing.assert_array_equal(offsets, np.cumsum([0] + [len(b) for b in bins]))
+        np.testing.assert_array_equal(items, np.concatenate([np.array(b, np.int64) for b in bins]))
+        cursor += 33 + work.size
+
+
 def _longest_segment(ids):
     """(batch row, start, stop) of the longest run of one nonzero id."""
 

@@ -41,6 +41,25 @@ def test_canonical_ids_match_oracle(ct, gpu, batch, seq):
         np.testing.assert_array_equal(_canon(ct, gpu, mask), attention_ref.canonicalize_segment_ids(mask))
 
 
+@pytest.mark.parametrize("batch,seq,offset", [(2, 4, 0), (3, 260, 0), (3, 260, 1), (2, 4100, 2), (2, 4099, 0), (1, 8192, 3)])
+def test_segment_scans_at_any_alignment(ct, gpu, batch, seq, offset):
+    """Rows that are moved in 16-byte quads and rows that are not: a view at any element, a length that is no multiple of 4."""
+
+    from oracle import layer_ref
+
+    rng = np.random.default_rng(seq + offset)
+    mask = (rng.random((batch, seq)) < 0.9).astype(np.int32)
+    labels = np.repeat(rng.integers(0, 3, (batch, seq // 3 + 1)), 3, axis=1)[:, :seq].astype(np.int32)
+
+    def view(values):
+        return torch.from_numpy(np.concatenate([np.full(offset, 7, np.int32), values.reshape(-1)])).to(gpu)[offset:].view(batch, seq)
+
+    np.testing.assert_array_equal(ct.canonicalize_segment_ids(view(mask), view(labels)).cpu().numpy(),
+                                  attention_ref.canonicalize_segment_ids(mask, labels))
+    np.testing.assert_array_equal(ct.make_position_ids(view(mask), view(labels)).cpu().numpy(),
+                                  layer_ref.make_position_ids(mask, labels))
+
+
 def _shifted(ct, gpu, ids, mask, segments=None, assistant=None, loss=None, labels=None, ignore_index=-100):
     def dev(x, dtype=None):
         if x is None:
