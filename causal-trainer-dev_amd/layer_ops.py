@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .prep import _dense, _int32, _mask_and_labels
+from .prep import _dense, _int32, _mask_and_labels, _plain
 
 _STYLES = {"gpt-j": 0, "gpt-neox": 1}
 
@@ -21,6 +21,9 @@ _STYLES = {"gpt-j": 0, "gpt-neox": 1}
 def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
     """Zero-based positions that reset at every packed segment (int32 ``[batch, sequence]``)."""
 
+    plain = _plain("segment_positions", attention_mask, segment_ids)
+    if plain is not None:
+        return plain
     mask = torch.as_tensor(attention_mask)
     if mask.ndim != 2:
         raise ValueError(f"attention_mask must have shape [batch, sequence], got {tuple(mask.shape)}")
@@ -33,6 +36,9 @@ def make_position_ids(attention_mask, segment_ids=None) -> torch.Tensor:
 def rotary_cos_sin(position_ids, inv_freq, dtype=torch.bfloat16):
     """Per-token cos / sin tables ``[batch, sequence, rotary_dim / 2]`` (f32 angles, one cast)."""
 
+    plain = _plain("rotary_tables", position_ids, inv_freq) if dtype == torch.bfloat16 else None
+    if plain is not None:
+        return plain
     positions = torch.as_tensor(position_ids)
     if positions.ndim != 2:
         raise ValueError(f"position_ids must have shape [batch, sequence], got {tuple(positions.shape)}")
