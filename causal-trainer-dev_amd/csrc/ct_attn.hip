@@ -17,7 +17,7 @@
 namespace ct {
 
 // ---------------------------------------------------------------------------
-// Tile bounds, in three launches: the summary of every 32-position block; from a row's summaries, what
+// Tile bounds, in three launches, two for short rows: the summary of every 32-position block; from a row's summaries, what
 // each block has to visit; from those ranges, the work-sorted schedules, the dS offsets and the bins.
 //
 // All of it is latency: the searches and the ranking are quadratic in a row's blocks, and one
@@ -55,26 +55,37 @@ CT_DEVICE int sum_over(int v, int lanes) {
   return over_lanes(v, lanes, [](int a, int b) { return a + b; });
 }
 
-// grid (ceil(S / 1024), B): 32 consecutive lanes per block
-__global__ __launch_bounds__(1024) void attn_blocks_kernel(const int* seg, const int* end, int S, int* meta) {
-  const int b = blockIdx.y, pos = blockIdx.x * 1024 + threadIdx.x;
-  if (pos >= S) return;  // (S % 128 == 0: whole wavefronts)
-  const int id = seg[(size_t)b * S + pos], e = end ? end[(size_t)b * S + pos] : pos;
-  const bool counts = id != 0;
-  const int low = min_over(counts ? id : INT_MAX, 32), high = max_over(counts ? id : INT_MIN, 32);
-  const int end_min = min_over(counts ? e : INT_MAX, 32), end_max = max_over(counts ? e : -1, 32);
-  const int zeros = 32 - __popcll(__ballot(counts) >> (threadIdx.x & 32) & 0xffffffffull);
-  if (pos % 32 == 0) {
-    const int max_id = max(high, 0);
-    int* m = meta + ((size_t)b * (S / 32) + pos / 32) * kMetaW;
-    m[kMinNz] = max_id == 0 ? 0 : low;  // reference: all-padding block -> (0, 0)
+// What a block's record says of its ids and visible ends; 32 consecutive lanes per block, all of them get it.
+struct BlockIds {
+  int min_nz, max_id, uniform, end_min, end_max;
+  CT_DEVICE BlockIds(const int* seg, const int* end, size_t row, int pos) {
+    const int id = seg[row + pos], e = end ? end[row + pos] : pos;
+    const bool counts = id != 0;
+    const int low = min_over(counts ? id : INT_MAX, 32), high = max_over(counts ? id : INT_MIN, 32);
+    end_min = min_over(counts ? e : INT_MAX, 32);
+    end_max = max_over(counts ? e : -1, 32);
+    const int zeros = 32 - __popcll(__ballot(counts) >> (threadIdx.x & 32) & 0xffffffffull);
+    max_id = max(high, 0);
+    min_nz = max_id == 0 ? 0 : low;  // reference: all-padding block -> (0, 0)
+    uniform = zeros == 0 && low == high ? low : 0;
+  }
+  CT_DEVICE void store(int* m) const {
+    m[kMinNz] = min_nz;
     m[kMaxId] = max_id;
-    m[kUniform] = zeros == 0 && low == high ? low : 0;
+    m[kUniform] = uniform;
     m[kEndMin] = end_min;
     m[kEndMax] = end_max;
     m[10] = 0;
     m[11] = 0;
   }
+};
+
+// grid (ceil(S / 1024), B)
+__global__ __launch_bounds__(1024) void attn_blocks_kernel(const int* seg, const int* end, int S, int* meta) {
+  const int b = blockIdx.y, pos = blockIdx.x * 1024 + threadIdx.x;
+  if (pos >= S) return;  // (S % 128 == 0: whole wavefronts)
+  const BlockIds block(seg, end, (size_t)b * S, pos);
+  if (pos % 32 == 0) block.store(meta + ((size_t)b * (S / 32) + pos / 32) * kMetaW);
 }
 
 // Block summaries in the reference's format (ct_attn_block_summary); `block` = 0: none.
@@ -84,13 +95,28 @@ struct SummaryOut {
 };
 
 // grid (ceil(nrb / 64), B): 16 lanes per block search what it has to visit; the workgroups of a row also
-// write its block summaries.
+// write its block summaries. With `seg` every workgroup forms the records of its whole row by itself and stores its
+// own: a launch and its latency less than with attn_blocks_kernel in front, for rows of up to kFusedRows positions
+// (8 loads per thread). Both sides, us: [4, 4096] 4.2 + 5.2 / 7.0, [8, 8192] 4.2 + 8.1 / 11.6, [4, 16384] 4.3 + 13.8 / 20.1,
+// [1, 32768] 4.2 + 25.1 / 36.2.
+constexpr int kFusedRows = 8192;
 __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, bool in_lds, SummaryOut queries,
-                                                           SummaryOut keys) {
+                                                           SummaryOut keys, const int* seg, const int* end) {
   extern __shared__ __align__(16) int lds_rows[];  // [3][nrb]: min_nz, max_id, end_max of the row's blocks
   const int b = blockIdx.y, nrb = S / 32, nt = S / kKeyTile;
   int* mb = meta + (size_t)b * nrb * kMetaW;
-  if (in_lds) {
+  if (seg) {
+    for (int pos = threadIdx.x; pos < S; pos += 1024) {  // (S % 128 == 0: whole wavefronts)
+      const BlockIds block(seg, end, (size_t)b * S, pos);
+      const int i = pos / 32;
+      if (pos % 32) continue;
+      lds_rows[i] = block.min_nz;
+      lds_rows[nrb + i] = block.max_id;
+      lds_rows[2 * nrb + i] = block.end_max;
+      if (i / 64 == (int)blockIdx.x) block.store(mb + i * kMetaW);
+    }
+    __syncthreads();
+  } else if (in_lds) {
     for (int i = threadIdx.x; i < nrb; i += 1024) {
       lds_rows[i] = mb[i * kMetaW + kMinNz];
       lds_rows[nrb + i] = mb[i * kMetaW + kMaxId];
@@ -733,6 +759,8 @@ extern "C" size_t ct_attn_bwd_workspace_bytes_from_ds(int32_t batch, int32_t seq
   return plan.spill ? plan.total : 0;
 }
 
+static_assert(kFusedRows / 32 <= kPrepareLdsRowBlocks, "the fused form keeps the row's records in LDS");
+
 static int32_t prepare_on(const char* fn, void* stream, const int32_t* segment_ids, const int32_t* attention_end,
                           int32_t batch, int32_t seq, int32_t* tile_meta, SummaryOut queries, SummaryOut keys) {
   CT_REQUIRE(segment_ids && tile_meta, "%s: null pointer", fn);
@@ -748,15 +776,18 @@ static int32_t prepare_on(const char* fn, void* stream, const int32_t* segment_i
   }
   int* bins_scratch = bins_fit_lds(batch, nrb) ? nullptr : scratch;
   hipStream_t st = (hipStream_t)stream;
-  LaunchScope scope5("attn_blocks_kernel", st);
-  hipLaunchKernelGGL(attn_blocks_kernel, dim3((seq + 1023) / 1024, batch), dim3(1024), 0, st, segment_ids, attention_end, seq,
-                     tile_meta);
-  if ((rc = scope5.done())) return rc;
+  const bool fused = seq <= kFusedRows;
+  if (!fused) {
+    LaunchScope scope5("attn_blocks_kernel", st);
+    hipLaunchKernelGGL(attn_blocks_kernel, dim3((seq + 1023) / 1024, batch), dim3(1024), 0, st, segment_ids, attention_end, seq,
+                       tile_meta);
+    if ((rc = scope5.done())) return rc;
+  }
   CT_ENSURE_LDS(fn, &attn_ranges_kernel, kPrepareLdsRowBlocks * 3 * 4);
   LaunchScope scope6("attn_ranges_kernel", st);
   hipLaunchKernelGGL(attn_ranges_kernel, dim3((nrb + 63) / 64, batch), dim3(1024),
                      prepare_scratch ? 0 : (size_t)nrb * 3 * sizeof(int), st, tile_meta, seq, prepare_scratch == nullptr,
-                     queries, keys);
+                     queries, keys, fused ? segment_ids : nullptr, attention_end);
   if ((rc = scope6.done())) return rc;
   const size_t bins_smem = bins_scratch ? 0 : (size_t)3 * batch * bin_tiles_per_row(nrb, 2) * sizeof(int);
   const size_t row_smem = prepare_scratch ? 0 : (size_t)nrb * sizeof(int);
