@@ -97,15 +97,18 @@ struct SummaryOut {
 // grid (ceil(nrb / 64), B): 16 lanes per block search what it has to visit; the workgroups of a row also
 // write its block summaries. With `seg` every workgroup forms the records of its whole row by itself and stores its
 // own: a launch and its latency less than with attn_blocks_kernel in front, for rows of up to kFusedRows positions
-// (8 loads per thread). Both sides, us: [4, 4096] 4.2 + 5.2 / 7.0, [8, 8192] 4.2 + 8.1 / 11.6, [4, 16384] 4.3 + 13.8 / 20.1,
-// [1, 32768] 4.2 + 25.1 / 36.2.
+// (8 loads per thread). Both sides, us: [4, 4096] 4.1 + 4.2 / 5.5, [8, 8192] 4.3 + 5.1 / 8.5, [4, 16384] 4.3 + 8.2 / 14.6,
+// [1, 32768] 4.1 + 14.0 / 25.1.
 constexpr int kFusedRows = 8192;
-__global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, bool in_lds, SummaryOut queries,
-                                                           SummaryOut keys, const int* seg, const int* end) {
+// LDS is compiled apart: one pointer to either kind of memory makes every access a flat one ([4, 16384] 13.8 -> 8.2 us,
+// [1, 32768] 25.1 -> 14.0).
+template <bool LDS>
+__global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, SummaryOut queries, SummaryOut keys,
+                                                           const int* seg, const int* end) {
   extern __shared__ __align__(16) int lds_rows[];  // [3][nrb]: min_nz, max_id, end_max of the row's blocks
   const int b = blockIdx.y, nrb = S / 32, nt = S / kKeyTile;
   int* mb = meta + (size_t)b * nrb * kMetaW;
-  if (seg) {
+  if (LDS && seg) {
     for (int pos = threadIdx.x; pos < S; pos += 1024) {  // (S % 128 == 0: whole wavefronts)
       const BlockIds block(seg, end, (size_t)b * S, pos);
       const int i = pos / 32;
@@ -116,7 +119,7 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, boo
       if (i / 64 == (int)blockIdx.x) block.store(mb + i * kMetaW);
     }
     __syncthreads();
-  } else if (in_lds) {
+  } else if (LDS) {
     for (int i = threadIdx.x; i < nrb; i += 1024) {
       lds_rows[i] = mb[i * kMetaW + kMinNz];
       lds_rows[nrb + i] = mb[i * kMetaW + kMaxId];
@@ -124,9 +127,9 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, boo
     }
     __syncthreads();
   }
-  auto min_nz = [&](int i) { return in_lds ? lds_rows[i] : mb[i * kMetaW + kMinNz]; };
-  auto max_id = [&](int i) { return in_lds ? lds_rows[nrb + i] : mb[i * kMetaW + kMaxId]; };
-  auto end_max = [&](int i) { return in_lds ? lds_rows[2 * nrb + i] : mb[i * kMetaW + kEndMax]; };
+  auto min_nz = [&](int i) { return LDS ? lds_rows[i] : mb[i * kMetaW + kMinNz]; };
+  auto max_id = [&](int i) { return LDS ? lds_rows[nrb + i] : mb[i * kMetaW + kMaxId]; };
+  auto end_max = [&](int i) { return LDS ? lds_rows[2 * nrb + i] : mb[i * kMetaW + kEndMax]; };
 
   constexpr int kLanes = 16;
   const int lane = threadIdx.x % kLanes, rb = blockIdx.x * (1024 / kLanes) + threadIdx.x / kLanes;
@@ -783,11 +786,10 @@ static int32_t prepare_on(const char* fn, void* stream, const int32_t* segment_i
                        tile_meta);
     if ((rc = scope5.done())) return rc;
   }
-  CT_ENSURE_LDS(fn, &attn_ranges_kernel, kPrepareLdsRowBlocks * 3 * 4);
+  CT_ENSURE_LDS(fn, &attn_ranges_kernel<true>, kPrepareLdsRowBlocks * 3 * 4);
   LaunchScope scope6("attn_ranges_kernel", st);
-  hipLaunchKernelGGL(attn_ranges_kernel, dim3((nrb + 63) / 64, batch), dim3(1024),
-                     prepare_scratch ? 0 : (size_t)nrb * 3 * sizeof(int), st, tile_meta, seq, prepare_scratch == nullptr,
-                     queries, keys, fused ? segment_ids : nullptr, attention_end);
+  hipLaunchKernelGGL((prepare_scratch ? attn_ranges_kernel<false> : attn_ranges_kernel<true>), dim3((nrb + 63) / 64, batch),
+                     dim3(1024), prepare_scratch ? 0 : (size_t)nrb * 3 * sizeof(int), st, tile_meta, seq, queries, keys, fused ? segment_ids : nullptr, attention_end);
   if ((rc = scope6.done())) return rc;
   const size_t bins_smem = bins_scratch ? 0 : (size_t)3 * batch * bin_tiles_per_row(nrb, 2) * sizeof(int);
   const size_t row_smem = prepare_scratch ? 0 : (size_t)nrb * sizeof(int);
