@@ -909,7 +909,8 @@ struct CutceSplits {
   float* head_sums;      // [parts][d][slab_width]
   size_t hidden_room;    // floats in hidden_sums
   int head_most;         // parts that head_sums has room for
-  int tile;              // 256 or 128: the output tile's sides
+  int tile;              // 256 or 128: the output tile's sides in this slab
+  int head_tile;         // and in a slab of the whole vocabulary
   int vocab;             // columns of the whole vocabulary, padded to 256
   bool with_head;
 };
@@ -938,7 +939,8 @@ CT_DEVICE int hidden_parts(const CutceSplits& sp, int tile, int n_act, int d, in
 }
 // A slab's dHead is cut as the whole vocabulary's is, whatever the slab: dHead is bit for bit the same
 // for every workspace. (dHidden adds over slabs anyway.)
-CT_DEVICE int head_parts(const CutceSplits& sp, int tile, int n_act, int d) {
+CT_DEVICE int head_parts(const CutceSplits& sp, int n_act, int d) {
+  const int tile = sp.head_tile;
   const int row_blocks = (n_act + tile - 1) / tile;
   if (row_blocks == 0) return 1;
   const float groups = (float)(row_blocks * (tile / 128));
@@ -1151,7 +1153,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
   const int col_blocks = (p.d + kTile - 1) / kTile, slab_tiles = sl.width / kTile;
   const int row_blocks = (n_act + kTile - 1) / kTile;
   const int parts_h = hidden_parts(sp, kTile, n_act, p.d, sl.width);
-  const int parts_w = HEAD ? head_parts(sp, kTile, n_act, p.d) : 1;
+  const int parts_w = HEAD ? head_parts(sp, n_act, p.d) : 1;
   const int total_h = row_blocks * col_blocks * parts_h, total_w = HEAD ? slab_tiles * col_blocks * parts_w : 0;
   // Short problems walk one list, the longer units first; large ones the hidden gradient's grid (row
   // block, (part, column block)) and then the head gradient's (vocabulary tile, (part, column block)).
@@ -1210,7 +1212,7 @@ __global__ __launch_bounds__(256) void cutce_reduce_kernel(CutceParams p, CutceS
     }
   }
   if (!sp.with_head) return;
-  const int parts_w = head_parts(sp, sp.tile, n_act, p.d);
+  const int parts_w = head_parts(sp, n_act, p.d);
   if (parts_w <= 1) return;
   const int width = min(sl.width, (p.V - sl.first + 3) & ~3);
   const int quads = width / 4;
@@ -1777,7 +1779,10 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
     sp.head_sums = reinterpret_cast<float*>(ws + L.head_sums);
     sp.hidden_room = L.hidden_sums_bytes / sizeof(float);
     sp.head_most = L.head_most;
-    sp.tile = gradient_tile(a->shape);
+    // (a slab of a bounded workspace is a short problem whatever the vocabulary: 496 x 640 x 30116 in chunks of 22 rows
+    // 1100 -> 722 us, 9540 x 512 x 7604 in chunks of 40 2616 -> 1913; dHead's parts go by the whole vocabulary's tile)
+    sp.tile = gradient_tile(ct_cutce_shape{a->shape.rows, a->shape.hidden, slab_width});
+    sp.head_tile = gradient_tile(a->shape);
     sp.vocab = tiles * kGemmTile;
     sp.with_head = dhead != nullptr;
     rc = (sp.tile == kGemmTile ? launch_grads<4> : launch_grads<2>)("ct_cutce_bwd", stream, p, slab, sp, guarded_head);
