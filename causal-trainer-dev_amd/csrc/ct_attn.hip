@@ -9,6 +9,7 @@
 #include "ct_attn_fwd_split.hip.h"
 #include "ct_attn_kernels.hip.h"
 #include "ct_error.h"
+#include "ct_lanes.hip.h"
 
 #include <string.h>
 
@@ -32,29 +33,6 @@ CT_DEVICE int lanes_per_item(int n, int threads) {
   while (lanes < 64 && lanes * 2 * n <= threads) lanes *= 2;
   return lanes;
 }
-// v over the aligned group of `lanes` lanes (a power of two) that the lane belongs to, for all of them. Up to 16 lanes by
-// lane moves of the vector ALU: a shuffle through LDS costs ten times their latency, and these kernels are nothing else.
-template <class F>
-CT_DEVICE int over_lanes(int v, int lanes, F f) {
-  const auto step = [&](auto control) { v = f(v, __builtin_amdgcn_mov_dpp(v, control.value, 0xf, 0xf, true)); };
-  if (lanes >= 2) step(std::integral_constant<int, 0xb1>{});    // quad_perm 1, 0, 3, 2
-  if (lanes >= 4) step(std::integral_constant<int, 0x4e>{});    // quad_perm 2, 3, 0, 1
-  if (lanes >= 8) step(std::integral_constant<int, 0x141>{});   // the other four of eight, mirrored
-  if (lanes >= 16) step(std::integral_constant<int, 0x140>{});  // the other eight of sixteen
-  if (lanes >= 32) v = f(v, __shfl_xor(v, 16, 64));
-  if (lanes >= 64) v = f(v, __shfl_xor(v, 32, 64));
-  return v;
-}
-CT_DEVICE int min_over(int v, int lanes) {
-  return over_lanes(v, lanes, [](int a, int b) { return min(a, b); });
-}
-CT_DEVICE int max_over(int v, int lanes) {
-  return over_lanes(v, lanes, [](int a, int b) { return max(a, b); });
-}
-CT_DEVICE int sum_over(int v, int lanes) {
-  return over_lanes(v, lanes, [](int a, int b) { return a + b; });
-}
-
 // What a block's record says of its ids and visible ends; 32 consecutive lanes per block, all of them get it.
 struct BlockIds {
   int min_nz, max_id, uniform, end_min, end_max;
@@ -383,12 +361,8 @@ CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
     }
     // back to lane = bin
     count = __builtin_amdgcn_ds_permute(lane < kBins ? (int)(key % kBins) * 4 : lane * 4, count);
+    const int incl = wave_scan(count);
     if (lane < kBins) {
-      int incl = count;
-      for (int off = 1; off < kBins; off <<= 1) {
-        const int below = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += below;
-      }
       start[lane] = incl - count;
       if (lane == kBins - 1) start[kBins] = incl;
     }

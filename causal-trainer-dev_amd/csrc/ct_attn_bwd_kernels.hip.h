@@ -14,6 +14,7 @@
 #pragma once
 
 #include "ct_attn_kernels.hip.h"
+#include "ct_lanes.hip.h"
 
 namespace ct {
 
@@ -387,51 +388,44 @@ CT_DEVICE int dkv_split_count(int items, int target) {
 CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int max_entries, int max_partials, int* header,
                             int2* entries, int* zeroed, int zeroed_count) {
   for (int i = threadIdx.x; i < zeroed_count; i += 1024) zeroed[i] = 0;  // dQ's work counters
-  __shared__ long long red[16];  // one value per wavefront
+  __shared__ int red[32];  // one value per wavefront, or two
   __shared__ int hist[256];
   __shared__ int fill[256];
   __shared__ int carry;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int nrb = S / 32, ntiles = B * (nrb / 4);
 
-  // Reductions and scans run inside the wavefronts (lane shuffles) and meet once in LDS: the
+  // Reductions and scans run inside the wavefronts (lane moves) and meet once in LDS: the
   // kernel is one workgroup on an otherwise idle GPU, so its time is its chain of barriers.
-  auto block_sum = [&](long long v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) red[wave] = v;
+  auto block_sums = [&](int u, int v, int* sum_u, int* sum_v) {
+    const int wave_u = lane_value(wave_scan(u), 63), wave_v = lane_value(wave_scan(v), 63);
+    if (lane == 0) {
+      red[wave] = wave_u;
+      red[16 + wave] = wave_v;
+    }
     __syncthreads();
-    long long out = 0;
-    for (int i = 0; i < 16; ++i) out += red[i];
+    const int sums = wave_scan(lane < 32 ? red[lane] : 0);
     __syncthreads();
-    return out;
+    *sum_u = lane_value(sums, 15);
+    *sum_v = lane_value(sums, 31) - *sum_u;
   };
   auto block_max = [&](int v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    if (lane == 0) red[wave] = v;
+    const int most = lane_value(wave_scan<true>(v), 63);
+    if (lane == 0) red[wave] = most;
     __syncthreads();
-    int out = (int)red[0];
-    for (int i = 1; i < 16; ++i) out = max(out, (int)red[i]);
+    const int out = lane_value(wave_scan<true>(lane < 16 ? red[lane] : 0), 15);
     __syncthreads();
     return out;
   };
   // exclusive prefix of v over the workgroup's threads, and the total
   auto block_scan = [&](int v, int* total) {
-    int inc = v;
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(inc, off, 64);
-      if (lane >= off) inc += up;
-    }
+    const int inc = wave_scan(v);
     if (lane == 63) red[wave] = inc;
     __syncthreads();
-    int before = 0, all = 0;
-    for (int i = 0; i < 16; ++i) {
-      const int part = (int)red[i];
-      if (i < wave) before += part;
-      all += part;
-    }
+    const int sums = wave_scan(lane < 16 ? red[lane] : 0);
     __syncthreads();
-    *total = all;
-    return before + inc - v;
+    *total = lane_value(sums, 15);
+    return (wave ? lane_value(sums, wave - 1) : 0) + inc - v;
   };
   // this thread's first tile is read once; further tiles (more than 1024) are re-read per pass
   const int items_first = tid < ntiles ? dkv_tile_items(meta, nrb, tid, g) : 0;
@@ -439,7 +433,10 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
 
   long long local = 0;
   for (int t = tid; t < ntiles; t += 1024) local += items_of(t);
-  const long long total = block_sum(local);
+  // (the threads' sums in halves: both fit in 32 bits over 1024 threads with up to 8192 tiles each)
+  int high = 0, low = 0;
+  block_sums((int)(local >> 16), (int)(local & 0xffff), &high, &low);
+  const long long total = ((long long)high << 16) + low;
   long long want = (total * Hkv + kDkvSlots - 1) / kDkvSlots;  // one compute slot's fair share
   const long long pairs = (long long)ntiles * Hkv;  // (key tile, KV head)
   const int least = pairs <= kDkvSlots / 16 ? kDkvMinChunk / 4 : pairs <= kDkvSlots / 2 ? kDkvMinChunk / 2 : kDkvMinChunk;
@@ -449,17 +446,18 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   // space the host reserved (cannot happen for target >= want, kept as a guard).
   int max_work = 1;
   for (;;) {
-    long long counts = 0;  // entries in the high half, partial slots in the low half
-    int local_max = 1;
+    int entry_count = 0, partial_count = 0, local_max = 1;
     for (int t = tid; t < ntiles; t += 1024) {
       const int items = items_of(t);
       const int ns = dkv_split_count(items, target);
-      counts += ((long long)ns << 32) + (ns > 1 ? ns : 0);
+      entry_count += ns;
+      partial_count += ns > 1 ? ns : 0;
       local_max = max(local_max, (items + ns - 1) / ns);
     }
-    const long long both = block_sum(counts);
+    int entries_wanted = 0, partials_wanted = 0;
+    block_sums(entry_count, partial_count, &entries_wanted, &partials_wanted);
     max_work = block_max(local_max);
-    if ((both >> 32) <= max_entries && (both & 0xffffffffll) <= max_partials) break;
+    if (entries_wanted <= max_entries && partials_wanted <= max_partials) break;
     target = target >= INT_MAX / 4 ? INT_MAX / 2 : target * 2;
   }
 

@@ -3,6 +3,7 @@
 // Integer work, bit-exact against the reference (src/modeling/rotary.py:13-50,
 // src/training/losses.py:21-85).
 #include "ct_error.h"
+#include "ct_lanes.hip.h"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -18,21 +19,6 @@ namespace ct {
 // take one pass. Rows at 16-byte addresses are moved in quads (ALIGNED), scans and exchanges are lane moves of the vector
 // ALU, where a shuffle through LDS has ten times the latency: [4, 4096] 5.5 -> 4.0 us.
 constexpr int kScanPer = 4;
-// Inclusive scan over the wavefront (values are not negative: 0 is neutral for sums and maxima).
-template <bool MAX>
-__device__ __forceinline__ int wave_scan(int v) {
-  const auto add = [&](int moved) { v = MAX ? max(v, moved) : v + moved; };
-  add(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));  // from 1, 2, 4, 8 lanes below in a row of 16
-  add(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
-  add(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
-  add(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
-  add(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // lane 15 to the second row, 47 to the fourth
-  add(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // lane 31 to the upper half
-  return v;
-}
-// The value of the lane below, `first` for lane 0.
-__device__ __forceinline__ int lane_below(int v, int first) { return __builtin_amdgcn_update_dpp(first, v, 0x138, 0xf, 0xf, false); }
-
 template <bool POSITIONS, bool ALIGNED>
 __global__ __launch_bounds__(1024) void segment_scan_kernel(const int* mask, const int* labels, int S, int* out) {
   __shared__ int wave_total[2][16];
@@ -76,9 +62,9 @@ __global__ __launch_bounds__(1024) void segment_scan_kernel(const int* mask, con
     if (lane == 63) total[wave] = incl;
     __syncthreads();
     const int totals = wave_scan<POSITIONS>(lane < nwaves ? total[lane] : 0);
-    int before = wave ? __builtin_amdgcn_readlane(totals, wave - 1) : 0;
+    int before = wave ? lane_value(totals, wave - 1) : 0;
     before = POSITIONS ? max(before, carry) : before + carry;
-    const int all = __builtin_amdgcn_readlane(totals, nwaves - 1);
+    const int all = lane_value(totals, nwaves - 1);
     carry = POSITIONS ? max(carry, all) : carry + all;
     const int left = lane_below(incl, 0);
     before = POSITIONS ? max(before, left) : before + left;
