@@ -123,6 +123,7 @@ SYMBOLS = {
     "ct_calibration_copy": (c_int32, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "ct_canonicalize_segment_ids": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "ct_transpose16": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
+    "ct_transpose16_padded": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_int32]),
     "ct_segment_positions": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "ct_shifted_targets_scratch_bytes": (c_size_t, [c_int32, c_int32]),
     "ct_shifted_targets_and_weights": (c_int32, [c_void_p, POINTER(ShiftedTargetsArgs)]),
@@ -156,6 +157,9 @@ SYMBOLS = {
     "ct_cutce_logits_cache_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_fwd": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
     "ct_cutce_bwd": (c_int32, [c_void_p, POINTER(CutceBwdArgs)]),
+    "ct_cutce_panel_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_fwd_panel": (c_int32, [c_void_p, POINTER(CutceFwdArgs), c_void_p, c_int32]),
+    "ct_cutce_bwd_panel": (c_int32, [c_void_p, POINTER(CutceBwdArgs), c_void_p]),
     "ct_cutce_fwd_noalloc_max_bytes": (c_size_t, []),
     "ct_cutce_fwd_noalloc": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
 }

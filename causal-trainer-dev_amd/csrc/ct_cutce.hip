@@ -1346,10 +1346,10 @@ struct BwdTileBytes {
   size_t g, panel, head_sums;
   size_t all() const { return g + panel + head_sums; }
 };
-static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, bool panel_in_cache, bool with_head) {
+static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, bool panel_elsewhere, bool with_head) {
   const int parts = with_head ? most_head_parts(s) : 1;
   return BwdTileBytes{(size_t)padded_rows(s.rows) * kGemmTile * sizeof(bf16),
-                      needs_panel(s) && !panel_in_cache ? panel_tile_bytes(s) : 0,
+                      needs_panel(s) && !panel_elsewhere ? panel_tile_bytes(s) : 0,
                       parts > 1 ? (size_t)parts * s.hidden * kGemmTile * sizeof(float) : 0};
 }
 static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
@@ -1358,7 +1358,7 @@ static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
 // The whole vocabulary as one slab if that fits in `bytes`, else the largest slab that does
 // (slab_cols = 0 if even one tile column does not). The partial sums of a cut dHidden come last: as
 // many parts as fit behind one slab, with several slabs in up to half of what is left for slabs.
-static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_in_cache, bool with_head) {
+static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_elsewhere, bool with_head) {
   const int n_pad = padded_rows(s.rows);
   const int tiles = vocab_tile_count(s.vocab);
   BwdLayout L = {};
@@ -1368,7 +1368,7 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_in
   L.packed = L.rowparams + 3 * align_up((size_t)n_pad * sizeof(int), 256);
   L.panel = bwd_fixed_bytes(n_pad, s.hidden);
   L.tail = L.panel - (size_t)s.hidden * 128 * sizeof(bf16);
-  const BwdTileBytes tile = bwd_tile_bytes(s, panel_in_cache, with_head);
+  const BwdTileBytes tile = bwd_tile_bytes(s, panel_elsewhere, with_head);
   const size_t per_tile = tile.all(), acc_bytes = bwd_acc_bytes(s);
   size_t fit = tiles, room;
   L.head_most = with_head ? most_head_parts(s) : 1;
@@ -1568,8 +1568,9 @@ static int launch_grads(const char* fn, hipStream_t stream, const CutceParams& p
 
 // Shared body of ct_cutce_fwd and ct_cutce_fwd_noalloc: `ws` / `ws_bytes` is the workspace to use
 // (the caller's, or this device's static scratch array), `fn` the name for error texts.
+// `lent`: the caller's panel or null, made here unless `filled`.
 static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_, size_t ws_bytes,
-                            const char* fn) {
+                            const char* fn, bf16* lent = nullptr, bool filled = false) {
   CT_REQUIRE(a->hidden && a->head && a->targets && a->weights && a->nll_sum && a->weight_sum &&
                  a->lse && ws_,
              "%s: null pointer", fn);
@@ -1595,13 +1596,18 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   p.slot_target = reinterpret_cast<int*>(ws + L.target);
   p.block_active = reinterpret_cast<int*>(ws + L.active);
   const StatsUnits units = stats_units(a->shape);
-  // The panel of a head with unaligned rows: at the end of the logits cache, where the backward finds
+  // The panel of a head with unaligned rows: lent by the caller, at the end of the logits cache, where the backward finds
   // it again, or in what the workspace has behind its fixed part, a number of chunks at a time.
   const int step_tiles = units.per_chunk, step_chunks = kGemmTile / units.tile;  // 256-column tiles and chunks of a panel step
   bf16* panel = nullptr;
   int chunks_per_pass = units.chunks;
-  if (needs_panel(a->shape)) {
-    if (a->logits_cache) {
+  if (!needs_panel(a->shape)) {
+    lent = nullptr;
+  } else {
+    if (lent) {
+      CT_REQUIRE(is_aligned16(lent), "%s: panel must be 16-byte aligned", fn);
+      panel = lent;
+    } else if (a->logits_cache) {
       panel = reinterpret_cast<bf16*>(static_cast<char*>(a->logits_cache) + logits_bytes(a->shape));
     } else {
       const size_t fit = ws_bytes >= L.total ? (size_t)units.chunks : (ws_bytes - L.base) / (panel_tile_bytes(a->shape) * step_tiles);
@@ -1616,7 +1622,7 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     if (panel) {
       const int tile0 = chunk0 / step_chunks * step_tiles;
       const int pass_tiles = min((pass_chunks + step_chunks - 1) / step_chunks * step_tiles, vocab_tile_count(p.V) - tile0);
-      copy = panel_copy(head, panel, tile0, pass_tiles);
+      if (!lent || !filled) copy = panel_copy(head, panel, tile0, pass_tiles);
       p.head = panel_view(panel, tile0, pass_tiles);
     }
     const int list_blocks = chunk0 == 0 ? (p.N + 1023) / 1024 : 0;
@@ -1687,7 +1693,18 @@ extern "C" int32_t ct_cutce_fwd_noalloc(void* stream, const ct_cutce_fwd_args* a
   return cutce_fwd_on(stream, a, ws, kNoAllocScratchBytes, "ct_cutce_fwd_noalloc");
 }
 
-extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
+extern "C" size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape) {
+  return valid_sizes(shape) ? full_panel_bytes(*shape) : 0;
+}
+
+extern "C" int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* a, uint16_t* panel, int32_t filled) {
+  CT_REQUIRE(a, "ct_cutce_fwd: null args");
+  return cutce_fwd_on(stream, a, a->workspace, a->workspace_bytes, "ct_cutce_fwd", reinterpret_cast<bf16*>(panel), filled != 0);
+}
+
+extern "C" int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* a) { return ct_cutce_bwd_panel(stream, a, nullptr); }
+
+extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a, const uint16_t* lent) {
   CT_REQUIRE(a, "ct_cutce_bwd: null args");
   CT_REQUIRE(a->hidden && a->head && a->targets && a->weights && a->lse && a->dy && a->dhidden &&
                  a->workspace,
@@ -1697,7 +1714,8 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   if (rc) return rc;
   CT_REQUIRE(is_aligned16(a->workspace) && is_aligned16(a->dhidden),
              "ct_cutce_bwd: workspace and dhidden must be 16-byte aligned");
-  const BwdLayout L = bwd_layout(a->shape, a->workspace_bytes, a->logits_cache != nullptr, a->dhead != nullptr);
+  CT_REQUIRE(is_aligned16(lent), "ct_cutce_bwd: panel must be 16-byte aligned");
+  const BwdLayout L = bwd_layout(a->shape, a->workspace_bytes, lent || a->logits_cache, a->dhead != nullptr);
   if (L.slab_cols == 0)
     return fail(CT_WORKSPACE_TOO_SMALL, "ct_cutce_bwd: workspace %zu < %zu bytes",
                 a->workspace_bytes, ct_cutce_bwd_workspace_min_bytes(&a->shape));
@@ -1733,7 +1751,9 @@ extern "C" int32_t ct_cutce_bwd(void* stream_, const ct_cutce_bwd_args* a) {
   p.head.tail = tail;
   bf16* panel = nullptr;
   if (needs_panel(a->shape)) {
-    if (cache) {  // the forward left it there
+    if (lent) {
+      p.head = panel_view(reinterpret_cast<const bf16*>(lent), 0, tiles);
+    } else if (cache) {  // the forward left it there
       p.head = panel_view(reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(cache) + logits_bytes(a->shape)), 0, tiles);
     } else {
       panel = reinterpret_cast<bf16*>(ws + L.panel);

@@ -124,14 +124,15 @@ static int launch_segment_scan(hipStream_t stream, const char* name, const int* 
   return scope.done();
 }
 
-// Transposed copy of 16-bit elements: dst [cols][rows] = src [rows][cols]^T. Bound by memory. A workgroup
+// Transposed copy of 16-bit elements: dst [cols][ld], of whose rows the first `rows` elements are src [rows][cols]^T and
+// the others zero. Bound by memory. A workgroup
 // takes a 64 x 64 tile, so both sides move whole 128-byte lines; a thread loads 8 columns of two rows and
 // stores 8 rows of two columns (memcpy: rows of an odd length start at any multiple of 2 bytes, which an
 // ordinary access may). LDS rows are 66 elements: the 8-element columns that a wavefront collects lie
 // 8 * 33 words apart per lane group and hit all banks. [76395, 1536]: 119 us (4.0 TB/s; a strided copy of the
 // transposed view 2264), [32000, 4096]: 116 us (4.5 TB/s; 1859).
 constexpr int kTransposeTile = 64, kTransposePitch = kTransposeTile + 2;
-__global__ __launch_bounds__(256) void transpose16_kernel(const unsigned short* src, int rows, int cols, unsigned short* dst) {
+__global__ __launch_bounds__(256) void transpose16_kernel(const unsigned short* src, int rows, int cols, unsigned short* dst, int ld) {
   __shared__ unsigned short tile[kTransposeTile * kTransposePitch];
   const unsigned col_tiles = ((unsigned)cols + kTransposeTile - 1) / kTransposeTile;
   const int r0 = (int)(blockIdx.x / col_tiles) * kTransposeTile, c0 = (int)(blockIdx.x % col_tiles) * kTransposeTile;
@@ -155,8 +156,8 @@ __global__ __launch_bounds__(256) void transpose16_kernel(const unsigned short* 
   __syncthreads();
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
-    const int c = line + 32 * pass, left = c0 + c < cols ? rows - (r0 + chunk) : 0;
-    unsigned short* to = dst + (size_t)(c0 + c) * rows + r0 + chunk;
+    const int c = line + 32 * pass, left = c0 + c < cols ? ld - (r0 + chunk) : 0;
+    unsigned short* to = dst + (size_t)(c0 + c) * ld + r0 + chunk;
     unsigned short v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = tile[(chunk + e) * kTransposePitch + c];
@@ -215,12 +216,17 @@ extern "C" int32_t ct_shifted_targets_and_weights(void* stream_, const ct_shifte
   return scope2.done();
 }
 
-extern "C" int32_t ct_transpose16(void* stream_, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst) {
+extern "C" int32_t ct_transpose16(void* stream, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst) {
+  return ct_transpose16_padded(stream, src, rows, cols, dst, rows);
+}
+extern "C" int32_t ct_transpose16_padded(void* stream_, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst,
+                                         int32_t ld) {
   CT_REQUIRE(src && dst, "ct_transpose16: null pointer");
   CT_REQUIRE(rows > 0 && cols > 0, "ct_transpose16: dimensions must be positive");
-  const long tiles = (long)(((unsigned)rows + kTransposeTile - 1) / kTransposeTile) * (((unsigned)cols + kTransposeTile - 1) / kTransposeTile);
+  CT_REQUIRE(ld >= rows, "ct_transpose16: rows of %d elements do not fit in %d", rows, ld);
+  const long tiles = (long)(((unsigned)ld + kTransposeTile - 1) / kTransposeTile) * (((unsigned)cols + kTransposeTile - 1) / kTransposeTile);
   CT_REQUIRE(tiles <= 0x7fffffff, "ct_transpose16: [%d, %d] has more tiles than a launch takes", rows, cols);
   LaunchScope scope("transpose16_kernel", (hipStream_t)stream_);
-  hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream_, src, rows, cols, dst);
+  hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream_, src, rows, cols, dst, ld);
   return scope.done();
 }

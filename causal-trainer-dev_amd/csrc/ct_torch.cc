@@ -523,14 +523,15 @@ ct_cutce_shape cut_shape(const Tensor& hidden, const Tensor& head) {
   return {(int32_t)(hidden.numel() / width), (int32_t)width, (int32_t)head.size(1)};
 }
 
-std::tuple<Tensor, Tensor, Tensor> cutce_forward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
-                                                 const Tensor& weights, bool compaction, const MaybeTensor& cache,
-                                                 int64_t workspace_bytes) {
+// head: [d, V], or the panel itself (then read from there only)
+std::tuple<Tensor, Tensor, Tensor> cutce_forward_on(const ct_cutce_shape& shape, const Tensor& hidden, const Tensor& head,
+                                                    const Tensor& targets, const Tensor& weights, bool compaction,
+                                                    const MaybeTensor& cache, int64_t workspace_bytes, const MaybeTensor& panel,
+                                                    bool filled) {
   const c10::DeviceGuard guard(hidden.device());
-  const ct_cutce_shape shape = cut_shape(hidden, head);
   // (with a logits cache the aligned copy of an unaligned head goes there)
   const bool cached = cache && cache->defined();
-  const size_t bytes = cached ? ct_cutce_fwd_workspace_min_bytes(&shape)
+  const size_t bytes = cached || panel ? ct_cutce_fwd_workspace_min_bytes(&shape)
                        : workspace_bytes >= 0 ? (size_t)workspace_bytes : ct_cutce_fwd_workspace_bytes(&shape);
   Tensor workspace = scratch(bytes, hidden);
   Tensor nll = floats({}, hidden), weight_sum = floats({}, hidden), lse = floats({shape.rows}, hidden);
@@ -548,19 +549,26 @@ std::tuple<Tensor, Tensor, Tensor> cutce_forward(const Tensor& hidden, const Ten
   a.sparse_compaction = compaction;
   a.logits_cache = cached ? cache->data_ptr() : nullptr;
   a.logits_cache_bytes = cached ? (size_t)cache->numel() : 0;
-  check(ct_cutce_fwd(current_stream(), &a));
+  check(ct_cutce_fwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr, filled));
   return {nll, weight_sum, lse};
 }
+std::tuple<Tensor, Tensor, Tensor> cutce_forward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
+                                                 const Tensor& weights, bool compaction, const MaybeTensor& cache,
+                                                 int64_t workspace_bytes) {
+  return cutce_forward_on(cut_shape(hidden, head), hidden, head, targets, weights, compaction, cache, workspace_bytes,
+                          std::nullopt, false);
+}
 
-std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
-                                               const Tensor& weights, const Tensor& lse, const Tensor& dy, bool compaction,
-                                               bool with_head, int64_t workspace_bytes, const MaybeTensor& cache) {
+std::tuple<Tensor, MaybeTensor> cutce_backward_on(const ct_cutce_shape& shape, const Tensor& hidden, const Tensor& head,
+                                                  const Tensor& targets, const Tensor& weights, const Tensor& lse,
+                                                  const Tensor& dy, bool compaction, bool with_head, int64_t workspace_bytes,
+                                                  const MaybeTensor& cache, const MaybeTensor& panel) {
   const c10::DeviceGuard guard(hidden.device());
-  const ct_cutce_shape shape = cut_shape(hidden, head);
-  const size_t bytes = workspace_bytes >= 0 ? (size_t)workspace_bytes : ct_cutce_bwd_workspace_bytes(&shape);
+  const size_t bytes = workspace_bytes >= 0 ? (size_t)workspace_bytes
+                                            : ct_cutce_bwd_workspace_bytes(&shape) - (panel ? ct_cutce_panel_bytes(&shape) : 0);
   Tensor workspace = scratch(bytes, hidden), dhidden = fresh(hidden);
   MaybeTensor dhead;
-  if (with_head) dhead = fresh(head);
+  if (with_head) dhead = at::empty({shape.hidden, shape.vocab}, hidden.options().requires_grad(false));
   const bool cached = cache && cache->defined();
   ct_cutce_bwd_args a = {};
   a.hidden = bits(hidden);
@@ -577,22 +585,32 @@ std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tenso
   a.sparse_compaction = compaction;
   a.logits_cache = cached ? cache->data_ptr() : nullptr;
   a.logits_cache_bytes = cached ? (size_t)cache->numel() : 0;
-  check(ct_cutce_bwd(current_stream(), &a));
+  check(ct_cutce_bwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr));
   return {dhidden, dhead};
+}
+std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
+                                               const Tensor& weights, const Tensor& lse, const Tensor& dy, bool compaction,
+                                               bool with_head, int64_t workspace_bytes, const MaybeTensor& cache) {
+  return cutce_backward_on(cut_shape(hidden, head), hidden, head, targets, weights, lse, dy, compaction, with_head,
+                           workspace_bytes, cache, std::nullopt);
 }
 
 // The reference's residual (src/causal_trainer/kernels/cut_cross_entropy.py:587-593) plus, when it
-// fits, the f32 logits cache, which the first backward gives back.
+// fits, the f32 logits cache, which the first backward gives back, and the aligned copy that the forward has
+// read an unaligned head from, or for a [V, d] head (whose `head` is then this copy) in the place of a plain transposed one.
 struct CutCeNode : OperatorNode {
   SavedVariable hidden, head, targets, weights, lse;
-  MaybeTensor cache;
+  MaybeTensor cache, panel;
+  ct_cutce_shape shape = {};
+  bool head_is_panel = false;
   bool compaction = false, trainable = true, vocab_major = false;
   int64_t workspace_bytes = -1;
   variable_list differentiate(variable_list&& grads) override {
     const Tensor X = hidden.unpack(), W = head.unpack(), T = targets.unpack(), w = weights.unpack(), L = lse.unpack();
     const Tensor dy = gradient(grads[0], {}, at::kFloat, X);
-    const MaybeTensor logits = std::exchange(cache, std::nullopt);
-    auto [dx, dw] = cutce_backward(X, W, T, w, L, dy, compaction, trainable, workspace_bytes, logits);
+    const MaybeTensor logits = std::exchange(cache, std::nullopt), copy = std::exchange(panel, std::nullopt);
+    auto [dx, dw] = cutce_backward_on(shape, X, W, T, w, L, dy, compaction, trainable, workspace_bytes, logits,
+                                      head_is_panel ? MaybeTensor(W) : copy);
     return {dx, !dw ? Tensor() : vocab_major ? dw->t() : *dw};
   }
   void release_variables() override {
@@ -602,6 +620,7 @@ struct CutCeNode : OperatorNode {
     weights.reset_data();
     lse.reset_data();
     cache.reset();
+    panel.reset();
   }
   std::string name() const override { return "CutCrossEntropyBackward"; }
 };
@@ -612,6 +631,10 @@ struct CutCeNode : OperatorNode {
 // 768: 974 / 971, 1024: 1130 / 1195. Logits that stay in the memory-side cache (256 MB) cost less: 4096 x 3200,
 // 512: 120 / 124; 130 x 76000, 512: 180 / 188; 1000 x 32003, 512: 225 / 224.
 bool cache_pays(const ct_cutce_shape& shape, size_t bytes) { return shape.hidden > 640 || bytes <= ((size_t)256 << 20); }
+
+// Train steps, us: 281 rows x 1152 x 105348 611 -> 538, 50 x 896 x 74295 270 -> 223; a [35263, 7552] head and 21 rows, whose
+// transposed copy was copied again in each direction, 1365 -> 815.
+constexpr size_t kPanelLimit = (size_t)1 << 30;
 
 // vocab_major: head is [V, d]; the kernels get a transposed copy, the gradient goes back as a view of theirs.
 std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Tensor& head, const Tensor& targets,
@@ -625,23 +648,36 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
       weights.device() != hidden.device())
     return std::nullopt;
   const bool graph = needs_graph({hidden, head});
-  Tensor columns = head;  // [d, V]
+  const int64_t width = hidden.size(2);
+  const ct_cutce_shape shape = {(int32_t)(hidden.numel() / width), (int32_t)width, (int32_t)head.size(vocab_major ? 0 : 1)};
+  const c10::DeviceGuard guard(head.device());
+  // (a bounded workspace: the copies keep to it)
+  const size_t panel_bytes = forward_bytes < 0 ? ct_cutce_panel_bytes(&shape) : 0;
+  const bool head_is_panel = vocab_major && panel_bytes;
+  Tensor columns = head;  // [d, V], padded in a panel
   if (vocab_major) {
-    const c10::DeviceGuard guard(head.device());
-    columns = at::empty({head.size(1), head.size(0)}, head.options().requires_grad(false));
-    check(ct_transpose16(current_stream(), bits(head), (int32_t)head.size(0), (int32_t)head.size(1), bits(columns)));
+    const int64_t ld = head_is_panel ? (int64_t)(panel_bytes / 2) / width : shape.vocab;
+    columns = at::empty({width, ld}, head.options().requires_grad(false));
+    check(ct_transpose16_padded(current_stream(), bits(head), shape.vocab, shape.hidden, bits(columns), (int32_t)ld));
   }
-  MaybeTensor cache;
+  MaybeTensor cache, panel;
   if (use_cache && graph) {
-    const ct_cutce_shape shape = cut_shape(hidden, columns);
     const size_t bytes = ct_cutce_logits_cache_bytes(&shape);
     if ((int64_t)bytes <= cache_limit && cache_pays(shape, bytes)) cache = scratch(bytes, hidden);
   }
-  auto [nll, weight_sum, lse] = cutce_forward(hidden, columns, targets, weights, compaction, cache, forward_bytes);
+  // An unaligned head is copied once for both directions where the copy is at most kPanelLimit (it lives as long as
+  // the other residuals; the peak is what it was, each direction had one in its workspace).
+  if (head_is_panel) panel = columns;
+  else if (graph && !cache && panel_bytes && panel_bytes <= kPanelLimit) panel = scratch(panel_bytes, hidden);
+  auto [nll, weight_sum, lse] =
+      cutce_forward_on(shape, hidden, columns, targets, weights, compaction, cache, forward_bytes, panel, head_is_panel);
   if (graph) {
     auto node = graph_node<CutCeNode>({hidden, head});
     node->hidden = SavedVariable(hidden, false);
     node->head = SavedVariable(columns, false);
+    node->shape = shape;
+    node->head_is_panel = head_is_panel;
+    if (!head_is_panel) node->panel = panel;
     node->targets = SavedVariable(targets, false);
     node->weights = SavedVariable(weights, false);
     node->lse = SavedVariable(lse, false);

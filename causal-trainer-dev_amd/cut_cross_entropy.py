@@ -131,7 +131,8 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
                                     lm_head_trainable: bool = True, local_chunk_size: int = 0,
                                     logits_cache: bool = True, head_layout: str = "dv"):
     """Return ``(nll_sum, weight_sum)``; logits are only ever kept in the bounded cache
-    described in the module docstring (``logits_cache=False`` disables it).
+    described in the module docstring (``logits_cache=False`` disables it). A head whose vocabulary is no multiple
+    of 8 is read through an aligned copy; one of up to 1 GiB that the forward made is left to the backward.
 
     hidden_states ``[B, S, d]``, lm_head_kernel ``[d, V]`` (same float dtype, bf16),
     targets int32 ``[B, S]``, weights f32 ``[B, S]``; a row is ignored iff its weight is 0.

@@ -261,6 +261,8 @@ int32_t ct_segment_positions(void* stream, const int32_t* attention_mask, const 
  * layout as the cut cross-entropy takes it (the reference transposes at load,
  * src/causal_trainer/checkpointing/huggingface.py:1-6). */
 int32_t ct_transpose16(void* stream, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst);
+/* The same with rows of ld >= rows elements in dst, zero from `rows` on (a panel, see ct_cutce_panel_bytes). */
+int32_t ct_transpose16_padded(void* stream, const uint16_t* src, int32_t rows, int32_t cols, uint16_t* dst, int32_t ld);
 
 typedef struct ct_shifted_targets_args {
   const int32_t* input_ids;       /* int32 [batch, seq] */
@@ -516,6 +518,18 @@ typedef struct ct_cutce_bwd_args {
  * (src/kernels/cut_cross_entropy.py:225-471) and the scatter at :638-642.
  */
 int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* args);
+
+/*
+ * Where vocab is no multiple of 8 the rows of the head are not aligned and both directions read an aligned copy of
+ * it, the panel: bf16 [hidden][vocab rounded up to 256], zero from column vocab on; 0 bytes where none is needed.
+ * ct_cutce_fwd and ct_cutce_bwd each make one in their workspace. With these two the caller lends the panel instead
+ * (16-byte aligned, ct_cutce_panel_bytes() long): the forward fills it unless it is `filled` already (by
+ * ct_transpose16_padded from a [vocab, hidden] head, or by an earlier call with the same head), the backward reads it.
+ * args->head is then not read, and the workspaces are smaller by its size. A panel where none is needed is ignored.
+ */
+size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape);
+int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* args, uint16_t* panel, int32_t filled);
+int32_t ct_cutce_bwd_panel(void* stream, const ct_cutce_bwd_args* args, const uint16_t* panel);
 
 #ifdef __cplusplus
 }

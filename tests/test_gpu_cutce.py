@@ -506,3 +506,33 @@ def test_tiles_one_after_the_other(ct, gpu, rows, width, vocab):
     for cache, compaction in ((False, True), (True, True), (False, False)):
         print("case", rows, width, vocab, cache, compaction, flush=True)
         _check(_gpu(ct, gpu, *case, 0.37, compaction=compaction, cache=cache), *case, 0.37)
+
+
+@pytest.mark.parametrize("rows,width,vocab", [(300, 256, 1031), (70, 128, 7), (513, 1152, 4098)])
+@pytest.mark.parametrize("layout,cache", [("dv", False), ("vd", False), ("vd", True)])
+def test_one_aligned_copy_for_both_directions(ct, gpu, rows, width, vocab, layout, cache):
+    """An unaligned head's copy that the forward leaves to the backward, or that is transposed into its place: the bits of
+    the two calls that make a copy each, in a first backward and in a second one, which makes its own."""
+
+    hidden, head, targets, weights = (t.to(gpu) for t in _case(rows + vocab, rows, width, vocab))
+    dy = torch.tensor(0.37, device=gpu)
+    nll, _, lse = ct.cutce_forward(hidden, head, targets, weights, sparse_compaction=True)
+    dx, dw = ct.cutce_backward(hidden, head, targets, weights, lse, dy, sparse_compaction=True)
+    x = hidden.view(1, rows, width).requires_grad_(True)
+    w = (head if layout == "dv" else head.t().contiguous()).requires_grad_(True)
+    got, _ = ct.pallas_cut_linear_cross_entropy(x, w, targets.view(1, -1), weights.view(1, -1), logits_cache=cache,
+                                                head_layout=layout)
+    assert torch.equal(got.detach(), nll)
+    for last in (False, True):
+        gx, gw = torch.autograd.grad(got, (x, w), dy, retain_graph=not last)
+        assert torch.equal(gx.view(rows, width), dx)
+        assert torch.equal(gw if layout == "dv" else gw.t(), dw)
+
+
+@pytest.mark.parametrize("rows,cols,ld", [(7, 128, 256), (65, 64, 65), (1031, 200, 1280)])
+def test_transpose16_into_padded_rows(ct, gpu, rows, cols, ld):
+    source = torch.randint(-2 ** 15, 2 ** 15, (rows, cols), dtype=torch.int16, device=gpu)
+    out = torch.full((cols, ld), 77, dtype=torch.int16, device=gpu)
+    ct._lib.check(ct._lib.load().ct_transpose16_padded(torch.cuda.current_stream().cuda_stream, source.data_ptr(), rows, cols,
+                                                       out.data_ptr(), ld))
+    assert torch.equal(out[:, :rows], source.t()) and not out[:, rows:].any()
