@@ -1158,6 +1158,10 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
   // Short problems walk one list, the longer units first; large ones the hidden gradient's grid (row
   // block, (part, column block)) and then the head gradient's (vocabulary tile, (part, column block)).
   const bool one_list = total_h + total_w <= kPlainRounds * (int)gridDim.x;
+  // The head's are the longer where there are more rows than vocabulary: few, and last they were alone at the end (both
+  // orders, us: 13908 rows x 5376 x 632: 288 / 234, 16384 x 4096 x 1024: 334 / 266, 8000 x 2048 x 2000: 164 / 125; units of
+  // about the same length, 5000 x 1024 x 3000: 84 / 87).
+  const bool head_first = HEAD && 2l * ((n_act + 127) / 128) * parts_h > 3l * (sl.width / 128) * parts_w;
   UnitQueue units;
   bool in_head = false;
   if (one_list) units.init(p.header->xcd_counter[0], total_h + total_w, 1, UnitQueue::kPlain);
@@ -1171,8 +1175,9 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
       continue;
     }
     if (one_list) {
-      in_head = a >= total_h;
-      const int index = in_head ? a - total_h : a, width = col_blocks * (in_head ? parts_w : parts_h);
+      in_head = head_first ? a < total_w : a >= total_h;
+      const int index = a - (in_head == head_first ? 0 : head_first ? total_w : total_h);
+      const int width = col_blocks * (in_head ? parts_w : parts_h);
       a = index / width;
       b = index % width;
     }

@@ -20,7 +20,7 @@ rows fit in ``LOGITS_CACHE_LIMIT_BYTES`` the forward also leaves them in a cache
 that lives until the backward of the loss (the adjacent step of a training
 iteration), and the backward then runs 3 GEMMs instead of 4. Above the limit, where
 the projection is cheaper than the cache's traffic (small hidden sizes), or with
-``logits_cache=False``, nothing but ``lse`` is kept and logits are recomputed.
+``logits_cache=False``, no logits are kept and they are recomputed.
 
 ``local_chunk_size`` (:697-825). The reference's chunk loop bounds what one TPU core holds at
 a time: it walks the rows in chunks, compacts inside the chunk and accumulates the head
