@@ -627,10 +627,11 @@ struct CutCeNode : OperatorNode {
 
 // The logits cache pays where it saves more than it costs: 8 bytes of traffic per logit and a pass of its
 // own against 2 * hidden operations. Measured with and without it (train step, us): 4096 rows x 32000, hidden
-// 256: 508 / 422, 512: 652 / 615, 768: 826 / 840, 1024: 944 / 993; 800 x 151936, 512: 818 / 738,
-// 768: 974 / 971, 1024: 1130 / 1195. Logits that stay in the memory-side cache (256 MB) cost less: 4096 x 3200,
-// 512: 120 / 124; 130 x 76000, 512: 180 / 188; 1000 x 32003, 512: 225 / 224.
-bool cache_pays(const ct_cutce_shape& shape, size_t bytes) { return shape.hidden > 640 || bytes <= ((size_t)256 << 20); }
+// 768: 815 / 782, 896: 885 / 876, 1024: 916 / 928, 1280: 1081 / 1128; 800 x 151936, 768: 929 / 917, 1024: 1110 / 1163;
+// 16384 x 50000, 896: 5553 / 5748. Logits that stay in the memory-side cache (256 MB) cost no less: 1000 x 32003, 512:
+// 208 / 187, 768: 261 / 255, 1024: 300 / 317; 2000 x 20000, 256: 187 / 159; 3000 x 16000, 512: 266 / 234, 640: 315 / 305;
+// 4096 x 3200, 512: 113 / 114, 1024: 147 / 159; 130 x 76000, 512: 163 / 165.
+bool cache_pays(const ct_cutce_shape& shape) { return shape.hidden > 768; }
 
 // Train steps, us: 281 rows x 1152 x 105348 611 -> 538, 50 x 896 x 74295 270 -> 223; a [35263, 7552] head and 21 rows, whose
 // transposed copy was copied again in each direction, 1365 -> 815.
@@ -663,7 +664,7 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
   MaybeTensor cache, panel;
   if (use_cache && graph) {
     const size_t bytes = ct_cutce_logits_cache_bytes(&shape);
-    if ((int64_t)bytes <= cache_limit && cache_pays(shape, bytes)) cache = scratch(bytes, hidden);
+    if ((int64_t)bytes <= cache_limit && cache_pays(shape)) cache = scratch(bytes, hidden);
   }
   // An unaligned head is copied once for both directions where the copy is at most kPanelLimit (it lives as long as
   // the other residuals; the peak is what it was, each direction had one in its workspace).

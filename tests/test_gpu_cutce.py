@@ -131,7 +131,7 @@ def test_transpose16(ct, gpu, rows, cols):
 
 
 def test_small_hidden_large_logits_match_with_and_without_cache(ct, gpu):
-    """Where the operator does without the logits cache (hidden <= 640, logits beyond 256 MB) the results
+    """Where the operator does without the logits cache (hidden sizes up to 768) the results
     are those of the recomputing form: the same f32 logits of the same products."""
 
     hidden, head, targets, weights = _case(9, 1100, 128, 65537)
