@@ -456,11 +456,10 @@ def bench_cutce(ct, torch, steps, warmup, logits_cache=True):
                         "cutce_dlogits_kernel": gemm, "cutce_grads_kernel": 2 * gemm}  # dHidden + dHead in one launch
     # the HBM-bound passes over per-row statistics: the merge of the per-chunk (max, sum exp, target
     # logit) partials into lse and the loss terms reads 12 bytes per (vocabulary chunk of 1024, active
-    # row) and the weights, and writes lse; the row packing copies the active hidden rows
+    # row) and the weights, and writes lse
     chunks = -(-(-(-config.vocab // 256)) // 4)
     per_kernel_bytes = {
         "cutce_merge_kernel": chunks * active * 12 + 8 * active + 8 * config.rows,
-        "cutce_rows_kernel": 2 * active * config.hidden * 2,
     }
     if logits_cache:
         per_kernel_bytes["cutce_dlogits_cached_kernel"] = (-(-active // 256) * 256) * config.vocab * 6

@@ -164,7 +164,7 @@ struct UnitQueue {
 
 // The head as the GEMM kernels read it: column v of row n at base[n * ld + v - col0]. Either the
 // caller's tensor (ld = V) or, where its rows are not 16-byte aligned (V % 8 != 0), an aligned copy
-// of the columns col0 .. in the workspace ("panel", cutce_panel_kernel), padded with zero columns to
+// of the columns col0 .. in the workspace ("panel", HeadCopy), padded with zero columns to
 // whole tiles.
 // An aligned head whose vocabulary is no multiple of 128 has the columns from the last such multiple
 // on a second time in `tail` [d][128], padded with zeros, for the contraction over the vocabulary.
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
 }
 
 // ---------------------------------------------------------------------------
-// merge + finalize
+// merge
 // ---------------------------------------------------------------------------
 // A workgroup merges the per-chunk partials of kMergeSlots row slots: kMergeParts threads per slot
 // each walk every kMergeParts-th vocabulary chunk (so a row's chain of dependent loads is an
@@ -1283,7 +1283,7 @@ static StatsUnits stats_units(const ct_cutce_shape& s) {
   return {kGemmTile, tiles, t, (tiles + t - 1) / t};
 }
 
-// Heads whose rows do not all start on 16 bytes go through an aligned copy (cutce_panel_kernel).
+// Heads whose rows do not all start on 16 bytes go through an aligned copy (HeadCopy).
 static bool needs_panel(const ct_cutce_shape& s) { return s.vocab % 8 != 0; }
 static size_t panel_tile_bytes(const ct_cutce_shape& s) { return (size_t)s.hidden * kGemmTile * sizeof(bf16); }
 // bytes of the panel of the whole vocabulary, 0 if none is needed
