@@ -125,10 +125,23 @@ attn_fwd_split_kernel(AttnParams p) {
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) oacc[db] = zero16();
   float m_run = kNegInf;  // softmax reference (a recent running max), log2 domain
+  // What a piece takes of it: the score that moves it and the term of its exponents (0 as long as nothing is visible).
+  // Kept where registers are to spare: at head dimension 64, whose loop the vector ALU bounds, with the addresses below 12 of
+  // the 90 instructions of a piece (1 to 4 % of the kernel; at 128, where 256 registers are in use, 0.7 % slower).
+  float moves_at = kNegInf, minus_m = 0.f;
   float l_run = 0.f;      // this lane's share of the running sum
   const int own = share * SUB * KB * RowFragOffsets<D / 8>::kRowBlockBytes;  // this wavefront's keys in a stage
-  const RowFragOffsets<D / 8> ro(lds0 + own);
-  const TrFragOffsets<D / 8, KSlots::kAccum> to(lds0 + own);
+  RowFragOffsets<D / 8> ro(lds0 + own);
+  TrFragOffsets<D / 8, KSlots::kAccum> to(lds0 + own);
+  // (Opaque from here on: the compiler otherwise forms the fragments' addresses again in every step.)
+  if constexpr (D == 64) {
+#pragma unroll
+    for (int k = 0; k < D / 16; ++k) asm volatile("" : "+v"(ro.ptr[k]));
+#pragma unroll
+    for (int second = 0; second < 2; ++second)
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) asm volatile("" : "+v"(to.ptr[second][db]));
+  }
 
   // KB x 32 keys from `key0` on, at byte offset OFF of this wavefront's keys in LDS
   auto piece = [&](auto off_tag, const KeyTileBounds& keys, int key0, lds_addr ids) {
@@ -165,7 +178,7 @@ attn_fwd_split_kernel(AttnParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[i][r]);
     mx = pair_max(mx) * kLog2e;
-    if (__any(mx > m_run + kRescaleSlack)) {  // (lazily, as attn_fwd_item)
+    if (__any(mx > (D == 64 ? moves_at : m_run + kRescaleSlack))) {  // (lazily, as attn_fwd_item)
       const float m_new = fmaxf(m_run, mx);
       const float alpha = exp2_fast(m_run - (m_new == kNegInf ? 0.f : m_new));
       l_run *= alpha;
@@ -174,14 +187,16 @@ attn_fwd_split_kernel(AttnParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
       m_run = m_new;
+      moves_at = m_new + kRescaleSlack;
+      minus_m = m_new == kNegInf ? 0.f : -m_new;
     }
-    const float m_use = m_run == kNegInf ? 0.f : m_run;
-    float psum = 0.f;
+    const float minus = D == 64 ? minus_m : m_run == kNegInf ? 0.f : -m_run;
+    float psum = D == 64 ? -0.f : 0.f;  // (the neutral element, so that the first addition falls away)
 #pragma unroll
     for (int i = 0; i < KB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s[i][r] = exp2_fast(fmaf(s[i][r], kLog2e, -m_use));
+        s[i][r] = exp2_fast(fmaf(s[i][r], kLog2e, minus));
         psum += s[i][r];
       }
     l_run += psum;
