@@ -4,8 +4,8 @@
 // One workgroup of NW wavefronts per query tile, launched heaviest tile first and dealt by the
 // hardware. Nothing runs in step across workgroups: what one of them spends on its prologue, its row
 // maxima and its stores is another one's time on the matrix pipe, and no hand-written interleaving is
-// needed. At head dimension 64 the loop is bound by the vector ALU (about 230 instructions and 32
-// exponentials against 16 MFMAs per 64 keys), and 4 wavefronts per SIMD at 103 registers keep it
+// needed. At head dimension 64 the loop is bound by the vector ALU (about 140 instructions, 32 of them
+// exponentials, against 16 MFMAs per 64 keys), and 4 wavefronts per SIMD at 103 registers keep it
 // busy; the 8-wavefront workgroup in two half-step-shifted groups that this replaces had 2. The forms:
 //
 //   KS = 1  a wavefront takes all keys of its 32 query rows
