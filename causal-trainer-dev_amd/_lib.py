@@ -21,7 +21,7 @@ CT_WORKSPACE_TOO_SMALL = -3
 CT_LAUNCH_FAILED = -4
 
 ATTN_META_WIDTH = 12
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 # ct_attn_bwd_args.variant (0 = every choice left to the library)
 ATTN_BWD_DKV_NARROW = 1
@@ -158,8 +158,8 @@ SYMBOLS = {
     "ct_cutce_fwd": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
     "ct_cutce_bwd": (c_int32, [c_void_p, POINTER(CutceBwdArgs)]),
     "ct_cutce_panel_bytes": (c_size_t, [POINTER(CutceShape)]),
-    "ct_cutce_fwd_panel": (c_int32, [c_void_p, POINTER(CutceFwdArgs), c_void_p, c_int32]),
-    "ct_cutce_bwd_panel": (c_int32, [c_void_p, POINTER(CutceBwdArgs), c_void_p]),
+    "ct_cutce_fwd_panel": (c_int32, [c_void_p, POINTER(CutceFwdArgs), c_void_p, c_size_t, c_int32]),
+    "ct_cutce_bwd_panel": (c_int32, [c_void_p, POINTER(CutceBwdArgs), c_void_p, c_size_t]),
     "ct_cutce_fwd_noalloc_max_bytes": (c_size_t, []),
     "ct_cutce_fwd_noalloc": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
 }

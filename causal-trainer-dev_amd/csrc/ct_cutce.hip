@@ -1571,11 +1571,29 @@ static int launch_grads(const char* fn, hipStream_t stream, const CutceParams& p
   return scope.done();
 }
 
+// The panel and the logits cache that a caller lends. A cache has room for a panel behind its logits, which a
+// forward with a lent panel would leave unwritten, so with one the cache ends behind the logits: the entries
+// without a panel refuse it as too small.
+static int validate_lent(const char* fn, const ct_cutce_shape& s, const void* panel, size_t panel_bytes, const void* cache,
+                         size_t cache_bytes) {
+  const bool lent = panel && needs_panel(s);
+  CT_REQUIRE(!lent || is_aligned16(panel), "%s: panel must be 16-byte aligned", fn);
+  if (lent && panel_bytes < full_panel_bytes(s))
+    return fail(CT_WORKSPACE_TOO_SMALL, "%s: panel %zu < %zu bytes", fn, panel_bytes, full_panel_bytes(s));
+  if (!cache) return CT_OK;
+  CT_REQUIRE(is_aligned16(cache), "%s: logits cache must be 16-byte aligned", fn);
+  const size_t need = logits_bytes(s) + (lent ? 0 : full_panel_bytes(s));
+  if (cache_bytes < need) return fail(CT_WORKSPACE_TOO_SMALL, "%s: logits cache %zu < %zu bytes", fn, cache_bytes, need);
+  CT_REQUIRE(!lent || cache_bytes == need, "%s: beside a panel the logits cache is %zu bytes, without room for one, not %zu", fn,
+             need, cache_bytes);
+  return CT_OK;
+}
+
 // Shared body of ct_cutce_fwd and ct_cutce_fwd_noalloc: `ws` / `ws_bytes` is the workspace to use
 // (the caller's, or this device's static scratch array), `fn` the name for error texts.
 // `lent`: the caller's panel or null, made here unless `filled`.
 static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_, size_t ws_bytes,
-                            const char* fn, bf16* lent = nullptr, bool filled = false) {
+                            const char* fn, bf16* lent = nullptr, size_t lent_bytes = 0, bool filled = false) {
   CT_REQUIRE(a->hidden && a->head && a->targets && a->weights && a->nll_sum && a->weight_sum &&
                  a->lse && ws_,
              "%s: null pointer", fn);
@@ -1585,12 +1603,7 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   if (ws_bytes < L.base)
     return fail(CT_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu bytes", fn, ws_bytes, L.base);
   CT_REQUIRE(is_aligned16(ws_), "%s: workspace must be 16-byte aligned", fn);
-  if (a->logits_cache) {
-    CT_REQUIRE(is_aligned16(a->logits_cache), "%s: logits cache must be 16-byte aligned", fn);
-    if (a->logits_cache_bytes < ct_cutce_logits_cache_bytes(&a->shape))
-      return fail(CT_WORKSPACE_TOO_SMALL, "%s: logits cache %zu < %zu bytes", fn,
-                  a->logits_cache_bytes, ct_cutce_logits_cache_bytes(&a->shape));
-  }
+  if ((rc = validate_lent(fn, a->shape, lent, lent_bytes, a->logits_cache, a->logits_cache_bytes))) return rc;
   hipStream_t stream = (hipStream_t)stream_;
   char* ws = static_cast<char*>(ws_);
   CutceParams p = make_params(a->hidden, a->head, a->targets, a->weights, a->shape, a->sparse_compaction, ws);
@@ -1610,7 +1623,6 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     lent = nullptr;
   } else {
     if (lent) {
-      CT_REQUIRE(is_aligned16(lent), "%s: panel must be 16-byte aligned", fn);
       panel = lent;
     } else if (a->logits_cache) {
       panel = reinterpret_cast<bf16*>(static_cast<char*>(a->logits_cache) + logits_bytes(a->shape));
@@ -1702,14 +1714,16 @@ extern "C" size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape) {
   return valid_sizes(shape) ? full_panel_bytes(*shape) : 0;
 }
 
-extern "C" int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* a, uint16_t* panel, int32_t filled) {
+extern "C" int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* a, uint16_t* panel, size_t panel_bytes,
+                                      int32_t filled) {
   CT_REQUIRE(a, "ct_cutce_fwd: null args");
-  return cutce_fwd_on(stream, a, a->workspace, a->workspace_bytes, "ct_cutce_fwd", reinterpret_cast<bf16*>(panel), filled != 0);
+  return cutce_fwd_on(stream, a, a->workspace, a->workspace_bytes, "ct_cutce_fwd", reinterpret_cast<bf16*>(panel), panel_bytes,
+                      filled != 0);
 }
 
-extern "C" int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* a) { return ct_cutce_bwd_panel(stream, a, nullptr); }
+extern "C" int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* a) { return ct_cutce_bwd_panel(stream, a, nullptr, 0); }
 
-extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a, const uint16_t* lent) {
+extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a, const uint16_t* lent, size_t lent_bytes) {
   CT_REQUIRE(a, "ct_cutce_bwd: null args");
   CT_REQUIRE(a->hidden && a->head && a->targets && a->weights && a->lse && a->dy && a->dhidden &&
                  a->workspace,
@@ -1719,7 +1733,7 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
   if (rc) return rc;
   CT_REQUIRE(is_aligned16(a->workspace) && is_aligned16(a->dhidden),
              "ct_cutce_bwd: workspace and dhidden must be 16-byte aligned");
-  CT_REQUIRE(is_aligned16(lent), "ct_cutce_bwd: panel must be 16-byte aligned");
+  if ((rc = validate_lent("ct_cutce_bwd", a->shape, lent, lent_bytes, a->logits_cache, a->logits_cache_bytes))) return rc;
   const BwdLayout L = bwd_layout(a->shape, a->workspace_bytes, lent || a->logits_cache, a->dhead != nullptr);
   if (L.slab_cols == 0)
     return fail(CT_WORKSPACE_TOO_SMALL, "ct_cutce_bwd: workspace %zu < %zu bytes",
@@ -1732,12 +1746,6 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
   bf16* dhidden = reinterpret_cast<bf16*>(a->dhidden);
   bf16* dhead = reinterpret_cast<bf16*>(a->dhead);
   const float* cache = static_cast<const float*>(a->logits_cache);
-  if (cache) {
-    CT_REQUIRE(is_aligned16(cache), "ct_cutce_bwd: logits cache must be 16-byte aligned");
-    if (a->logits_cache_bytes < ct_cutce_logits_cache_bytes(&a->shape))
-      return fail(CT_WORKSPACE_TOO_SMALL, "ct_cutce_bwd: logits cache %zu < %zu bytes",
-                  a->logits_cache_bytes, ct_cutce_logits_cache_bytes(&a->shape));
-  }
   const int row_blocks = p.n_pad / kGemmTile;
   const size_t params_stride = align_up((size_t)p.n_pad * sizeof(int), 256);
   CutceRowParams rp;

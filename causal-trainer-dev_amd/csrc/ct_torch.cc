@@ -549,7 +549,7 @@ std::tuple<Tensor, Tensor, Tensor> cutce_forward_on(const ct_cutce_shape& shape,
   a.sparse_compaction = compaction;
   a.logits_cache = cached ? cache->data_ptr() : nullptr;
   a.logits_cache_bytes = cached ? (size_t)cache->numel() : 0;
-  check(ct_cutce_fwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr, filled));
+  check(ct_cutce_fwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr, panel ? panel->nbytes() : 0, filled));
   return {nll, weight_sum, lse};
 }
 std::tuple<Tensor, Tensor, Tensor> cutce_forward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
@@ -585,7 +585,7 @@ std::tuple<Tensor, MaybeTensor> cutce_backward_on(const ct_cutce_shape& shape, c
   a.sparse_compaction = compaction;
   a.logits_cache = cached ? cache->data_ptr() : nullptr;
   a.logits_cache_bytes = cached ? (size_t)cache->numel() : 0;
-  check(ct_cutce_bwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr));
+  check(ct_cutce_bwd_panel(current_stream(), &a, panel ? bits(*panel) : nullptr, panel ? panel->nbytes() : 0));
   return {dhidden, dhead};
 }
 std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tensor& head, const Tensor& targets,
@@ -663,7 +663,7 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
   }
   MaybeTensor cache, panel;
   if (use_cache && graph) {
-    const size_t bytes = ct_cutce_logits_cache_bytes(&shape);
+    const size_t bytes = ct_cutce_logits_cache_bytes(&shape) - (head_is_panel ? panel_bytes : 0);
     if ((int64_t)bytes <= cache_limit && cache_pays(shape)) cache = scratch(bytes, hidden);
   }
   // An unaligned head is copied once for both directions where the copy is at most kPanelLimit (it lives as long as

@@ -526,10 +526,12 @@ int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* args);
  * (16-byte aligned, ct_cutce_panel_bytes() long): the forward fills it unless it is `filled` already (by
  * ct_transpose16_padded from a [vocab, hidden] head, or by an earlier call with the same head), the backward reads it.
  * args->head is then not read, and the workspaces are smaller by its size. A panel where none is needed is ignored.
+ * A logits cache beside a panel has no room for another one: exactly ct_cutce_logits_cache_bytes() less
+ * ct_cutce_panel_bytes(); any other size is refused, and ct_cutce_bwd without the panel refuses such a cache.
  */
 size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape);
-int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* args, uint16_t* panel, int32_t filled);
-int32_t ct_cutce_bwd_panel(void* stream, const ct_cutce_bwd_args* args, const uint16_t* panel);
+int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* args, uint16_t* panel, size_t panel_bytes, int32_t filled);
+int32_t ct_cutce_bwd_panel(void* stream, const ct_cutce_bwd_args* args, const uint16_t* panel, size_t panel_bytes);
 
 #ifdef __cplusplus
 }

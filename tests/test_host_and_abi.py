@@ -104,6 +104,45 @@ def test_cutce_backward_refuses_strides_beyond_its_32_bit_offsets(ct):
         assert library.ct_cutce_bwd(None, ctypes.byref(args)) == status, (rows, vocab, dhead, library.ct_last_error())
 
 
+def test_cutce_panel_and_logits_cache_cannot_be_mixed_up(ct):
+    """A forward with a lent panel writes no panel into its logits cache: the cache it takes is one that the backward
+    without a panel refuses, and the other way round. A panel that is too short is refused too. (No workspace or a
+    misaligned output ends the calls that get past these checks, so nothing is launched.)"""
+
+    library, shape = ct._lib.load(), ct._lib.CutceShape(10, 128, 1031)
+    query = lambda name: int(getattr(library, name)(ctypes.byref(shape)))  # noqa: E731
+    panel, with_panel = query("ct_cutce_panel_bytes"), query("ct_cutce_logits_cache_bytes")
+    assert panel == 128 * 1280 * 2 and with_panel == 256 * 1280 * 4 + panel
+    forward = ct._lib.CutceFwdArgs(shape=shape, logits_cache=4096, workspace_bytes=query("ct_cutce_fwd_workspace_bytes"))
+    for field in ("hidden", "head", "targets", "weights", "nll_sum", "weight_sum", "lse", "workspace"):
+        setattr(forward, field, 4096)       # never dereferenced: validation fails first
+    backward = ct._lib.CutceBwdArgs(shape=shape, logits_cache=4096, workspace_bytes=16)
+    for field in ("hidden", "head", "targets", "weights", "lse", "dy", "dhidden", "workspace"):
+        setattr(backward, field, 4096)
+    refused, short, misaligned = ct._lib.CT_INVALID_ARGUMENT, ct._lib.CT_WORKSPACE_TOO_SMALL, 4096 + 2
+
+    def run(cache_bytes, lent, lent_bytes):
+        forward.logits_cache_bytes = backward.logits_cache_bytes = cache_bytes
+        return (library.ct_cutce_fwd_panel(None, ctypes.byref(forward), lent, lent_bytes, 1),
+                library.ct_cutce_bwd_panel(None, ctypes.byref(backward), lent, lent_bytes))
+
+    for cache_bytes in (with_panel, with_panel - panel + 16, 2 * with_panel):
+        assert run(cache_bytes, 4096, panel) == (refused, refused)
+        assert b"without room for one" in library.ct_last_error()
+    assert run(with_panel - panel - 16, 4096, panel) == (short, short)
+    assert run(with_panel - panel, 4096, panel - 2) == (short, short)
+    assert b"panel" in library.ct_last_error()
+    assert run(with_panel - panel, misaligned, panel) == (refused, refused)
+    assert run(with_panel - panel, None, 0) == (short, short)         # what a forward with a panel has filled
+    assert b"logits cache" in library.ct_last_error()
+    assert library.ct_cutce_bwd(None, ctypes.byref(backward)) == short and b"logits cache" in library.ct_last_error()
+    # the sizes that belong together pass these checks: the backward gets as far as its workspace
+    for cache_bytes, lent, lent_bytes in ((with_panel - panel, 4096, panel), (with_panel, None, 0)):
+        backward.logits_cache_bytes = cache_bytes
+        assert library.ct_cutce_bwd_panel(None, ctypes.byref(backward), lent, lent_bytes) == short
+        assert b"workspace" in library.ct_last_error()
+
+
 @pytest.mark.parametrize("torch_side", ["absent", "broken", "there"])
 def test_library_is_linked_whatever_becomes_of_the_torch_side(monkeypatch, tmp_path, torch_side):
     """libct_hotpath.so needs hipcc only: it is linked without torch, and before a torch side that fails to compile
