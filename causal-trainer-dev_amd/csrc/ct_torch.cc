@@ -595,9 +595,10 @@ std::tuple<Tensor, MaybeTensor> cutce_backward(const Tensor& hidden, const Tenso
                            workspace_bytes, cache, std::nullopt);
 }
 
-// The reference's residual (src/causal_trainer/kernels/cut_cross_entropy.py:587-593) plus, when it
-// fits, the f32 logits cache, which the first backward gives back, and the aligned copy that the forward has
-// read an unaligned head from, or for a [V, d] head (whose `head` is then this copy) in the place of a plain transposed one.
+// The reference's residual (src/causal_trainer/kernels/cut_cross_entropy.py:587-593), for a [V, d] head with its transposed
+// copy (a panel where the vocabulary is unaligned) in the head's place. Where the caller lets the operator keep more
+// than that (use_cache), one of two buffers that the first backward gives back: the f32 logits cache, or the panel that
+// the forward has read an unaligned head from.
 struct CutCeNode : OperatorNode {
   SavedVariable hidden, head, targets, weights, lse;
   MaybeTensor cache, panel;
@@ -633,9 +634,9 @@ struct CutCeNode : OperatorNode {
 // 4096 x 3200, 512: 113 / 114, 1024: 147 / 159; 130 x 76000, 512: 163 / 165.
 bool cache_pays(const ct_cutce_shape& shape) { return shape.hidden > 768; }
 
-// Train steps, us: 281 rows x 1152 x 105348 611 -> 538, 50 x 896 x 74295 270 -> 223; a [35263, 7552] head and 21 rows, whose
-// transposed copy was copied again in each direction, 1365 -> 815.
-constexpr size_t kPanelLimit = (size_t)1 << 30;
+// The largest panel that is kept. Train steps, us, panel kept / made by each direction: 1000 rows x 32003, hidden 512: 192 / 199,
+// 768: 256 / 263; 300 x 105349, 256: 240 / 252; 4096 x 50257, 768: 1094 / 1136; 50 x 74295, 768: 246 / 285.
+constexpr int64_t kPanelLimit = (int64_t)1 << 30;
 
 // vocab_major: head is [V, d]; the kernels get a transposed copy, the gradient goes back as a view of theirs.
 std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Tensor& head, const Tensor& targets,
@@ -652,7 +653,8 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
   const int64_t width = hidden.size(2);
   const ct_cutce_shape shape = {(int32_t)(hidden.numel() / width), (int32_t)width, (int32_t)head.size(vocab_major ? 0 : 1)};
   const c10::DeviceGuard guard(head.device());
-  // (a bounded workspace: the copies keep to it)
+  // (A bounded workspace: the copies keep to it. A [V, d] head is otherwise transposed straight into a panel: [35263, 7552] and
+  // 21 rows 1366 -> 875 us, its plain transposed copy was copied again by each direction.)
   const size_t panel_bytes = forward_bytes < 0 ? ct_cutce_panel_bytes(&shape) : 0;
   const bool head_is_panel = vocab_major && panel_bytes;
   Tensor columns = head;  // [d, V], padded in a panel
@@ -666,10 +668,11 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
     const size_t bytes = ct_cutce_logits_cache_bytes(&shape) - (head_is_panel ? panel_bytes : 0);
     if ((int64_t)bytes <= cache_limit && cache_pays(shape)) cache = scratch(bytes, hidden);
   }
-  // An unaligned head is copied once for both directions where the copy is at most kPanelLimit (it lives as long as
-  // the other residuals; the peak is what it was, each direction had one in its workspace).
+  // An unaligned head is copied once for both directions only where the caller lets a buffer be kept between them, like
+  // the logits cache, which holds such a copy itself. Otherwise each direction makes one in its workspace.
   if (head_is_panel) panel = columns;
-  else if (graph && !cache && panel_bytes && panel_bytes <= kPanelLimit) panel = scratch(panel_bytes, hidden);
+  else if (use_cache && graph && !cache && panel_bytes && (int64_t)panel_bytes <= std::min(kPanelLimit, cache_limit))
+    panel = scratch(panel_bytes, hidden);
   auto [nll, weight_sum, lse] =
       cutce_forward_on(shape, hidden, columns, targets, weights, compaction, cache, forward_bytes, panel, head_is_panel);
   if (graph) {

@@ -18,9 +18,12 @@ a TPU core has little memory, and pays for it by recomputing the projection in
 each backward kernel. A MI355X has 288 GB: when the f32 logits of the active
 rows fit in ``LOGITS_CACHE_LIMIT_BYTES`` the forward also leaves them in a cache
 that lives until the backward of the loss (the adjacent step of a training
-iteration), and the backward then runs 3 GEMMs instead of 4. Above the limit, where
-the projection is cheaper than the cache's traffic (small hidden sizes), or with
-``logits_cache=False``, no logits are kept and they are recomputed.
+iteration), and the backward then runs 3 GEMMs instead of 4. Above the limit, or where
+the projection is cheaper than the cache's traffic (small hidden sizes), the logits are
+recomputed, and what is kept in the cache's place is the aligned copy that a head whose
+vocabulary is no multiple of 8 is read through, up to the limit and 1 GiB. Like the cache it
+is no saved tensor (hooks do not see it) and goes with the first backward. With
+``logits_cache=False`` nothing but ``lse`` is kept: logits and copy are made again.
 
 ``local_chunk_size`` (:697-825). The reference's chunk loop bounds what one TPU core holds at
 a time: it walks the rows in chunks, compacts inside the chunk and accumulates the head
@@ -131,8 +134,8 @@ def pallas_cut_linear_cross_entropy(hidden_states, lm_head_kernel, targets, weig
                                     lm_head_trainable: bool = True, local_chunk_size: int = 0,
                                     logits_cache: bool = True, head_layout: str = "dv"):
     """Return ``(nll_sum, weight_sum)``; logits are only ever kept in the bounded cache
-    described in the module docstring (``logits_cache=False`` disables it). A head whose vocabulary is no multiple
-    of 8 is read through an aligned copy; one of up to 1 GiB that the forward made is left to the backward.
+    described in the module docstring, which also says what is kept where it does not pay
+    (``logits_cache=False``: nothing but the residuals of the module docstring's first paragraph).
 
     hidden_states ``[B, S, d]``, lm_head_kernel ``[d, V]`` (same float dtype, bf16),
     targets int32 ``[B, S]``, weights f32 ``[B, S]``; a row is ignored iff its weight is 0.

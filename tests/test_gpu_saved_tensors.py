@@ -1,5 +1,6 @@
 """The operators' residuals go through torch's saved-tensor mechanism: hooks (offloading, checkpointing) see each of
-them, and the gradients from what the hooks give back are bit for bit those without hooks."""
+them, and the gradients from what the hooks give back are bit for bit those without hooks. What Cut cross-entropy keeps
+besides under ``logits_cache=True`` (logits, or an aligned copy of the head) is no residual; without it there is nothing."""
 
 import pytest
 import torch
@@ -71,3 +72,32 @@ def test_residuals_pass_the_saved_tensor_hooks(ct, gpu, name):
     recomputed = gradients(lambda: checkpoint(function, *inputs, use_reentrant=False))
     for other in (offloaded, recomputed):
         assert all(torch.equal(a, b) for a, b in zip(expected, other))
+
+
+@pytest.mark.parametrize("vocab,layout", [(512, "dv"), (515, "dv"), (515, "vd")])
+def test_cut_ce_without_a_logits_cache_keeps_its_residuals_only(ct, gpu, vocab, layout):
+    """Device memory held between the two directions, with an aligned head and with one that the kernels copy: the
+    outputs and ``lse`` (of a [V, d] head also the transposed copy, which is its residual), and under hooks that
+    offload every residual the outputs alone."""
+
+    rows, hidden = 512, 256
+    generator = torch.Generator(device=gpu).manual_seed(3)
+    normal = lambda *shape: torch.randn(shape, generator=generator, device=gpu, dtype=torch.bfloat16)  # noqa: E731
+    x = normal(1, rows, hidden).requires_grad_(True)
+    head = (normal(hidden, vocab) if layout == "dv" else normal(vocab, hidden)).requires_grad_(True)
+    targets = torch.randint(vocab, (1, rows), generator=generator, device=gpu, dtype=torch.int32)
+    weights = torch.ones((1, rows), device=gpu)
+
+    def kept():
+        before = torch.cuda.memory_allocated()
+        outputs = ct.pallas_cut_linear_cross_entropy(x, head, targets, weights, logits_cache=False, head_layout=layout)
+        held = torch.cuda.memory_allocated() - before
+        torch.autograd.grad(outputs[0], (x, head))
+        return held
+
+    kept()                                  # (what a first call sets up for good)
+    outputs = 2 * 512                       # two scalars, in the allocator's units of 512 bytes
+    transposed = 2 * hidden * 768 if layout == "vd" else 0      # rows padded to a multiple of 256
+    assert kept() == outputs + 4 * rows + transposed
+    with torch.autograd.graph.saved_tensors_hooks(lambda tensor: tensor.cpu(), lambda tensor: tensor.to(gpu)):
+        assert kept() == outputs
