@@ -476,18 +476,6 @@ CT_DEVICE void merge_stats(float& m, float& s, float m_o, float s_o) {
   m = m_new;
 }
 
-// The rows of a wavefront's tile in the order of its accumulators (0..3, 8..11, ...; lanes of the other half
-// are 4 rows on), as a scalar address that advances. The stride is opaque: as a loop invariant its
-// 64 multiples are formed in front of the persistent loop and spilled.
-struct TileRows {
-  char* row;
-  int stride;  // bytes
-  CT_DEVICE TileRows(void* origin, int stride_) : row(reinterpret_cast<char*>(origin)), stride(uniform(stride_)) {
-    asm volatile("" : "+s"(stride));
-  }
-  CT_DEVICE void advance(int r) { row += (long)stride * ((r & 3) == 3 ? 5 : 1); }
-};
-
 // Bound by the matrix pipe at long contractions; at short ones by what lies between two products, for the large tile
 // has its compute unit to itself. In clocks a tile, 4096 x 32000 at d = 256: product 10.1 k (8.2 k of MFMAs), first
 // copies of the next tile 2.5 k (96 KB at 64 bytes a clock), epilogue 8.5 k, end of a unit 2.4 k; the copies'
@@ -520,7 +508,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
   bool more = next_unit(chunk, rb);
   McLoader<NB> A;
   KcLoader<NB> B;
-  GemmTiles<NB, GUARDED, CACHE ? 16 * NB : 0> gemm;
+  GemmTiles<NB, GUARDED, CACHE> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
   typedef int LaneInts __attribute__((ext_vector_type(NB)));
@@ -570,10 +558,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            store_lane(rows.row, lane_off, acc.lane(i, r));
-            rows.advance(r);
-          }
+          for (int r = 0; r < 16; ++r) gemm.store(rows, lane_off, r, acc.lane(i, r));
       }
       // A column block's 16 NB elements are read once. (The limit is opaque: comparison masks kept for the next
       // block do not fit and spill, and so is every 16 elements' result, or their use is put off past a branch.)
@@ -774,7 +759,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
   bool more = units.next(chunk, rb, &unit_s);
   McLoader<NB> A;
   KcLoader<NB> B;
-  GemmTiles<NB, GUARDED, 16 * NB> gemm;
+  GemmTiles<NB, GUARDED, true> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
   LaneFloats next_fac, next_lse2;
@@ -822,8 +807,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) x[nb] = fac[nb] * exp2_fast(x[nb] * kLog2e - lse2[nb]);
             if (ragged_tile.value && 32 * i + acc_row(r, 0) >= limit) x = LaneFloats{};
-            store_lane(rows.row, lane_off, to_bf16(x));
-            rows.advance(r);
+            gemm.store(rows, lane_off, r, to_bf16(x));
           }
       };
       if (v0 + kTile > p.V) store(std::true_type{});

@@ -260,7 +260,8 @@ CT_DEVICE void workgroup_barrier() { __builtin_amdgcn_s_barrier(); }
 // The pipelined main loop with a fixed instruction order (see gen_gemm_asm.py), for an
 // m-contiguous A, a k-contiguous B and a step count that is a positive multiple of 4. Entered with the copies of steps 0..2 issued and step 0 landed for every
 // wavefront; returns with nothing in flight and the LDS tiles free. It adds to the accumulators (kAdd) or writes them
-// (kFresh; kFreshBehindStores: at least 51 stores of every wavefront follow the copies of step 2, or these have landed).
+// (kFresh; kFreshBehindStores: at least kStoresBehindCopies stores of every wavefront follow the copies of step 2, or
+// these have landed).
 enum class GemmStart { kAdd, kFresh, kFreshBehindStores };
 CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned long long b = (unsigned long long)(uintptr_t)p;
@@ -312,16 +313,16 @@ CT_DEVICE void gemm_copy_ahead(const McLoader<4>& A, const KcLoader<4>& B, lds_a
 }
 
 // acc = A[m-tile, 0:k_end] * B[n-tile, 0:k_end]^T behind gemm_copy_ahead, k_end a positive multiple of 128. STORES:
-// how many stores every wavefront has issued since, 0 or at least 51; `landed`: it waits for all of the copies instead.
-template <int STORES>
+// every wavefront has issued at least kStoresBehindCopies stores since, or it waits for all of the copies (`landed`).
+constexpr int kStoresBehindCopies = 51;  // what the waits of CT_GEMM_FRESH_LOOP_BEHIND_STORES need (gen_gemm_asm.py)
+template <bool STORES>
 CT_DEVICE void gemm_tile_fresh(const McLoader<4>& A, const KcLoader<4>& B, int k_end, lds_addr smem, GemmAcc<4>& acc, bool landed) {
-  static_assert(STORES == 0 || STORES >= 51, "the waits of the first steps count on it");
   constexpr GemmStart kStart = STORES ? GemmStart::kFreshBehindStores : GemmStart::kFresh;
   const int w = threadIdx.x >> 6;
   const McLoader<4>::FragOffsets afo(smem);
   const KcLoader<4>::FragOffsets bfo(smem);
   // step 0's copies: at least 16 + 51 others behind them, or the 16 of steps 1 and 2
-  if (STORES == 0) wait_vmcnt16();
+  if (!STORES) wait_vmcnt16();
   else if (landed) dma_wait_all();
   else asm volatile("s_waitcnt vmcnt(63)" ::: "memory");
   workgroup_barrier();
@@ -449,21 +450,43 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
   }
 }
 
+// The rows of a wavefront's tile in the order of its accumulators (0..3, 8..11, ...; lanes of the other half
+// are 4 rows on), as a scalar address that advances. The stride is opaque: as a loop invariant its
+// 64 multiples are formed in front of the persistent loop and spilled.
+struct TileRows {
+  char* row;
+  int stride;  // bytes
+  CT_DEVICE TileRows(void* origin, int stride_) : row(reinterpret_cast<char*>(origin)), stride(uniform(stride_)) {
+    asm volatile("" : "+s"(stride));
+  }
+  CT_DEVICE void advance(int r) { row += (long)stride * ((r & 3) == 3 ? 5 : 1); }
+};
+
 // The tiles of a kernel one after the other: begin() as soon as a tile's loaders are known (the LDS stages are
-// free from the end of the last run() on), run() for its product. In the large tile's pipelined form the copies
-// of its first three steps then travel behind the epilogue of the tile before: with one workgroup on a
-// compute unit nothing else hides them.
-template <int NB, bool GUARDED, int STORES>
+// free from the end of the last run() on), run() for its product, store() for the rows that an epilogue writes.
+// In the large tile's pipelined form the copies of a tile's first three steps then travel behind the epilogue of
+// the tile before: with one workgroup on a compute unit nothing else hides them. What run() waits for goes by the
+// stores counted since begin() (a constant wherever an epilogue issues them on every path): where they are too
+// few for the counted waits, as on a kernel's first tile, it waits for all copies.
+template <int NB, bool GUARDED, bool STORES>
 struct GemmTiles {
   static constexpr bool kAhead = NB == 4 && !GUARDED;
-  bool landed = true;  // the first tile's copies have no stores behind them
+  int stores = 0;  // of this wavefront behind the copies of begin()
   CT_DEVICE void begin(const McLoader<NB>& A, const KcLoader<NB>& B, lds_addr smem) {
     if constexpr (kAhead) gemm_copy_ahead(A, B, smem);
   }
+  // a lane's NB consecutive elements of accumulator row r of a block (wave-uniform control flow only)
+  template <class Elements>
+  CT_DEVICE void store(TileRows& rows, unsigned lane_offset, int r, Elements x) {
+    static_assert(STORES, "a kernel that stores this way waits by their count");
+    store_lane(rows.row, lane_offset, x);
+    rows.advance(r);
+    if constexpr (kAhead) ++stores;
+  }
   CT_DEVICE void run(McLoader<NB>& A, KcLoader<NB>& B, int k_end, lds_addr smem, GemmAcc<NB>& acc) {
     if constexpr (kAhead) {
-      gemm_tile_fresh<STORES>(A, B, k_end, smem, acc, landed);
-      landed = false;
+      gemm_tile_fresh<STORES>(A, B, k_end, smem, acc, stores < kStoresBehindCopies);
+      stores = 0;
     } else {
       acc.clear();
       gemm_tile<GUARDED>(A, B, 0, k_end, smem, acc);

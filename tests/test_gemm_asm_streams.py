@@ -1,0 +1,306 @@
+"""The main loops that gen_gemm_asm.py emits, run on a model of one wavefront.
+
+The loops count their copies and LDS reads in flight themselves, so a wait that is too weak is a race on LDS that no GPU
+test reliably shows. In the model copies and stores complete in the order of their issue and no sooner than a wait asks for;
+the four wavefronts of a workgroup run the same stream, so what one of them has waited for before a barrier, all have.
+Checked for every instruction: an LDS read finds the copies of its step landed in front of a barrier, a copy goes where
+every read is done in front of a barrier and no other copy is on its way, and every MFMA has the fragments of its step.
+"""
+
+import importlib.util
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "causal-trainer-dev_amd", "csrc")
+GENERATOR = os.path.join(CSRC, "gen_gemm_asm.py")
+
+
+@pytest.fixture(scope="module")
+def gen():
+    spec = importlib.util.spec_from_file_location("gen_gemm_asm", GENERATOR)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+class Tile:
+    """What the operands of a loop's asm statement stand for, and the layout of its LDS stages."""
+
+    def __init__(self, small):
+        self.blocks = 2 if small else 4                     # of a wavefront, in each direction
+        self.chunks = self.blocks                           # copies of a wavefront per operand and step
+        self.ahead = 4 if small else 3                      # steps copied in front of the loop
+        self.stage = 16384 if small else 32768
+        first = self.blocks ** 2                            # (the accumulators are operands 0 ..)
+        self.src = {"%%%d" % first: 0, "%%%d" % (first + 1): 1}
+        self.stride, self.steps, self.lds_wave = ("%%%d" % (first + k) for k in (2, 3, 4))
+        self.reads, self.copies = {}, {}                    # operand -> (matrix, second, block or k-step), (matrix, chunk)
+        at = first + 5
+        for second in range(2):
+            for block in range(self.blocks):
+                self.reads["%%%d" % at] = (0, second, block)
+                at += 1
+        for ks in range(2):
+            self.reads["%%%d" % at] = (1, None, ks)
+            at += 1
+        for matrix in range(2):
+            for chunk in range(self.chunks):
+                self.copies["%%%d" % at] = (matrix, chunk)
+                at += 1
+
+
+class Machine:
+    """One wavefront on a loop of `steps` steps. `stores` lie behind the copies of the first steps; `start_wait`: the
+    vmcnt in front of the loop."""
+
+    # bytes from step to step of the two sources (the first carries into the upper half of the address), and between them
+    STRIDE, HIGH = ((1 << 32) - 4096, 64), 1 << 40
+
+    def __init__(self, tile, steps, fresh, stores, start_wait):
+        self.tile, self.steps, self.fresh = tile, steps, fresh
+        self.scalar, self.scc, self.address, self.fragment = {}, 0, {}, {}
+        self.memory, self.lds_reads = [], []                # in flight, in the order of their issue
+        self.slots, self.mfmas, self.started = {}, 0, set()
+        for step in range(tile.ahead):
+            for matrix in range(2):
+                for chunk in range(tile.chunks):
+                    self._copy(matrix, chunk, step, step)
+        self.memory += [None] * stores
+        self._wait_memory(start_wait)
+        self._barrier()
+
+    # -- events
+    def _copy(self, matrix, chunk, step, stage):
+        slot = self.slots.setdefault((stage, matrix, chunk), dict(state="free", readers=[]))
+        assert slot["state"] != "flying", ("a copy on its way to the same place", stage, matrix, chunk)
+        assert all(reader == "fenced" for reader in slot["readers"]), ("a copy over data being read", stage, matrix, chunk)
+        slot.update(state="flying", step=step, readers=[])
+        self.memory.append(slot)
+
+    def _wait_memory(self, most):
+        assert most <= 63
+        while len(self.memory) > most:
+            slot = self.memory.pop(0)
+            if slot is not None:
+                slot["state"] = "landed"
+
+    def _wait_lds(self):
+        for slots, registers in self.lds_reads:
+            for slot, index in slots:
+                slot["readers"][index] = "done"
+            for register in registers:
+                self.fragment[register][1] = True
+        self.lds_reads = []
+
+    def _barrier(self):
+        for slot in self.slots.values():
+            if slot["state"] == "landed":
+                slot["state"] = "there"
+            slot["readers"] = ["fenced" if reader in ("done", "fenced") else reader for reader in slot["readers"]]
+
+    def _read(self, registers, operand, offset):
+        base, extra = self.address.get(operand, (operand, 0))
+        matrix, second, which = self.tile.reads[base]
+        stage, offset = divmod(offset + extra, self.tile.stage)
+        half = self.tile.stage // 4                         # of one operand's tile
+        if matrix == 0:                                     # rows of the contraction: half of the tile per k-step
+            ks, rest = divmod(offset, half)
+            assert rest == 0, operand
+            block, chunks = which, range(ks * self.tile.chunks // 2, (ks + 1) * self.tile.chunks // 2)
+        else:
+            ks, (block, rest) = which, divmod(offset, 2048)
+            assert rest == 0 and block < self.tile.blocks, operand
+            chunks = range(self.tile.chunks)                # (two of four, by the wavefront)
+        slots = []
+        for chunk in chunks:
+            slot = self.slots[stage, matrix, chunk]
+            assert slot["state"] == "there", ("LDS read ahead of its copies", stage, matrix, chunk, slot["state"])
+            slot["readers"].append("pending")
+            slots.append((slot, len(slot["readers"]) - 1))
+        step = slots[0][0]["step"]
+        assert all(slot["step"] == step for slot, _ in slots)
+        for k, register in enumerate(registers):
+            assert self.fragment.get(register, [None, True])[1], ("register of a read in flight", register)
+            self.fragment[register] = [(matrix, step, ks, block, second if matrix == 0 else k // 2), False]
+        self.lds_reads.append((slots, registers))
+        assert len(self.lds_reads) <= 15
+
+    def _mfma(self, d, a, b, c):
+        blocks = self.tile.blocks
+        per_step = 2 * blocks ** 2
+        step, (ks, (i, j)) = self.mfmas // per_step, (self.mfmas % per_step // blocks ** 2, divmod(self.mfmas % blocks ** 2, blocks))
+        assert d == "%%%d" % (blocks * i + j)
+        for matrix, block, operand in ((0, i, a), (1, j, b)):
+            for k, register in enumerate(_registers(operand)):
+                assert self.fragment[register] == [(matrix, step, ks, block, k // 2), True], (step, d, operand, self.fragment[register])
+        if self.fresh and d not in self.started:
+            assert c == "0"
+        else:
+            assert c == d
+        self.started.add(d)
+        self.mfmas += 1
+
+    # -- scalar instructions
+    def _get(self, operand):
+        if operand in self.tile.src:                        # address of the copies of step 3
+            matrix = self.tile.src[operand]
+            return matrix * self.HIGH + 3 * self.STRIDE[matrix]
+        if operand == self.tile.stride:
+            return self.STRIDE[0]
+        if operand == self.tile.steps:
+            return self.steps
+        if operand == self.tile.lds_wave:
+            return 0
+        if operand.startswith(("s", "m0")):
+            return self.scalar[operand]
+        return int(operand, 0)
+
+    def run(self, lines):
+        labels = {line[:-1]: at for at, line in enumerate(lines) if line.endswith(":")}
+        at = executed = 0
+        while at < len(lines):
+            line = lines[at]
+            at += 1
+            executed += 1
+            assert executed < 100000
+            if line.endswith(":"):
+                continue
+            name, _, rest = line.partition(" ")
+            ops = [part.strip() for part in rest.split(",")]
+            if name == "s_waitcnt":
+                counter, most = re.fullmatch(r"(vmcnt|lgkmcnt)\((\d+)\)", rest).groups()
+                if counter == "vmcnt":
+                    self._wait_memory(int(most))
+                else:
+                    assert int(most) == 0
+                    self._wait_lds()
+            elif name == "s_barrier":
+                self._barrier()
+            elif name.startswith("ds_read"):
+                where, _, offset = ops[1].partition(" offset:")
+                self._read(_registers(ops[0]), where, int(offset))
+            elif name == "global_load_lds_dwordx4":
+                matrix, chunk = self.tile.copies[ops[0]]
+                low = int(re.fullmatch(r"s\[(\d+):\d+\]", ops[1]).group(1))
+                source = (self.scalar["s%d" % (low + 1)] << 32 | self.scalar["s%d" % low]) - matrix * self.HIGH
+                step, rest = divmod(source, self.STRIDE[matrix])
+                assert rest == 0 and 0 <= step < self.steps, ("copy from outside of the matrix", step)
+                stage, where = divmod(self.scalar["m0"], self.tile.stage)
+                assert where == matrix * self.tile.stage // 2 + chunk * 4096
+                self._copy(matrix, chunk, step, stage)
+            elif name == "v_mfma_f32_32x32x16_bf16":
+                self._mfma(*ops)
+            elif name == "v_add_u32":
+                self.address[ops[0]] = (ops[2], int(ops[1], 0))
+            elif name == "s_mov_b64":
+                low, high = re.fullmatch(r"s\[(\d+):(\d+)\]", ops[0]).groups()
+                value = self._get(ops[1])
+                self.scalar["s" + low], self.scalar["s" + high] = value & 0xffffffff, value >> 32
+            elif name == "s_mov_b32":
+                self.scalar[ops[0]] = self._get(ops[1])
+            elif name in ("s_add_u32", "s_addc_u32"):
+                value = self._get(ops[1]) + self._get(ops[2]) + (self.scc if name == "s_addc_u32" else 0)
+                self.scalar[ops[0]], self.scc = value & 0xffffffff, value >> 32
+            elif name == "s_sub_u32":
+                value = self._get(ops[1]) - self._get(ops[2])
+                self.scalar[ops[0]], self.scc = value & 0xffffffff, int(value < 0)
+            elif name == "s_cmp_lt_u32":
+                self.scc = int(self._get(ops[0]) < self._get(ops[1]))
+            elif name == "s_cselect_b32":
+                self.scalar[ops[0]] = self._get(ops[1] if self.scc else ops[2])
+            elif name in ("s_cbranch_scc0", "s_cbranch_scc1"):
+                if self.scc == int(name[-1]):
+                    at = labels[rest]
+            else:
+                assert name == "s_nop", line
+        assert self.mfmas == self.steps * 2 * self.tile.blocks ** 2
+        assert not self.memory and not self.lds_reads
+        # the next tile's copies may go anywhere
+        assert all(reader == "fenced" for slot in self.slots.values() for reader in slot["readers"])
+
+
+def _registers(operand):
+    low, high = re.fullmatch(r"v\[(\d+):(\d+)\]", operand).groups()
+    return range(int(low), int(high) + 1)
+
+
+# loop -> (small tile, from C = 0, vmcnt in front of it, stores that may lie behind the first copies; as in ct_gemm.hip.h)
+LOOPS = {"CT_GEMM_LOOP": (False, False, 16, (0,)), "CT_GEMM_FRESH_LOOP": (False, True, 16, (0,)),
+         "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (51, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 12, (0,))}
+
+
+def _lines(gen, name):
+    return {"CT_GEMM_LOOP": lambda: gen.gemm_loop(), "CT_GEMM_FRESH_LOOP": lambda: gen.gemm_loop(fresh=True),
+            "CT_GEMM_FRESH_LOOP_BEHIND_STORES": lambda: gen.gemm_loop(fresh=True, behind_stores=True),
+            "CT_GEMM_SMALL_LOOP": lambda: gen.small_loop()}[name]()
+
+
+def _run(lines, name, steps, stores, start_wait=None):
+    small, fresh, wait, _ = LOOPS[name]
+    machine = Machine(Tile(small), steps, fresh, stores, wait if start_wait is None else start_wait)
+    machine.run(lines)
+
+
+@pytest.mark.parametrize("name", LOOPS)
+def test_waits_and_fragments(gen, name):
+    lines = _lines(gen, name)
+    for steps in (4, 8, 12, 20):
+        for stores in LOOPS[name][3]:
+            _run(lines, name, steps, stores)
+
+
+def test_copies_that_have_landed_need_no_stores(gen):
+    """A kernel's first tile, and one behind an epilogue with too few stores, wait for all copies in front of the loop."""
+
+    for stores in (0, 7, 50):
+        _run(_lines(gen, "CT_GEMM_FRESH_LOOP_BEHIND_STORES"), "CT_GEMM_FRESH_LOOP_BEHIND_STORES", 8, stores, start_wait=0)
+
+
+def test_fewest_stores_are_what_the_header_waits_by(gen):
+    with open(os.path.join(CSRC, "ct_gemm.hip.h")) as handle:
+        fewest = int(re.search(r"kStoresBehindCopies = (\d+);", handle.read()).group(1))
+    lines = _lines(gen, "CT_GEMM_FRESH_LOOP_BEHIND_STORES")
+    _run(lines, "CT_GEMM_FRESH_LOOP_BEHIND_STORES", 8, fewest)
+    with pytest.raises(AssertionError, match="LDS read ahead of its copies"):
+        _run(lines, "CT_GEMM_FRESH_LOOP_BEHIND_STORES", 8, fewest - 1)
+
+
+@pytest.mark.parametrize("name", LOOPS)
+def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
+    stores = LOOPS[name][3][0]
+    good = _lines(gen, name)
+
+    def broken(change):
+        lines = list(good)
+        change(lines)
+        with pytest.raises(AssertionError):
+            _run(lines, name, 8, stores)
+
+    # every wait for copies, one copy weaker (63 is the largest there is)
+    for at, line in enumerate(good):
+        counted = re.fullmatch(r"s_waitcnt vmcnt\((\d+)\)", line)
+        if counted and 0 < int(counted.group(1)) < 63:
+            broken(lambda lines: lines.__setitem__(at, "s_waitcnt vmcnt(%d)" % (int(counted.group(1)) + 1)))
+    # every barrier and every wait for LDS reads in front of the last ones gone
+    for at, line in enumerate(good[:-6]):
+        if line in ("s_barrier", "s_waitcnt lgkmcnt(0)"):
+            broken(lambda lines: lines.__setitem__(at, "s_nop 0"))
+    # a fragment read from the next stage, and a copy to it
+    first = next(at for at, line in enumerate(good) if line.startswith("ds_read") and line.endswith("offset:0"))
+    broken(lambda lines: lines.__setitem__(first, good[first].replace("offset:0", "offset:%d" % Tile(LOOPS[name][0]).stage)))
+    copy = next(at for at, line in enumerate(good) if line.startswith("s_add_u32 m0"))
+    operand, offset = re.fullmatch(r"s_add_u32 m0, (\S+), (\d+)", good[copy]).groups()
+    other = (int(offset) + Tile(LOOPS[name][0]).stage) % (4 * Tile(LOOPS[name][0]).stage)
+    broken(lambda lines: lines.__setitem__(copy, "s_add_u32 m0, %s, %d" % (operand, other)))
+    # a source that moves on past the last step
+    broken(lambda lines: [lines.__setitem__(at, "s_cselect_b32 s46, 64, 64") for at, line in enumerate(good) if "s_cselect_b32 s46" in line])
+
+
+def test_committed_include_is_what_the_generator_prints():
+    printed = subprocess.run([sys.executable, GENERATOR], capture_output=True, text=True, check=True).stdout
+    with open(os.path.join(CSRC, "ct_gemm_asm.inc")) as handle:
+        assert handle.read() == printed
