@@ -522,16 +522,20 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 // documents from 36 positions to the whole row:
 //   head dimension 64: sharing by four wins up to 512 row blocks (half a wavefront per SIMD), sharing
 //     by two up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47 us).
-//   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920) and with packed documents up to
-//     2304 (us, large launch / by two, documents up to the row, up to 512, whole rows: [1, 4096, 16/16] 45.6 / 36.1,
-//     25.2 / 25.1, 94.3 / 87.8, [2, 1536, 24/8] 36.9 / 28.6, 29.3 / 24.1, 44.7 / 48.7, [1, 3968, 18/6] 55.7 / 38.5, 32.1 /
-//     27.7, 94.4 / 100.1). Above, the large launch's interleaved loop is ahead where rows see 8 key tiles or more
-//     (229 against 242 us), and is behind where they see few (61 against 46 us). The line is where whole-row documents
-//     cost 4 % and goes by the rows that a workgroup of the large launch walks in step: with 4 heads
-//     64 of them, 20 key tiles; with 2 heads 128, 32; with 1 head 256, most of which do not see most of what they wait
-//     for, 64 (us, large / here, documents from 28 to the row, 32 to 256, whole rows: [8, 2048, 32/16] 163 / 159, 120 / 99,
-//     311 / 321, [10, 1408, 24/8] 109 / 82, 92 / 69, 182 / 157, [4, 2944, 24/8] 131 / 112, 84 / 61, 229 / 228,
-//     [4, 4096, 16/16] 126 / 108, 74 / 64, 271 / 282). Images: [6, 2176, 16/16] 132 / 123, 32/16 222 / 231, [4, 4096, 16/16] 191 / 204.
+//   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920); from there to 2304 the longest row's
+//     chain still counts in long rows (large launch / by two: [1, 4096, 16/16] with documents up to the row 58.5 / 42.0),
+//     but whole rows and short ones lose (44.0 / 48.9 at [2, 1536, 24/8], and [4, 768, 24/8] 26.4 by four-wavefront workgroups /
+//     33.3). Above, the large launch's interleaved loop is ahead where rows see 8 key tiles or more
+//     (229 against 242 us), and is behind where they see few (61 against 46 us), which is certain
+//     only for short rows: the line at 20 key tiles per row is where whole-row documents cost 4 %.
+//     The large launch walks 8 row blocks in step: with 4 heads per slice 64 rows, but with 2 heads 128 and with 1 head 256,
+//     most of which do not see most of what they wait for. There the four-wavefront workgroups are ahead in longer rows
+//     too, whatever the documents, where KV heads come in eights (each XCD then has its own heads' K and V in its L2), row
+//     blocks are enough for every place (3072) and not too many (9216). 99 shapes inside these lines (large / here): whole
+//     rows 1.07 times in the geometric mean and 0.995 at least, documents up to the row 1.23 and 1.05, up to 100 positions
+//     1.37 and 1.15. Past each line whole rows lose (us): [8, 2944, 8/8] 148 / 152, [4, 4096, 16/16] 260 / 271, [8, 2048, 32/16]
+//     296 / 314; 12 KV heads, [16, 2560, 12/12] 360 / 396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64]
+//     392 / 417; image blocks in a call with ends, [8, 2304, 8/8] 88 / 103.
 //     Sharing by four takes a compute unit's LDS, so it wins as long as there is a workgroup per compute unit: up to
 //     256 row blocks with one in a workgroup (by two / by four: 33.5 / 22.9 us at 136 with images, 8.9 / 8.5 at 128
 //     short), up to 512 with two (36.9 / 27.6 at 432 with images, 15.1 / 13.6 and, documents up to 300, 12.1 / 11.4 at
@@ -552,9 +556,10 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   } else {
     if (blocks <= 256) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
     if ((blocks <= 512 && p.S > 512) || (images && blocks <= 1024)) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
+    if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     const int hs = heads_per_group(p.Hq, p.Hkv);
-    if (blocks <= (images ? 2047 : 2304)) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
-    const int short_row = hs == 4 ? 20 : images ? (hs == 1 ? 36 : 20) : hs == 2 ? 32 : 64;
+    const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;
+    const int short_row = !local || hs == 4 ? 20 : hs == 2 ? 26 : 40;
     if (p.S <= short_row * kKeyTile) return launch_fwd_split<D, 4, 1, 2, 1>(stream, p);
     switch (hs) {
       case 4: return launch_fwd<D, 4>(stream, p);

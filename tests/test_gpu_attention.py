@@ -403,10 +403,13 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     (1, 2176, 16, 2, 128), (2, 2560, 8, 2, 64), (1, 2048, 20, 20, 64), (1, 2688, 16, 16, 64),
     # 12, 2 and 3 workgroup groups: 2, 4 and 8 workgroups walk a work bin of the large form
     (2, 1408, 24, 12, 128), (24, 1408, 2, 2, 128), (16, 1408, 3, 3, 128),
-    # the same groups where the large form still takes them, and both sides of its lines at D = 128: 2304 row blocks, rows of
-    # 4096 with one head per slice (2304 with ends) and of 2048 with two
+    # the same groups and others in rows of the large form
     (2, 4224, 12, 12, 128), (9, 4224, 2, 2, 128), (6, 4224, 3, 3, 128), (2, 4096, 12, 12, 128), (1, 2304, 32, 32, 128),
-    (2, 2048, 32, 16, 128), (2, 2176, 24, 12, 128), (4, 2304, 9, 9, 128), (4, 2432, 9, 9, 128)],
+    (2, 2048, 32, 16, 128), (2, 2176, 24, 12, 128), (4, 2304, 9, 9, 128), (4, 2432, 9, 9, 128),
+    # calls without ends, KV heads in eights: rows of 2560 positions with one head per slice and of 1664 with two, 3072 and 9216
+    # row blocks
+    (2, 2560, 24, 8, 128), (2, 2688, 24, 8, 128), (2, 1664, 32, 16, 128), (2, 1792, 32, 16, 128), (2, 2048, 24, 8, 128),
+    (2, 1920, 24, 8, 128), (8, 1536, 24, 8, 128), (9, 1408, 24, 8, 128)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_forms_of_the_forward(ct, gpu, shape, with_ends):
