@@ -537,25 +537,21 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     296 / 314; 12 KV heads, [16, 2560, 12/12] 360 / 396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64]
 //     392 / 417; image blocks in a call with ends, [8, 2304, 8/8] 88 / 103.
 //     Sharing by four takes a compute unit's LDS, so it wins as long as there is a workgroup per compute unit: up to
-//     256 row blocks with one in a workgroup (by two / by four: 33.5 / 22.9 us at 136 with images, 8.9 / 8.5 at 128
-//     short), up to 512 with two (36.9 / 27.6 at 432 with images, 15.1 / 13.6 and, documents up to 300, 12.1 / 11.4 at
-//     512), not for rows that have no chain to share (9.1 / 10.0 at 384 of 384 positions); at 576 with
-//     documents up to 80 it is 9.0 / 15.8.
-//   Calls with visible ends have image blocks, so rows see more: two row blocks by four win there up to 1024 (47.7 /
-//     35.5 at 736, 50.1 / 52.2 at 1104, 52.3 / 48.8 at 1280), at head dimension 64 up to 1280 (31.2 / 25.6 at 736,
-//     38.0 / 30.1 at 1280, 33.1 / 32.9 at 1408); with documents up to 100 they lose (7.8 / 9.9 at 1024).
+//     256 row blocks with one in a workgroup (us, by two / by four: 33.5 / 22.9 at 136 with images; at 256, documents up to
+//     the row, 512 and 100: [1, 2048, 4/4] 23.9 / 17.1, 12.8 / 11.1, 8.8 / 8.7, [2, 512, 8/8] 11.8 / 10.1, 12.8 / 11.1, 7.8 / 8.8),
+//     up to 512 with two in rows of 1024 or more ([1, 2048, 8/8] 24.3 / 19.0, 13.2 / 12.4, 9.1 / 10.1, whole rows 33.6 / 25.2).
+//     Shorter rows have less of a chain to share (640 positions, documents up to 640 and 100: 12.9 / 12.2, 7.9 / 9.7), and with
+//     more row blocks short documents lose most ([2, 2048, 8/8] 26.4 / 26.2, 11.0 / 18.7).
 template <int D>
 static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   const long blocks = (long)p.B * p.Hq * (p.S / 32);
-  const bool images = p.end != nullptr && p.S >= 2048;
   if constexpr (D == 64) {
     if (blocks <= 512) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
-    if (images && blocks <= 1280) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
     if (blocks < 7168) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     return launch_fwd_split<D, 4, 1, 1, 2>(stream, p);
   } else {
     if (blocks <= 256) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
-    if ((blocks <= 512 && p.S > 512) || (images && blocks <= 1024)) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
+    if (blocks <= 512 && p.S >= 1024) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
     if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     const int hs = heads_per_group(p.Hq, p.Hkv);
     const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;

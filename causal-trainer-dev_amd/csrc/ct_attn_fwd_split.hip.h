@@ -23,7 +23,7 @@
 //   (3, 4224, 48/8, 64, 2.3)      121.2 -> 68.9  KS = 1     (8, 4096, 32/8, 64, 32)   796 -> 660   KS = 1
 //   (3, 2560, 8/8, 128, 7.8)       55.3 -> 42.0  KS = 2     (6, 1280, 32/16, 128, 0.4) 61.1 -> 46.2  KS = 1
 // Head dimension 128 by four (KS = 2 -> 4; images of 1056 positions): (1, 2176, 2/2) 33.5 -> 22.9 NW = 4,
-//   (1, 2304, 6/1) 36.9 -> 27.6 and (1, 2944, 8/1) 47.7 -> 35.5 NW = 8.
+//   (1, 2304, 6/1) 36.9 -> 27.6 NW = 8.
 #pragma once
 
 #include "ct_attn_kernels.hip.h"

@@ -397,8 +397,7 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     (1, 1024, 16, 8, 64), (9, 128, 15, 5, 64), (2, 384, 48, 6, 64), (7, 1024, 30, 5, 64), (7, 1024, 32, 8, 64),
     (8, 1024, 28, 14, 64), (8, 1024, 28, 28, 64), (2, 1024, 30, 10, 128), (1, 1920, 32, 4, 128), (2, 1024, 32, 4, 128),
     (2, 1280, 26, 13, 128), (2, 1280, 26, 26, 128),
-    # keys shared by four at D = 128 (256 and 512 row blocks, rows above 512) and, in calls with ends and rows from 2048
-    # on, in workgroups of two row blocks (1024 for D = 128, 1280 for D = 64)
+    # keys shared by four at D = 128 (256 row blocks, and 512 in rows from 1024 on) and by two past these lines
     (2, 128, 32, 8, 128), (1, 1152, 8, 4, 128), (2, 1024, 8, 8, 128), (3, 768, 7, 7, 128), (1, 2048, 16, 4, 128),
     (1, 2176, 16, 2, 128), (2, 2560, 8, 2, 64), (1, 2048, 20, 20, 64), (1, 2688, 16, 16, 64),
     # 12, 2 and 3 workgroup groups: 2, 4 and 8 workgroups walk a work bin of the large form
@@ -409,7 +408,9 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     # calls without ends, KV heads in eights: rows of 2560 positions with one head per slice and of 1664 with two, 3072 and 9216
     # row blocks
     (2, 2560, 24, 8, 128), (2, 2688, 24, 8, 128), (2, 1664, 32, 16, 128), (2, 1792, 32, 16, 128), (2, 2048, 24, 8, 128),
-    (2, 1920, 24, 8, 128), (8, 1536, 24, 8, 128), (9, 1408, 24, 8, 128)],
+    (2, 1920, 24, 8, 128), (8, 1536, 24, 8, 128), (9, 1408, 24, 8, 128),
+    # 448 and 512 row blocks in rows of 896 and 1024 positions
+    (1, 896, 16, 16, 128), (1, 1024, 16, 8, 128)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_forms_of_the_forward(ct, gpu, shape, with_ends):
