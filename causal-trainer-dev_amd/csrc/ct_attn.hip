@@ -531,11 +531,12 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     The large launch walks 8 row blocks in step: with 4 heads per slice 64 rows, but with 2 heads 128 and with 1 head 256,
 //     most of which do not see most of what they wait for. There the four-wavefront workgroups are ahead in longer rows
 //     too, whatever the documents, where KV heads come in eights (each XCD then has its own heads' K and V in its L2), row
-//     blocks are enough for every place (3072) and not too many (9216). 99 shapes inside these lines (large / here): whole
-//     rows 1.07 times in the geometric mean and 0.995 at least, documents up to the row 1.23 and 1.05, up to 100 positions
-//     1.37 and 1.15. Past each line whole rows lose (us): [8, 2944, 8/8] 148 / 152, [4, 4096, 16/16] 260 / 271, [8, 2048, 32/16]
-//     296 / 314; 12 KV heads, [16, 2560, 12/12] 360 / 396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64]
-//     392 / 417; image blocks in a call with ends, [8, 2304, 8/8] 88 / 103.
+//     blocks are enough for every place (3072) and not too many (9216): up to 26 key tiles per row with 2 heads, 46 with 1, 40
+//     with 8 heads in all. 112 shapes inside these lines (large / here): whole rows 1.07 times in the geometric mean and 0.995
+//     at least, documents up to the row 1.23 and 1.05, up to 100 positions 1.37 and 1.15. Past each line whole rows lose (us):
+//     [8, 2944, 8/8] 148 / 152, [4, 4096, 16/16] 260 / 271, [8, 2048, 32/16] 296 / 314; 12 KV heads, [16, 2560, 12/12] 360 /
+//     396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64] 392 / 417; image blocks in a call with ends,
+//     [8, 2304, 8/8] 88 / 103.
 //     Sharing by four takes a compute unit's LDS, so it wins as long as there is a workgroup per compute unit: up to
 //     256 row blocks with one in a workgroup (us, by two / by four: 33.5 / 22.9 at 136 with images; at 256, documents up to
 //     the row, 512 and 100: [1, 2048, 4/4] 23.9 / 17.1, 12.8 / 11.1, 8.8 / 8.7, [2, 512, 8/8] 11.8 / 10.1, 12.8 / 11.1, 7.8 / 8.8),
@@ -555,7 +556,7 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
     if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     const int hs = heads_per_group(p.Hq, p.Hkv);
     const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;
-    const int short_row = !local || hs == 4 ? 20 : hs == 2 ? 26 : 40;
+    const int short_row = !local || hs == 4 ? 20 : hs == 2 ? 26 : p.Hq < 16 ? 40 : 46;
     if (p.S <= short_row * kKeyTile) return launch_fwd_split<D, 4, 1, 2, 1>(stream, p);
     switch (hs) {
       case 4: return launch_fwd<D, 4>(stream, p);

@@ -405,8 +405,9 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     # the same groups and others in rows of the large form
     (2, 4224, 12, 12, 128), (9, 4224, 2, 2, 128), (6, 4224, 3, 3, 128), (2, 4096, 12, 12, 128), (1, 2304, 32, 32, 128),
     (2, 2048, 32, 16, 128), (2, 2176, 24, 12, 128), (4, 2304, 9, 9, 128), (4, 2432, 9, 9, 128),
-    # calls without ends, KV heads in eights: rows of 2560 positions with one head per slice and of 1664 with two, 3072 and 9216
-    # row blocks
+    # calls without ends, KV heads in eights: rows of 2944 positions with one head per slice (2560 with 8 heads) and of 1664
+    # with two, 3072 and 9216 row blocks
+    (2, 2944, 24, 8, 128), (2, 3072, 24, 8, 128), (5, 2560, 8, 8, 128), (5, 2688, 8, 8, 128),
     (2, 2560, 24, 8, 128), (2, 2688, 24, 8, 128), (2, 1664, 32, 16, 128), (2, 1792, 32, 16, 128), (2, 2048, 24, 8, 128),
     (2, 1920, 24, 8, 128), (8, 1536, 24, 8, 128), (9, 1408, 24, 8, 128),
     # 448 and 512 row blocks in rows of 896 and 1024 positions
