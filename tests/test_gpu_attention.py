@@ -861,8 +861,9 @@ def test_million_token_sequence(ct, gpu):
 
 @pytest.mark.parametrize("batch,seq", [(2, 262144 + 384), (1, 262144 + 128), (40, 32768), (2, 640)])
 def test_schedules_are_the_stable_order_by_work(ct, gpu, batch, seq):
-    """All five schedules of every row and the order inside the bins, with working arrays in LDS (the last shape) and in
-    the scratch region, where rows of a length like these start them at any multiple of 4 bytes."""
+    """All five schedules of every row and the order inside the bins, with working arrays in LDS and in the scratch
+    region (the schedules' beyond 262144 positions, the bins' beyond 13568 tiles of the batch), where rows of a length like
+    the first start them at any multiple of 4 bytes."""
 
     rng = np.random.default_rng(seq)
     ids = np.cumsum(rng.random((batch, seq)) < 0.002, axis=1).astype(np.int32) + 1
@@ -897,10 +898,12 @@ def test_schedules_are_the_stable_order_by_work(ct, gpu, batch, seq):
         cursor += 33 + spans.size
 
 
-@pytest.mark.parametrize("batch,seq,rate", [(1, 128, 0.01), (2, 1152, 0.02), (4, 4096, 0.002), (3, 8320, 0.0), (1, 262144 + 128, 0.001)])
+@pytest.mark.parametrize("batch,seq,rate", [(1, 128, 0.01), (2, 1152, 0.02), (4, 4096, 0.002), (3, 8320, 0.0), (1, 262144 + 128, 0.001),
+                                            (40, 21632, 0.002), (41, 21376, 0.002), (41, 21376, 0.0), (4, 262144 + 128, 0.001)])
 def test_work_bins_are_the_greedy_packing(ct, gpu, batch, seq, rate):
     """Longest tile first onto the least loaded bin, ties to the lowest: fewer tiles than bins, rows of equal and of
-    padded tiles (whose loads tie), many rounds, and arrays in the scratch region (the last shape)."""
+    padded tiles (whose loads tie), many rounds, and both forms of the packer: 13520 tiles are the most here that stay in
+    LDS with keys of 32 bits, 13694 and more go to the scratch region with keys of 64 (the last three shapes)."""
 
     import heapq
 
