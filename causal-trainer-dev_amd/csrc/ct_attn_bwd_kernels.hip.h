@@ -68,11 +68,12 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
 
   // The first key tile's copies go first (stage 0), the rows of Q, dO and O behind them; their
   // way into fragments leads through this wavefront's patch in stage 1, which nothing uses yet.
-  const KvFetcher<D> fetch(ctx.kbase, ctx.vbase, ctx.segb, kv_row_stride);
   int t = ctx.first;
+  const bool any_tile = t <= ctx.last;
+  KvCursor<D> next(ctx.kbase, ctx.vbase, ctx.segb, kv_row_stride, any_tile ? t : 0);
   KeyTileBounds kb = {0, 0, 0};
-  if (t <= ctx.last) {
-    fetch.issue(t, lds0);
+  if (any_tile) {
+    next.issue(lds_base);
     kb = key_tile_bounds(ctx.meta_b, t);
   }
   bf16x8 qf[D / 16], dof[D / 16];
@@ -123,12 +124,11 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
   auto step = [&](auto stage_tag) {
     constexpr int CUR = decltype(stage_tag)::value;
     const lds_addr stage = lds0 + CUR * kStage;
-    const bool more = t + 1 <= ctx.last;
-    KeyTileBounds nb = kb;
-    if (more) {
-      fetch.issue(t + 1, lds0 + (CUR ^ 1) * kStage);
-      nb = key_tile_bounds(ctx.meta_b, t + 1);
+    if (t + 1 <= ctx.last) {
+      next.advance();
+      next.issue(lds_base + (CUR ^ 1) * kStage);
     }
+    KeyTileRecords ahead(ctx.meta_b, min(t + 1, ctx.last));
     if (ctx.wave_visits(kb, t)) {
       // Same specialisation as the forward: masked scores become -inf, so their
       // probability exp2(-inf) is exactly 0 and so is dS.
@@ -173,9 +173,10 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
         accumulate_t<D>(kOff, LeanTrFrags<D>::fresh(lds_base), s, dqacc);
       }
     }
+    ahead.pin();
     dma_wait_all();
     __syncthreads();
-    kb = nb;
+    kb = ahead.bounds();
     ++t;
   };
   while (t <= ctx.last) {
@@ -254,32 +255,63 @@ struct QdoStage {
   static constexpr int kTotalBytes = 2 * kBytes + kPatchBytes;
 };
 
-// Starts the asynchronous copy of query block qb of head h into `stage`: Q and dO rows, and
-// the per-row statistics. The four statistics arrays (lse2, delta: head-major f32; segment ids,
-// visible ends: i32) are 128 contiguous bytes each for the 32 rows and sit in the stage in that
-// order; wavefront w fetches array w with its first 8 lanes (one copy instruction, the source
-// chosen with scalar selects), so no wavefront carries a divergent address computation.
-// Without visible ends (plain causal) wavefront 3 has nothing to fetch.
+// The walk of a dK/dV workgroup over its (head, query block) items, query block fastest, as the addresses that
+// move with it: the rows of Q and dO, the statistics this wavefront fetches and the block's bounds. A step adds a
+// constant, the one of a next query block or the one of a next head's first block. (Formed from the coordinates
+// for every item, the same addresses were 64-bit products and a chain of branches over the statistics array,
+// about 60 scalar instructions a step of 300.)
+//
+// The four statistics arrays (lse2, delta: head-major f32; segment ids, visible ends: i32) are 128 contiguous
+// bytes each for the 32 rows and sit in the stage in that order; wavefront w fetches array w with its first 8
+// lanes, one copy instruction. Without visible ends (plain causal) wavefront 3 fetches nothing.
 template <int D>
-CT_DEVICE void qdo_fetch(const TileDma<kQueryTile, D / 8>& dma, const AttnParams& p, int b, int h,
-                         int qb, lds_addr stage) {
-  const size_t origin = (((size_t)b * p.S + qb * kQueryTile) * p.Hq + h) * D;
-  dma.issue(reinterpret_cast<const char*>(p.q + origin), stage + QdoStage<D>::kQ);
-  dma.issue(reinterpret_cast<const char*>(p.dout + origin), stage + QdoStage<D>::kDo);
-  const int which = uniform(threadIdx.x >> 6);
-  if (which < (p.end ? 4 : 3)) {
-    const size_t head_major = ((size_t)b * p.Hq + h) * p.S + qb * kQueryTile;
-    const size_t row_major = (size_t)b * p.S + qb * kQueryTile;
-    const char* src = which == 0   ? reinterpret_cast<const char*>(p.lse2 + head_major)
-                      : which == 1 ? reinterpret_cast<const char*>(p.delta + head_major)
-                      : which == 2 ? reinterpret_cast<const char*>(p.seg + row_major)
-                                   : reinterpret_cast<const char*>(p.end + row_major);
-    // (head dimension 64, at its register limit: an offset kept for the loop is spilled, and its reload
-    // waits for the copies)
-    const unsigned lane = D == 64 ? (unsigned)lane_id_here() : threadIdx.x & 63;
-    if (lane < 8) dma16_s(src, lane * 16, stage + QdoStage<D>::kLse + which * (kQueryTile * 4));
+struct QdoCursor {
+  int head, left;  // (the blocks of the head behind this one, not its number: a number that the masks use as well moves to
+                   // the vector unit, and the selects of `advance` with it)
+  const char* q;
+  const char* dout;
+  const char* stat;
+  const char* bounds;
+  long long row_step, row_wrap, stat_wrap, bounds_wrap;
+  unsigned long long stat_lanes;
+
+  CT_DEVICE QdoCursor(const AttnParams& p, int b, int head_, int qb, int q_lo, int q_hi, int which) : head(head_), left(q_hi - qb) {
+    const size_t origin = (((size_t)b * p.S + qb * kQueryTile) * p.Hq + head) * D * sizeof(bf16);
+    q = reinterpret_cast<const char*>(p.q) + origin;
+    dout = reinterpret_cast<const char*>(p.dout) + origin;
+    bounds = reinterpret_cast<const char*>(p.meta) + ((size_t)b * (p.S / 32) + qb) * (kMetaW * sizeof(int));
+    const bool head_major = which < 2;
+    const size_t row = (head_major ? (size_t)b * p.Hq + head : (size_t)b) * p.S + qb * kQueryTile;
+    const char* array = which == 0   ? reinterpret_cast<const char*>(p.lse2)
+                        : which == 1 ? reinterpret_cast<const char*>(p.delta)
+                        : which == 2 ? reinterpret_cast<const char*>(p.seg)
+                                     : reinterpret_cast<const char*>(p.end);
+    stat = array + row * 4;
+    stat_lanes = which == 3 && !p.end ? 0 : 0xff;
+    const long long back = q_hi - q_lo;  // from the last query block of a head to its first
+    row_step = (long long)kQueryTile * p.Hq * D * (long long)sizeof(bf16);
+    row_wrap = D * (long long)sizeof(bf16) - back * row_step;
+    stat_wrap = (head_major ? (long long)p.S * 4 : 0) - back * (kQueryTile * 4);
+    bounds_wrap = -back * (long long)(kMetaW * sizeof(int));
   }
-}
+  CT_DEVICE void advance(int blocks) {
+    const bool wrap = left == 0;
+    const long long rows = wrap ? row_wrap : row_step;
+    q += rows;
+    dout += rows;
+    stat += wrap ? stat_wrap : (long long)(kQueryTile * 4);
+    bounds += wrap ? bounds_wrap : (long long)(kMetaW * sizeof(int));
+    left = wrap ? blocks - 1 : left - 1;
+    head += wrap ? 1 : 0;
+  }
+  // asynchronous copy of the item into `stage`
+  CT_DEVICE void fetch(const TileDma<kQueryTile, D / 8>& dma, lds_addr stage, int wave) const {
+    dma.issue(q, stage + QdoStage<D>::kQ, wave);
+    dma.issue(dout, stage + QdoStage<D>::kDo, wave);
+    dma16_lanes_s(stat, (unsigned)lane_id_here() * 16, stage + QdoStage<D>::kLse + wave * (kQueryTile * 4), stat_lanes);
+  }
+  CT_DEVICE QueryBlockBounds query_bounds() const { return query_block_bounds(reinterpret_cast<const int*>(bounds), 0); }
+};
 
 // Fragment address structures of the dK/dV kernel: the register-lean ones where the tile is
 // wide enough for them (the kernel is at the register limit).
@@ -685,7 +717,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
   const lds_addr lds0 = lds_address_of(smem_raw);
   constexpr int kStage = QdoStage<D>::kBytes;
 
-  const int l = lane_id(), j = l & 31, half = l >> 5, w = threadIdx.x >> 6;
+  const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
   const int kvh = p.kvh_base + blockIdx.x % p.kvh_count, entry = blockIdx.x / p.kvh_count;
   if (entry >= uniform(p.dkv_header[0])) return;
@@ -721,7 +753,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
   // K fragments stay in registers; V fragments are parked in LDS (this wavefront's
   // private 32-row patch) and re-read per block, which keeps the kernel under 256
   // registers so that two workgroups share a CU.
-  const int vpatch_off = QdoStage<D>::kVResident + uniform(w) * 32 * D * 2;
+  const int vpatch_off = QdoStage<D>::kVResident + w * 32 * D * 2;
   const lds_addr vpatch = lds0 + vpatch_off;
   bf16x8 kf[D / 16];
 #pragma unroll
@@ -753,35 +785,28 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
   const int per_chunk = (nq * g + nsplit - 1) / nsplit;
   int it = chunk * per_chunk;
   const int items = min(nq * g, it + per_chunk);  // end of this chunk's item range
-  int qb = q_lo, head = kvh * g;
-  if (it < items) {
-    head += it / nq;
-    qb += it % nq;
-  }
   const TileDma<kQueryTile, D / 8> dma((size_t)p.Hq * D * 2);
+  // (a chunk without items: an address inside the arrays all the same)
+  QdoCursor<D> next(p, b, uniform(kvh * g + (it < items ? it / nq : 0)), uniform(it < items ? q_lo + it % nq : 0), q_lo, q_hi, w);
   if (it < items) {
-    qdo_fetch<D>(dma, p, b, head, qb, lds0);
+    next.fetch(dma, lds0, w);
     dma_wait_all();
   }
   __syncthreads();
 
-  QueryBlockBounds qb_bounds = query_block_bounds(meta_b, min(qb, nrb - 1));
+  QueryBlockBounds qb_bounds = next.query_bounds();
   auto step = [&](auto stage_tag) {
     constexpr int CUR = decltype(stage_tag)::value;
     const lds_addr stage = lds0 + CUR * kStage;
-    const bool more = it + 1 < items;
-    int qb_next = qb + 1, head_next = head;
-    if (qb_next > q_hi) {
-      qb_next = q_lo;
-      ++head_next;
-    }
-    if (more) qdo_fetch<D>(dma, p, b, head_next, qb_next, lds0 + (CUR ^ 1) * kStage);
-
-    // bounds of this query block (read one item ahead: the scalar loads are long done when
-    // the next item needs them)
+    const int qb = q_hi - next.left, head = next.head;
+    // bounds of this query block, read one item ahead
     const int q_min = qb_bounds.min_nz, q_max = qb_bounds.max_id, q_end_max = qb_bounds.end_max,
               q_end_min = qb_bounds.end_min, q_uni = qb_bounds.uniform;
-    if (more) qb_bounds = query_block_bounds(meta_b, qb_next);
+    if (it + 1 < items) {
+      next.advance(nq);
+      next.fetch(dma, lds0 + (CUR ^ 1) * kStage, w);
+    }
+    QueryBlockBounds bounds_ahead = next.query_bounds();  // (behind the last item: the same bounds again)
     const bool visit = blocks_interact(q_min, q_max, q_end_max, my_min, my_max, my_rb * 32);
     if (visit) {
       // The row offsets below depend on the lane only; hoisted out of the loop they become
@@ -861,6 +886,11 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
         accumulate_keys<D>(CUR * kStage + QdoStage<D>::kQ, to, dp, dkacc);
       }
     }
+    // The next block's bounds are waited for here, where the step has given them the time. Left to their first use
+    // the wait stands in the next step behind the loads for the step after it, and as scalar loads return in any
+    // order it waits for those too: a round trip of the scalar cache in every step.
+    bounds_ahead.pin();
+    qb_bounds = bounds_ahead;
     // Vector memory operations complete in the order they were issued: the two stores of this
     // step are the youngest, so waiting for all but two has waited for every copy of the next
     // stage without waiting for the stores (they are long done one step later).
@@ -868,8 +898,6 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
     else dma_wait_all();
     __syncthreads();
     ++it;
-    qb = qb_next;
-    head = head_next;
   };
   while (it < items) {
     step(std::integral_constant<int, 0>{});

@@ -77,23 +77,34 @@ struct KvStage {
   static constexpr int kBytes = 2 * kTileBytes + kKeyTile * 4;
 };
 
-// Asynchronous fetch of key tile `tile` (K rows, V rows, segment ids) into an LDS stage.
+// Asynchronous fetch of a key tile (K rows, V rows, segment ids) into an LDS stage, for a walk from tile to tile:
+// addresses that a step advances by a constant, the LDS address in scalar registers, the ids by a copy whose lanes are all off in three of the four wavefronts. (Formed from the tile's number
+// every time, a copy of a tile costs 80 scalar and vector instructions beside its nine copies.)
 template <int D>
-struct KvFetcher {
+struct KvCursor {
   TileDma<kKeyTile, D / 8> dma;
-  const char* kbase;
-  const char* vbase;
-  const int* segb;
-  size_t row_stride_bytes;
-  CT_DEVICE KvFetcher(const bf16* k, const bf16* v, const int* seg, size_t row_stride_elems)
-      : dma(row_stride_elems * 2), kbase(reinterpret_cast<const char*>(k)),
-        vbase(reinterpret_cast<const char*>(v)), segb(seg), row_stride_bytes(row_stride_elems * 2) {}
-  CT_DEVICE void issue(int tile, lds_addr stage) const {
-    const size_t origin = (size_t)tile * kKeyTile * row_stride_bytes;
-    dma.issue(kbase + origin, stage + KvStage<D>::kK);
-    dma.issue(vbase + origin, stage + KvStage<D>::kV);
-    if (threadIdx.x < 16)  // 64 ids = 16 lanes x 16 bytes, linear layout
-      dma16_s(segb + tile * kKeyTile, threadIdx.x * 16, stage + KvStage<D>::kSeg);
+  const char* k;
+  const char* v;
+  const char* seg;
+  size_t step;
+  unsigned long long seg_lanes;
+  int wave;
+  CT_DEVICE KvCursor(const bf16* k_, const bf16* v_, const int* seg_, size_t row_stride_elems, int tile)
+      : dma(row_stride_elems * 2), step(kKeyTile * row_stride_elems * 2), wave(uniform(threadIdx.x >> 6)) {
+    k = reinterpret_cast<const char*>(k_) + tile * step;
+    v = reinterpret_cast<const char*>(v_) + tile * step;
+    seg = reinterpret_cast<const char*>(seg_ + tile * kKeyTile);
+    seg_lanes = wave == 0 ? 0xffff : 0;  // 64 ids = 16 lanes x 16 bytes, linear layout
+  }
+  CT_DEVICE void advance() {
+    k += step;
+    v += step;
+    seg += kKeyTile * 4;
+  }
+  CT_DEVICE void issue(lds_addr stage) const {
+    dma.issue(k, stage + KvStage<D>::kK, wave);
+    dma.issue(v, stage + KvStage<D>::kV, wave);
+    dma16_lanes_s(seg, (unsigned)lane_id_here() * 16, stage + KvStage<D>::kSeg, seg_lanes);
   }
 };
 

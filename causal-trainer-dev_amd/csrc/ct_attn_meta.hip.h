@@ -262,6 +262,29 @@ CT_DEVICE KeyTileBounds key_tile_bounds(const int* meta_b, int t) {
   return out;
 }
 
+// The same from records that were read earlier: the loads go out where the records are made and are waited for at
+// `pin`, which a loop calls where it has given them the time. Without it the wait stands at the bounds' first use, in
+// the next step and behind the loads of the step after it, and covers those too: scalar loads return in any order.
+struct KeyTileRecords {
+  int a_min, a_max, a_uniform, c_min, c_max, c_uniform;
+  CT_DEVICE KeyTileRecords(const int* meta_b, int t) {
+    const MetaPtr a = meta_const(meta_b + (2 * t) * kMetaW);
+    const MetaPtr c = a + kMetaW;
+    a_min = a[kMinNz], a_max = a[kMaxId], a_uniform = a[kUniform];
+    c_min = c[kMinNz], c_max = c[kMaxId], c_uniform = c[kUniform];
+  }
+  CT_DEVICE void pin() {
+    asm volatile("" : "+s"(a_min), "+s"(a_max), "+s"(a_uniform), "+s"(c_min), "+s"(c_max), "+s"(c_uniform));
+  }
+  CT_DEVICE KeyTileBounds bounds() const {
+    KeyTileBounds out;
+    out.min_nz = a_min == 0 ? c_min : (c_min == 0 ? a_min : min(a_min, c_min));
+    out.max_id = max(a_max, c_max);
+    out.uniform = a_uniform == c_uniform ? a_uniform : 0;
+    return out;
+  }
+};
+
 // The same in two steps, for a caller that wants the loads to complete under a wait it has anyway:
 // key_tile_words_request issues the scalar loads and returns at once (the compiler does not know
 // that the registers are still in flight, so it neither waits nor moves the loads behind the
@@ -298,6 +321,8 @@ CT_DEVICE KeyTileBounds key_tile_bounds(const KeyTileWords& w) {
 
 struct QueryBlockBounds {
   int min_nz, max_id, uniform, end_min, end_max, kv_first, kv_last;
+  // waits for the scalar loads that the bounds come from (the ranges of key tiles are not among them)
+  CT_DEVICE void pin() { asm volatile("" : "+s"(min_nz), "+s"(max_id), "+s"(uniform), "+s"(end_min), "+s"(end_max)); }
 };
 
 CT_DEVICE QueryBlockBounds query_block_bounds(const int* meta_b, int rb) {

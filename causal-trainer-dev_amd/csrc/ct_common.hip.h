@@ -141,6 +141,19 @@ CT_DEVICE void dma16_s(const void* uniform_base, unsigned lane_offset, lds_addr 
                : "v"(lane_offset), "s"(base), "s"(m0_value)
                : "memory", "m0");
 }
+// The same for the lanes of a wave-uniform mask (none: nothing is copied), without a branch around it. The whole
+// wavefront has to be active where it is called: the statement leaves all lanes on.
+CT_DEVICE void dma16_lanes_s(const void* uniform_base, unsigned lane_offset, lds_addr dst, unsigned long long lanes) {
+  const unsigned m0_value = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)dst);
+  const unsigned long long b = (unsigned long long)(uintptr_t)uniform_base;
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+  const unsigned long long base = ((unsigned long long)hi << 32) | (unsigned long long)lo;
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1"
+               :
+               : "v"(lane_offset), "s"(base), "s"(m0_value), "s"(lanes)
+               : "memory", "m0");
+}
 // s_waitcnt vmcnt(0) only (expcnt / lgkmcnt fields left at "no wait")
 CT_DEVICE void dma_wait_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
@@ -189,8 +202,10 @@ struct TileDma {
       lane_off[n] = (unsigned)((size_t)(row0 + n * kRowsPerPass) * row_stride_bytes + chunk * 16);
   }
   // origin and tile are workgroup-uniform
-  CT_DEVICE void issue(const char* origin, lds_addr tile) const {
-    const int wave = uniform(threadIdx.x >> 6);
+  CT_DEVICE void issue(const char* origin, lds_addr tile) const { issue(origin, tile, uniform(threadIdx.x >> 6)); }
+  // (the number of the wavefront from a register that the caller keeps: the compiler forms it again, by a lane read
+  // and five scalar instructions, for every call in a loop)
+  CT_DEVICE void issue(const char* origin, lds_addr tile, int wave) const {
 #pragma unroll
     for (int n = 0; n < kPasses; ++n) dma16_s(origin, lane_off[n], tile + (n * THREADS + wave * 64) * 16);
   }
