@@ -48,6 +48,12 @@ CT_DEVICE void dq_arith(f32x16& s, const f32x16& dp, float lse2, float delta_q) 
   }
 }
 
+// The same for dp = dP - delta.
+CT_DEVICE void dq_arith(f32x16& s, const f32x16& dp, float lse2) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s[r] = exp2_fast(fmaf(s[r], kLog2e, -lse2)) * dp[r];
+}
+
 // One query tile (4 / HS row blocks x HS heads of one KV head), start to finish.
 template <int D, int HS>
 CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int qt, const lds_addr lds_base) {
@@ -114,6 +120,12 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
     }
   }
   const float delta_q = pair_sum(delta_part);
+  f32x16 minus_delta;
+  if constexpr (D == 64) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) minus_delta[r] = -delta_q;
+    asm volatile("" : "+v"(minus_delta));
+  }
   if (ctx.active && half == 0) {
     // for the dK/dV kernel: the values it adds to its S and dP blocks, P = exp2((S - lse / scale) *
     // scale * log2(e)) and dS = P (dP - delta)
@@ -128,8 +140,12 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
       next.advance();
       next.issue(lds_base + (CUR ^ 1) * kStage);
     }
-    KeyTileRecords ahead(ctx.meta_b, min(t + 1, ctx.last));
-    if (ctx.wave_visits(kb, t)) {
+    // (requested behind the products of D = 64: a wait for LDS reads is one for all scalar loads too)
+    KeyTileRecords ahead;
+    const auto request = [&]() { ahead = KeyTileRecords(ctx.meta_b, min(t + 1, ctx.last)); };
+    const bool visits = ctx.wave_visits(kb, t);
+    if (D != 64 || !visits) request();
+    if (visits) {
       // Same specialisation as the forward: masked scores become -inf, so their
       // probability exp2(-inf) is exactly 0 and so is dS.
       const int k_uniform = uniform(kb.uniform);
@@ -162,15 +178,30 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
         half_tile(std::integral_constant<int, 1>{});
       } else {
         f32x16 s[2], dp[2];
-        scores_t<D>(kOff, ro, qf, s);
-        scores_t<D>(vOff, ro, dof, dp);
+        // (dP starts from -delta, a register block of its own, and needs no subtraction)
+        constexpr int kSteps = D / 16;
+        fragments_ahead<4 * kSteps, 6>(
+            [&](int i) { return ro.load(i < 2 * kSteps ? kOff : vOff, i & 1, i / 2 % kSteps); },
+            [&](int i, bf16x8 keys) {
+              const int kb = i & 1, ks = i / 2 % kSteps;
+              if (i < 2 * kSteps) s[kb] = mfma32(keys, qf[ks], ks ? s[kb] : zero16());
+              else dp[kb] = mfma32(keys, dof[ks], ks ? dp[kb] : minus_delta);
+            });
+        request();
         if (need_seg || need_causal) {
           if (k_uniform == 0) mask_scores_t<true, true>(stage + KvStage<D>::kSeg, seg_cmp, last_rel, s);
           else mask_scores_t<false, true>(stage, seg_cmp, last_rel, s);
         }
-        dq_arith(s[0], dp[0], lse2, delta_q);
-        dq_arith(s[1], dp[1], lse2, delta_q);
-        accumulate_t<D>(kOff, LeanTrFrags<D>::fresh(lds_base), s, dqacc);
+        dq_arith(s[0], dp[0], lse2);
+        dq_arith(s[1], dp[1], lse2);
+        bf16x8 ds[4];
+#pragma unroll
+        for (int step = 0; step < 4; ++step) ds[step] = pack_acc8(s[step >> 1], step & 1);
+        constexpr int kBlocks = D / 32;
+        fragments_ahead<4 * kBlocks, 4>([&](int i) { return to.load(kOff, i / kBlocks, i % kBlocks); },
+                                        [&](int i, bf16x8 keys) {
+                                          dqacc[i % kBlocks] = mfma32(keys, ds[i / kBlocks], dqacc[i % kBlocks]);
+                                        });
       }
     }
     ahead.pin();
@@ -266,8 +297,7 @@ struct QdoStage {
 // lanes, one copy instruction. Without visible ends (plain causal) wavefront 3 fetches nothing.
 template <int D>
 struct QdoCursor {
-  int head, left;  // (the blocks of the head behind this one, not its number: a number that the masks use as well moves to
-                   // the vector unit, and the selects of `advance` with it)
+  int head, left;  // left: query blocks of this head behind this one
   const char* q;
   const char* dout;
   const char* stat;
@@ -321,15 +351,6 @@ template <int D>
 using DkvTrFrags = std::conditional_t<(D / 8 >= 16), TrFragCompact<D / 8, KSlots::kAccum>,
                                       TrFragOffsets<D / 8, KSlots::kAccum>>;
 
-// X (32 rows of an LDS tile) times register fragments: C[row, key] = sum_d X[row, d] F[key, d].
-template <int D>
-CT_DEVICE f32x16 rows_times_frags(int tile_off, const DkvRowFrags<D>& ro, const bf16x8* frags,
-                                  f32x16 c = zero16()) {
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) c = mfma32(ro.load(tile_off, 0, ks), frags[ks], c);
-  return c;
-}
-
 // Hand-scheduled MFMA sequences of the dK/dV kernel for D = 128 (gen_attn_asm.py): the
 // compiler's own schedule issues each LDS fragment read directly in front of the MFMA that
 // consumes it, so with two wavefronts per SIMD every MFMA pays most of the LDS latency.
@@ -357,19 +378,6 @@ CT_DEVICE void dkv_acc_sequence_128(const TrFragOffsets<16, KSlots::kAccum>& to,
                  "v"(to.ptr[1][0]), "v"(to.ptr[1][1]), "v"(to.ptr[1][2]), "v"(to.ptr[1][3]), "v"(p0),
                  "v"(p1), "v"(d0), "v"(d1), "i"(STAGE_OFF)
                : "memory", CT_DKV_ASM_SCRATCH);
-}
-
-// acc (32 keys x D) += W^T X, W in accumulator layout (rows = the 32 tile rows,
-// cols = keys), X the 32-row LDS tile read transposed.
-template <int D>
-CT_DEVICE void accumulate_keys(int tile_off, const DkvTrFrags<D>& to, const f32x16& wt,
-                               f32x16* acc) {
-#pragma unroll
-  for (int step = 0; step < 2; ++step) {
-    const bf16x8 aop = pack_acc8(wt, step);
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db) acc[db] = mfma32(aop, to.load(tile_off, step, db), acc[db]);
-  }
 }
 
 // Store a (32 rows x D) accumulator (lanes along D) as bf16 rows via an LDS patch.
@@ -710,7 +718,8 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
 //
 // Head dimension 64 is held to 168 registers, three workgroups per compute unit (LDS has room for four): its steps are
 // short and the vector ALU waits between the matrix instructions. With 177 registers and two workgroups:
-// [2, 15616, 12/2 heads of 64] 544 -> 445 us, [1, 7424, 6/1] 95 -> 80.
+// [2, 15616, 12/2 heads of 64] 544 -> 445 us, [1, 7424, 6/1] 95 -> 80. Its fragments are read ahead of the products
+// (fragments_ahead): [1, 25472, 64/8], image blocks, 1800 -> 1690; the dQ kernel above likewise, 1280 -> 1190.
 template <int D, bool SPILL>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
@@ -737,6 +746,9 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
     q_lo = min(q_lo, uniform(m[kQFirst]));
     q_hi = max(q_hi, uniform(m[kQLast]));
   }
+  // (the extremes of several come out of the vector unit, and what is selected and added by them would stay there)
+  q_lo = uniform(q_lo);
+  q_hi = uniform(q_hi);
   const int my_rb = kt * 4 + w;
   const int my_min = uniform(meta_const(meta_b)[my_rb * kMetaW + kMinNz]);
   const int my_max = uniform(meta_const(meta_b)[my_rb * kMetaW + kMaxId]);
@@ -806,8 +818,9 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
       next.advance(nq);
       next.fetch(dma, lds0 + (CUR ^ 1) * kStage, w);
     }
-    QueryBlockBounds bounds_ahead = next.query_bounds();  // (behind the last item: the same bounds again)
+    QueryBlockBounds bounds_ahead;  // (behind the last item: the same bounds again)
     const bool visit = blocks_interact(q_min, q_max, q_end_max, my_min, my_max, my_rb * 32);
+    if (D != 64 || !visit) bounds_ahead = next.query_bounds();
     if (visit) {
       // The row offsets below depend on the lane only; hoisted out of the loop they become
       // spilled registers whose reloads wait for every copy in flight. Recompute them here.
@@ -834,10 +847,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
         const RowFragOffsets<16> rp = RowFragOffsets<16>::expand(RowFragCompact<16>(lds0, lane_id_here()));
         dkv_sdp_sequence_128<CUR * kStage>(rp, kf, (unsigned)vpatch_off, s, dp);
       } else {
-        s = rows_times_frags<D>(CUR * kStage + QdoStage<D>::kQ, ro, kf, s);
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks)
-          dp = mfma32(ro.load(CUR * kStage + QdoStage<D>::kDo, 0, ks), ro.load(vpatch_off, 0, ks), dp);
+        constexpr int kSteps = D / 16, qOff = CUR * kStage + QdoStage<D>::kQ, doOff = CUR * kStage + QdoStage<D>::kDo;
+        fragments_ahead<kSteps, kSteps>([&](int i) { return ro.load(qOff, 0, i); },
+                                        [&](int i, bf16x8 queries) { s = mfma32(queries, kf[i], s); });
+        struct Pair {
+          bf16x8 dout, v;
+        };
+        fragments_ahead<kSteps, 2>([&](int i) { return Pair{ro.load(doOff, 0, i), ro.load(vpatch_off, 0, i)}; },
+                                   [&](int i, const Pair& rows) { dp = mfma32(rows.dout, rows.v, dp); });
+        bounds_ahead = next.query_bounds();  // (a wait for LDS reads is one for all scalar loads too)
       }
       const bool interior = tile_is_interior(q_uni, q_end_min, my_uni, my_rb * 32 + 31);
       f32x16 prob;
@@ -882,8 +900,16 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
             TrFragOffsets<16, KSlots::kAccum>::expand(TrFragCompact<16, KSlots::kAccum>(lds0, lane_id_here()));
         dkv_acc_sequence_128<CUR * kStage>(tp, prob, dp, dvacc, dkacc);
       } else {
-        accumulate_keys<D>(CUR * kStage + QdoStage<D>::kDo, to, prob, dvacc);
-        accumulate_keys<D>(CUR * kStage + QdoStage<D>::kQ, to, dp, dkacc);
+        const bf16x8 keys[4] = {pack_acc8(prob, 0), pack_acc8(prob, 1), pack_acc8(dp, 0), pack_acc8(dp, 1)};
+        constexpr int kBlocks = D / 32;
+        fragments_ahead<4 * kBlocks, 4>(
+            [&](int i) {
+              return to.load(CUR * kStage + (i < 2 * kBlocks ? QdoStage<D>::kDo : QdoStage<D>::kQ), i / kBlocks % 2, i % kBlocks);
+            },
+            [&](int i, bf16x8 rows) {
+              f32x16& acc = (i < 2 * kBlocks ? dvacc : dkacc)[i % kBlocks];
+              acc = mfma32(keys[i / kBlocks], rows, acc);
+            });
       }
     }
     // The next block's bounds are waited for here, where the step has given them the time. Left to their first use

@@ -145,19 +145,6 @@ struct QueryWork {
   }
 };
 
-// S^T (two 32-key blocks) = K_tile Q^T for this wavefront's 32 queries.
-// `tile_off` is the tile's byte offset from the LDS base the offsets were built on.
-template <int D, class RowFrags>
-CT_DEVICE void scores_t(int tile_off, const RowFrags& ro, const bf16x8* qf, f32x16* s) {
-  s[0] = zero16();
-  s[1] = zero16();
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) s[kb] = mfma32(ro.load(tile_off, kb, ks), qf[ks], s[kb]);
-  }
-}
-
 // Sets the scores of disallowed (query, key) pairs of a transposed score tile to -inf.
 // The pair rule is seg_k == seg_q != 0 and key <= end_q (src/modeling/attention.py:67-97);
 // each half is only evaluated where the tile's summaries do not already prove it:
@@ -191,18 +178,6 @@ template <bool SEG, bool CAUSAL>
 CT_DEVICE void mask_scores_t(lds_addr segk, int seg_q_or_never, int last_rel, f32x16* s) {
   mask_block_t<SEG, CAUSAL>(segk, seg_q_or_never, last_rel, 0, s[0]);
   mask_block_t<SEG, CAUSAL>(segk, seg_q_or_never, last_rel, 1, s[1]);
-}
-
-// acc (D x 32 queries, transposed) += X^T W^T where X is a 64-row LDS tile read
-// transposed and W^T are the accumulator-layout weights wt[2].
-template <int D, class TrFrags>
-CT_DEVICE void accumulate_t(int tile_off, const TrFrags& to, const f32x16* wt, f32x16* acc) {
-#pragma unroll
-  for (int step = 0; step < 4; ++step) {
-    const bf16x8 bop = pack_acc8(wt[step >> 1], step & 1);
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db) acc[db] = mfma32(to.load(tile_off, step, db), bop, acc[db]);
-  }
 }
 
 // Write a transposed accumulator (D x 32 rows) as bf16 rows of D elements to

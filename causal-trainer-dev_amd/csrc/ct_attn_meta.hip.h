@@ -267,6 +267,7 @@ CT_DEVICE KeyTileBounds key_tile_bounds(const int* meta_b, int t) {
 // the next step and behind the loads of the step after it, and covers those too: scalar loads return in any order.
 struct KeyTileRecords {
   int a_min, a_max, a_uniform, c_min, c_max, c_uniform;
+  KeyTileRecords() = default;
   CT_DEVICE KeyTileRecords(const int* meta_b, int t) {
     const MetaPtr a = meta_const(meta_b + (2 * t) * kMetaW);
     const MetaPtr c = a + kMetaW;

@@ -68,6 +68,24 @@ CT_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// N matrix instructions, each fed by a fragment that `load(i)` reads from LDS and `use(i, fragment)` multiplies, with
+// the reads AHEAD instructions in front of their use. Left alone the compiler reads a fragment right where it is needed, and
+// every pair of instructions waits for LDS; here nothing but vector and scalar arithmetic moves past an instruction.
+template <int N, int AHEAD, class Load, class Use>
+CT_DEVICE void fragments_ahead(Load load, Use use) {
+  constexpr int kArithmeticMoves = 0x2 | 0x4 | 0x400;
+  decltype(load(0)) fragment[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) fragment[i] = load(i);
+  __builtin_amdgcn_sched_barrier(kArithmeticMoves);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    use(i, fragment[i % AHEAD]);
+    if (i + AHEAD < N) fragment[i % AHEAD] = load(i + AHEAD);
+    __builtin_amdgcn_sched_barrier(kArithmeticMoves);
+  }
+}
+
 // Row index (0..31) that accumulator register r of this lane holds.
 CT_DEVICE int acc_row(int r, int half) { return 8 * (r >> 2) + 4 * half + (r & 3); }
 
