@@ -1161,9 +1161,12 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
     if (one_list) {
       in_head = head_first ? a < total_w : a >= total_h;
       const int index = a - (in_head == head_first ? 0 : head_first ? total_w : total_h);
-      const int width = col_blocks * (in_head ? parts_w : parts_h);
-      a = index / width;
-      b = index % width;
+      // the part is the slowest: the 32 units of an XCD are all tiles of a few parts, which read the operands' terms of
+      // these parts and no others (the tile slowest, an XCD reads all of one operand)
+      const int tiles_a = in_head ? slab_tiles : row_blocks, grid = tiles_a * col_blocks;
+      const int part = index / grid, tile = index % grid;
+      a = tile / col_blocks;
+      b = part * col_blocks + tile % col_blocks;
     }
     if (!in_head) {
       dhidden_unit<NB, GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
