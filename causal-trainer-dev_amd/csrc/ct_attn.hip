@@ -583,14 +583,18 @@ static int launch_dq(hipStream_t stream, const AttnParams& p) {
   return scope2.done();
 }
 
+// `reduce`: the launch also adds the chunks of split key tiles, where its form can (KS > 1). 128 workgroups of eight
+// wavefronts: pieces are rarely more than twice as many.
 template <int D, int HS, int KS>
-static int launch_dq_blocks(hipStream_t stream, const AttnParams& p) {
+static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
   const size_t smem = DsStage<D, KS>::kTotalBytes;
   CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_blocks_kernel<D, HS, KS>), smem);
   const int groups = p.Hq / p.Hkv / HS * p.kvh_count;
   const int grid = KS == 1 ? dq_grid(p, HS) : groups * p.B * bin_tiles_per_row(p.S / 32, kDqbWaves / KS / HS);
+  reduce = reduce && KS > 1;
+  const int reduce_groups = reduce ? 128 : 0;
   LaunchScope scope("attn_dq_blocks_kernel", stream);
-  hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS, KS>), dim3(grid), dim3(kDqbWaves * 64), smem, stream, p);
+  hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS, KS>), dim3(grid + reduce_groups), dim3(kDqbWaves * 64), smem, stream, p, reduce_groups);
   return scope.done();
 }
 
@@ -604,17 +608,17 @@ static int launch_dq_blocks(hipStream_t stream, const AttnParams& p) {
 //   3744, D = 128: 124 / 102 / 127, but 2.5 us slower by two with short documents (a compute unit holds one of its
 //   workgroups, of the others two); 7680: 201 / 227
 template <int D>
-static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p) {
+static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
   const long blocks = (long)p.B * p.kvh_count * (p.Hq / p.Hkv) * (p.S / 32);
   const int hs = heads_per_group(p.Hq, p.Hkv);
-  if (blocks <= 768) return hs == 1 ? launch_dq_blocks<D, 1, 4>(stream, p) : launch_dq_blocks<D, 2, 4>(stream, p);
+  if (blocks <= 768) return hs == 1 ? launch_dq_blocks<D, 1, 4>(stream, p, reduce) : launch_dq_blocks<D, 2, 4>(stream, p, reduce);
   if (blocks <= (D == 64 ? 8192 : 3072))
-    return hs == 4   ? launch_dq_blocks<D, 4, 2>(stream, p)
-           : hs == 2 ? launch_dq_blocks<D, 2, 2>(stream, p)
-                     : launch_dq_blocks<D, 1, 2>(stream, p);
-  return hs == 4   ? launch_dq_blocks<D, 4, 1>(stream, p)
-         : hs == 2 ? launch_dq_blocks<D, 2, 1>(stream, p)
-                   : launch_dq_blocks<D, 1, 1>(stream, p);
+    return hs == 4   ? launch_dq_blocks<D, 4, 2>(stream, p, reduce)
+           : hs == 2 ? launch_dq_blocks<D, 2, 2>(stream, p, reduce)
+                     : launch_dq_blocks<D, 1, 2>(stream, p, reduce);
+  return hs == 4   ? launch_dq_blocks<D, 4, 1>(stream, p, reduce)
+         : hs == 2 ? launch_dq_blocks<D, 2, 1>(stream, p, reduce)
+                   : launch_dq_blocks<D, 1, 1>(stream, p, reduce);
 }
 
 // Which dK/dV kernel runs for head dimension 128 when the caller leaves the choice open: the wide
@@ -707,15 +711,17 @@ static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pas
     rc = scope.done();
   }
   if (rc) return rc;
+  bool reduced = false;
   for (int base = 0; base < p.Hkv; base += kvh_per_pass) {
     p.kvh_base = base;
     p.kvh_count = min(kvh_per_pass, p.Hkv - base);
     rc = launch_dkv<D>(stream, p, wide);
     if (rc) return rc;
-    rc = dispatch_dq_blocks<D>(stream, p);
+    reduced = base + p.kvh_count == p.Hkv;  // with the last pass all chunks are there
+    rc = dispatch_dq_blocks<D>(stream, p, reduced);
     if (rc) return rc;
   }
-  return launch_dkv_reduce<D>(stream, p);
+  return reduced ? CT_OK : launch_dkv_reduce<D>(stream, p);
 }
 
 }  // namespace ct

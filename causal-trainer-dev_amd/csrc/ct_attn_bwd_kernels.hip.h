@@ -596,58 +596,59 @@ CT_DEVICE size_t dkv_partial_offset(int slot, int Hkv, int kvh, int wave) {
 // hundred entries). One workgroup per tile and KV head walked up to 32 chunks on a few dozen compute units:
 // [1, 7424, 6/1 heads of 64] 52 -> 12 us, [1, 2432, 16/4 of 64] 25 -> 7, [4, 4096, 32/8 of 128] 22 -> 15,
 // [2, 2432, 16/16 of 128] 19 -> 14, [4, 4224, 8/1 of 128] 25 -> 16.
-// Where there are fewer such pieces than workgroups, the four wavefronts of a workgroup share one, 8 of its rows each,
+// Where there are fewer such pieces than sets of four wavefronts, four wavefronts share one, 8 of its rows each,
 // with 16 chunks in flight.
 constexpr int kReduceGroups = 1024;
-template <int D>
-__global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
-  constexpr int kMaxSplitTiles = kDkvSlots + 8;  // dkv_layout: at most half of max_partials <= 2 (kDkvSlots + 2)
+template <int WAVES>
+struct DkvReduceLds {
+  static constexpr int kMaxSplitTiles = kDkvSlots + 8;  // dkv_layout: at most half of max_partials <= 2 (kDkvSlots + 2)
+  int2 split[kMaxSplitTiles];
+  int wave_count[4][WAVES];
+  __align__(16) bf16 patches[WAVES][32 * 32];
+};
+// Workgroup `group` of `groups`, WAVES wavefronts each (four or eight).
+template <int D, int WAVES>
+CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceLds<WAVES>& lds) {
+  constexpr int kMaxSplitTiles = DkvReduceLds<WAVES>::kMaxSplitTiles;
   constexpr int kPieces = 2 * 4 * (D / 32);      // (tensor, wavefront of the dK/dV kernel, 32 columns)
-  __shared__ int2 split[kMaxSplitTiles];
-  __shared__ int wave_count[4][4];
-  __shared__ __align__(16) bf16 patches[4][32 * 32];
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
-  // This is the last kernel of a backward call: it leaves the dQ kernel's work counters at zero,
-  // so that a later call on the same workspace can keep the work list and skip the kernel that
-  // builds it (and clears the counters).
-  if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i < kDqCounters; i += blockDim.x) p.dq_counters[i] = 0;
   const int entries = uniform(p.dkv_header[0]);
   int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
-  for (int base = 0; base < entries; base += 1024) {
+  for (int base = 0; base < entries; base += 256 * WAVES) {
     int2 entry[4];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      const int i = base + n * 256 + threadIdx.x;
+      const int i = base + n * 64 * WAVES + threadIdx.x;
       entry[n] = i < entries ? p.dkv_entries[i] : make_int2(0, 0);
     }
     unsigned long long ballot[4];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       ballot[n] = __ballot((entry[n].y & 255) == 0 && ((entry[n].y >> 8) & 255) > 1);  // chunk 0 of several
-      if (l == 0) wave_count[n][w] = __popcll(ballot[n]);
+      if (l == 0) lds.wave_count[n][w] = __popcll(ballot[n]);
     }
     __syncthreads();
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      if (base + n * 256 >= entries) break;
+      if (base + n * 64 * WAVES >= entries) break;
       int at = tiles + __popcll(ballot[n] & ((1ull << l) - 1ull));
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (k < w) at += wave_count[n][k];
-        tiles += wave_count[n][k];
+      for (int k = 0; k < WAVES; ++k) {
+        if (k < w) at += lds.wave_count[n][k];
+        tiles += lds.wave_count[n][k];
       }
-      if ((ballot[n] >> l & 1) && at < kMaxSplitTiles) split[at] = entry[n];
+      if ((ballot[n] >> l & 1) && at < kMaxSplitTiles) lds.split[at] = entry[n];
     }
     __syncthreads();
   }
   tiles = uniform(min(tiles, kMaxSplitTiles));
   const int items = tiles * p.Hkv * kPieces;
-  const bool shared = items <= (int)gridDim.x;  // (then a workgroup has one piece at most)
-  for (int item = shared ? blockIdx.x : blockIdx.x * 4 + w; item < items; item += gridDim.x * 4) {
+  const bool shared = items <= groups * (WAVES / 4);  // (then four wavefronts have one piece at most)
+  const int set = w / 4, member = w % 4;
+  for (int item = shared ? group * (WAVES / 4) + set : group * WAVES + w; item < items; item += groups * WAVES) {
     const int piece = item % kPieces, kvh = item / kPieces % p.Hkv;
-    const int2 entry = split[item / kPieces / p.Hkv];
+    const int2 entry = lds.split[item / kPieces / p.Hkv];
     const int tile = uniform(entry.x), nsplit = uniform((entry.y >> 8) & 255), slot0 = uniform((unsigned)entry.y >> 16);
     const int db = piece % (D / 32), keys = piece / (D / 32) % 4, tensor = piece / (D / 32) / 4;
     const float* src = p.dkv_partials + dkv_partial_offset<D>(slot0, p.Hkv, kvh, keys) + tensor * DkvPartial<D>::kPerTensor +
@@ -655,24 +656,24 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
     const size_t chunk_stride = (size_t)p.Hkv * DkvPartial<D>::kPerChunk;
     const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
     bf16* out = (tensor ? p.dv : p.dk) + (((size_t)b * p.S + (kt * 4 + keys) * 32) * p.Hkv + kvh) * D + db * 32;
-    if (shared) {  // keys 8 w .. 8 w + 7 of the piece
+    if (shared) {  // keys 8 member .. 8 member + 7 of the piece
       f32x4 sum = {};
       for (int c = 0; c < nsplit; c += 16) {
         f32x4 v[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k)
-          v[k] = c + k < nsplit ? *reinterpret_cast<const f32x4*>(src + (c + k) * chunk_stride + w * 256) : f32x4{0.f, 0.f, 0.f, 0.f};
+          v[k] = c + k < nsplit ? *reinterpret_cast<const f32x4*>(src + (c + k) * chunk_stride + member * 256) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 16; ++k)
           if (c + k < nsplit) sum += v[k];
       }
-      bf16* patch = patches[w];
+      bf16* patch = lds.patches[w];
 #pragma unroll
       for (int e = 0; e < 4; ++e) patch[(4 * half + e) * 32 + j] = (bf16)sum[e];
       __builtin_amdgcn_wave_barrier();
       const int row = l >> 2, chunk = (l & 3) * 8;
       if (row < 8)
-        store_global16(out + (size_t)(8 * w + row) * p.Hkv * D + chunk, *reinterpret_cast<const u32x4*>(patch + row * 32 + chunk));
+        store_global16(out + (size_t)(8 * member + row) * p.Hkv * D + chunk, *reinterpret_cast<const u32x4*>(patch + row * 32 + chunk));
       return;
     }
     f32x4 sum[4] = {};
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
           for (int q = 0; q < 4; ++q) sum[q] += v[k][q];
     }
     // lane (j, half) holds column j of the keys 8 q + 4 half + e: through LDS to rows of 64 bytes
-    bf16* patch = patches[w];
+    bf16* patch = lds.patches[w];
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -703,6 +704,17 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
       store_global16(out + (size_t)row * p.Hkv * D + chunk, *reinterpret_cast<const u32x4*>(patch + row * 32 + chunk));
     }
   }
+}
+
+// On its own, the last kernel of a backward call: it also leaves the dQ kernel's work counters at zero,
+// so that a later call on the same workspace can keep the work list and skip the kernel that
+// builds it (and clears the counters).
+template <int D>
+__global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
+  __shared__ DkvReduceLds<4> lds;
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < kDqCounters; i += blockDim.x) p.dq_counters[i] = 0;
+  dkv_reduce<D, 4>(p, blockIdx.x, gridDim.x, lds);
 }
 
 // Byte address of the dS block (key block rb with table entries ds_off / q_first, query block qb)
@@ -1240,9 +1252,22 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
   }
 }
 
+// KS > 1: the last reduce_groups workgroups add the chunks of split key tiles (dkv_reduce). The two passes read what the
+// dK/dV kernel left and write different tensors, and a workgroup per tile leaves room for the other one where its tiles
+// are light: a launch and, in small calls, most of the sums' time less. (The pulling form, KS = 1, fills the device to
+// the end; there the sums have the device to themselves afterwards.) It uses no work counters and leaves them at zero.
 template <int D, int HS, int KS>
-__global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p) {
+__global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p, int reduce_groups) {
   extern __shared__ __align__(16) char smem_raw[];
+  if constexpr (KS > 1) {
+    typedef DkvReduceLds<kDqbWaves> ReduceLds;
+    static_assert(sizeof(ReduceLds) <= DsStage<D, KS>::kTotalBytes, "the sums' list and patches fit");
+    const int group = (int)blockIdx.x - ((int)gridDim.x - reduce_groups);
+    if (group >= 0) {
+      dkv_reduce<D, kDqbWaves>(p, group, reduce_groups, *reinterpret_cast<ReduceLds*>(smem_raw));
+      return;
+    }
+  }
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
   using Stage = DsStage<D, KS>;
