@@ -6,6 +6,7 @@
 
 #include "ct_attn_bwd_kernels.hip.h"
 #include "ct_attn_dkv_wide.hip.h"
+#include "ct_attn_fwd_shares.hip.h"
 #include "ct_attn_fwd_split.hip.h"
 #include "ct_attn_kernels.hip.h"
 #include "ct_error.h"
@@ -497,6 +498,15 @@ static int launch_fwd(hipStream_t stream, const AttnParams& p) {
   return scope1.done();
 }
 
+template <int D, int NW>
+static int launch_fwd_shares(hipStream_t stream, const AttnParams& p) {
+  const size_t smem = NW * ShareRegion<D>::kBytes;
+  CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_shares_kernel<D, NW>), smem);
+  LaunchScope scope("attn_fwd_shares_kernel", stream);
+  hipLaunchKernelGGL((attn_fwd_shares_kernel<D, NW>), dim3(p.Hq * p.B * (p.S / 32)), dim3(NW * 64), smem, stream, p);
+  return scope.done();
+}
+
 template <int D, int HS, int NW, int KS, int KB, int SUB>
 static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
   const size_t smem = SplitStage<D, NW, KS, KB, SUB>::kTotalBytes;
@@ -520,8 +530,13 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 // 1024 SIMDs). Few of them leave SIMDs idle while the longest row's chain of steps runs: its keys
 // are then shared by wavefronts. Where the lines lie was measured over row lengths 128 to 26496 and
 // documents from 36 positions to the whole row:
-//   head dimension 64: sharing by four wins up to 512 row blocks (half a wavefront per SIMD), sharing
-//     by two up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47 us).
+//   few row blocks: attn_fwd_shares_kernel as long as all its workgroups are on the device at once, two on a compute unit with
+//     four wavefronts at head dimension 128, four at 64. Past that short documents pay for a second round (128: [2, 4480, 2/2],
+//     560 row blocks, images 66 / 40 but documents of 32 to 64 positions 9.5 / 11.4; 64: [1, 3456, 8/2], 864, 7.6 / 8.0;
+//     at 560 and 640 7.8 / 7.5 and 7.6 / 7.5, images 45 / 30), and in rows below 512 positions there is little to share. Eight wavefronts, half as many on a
+//     compute unit, pay from 1024 positions on up to 256 and 512 row blocks (by four / eight: [1, 8192, 1/1, 128] 65 / 44,
+//     [1, 4096, 4/4, 64] 27 / 22, documents of 100 to 200 there 7.6 / 8.0; [1, 4096, 4/4, 128], 512 row blocks, such documents 8.7 / 12.6).
+//   head dimension 64: sharing by two wins up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47).
 //   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920); from there to 2304 the longest row's
 //     chain still counts in long rows (large launch / by two: [1, 4096, 16/16] with documents up to the row 58.5 / 42.0),
 //     but whole rows and short ones lose (44.0 / 48.9 at [2, 1536, 24/8], and [4, 768, 24/8] 26.4 by four-wavefront workgroups /
@@ -537,22 +552,17 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     [8, 2944, 8/8] 148 / 152, [4, 4096, 16/16] 260 / 271, [8, 2048, 32/16] 296 / 314; 12 KV heads, [16, 2560, 12/12] 360 /
 //     396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64] 392 / 417; image blocks in a call with ends,
 //     [8, 2304, 8/8] 88 / 103.
-//     Sharing by four takes a compute unit's LDS, so it wins as long as there is a workgroup per compute unit: up to
-//     256 row blocks with one in a workgroup (us, by two / by four: 33.5 / 22.9 at 136 with images; at 256, documents up to
-//     the row, 512 and 100: [1, 2048, 4/4] 23.9 / 17.1, 12.8 / 11.1, 8.8 / 8.7, [2, 512, 8/8] 11.8 / 10.1, 12.8 / 11.1, 7.8 / 8.8),
-//     up to 512 with two in rows of 1024 or more ([1, 2048, 8/8] 24.3 / 19.0, 13.2 / 12.4, 9.1 / 10.1, whole rows 33.6 / 25.2).
-//     Shorter rows have less of a chain to share (640 positions, documents up to 640 and 100: 12.9 / 12.2, 7.9 / 9.7), and with
-//     more row blocks short documents lose most ([2, 2048, 8/8] 26.4 / 26.2, 11.0 / 18.7).
 template <int D>
 static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   const long blocks = (long)p.B * p.Hq * (p.S / 32);
   if constexpr (D == 64) {
-    if (blocks <= 512) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
+    if (blocks <= 512) return p.S >= 1024 ? launch_fwd_shares<D, 8>(stream, p) : launch_fwd_shares<D, 4>(stream, p);
+    if (blocks <= 768 && p.S >= 512) return launch_fwd_shares<D, 4>(stream, p);
     if (blocks < 7168) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     return launch_fwd_split<D, 4, 1, 1, 2>(stream, p);
   } else {
-    if (blocks <= 256) return launch_fwd_split<D, 4, 4, 1, 1>(stream, p);
-    if (blocks <= 512 && p.S >= 1024) return launch_fwd_split<D, 8, 4, 1, 1>(stream, p);
+    if (blocks <= 256 && p.S >= 1024) return launch_fwd_shares<D, 8>(stream, p);
+    if (blocks <= 512) return launch_fwd_shares<D, 4>(stream, p);
     if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     const int hs = heads_per_group(p.Hq, p.Hkv);
     const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;

@@ -10,20 +10,16 @@
 //
 //   KS = 1  a wavefront takes all keys of its 32 query rows
 //   KS = 2  two wavefronts share them, 32 keys each per step: half the chain of steps per row
-//   KS = 4  four share them; a workgroup has one row block, or with NW = 8 two that share the staged keys
 //
-// For KS > 1 the sums are merged through LDS at the end (in a fixed order). A step stages
+// For KS = 2 the sums are merged through LDS at the end (in a fixed order). A step stages
 // SUB x KS x KB x 32 keys; a wavefront works on KB x 32 of them at a time, SUB times. 32 at a time
 // (KB = 1) keep the score registers few and skip what is masked in finer pieces.
 //
 // Measured, us (batch, row length, query / KV heads, head dimension, visible 64-key tiles per row on
 // average): before = the 8-wavefront workgroups
-//   (2, 1024, 8/8, 64, 2.0)        24.4 -> 10.2  KS = 4     (1, 2304, 1/1, 64, 18)   52.5 -> 16.2  KS = 4
 //   (2, 4096, 8/8, 64, 4.2)        37.3 -> 20.4  KS = 2     (3, 2944, 24/8, 64, 5.7) 72.7 -> 45.4  KS = 2
 //   (3, 4224, 48/8, 64, 2.3)      121.2 -> 68.9  KS = 1     (8, 4096, 32/8, 64, 32)   796 -> 660   KS = 1
 //   (3, 2560, 8/8, 128, 7.8)       55.3 -> 42.0  KS = 2     (6, 1280, 32/16, 128, 0.4) 61.1 -> 46.2  KS = 1
-// Head dimension 128 by four (KS = 2 -> 4; images of 1056 positions): (1, 2176, 2/2) 33.5 -> 22.9 NW = 4,
-//   (1, 2304, 6/1) 36.9 -> 27.6 NW = 8.
 #pragma once
 
 #include "ct_attn_kernels.hip.h"
@@ -48,7 +44,7 @@ struct SplitStage {
 };
 
 template <int D, int HS, int NW, int KS, int KB, int SUB>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : KB == 1 ? NW == 4 ? 3 : 2 : 2))) void
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : KB == 1 ? 3 : 2))) void
 attn_fwd_split_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr lds0 = lds_address_of(smem_raw);

@@ -411,7 +411,10 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     (2, 2560, 24, 8, 128), (2, 2688, 24, 8, 128), (2, 1664, 32, 16, 128), (2, 1792, 32, 16, 128), (2, 2048, 24, 8, 128),
     (2, 1920, 24, 8, 128), (8, 1536, 24, 8, 128), (9, 1408, 24, 8, 128),
     # 448 and 512 row blocks in rows of 896 and 1024 positions
-    (1, 896, 16, 16, 128), (1, 1024, 16, 8, 128)],
+    (1, 896, 16, 16, 128), (1, 1024, 16, 8, 128),
+    # a workgroup per row block: one row block per head and the most of them, by four wavefronts and by eight
+    (1, 128, 1, 1, 64), (1, 128, 1, 1, 128), (3, 896, 3, 1, 64), (1, 1024, 1, 1, 64), (1, 1024, 3, 1, 128), (1, 2048, 4, 2, 128),
+    (1, 8192, 2, 1, 64), (1, 3072, 8, 8, 64), (1, 3200, 8, 8, 64), (6, 512, 8, 8, 64), (8, 384, 8, 8, 64)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_forms_of_the_forward(ct, gpu, shape, with_ends):
