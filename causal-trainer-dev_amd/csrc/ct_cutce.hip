@@ -1347,9 +1347,28 @@ static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, bool panel_elsewhere
 static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
   return align_up((size_t)padded_rows(s.rows) * s.hidden * sizeof(float), 256);
 }
-// The whole vocabulary as one slab if that fits in `bytes`, else the largest slab that does
-// (slab_cols = 0 if even one tile column does not). The partial sums of a cut dHidden come last: as
-// many parts as fit behind one slab, with several slabs in up to half of what is left for slabs.
+// Estimated time (us) of a backward in slabs of `slab_tiles` tile columns with `spare` bytes for the partial sums of dHidden. A
+// group of 128 terms of a tile takes 2 us (256 x 256) or 1 (128 x 128); a dHidden unit walks all groups of its part, and without
+// room for parts a slab's few units leave the device idle (704 rows x 1152 x 41694 in four slabs: ten units of 160 us). A slab pays
+// for four launches and, in its dlogits, for one walk along the hidden size at least.
+static float slabs_time(const ct_cutce_shape& s, int slab_tiles, size_t spare, bool with_head) {
+  const int tile = gradient_tile(ct_cutce_shape{s.rows, s.hidden, slab_tiles * kGemmTile});
+  const int row_blocks = (s.rows + tile - 1) / tile, col_blocks = (s.hidden + tile - 1) / tile;
+  const float group = tile == kGemmTile ? 2.f : 1.f, slots = (float)(tile == kGemmTile ? kComputeUnits : 2 * kComputeUnits);
+  const float groups = 2.f * slab_tiles;
+  const float want = groups / part_length(tile, row_blocks, s.hidden, slab_tiles * kGemmTile, with_head);
+  const float fit = (float)(spare / ((size_t)row_blocks * tile * s.hidden * sizeof(float)));
+  const float parts = fmaxf(1.f, fminf(want, fit));
+  const float all = (with_head ? 2.f : 1.f) * row_blocks * col_blocks * groups / slots;
+  const float slab = fmaxf(groups / parts, all) * group + 20.f + s.hidden / 128.f;
+  return slab * ((vocab_tile_count(s.vocab) + slab_tiles - 1) / slab_tiles);
+}
+// The whole vocabulary as one slab if that fits in `bytes` with room for all parts of dHidden behind it, else the size
+// of a slab that takes the least time (slab_cols = 0 if not even one tile column fits). The partial sums of a cut
+// dHidden come last: as many parts as fit behind a slab. The largest slab that fits, or one down to half
+// of it where all parts then fit, and the present size (us of a pass; slabs): 638 x 256 x 133066 in chunks of 36 rows 2635 (16) / 731 (20),
+// 84 x 2432 x 132192 by 22 3735 (10) / 1117 (16), 290 x 768 x 141343 by 32, frozen head, 2620 (14) / 778 (20), 456 x 256 x 24749 by 23
+// 398 (13) / 405 (15), 5058 x 1024 x 108442 by 125 5960 / 5930 (as many).
 static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_elsewhere, bool with_head) {
   const int n_pad = padded_rows(s.rows);
   const int tiles = vocab_tile_count(s.vocab);
@@ -1364,17 +1383,20 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_el
   const size_t per_tile = tile.all(), acc_bytes = bwd_acc_bytes(s);
   size_t fit = tiles, room;
   L.head_most = with_head ? most_head_parts(s) : 1;
-  if (bytes < L.panel + per_tile * tiles) {
-    if (bytes < L.panel + acc_bytes + per_tile) return L;
-    room = bytes - L.panel - acc_bytes;
-    fit = room / per_tile;
-    for (size_t fewer = fit; fewer > fit / 2; fewer -= (fewer + 7) / 8) {
-      if (per_tile * fewer + hidden_sums_bytes(s, (int)fewer, with_head) > room) continue;
+  const bool whole = bytes >= L.panel + per_tile * tiles;
+  room = whole ? bytes - L.panel : 0;
+  if (!whole || room - per_tile * tiles < hidden_sums_bytes(s, tiles, with_head)) {
+    float least = whole ? slabs_time(s, tiles, room - per_tile * tiles, with_head) : __builtin_inff();
+    const size_t slabs_room = bytes < L.panel + acc_bytes ? 0 : bytes - L.panel - acc_bytes;
+    const size_t most = slabs_room / per_tile;
+    if (!whole && most == 0) return L;
+    for (size_t fewer = most < (size_t)tiles ? most : (size_t)tiles - 1; fewer > 0; fewer -= (fewer + 7) / 8) {
+      const float time = slabs_time(s, (int)fewer, slabs_room - per_tile * fewer, with_head);
+      if (time >= least) continue;
+      least = time;
       fit = fewer;
-      break;
+      room = slabs_room;
     }
-  } else {
-    room = bytes - L.panel;
   }
   const size_t want = hidden_sums_bytes(s, (int)fit, with_head), spare = (room - per_tile * fit) / 256 * 256;
   L.hidden_sums_bytes = want < spare ? want : spare;

@@ -255,6 +255,20 @@ def test_small_workspace_walks_vocabulary_slabs(ct, gpu):
         _gpu(ct, gpu, *case, 0.5, compaction=True, workspace=least - 256)
 
 
+@pytest.mark.parametrize("rows,width,vocab,chunk", [(300, 256, 20001, 30), (84, 384, 9000, 22), (260, 128, 4097, 200),
+                                                    (513, 128, 3000, 17)])
+def test_slabs_leave_room_for_the_parts_of_dhidden(ct, gpu, rows, width, vocab, chunk):
+    """A bounded workspace in slabs that are chosen by their time: few row blocks of long contractions, one slab without
+    room for all parts, more row blocks."""
+
+    case = _case(rows, rows, width, vocab)
+    workspace = ct.cut_cross_entropy.backward_workspace_bytes(rows, width, vocab, chunk)
+    one_slab = _gpu(ct, gpu, *case, 0.5, compaction=True)
+    slabs = _gpu(ct, gpu, *case, 0.5, compaction=True, workspace=workspace)
+    _check(slabs, *case, 0.5)
+    assert torch.equal(slabs[4], one_slab[4])
+
+
 def test_reference_seeded_fixture_and_frozen_head(ct, gpu):
     # inputs of the reference's tests/kernels/test_tiled_cut.py:66-128 (cotangent 0.37)
     golden = np.load("tests/golden/cutce_rng460.npz")
