@@ -682,7 +682,7 @@ static int launch_delta(hipStream_t stream, const bf16* out, const bf16* dout, f
 template <int D>
 static int launch_schedule(hipStream_t stream, const AttnParams& p, int kvh_side_by_side) {
   LaunchScope scope7("attn_dkv_schedule_kernel", stream);
-  hipLaunchKernelGGL(attn_dkv_schedule_kernel, dim3(1), dim3(1024), 0, stream, p, kvh_side_by_side);
+  hipLaunchKernelGGL(attn_dkv_schedule_kernel<D>, dim3(1), dim3(1024), 0, stream, p, kvh_side_by_side);
   return scope7.done();
 }
 

@@ -425,6 +425,7 @@ CT_DEVICE int dkv_split_count(int items, int target) {
 // Builds the dK/dV work list (one workgroup of 1024 threads): chunk target from
 // the total amount of work, chunk count per tile, entries bucketed by
 // decreasing work. Clears the dQ kernel's work counters.
+template <int D>
 CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int max_entries, int max_partials, int* header,
                             int2* entries, int* zeroed, int zeroed_count) {
   for (int i = threadIdx.x; i < zeroed_count; i += 1024) zeroed[i] = 0;  // dQ's work counters
@@ -481,6 +482,70 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   const long long pairs = (long long)ntiles * Hkv;  // (key tile, KV head)
   const int least = pairs <= kDkvSlots / 16 ? kDkvMinChunk / 4 : pairs <= kDkvSlots / 2 ? kDkvMinChunk / 2 : kDkvMinChunk;
   int target = (int)min((long long)INT_MAX / 2, max((long long)least, want));
+
+  // Where there are somewhat fewer tiles than slots the share is not always the best target: 432 tiles of 1.2 shares cut in two
+  // take two rounds of the slots, as long as they take whole in one, and leave 80 MB of partial sums to write, read and add. The
+  // target is the one of four with the least estimated end, in items: the longest chunk, or where there are more chunks than
+  // slots the one that is dealt second to the slot of the slots' shortest (twice its length), and the sums at 0.03 items per
+  // partial sum (131 KB written and read, an item 1.8 us). It has to be 8 % better than the share: a workgroup that is left alone on its compute
+  // unit at the end is the faster for it. Fewer tiles leave slots idle and are cut by the share, longer lists end evenly; at head
+  // dimension 64 shorter chunks gain more than half as large sums cost ([2, 10368, 12/2 of 64], documents of 50 to 414: dK/dV 46 us,
+  // by such an estimate 58). The whole pass, us: [3, 4480, 32/4 of 128], documents of
+  // 36 to 58, 317 -> 269; [2, 2048, 16/16], images, 222 -> 191; [1, 3456, 64/16], 87 to 178, 210 -> 184; 40 drawn shapes 0.99 to 1.18.
+  // (Counted a wavefront at a time: with an atomic per tile and target the list took 6 us more.)
+  if (D == 128 && pairs > kDkvSlots / 2 && pairs <= kDkvSlots) {
+    constexpr int kTargets = 4, kBuckets = 256;
+    __shared__ int chunks[kTargets * kBuckets];  // by length, the longest in the last one
+    __shared__ int split[kTargets], longest[kTargets];
+    __shared__ float ends[kTargets];
+    const auto candidate = [&](int k) { return (int)min((long long)INT_MAX / 4, (long long)target * (k == 3 ? 8 : 4 + k) / 4); };
+    const float bucket_items = (float)candidate(kTargets - 1) / kBuckets;
+    for (int i = tid; i < kTargets * kBuckets; i += 1024) chunks[i] = 0;
+    if (tid < kTargets) split[tid] = longest[tid] = 0;
+    __syncthreads();
+    const float buckets_per_item = 1.f / bucket_items;
+    if (wave * 64 < ntiles) {  // (at most kDkvSlots tiles: one per thread)
+      const int items = tid < ntiles ? items_first : 0;
+#pragma unroll
+      for (int k = 0; k < kTargets; ++k) {
+        const int ns = dkv_split_count(items, candidate(k)), per = (items + ns - 1) / ns;
+        if (items) atomicAdd(&chunks[k * kBuckets + min(kBuckets - 1, (int)((float)per * buckets_per_item))], ns);
+        const int parts = lane_value(wave_scan(ns > 1 ? ns : 0), 63), most = lane_value(wave_scan<true>(per), 63);
+        if (lane == 0) {
+          if (parts) atomicAdd(&split[k], parts);
+          atomicMax(&longest[k], most);
+        }
+      }
+    }
+    __syncthreads();
+    if (wave < kTargets) {  // a wavefront per target, four buckets per lane, the longest chunks in lane 0
+      int count[4], mine = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mine += count[j] = chunks[wave * kBuckets + (kBuckets - 1 - 4 * lane - j)];
+      const int upto = wave_scan(mine);
+      int second = 0;  // bucket of chunk kDkvSlots + 1, where it is one of this lane's
+      int before = upto - mine;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool here = (long long)before * Hkv <= kDkvSlots && (long long)(before + count[j]) * Hkv > kDkvSlots;
+        before += count[j];
+        if (here) second = kBuckets - 4 * lane - j;
+      }
+      second = lane_value(wave_scan<true>(second), 63);
+      const float chunk = (float)longest[wave];
+      if (lane == 0) ends[wave] = fmaxf(chunk, 2.f * (float)second * bucket_items) + 0.03f * (float)split[wave] * (float)Hkv;
+    }
+    __syncthreads();
+    float least_end = 0.92f * ends[0];
+    int best = target;
+#pragma unroll
+    for (int k = 1; k < kTargets; ++k)
+      if (ends[k] < least_end) {
+        least_end = ends[k];
+        best = candidate(k);
+      }
+    target = uniform(best);
+  }
 
   // Entry and partial-slot counts for this target; coarsen the target if they overflow the
   // space the host reserved (cannot happen for target >= want, kept as a guard).
@@ -558,8 +623,9 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   }
 }
 
+template <int D>
 __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, int kvh_side_by_side) {
-  dkv_schedule(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
+  dkv_schedule<D>(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
                p.dkv_entries, p.dq_counters, kDqCounters);
 }
 
@@ -569,7 +635,7 @@ __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, i
 template <int D>
 __global__ __launch_bounds__(1024) void attn_bwd_setup_kernel(AttnParams p, int kvh_side_by_side, float exponent_scale) {
   if (blockIdx.x == 0) {
-    dkv_schedule(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
+    dkv_schedule<D>(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
                  p.dkv_entries, p.dq_counters, kDqCounters);
     return;
   }

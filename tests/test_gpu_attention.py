@@ -739,6 +739,34 @@ def test_split_key_tiles_match_oracle(ct, gpu, bwd_variant):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("shape,max_len", [
+    # batch, seq, Hq, Hkv: 257 to 512 (key tile, KV head) pairs at head dimension 128, where the length of a chunk is chosen by
+    # the estimated end of the list: even tiles, one long document among short ones, no pair beyond the lines
+    ((1, 1152, 29, 29), 200), ((2, 2176, 16, 8), 160), ((4, 1024, 18, 9), 1024), ((1, 2176, 32, 16), 2176), ((2, 2048, 32, 16), 60),
+    ((1, 2176, 64, 32), 100)], ids=str)
+def test_chunk_length_by_the_lists_end(ct, gpu, bwd_variant, shape, max_len):
+    """dK / dV (and what else a pass gives) of one batch row and KV head against the oracle; the same bits on every call."""
+
+    batch, seq, q_heads, kv_heads = shape
+    rng = np.random.default_rng(seq + kv_heads)
+    generator = torch.Generator().manual_seed(seq)
+    q, k, v, dout = (torch.randn((batch, seq, heads, 128), generator=generator).to(torch.bfloat16)
+                     for heads in (q_heads, kv_heads, kv_heads, q_heads))
+    ids = _layout(rng, batch, seq, max_len=max_len)
+    ids[-1, seq - 300:] = 0
+    results = _run_gpu(ct, gpu, q, k, v, dout, ids, None, 128 ** -0.5)
+    again = _run_gpu(ct, gpu, q, k, v, dout, ids, None, 128 ** -0.5)
+    assert all(torch.equal(a, b) for a, b in zip(results, again))
+    head, group, row = kv_heads // 2, q_heads // kv_heads, slice(batch - 1, batch)
+    heads, own = slice(head * group, (head + 1) * group), slice(head, head + 1)
+    cut = lambda t: t[row, :, heads if t.shape[2] == q_heads else own]  # noqa: E731
+    out, lse, dq, dk, dv = results
+    if q_heads == kv_heads:
+        heads = own
+    _check_against_oracle((cut(out), lse[row, :, heads], cut(dq), cut(dk), cut(dv)), cut(q), cut(k), cut(v), cut(dout),
+                          ids[row], None, 128 ** -0.5)
+
+
 def _visit_ranges_of_canonical_ids(ids_row, ends_row):
     """Columns 5..8 of the tile table (first / last 64-key tile a 32-row query block visits, first /
     last query block that visits a 32-key block) for one row of canonical ids, i.e. nonzero ids
