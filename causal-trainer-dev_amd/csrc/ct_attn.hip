@@ -576,21 +576,28 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   }
 }
 
-// Workgroups of the persistent dQ kernels: 64 per (head slice, KV head) group, two per compute
+// Workgroups of the persistent dQ kernels: 64 or 96 per (head slice, KV head) group, two or three per compute
 // unit when there are 8 groups; more per group when a pass has fewer groups than that.
-static int dq_grid(const AttnParams& p, int hs) {
+static int dq_grid(const AttnParams& p, int hs, int per_unit = 2) {
   const int groups = ((p.Hq / p.Hkv) / hs) * p.kvh_count;
-  const int members = groups >= 8 ? 2 * kBins : (2 * kBins * 8 + groups - 1) / groups;
+  const int members = groups >= 8 ? per_unit * kBins : (per_unit * kBins * 8 + groups - 1) / groups;
   return groups * members;
 }
 
-template <int D, int HS>
+template <int D, int HS, int PER_UNIT>
 static int launch_dq(hipStream_t stream, const AttnParams& p) {
   const size_t smem = 2 * KvStage<D>::kBytes;
-  CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_kernel<D, HS>), smem);
+  CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_kernel<D, HS, PER_UNIT>), smem);
   LaunchScope scope2("attn_dq_kernel", stream);
-  hipLaunchKernelGGL((attn_dq_kernel<D, HS>), dim3(dq_grid(p, HS)), dim3(256), smem, stream, p);
+  hipLaunchKernelGGL((attn_dq_kernel<D, HS, PER_UNIT>), dim3(dq_grid(p, HS, PER_UNIT)), dim3(256), smem, stream, p);
   return scope2.done();
+}
+// (where the line lies: attn_dq_kernel)
+template <int D, int HS>
+static int launch_dq(hipStream_t stream, const AttnParams& p) {
+  if constexpr (D == 64)
+    if ((long)p.B * p.Hq * (p.S / 32) >= 12288) return launch_dq<D, HS, 3>(stream, p);
+  return launch_dq<D, HS, 2>(stream, p);
 }
 
 // `reduce`: the launch also adds the chunks of split key tiles, where its form can (KS > 1). 128 workgroups of eight

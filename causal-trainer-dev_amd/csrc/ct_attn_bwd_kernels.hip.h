@@ -55,7 +55,7 @@ CT_DEVICE void dq_arith(f32x16& s, const f32x16& dp, float lse2) {
 }
 
 // One query tile (4 / HS row blocks x HS heads of one KV head), start to finish.
-template <int D, int HS>
+template <int D, int HS, int PER_UNIT>
 CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int qt, const lds_addr lds_base) {
   constexpr int kStage = KvStage<D>::kBytes;
   // (the fragment pointers are rebuilt per item from an opaque base: kept across the item loop
@@ -177,31 +177,39 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
         half_tile(std::integral_constant<int, 0>{});
         half_tile(std::integral_constant<int, 1>{});
       } else {
-        f32x16 s[2], dp[2];
+        // Both 32-key blocks at once, or one after the other where registers are for three workgroups on a compute unit.
         // (dP starts from -delta, a register block of its own, and needs no subtraction)
-        constexpr int kSteps = D / 16;
-        fragments_ahead<4 * kSteps, 6>(
-            [&](int i) { return ro.load(i < 2 * kSteps ? kOff : vOff, i & 1, i / 2 % kSteps); },
-            [&](int i, bf16x8 keys) {
-              const int kb = i & 1, ks = i / 2 % kSteps;
-              if (i < 2 * kSteps) s[kb] = mfma32(keys, qf[ks], ks ? s[kb] : zero16());
-              else dp[kb] = mfma32(keys, dof[ks], ks ? dp[kb] : minus_delta);
-            });
-        request();
-        if (need_seg || need_causal) {
-          if (k_uniform == 0) mask_scores_t<true, true>(stage + KvStage<D>::kSeg, seg_cmp, last_rel, s);
-          else mask_scores_t<false, true>(stage, seg_cmp, last_rel, s);
-        }
-        dq_arith(s[0], dp[0], lse2);
-        dq_arith(s[1], dp[1], lse2);
-        bf16x8 ds[4];
+        constexpr int kSteps = D / 16, kBlocks = D / 32, N = PER_UNIT == 2 ? 2 : 1;
+        auto blocks = [&](auto first_tag) {
+          constexpr int FIRST = decltype(first_tag)::value;
+          f32x16 s[N], dp[N];
+          fragments_ahead<2 * N * kSteps, N == 2 ? 6 : 4>(
+              [&](int i) { return ro.load(i < N * kSteps ? kOff : vOff, FIRST + i % N, i / N % kSteps); },
+              [&](int i, bf16x8 keys) {
+                const int kb = i % N, ks = i / N % kSteps;
+                if (i < N * kSteps) s[kb] = mfma32(keys, qf[ks], ks ? s[kb] : zero16());
+                else dp[kb] = mfma32(keys, dof[ks], ks ? dp[kb] : minus_delta);
+              });
+          if constexpr (FIRST == 0) request();
+          if (need_seg || need_causal) {
 #pragma unroll
-        for (int step = 0; step < 4; ++step) ds[step] = pack_acc8(s[step >> 1], step & 1);
-        constexpr int kBlocks = D / 32;
-        fragments_ahead<4 * kBlocks, 4>([&](int i) { return to.load(kOff, i / kBlocks, i % kBlocks); },
-                                        [&](int i, bf16x8 keys) {
-                                          dqacc[i % kBlocks] = mfma32(keys, ds[i / kBlocks], dqacc[i % kBlocks]);
-                                        });
+            for (int i = 0; i < N; ++i) {
+              if (k_uniform == 0) mask_block_t<true, true>(stage + KvStage<D>::kSeg, seg_cmp, last_rel, FIRST + i, s[i]);
+              else mask_block_t<false, true>(stage, seg_cmp, last_rel, FIRST + i, s[i]);
+            }
+          }
+          bf16x8 ds[2 * N];
+#pragma unroll
+          for (int i = 0; i < N; ++i) dq_arith(s[i], dp[i], lse2);
+#pragma unroll
+          for (int i = 0; i < 2 * N; ++i) ds[i] = pack_acc8(s[i >> 1], i & 1);
+          fragments_ahead<2 * N * kBlocks, 4>([&](int i) { return to.load(kOff, 2 * FIRST + i / kBlocks, i % kBlocks); },
+                                              [&](int i, bf16x8 keys) {
+                                                dqacc[i % kBlocks] = mfma32(keys, ds[i / kBlocks], dqacc[i % kBlocks]);
+                                              });
+        };
+        blocks(std::integral_constant<int, 0>{});
+        if constexpr (N == 1) blocks(std::integral_constant<int, 1>{});
       }
     }
     ahead.pin();
@@ -234,8 +242,14 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
 // of a tile depends on its mix of masked and unmasked key tiles, not just on their number.)
 // The group is the fast index of blockIdx: a group stays on one XCD and its K / V rows in that
 // XCD's L2. With more groups than counters (kDqCounters) the tiles are dealt round robin.
-template <int D, int HS>
-__global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnParams p) {
+//
+// PER_UNIT workgroups on a compute unit: at head dimension 64 two, or for large launches three (168 registers: the wavefronts
+// of a SIMD wait less for each other's products, but each takes a tile's two blocks one after the other and has more to do per
+// query tile). dQ, us, two / three: [1, 25472, 64/8 heads of 64], images, 1289 / 1186; [6, 2816, 64/16], images, 692 / 642; [4, 4096, 64/8]
+// 374 / 342; [4, 4992, 48/8], documents of 99 to 152, 160 / 151. Below 12288 row blocks short documents lose more than long ones
+// gain: [4, 5376, 16/16], 10752, 45 to 111, 74 / 81, [1, 17280, 12/4], 6480, 121 to 236, 49 / 55, [1, 16384, 16/2], whole rows, 813 / 752.
+template <int D, int HS, int PER_UNIT>
+__global__ __launch_bounds__(256, PER_UNIT) void attn_dq_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
@@ -259,7 +273,7 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnParams p) {
     if (pull >= total) break;
     const int b = pull % p.B, rank = pull / p.B;
     const int qt = uniform(sched[(size_t)b * schedule_ints(nrb) + rank]);
-    attn_dq_item<D, HS>(p, b, kvh, slice, qt, lds0);
+    attn_dq_item<D, HS, PER_UNIT>(p, b, kvh, slice, qt, lds0);
   }
 }
 

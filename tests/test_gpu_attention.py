@@ -1064,7 +1064,9 @@ def test_benchmark_shapes(ct, gpu, name, bwd_variant):
     # a row are shared by four wavefronts (768), two (3072 for D = 128, 8192 for D = 64) or none, in groups of 1, 2, 4 heads
     (1, 128, 1, 1, 128), (2, 384, 4, 4, 64), (2, 768, 16, 4, 128), (3, 1024, 8, 4, 64),
     (1, 896, 28, 28, 128), (2, 1024, 14, 7, 64), (3, 2048, 16, 4, 128), (2, 1920, 68, 17, 64),
-    (1, 2048, 49, 49, 128), (1, 2176, 122, 61, 64), (1, 3200, 84, 21, 64)],
+    (1, 2048, 49, 49, 128), (1, 2176, 122, 61, 64), (1, 3200, 84, 21, 64),
+    # and the recomputing form with three workgroups per compute unit: 12288 row blocks at D = 64 in the same groups
+    (4, 1024, 96, 24, 64), (4, 1024, 96, 48, 64), (6, 1024, 64, 64, 64), (3, 1408, 93, 31, 64)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_forms_of_dq_from_stored_blocks(ct, gpu, shape, with_ends):
