@@ -19,7 +19,7 @@
 namespace ct {
 
 // ---------------------------------------------------------------------------
-// Tile bounds, in three launches, two for short rows: the summary of every 32-position block; from a row's summaries, what
+// Tile bounds, in three launches, two for short rows, one for few positions: the summary of every 32-position block; from a row's summaries, what
 // each block has to visit; from those ranges, the work-sorted schedules, the dS offsets and the bins.
 //
 // All of it is latency: the searches and the ranking are quadratic in a row's blocks, and one
@@ -59,6 +59,43 @@ struct BlockIds {
   }
 };
 
+// What the searches read of the records of n blocks from position `first` on (of one row or of several, one behind the other):
+// four lanes per block, eight positions each.
+CT_DEVICE void search_records(const int* seg, const int* end, size_t first, int S, int n, int* min_nz, int* max_id, int* end_max) {
+  const int nrb = S / 32, quarter = threadIdx.x % 4;
+  for (int i0 = threadIdx.x / 4; i0 < n; i0 += 512) {  // (n is a multiple of 4: whole rows of 16 lanes)
+    int id[2][8], e[2][8];  // two blocks in flight
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const size_t at = first + (size_t)(i0 + 256 * j < n ? i0 + 256 * j : i0) * 32 + quarter * 8;
+      __builtin_memcpy(id[j], seg + at, sizeof id[j]);
+      if (end) __builtin_memcpy(e[j], end + at, sizeof e[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = i0 + 256 * j;
+      if (i >= n) break;
+      const int pos = i % nrb * 32 + quarter * 8;
+      int low = INT_MAX, high = 0, last = -1;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const bool counts = id[j][k] != 0;
+        low = min(low, counts ? id[j][k] : INT_MAX);
+        high = max(high, id[j][k]);
+        last = max(last, counts ? (end ? e[j][k] : pos + k) : -1);
+      }
+      low = min_over(low, 4);
+      high = max_over(high, 4);
+      last = max_over(last, 4);
+      if (quarter == 0) {
+        min_nz[i] = high == 0 ? 0 : low;
+        max_id[i] = high;
+        end_max[i] = last;
+      }
+    }
+  }
+}
+
 // grid (ceil(S / 1024), B)
 __global__ __launch_bounds__(1024) void attn_blocks_kernel(const int* seg, const int* end, int S, int* meta) {
   const int b = blockIdx.y, pos = blockIdx.x * 1024 + threadIdx.x;
@@ -73,6 +110,47 @@ struct SummaryOut {
   int block, width;  // width 3: with the largest visible end
 };
 
+// 16 lanes share the search of a block: the first and last 64-key tile that row block rb has to visit as queries, and the first
+// and last 32-row query block that it is visited by as keys; all of the lanes get them.
+constexpr int kSearchLanes = 16;
+struct VisitRange {
+  int first = INT_MAX, last = -1;
+  CT_DEVICE void add(int i) {
+    first = min(first, i);
+    last = i;
+  }
+  CT_DEVICE void over_lanes() {
+    first = min_over(first, kSearchLanes);
+    last = max_over(last, kSearchLanes);
+  }
+};
+template <class MinNz, class MaxId, class EndMax>
+CT_DEVICE VisitRange visited_tiles(MinNz min_nz, MaxId max_id, EndMax end_max, int S, int rb, int lane) {
+  VisitRange range;
+  const int my_min = min_nz(rb), my_max = max_id(rb), my_end = end_max(rb);
+  if (my_min != 0) {
+    const int t_hi = min(my_end / kKeyTile, S / kKeyTile - 1);
+    for (int t = lane; t <= t_hi; t += kSearchLanes) {
+      const int a_min = min_nz(2 * t), c_min = min_nz(2 * t + 1);
+      const int k_min = a_min == 0 ? c_min : (c_min == 0 ? a_min : min(a_min, c_min));
+      const int k_max = max(max_id(2 * t), max_id(2 * t + 1));
+      if (blocks_interact(my_min, my_max, my_end, k_min, k_max, t * kKeyTile)) range.add(t);
+    }
+  }
+  range.over_lanes();
+  return range;
+}
+template <class MinNz, class MaxId, class EndMax>
+CT_DEVICE VisitRange visiting_blocks(MinNz min_nz, MaxId max_id, EndMax end_max, int S, int rb, int lane) {
+  VisitRange range;
+  const int my_min = min_nz(rb), my_max = max_id(rb);
+  if (my_min != 0)
+    for (int qb = lane; qb < S / 32; qb += kSearchLanes)
+      if (blocks_interact(min_nz(qb), max_id(qb), end_max(qb), my_min, my_max, rb * 32)) range.add(qb);
+  range.over_lanes();
+  return range;
+}
+
 // grid (ceil(nrb / 64), B): 16 lanes per block search what it has to visit; the workgroups of a row also
 // write its block summaries. With `seg` every workgroup forms the records of its whole row by itself and stores its
 // own: a launch and its latency less than with attn_blocks_kernel in front, for rows of up to kFusedRows positions
@@ -82,20 +160,15 @@ constexpr int kFusedRows = 8192;
 // LDS is compiled apart: one pointer to either kind of memory makes every access a flat one ([4, 16384] 13.8 -> 8.2 us,
 // [1, 32768] 25.1 -> 14.0).
 template <bool LDS>
-__global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, SummaryOut queries, SummaryOut keys,
-                                                           const int* seg, const int* end) {
-  extern __shared__ __align__(16) int lds_rows[];  // [3][nrb]: min_nz, max_id, end_max of the row's blocks
-  const int b = blockIdx.y, nrb = S / 32, nt = S / kKeyTile;
+CT_DEVICE void build_ranges(int* meta, int S, const SummaryOut& queries, const SummaryOut& keys, const int* seg, const int* end,
+                            int part, int parts, int b, int* lds_rows) {  // lds_rows [3][nrb]: min_nz, max_id, end_max
+  const int nrb = S / 32;
   int* mb = meta + (size_t)b * nrb * kMetaW;
   if (LDS && seg) {
-    for (int pos = threadIdx.x; pos < S; pos += 1024) {  // (S % 128 == 0: whole wavefronts)
+    search_records(seg, end, (size_t)b * S, S, nrb, lds_rows, lds_rows + nrb, lds_rows + 2 * nrb);
+    for (int pos = part * 2048 + threadIdx.x; pos < min(S, (part + 1) * 2048); pos += 1024) {  // (S % 128 == 0: whole wavefronts)
       const BlockIds block(seg, end, (size_t)b * S, pos);
-      const int i = pos / 32;
-      if (pos % 32) continue;
-      lds_rows[i] = block.min_nz;
-      lds_rows[nrb + i] = block.max_id;
-      lds_rows[2 * nrb + i] = block.end_max;
-      if (i / 64 == (int)blockIdx.x) block.store(mb + i * kMetaW);
+      if (pos % 32 == 0) block.store(mb + pos / 32 * kMetaW);
     }
     __syncthreads();
   } else if (LDS) {
@@ -110,41 +183,17 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, Sum
   auto max_id = [&](int i) { return LDS ? lds_rows[nrb + i] : mb[i * kMetaW + kMaxId]; };
   auto end_max = [&](int i) { return LDS ? lds_rows[2 * nrb + i] : mb[i * kMetaW + kEndMax]; };
 
-  constexpr int kLanes = 16;
-  const int lane = threadIdx.x % kLanes, rb = blockIdx.x * (1024 / kLanes) + threadIdx.x / kLanes;
+  constexpr int kLanes = kSearchLanes;
+  const int lane = threadIdx.x % kLanes, rb = part * (1024 / kLanes) + threadIdx.x / kLanes;
   if (rb < nrb) {
-    const int my_min = min_nz(rb), my_max = max_id(rb), my_end = end_max(rb);
-    int kv_first = INT_MAX, kv_last = -1, q_first = INT_MAX, q_last = -1;
-    if (my_min != 0) {
-      // As queries: which 64-key tiles?
-      const int t_hi = min(my_end / kKeyTile, nt - 1);
-      for (int t = lane; t <= t_hi; t += kLanes) {
-        const int a_min = min_nz(2 * t), c_min = min_nz(2 * t + 1);
-        const int k_min = a_min == 0 ? c_min : (c_min == 0 ? a_min : min(a_min, c_min));
-        const int k_max = max(max_id(2 * t), max_id(2 * t + 1));
-        if (blocks_interact(my_min, my_max, my_end, k_min, k_max, t * kKeyTile)) {
-          kv_first = min(kv_first, t);
-          kv_last = t;
-        }
-      }
-      // As keys: which 32-row query blocks?
-      for (int qb = lane; qb < nrb; qb += kLanes) {
-        if (blocks_interact(min_nz(qb), max_id(qb), end_max(qb), my_min, my_max, rb * 32)) {
-          q_first = min(q_first, qb);
-          q_last = qb;
-        }
-      }
-    }
-    kv_first = min_over(kv_first, kLanes);
-    kv_last = max_over(kv_last, kLanes);
-    q_first = min_over(q_first, kLanes);
-    q_last = max_over(q_last, kLanes);
+    const VisitRange tiles = visited_tiles(min_nz, max_id, end_max, S, rb, lane);
+    const VisitRange blocks = visiting_blocks(min_nz, max_id, end_max, S, rb, lane);
     if (lane == 0) {
       int* m = mb + rb * kMetaW;
-      m[kKvFirst] = kv_first;
-      m[kKvLast] = kv_last;
-      m[kQFirst] = q_first;
-      m[kQLast] = q_last;
+      m[kKvFirst] = tiles.first;
+      m[kKvLast] = tiles.last;
+      m[kQFirst] = blocks.first;
+      m[kQLast] = blocks.last;
     }
   }
 
@@ -152,7 +201,7 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, Sum
     const SummaryOut& summary = side ? keys : queries;
     if (!summary.block) continue;
     const int per = summary.block / 32, count = S / summary.block, groups = 1024 / kLanes;
-    for (int i = blockIdx.x * groups + threadIdx.x / kLanes; i < count; i += gridDim.x * groups) {
+    for (int i = part * groups + threadIdx.x / kLanes; i < count; i += parts * groups) {
       int low = INT_MAX, high = 0, last = 0;
       for (int k = i * per + lane; k < (i + 1) * per; k += kLanes) {
         if (min_nz(k) != 0) low = min(low, min_nz(k));
@@ -170,6 +219,12 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, Sum
       }
     }
   }
+}
+template <bool LDS>
+__global__ __launch_bounds__(1024) void attn_ranges_kernel(int* meta, int S, SummaryOut queries, SummaryOut keys,
+                                                           const int* seg, const int* end) {
+  extern __shared__ __align__(16) int lds_rows[];
+  build_ranges<LDS>(meta, S, queries, keys, seg, end, blockIdx.x, gridDim.x, blockIdx.y, lds_rows);
 }
 
 // The working arrays are in LDS or, for rows beyond 262144 positions and for many tiles, in the metadata buffer's
@@ -204,24 +259,38 @@ CT_DEVICE int rank_of(const int* w, int n, int i, int lanes) {
   for (int k = head + 4 * quads + lane; k < n; k += lanes) count(w[k], k);
   return sum_over(rank, lanes);
 }
-// Tiles between the first and the last that row blocks first .. end - 1 have to visit (`from`: kKvFirst or
-// kQFirst, followed by the last).
-CT_DEVICE int visit_span(const int* mb, int first_block, int end_block, int from) {
+// What the row blocks of a row have to visit, as queries (64-key tiles) or as keys (32-row query blocks): from the table ...
+struct TableRanges {
+  const int* row;
+  int from;  // kKvFirst or kQFirst, followed by the last
+  CT_DEVICE int first(int rb) const { return row[rb * kMetaW + from]; }
+  CT_DEVICE int last(int rb) const { return row[rb * kMetaW + from + 1]; }
+};
+// ... or from LDS, where a workgroup has searched them by itself.
+struct LocalRanges {
+  const int *firsts, *lasts;
+  CT_DEVICE int first(int rb) const { return firsts[rb]; }
+  CT_DEVICE int last(int rb) const { return lasts[rb]; }
+};
+// Tiles between the first and the last that row blocks first .. end - 1 have to visit.
+template <class Ranges>
+CT_DEVICE int visit_span(const Ranges& ranges, int first_block, int end_block) {
   int first = INT_MAX, last = -1;
   for (int k = first_block; k < end_block; ++k) {
-    first = min(first, mb[k * kMetaW + from]);
-    last = max(last, mb[k * kMetaW + from + 1]);
+    first = min(first, ranges.first(k));
+    last = max(last, ranges.last(k));
   }
   return last >= first ? last - first + 1 : 0;
 }
 
 // One of the five schedules of a batch row: query tiles of 1, 2, 4 row blocks, 128-key tiles, query
 // tiles of 8.
-template <bool LDS>
-CT_DEVICE void build_schedule(int job, const int* mb, int nrb, int* sched, int* work) {
+// (`ranges`: the row's, as keys for job 3, else as queries)
+template <bool LDS, class Ranges>
+CT_DEVICE void build_schedule(int job, const Ranges& ranges, int nrb, int* sched, int* work) {
   const int pb = job == 3 ? 4 : job == 4 ? 8 : 1 << job, n = job == 4 ? (nrb + 7) / 8 : nrb / pb;
   for (int i = threadIdx.x; i < n; i += 1024)
-    work[i] = TileWork<LDS>::pack(visit_span(mb, i * pb, min(nrb, (i + 1) * pb), job == 3 ? kQFirst : kKvFirst), i);
+    work[i] = TileWork<LDS>::pack(visit_span(ranges, i * pb, min(nrb, (i + 1) * pb)), i);
   __syncthreads();
   const int lanes = lanes_per_item(n, 1024);
   int* out = sched + (job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, pb));
@@ -234,12 +303,13 @@ CT_DEVICE void build_schedule(int job, const int* mb, int nrb, int* sched, int* 
 // Where the dS blocks of each key block of a row start (kDsOff): exclusive prefix sum of the lengths of
 // the query-block ranges. Every thread sums a contiguous run of row blocks, the runs are
 // scanned across the workgroup, and each thread then walks its run again.
-CT_DEVICE void build_ds_offsets(int* mb, int nrb) {
+template <class Ranges>
+CT_DEVICE void build_ds_offsets(const Ranges& ranges, int* mb, int nrb) {
   __shared__ long long wave_sum[16];
   const int per = (nrb + 1023) / 1024, lane = threadIdx.x & 63;
   const int lo = min(nrb, (int)threadIdx.x * per), hi = min(nrb, lo + per);
   long long local = 0;
-  for (int rb = lo; rb < hi; ++rb) local += visit_span(mb, rb, rb + 1, kQFirst);
+  for (int rb = lo; rb < hi; ++rb) local += visit_span(ranges, rb, rb + 1);
   long long incl = local;
   for (int off = 1; off < 64; off <<= 1) {
     const long long below = __shfl_up(incl, off, 64);
@@ -251,7 +321,7 @@ CT_DEVICE void build_ds_offsets(int* mb, int nrb) {
   for (int k = 0; k < (int)threadIdx.x >> 6; ++k) run += wave_sum[k];
   for (int rb = lo; rb < hi; ++rb) {
     mb[rb * kMetaW + kDsOff] = (int)min(run, (long long)INT_MAX);
-    run += visit_span(mb, rb, rb + 1, kQFirst);
+    run += visit_span(ranges, rb, rb + 1);
   }
 }
 
@@ -302,8 +372,9 @@ CT_DEVICE unsigned long long sent_to(unsigned long long v, int to) {
 // to 32 tiles is a chain of some 800 clocks: 32 comparisons for the ranks, one exchange through LDS, a running minimum by lane
 // moves. Nine rounds at four rows of 4096 (256 tiles); with shuffles, unpacked loads and arrays behind generic pointers a
 // round took 2500 and the kernel 15.2 us, now 8.0.
-template <bool LDS>
-CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
+// `ranges_of(b)`: what the row blocks of batch row b have to visit as queries.
+template <bool LDS, class RangesOf>
+CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins, RangesOf ranges_of) {
   typedef std::conditional_t<LDS, unsigned, unsigned long long> Key;
   __shared__ int start[kBins + 1];
   const int nrb = S / 32;
@@ -314,9 +385,8 @@ CT_DEVICE void build_bins(int* meta, int B, int S, int pb, int* lds_bins) {
   int* region = meta + bin_region_offset(B, nrb, pb);
   for (int i = threadIdx.x; i < n; i += 1024) {
     const int b = i / tpr, qt = i % tpr;
-    const int* mb = meta + (size_t)b * nrb * kMetaW;
     // a tile without keys still costs a launch of the prologue; +3 ~ prologue and store
-    work[i] = TileWork<LDS>::pack(visit_span(mb, qt * pb, min(nrb, (qt + 1) * pb), kKvFirst) + 3, i);
+    work[i] = TileWork<LDS>::pack(visit_span(ranges_of(b), qt * pb, min(nrb, (qt + 1) * pb)) + 3, i);
   }
   __syncthreads();
   const int lanes = lanes_per_item(n, 1024);
@@ -383,19 +453,68 @@ __global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, 
   const int nrb = S / 32;
   if (blockIdx.x < 3) {
     const int pb = 2 << blockIdx.x;
-    if (bins_scratch) build_bins<false>(meta, B, S, pb, bins_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2));
-    else build_bins<true>(meta, B, S, pb, lds_work);
+    const auto ranges_of = [&](int b) { return TableRanges{meta + (size_t)b * nrb * kMetaW, kKvFirst}; };
+    if (bins_scratch) build_bins<false>(meta, B, S, pb, bins_scratch + (size_t)blockIdx.x * 3 * B * bin_tiles_per_row(nrb, 2), ranges_of);
+    else build_bins<true>(meta, B, S, pb, lds_work, ranges_of);
     return;
   }
   const int b = (blockIdx.x - 3) / 6, job = (blockIdx.x - 3) % 6;
   int* mb = meta + (size_t)b * nrb * kMetaW;
+  const TableRanges ranges = {mb, job == 3 || job == 5 ? kQFirst : kKvFirst};
   if (job == 5) {
-    build_ds_offsets(mb, nrb);
+    build_ds_offsets(ranges, mb, nrb);
   } else {
     const int offset = job == 3 ? key_schedule_offset(nrb) : query_schedule_offset(nrb, job == 4 ? 8 : 1 << job);
     int* sched = sched_all + (size_t)b * schedule_ints(nrb);
-    if (row_scratch) build_schedule<false>(job, mb, nrb, sched, row_scratch + (size_t)b * 3 * nrb + offset);
-    else build_schedule<true>(job, mb, nrb, sched, lds_work);
+    if (row_scratch) build_schedule<false>(job, ranges, nrb, sched, row_scratch + (size_t)b * 3 * nrb + offset);
+    else build_schedule<true>(job, ranges, nrb, sched, lds_work);
+  }
+}
+
+// Ranges, schedules, offsets and bins in one launch: a workgroup that needs the ranges of a row (or, for the bins, of all
+// rows) forms the records and searches them by itself, the one side that it needs. That repeats work on compute units that have none,
+// and saves a launch and the wait between two. grid: the bins' three workgroups, six per batch row, then build_ranges' ones.
+// LDS, ints: 3 + 2 per row block that a workgroup searches, then its working arrays. Us of GPU time, two launches / one, and 2.3 of
+// the host's: [1, 128] 6.6 / 3.9, [2, 1024] 7.7 / 4.5, [1, 8192] 12.5 / 8.5, [3, 2944] 10.4 / 9.1, [4, 4096] 13.1 / 14.0 (a batch's preparation
+// as a whole 31.0 / 28.9). Past the lines the bins' search of the whole batch is the longest, or a long row's: [1, 12160] 17.4 / 20.3.
+constexpr int kOneLaunchPositions = 16384;
+__global__ __launch_bounds__(1024) void attn_prepare_kernel(int* meta, int B, int S, SummaryOut queries, SummaryOut keys,
+                                                            const int* seg, const int* end, int* sched_all) {
+  extern __shared__ __align__(16) int lds[];
+  const int nrb = S / 32, parts = (nrb + 63) / 64;
+  int index = blockIdx.x;
+  if (index >= 3 + 6 * B) {
+    index -= 3 + 6 * B;
+    build_ranges<true>(meta, S, queries, keys, seg, end, index % parts, parts, index / parts, lds);
+    return;
+  }
+  const bool bins = index < 3;
+  const int job = bins ? 0 : (index - 3) % 6, row0 = bins ? 0 : (index - 3) / 6, rows = bins ? B : 1, n = rows * nrb;
+  const bool as_keys = job == 3 || job == 5;
+  int *mins = lds, *maxs = lds + n, *ends = lds + 2 * n, *firsts = lds + 3 * n, *lasts = lds + 4 * n, *work = lds + 5 * n;
+  search_records(seg, end, (size_t)row0 * S, S, n, mins, maxs, ends);
+  __syncthreads();
+  const int lane = threadIdx.x % kSearchLanes;
+  for (int i = threadIdx.x / kSearchLanes; i < n; i += 1024 / kSearchLanes) {
+    const int first_of_row = i / nrb * nrb;
+    const auto min_nz = [&](int k) { return mins[first_of_row + k]; };
+    const auto max_id = [&](int k) { return maxs[first_of_row + k]; };
+    const auto end_max = [&](int k) { return ends[first_of_row + k]; };
+    const VisitRange range = as_keys ? visiting_blocks(min_nz, max_id, end_max, S, i - first_of_row, lane)
+                                     : visited_tiles(min_nz, max_id, end_max, S, i - first_of_row, lane);
+    if (lane == 0) {
+      firsts[i] = range.first;
+      lasts[i] = range.last;
+    }
+  }
+  __syncthreads();
+  const LocalRanges ranges = {firsts, lasts};
+  if (bins) {
+    build_bins<true>(meta, B, S, 2 << index, work, [&](int b) { return LocalRanges{firsts + b * nrb, lasts + b * nrb}; });
+  } else if (job == 5) {
+    build_ds_offsets(ranges, meta + (size_t)row0 * nrb * kMetaW, nrb);
+  } else {
+    build_schedule<true>(job, ranges, nrb, sched_all + (size_t)row0 * schedule_ints(nrb), work);
   }
 }
 
@@ -786,6 +905,14 @@ static int32_t prepare_on(const char* fn, void* stream, const int32_t* segment_i
   }
   int* bins_scratch = bins_fit_lds(batch, nrb) ? nullptr : scratch;
   hipStream_t st = (hipStream_t)stream;
+  if ((long)batch * seq <= kOneLaunchPositions && seq <= kFusedRows) {
+    const int tiles = batch * bin_tiles_per_row(nrb, 2);
+    const size_t smem = ((size_t)5 * batch * nrb + (3 * tiles > nrb ? 3 * tiles : nrb)) * sizeof(int);
+    LaunchScope scope("attn_prepare_kernel", st);
+    hipLaunchKernelGGL(attn_prepare_kernel, dim3(3 + 6 * batch + (nrb + 63) / 64 * batch), dim3(1024), smem, st, tile_meta, batch, seq,
+                       queries, keys, segment_ids, attention_end, tile_meta + (size_t)batch * nrb * kMetaW);
+    return scope.done();
+  }
   const bool fused = seq <= kFusedRows;
   if (!fused) {
     LaunchScope scope5("attn_blocks_kernel", st);

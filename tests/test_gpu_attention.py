@@ -739,6 +739,37 @@ def test_split_key_tiles_match_oracle(ct, gpu, bwd_variant):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("batch,seq", [(129, 128), (33, 512), (9, 1920), (6, 2944), (5, 4096), (3, 8064), (3, 8192)])
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_metadata_of_a_row_is_that_of_the_row_alone(ct, gpu, batch, seq, with_ends):
+    """Batches of more than 16384 positions take two launches, their rows by themselves one: the same tables, schedules and
+    summaries. The ids lie at an address that is a multiple of 4 bytes only."""
+
+    rng = np.random.default_rng(batch + seq)
+    ids = _layout(rng, batch, seq, holes=True, max_len=seq // 2)
+    ids[0], ids[-1, seq // 3:] = 1, 0
+    ends = _random_ends(rng, ids, 9) if with_ends else None
+    def odd(values):  # noqa: E306
+        buffer = torch.zeros(values.size + 1, dtype=torch.int32, device=gpu)
+        buffer[1:] = torch.from_numpy(np.ascontiguousarray(values)).to(gpu).flatten()
+        return buffer[1:].view(values.shape)
+    def metadata(rows):  # noqa: E306
+        count = len(range(batch)[rows])
+        profile = ct.resolve_attention_profile((count, seq, 2, 64), (count, seq, 2, 64), None, has_attention_end=with_ends)
+        return ct.prepare_attention_metadata(odd(ids[rows]), mesh=None, profile=profile,
+                                             attention_end=odd(ends[rows]) if with_ends else None)
+    blocks, scheduled = seq // 32, 2 * (seq // 32) + seq // 128
+    def schedules(m, count, row):  # noqa: E306
+        return m.tile_bounds[count * blocks * 12:][row * scheduled:][:2 * blocks + (blocks + 7) // 8]
+    whole = metadata(slice(None))
+    for row in sorted({0, 1, batch // 2, batch - 1}):
+        alone = metadata(slice(row, row + 1))
+        assert torch.equal(ct.tile_bounds_table(alone)[0], ct.tile_bounds_table(whole)[row])
+        assert torch.equal(schedules(alone, 1, 0), schedules(whole, batch, row))
+        assert torch.equal(alone.q_block_segments[0], whole.q_block_segments[row])
+        assert torch.equal(alone.kv_block_segments[0], whole.kv_block_segments[row])
+
+
 @pytest.mark.parametrize("shape,max_len", [
     # batch, seq, Hq, Hkv: 257 to 512 (key tile, KV head) pairs at head dimension 128, where the length of a chunk is chosen by
     # the estimated end of the list: even tiles, one long document among short ones, no pair beyond the lines
