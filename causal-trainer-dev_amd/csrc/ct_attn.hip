@@ -475,9 +475,11 @@ __global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, 
 // rows) forms the records and searches them by itself, the one side that it needs. That repeats work on compute units that have none,
 // and saves a launch and the wait between two. grid: the bins' three workgroups, six per batch row, then build_ranges' ones.
 // LDS, ints: 3 + 2 per row block that a workgroup searches, then its working arrays. Us of GPU time, two launches / one, and 2.3 of
-// the host's: [1, 128] 6.6 / 3.9, [2, 1024] 7.7 / 4.5, [1, 8192] 12.5 / 8.5, [3, 2944] 10.4 / 9.1, [4, 4096] 13.1 / 14.0 (a batch's preparation
-// as a whole 31.0 / 28.9). Past the lines the bins' search of the whole batch is the longest, or a long row's: [1, 12160] 17.4 / 20.3.
-constexpr int kOneLaunchPositions = 16384;
+// the host's: [1, 128] 6.6 / 3.9, [2, 1024] 7.7 / 4.5, [1, 8192] 12.5 / 8.5, [3, 2944] 10.4 / 9.1. Past the lines the bins' search of the
+// whole batch is the longest, or a long row's: [4, 4096] 13.1 / 14.0 (a batch's preparation as a whole 28.2 / 30.0 where the host keeps
+// ahead), [1, 12160] 17.4 / 20.3. (A wavefront per row block with a key tile per lane and a ballot: a chain of LDS reads per
+// block, [4, 4096] 19.7.)
+constexpr int kOneLaunchPositions = 12288;
 __global__ __launch_bounds__(1024) void attn_prepare_kernel(int* meta, int B, int S, SummaryOut queries, SummaryOut keys,
                                                             const int* seg, const int* end, int* sched_all) {
   extern __shared__ __align__(16) int lds[];

@@ -742,7 +742,7 @@ def test_split_key_tiles_match_oracle(ct, gpu, bwd_variant):
 @pytest.mark.parametrize("batch,seq", [(129, 128), (33, 512), (9, 1920), (6, 2944), (5, 4096), (3, 8064), (3, 8192)])
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_metadata_of_a_row_is_that_of_the_row_alone(ct, gpu, batch, seq, with_ends):
-    """Batches of more than 16384 positions take two launches, their rows by themselves one: the same tables, schedules and
+    """Batches of more than 12288 positions take two launches, their rows by themselves one: the same tables, schedules and
     summaries. The ids lie at an address that is a multiple of 4 bytes only."""
 
     rng = np.random.default_rng(batch + seq)
