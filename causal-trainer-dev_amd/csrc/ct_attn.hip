@@ -657,6 +657,13 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     at 560 and 640 7.8 / 7.5 and 7.6 / 7.5, images 45 / 30), and in rows below 512 positions there is little to share. Eight wavefronts, half as many on a
 //     compute unit, pay from 1024 positions on up to 256 and 512 row blocks (by four / eight: [1, 8192, 1/1, 128] 65 / 44,
 //     [1, 4096, 4/4, 64] 27 / 22, documents of 100 to 200 there 7.6 / 8.0; [1, 4096, 4/4, 128], 512 row blocks, such documents 8.7 / 12.6).
+//     Three wavefronts at head dimension 128 (three workgroups on a compute unit, 768 at once) where every head has its own keys, in
+//     rows of 1024 positions or more (by two wavefronts with shared stages / by three; documents of 32 to 64, 100 to 200, 400 to 500,
+//     whole rows): [1, 4608, 4/4], 576 row blocks, 9.8 / 8.8, 10.7 / 9.6, 16.0 / 12.8, 68 / 51; [1, 6144, 4/4], 768, 10.7 / 9.7, 11.1 /
+//     11.1, 16.9 / 13.9, 91 / 71; [1, 9216, 2/2], 576, 9.8 / 9.2, 11.0 / 10.1, 16.3 / 13.6, 141 / 95. Below 540 the shortest documents lose
+//     ([1, 4224, 4/4], 528, 8.2 / 8.6). Heads in no multiple of four put keys of all heads on every XCD and lose from 600 on
+//     ([1, 7424, 3/3], 696, 100 to 200, 11.7 / 13.3), shared keys with short documents (they are staged for every head:
+//     [1, 2304, 8/2], 576, 8.2 / 8.7, though 14.7 / 12.0 and 37 / 29 with longer ones), and so does a second round (832, 10.8 / 12.5).
 //   head dimension 64: sharing by two wins up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47).
 //   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920); from there to 2304 the longest row's
 //     chain still counts in long rows (large launch / by two: [1, 4096, 16/16] with documents up to the row 58.5 / 42.0),
@@ -684,6 +691,8 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   } else {
     if (blocks <= 256 && p.S >= 1024) return launch_fwd_shares<D, 8>(stream, p);
     if (blocks <= 512) return launch_fwd_shares<D, 4>(stream, p);
+    if (p.Hq == p.Hkv && p.S >= 1024 && blocks > 536 && blocks <= (p.Hq % 4 == 0 ? 768 : 592))
+      return launch_fwd_shares<D, 3>(stream, p);
     if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
     const int hs = heads_per_group(p.Hq, p.Hkv);
     const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;

@@ -414,7 +414,9 @@ def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     (1, 896, 16, 16, 128), (1, 1024, 16, 8, 128),
     # a workgroup per row block: one row block per head and the most of them, by four wavefronts and by eight
     (1, 128, 1, 1, 64), (1, 128, 1, 1, 128), (3, 896, 3, 1, 64), (1, 1024, 1, 1, 64), (1, 1024, 3, 1, 128), (1, 2048, 4, 2, 128),
-    (1, 8192, 2, 1, 64), (1, 3072, 8, 8, 64), (1, 3200, 8, 8, 64), (6, 512, 8, 8, 64), (8, 384, 8, 8, 64)],
+    (1, 8192, 2, 1, 64), (1, 3072, 8, 8, 64), (1, 3200, 8, 8, 64), (6, 512, 8, 8, 64), (8, 384, 8, 8, 64),
+    # by three, which share the columns of a row unevenly: the first and the last row blocks, and launches beside them
+    (2, 2176, 4, 4, 128), (1, 1408, 12, 12, 128), (2, 1536, 8, 8, 128), (1, 3200, 8, 8, 128), (1, 9216, 2, 2, 128), (2, 3200, 3, 3, 128)],
     ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_forms_of_the_forward(ct, gpu, shape, with_ends):
