@@ -686,13 +686,17 @@ struct DkvReduceLds {
   int wave_count[4][WAVES];
   __align__(16) bf16 patches[WAVES][32 * 32];
 };
-// Workgroup `group` of `groups`, WAVES wavefronts each (four or eight).
+// Workgroup `group` of `groups`, WAVES wavefronts each (four or eight). Every backward call ends with a launch that does this, and
+// it leaves the dQ kernels' work counters at zero, so that a later call on the same workspace can keep the work list and skip
+// the kernel that builds it (and clears the counters). Nothing in such a launch uses them; an earlier pass of the call may have.
 template <int D, int WAVES>
 CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceLds<WAVES>& lds) {
   constexpr int kMaxSplitTiles = DkvReduceLds<WAVES>::kMaxSplitTiles;
   constexpr int kPieces = 2 * 4 * (D / 32);      // (tensor, wavefront of the dK/dV kernel, 32 columns)
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
+  if (group == 0)
+    for (int i = threadIdx.x; i < kDqCounters; i += 64 * WAVES) p.dq_counters[i] = 0;
   const int entries = uniform(p.dkv_header[0]);
   int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
   for (int base = 0; base < entries; base += 256 * WAVES) {
@@ -786,14 +790,10 @@ CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceL
   }
 }
 
-// On its own, the last kernel of a backward call: it also leaves the dQ kernel's work counters at zero,
-// so that a later call on the same workspace can keep the work list and skip the kernel that
-// builds it (and clears the counters).
+// On its own, the last kernel of a backward call.
 template <int D>
 __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(AttnParams p) {
   __shared__ DkvReduceLds<4> lds;
-  if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i < kDqCounters; i += blockDim.x) p.dq_counters[i] = 0;
   dkv_reduce<D, 4>(p, blockIdx.x, gridDim.x, lds);
 }
 
@@ -1335,7 +1335,7 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
 // KS > 1: the last reduce_groups workgroups add the chunks of split key tiles (dkv_reduce). The two passes read what the
 // dK/dV kernel left and write different tensors, and a workgroup per tile leaves room for the other one where its tiles
 // are light: a launch and, in small calls, most of the sums' time less. (The pulling form, KS = 1, fills the device to
-// the end; there the sums have the device to themselves afterwards.) It uses no work counters and leaves them at zero.
+// the end; there the sums have the device to themselves afterwards.) It uses no work counters.
 template <int D, int HS, int KS>
 __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p, int reduce_groups) {
   extern __shared__ __align__(16) char smem_raw[];

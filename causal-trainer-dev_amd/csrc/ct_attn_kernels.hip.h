@@ -54,7 +54,7 @@ struct AttnParams {
   // dK/dV work list (backward only)
   int* dkv_header;
   int2* dkv_entries;
-  int* dq_counters;  // kDqCounters ints, zeroed by the work-list kernel of the same call
+  int* dq_counters;  // kDqCounters ints, zeroed by the work-list kernel and with the sums that end a call
   float* dkv_partials;
   int dkv_max_entries, dkv_max_partials;
   // KV heads [kvh_base, kvh_base + kvh_count) are what a backward launch works on (all of them

@@ -260,6 +260,44 @@ def test_kept_work_list(ct, gpu, form):
     assert built == [True, False, False, True, False], launches
 
 
+@pytest.mark.parametrize("shape,first_pass", [
+    # (batch, seq, query / KV heads, head dimension), KV heads of the first of two passes: its dQ kernel pulls its tiles, the last
+    # one's has a workgroup per tile and adds the chunks of split key tiles
+    ((1, 4096, 26, 26, 128), 25), ((1, 4096, 72, 72, 64), 70), ((2, 2048, 36, 9, 128), 8)], ids=str)
+def test_kept_work_list_of_several_passes(ct, gpu, shape, first_pass):
+    """A call whose passes over the KV heads take different forms of the dQ kernel leaves the work counters at zero as
+    every call does: with the kept list the next one gives the bits of a call without."""
+
+    from causal_trainer_dev_amd import profiling
+
+    batch, seq, q_heads, kv_heads, dim = shape
+    library = ct._lib.load()
+    one_pass = int(library.ct_attn_bwd_workspace_bytes_from_ds(batch, seq, q_heads, kv_heads, dim, 0))
+    per_head = (one_pass - int(library.ct_attn_bwd_workspace_bytes(batch, seq, q_heads, kv_heads, dim))) // kv_heads
+    room = one_pass - (kv_heads - first_pass) * per_head + per_head // 2
+    ids = torch.from_numpy(_layout(np.random.default_rng(seq), batch, seq, max_len=900)).to(gpu)
+    profile = ct.resolve_attention_profile((batch, seq, q_heads, dim), (batch, seq, kv_heads, dim), None, has_attention_end=False)
+    metadata = ct.prepare_attention_metadata(ids, mesh=None, profile=profile)
+    kept = ct.BackwardWorkspace()
+    generator = torch.Generator().manual_seed(dim)
+    for call in range(3):
+        q, k, v, dout = (torch.randn((batch, seq, heads, dim), generator=generator).to(torch.bfloat16).to(gpu)
+                         for heads in (q_heads, kv_heads, kv_heads, q_heads))
+        out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+        print(shape, "call", call, flush=True)
+        expected = ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="from_ds", workspace_bytes=room)
+        stale = torch.full_like(q, float("nan"))    # (what the result's memory holds)
+        del stale
+        with profiling.KernelTimer() as timer:
+            got = ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="from_ds", workspace_bytes=room,
+                                        workspace=kept)
+        launches = timer.durations_ms()
+        assert len(launches["attn_dq_blocks_kernel"]) == 2
+        assert ("attn_bwd_stats_kernel" in launches) == (call > 0)
+        for name, a, b in zip(("dq", "dk", "dv"), expected, got):
+            assert torch.equal(a, b), (call, name)
+
+
 def _kept_list_layers(ct, gpu):
     """A layer's backward with a shared workspace and without one: ``layer(metadata, kept)`` runs both and compares."""
 
