@@ -22,6 +22,7 @@
 // The cache is vocabulary-major [vocab, rows] like G^T: in the transposed tile
 // the GEMMs produce, the lanes of a wavefront run along the rows, so both are
 // written with contiguous stores.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -912,7 +913,10 @@ __host__ __device__ inline float part_length(int tile, int row_blocks, int d, in
   const float least = __builtin_sqrtf((tile == kGemmTile ? 0.05f : 0.026f) * total);
   return share > least ? share : least;
 }
-__host__ __device__ inline int whole_parts(float parts) { return parts < 1.5f ? 1 : parts > 64.f ? 64 : (int)(parts + 0.5f); }
+constexpr int kMostParts = 64;
+__host__ __device__ inline int whole_parts(float parts) {
+  return parts < 1.5f ? 1 : parts > (float)kMostParts ? kMostParts : (int)(parts + 0.5f);
+}
 
 CT_DEVICE int hidden_parts(const CutceSplits& sp, int tile, int n_act, int d, int slab_width) {
   const int row_blocks = (n_act + tile - 1) / tile;
@@ -1311,6 +1315,11 @@ static size_t hidden_sums_bytes(const ct_cutce_shape& s, int slab_tiles, bool wi
   const size_t chosen = hidden_sums_bytes(s, gradient_tile(s), slab_tiles, with_head);
   return large > chosen ? large : chosen;
 }
+// What kMostParts parts take, with the tile of a slab of this size: more room than that is never used.
+static size_t most_hidden_sums_bytes(const ct_cutce_shape& s, int slab_tiles) {
+  const int tile = gradient_tile(ct_cutce_shape{s.rows, s.hidden, slab_tiles * kGemmTile});
+  return (size_t)kMostParts * ((s.rows + tile - 1) / tile) * tile * s.hidden * sizeof(float);
+}
 static int most_head_parts(const ct_cutce_shape& s, int tile) {
   const int row_blocks = (s.rows + tile - 1) / tile;
   return whole_parts((float)(row_blocks * (tile / 128)) /
@@ -1348,27 +1357,36 @@ static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
   return align_up((size_t)padded_rows(s.rows) * s.hidden * sizeof(float), 256);
 }
 // Estimated time (us) of a backward in slabs of `slab_tiles` tile columns with `spare` bytes for the partial sums of dHidden. A
-// group of 128 terms of a tile takes 2 us (256 x 256) or 1 (128 x 128); a dHidden unit walks all groups of its part, and without
-// room for parts a slab's few units leave the device idle (704 rows x 1152 x 41694 in four slabs: ten units of 160 us). A slab pays
-// for four launches and, in its dlogits, for one walk along the hidden size at least.
+// group of 128 terms of a tile takes 2 us (256 x 256; 1.5 where a hidden size of 128 leaves half of it empty) or 1 (128 x 128). A
+// dHidden unit walks all groups of its part, of which there are kMostParts at most: without room for parts a slab's few units
+// leave the device idle (704 rows x 1152 x 41694 in four slabs: ten units of 160 us). A dHead unit walks its part of the
+// rows in every slab, however narrow, in parts that the whole vocabulary has set; those chains have the device almost to themselves and
+// take 0.6 of the time per group. A slab pays for four launches, for large sums to write, read and add (8 bytes per part and element, at
+// 5 TB/s) and, in its dlogits, for one walk along the hidden size at least. Us of a pass with the chains, the large sums and the
+// most parts left out / counted, and the largest slab that fits: 4180 x 896 x 42590 in chunks of 469 rows 1950 / 1390, 1390;
+// 4270 x 512 x 26982 by 439 1595 / 895, 898; 9149 x 256 x 8364 by 1887 513 / 400, 509; 3556 x 256 x 89215 by 297 1464 / 1247, 1818;
+// 13 x 256 x 102429 by 10, frozen head, 114 / 97, 97; 100 drawn shapes where the choice differs 0.56 to 1.12 times, 0.92 in the mean.
 static float slabs_time(const ct_cutce_shape& s, int slab_tiles, size_t spare, bool with_head) {
-  const int tile = gradient_tile(ct_cutce_shape{s.rows, s.hidden, slab_tiles * kGemmTile});
+  const int tile = gradient_tile(ct_cutce_shape{s.rows, s.hidden, slab_tiles * kGemmTile}), head_tile = gradient_tile(s);
   const int row_blocks = (s.rows + tile - 1) / tile, col_blocks = (s.hidden + tile - 1) / tile;
-  const float group = tile == kGemmTile ? 2.f : 1.f, slots = (float)(tile == kGemmTile ? kComputeUnits : 2 * kComputeUnits);
-  const float groups = 2.f * slab_tiles;
+  const float group = tile != kGemmTile ? 1.f : s.hidden > 128 ? 2.f : 1.5f;
+  const float slots = (float)(tile == kGemmTile ? kComputeUnits : 2 * kComputeUnits), groups = 2.f * slab_tiles;
   const float want = groups / part_length(tile, row_blocks, s.hidden, slab_tiles * kGemmTile, with_head);
   const float fit = (float)(spare / ((size_t)row_blocks * tile * s.hidden * sizeof(float)));
-  const float parts = fmaxf(1.f, fminf(want, fit));
+  const float parts = fmaxf(1.f, fminf(fminf(want, (float)kMostParts), fit));
+  const float row_groups = (float)((s.rows + head_tile - 1) / head_tile * (head_tile / 128));
+  const float head_chain = with_head ? 0.6f * row_groups / most_head_parts(s, head_tile) : 0.f;
   const float all = (with_head ? 2.f : 1.f) * row_blocks * col_blocks * groups / slots;
-  const float slab = fmaxf(groups / parts, all) * group + 20.f + s.hidden / 128.f;
+  const float sums = (parts < 1.5f ? 1.f : 1.f + parts) * s.rows * s.hidden * (8.f / 5e6f);
+  const float slab = fmaxf(fmaxf(groups / parts, head_chain), all) * group + fmaxf(20.f, 5.f + sums) + s.hidden / 128.f;
   return slab * ((vocab_tile_count(s.vocab) + slab_tiles - 1) / slab_tiles);
 }
 // The whole vocabulary as one slab if that fits in `bytes` with room for all parts of dHidden behind it, else the size
 // of a slab that takes the least time (slab_cols = 0 if not even one tile column fits). The partial sums of a cut
 // dHidden come last: as many parts as fit behind a slab. The largest slab that fits, or one down to half
-// of it where all parts then fit, and the present size (us of a pass; slabs): 638 x 256 x 133066 in chunks of 36 rows 2635 (16) / 731 (20),
-// 84 x 2432 x 132192 by 22 3735 (10) / 1117 (16), 290 x 768 x 141343 by 32, frozen head, 2620 (14) / 778 (20), 456 x 256 x 24749 by 23
-// 398 (13) / 405 (15), 5058 x 1024 x 108442 by 125 5960 / 5930 (as many).
+// of it where all parts then fit, and the present size (us of a pass): 638 x 256 x 133066 in chunks of 36 rows, 18 slabs now, 2500 / 709,
+// 84 x 2432 x 132192 by 22, 4, 3516 / 913, 290 x 768 x 141343 by 32, frozen head, 12, 2420 / 732, 456 x 256 x 24749 by 23, 14,
+// 432 / 388, 5058 x 1024 x 108442 by 125, 39, 5105 / 5100.
 static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_elsewhere, bool with_head) {
   const int n_pad = padded_rows(s.rows);
   const int tiles = vocab_tile_count(s.vocab);
@@ -1385,7 +1403,8 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_el
   L.head_most = with_head ? most_head_parts(s) : 1;
   const bool whole = bytes >= L.panel + per_tile * tiles;
   room = whole ? bytes - L.panel : 0;
-  if (!whole || room - per_tile * tiles < hidden_sums_bytes(s, tiles, with_head)) {
+  const size_t all_sums = std::min(hidden_sums_bytes(s, tiles, with_head), most_hidden_sums_bytes(s, tiles));
+  if (!whole || room - per_tile * tiles < all_sums) {
     float least = whole ? slabs_time(s, tiles, room - per_tile * tiles, with_head) : __builtin_inff();
     const size_t slabs_room = bytes < L.panel + acc_bytes ? 0 : bytes - L.panel - acc_bytes;
     const size_t most = slabs_room / per_tile;

@@ -269,6 +269,26 @@ def test_slabs_leave_room_for_the_parts_of_dhidden(ct, gpu, rows, width, vocab, 
     assert torch.equal(slabs[4], one_slab[4])
 
 
+@pytest.mark.parametrize("rows,width,vocab,chunk,trainable,slabs", [
+    # 64 parts of dHidden fit behind one slab of the whole vocabulary, and no more are ever made
+    (13, 256, 102429, 10, False, 1), (15, 128, 145924, 13, True, 1),
+    # dHead's chains along the rows are walked once per slab; large partial sums
+    (5542, 256, 23076, 698, True, 7), (5246, 1280, 12486, 2202, False, 2)])
+def test_number_of_slabs_of_a_bounded_workspace(ct, gpu, rows, width, vocab, chunk, trainable, slabs):
+    """The vocabulary is walked in no more slabs than is faster (the launches of a backward tell); a wider call's gradients."""
+
+    hidden, head, targets, weights = (t.to(gpu) for t in _case(rows, rows, width, vocab))
+    _, _, lse = ct.cutce_forward(hidden, head, targets, weights)
+    workspace = ct.cut_cross_entropy.backward_workspace_bytes(rows, width, vocab, chunk)
+    arguments = (hidden, head, targets, weights, lse, torch.ones(1))
+    with ct.profiling.KernelTimer() as timer:
+        bounded = ct.cutce_backward(*arguments, lm_head_trainable=trainable, workspace_bytes=workspace)
+    assert len(timer.durations_ms()["cutce_dlogits_kernel"]) == slabs
+    whole = ct.cutce_backward(*arguments, lm_head_trainable=trainable)
+    assert relative_l2(bounded[0], whole[0]) <= 2.0 ** -8     # (f32 sums in another order, rounded to bf16 once)
+    assert not trainable or torch.equal(bounded[1], whole[1])
+
+
 def test_reference_seeded_fixture_and_frozen_head(ct, gpu):
     # inputs of the reference's tests/kernels/test_tiled_cut.py:66-128 (cotangent 0.37)
     golden = np.load("tests/golden/cutce_rng460.npz")
