@@ -782,8 +782,8 @@ def test_split_key_tiles_match_oracle(ct, gpu, bwd_variant):
 @pytest.mark.parametrize("batch,seq", [(129, 128), (33, 512), (9, 1920), (6, 2944), (5, 4096), (3, 8064), (3, 8192)])
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_metadata_of_a_row_is_that_of_the_row_alone(ct, gpu, batch, seq, with_ends):
-    """Batches of more than 12288 positions take two launches, their rows by themselves one: the same tables, schedules and
-    summaries. The ids lie at an address that is a multiple of 4 bytes only."""
+    """Batches of more than 12288 positions take two launches, their rows by themselves, and as many of them as fit that line, one:
+    the same tables, schedules and summaries. The ids lie at an address that is a multiple of 4 bytes only."""
 
     rng = np.random.default_rng(batch + seq)
     ids = _layout(rng, batch, seq, holes=True, max_len=seq // 2)
@@ -802,12 +802,14 @@ def test_metadata_of_a_row_is_that_of_the_row_alone(ct, gpu, batch, seq, with_en
     def schedules(m, count, row):  # noqa: E306
         return m.tile_bounds[count * blocks * 12:][row * scheduled:][:2 * blocks + (blocks + 7) // 8]
     whole = metadata(slice(None))
-    for row in sorted({0, 1, batch // 2, batch - 1}):
-        alone = metadata(slice(row, row + 1))
-        assert torch.equal(ct.tile_bounds_table(alone)[0], ct.tile_bounds_table(whole)[row])
-        assert torch.equal(schedules(alone, 1, 0), schedules(whole, batch, row))
-        assert torch.equal(alone.q_block_segments[0], whole.q_block_segments[row])
-        assert torch.equal(alone.kv_block_segments[0], whole.kv_block_segments[row])
+    several = min(batch, 12288 // seq)
+    for start, count in [(row, 1) for row in sorted({0, 1, batch // 2, batch - 1})] + [(0, several), (batch - several, several)]:
+        part = metadata(slice(start, start + count))
+        assert torch.equal(ct.tile_bounds_table(part), ct.tile_bounds_table(whole)[start:start + count])
+        assert torch.equal(part.q_block_segments, whole.q_block_segments[start:start + count])
+        assert torch.equal(part.kv_block_segments, whole.kv_block_segments[start:start + count])
+        for row in range(count):
+            assert torch.equal(schedules(part, count, row), schedules(whole, batch, start + row))
 
 
 @pytest.mark.parametrize("shape,max_len", [
@@ -1001,11 +1003,14 @@ def test_schedules_are_the_stable_order_by_work(ct, gpu, batch, seq):
 
 
 @pytest.mark.parametrize("batch,seq,rate", [(1, 128, 0.01), (2, 1152, 0.02), (4, 4096, 0.002), (3, 8320, 0.0), (1, 262144 + 128, 0.001),
-                                            (40, 21632, 0.002), (41, 21376, 0.002), (41, 21376, 0.0), (4, 262144 + 128, 0.001)])
+                                            (40, 21632, 0.002), (41, 21376, 0.002), (41, 21376, 0.0), (4, 262144 + 128, 0.001),
+                                            # several rows of a batch that takes one launch, and the first that takes two
+                                            (96, 128, 0.02), (97, 128, 0.02), (3, 2944, 0.003), (12, 1024, 0.01), (1, 8192, 0.002),
+                                            (3, 4096, 0.0)])
 def test_work_bins_are_the_greedy_packing(ct, gpu, batch, seq, rate):
     """Longest tile first onto the least loaded bin, ties to the lowest: fewer tiles than bins, rows of equal and of
     padded tiles (whose loads tie), many rounds, and both forms of the packer: 13520 tiles are the most here that stay in
-    LDS with keys of 32 bits, 13694 and more go to the scratch region with keys of 64 (the last three shapes)."""
+    LDS with keys of 32 bits, 13694 and more go to the scratch region with keys of 64 (41 rows, and four beyond 262144)."""
 
     import heapq
 
