@@ -28,6 +28,7 @@ namespace ct {
 
 template <int D, int NW, int KS, int KB, int SUB>
 struct SplitStage {
+  static_assert(KS <= 2, "the merge is one hand-over");
   static constexpr int kKeys = SUB * KS * KB * 32;  // keys per step
   static constexpr int kTileBytes = kKeys * D * 2;
   static constexpr int kK = 0;
@@ -236,42 +237,34 @@ attn_fwd_split_kernel(AttnParams p) {
   }
   __syncthreads();  // the stages become hand-over space and store patches
 
-  if constexpr (KS > 1) {
+  if constexpr (KS == 2) {  // share 1 of a row block hands its sums to share 0
+    const lds_addr sums = lds0 + slot * Stage::kMergeBytes, row = sums + l * 16, stats = sums + D * 128 + l * 4;
+    if (share == 1) {
 #pragma unroll
-    for (int live = KS / 2; live > 0; live /= 2) {
-      // shares [live, 2 live) of a row block hand their sums to [0, live)
-      const lds_addr sums = lds0 + ((share % live) * kSlots + slot) * Stage::kMergeBytes;
-      const lds_addr row = sums + l * 16, stats = sums + D * 128 + l * 4;
-      if (share >= live && share < 2 * live) {
+      for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-          for (int qd = 0; qd < 4; ++qd)
-            lds_store<f32x4>(row + (db * 4 + qd) * 1024,
-                             f32x4{oacc[db][4 * qd], oacc[db][4 * qd + 1], oacc[db][4 * qd + 2], oacc[db][4 * qd + 3]});
-        lds_store<float>(stats, m_run);
-        lds_store<float>(stats + 256, l_run);
-      }
-      __syncthreads();
-      if (share < live) {
-        const float m_other = lds_load<float>(stats), l_other = lds_load<float>(stats + 256);
-        const float m_new = fmaxf(m_run, m_other);
-        const float m_use = m_new == kNegInf ? 0.f : m_new;
-        const float mine_by = exp2_fast(m_run - m_use), other_by = exp2_fast(m_other - m_use);
-        l_run = l_run * mine_by + l_other * other_by;
-        m_run = m_new;
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-          for (int qd = 0; qd < 4; ++qd) {
-            const f32x4 o = lds_load<f32x4>(row + (db * 4 + qd) * 1024);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) oacc[db][4 * qd + e] = oacc[db][4 * qd + e] * mine_by + o[e] * other_by;
-          }
-      }
-      if (live > 1) __syncthreads();
+        for (int qd = 0; qd < 4; ++qd)
+          lds_store<f32x4>(row + (db * 4 + qd) * 1024,
+                           f32x4{oacc[db][4 * qd], oacc[db][4 * qd + 1], oacc[db][4 * qd + 2], oacc[db][4 * qd + 3]});
+      lds_store<float>(stats, m_run);
+      lds_store<float>(stats + 256, l_run);
     }
+    __syncthreads();
     if (share != 0) return;
+    const float m_other = lds_load<float>(stats), l_other = lds_load<float>(stats + 256);
+    const float m_new = fmaxf(m_run, m_other);
+    const float m_use = m_new == kNegInf ? 0.f : m_new;
+    const float mine_by = exp2_fast(m_run - m_use), other_by = exp2_fast(m_other - m_use);
+    l_run = l_run * mine_by + l_other * other_by;
+    m_run = m_new;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        const f32x4 o = lds_load<f32x4>(row + (db * 4 + qd) * 1024);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[db][4 * qd + e] = oacc[db][4 * qd + e] * mine_by + o[e] * other_by;
+      }
   }
 
   const float l_tot = pair_sum(l_run);

@@ -174,12 +174,6 @@ CT_DEVICE void mask_block_t(lds_addr segk, int seg_q_or_never, int last_rel, int
     }
   }
 }
-template <bool SEG, bool CAUSAL>
-CT_DEVICE void mask_scores_t(lds_addr segk, int seg_q_or_never, int last_rel, f32x16* s) {
-  mask_block_t<SEG, CAUSAL>(segk, seg_q_or_never, last_rel, 0, s[0]);
-  mask_block_t<SEG, CAUSAL>(segk, seg_q_or_never, last_rel, 1, s[1]);
-}
-
 // Write a transposed accumulator (D x 32 rows) as bf16 rows of D elements to
 // global memory, staged through this wavefront's private LDS patch so that
 // the global stores are 16 bytes per lane and contiguous per row.
