@@ -501,13 +501,15 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
   // take two rounds of the slots, as long as they take whole in one, and leave 80 MB of partial sums to write, read and add. The
   // target is the one of four with the least estimated end, in items: the longest chunk, or where there are more chunks than
   // slots the one that is dealt second to the slot of the slots' shortest (twice its length), and the sums at 0.03 items per
-  // partial sum (131 KB written and read, an item 1.8 us). It has to be 8 % better than the share: a workgroup that is left alone on its compute
-  // unit at the end is the faster for it. Fewer tiles leave slots idle and are cut by the share, longer lists end evenly; at head
-  // dimension 64 shorter chunks gain more than half as large sums cost ([2, 10368, 12/2 of 64], documents of 50 to 414: dK/dV 46 us,
-  // by such an estimate 58). The whole pass, us: [3, 4480, 32/4 of 128], documents of
-  // 36 to 58, 317 -> 269; [2, 2048, 16/16], images, 222 -> 191; [1, 3456, 64/16], 87 to 178, 210 -> 184; 40 drawn shapes 0.99 to 1.18.
-  // (Counted a wavefront at a time: with an atomic per tile and target the list took 6 us more.)
-  if (D == 128 && pairs > kDkvSlots / 2 && pairs <= kDkvSlots) {
+  // partial sum (131 KB written and read, an item 1.8 us). It has to be 8 % better than the share: a workgroup that is left
+  // alone on its compute unit at the end is the faster for it. Fewer tiles leave slots idle and are cut by the share, longer
+  // lists end evenly; at head dimension 64 shorter chunks gain more than half as large sums cost ([2, 10368, 12/2 of 64],
+  // documents of 50 to 414: dK/dV 46 us, by such an estimate 58). The whole pass, us: [3, 4480, 32/4 of 128], documents of
+  // 36 to 58, 317 -> 269; [2, 2048, 16/16], images, 222 -> 191; [1, 3456, 64/16], 87 to 178, 210 -> 184; 40 drawn shapes
+  // 0.99 to 1.18. (Counted a wavefront at a time: with an atomic per tile and target the list took 6 us more.) The estimate
+  // itself takes 2.3 us, and where the share cuts no tile all four targets give one list: it is left out there (the list of
+  // [1, 5248, 8/8], documents of 16 to 32, 9.6 -> 7.8 us).
+  if (D == 128 && pairs > kDkvSlots / 2 && pairs <= kDkvSlots && __syncthreads_or(items_first > target)) {
     constexpr int kTargets = 4, kBuckets = 256;
     __shared__ int chunks[kTargets * kBuckets];  // by length, the longest in the last one
     __shared__ int split[kTargets], longest[kTargets];
