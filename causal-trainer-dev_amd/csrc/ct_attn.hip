@@ -19,8 +19,8 @@
 namespace ct {
 
 // ---------------------------------------------------------------------------
-// Tile bounds, in three launches, two for short rows, one for few positions: the summary of every 32-position block; from a row's summaries, what
-// each block has to visit; from those ranges, the work-sorted schedules, the dS offsets and the bins.
+// Tile bounds, in three launches, two for short rows, one for few positions: the summary of every 32-position block; from a
+// row's summaries, what each block has to visit; from those ranges, the work-sorted schedules, the dS offsets and the bins.
 //
 // All of it is latency: the searches and the ranking are quadratic in a row's blocks, and one
 // workgroup per row for everything took 43 us at S = 4096 and 0.6 ms at S = 32768 (its LDS pipe). Now
@@ -472,13 +472,15 @@ __global__ __launch_bounds__(1024) void attn_schedules_kernel(int* meta, int B, 
 }
 
 // Ranges, schedules, offsets and bins in one launch: a workgroup that needs the ranges of a row (or, for the bins, of all
-// rows) forms the records and searches them by itself, the one side that it needs. That repeats work on compute units that have none,
-// and saves a launch and the wait between two. grid: the bins' three workgroups, six per batch row, then build_ranges' ones.
-// LDS, ints: 3 + 2 per row block that a workgroup searches, then its working arrays. Us of GPU time, two launches / one, and 2.3 of
-// the host's: [1, 128] 6.6 / 3.9, [2, 1024] 7.7 / 4.5, [1, 8192] 12.5 / 8.5, [3, 2944] 10.4 / 9.1. Past the lines the bins' search of the
-// whole batch is the longest, or a long row's: [4, 4096] 13.1 / 14.0 (a batch's preparation as a whole 28.2 / 30.0 where the host keeps
-// ahead), [1, 12160] 17.4 / 20.3. (A wavefront per row block with a key tile per lane and a ballot: a chain of LDS reads per
-// block, [4, 4096] 19.7.)
+// rows) forms the records and searches them by itself, the one side that it needs. That repeats work on compute units that have
+// none, and saves a launch and the wait between two. grid: the bins' three workgroups, six per batch row, then build_ranges' ones.
+// LDS, ints: 3 + 2 per row block that a workgroup searches, then its working arrays. Us of GPU time, two launches / one, and 2.3
+// of the host's: [1, 128] 6.6 / 3.9, [2, 1024] 7.7 / 4.5, [1, 8192] 13.0 / 11.5, [3, 2944] 10.4 / 9.1. The bins' workgroups search
+// the whole batch: with four rows or more the GPU's times meet at 9216 positions (4 to 12 rows 9.6 / 9.6, 9.1 / 9.1) and from
+// 10240 on one launch is the longer one by less than the host saves ([4, 2560] 9.8 / 10.2, [3, 4096] 11.7 / 12.2, [12, 1024] 9.8 /
+// 10.8, [96, 128] 9.5 / 10.8). Past the lines it is that, or a long row's search, by as much or more: [4, 4096] 13.1 / 14.0 (a
+// batch's preparation as a whole 28.2 / 30.0 where the host keeps ahead), [1, 12160] 17.4 / 20.3. (A wavefront per row block with
+// a key tile per lane and a ballot: a chain of LDS reads per block, [4, 4096] 19.7.)
 constexpr int kOneLaunchPositions = 12288;
 __global__ __launch_bounds__(1024) void attn_prepare_kernel(int* meta, int B, int S, SummaryOut queries, SummaryOut keys,
                                                             const int* seg, const int* end, int* sched_all) {
@@ -653,17 +655,28 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 // documents from 36 positions to the whole row:
 //   few row blocks: attn_fwd_shares_kernel as long as all its workgroups are on the device at once, two on a compute unit with
 //     four wavefronts at head dimension 128, four at 64. Past that short documents pay for a second round (128: [2, 4480, 2/2],
-//     560 row blocks, images 66 / 40 but documents of 32 to 64 positions 9.5 / 11.4; 64: [1, 3456, 8/2], 864, 7.6 / 8.0;
-//     at 560 and 640 7.8 / 7.5 and 7.6 / 7.5, images 45 / 30), and in rows below 512 positions there is little to share. Eight wavefronts, half as many on a
-//     compute unit, pay from 1024 positions on up to 256 and 512 row blocks (by four / eight: [1, 8192, 1/1, 128] 65 / 44,
-//     [1, 4096, 4/4, 64] 27 / 22, documents of 100 to 200 there 7.6 / 8.0; [1, 4096, 4/4, 128], 512 row blocks, such documents 8.7 / 12.6).
-//     Three wavefronts at head dimension 128 (three workgroups on a compute unit, 768 at once) where every head has its own keys, in
-//     rows of 1024 positions or more (by two wavefronts with shared stages / by three; documents of 32 to 64, 100 to 200, 400 to 500,
-//     whole rows): [1, 4608, 4/4], 576 row blocks, 9.8 / 8.8, 10.7 / 9.6, 16.0 / 12.8, 68 / 51; [1, 6144, 4/4], 768, 10.7 / 9.7, 11.1 /
-//     11.1, 16.9 / 13.9, 91 / 71; [1, 9216, 2/2], 576, 9.8 / 9.2, 11.0 / 10.1, 16.3 / 13.6, 141 / 95. Below 540 the shortest documents lose
-//     ([1, 4224, 4/4], 528, 8.2 / 8.6). Heads in no multiple of four put keys of all heads on every XCD and lose from 600 on
-//     ([1, 7424, 3/3], 696, 100 to 200, 11.7 / 13.3), shared keys with short documents (they are staged for every head:
-//     [1, 2304, 8/2], 576, 8.2 / 8.7, though 14.7 / 12.0 and 37 / 29 with longer ones), and so does a second round (832, 10.8 / 12.5).
+//     560 row blocks, images 66 / 40 but documents of 32 to 64 positions 9.5 / 11.4; 64: [1, 3456, 8/2], 864, 7.6 / 8.0), and in
+//     rows below 512 positions there is little to share. Eight wavefronts, half as many on a compute unit, pay from 1024
+//     positions on up to 256 and 512 row blocks (by four / eight: [1, 8192, 1/1, 128] 65 / 44, [1, 4096, 4/4, 64] 27 / 22,
+//     documents of 100 to 200 there 7.6 / 8.0; [1, 4096, 4/4, 128], 512 row blocks, such documents 8.7 / 12.6).
+//     Head dimension 64 from 513 row blocks on, 57 shapes, time here over that by two wavefronts with shared stages: documents
+//     of 256 to 900 0.70 to 0.91, whole rows 0.56 to 0.95, 100 to 200 0.86 to 1.02. Documents of 16 to 64 take 0.94 to 1.01
+//     where each head has stages of its own either way (up to 544 row blocks 0.98 to 1.11), and 1.06 to 1.13, half a
+//     microsecond, where two or four heads could share them ([1, 2176, 8/4] 6.1 -> 6.8, but whole rows 23.8 -> 16.6).
+//     Three wavefronts at head dimension 128 (three workgroups on a compute unit, 768 at once) where every head has its own
+//     keys, in rows of 1024 positions or more. 36 shapes, time by three over that by two wavefronts with shared stages:
+//     documents of 256 to 900 0.75 to 0.86, whole rows 0.67 to 0.87, 100 to 200 0.88 to 1.02, 16 to 64 from 548 row blocks on
+//     0.89 to 1.00 (one call of 66 1.05), 60 to 120 0.93 to 1.04 up to 671 row blocks and 0.94 to 1.08 from 672 on. Us,
+//     documents of 32 to 64, 100 to 200, 400 to 500, whole rows: [1, 4608, 4/4], 576 row blocks, 9.6 -> 8.8, 10.6 -> 9.6,
+//     15.8 -> 13.0, 68 -> 51; [1, 6144, 4/4], 768, 10.7 -> 9.7, 11.1 -> 11.1, 16.9 -> 13.9, 91 -> 71.
+//     The lower line: up to 512 the workgroups of four wavefronts are all there at once. From 516 to 536 documents of 16 to 64
+//     lose 2 to 10 % in 25 of 34 calls of one to twelve heads ([1, 8320, 2/2], 520, 8.4 -> 9.1), at 540 and 544 2 to 7 % in 5
+//     of 14, from 548 to 556 in none of 12; longer ones gain throughout ([1, 4224, 4/4], 528, 400 to 500, 16.1 -> 13.2;
+//     [1, 4352, 4/4], 544, whole rows 64.6 -> 48.7). The upper one: heads in no multiple of four put keys of all heads on
+//     every XCD. From 600 on documents of 60 to 120 lose 2 to 24 % in 49 of 55 calls of one to ten heads, of 100 to 200 2 to 16 % in
+//     46 ([1, 3840, 5/5], 600, 10.2 -> 10.9, 11.1 -> 12.4; [1, 10368, 2/2], 648, 10.4 -> 11.3, 11.1 -> 11.7); up to 592 the first 0
+//     to 4 % in 7, the second none. Shared keys lose with short documents (they are staged for every head: [1, 2304, 8/2], 576,
+//     8.2 -> 8.7, though 14.7 -> 12.0 and 37 -> 29 with longer ones), and so does a second round (832, 10.8 -> 12.5).
 //   head dimension 64: sharing by two wins up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47).
 //   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920); from there to 2304 the longest row's
 //     chain still counts in long rows (large launch / by two: [1, 4096, 16/16] with documents up to the row 58.5 / 42.0),
@@ -730,8 +743,12 @@ static int launch_dq(hipStream_t stream, const AttnParams& p) {
   return launch_dq<D, HS, 2>(stream, p);
 }
 
-// `reduce`: the launch also adds the chunks of split key tiles, where its form can (KS > 1). 128 workgroups of eight
-// wavefronts: pieces are rarely more than twice as many.
+// `reduce`: the launch also adds the chunks of split key tiles, where its form can (KS > 1), by 128 workgroups of eight
+// wavefronts. There can be many more pieces than these 1024 wavefronts (17408 at [1, 3072, 32/32 of 128]), which then take several
+// each beside the tiles. A pass, us, with the sums in a launch of their own / by 128 / by 256: [2, 1024, 8/8 of 64], whole rows,
+// 40.7 / 38.0 / 37.5; [1, 2304, 6/1 of 64], documents of 256 to 900, 39.6 / 38.7 / 34.3; [1, 2688, 16/16 of 64], whole rows,
+// 91.6 / 87.4 / 88.0; [4, 1792, 16/8 of 64] 153.5 / 152.6 / 148.5; [1, 3072, 32/32 of 128] 311 / 306 / 301; [2, 1536, 8/2 of
+// 128], documents of 32 to 128, 46.1 / 41.4 / 42.3. Over 33 calls of 64 to 8192 row blocks 0.88 to 1.01 of their own launch.
 template <int D, int HS, int KS>
 static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
   const size_t smem = DsStage<D, KS>::kTotalBytes;

@@ -4,14 +4,18 @@
 // region of LDS that is its own, so nothing in the loop waits for another wavefront: K's copies for the next piece go out as
 // soon as the scores of this one are formed, V's behind the product with V. The sums are merged once, at the end, every
 // wavefront adding its share of the columns. The time is that of the longest row's chain of pieces, each about
-// 0.75 us at head dimension 64 and 0.95 at 128 for a lone wavefront (copies, 8 or 16 products, softmax, one after the other), and,
-// where compute units hold all the workgroups that fit, of the 64 bytes a clock that reach a compute unit's LDS (8 or 16 KB per
-// piece). What this replaces staged the keys of four wavefronts together, twice, with a barrier per step; at head dimension 128 a compute unit held
-// one such workgroup, of these two. Measured, us (batch, row length, query / KV heads, head dimension; documents):
-//   NW = 4: (2, 1024, 8/8, 128; 32-512) 13.9 -> 11.7      (1, 4096, 4/4, 128; 400-500) 14.2 -> 11.1     (4, 1024, 4/4, 128; rows) 16.5 -> 14.5
-//           (1, 7168, 4/4, 64; rows)    68 -> 51          (2, 4480, 2/2, 64; images)   45 -> 30         (3, 2944, 24/8, 64) 42 / 57: not taken
-//   NW = 8: (1, 2176, 2/2, 128; images) 23.4 -> 15.5      (1, 8192, 1/1, 128; rows)    83 -> 44         (1, 16384, 1/1, 64; rows) 106 -> 71
-//   NW = 3: (1, 6144, 4/4, 128; rows)   91 -> 71          (1, 2048, 12/12, 128; 256-2048) 36.6 -> 28.7  (4, 1280, 4/4, 128; 400-500) 15.1 -> 12.3
+// 0.75 us at head dimension 64 and 0.95 at 128 for a lone wavefront (copies, 8 or 16 products, softmax, one after the other),
+// and, where compute units hold all the workgroups that fit, of the 64 bytes a clock that reach a compute unit's LDS (8 or
+// 16 KB per piece). What this replaces staged the keys of four wavefronts together, twice, with a barrier per step; at head
+// dimension 128 a compute unit held one such workgroup, of these two. Measured, us (batch, row length, query / KV heads, head
+// dimension; documents):
+//   NW = 4: (2, 1024, 8/8, 128; 32-512) 13.9 -> 11.7      (1, 4096, 4/4, 128; 400-500) 14.2 -> 11.1
+//           (4, 1024, 4/4, 128; rows)   16.5 -> 14.5      (1, 7168, 4/4, 64; rows)     68 -> 51
+//           (2, 4480, 2/2, 64; images)  45 -> 30          (3, 2944, 24/8, 64)          42 / 57: not taken
+//   NW = 8: (1, 2176, 2/2, 128; images) 23.4 -> 15.5      (1, 8192, 1/1, 128; rows)    83 -> 44
+//           (1, 16384, 1/1, 64; rows)   106 -> 71
+//   NW = 3: (1, 6144, 4/4, 128; rows)   91 -> 71          (1, 2048, 12/12, 128; 256-2048) 36.6 -> 28.7
+//           (4, 1280, 4/4, 128; 400-500) 15.1 -> 12.3
 // Two query blocks per wavefront, which would halve the copies, need more registers than there are (58 spilled, 1.5 to 2
 // times as long); two short row blocks in one workgroup, found out from the bounds, wait for them first (9.5 -> 15.6 us).
 #pragma once

@@ -77,9 +77,10 @@ struct KvStage {
   static constexpr int kBytes = 2 * kTileBytes + kKeyTile * 4;
 };
 
-// Asynchronous fetch of a key tile (K rows, V rows, segment ids) into an LDS stage, for a walk from tile to tile:
-// addresses that a step advances by a constant, the LDS address in scalar registers, the ids by a copy whose lanes are all off in three of the four wavefronts. (Formed from the tile's number
-// every time, a copy of a tile costs 80 scalar and vector instructions beside its nine copies.)
+// Asynchronous fetch of a key tile (K rows, V rows, segment ids) into an LDS stage, for a walk from tile to tile: addresses
+// that a step advances by a constant, the LDS address in scalar registers, the ids by a copy whose lanes are all off in three
+// of the four wavefronts. (Formed from the tile's number every time, a copy of a tile costs 80 scalar and vector instructions
+// beside its nine copies.)
 template <int D>
 struct KvCursor {
   TileDma<kKeyTile, D / 8> dma;
