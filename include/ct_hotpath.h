@@ -169,8 +169,8 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * only, not on the tensors: a caller that runs the backward of several layers over one packing
  * (same tile_meta, shape, variant and workspace size) can keep the list. With this flag the call
  * does not build it: the head of `workspace` must be as the previous ct_attn_bwd call on this
- * workspace left it (every call leaves the list in place and the work counters of the dQ kernel at
- * zero). Saves a launch and 0.01 ms per call of the recomputing form, and in the stored-dS form the list's share of
+ * workspace left it (every call leaves the list in place and, whatever the forms of its passes, the work
+ * counters of the dQ kernels at zero). Saves a launch and 0.01 ms per call of the recomputing form, and in the stored-dS form the list's share of
  * the launch that also forms the row statistics (up to 7 us of small launches); anything else in the workspace
  * may be overwritten between the calls. */
 #define CT_ATTN_BWD_WORK_LIST_KEPT 0x100
@@ -220,7 +220,8 @@ size_t ct_attn_bwd_workspace_bytes_from_ds(int32_t batch, int32_t seq, int32_t q
  * -lse / scale) for its rows; dk/dv per key tile; the sum of the chunks of split key tiles (in
  * a fixed order, so the result is deterministic). With CT_ATTN_BWD_DQ_FROM_DS: the row
  * statistics as a pass of their own, the work list, then per pass of KV heads dk/dv (which
- * stores its dS blocks) and dq as the product of those blocks with K, and the sum.
+ * stores its dS blocks) and dq as the product of those blocks with K, and the sum, in the last dq launch
+ * where that has a workgroup per query tile.
  * Replaces: delta at src/kernels/efficient_attention.py:1735-1738,
  * _local_attention_dq (:985-1267), _local_attention_dkv (:1270-1602) and the
  * f32 -> bf16 cast at :1774.
