@@ -61,7 +61,11 @@ CT_DEVICE void reset_dlogits_counters(CutceHeader* header) {
 //
 // Plain order, up to kPlainRounds units per workgroup: the grid is walked with a as the slow index, the
 // first unit of a workgroup is its own number, the others come from one counter. Within a round
-// every XCD gets 32 consecutive units, which share operands. (Short problems have no use for the orders
+// every XCD gets an eighth of the units, consecutive ones, which share operands; a last round that fills only part of the
+// device likewise (one round of the statistics kernel, every unit on the next XCD / consecutive ones, us: 380 x 17624,
+// d = 1664, 414 small tiles 47.8 / 37.0; 385 x 3120, d = 7296, 100 small ones 72.9 / 68.4; 335 x 28712, d = 2432, 226 large ones
+// 66.3 / 61.8). A list of units of two lengths (`mixed`) that is over in less than a round is dealt to the XCDs one by
+// one: the long ones would meet on some of them (both gradients of 4000 x 1900, d = 1024: 39.8 / 43.9). (Short problems have no use for the orders
 // below: counters of XCDs that own nothing, indices that fall outside ragged grids and rounds of
 // asking the other XCDs cost 10-20 us a launch.)
 //
@@ -85,14 +89,15 @@ struct UnitQueue {
   int a_count, b_count, total, b_groups, padded_total, per_xcd, my_xcd;
   int helping;  // how many XCDs further the counter in use belongs to
   Order order;
-  bool requested, started;
+  bool requested, started, mixed;
   int pending;  // of thread 0: the counter's answer
-  CT_DEVICE void init(int* counters_, int a_count_, int b_count_, Order large) {
+  CT_DEVICE void init(int* counters_, int a_count_, int b_count_, Order large, bool mixed_ = false) {
     counters = counters_;
     a_count = a_count_;
     b_count = b_count_;
     total = a_count * b_count;
     order = total <= kPlainRounds * (int)gridDim.x ? kPlain : large;
+    mixed = mixed_;
     b_groups = (b_count + kB - 1) / kB;
     padded_total = ((a_count + kA - 1) / kA) * b_groups * kA * kB;
     per_xcd = (padded_total + kXcds - 1) / kXcds;
@@ -124,9 +129,9 @@ struct UnitQueue {
     const int n = gridDim.x;
     const int i = started ? n + receive(lds_slot) : (int)blockIdx.x;
     started = true;
-    const int round = i / n * n;
-    if (round + n > total || n % kXcds) return i;
-    return round + (i - round) % kXcds * (n / kXcds) + (i - round) / kXcds;
+    const int round = i / n * n, in = min(n, total - round), at = i - round;
+    if (at >= in || (in < n && round == 0 && mixed)) return i;
+    return round + at % kXcds * (in / kXcds) + min(at % kXcds, in % kXcds) + at / kXcds;
   }
   // Called by all threads of the workgroup (contains barriers); false when nothing is left.
   CT_DEVICE bool next(int& a, int& b, int* lds_slot) {
@@ -1152,7 +1157,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
   const bool head_first = HEAD && 2l * ((n_act + 127) / 128) * parts_h > 3l * (sl.width / 128) * parts_w;
   UnitQueue units;
   bool in_head = false;
-  if (one_list) units.init(p.header->xcd_counter[0], total_h + total_w, 1, UnitQueue::kPlain);
+  if (one_list) units.init(p.header->xcd_counter[0], total_h + total_w, 1, UnitQueue::kPlain, true);
   else units.init(p.header->xcd_counter[0], row_blocks, col_blocks * parts_h, UnitQueue::kBlocks);
   for (;;) {
     int a, b;
@@ -1244,9 +1249,9 @@ static int tiles_per_chunk(int tiles, int row_blocks) {
 // compute unit, half the time per step. Measured (us, large / small; statistics kernel and dlogits kernel):
 // 32 large tiles 500 x 4000, d = 512: 19 / 10 and 20 / 11, d = 6144: 98 / 50 and 100 / 51; 96 large =
 // 376 small tiles 1000 x 6000, d = 512: 19 / 17 and 22 / 17, d = 2048: 42 / 40 and 45 / 41; 500 small tiles
-// 250 x 32000, d = 2048: 49 / 56 and 47 / 55; 414, 380 x 17624, d = 1664: 39 / 47 and 41 / 49; 704, 4000 x 2800,
-// d = 1024: 30 / 38 and 34 / 40.
-constexpr int kMostSmallTiles = 384;
+// 1000 x 7160, d = 2048: 42 / 41 and 45 / 42, 384 x 19192: 43 / 43 and 46 / 45; 512, 384 x 21880: 47 / 58 and 49 / 60,
+// d = 512 21 / 21 and 23 / 24; 704, 4000 x 2800, d = 1024: 30 / 38 and 34 / 40.
+constexpr int kMostSmallTiles = 480;
 static int projection_tile(int rows, int tiles) {
   return (long)((rows + 127) / 128) * (2 * tiles) <= kMostSmallTiles ? 128 : kGemmTile;
 }

@@ -499,8 +499,10 @@ def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
 @pytest.mark.parametrize("rows,width,vocab", [
     (129, 128, 248),      # both products in 128 x 128 tiles, one column and one row past a tile
     (50, 4224, 520),      # rows longer than what is read ahead of the list
-    (1024, 256, 6144),    # 8 x 48 small tiles: the last projection that takes them, gradients in large ones
-    (1025, 256, 5500),    # 9 x 44: the first in large tiles, unaligned rows
+    (1024, 256, 6144),    # 8 x 48 small tiles, gradients in large ones
+    (1025, 256, 5500),    # 9 x 43, unaligned rows
+    (1024, 256, 7680),    # 8 x 60 small tiles: the last projection that takes them
+    (1025, 256, 6912),    # 9 x 54: the first in large tiles, 5 x 27 of them: a round that fills part of the device
     (897, 640, 1288),     # gradients in small tiles, the last 8 columns from the tail
     (1025, 1152, 1288),   # small tiles for the projection, large ones for the gradients
     (4099, 128, 300),     # row lists: two rounds of 16 rows per workgroup, the last one ragged
