@@ -648,16 +648,18 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
 // ---------------------------------------------------------------------------
 // merge
 // ---------------------------------------------------------------------------
-// A workgroup merges the per-chunk partials of kMergeSlots row slots: kMergeParts threads per slot
-// each walk every kMergeParts-th vocabulary chunk (so a row's chain of dependent loads is an
-// eighth as long and eight times as many loads are in flight: the pass is bound by the bytes of
-// the partials, not by their latency), then the parts are combined in a fixed order.
-constexpr int kMergeSlots = 32, kMergeParts = 8;
-__global__ __launch_bounds__(kMergeSlots * kMergeParts) void cutce_merge_kernel(CutceParams p, const float* part,
-                                                                                int chunks, float* lse_out,
-                                                                                double* block_sums, float* nll_sum,
-                                                                                float* weight_sum_out) {
-  __shared__ float exch[kMergeParts][kMergeSlots][3];
+// A workgroup merges the per-chunk partials of kMergeSlots row slots: PARTS threads per slot each walk every
+// PARTS-th vocabulary chunk, then the parts are combined in a fixed order: the two of a wavefront, then the
+// wavefronts. The pass is bound by the latency of those walks, so long ones are shared by 32 threads, short
+// ones by 8 (us with 8 / 32: 60 rows x 1002 chunks 12.7 / 9.2, 128 x 300 8.4 / 5.9, 384 x 167 5.7 / 5.4; 64 x 5
+// 4.2 / 4.7, 4000 x 15 5.5 / 6.0).
+constexpr int kMergeSlots = 32, kShortMerge = 64;
+template <int PARTS>
+__global__ __launch_bounds__(kMergeSlots * PARTS) void cutce_merge_kernel(CutceParams p, const float* part, int chunks,
+                                                                          float* lse_out, double* block_sums,
+                                                                          float* nll_sum, float* weight_sum_out) {
+  constexpr int kWaves = kMergeSlots * PARTS / 64;
+  __shared__ float exch[kWaves][kMergeSlots][3];
   __shared__ double red[2][64];
   __shared__ bool last_s;
   const int tid = threadIdx.x, lane_slot = tid % kMergeSlots, piece = tid / kMergeSlots;
@@ -676,21 +678,25 @@ __global__ __launch_bounds__(kMergeSlots * kMergeParts) void cutce_merge_kernel(
     wr = p.weights[row];
   }
   float m = kNegInfF, s = 0.f, t = 0.f;
-  if (wr != 0.f) {
+  if (slot < n_act) {  // (not by wr, which is still on its way; a row without weight is not stored below)
 #pragma unroll 4
-    for (int c = piece; c < chunks; c += kMergeParts) {  // (several chunks' loads in flight)
+    for (int c = piece; c < chunks; c += PARTS) {  // (several chunks' loads in flight)
       const float* e = part + ((size_t)c * p.n_pad + slot) * 3;
       merge_stats(m, s, e[0], e[1]);
       t += e[2];
     }
   }
-  exch[piece][lane_slot][0] = m;
-  exch[piece][lane_slot][1] = s;
-  exch[piece][lane_slot][2] = t;
+  merge_stats(m, s, xor32(m), xor32(s));
+  t += xor32(t);
+  if (piece % 2 == 0) {
+    exch[piece / 2][lane_slot][0] = m;
+    exch[piece / 2][lane_slot][1] = s;
+    exch[piece / 2][lane_slot][2] = t;
+  }
   __syncthreads();
   if (piece == 0) {
     if (wr != 0.f) {
-      for (int k = 1; k < kMergeParts; ++k) {
+      for (int k = 1; k < kWaves; ++k) {
         merge_stats(m, s, exch[k][lane_slot][0], exch[k][lane_slot][1]);
         t += exch[k][lane_slot][2];
       }
@@ -1684,8 +1690,10 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
 
   const int merge_blocks = p.n_pad / kMergeSlots;
   LaunchScope scope3("cutce_merge_kernel", stream);
-  hipLaunchKernelGGL(cutce_merge_kernel, dim3(merge_blocks), dim3(kMergeSlots * kMergeParts), 0, stream, p, part,
-                     units.chunks, a->lse, sums, a->nll_sum, a->weight_sum);
+  const bool short_merge = units.chunks <= kShortMerge;
+  hipLaunchKernelGGL((short_merge ? cutce_merge_kernel<8> : cutce_merge_kernel<32>), dim3(merge_blocks),
+                     dim3(kMergeSlots * (short_merge ? 8 : 32)), 0, stream, p, part, units.chunks, a->lse, sums, a->nll_sum,
+                     a->weight_sum);
   return scope3.done();
 }
 

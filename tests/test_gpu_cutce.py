@@ -526,6 +526,13 @@ def test_output_tile_sizes(ct, gpu, rows, width, vocab):
     assert relative_l2(slabs[0].cpu(), whole[0].cpu()) <= GRAD_RTOL
 
 
+@pytest.mark.parametrize("rows,vocab", [(257, 128 * 64), (257, 128 * 65), (33, 128 * 64 + 1), (1, 16381)])
+def test_merge_of_long_and_short_walks(ct, gpu, rows, vocab):
+    """64 chunks of the vocabulary for a row, the most that 8 threads merge, and 65 and more, which 32 do."""
+
+    _check(_gpu(ct, gpu, *_case(rows + vocab, rows, 128, vocab), 0.37, compaction=True), *_case(rows + vocab, rows, 128, vocab), 0.37)
+
+
 @pytest.mark.parametrize("rows,width,vocab", [
     (4200, 128, 16380),   # four to five large tiles per workgroup of four steps each, unaligned rows
     (8500, 128, 20008),   # units of two tiles, the last of one
