@@ -158,6 +158,7 @@ SYMBOLS = {
     "ct_cutce_fwd": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
     "ct_cutce_bwd": (c_int32, [c_void_p, POINTER(CutceBwdArgs)]),
     "ct_cutce_panel_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_head_in_place": (c_int32, [POINTER(CutceShape)]),
     "ct_cutce_fwd_panel": (c_int32, [c_void_p, POINTER(CutceFwdArgs), c_void_p, c_size_t, c_int32]),
     "ct_cutce_bwd_panel": (c_int32, [c_void_p, POINTER(CutceBwdArgs), c_void_p, c_size_t]),
     "ct_cutce_fwd_noalloc_max_bytes": (c_size_t, []),

@@ -169,16 +169,19 @@ struct UnitQueue {
 };
 
 // The head as the GEMM kernels read it: column v of row n at base[n * ld + v - col0]. Either the
-// caller's tensor (ld = V) or, where its rows are not 16-byte aligned (V % 8 != 0), an aligned copy
-// of the columns col0 .. in the workspace ("panel", HeadCopy), padded with zero columns to
-// whole tiles.
+// caller's tensor (ld = V) or, where its rows are not 16-byte aligned (V % 8 != 0) and it is not read in place
+// (forward_in_place, backward_in_place), an aligned copy of the columns col0 .. in the workspace ("panel", HeadCopy), padded with
+// zero columns to whole tiles.
 // An aligned head whose vocabulary is no multiple of 128 has the columns from the last such multiple
-// on a second time in `tail` [d][128], padded with zeros, for the contraction over the vocabulary.
+// on a second time in `tail` [d][128], padded with zeros, for the contraction over the vocabulary; an unaligned
+// one that is read in place the columns from the last multiple of 256 on in `tail` [d][256], for that and for the
+// projections' last tile: nothing past the end of a row is read from the caller's tensor.
 struct HeadView {
   const bf16* base;
   const bf16* tail;
   long ld;
   int col0;
+  int tail_first, tail_cols;  // vocabulary id of the tail's first column, and its row length
   bool padded;
 };
 
@@ -420,11 +423,12 @@ struct HeadCopy {
   bf16* panel;  // `cols` (a multiple of 256) columns from col0 on, zero-padded, or null
   bf16* tail;   // HeadView::tail, or null
   int col0, cols;
+  int tail_first, tail_cols;
 };
 constexpr int kPanelRows = 4, kPanelColumns = 2048;  // of 256 threads
 __host__ __device__ inline int head_copy_blocks(const HeadCopy& copy, int d) {
   if (copy.panel) return (copy.cols + kPanelColumns - 1) / kPanelColumns * (d / (4 * kPanelRows));
-  return copy.tail ? (d + 63) / 64 : 0;
+  return copy.tail ? (d * (copy.tail_cols / 8) + 1023) / 1024 : 0;
 }
 CT_DEVICE void copy_head(const HeadCopy& copy, int V, int d, int block) {
   const int tid = threadIdx.x;
@@ -447,11 +451,18 @@ CT_DEVICE void copy_head(const HeadCopy& copy, int V, int d, int block) {
 #pragma unroll
     for (int r = 0; r < kPanelRows; ++r) store_global16(dst + (size_t)r * copy.cols, as_u32x4(v[r]));
   } else {
-    const int row = block * 64 + tid / 16, v = V / 128 * 128 + tid % 16 * 8;
+    const int chunks = copy.tail_cols / 8, index = block * 1024 + tid, row = index / chunks, c = index % chunks * 8;
     if (row >= d) return;
-    u32x4 chunk = {0u, 0u, 0u, 0u};
-    if (v < V) chunk = load_global16(copy.head + (size_t)row * V + v);
-    store_global16(copy.tail + (size_t)row * 128 + tid % 16 * 8, chunk);
+    const bf16* src = copy.head + (size_t)row * V + copy.tail_first + c;
+    const int left = V - (copy.tail_first + c);
+    bf16x8 chunk;
+    if (left >= 8) {
+      __builtin_memcpy(&chunk, src, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) chunk[e] = e < left ? src[e] : (bf16)0.f;
+    }
+    store_global16(copy.tail + (size_t)row * copy.tail_cols + c, as_u32x4(chunk));
   }
 }
 
@@ -482,13 +493,25 @@ CT_DEVICE void merge_stats(float& m, float& s, float m_o, float s_o) {
   m = m_new;
 }
 
+// The head's tile of a projection, vocabulary ids v0 ..
+template <GemmLoads LOADS, int NB>
+CT_DEVICE void head_tile(McLoader<NB>& A, const CutceParams& p, int v0) {
+  if constexpr (LOADS == GemmLoads::kThroughRegisters) {
+    const bool inside = v0 + GemmShape<NB>::kTile <= p.V;
+    const int first = inside ? v0 : v0 - p.head.tail_first;
+    A.init(inside ? p.head.base : p.head.tail, inside ? p.head.ld : p.head.tail_cols, first, first + GemmShape<NB>::kTile, p.d);
+  } else {
+    A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
+  }
+}
+
 // Bound by the matrix pipe at long contractions; at short ones by what lies between two products, for the large tile
 // has its compute unit to itself. In clocks a tile, 4096 x 32000 at d = 256: product 10.1 k (8.2 k of MFMAs), first
 // copies of the next tile 2.5 k (96 KB at 64 bytes a clock), epilogue 8.5 k, end of a unit 2.4 k; the copies'
 // latency, the cleared accumulators and a second reading of them in the epilogue took 116 us to 104 there, 67 to 65
 // at 900 x 32003, d = 1024, 175 to 162 at 1845 x 67203, d = 512. (Small tiles on two workgroups per compute unit, whose epilogues could
 // fall behind each other's products: 152, 81 and 196, bound by the bytes that reach LDS.)
-template <int NB, bool CACHE, bool GUARDED>
+template <int NB, bool CACHE, GemmLoads LOADS>
 __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
                                                                     int tiles_per_chunk, float* cache) {
   constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
@@ -514,7 +537,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
   bool more = next_unit(chunk, rb);
   McLoader<NB> A;
   KcLoader<NB> B;
-  GemmTiles<NB, GUARDED, CACHE> gemm;
+  GemmTiles<NB, LOADS, CACHE> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
   typedef int LaneInts __attribute__((ext_vector_type(NB)));
@@ -527,7 +550,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
       B.init(p.hidden, p.d, p.gather(), rb * kTile, n_act, p.d, true);
       asm volatile("" : "+v"(next_tgt));
     }
-    A.init(p.head.base, p.head.ld, vt * kTile - p.head.col0, p.head_cols(vt * kTile), p.d);
+    head_tile<LOADS>(A, p, vt * kTile);
     gemm.begin(A, B, smem);
   };
   if (more) begin_tile((chunk0 + chunk) * tiles_per_chunk, true);
@@ -748,7 +771,7 @@ CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
 // G^T[v - slab0][slot], logits recomputed (transposed tile as in the statistics kernel: rows =
 // vocabulary, lanes = row slots). Persistent like the statistics kernel and with its unit order:
 // a unit is tiles_per_chunk vocabulary tiles of the slab times one block of 256 active rows.
-template <int NB, bool GUARDED>
+template <int NB, GemmLoads LOADS>
 __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
                                                                       int slab0, int slab_tiles, int tiles_per_chunk,
                                                                       bf16* G) {
@@ -771,7 +794,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
   bool more = units.next(chunk, rb, &unit_s);
   McLoader<NB> A;
   KcLoader<NB> B;
-  GemmTiles<NB, GUARDED, true> gemm;
+  GemmTiles<NB, LOADS, true> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
   LaneFloats next_fac, next_lse2;
@@ -786,7 +809,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
       B.init(p.hidden, p.d, p.gather(), rb * kTile, n_act, p.d, true);
       asm volatile("" : "+v"(next_fac), "+v"(next_lse2), "+v"(next_tgt));
     }
-    A.init(p.head.base, p.head.ld, v0 - p.head.col0, p.head_cols(v0), p.d);
+    head_tile<LOADS>(A, p, v0);
     gemm.begin(A, B, smem);
   };
   if (more) begin_tile(chunk * tiles_per_chunk, true);
@@ -963,7 +986,7 @@ struct CutceSlab {
 
 // dHidden[idx[slot], n] (+)= sum_v G^T[v, slot] head[n, first + v] of row block rb, column block cb and
 // part `split` of the contraction.
-template <int NB, bool GUARDED>
+template <int NB, GemmLoads LOADS>
 CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int rb, int cb, int split,
                             int parts, int n_act, UnitQueue& units, const lds_addr smem) {
   constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
@@ -971,12 +994,14 @@ CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const Cut
   const int wm = (w >> 1) * kWave, wn = (w & 1) * kWave;
   // Terms of the contraction: the whole slab where the head is padded, else up to the end of the
   // vocabulary; the last k_width % 128 of them from the tail, since nothing past a row's end may be
-  // read (G^T is zero from the vocabulary's end to the end of the slab).
-  const int k_width = p.head.padded ? sl.width : min(sl.width, p.V - sl.first);
-  const int groups = k_width / 128;
+  // read (G^T is zero from the vocabulary's end to the end of the slab). The parts are those of the
+  // whole slab in each case: the same sums, whether the head is padded or not.
+  const int k_width = p.head.padded ? sl.width : min(sl.width, p.V - sl.first), k_whole = k_width / 128 * 128;
+  const int groups = sl.width / 128;
   const int n0 = rb * kTile, c0 = cb * kTile;
-  const int k_begin = split_begin(groups, split, parts) * 128, k_mid = split_begin(groups, split + 1, parts) * 128;
-  const bool with_tail = split == parts - 1 && k_mid < k_width;
+  const int k_begin = split_begin(groups, split, parts) * 128, k_end = split_begin(groups, split + 1, parts) * 128;
+  const int k_mid = min(k_end, k_whole);
+  const bool with_tail = k_begin <= k_whole && k_whole < min(k_end, k_width);
   McLoader<NB> A;
   A.init(sl.G, p.n_pad, n0, p.n_pad, sl.width);
   GemmAcc<NB> acc;
@@ -984,16 +1009,26 @@ CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const Cut
   // (rows of B interleaved: lane j owns the NB consecutive columns c0 + wn + NB j + nb; rows past d
   // are copies of the first, their columns are not stored)
   const bf16* head = p.head.base + (sl.first - p.head.col0);
-  if constexpr (GUARDED) {
+  if constexpr (LOADS == GemmLoads::kGuarded) {
     KcLoader<NB> B;
     B.init(head, p.head.ld, nullptr, c0, p.d, k_width, true);
-    gemm_tile<true>(A, B, k_begin, with_tail ? k_width : k_mid, smem, acc);
+    gemm_tile<LOADS>(A, B, k_begin, with_tail ? k_width : k_mid, smem, acc);
   } else {
+    const bf16* tail = p.head.tail + (sl.first - p.head.tail_first);
 #pragma nounroll
     for (int part = 0; part <= (int)with_tail; ++part) {
-      KcLoader<NB> B;
-      B.init(part ? p.head.tail - k_mid : head, part ? 128 : p.head.ld, nullptr, c0, p.d, k_width, true);
-      gemm_tile<false>(A, B, part ? k_mid : k_begin, part ? k_mid + 128 : k_mid, smem, acc);
+      const bf16* from = part ? tail : head;
+      const long ld = part ? p.head.tail_cols : p.head.ld;
+      const int begin = part ? k_mid : k_begin, end = part ? k_mid + 128 : k_mid;
+      if constexpr (LOADS == GemmLoads::kThroughRegisters) {
+        KcPairLoader<NB> B;
+        B.init(from, ld, c0, p.d);
+        gemm_tile(A, B, begin, end, smem, acc);
+      } else {
+        KcLoader<NB> B;
+        B.init(from, ld, nullptr, c0, p.d, k_width, true);
+        gemm_tile<LOADS>(A, B, begin, end, smem, acc);
+      }
     }
   }
   units.request();
@@ -1070,7 +1105,7 @@ CT_DEVICE void store_dhead4(bf16* dst, int left, f32x4 val) {
 
 // dHead[m, first + v] = sum_slot packed[slot, m] G^T[v, slot], packed[slot] = hidden[idx[slot]], of
 // vocabulary tile vt, hidden column block mb and part `split` of the contraction.
-template <int NB, bool GUARDED>
+template <int NB, GemmLoads LOADS>
 CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const CutceSplits& sp, int vt, int mb, int split,
                           int parts, int n_act, UnitQueue& units, const lds_addr smem) {
   constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
@@ -1088,7 +1123,7 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
   B.init(sl.G, p.n_pad, nullptr, v0, sl.width, k_end, true);
   GemmAcc<NB> acc;
   acc.clear();
-  gemm_tile<GUARDED>(A, B, k_begin, k_end, smem, acc);
+  gemm_tile<LOADS>(A, B, k_begin, k_end, smem, acc);
   units.request();
 
   const int row0 = m0 + uniform(wm), col0 = v0 + uniform(wn);
@@ -1140,7 +1175,7 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
 // device idle); a workgroup that finds no hidden-gradient unit left goes on to the head-gradient
 // units, which are many and short, and the idle tail of the first fills with work of the second. The
 // two read the same G^T and write different tensors: neither waits for the other.
-template <int NB, bool HEAD, bool GUARDED>
+template <int NB, bool HEAD, GemmLoads LOADS>
 __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kernel(CutceParams p, CutceSlab sl, CutceSplits sp) {
   constexpr int kTile = GemmShape<NB>::kTile;
   extern __shared__ __align__(16) char smem_raw[];
@@ -1184,9 +1219,11 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_grads_kerne
       b = part * col_blocks + tile % col_blocks;
     }
     if (!in_head) {
-      dhidden_unit<NB, GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
+      dhidden_unit<NB, LOADS>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_h, n_act, units, smem);
     } else if constexpr (HEAD) {
-      dhead_unit<NB, GUARDED>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_w, n_act, units, smem);
+      // (its operands are the workspace's own)
+      constexpr GemmLoads kLoads = LOADS == GemmLoads::kGuarded ? LOADS : GemmLoads::kCopies;
+      dhead_unit<NB, kLoads>(p, sl, sp, a, b % col_blocks, b / col_blocks, parts_w, n_act, units, smem);
     }
   }
 }
@@ -1287,6 +1324,27 @@ static StatsUnits stats_units(const ct_cutce_shape& s) {
 
 // Heads whose rows do not all start on 16 bytes go through an aligned copy (HeadCopy).
 static bool needs_panel(const ct_cutce_shape& s) { return s.vocab % 8 != 0; }
+// ... or are read in place by loads through registers, which need a copy of the last columns only (HeadView::tail). The copy
+// of the whole takes 4 bytes of traffic per element and direction, and leaves aligned 16-byte chunks: unaligned ones make
+// a product 5 to 15 % longer (24 % where two small tiles share a compute unit), so it pays from some number of
+// rows on. Us, copy / in place, one GPU.
+// Forward (copy and statistics kernel): 128 x 150001, d = 4096 768 / 340; 250 x 50001, d = 1024 74 / 38; 1000 x 16001,
+// d = 1024 46 / 42; 2000 x 50001, d = 4096 833 / 811, d = 256 98 / 97; 4000 x 50001, d = 1024 417 / 428, d = 256 165 / 175. Fewer
+// than 8 columns per row: 1000 x 5001, d = 4096 79 / 85, d = 1024 28.0 / 30.5; a chain along d longer than the copy: 128 x
+// 1501, d = 4096 41 / 44, d = 1024 19.0 / 16.5.
+static bool forward_in_place(const ct_cutce_shape& s) {
+  return needs_panel(s) && s.rows <= 2048 && s.vocab >= 8l * s.rows && 2l * s.vocab >= s.hidden;
+}
+// Backward (copy, dlogits and gradients), where dHidden reads short rows: 64 x 150001, d = 4096 1466 / 1165, d = 256 163 / 132;
+// 250 x 50001, d = 1024 149 / 122; 500 x 16001, d = 1024 88 / 85, x 50001, d = 4096 790 / 723; 1000 x 50001, d = 1024 351 /
+// 335, 1000 x 16001, d = 4096 388 / 361, but x 150001, d = 1024 985 / 1004, x 50001, d = 4096 1265 / 1296; 2000 x 50001,
+// d = 1024 628 / 636. Small heads: 64 x 16001, d = 256 31.2 / 32.0, 500 x 5001, d = 1024 46.8 / 50.6.
+static bool backward_in_place(const ct_cutce_shape& s) {
+  const long elements = (long)s.hidden * s.vocab;
+  return needs_panel(s) && s.vocab >= 8192 && elements >= 12000000 && s.rows <= (elements <= 100000000 ? 1024 : 512);
+}
+// With a logits cache the forward leaves the backward panel or tail, with nothing kept each direction has its own.
+static bool both_in_place(const ct_cutce_shape& s) { return forward_in_place(s) && backward_in_place(s); }
 static size_t panel_tile_bytes(const ct_cutce_shape& s) { return (size_t)s.hidden * kGemmTile * sizeof(bf16); }
 // bytes of the panel of the whole vocabulary, 0 if none is needed
 static size_t full_panel_bytes(const ct_cutce_shape& s) {
@@ -1533,7 +1591,7 @@ static CutceParams make_params(const uint16_t* hidden, const uint16_t* head, con
                                const float* weights, const ct_cutce_shape& s, int compact, char* ws) {
   CutceParams p = {};
   p.hidden = reinterpret_cast<const bf16*>(hidden);
-  p.head = HeadView{reinterpret_cast<const bf16*>(head), nullptr, s.vocab, 0, false};
+  p.head = HeadView{reinterpret_cast<const bf16*>(head), nullptr, s.vocab, 0, 0, 0, false};
   p.compact = compact && gather_reaches(s);  // (rows in place give the same results)
   p.targets = targets;
   p.weights = weights;
@@ -1558,21 +1616,37 @@ static int launch_prepare(hipStream_t stream, const CutceParams& p, const CutceR
 }
 // `panel` with the tile columns tile0 .. tile0 + tiles - 1 of the head.
 static HeadCopy panel_copy(const bf16* head, bf16* panel, int tile0, int tiles) {
-  return HeadCopy{head, panel, nullptr, tile0 * kGemmTile, tiles * kGemmTile};
+  return HeadCopy{head, panel, nullptr, tile0 * kGemmTile, tiles * kGemmTile, 0, 0};
 }
 static HeadView panel_view(const bf16* panel, int tile0, int tiles) {
-  return HeadView{panel, nullptr, (long)tiles * kGemmTile, tile0 * kGemmTile, true};
+  return HeadView{panel, nullptr, (long)tiles * kGemmTile, tile0 * kGemmTile, 0, 0, true};
+}
+// A view of the caller's head with a tail of `cols` columns, and the copy that fills it.
+static HeadView tail_view(const CutceParams& p, const bf16* tail, int cols) {
+  return HeadView{p.head.base, tail, p.V, 0, p.V / cols * cols, cols, false};
+}
+static HeadCopy tail_copy(const HeadView& view) {
+  return HeadCopy{view.base, nullptr, const_cast<bf16*>(view.tail), 0, 0, view.tail_first, view.tail_cols};
+}
+
+constexpr GemmLoads kCopies = GemmLoads::kCopies, kThrough = GemmLoads::kThroughRegisters, kGuarded = GemmLoads::kGuarded;
+template <class Kernel>
+static Kernel by_loads(GemmLoads loads, Kernel copies, Kernel through, Kernel guarded) {
+  return loads == kCopies ? copies : loads == kThrough ? through : guarded;
 }
 
 template <int NB>
-static int launch_stats(const char* fn, hipStream_t stream, const CutceParams& p, bool guarded, float* part, int chunk0,
+static int launch_stats(const char* fn, hipStream_t stream, const CutceParams& p, GemmLoads loads, float* part, int chunk0,
                         int chunks, int tiles_per_chunk, float* cache) {
   static std::atomic<unsigned> lds_allowed{0};
-  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<NB, false, false>, cutce_stats_kernel<NB, true, false>,
-                                cutce_stats_kernel<NB, false, true>, cutce_stats_kernel<NB, true, true>);
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<NB, false, kCopies>, cutce_stats_kernel<NB, true, kCopies>,
+                                cutce_stats_kernel<NB, false, kThrough>, cutce_stats_kernel<NB, true, kThrough>,
+                                cutce_stats_kernel<NB, false, kGuarded>, cutce_stats_kernel<NB, true, kGuarded>);
   if (rc) return rc;
-  const auto kernel = cache ? (guarded ? cutce_stats_kernel<NB, true, true> : cutce_stats_kernel<NB, true, false>)
-                            : (guarded ? cutce_stats_kernel<NB, false, true> : cutce_stats_kernel<NB, false, false>);
+  const auto kernel = cache ? by_loads(loads, cutce_stats_kernel<NB, true, kCopies>, cutce_stats_kernel<NB, true, kThrough>,
+                                       cutce_stats_kernel<NB, true, kGuarded>)
+                            : by_loads(loads, cutce_stats_kernel<NB, false, kCopies>, cutce_stats_kernel<NB, false, kThrough>,
+                                       cutce_stats_kernel<NB, false, kGuarded>);
   const int slots = device_cu_count() * GemmShape<NB>::kGroups, units = chunks * ((p.N + 64 * NB - 1) / (64 * NB));
   LaunchScope scope("cutce_stats_kernel", stream);
   hipLaunchKernelGGL(kernel, dim3(min(slots, units)), dim3(256), GemmShape<NB>::kBytes, stream, p, part, chunk0, chunks,
@@ -1582,28 +1656,33 @@ static int launch_stats(const char* fn, hipStream_t stream, const CutceParams& p
 
 // slab_tiles: of the kernel's tile size
 template <int NB>
-static int launch_dlogits(const char* fn, hipStream_t stream, const CutceParams& p, const CutceRowParams& rp, bool guarded,
+static int launch_dlogits(const char* fn, hipStream_t stream, const CutceParams& p, const CutceRowParams& rp, GemmLoads loads,
                           int slab0, int slab_tiles, int tiles_per_chunk, bf16* G) {
   static std::atomic<unsigned> lds_allowed{0};
-  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_dlogits_kernel<NB, false>, cutce_dlogits_kernel<NB, true>);
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_dlogits_kernel<NB, kCopies>, cutce_dlogits_kernel<NB, kThrough>,
+                                cutce_dlogits_kernel<NB, kGuarded>);
   if (rc) return rc;
   const int slots = device_cu_count() * GemmShape<NB>::kGroups;
   const int units = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk * ((p.N + 64 * NB - 1) / (64 * NB));
   LaunchScope scope("cutce_dlogits_kernel", stream);
-  hipLaunchKernelGGL((guarded ? cutce_dlogits_kernel<NB, true> : cutce_dlogits_kernel<NB, false>), dim3(min(slots, units)),
+  hipLaunchKernelGGL(by_loads(loads, cutce_dlogits_kernel<NB, kCopies>, cutce_dlogits_kernel<NB, kThrough>,
+                              cutce_dlogits_kernel<NB, kGuarded>), dim3(min(slots, units)),
                      dim3(256), GemmShape<NB>::kBytes, stream, p, rp, slab0, slab_tiles, tiles_per_chunk, G);
   return scope.done();
 }
 
 template <int NB>
 static int launch_grads(const char* fn, hipStream_t stream, const CutceParams& p, const CutceSlab& slab, const CutceSplits& sp,
-                        bool guarded) {
+                        GemmLoads loads) {
   static std::atomic<unsigned> lds_allowed{0};
-  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_grads_kernel<NB, false, false>, cutce_grads_kernel<NB, true, false>,
-                                cutce_grads_kernel<NB, false, true>, cutce_grads_kernel<NB, true, true>);
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_grads_kernel<NB, false, kCopies>, cutce_grads_kernel<NB, true, kCopies>,
+                                cutce_grads_kernel<NB, false, kThrough>, cutce_grads_kernel<NB, true, kThrough>,
+                                cutce_grads_kernel<NB, false, kGuarded>, cutce_grads_kernel<NB, true, kGuarded>);
   if (rc) return rc;
-  const auto kernel = sp.with_head ? (guarded ? cutce_grads_kernel<NB, true, true> : cutce_grads_kernel<NB, true, false>)
-                                   : (guarded ? cutce_grads_kernel<NB, false, true> : cutce_grads_kernel<NB, false, false>);
+  const auto kernel = sp.with_head ? by_loads(loads, cutce_grads_kernel<NB, true, kCopies>, cutce_grads_kernel<NB, true, kThrough>,
+                                              cutce_grads_kernel<NB, true, kGuarded>)
+                                   : by_loads(loads, cutce_grads_kernel<NB, false, kCopies>, cutce_grads_kernel<NB, false, kThrough>,
+                                              cutce_grads_kernel<NB, false, kGuarded>);
   LaunchScope scope(sp.with_head ? "cutce_grads_kernel" : "cutce_dhidden_kernel", stream);
   hipLaunchKernelGGL(kernel, dim3(device_cu_count() * GemmShape<NB>::kGroups), dim3(256), GemmShape<NB>::kBytes, stream, p, slab,
                      sp);
@@ -1656,13 +1735,22 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
   // The panel of a head with unaligned rows: lent by the caller, at the end of the logits cache, where the backward finds
   // it again, or in what the workspace has behind its fixed part, a number of chunks at a time.
   const int step_tiles = units.per_chunk, step_chunks = kGemmTile / units.tile;  // 256-column tiles and chunks of a panel step
+  // Read in place it needs the panel's first tile column only, for its tail.
   bf16* panel = nullptr;
+  HeadCopy tail = {};
   int chunks_per_pass = units.chunks;
   if (!needs_panel(a->shape)) {
     lent = nullptr;
   } else {
     if (lent) {
       panel = lent;
+    } else if (a->logits_cache ? both_in_place(a->shape) : forward_in_place(a->shape)) {
+      char* place = a->logits_cache ? static_cast<char*>(a->logits_cache) + logits_bytes(a->shape)
+                                    : ws_bytes - L.base >= panel_tile_bytes(a->shape) ? ws + L.base : nullptr;
+      if (place) {
+        p.head = tail_view(p, reinterpret_cast<const bf16*>(place), kGemmTile);
+        tail = tail_copy(p.head);
+      }
     } else if (a->logits_cache) {
       panel = reinterpret_cast<bf16*>(static_cast<char*>(a->logits_cache) + logits_bytes(a->shape));
     } else {
@@ -1671,10 +1759,11 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
       if (fit) chunks_per_pass = (int)(fit * step_chunks < (size_t)units.chunks ? fit * step_chunks : (size_t)units.chunks);
     }
   }
-  const bool guarded = !p.hidden_aligned || (!panel && !(is_aligned16(head) && p.V % 8 == 0));
+  const bool guarded = !p.hidden_aligned || (!panel && !tail.tail && !(is_aligned16(head) && p.V % 8 == 0));
+  const GemmLoads loads = guarded ? kGuarded : tail.tail ? kThrough : kCopies;
   for (int chunk0 = 0; chunk0 < units.chunks; chunk0 += chunks_per_pass) {
     const int pass_chunks = min(chunks_per_pass, units.chunks - chunk0);
-    HeadCopy copy = {};
+    HeadCopy copy = tail;
     if (panel) {
       const int tile0 = chunk0 / step_chunks * step_tiles;
       const int pass_tiles = min((pass_chunks + step_chunks - 1) / step_chunks * step_tiles, vocab_tile_count(p.V) - tile0);
@@ -1684,7 +1773,7 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     const int list_blocks = chunk0 == 0 ? (p.N + 1023) / 1024 : 0;
     if ((rc = launch_prepare<false>(stream, p, CutceRowWork{}, copy, list_blocks, list_blocks == 0))) return rc;
     const auto launch = units.tile == kGemmTile ? launch_stats<4> : launch_stats<2>;
-    if ((rc = launch(fn, stream, p, guarded, part, chunk0, pass_chunks, units.per_chunk, static_cast<float*>(a->logits_cache))))
+    if ((rc = launch(fn, stream, p, loads, part, chunk0, pass_chunks, units.per_chunk, static_cast<float*>(a->logits_cache))))
       return rc;
   }
 
@@ -1755,6 +1844,10 @@ extern "C" size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape) {
   return valid_sizes(shape) ? full_panel_bytes(*shape) : 0;
 }
 
+extern "C" int32_t ct_cutce_head_in_place(const ct_cutce_shape* shape) {
+  return valid_sizes(shape) && both_in_place(*shape);
+}
+
 extern "C" int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* a, uint16_t* panel, size_t panel_bytes,
                                       int32_t filled) {
   CT_REQUIRE(a, "ct_cutce_fwd: null args");
@@ -1795,27 +1888,36 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
   rp.tgt = reinterpret_cast<int*>(ws + L.rowparams + 2 * params_stride);
   bf16* packed = dhead ? reinterpret_cast<bf16*>(ws + L.packed) : nullptr;
   const bool head_aligned = is_aligned16(a->head) && p.V % 8 == 0;
-  bf16* tail = head_aligned && p.V % 128 ? reinterpret_cast<bf16*>(ws + L.tail) : nullptr;
   const CutceRowWork work = {a->lse, a->dy, rp, packed, dhidden};
 
   const int cus = device_cu_count();
   const int tiles = vocab_tile_count(p.V);
   const int tiles_per_slab = L.slab_cols / kGemmTile;
   const bf16* head = p.head.base;
-  p.head.tail = tail;
   bf16* panel = nullptr;
-  if (needs_panel(a->shape)) {
+  HeadCopy tail = {};
+  const bool in_place = !lent && (cache ? both_in_place(a->shape) : L.slabs == 1 && backward_in_place(a->shape));
+  if (head_aligned && p.V % 128) {
+    p.head = tail_view(p, reinterpret_cast<const bf16*>(ws + L.tail), 128);
+    tail = tail_copy(p.head);
+  } else if (needs_panel(a->shape)) {
+    // (the forward left panel or tail in the cache)
+    const bf16* left = cache ? reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(cache) + logits_bytes(a->shape)) : nullptr;
     if (lent) {
       p.head = panel_view(reinterpret_cast<const bf16*>(lent), 0, tiles);
-    } else if (cache) {  // the forward left it there
-      p.head = panel_view(reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(cache) + logits_bytes(a->shape)), 0, tiles);
+    } else if (in_place) {
+      p.head = tail_view(p, left ? left : reinterpret_cast<const bf16*>(ws + L.panel), kGemmTile);
+      if (!left) tail = tail_copy(p.head);
+    } else if (left) {
+      p.head = panel_view(left, 0, tiles);
     } else {
       panel = reinterpret_cast<bf16*>(ws + L.panel);
     }
   }
   // (an unaligned head with a multiple of 8 columns has no panel)
   const bool guarded_head = !needs_panel(a->shape) && !head_aligned;
-  const bool guarded_logits = guarded_head || !p.hidden_aligned;
+  const GemmLoads head_loads = guarded_head ? kGuarded : in_place ? kThrough : kCopies;
+  const GemmLoads logits_loads = p.hidden_aligned ? head_loads : kGuarded;
   for (int s = 0; s < L.slabs; ++s) {
     const int slab0 = s * L.slab_cols;
     const int slab_tiles = min(tiles_per_slab, tiles - s * tiles_per_slab);
@@ -1825,8 +1927,7 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
       copy = panel_copy(head, panel, s * tiles_per_slab, slab_tiles);
       p.head = panel_view(panel, s * tiles_per_slab, slab_tiles);
     } else if (s == 0) {
-      copy.head = head;
-      copy.tail = tail;
+      copy = tail;
     }
     const int list_blocks = s == 0 ? (p.N + 16 * row_rounds(p.N) - 1) / (16 * row_rounds(p.N)) : 0;
     if ((list_blocks || panel) && (rc = launch_prepare<true>(stream, p, work, copy, list_blocks, false))) return rc;
@@ -1838,11 +1939,11 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
       if ((rc = scope11.done())) return rc;
     } else {
       if (projection_tile(p.N, slab_tiles) == kGemmTile) {
-        rc = launch_dlogits<4>("ct_cutce_bwd", stream, p, rp, guarded_logits, slab0, slab_tiles,
+        rc = launch_dlogits<4>("ct_cutce_bwd", stream, p, rp, logits_loads, slab0, slab_tiles,
                                tiles_per_chunk(slab_tiles, row_blocks), G);
       } else {  // (an unpadded head has no columns past the vocabulary to read)
         const int columns = p.head.padded ? slab_width : min(slab_width, p.V - slab0);
-        rc = launch_dlogits<2>("ct_cutce_bwd", stream, p, rp, guarded_logits, slab0, (columns + 127) / 128, 1, G);
+        rc = launch_dlogits<2>("ct_cutce_bwd", stream, p, rp, logits_loads, slab0, (columns + 127) / 128, 1, G);
       }
       if (rc) return rc;
     }
@@ -1859,7 +1960,7 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
     sp.head_tile = gradient_tile(a->shape);
     sp.vocab = tiles * kGemmTile;
     sp.with_head = dhead != nullptr;
-    rc = (sp.tile == kGemmTile ? launch_grads<4> : launch_grads<2>)("ct_cutce_bwd", stream, p, slab, sp, guarded_head);
+    rc = (sp.tile == kGemmTile ? launch_grads<4> : launch_grads<2>)("ct_cutce_bwd", stream, p, slab, sp, head_loads);
     if (rc) return rc;
     if (sp.hidden_room || sp.head_most > 1) {
       LaunchScope scope9("cutce_reduce_kernel", stream);

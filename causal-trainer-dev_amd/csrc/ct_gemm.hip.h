@@ -14,13 +14,16 @@
 //             with transposed LDS reads.
 // The rows of a k-contiguous operand can be addressed through an index list (gather).
 //
-// Two main loops share the loaders; a kernel is compiled for one of them (GUARDED), because both in
-// one kernel cost it registers, spills and instruction cache:
+// Three main loops share the loaders; a kernel is compiled for one of them (GemmLoads), because more than one in
+// a kernel cost it registers, spills and instruction cache:
 //   pipelined  operands 16-byte aligned, contraction a multiple of 128: tiles are copied global ->
 //              LDS asynchronously, three steps ahead, into a ring of 4 LDS stages; MFMA fragments
 //              are double buffered in registers so that LDS reads of the next half step overlap
 //              the current MFMAs; one barrier per step (gen_gemm_asm.py). Rows or
 //              columns of a tile past the end of the matrix are copies of valid ones.
+//   through registers  the same loop where the rows of one operand start at any multiple of 2 bytes and the tile
+//              lies inside of the matrix: that operand's chunks are loaded into registers two to three steps ahead
+//              and stored to the LDS ring one step ahead (unaligned global loads; the copies need aligned chunks).
 //   guarded    unaligned operands: element-wise guarded loads that zero fill, staged through
 //              registers, 2 LDS stages.
 #pragma once
@@ -32,6 +35,8 @@ namespace ct {
 
 constexpr int kGemmTile = 256;  // of the large tile, and what row blocks and vocabulary are padded to
 constexpr int kGemmBK = 32;
+
+enum class GemmLoads { kCopies, kThroughRegisters, kGuarded };
 
 CT_DEVICE u32x4 load_chunk_guarded(const bf16* p, int count) {
   bf16x8 v;
@@ -122,6 +127,29 @@ struct KcLoader {
   typedef RowFragOffsets<CPR> FragOffsets;
   static CT_DEVICE bf16x8 frag(int tile_off, const FragOffsets& fo, int ks, int wave_first, int i) {
     return fo.load(tile_off + (wave_first / 32) * FragOffsets::kRowBlockBytes, i, ks);
+  }
+};
+
+// The rows of a k-contiguous tile through registers, two steps (128 bytes of a row) at a time: thread t loads 16-byte
+// chunk t % 8 of the rows t / 8 + 32 n of the tile, n < 2 NB, and stores it to the stage of its step. Rows as in KcLoader
+// with interleave_rows, which may start at any multiple of 2 bytes.
+template <int NB>
+struct KcPairLoader {
+  static constexpr int CPR = kGemmBK / 8, NCH = 2 * NB;
+  const char* base;  // uniform
+  unsigned voff[NCH];
+  int lds;  // byte offset of the thread's first chunk from the B tile of an even stage
+
+  CT_DEVICE void init(const bf16* base_, long ld, int m0, int rows_valid) {
+    const int t = threadIdx.x, r0 = t / 8, chunk = t % 8;
+    base = reinterpret_cast<const char*>(base_ + (size_t)m0 * ld);
+    lds = (chunk / CPR) * GemmShape<NB>::kStageBytes + tile_byte_offset<CPR>(r0, chunk % CPR);
+#pragma unroll
+    for (int n = 0; n < NCH; ++n) {
+      const int tile_row = r0 + 32 * n;
+      const int r = (tile_row & (32 * NB)) | ((tile_row & 31) * NB) | ((tile_row >> 5) % NB);
+      voff[n] = (unsigned)(((long)(m0 + r < rows_valid ? r : 0) * ld + chunk * 8) * 2);
+    }
   }
 };
 
@@ -269,15 +297,18 @@ CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
   return ((unsigned long long)hi << 32) | (unsigned long long)lo;
 }
-template <GemmStart START>
-CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, int steps,
+// Operands of the loops' asm statements. THROUGH: the operand that comes through registers (A: CT_GEMM_VIA_A_LOOP, from C = 0;
+// B: CT_GEMM_VIA_B_LOOP, adding), entered with the other one's copies of steps 0..2 issued and none of its own loads.
+enum class Through { kNone, kA, kB };
+template <GemmStart START, Through THROUGH = Through::kNone, class LoaderB = KcLoader<4>>
+CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const LoaderB& B, int k_begin, int steps,
                                    lds_addr smem, const McLoader<4>::FragOffsets& afo,
                                    const KcLoader<4>::FragOffsets& bfo, int wm, int wn, GemmAcc<4>& acc) {
   const int wave = uniform(threadIdx.x >> 6);
-  // sources of the copies of step 3
-  const unsigned long long src_a =
-      uniform64(A.base + (size_t)(k_begin + 3 * kGemmBK) * (size_t)A.ld * 2);
-  const unsigned long long src_b = uniform64(B.base + (size_t)(k_begin + 3 * kGemmBK) * 2);
+  // sources of the copies of step 3, of the loads of step 0
+  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK), first_b = k_begin + (THROUGH == Through::kB ? 0 : 3 * kGemmBK);
+  const unsigned long long src_a = uniform64(A.base + (size_t)first_a * (size_t)A.ld * 2);
+  const unsigned long long src_b = uniform64(B.base + (size_t)first_b * 2);
   const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
   const unsigned steps_u = (unsigned)uniform(steps);
   const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + wave * 1024));
@@ -292,7 +323,19 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, i
       "v"(afo.ptr[1][1] + a_off), "v"(afo.ptr[1][2] + a_off), "v"(afo.ptr[1][3] + a_off), "v"(bfo.ptr[0] + b_off), \
       "v"(bfo.ptr[1] + b_off), "v"(A.voff[0]), "v"(A.voff[1]), "v"(A.voff[2]), "v"(A.voff[3]), "v"(B.voff[0]), \
       "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
-  if constexpr (START == GemmStart::kAdd)
+  if constexpr (THROUGH != Through::kNone) {
+    static_assert((THROUGH == Through::kA) == (START != GemmStart::kAdd), "the forms that there are");
+    if constexpr (THROUGH == Through::kA) {
+      const lds_addr thread = smem + (int)threadIdx.x * 16;
+      asm volatile(CT_GEMM_VIA_A_LOOP : CT_GEMM_ACC("=&a") : CT_GEMM_IN, "v"(thread)
+                   : "memory", "m0", "scc", CT_GEMM_VIA_LOOP_CLOBBERS);
+    } else {
+      const lds_addr thread = smem + B.lds;
+      asm volatile(CT_GEMM_VIA_B_LOOP : CT_GEMM_ACC("+a")
+                   : CT_GEMM_IN, "v"(B.voff[4]), "v"(B.voff[5]), "v"(B.voff[6]), "v"(B.voff[7]), "v"(thread)
+                   : "memory", "m0", "scc", CT_GEMM_VIA_LOOP_CLOBBERS);
+    }
+  } else if constexpr (START == GemmStart::kAdd)
     asm volatile(CT_GEMM_LOOP : CT_GEMM_ACC("+a") : CT_GEMM_IN : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
   else if constexpr (START == GemmStart::kFresh)
     asm volatile(CT_GEMM_FRESH_LOOP : CT_GEMM_ACC("=&a") : CT_GEMM_IN : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
@@ -301,6 +344,14 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, i
                  : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
 #undef CT_GEMM_ACC
 #undef CT_GEMM_IN
+}
+
+// The copies of an operand's first three steps (four in the small tile).
+template <class Loader>
+CT_DEVICE void copy_first_steps(const Loader& loader, int k_begin, lds_addr tile) {
+  constexpr int kNb = Loader::NCH;
+#pragma unroll
+  for (int i = 0; i < (kNb == 4 ? 3 : 4); ++i) loader.dma(k_begin + i * kGemmBK, tile + i * GemmShape<kNb>::kStageBytes);
 }
 
 // The copies of a tile's first three steps, ahead of gemm_tile_fresh (nothing may be using the LDS stages).
@@ -329,9 +380,17 @@ CT_DEVICE void gemm_tile_fresh(const McLoader<4>& A, const KcLoader<4>& B, int k
   gemm_loop_scheduled<kStart>(A, B, 0, k_end / kGemmBK, smem, afo, bfo, (w >> 1) * 128, (w & 1) * 128, acc);
 }
 
+// acc = the same product with A through registers, behind copy_first_steps of B.
+CT_DEVICE void gemm_tile_through_a(const McLoader<4>& A, const KcLoader<4>& B, int k_end, lds_addr smem, GemmAcc<4>& acc) {
+  const int w = threadIdx.x >> 6;
+  const McLoader<4>::FragOffsets afo(smem);
+  const KcLoader<4>::FragOffsets bfo(smem);
+  gemm_loop_scheduled<GemmStart::kFresh, Through::kA>(A, B, 0, k_end / kGemmBK, smem, afo, bfo, (w >> 1) * 128, (w & 1) * 128, acc);
+}
+
 // acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T (k_end - k_begin a multiple of 128
-// unless GUARDED). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
-template <bool GUARDED>
+// unless kGuarded). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
+template <GemmLoads LOADS>
 CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
   constexpr int BK = kGemmBK, kTile = GemmShape<4>::kTileBytes, kStage = GemmShape<4>::kStageBytes;
   const int w = threadIdx.x >> 6;
@@ -339,7 +398,7 @@ CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end,
   if (k_begin >= k_end) return;
   const McLoader<4>::FragOffsets afo(smem);
   const KcLoader<4>::FragOffsets bfo(smem);
-  if constexpr (!GUARDED) {
+  if constexpr (LOADS == GemmLoads::kCopies) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -382,45 +441,87 @@ CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end,
   }
 }
 
-// The same sum for the small tile (NB = 2: 128 x 128, 64 accumulator registers, two workgroups per
-// compute unit), with a fixed order of its own (gen_gemm_asm.py).
-template <bool GUARDED>
-CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
-  typedef GemmShape<2> Shape;
-  typedef RowFragOffsets<KcLoader<2>::CPR> BOffsets;
-  constexpr int kStage = Shape::kStageBytes, kTile = Shape::kTileBytes;
+// The same with B through registers.
+CT_DEVICE void gemm_tile(McLoader<4>& A, KcPairLoader<4>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
   if (k_begin >= k_end) return;
-  const int w = uniform(threadIdx.x >> 6), wm = (w >> 1) * Shape::kWave, wn = (w & 1) * Shape::kWave, l = lane_id();
-  // this lane's part of the wavefront's fragments, stage 0
-  lds_addr a_ptr[2][2];
+  const int w = threadIdx.x >> 6;
+  const McLoader<4>::FragOffsets afo(smem);
+  const KcLoader<4>::FragOffsets bfo(smem);
+  dma_wait_all();
+  copy_first_steps(A, k_begin, smem);
+  gemm_loop_scheduled<GemmStart::kAdd, Through::kB>(A, B, k_begin, (k_end - k_begin) / kGemmBK, smem, afo, bfo, (w >> 1) * 128,
+                                                    (w & 1) * 128, acc);
+}
+
+// The small tile (NB = 2: 128 x 128, 64 accumulator registers, two workgroups per compute unit), with a fixed order of its
+// own (gen_gemm_asm.py).
+struct SmallFrags {
+  lds_addr a[2][2];  // this lane's part of the wavefront's fragments, stage 0
+  RowFragOffsets<KcLoader<2>::CPR> b;
+  CT_DEVICE explicit SmallFrags(lds_addr smem)
+      : b(smem + GemmShape<2>::kTileBytes + (uniform(threadIdx.x >> 6) & 1) * 2 * RowFragOffsets<KcLoader<2>::CPR>::kRowBlockBytes) {
+    const int wm = (uniform(threadIdx.x >> 6) >> 1) * GemmShape<2>::kWave, l = lane_id();
 #pragma unroll
-  for (int second = 0; second < 2; ++second)
+    for (int second = 0; second < 2; ++second)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 8 * (l >> 5) + 4 * second + ((l & 15) >> 2), col = wm + 32 * i + 16 * ((l >> 4) & 1) + 4 * (l & 3);
-      a_ptr[second][i] = smem + tile_byte_offset<McLoader<2>::CPR>(row, col >> 3) + (col & 4) * 2;
-    }
-  const BOffsets b_ptr(smem + kTile + (wn / 32) * BOffsets::kRowBlockBytes);
-  if constexpr (!GUARDED) {
-    static_assert(McLoader<2>::NCH + KcLoader<2>::NCH == 4, "the waits count the copies of a step");
+      for (int i = 0; i < 2; ++i) {
+        const int row = 8 * (l >> 5) + 4 * second + ((l & 15) >> 2), col = wm + 32 * i + 16 * ((l >> 4) & 1) + 4 * (l & 3);
+        a[second][i] = smem + tile_byte_offset<McLoader<2>::CPR>(row, col >> 3) + (col & 4) * 2;
+      }
+  }
+};
+
+// acc += the product, entered with the first four steps' copies issued (step 0's landed, for every wavefront), of an
+// operand through registers none.
+template <Through THROUGH, class LoaderB>
+CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const LoaderB& B, int k_begin, int k_end, lds_addr smem, const SmallFrags& f,
+                               GemmAcc<2>& acc) {
+  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK), first_b = k_begin + (THROUGH == Through::kB ? 0 : 3 * kGemmBK);
+  const unsigned long long src_a = uniform64(A.base + (size_t)first_a * (size_t)A.ld * 2);
+  const unsigned long long src_b = uniform64(B.base + (size_t)first_b * 2);
+  const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
+  const unsigned steps = (unsigned)uniform((k_end - k_begin) / kGemmBK);
+  const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + uniform(threadIdx.x >> 6) * 1024));
+#define CT_GEMM_SMALL_ACC "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[1][0]), "+a"(acc.c[1][1])
+#define CT_GEMM_SMALL_IN \
+  "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps), "s"(lds_wave), "v"(f.a[0][0]), "v"(f.a[0][1]), "v"(f.a[1][0]), \
+      "v"(f.a[1][1]), "v"(f.b.ptr[0]), "v"(f.b.ptr[1]), "v"(A.voff[0]), "v"(A.voff[1]), "v"(B.voff[0]), "v"(B.voff[1])
+  if constexpr (THROUGH == Through::kNone) {
+    asm volatile(CT_GEMM_SMALL_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN
+                 : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
+  } else if constexpr (THROUGH == Through::kA) {
+    const lds_addr thread = smem + (int)threadIdx.x * 16;
+    asm volatile(CT_GEMM_SMALL_VIA_A_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
+                 : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
+  } else {
+    const lds_addr thread = smem + B.lds;
+    asm volatile(CT_GEMM_SMALL_VIA_B_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(B.voff[2]), "v"(B.voff[3]), "v"(thread)
+                 : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
+  }
+#undef CT_GEMM_SMALL_ACC
+#undef CT_GEMM_SMALL_IN
+}
+
+// acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T in the small tile; kThroughRegisters: A comes through them.
+template <GemmLoads LOADS>
+CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
+  constexpr int kTile = GemmShape<2>::kTileBytes;
+  if (k_begin >= k_end) return;
+  const SmallFrags frags(smem);
+  static_assert(McLoader<2>::NCH + KcLoader<2>::NCH == 4, "the waits count the copies of a step");
+  if constexpr (LOADS == GemmLoads::kCopies) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      A.dma(k_begin + i * kGemmBK, smem + i * kStage);
-      B.dma(k_begin + i * kGemmBK, smem + i * kStage + kTile);
+      A.dma(k_begin + i * kGemmBK, smem + i * GemmShape<2>::kStageBytes);
+      B.dma(k_begin + i * kGemmBK, smem + i * GemmShape<2>::kStageBytes + kTile);
     }
     asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // step 0 has landed
-    const unsigned long long src_a = uniform64(A.base + (size_t)(k_begin + 3 * kGemmBK) * (size_t)A.ld * 2);
-    const unsigned long long src_b = uniform64(B.base + (size_t)(k_begin + 3 * kGemmBK) * 2);
-    const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
-    const unsigned steps = (unsigned)uniform((k_end - k_begin) / kGemmBK);
-    const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + w * 1024));
-    asm volatile(CT_GEMM_SMALL_LOOP
-                 : "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[1][0]), "+a"(acc.c[1][1])
-                 : "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps), "s"(lds_wave), "v"(a_ptr[0][0]), "v"(a_ptr[0][1]),
-                   "v"(a_ptr[1][0]), "v"(a_ptr[1][1]), "v"(b_ptr.ptr[0]), "v"(b_ptr.ptr[1]), "v"(A.voff[0]), "v"(A.voff[1]),
-                   "v"(B.voff[0]), "v"(B.voff[1])
-                 : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
+    gemm_small_loop<Through::kNone>(A, B, k_begin, k_end, smem, frags, acc);
+  } else if constexpr (LOADS == GemmLoads::kThroughRegisters) {
+    dma_wait_all();
+    copy_first_steps(B, k_begin, smem + kTile);
+    gemm_small_loop<Through::kA>(A, B, k_begin, k_end, smem, frags, acc);
   } else {
 #pragma nounroll
     for (int k0 = k_begin; k0 < k_end; k0 += kGemmBK) {
@@ -435,9 +536,9 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int off = ks * (16 * McLoader<2>::CPR * 16);
-          const bf16x4_vs lo = lds_load_tr(a_ptr[0][i] + off), hi = lds_load_tr(a_ptr[1][i] + off);
+          const bf16x4_vs lo = lds_load_tr(frags.a[0][i] + off), hi = lds_load_tr(frags.a[1][i] + off);
           a[i] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          b[i] = b_ptr.load(0, i, ks);
+          b[i] = frags.b.load(0, i, ks);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -448,6 +549,14 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
     }
     acc.settle();
   }
+}
+
+// The same with B through registers.
+CT_DEVICE void gemm_tile(McLoader<2>& A, KcPairLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
+  if (k_begin >= k_end) return;
+  dma_wait_all();
+  copy_first_steps(A, k_begin, smem);
+  gemm_small_loop<Through::kB>(A, B, k_begin, k_end, smem, SmallFrags(smem), acc);
 }
 
 // The rows of a wavefront's tile in the order of its accumulators (0..3, 8..11, ...; lanes of the other half
@@ -468,12 +577,14 @@ struct TileRows {
 // the tile before: with one workgroup on a compute unit nothing else hides them. What run() waits for goes by the
 // stores counted since begin() (a constant wherever an epilogue issues them on every path): where they are too
 // few for the counted waits, as on a kernel's first tile, it waits for all copies.
-template <int NB, bool GUARDED, bool STORES>
+// kThroughRegisters (A): only B's copies travel ahead.
+template <int NB, GemmLoads LOADS, bool STORES>
 struct GemmTiles {
-  static constexpr bool kAhead = NB == 4 && !GUARDED;
+  static constexpr bool kAhead = NB == 4 && LOADS == GemmLoads::kCopies;
   int stores = 0;  // of this wavefront behind the copies of begin()
   CT_DEVICE void begin(const McLoader<NB>& A, const KcLoader<NB>& B, lds_addr smem) {
     if constexpr (kAhead) gemm_copy_ahead(A, B, smem);
+    else if constexpr (NB == 4 && LOADS == GemmLoads::kThroughRegisters) copy_first_steps(B, 0, smem + GemmShape<4>::kTileBytes);
   }
   // a lane's NB consecutive elements of accumulator row r of a block (wave-uniform control flow only)
   template <class Elements>
@@ -487,9 +598,11 @@ struct GemmTiles {
     if constexpr (kAhead) {
       gemm_tile_fresh<STORES>(A, B, k_end, smem, acc, stores < kStoresBehindCopies);
       stores = 0;
+    } else if constexpr (NB == 4 && LOADS == GemmLoads::kThroughRegisters) {
+      gemm_tile_through_a(A, B, k_end, smem, acc);
     } else {
       acc.clear();
-      gemm_tile<GUARDED>(A, B, 0, k_end, smem, acc);
+      gemm_tile<LOADS>(A, B, 0, k_end, smem, acc);
     }
   }
 };

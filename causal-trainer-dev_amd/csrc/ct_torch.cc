@@ -669,9 +669,11 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
     if ((int64_t)bytes <= cache_limit && cache_pays(shape)) cache = scratch(bytes, hidden);
   }
   // An unaligned head is copied once for both directions only where the caller lets a buffer be kept between them, like
-  // the logits cache, which holds such a copy itself. Otherwise each direction makes one in its workspace.
+  // the logits cache, which holds such a copy itself. Otherwise each direction makes one in its workspace or reads it in
+  // place; with few rows both do.
   if (head_is_panel) panel = columns;
-  else if (use_cache && graph && !cache && panel_bytes && (int64_t)panel_bytes <= std::min(kPanelLimit, cache_limit))
+  else if (use_cache && graph && !cache && panel_bytes && (int64_t)panel_bytes <= std::min(kPanelLimit, cache_limit) &&
+           !ct_cutce_head_in_place(&shape))
     panel = scratch(panel_bytes, hidden);
   auto [nll, weight_sum, lse] =
       cutce_forward_on(shape, hidden, columns, targets, weights, compaction, cache, forward_bytes, panel, head_is_panel);

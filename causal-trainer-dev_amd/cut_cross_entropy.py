@@ -21,7 +21,8 @@ that lives until the backward of the loss (the adjacent step of a training
 iteration), and the backward then runs 3 GEMMs instead of 4. Above the limit, or where
 the projection is cheaper than the cache's traffic (small hidden sizes), the logits are
 recomputed, and what is kept in the cache's place is the aligned copy that a head whose
-vocabulary is no multiple of 8 is read through, up to the limit and 1 GiB. Like the cache it
+vocabulary is no multiple of 8 is read through, up to the limit and 1 GiB (with few rows such a head is read
+in place, and nothing is kept). Like the cache it
 is no saved tensor (hooks do not see it) and goes with the first backward. With
 ``logits_cache=False`` nothing but ``lse`` is kept: logits and copy are made again.
 

@@ -424,7 +424,8 @@ typedef struct ct_cutce_shape {
 /* Preferred and smallest workspace for ct_cutce_fwd. The two differ where vocab is no multiple of
  * 8: the kernels then read the head through an aligned copy of its columns (2 bytes per element),
  * made in the workspace behind its fixed part as many columns at a time as fit, or in the logits
- * cache if there is one; with no room for it the projection runs in a slower guarded loop. Same
+ * cache if there is one, or, where rows are few, in place but for its last columns, whose copy takes 512
+ * bytes per hidden column there; with no room for it the projection runs in a slower guarded loop. Same
  * results in each case. */
 size_t ct_cutce_fwd_workspace_bytes(const ct_cutce_shape* shape);
 size_t ct_cutce_fwd_workspace_min_bytes(const ct_cutce_shape* shape);
@@ -529,8 +530,11 @@ int32_t ct_cutce_bwd(void* stream, const ct_cutce_bwd_args* args);
  * args->head is then not read, and the workspaces are smaller by its size. A panel where none is needed is ignored.
  * A logits cache beside a panel has no room for another one: exactly ct_cutce_logits_cache_bytes() less
  * ct_cutce_panel_bytes(); any other size is refused, and ct_cutce_bwd without the panel refuses such a cache.
+ * With few rows and a large head the kernels read an unaligned head in place rather than make a panel (a lent one they use
+ * all the same): ct_cutce_head_in_place() is 1 where both directions do, and lending one to be filled only costs its copy.
  */
 size_t ct_cutce_panel_bytes(const ct_cutce_shape* shape);
+int32_t ct_cutce_head_in_place(const ct_cutce_shape* shape);
 int32_t ct_cutce_fwd_panel(void* stream, const ct_cutce_fwd_args* args, uint16_t* panel, size_t panel_bytes, int32_t filled);
 int32_t ct_cutce_bwd_panel(void* stream, const ct_cutce_bwd_args* args, const uint16_t* panel, size_t panel_bytes);
 

@@ -5,6 +5,8 @@ test reliably shows. In the model copies and stores complete in the order of the
 the four wavefronts of a workgroup run the same stream, so what one of them has waited for before a barrier, all have.
 Checked for every instruction: an LDS read finds the copies of its step landed in front of a barrier, a copy goes where
 every read is done in front of a barrier and no other copy is on its way, and every MFMA has the fragments of its step.
+An operand that comes through registers: a chunk's load has landed when it is stored to LDS, and the store counts as a copy
+that has landed once the wavefront has waited for it.
 """
 
 import importlib.util
@@ -30,7 +32,7 @@ def gen():
 class Tile:
     """What the operands of a loop's asm statement stand for, and the layout of its LDS stages."""
 
-    def __init__(self, small):
+    def __init__(self, small, via=None):
         self.blocks = 2 if small else 4                     # of a wavefront, in each direction
         self.chunks = self.blocks                           # copies of a wavefront per operand and step
         self.ahead = 4 if small else 3                      # steps copied in front of the loop
@@ -47,39 +49,63 @@ class Tile:
         for ks in range(2):
             self.reads["%%%d" % at] = (1, None, ks)
             at += 1
+        self.pairs = via == 1                               # B through registers, two steps at a time
+        self.per_operand = (self.chunks, self.chunks * (2 if self.pairs else 1))
         for matrix in range(2):
-            for chunk in range(self.chunks):
+            for chunk in range(self.per_operand[matrix]):
                 self.copies["%%%d" % at] = (matrix, chunk)
                 at += 1
+        self.thread = "%%%d" % at
 
 
 class Machine:
     """One wavefront on a loop of `steps` steps. `stores` lie behind the copies of the first steps; `start_wait`: the
-    vmcnt in front of the loop."""
+    vmcnt in front of the loop; `via`: the operand that comes through registers."""
 
     # bytes from step to step of the two sources (the first carries into the upper half of the address), and between them
     STRIDE, HIGH = ((1 << 32) - 4096, 64), 1 << 40
 
-    def __init__(self, tile, steps, fresh, stores, start_wait):
-        self.tile, self.steps, self.fresh = tile, steps, fresh
+    def __init__(self, tile, steps, fresh, stores, start_wait, via=None):
+        self.tile, self.steps, self.fresh, self.via = tile, steps, fresh, via
         self.scalar, self.scc, self.address, self.fragment = {}, 0, {}, {}
+        self.loaded, self.lds_stores = {}, []               # first register -> what a load puts there; on their way to LDS
         self.memory, self.lds_reads = [], []                # in flight, in the order of their issue
         self.slots, self.mfmas, self.started = {}, 0, set()
         for step in range(tile.ahead):
             for matrix in range(2):
                 for chunk in range(tile.chunks):
-                    self._copy(matrix, chunk, step, step)
+                    if matrix != via:
+                        self._copy(matrix, chunk, step, step)
         self.memory += [None] * stores
-        self._wait_memory(start_wait)
-        self._barrier()
+        if start_wait is not None:
+            self._wait_memory(start_wait)
+            self._barrier()
 
     # -- events
-    def _copy(self, matrix, chunk, step, stage):
+    def _copy(self, matrix, chunk, step, stage, flight=None):
         slot = self.slots.setdefault((stage, matrix, chunk), dict(state="free", readers=[]))
         assert slot["state"] != "flying", ("a copy on its way to the same place", stage, matrix, chunk)
         assert all(reader == "fenced" for reader in slot["readers"]), ("a copy over data being read", stage, matrix, chunk)
         slot.update(state="flying", step=step, readers=[])
-        self.memory.append(slot)
+        (self.memory if flight is None else flight).append(slot)
+
+    def _load(self, matrix, chunk, step, registers):
+        assert matrix == self.via
+        for register in registers:
+            assert self.fragment.get(register, [None, True])[1], ("load into a register of a read in flight", register)
+            self.fragment.pop(register, None)
+        held = self.loaded[registers[0]] = dict(state="flying", matrix=matrix, chunk=chunk, step=step)
+        self.memory.append(held)
+
+    def _store(self, registers, where, offset):
+        base, extra = self.address.get(where, (where, 0))
+        assert base == self.tile.thread
+        stage, rest = divmod(offset + extra, self.tile.stage)
+        held = self.loaded[registers[0]]
+        assert held["state"] == "landed", ("store of a chunk that has not landed", held)
+        assert rest == held["matrix"] * self.tile.stage // 2 + held["chunk"] * (2048 if self.tile.pairs else 4096)
+        for second in range(2 if self.tile.pairs else 1):   # (half of the lanes have the next step's chunk)
+            self._copy(held["matrix"], held["chunk"], held["step"] + second, stage + second, self.lds_stores)
 
     def _wait_memory(self, most):
         assert most <= 63
@@ -89,6 +115,9 @@ class Machine:
                 slot["state"] = "landed"
 
     def _wait_lds(self):
+        for slot in self.lds_stores:
+            slot["state"] = "landed"
+        self.lds_stores = []
         for slots, registers in self.lds_reads:
             for slot, index in slots:
                 slot["readers"][index] = "done"
@@ -114,13 +143,16 @@ class Machine:
         else:
             ks, (block, rest) = which, divmod(offset, 2048)
             assert rest == 0 and block < self.tile.blocks, operand
-            chunks = range(self.tile.chunks)                # (two of four, by the wavefront)
+            chunks = range(self.tile.per_operand[1])        # (half of them, by the wavefront)
         slots = []
         for chunk in chunks:
+            assert (stage, matrix, chunk) in self.slots, ("LDS read of a place that nothing was copied to", stage, matrix, chunk)
             slot = self.slots[stage, matrix, chunk]
             assert slot["state"] == "there", ("LDS read ahead of its copies", stage, matrix, chunk, slot["state"])
             slot["readers"].append("pending")
             slots.append((slot, len(slot["readers"]) - 1))
+        assert not any(register in range(first, first + 4) and held["state"] == "flying"
+                       for first, held in self.loaded.items() for register in registers)
         step = slots[0][0]["step"]
         assert all(slot["step"] == step for slot, _ in slots)
         for k, register in enumerate(registers):
@@ -148,7 +180,7 @@ class Machine:
     def _get(self, operand):
         if operand in self.tile.src:                        # address of the copies of step 3
             matrix = self.tile.src[operand]
-            return matrix * self.HIGH + 3 * self.STRIDE[matrix]
+            return matrix * self.HIGH + (0 if matrix == self.via else 3) * self.STRIDE[matrix]
         if operand == self.tile.stride:
             return self.STRIDE[0]
         if operand == self.tile.steps:
@@ -183,12 +215,20 @@ class Machine:
             elif name.startswith("ds_read"):
                 where, _, offset = ops[1].partition(" offset:")
                 self._read(_registers(ops[0]), where, int(offset))
-            elif name == "global_load_lds_dwordx4":
+            elif name == "ds_write_b128":
+                registers, _, offset = ops[1].partition(" offset:")
+                self._store(_registers(registers), ops[0], int(offset))
+            elif name in ("global_load_lds_dwordx4", "global_load_dwordx4"):
+                target = ops.pop(0) if name == "global_load_dwordx4" else None
                 matrix, chunk = self.tile.copies[ops[0]]
                 low = int(re.fullmatch(r"s\[(\d+):\d+\]", ops[1]).group(1))
                 source = (self.scalar["s%d" % (low + 1)] << 32 | self.scalar["s%d" % low]) - matrix * self.HIGH
                 step, rest = divmod(source, self.STRIDE[matrix])
                 assert rest == 0 and 0 <= step < self.steps, ("copy from outside of the matrix", step)
+                assert target is None or not self.tile.pairs or step % 2 == 0 and step + 1 < self.steps
+                if target is not None:
+                    self._load(matrix, chunk, step, _registers(target))
+                    continue
                 stage, where = divmod(self.scalar["m0"], self.tile.stage)
                 assert where == matrix * self.tile.stage // 2 + chunk * 4096
                 self._copy(matrix, chunk, step, stage)
@@ -218,7 +258,7 @@ class Machine:
             else:
                 assert name == "s_nop", line
         assert self.mfmas == self.steps * 2 * self.tile.blocks ** 2
-        assert not self.memory and not self.lds_reads
+        assert not self.memory and not self.lds_reads and not self.lds_stores
         # the next tile's copies may go anywhere
         assert all(reader == "fenced" for slot in self.slots.values() for reader in slot["readers"])
 
@@ -230,18 +270,23 @@ def _registers(operand):
 
 # loop -> (small tile, from C = 0, vmcnt in front of it, stores that may lie behind the first copies; as in ct_gemm.hip.h)
 LOOPS = {"CT_GEMM_LOOP": (False, False, 16, (0,)), "CT_GEMM_FRESH_LOOP": (False, True, 16, (0,)),
-         "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (51, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 12, (0,))}
+         "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (51, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 12, (0,)),
+         "CT_GEMM_VIA_A_LOOP": (False, True, None, (0, 70)), "CT_GEMM_VIA_B_LOOP": (False, False, None, (0,)),
+         "CT_GEMM_SMALL_VIA_A_LOOP": (True, False, None, (0, 70)), "CT_GEMM_SMALL_VIA_B_LOOP": (True, False, None, (0,))}
+VIA = {"CT_GEMM_VIA_A_LOOP": 0, "CT_GEMM_VIA_B_LOOP": 1, "CT_GEMM_SMALL_VIA_A_LOOP": 0, "CT_GEMM_SMALL_VIA_B_LOOP": 1}
 
 
 def _lines(gen, name):
     return {"CT_GEMM_LOOP": lambda: gen.gemm_loop(), "CT_GEMM_FRESH_LOOP": lambda: gen.gemm_loop(fresh=True),
             "CT_GEMM_FRESH_LOOP_BEHIND_STORES": lambda: gen.gemm_loop(fresh=True, behind_stores=True),
-            "CT_GEMM_SMALL_LOOP": lambda: gen.small_loop()}[name]()
+            "CT_GEMM_SMALL_LOOP": lambda: gen.small_loop(), "CT_GEMM_VIA_A_LOOP": lambda: gen.gemm_loop(fresh=True, via=0),
+            "CT_GEMM_VIA_B_LOOP": lambda: gen.gemm_loop(via=1), "CT_GEMM_SMALL_VIA_A_LOOP": lambda: gen.small_loop(via=0),
+            "CT_GEMM_SMALL_VIA_B_LOOP": lambda: gen.small_loop(via=1)}[name]()
 
 
 def _run(lines, name, steps, stores, start_wait=None):
     small, fresh, wait, _ = LOOPS[name]
-    machine = Machine(Tile(small), steps, fresh, stores, wait if start_wait is None else start_wait)
+    machine = Machine(Tile(small, VIA.get(name)), steps, fresh, stores, wait if start_wait is None else start_wait, VIA.get(name))
     machine.run(lines)
 
 
@@ -278,16 +323,22 @@ def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
         lines = list(good)
         change(lines)
         with pytest.raises(AssertionError):
-            _run(lines, name, 8, stores)
+            _run(lines, name, 12, stores)
 
     # every wait for copies, one copy weaker (63 is the largest there is)
+    loop = next(at for at, line in enumerate(good) if "_loop_" in line)
+    fragments = next(at for at, line in enumerate(good) if line.startswith("ds_read"))
+
+    def binds(at):      # (the first iteration of an operand through registers finds the other's first copies landed)
+        return name not in VIA or not fragments < at < loop or good[at + 1].startswith("ds_write")
+
     for at, line in enumerate(good):
         counted = re.fullmatch(r"s_waitcnt vmcnt\((\d+)\)", line)
-        if counted and 0 < int(counted.group(1)) < 63:
+        if counted and 0 < int(counted.group(1)) < 63 and binds(at):
             broken(lambda lines: lines.__setitem__(at, "s_waitcnt vmcnt(%d)" % (int(counted.group(1)) + 1)))
     # every barrier and every wait for LDS reads in front of the last ones gone
     for at, line in enumerate(good[:-6]):
-        if line in ("s_barrier", "s_waitcnt lgkmcnt(0)"):
+        if line in ("s_barrier", "s_waitcnt lgkmcnt(0)") and binds(at):
             broken(lambda lines: lines.__setitem__(at, "s_nop 0"))
     # a fragment read from the next stage, and a copy to it
     first = next(at for at, line in enumerate(good) if line.startswith("ds_read") and line.endswith("offset:0"))
@@ -297,7 +348,8 @@ def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
     other = (int(offset) + Tile(LOOPS[name][0]).stage) % (4 * Tile(LOOPS[name][0]).stage)
     broken(lambda lines: lines.__setitem__(copy, "s_add_u32 m0, %s, %d" % (operand, other)))
     # a source that moves on past the last step
-    broken(lambda lines: [lines.__setitem__(at, "s_cselect_b32 s46, 64, 64") for at, line in enumerate(good) if "s_cselect_b32 s46" in line])
+    for chosen in dict.fromkeys(line for line in good if line.startswith("s_cselect_b32")):
+        broken(lambda lines: [lines.__setitem__(at, chosen[:-1] + chosen.split(", ")[1]) for at, line in enumerate(good) if line == chosen])
 
 
 def test_committed_include_is_what_the_generator_prints():

@@ -572,6 +572,49 @@ def test_one_aligned_copy_for_both_directions(ct, gpu, rows, width, vocab, layou
         assert torch.equal(gw if layout == "dv" else gw.t(), dw)
 
 
+@pytest.mark.parametrize("rows,width,vocab,both", [
+    (64, 1536, 8209, True),     # small tiles in the projections; the last one is the tail's first half
+    (100, 128, 96001, True),    # large projections, small tiles in the gradients
+    (300, 1024, 12543, True),   # small tiles, the last one the tail's second half; a tail of 255 columns
+    (500, 1024, 16250, True),   # large tiles; a tail of 122 columns, 4-byte aligned rows
+    (1024, 1152, 10890, True),  # the most rows that both directions read in place, a tail of 138 columns
+    (1025, 1152, 10891, False),  # one more: the forward only
+    (1500, 256, 16001, False),  # a tail of 129 columns
+    (513, 768, 32021, True),    # more parts of dHidden than tiles, the last of them the tail's
+])
+@pytest.mark.parametrize("cache,trainable", [(False, True), (True, True), (False, False)])
+def test_head_read_in_place(ct, gpu, rows, width, vocab, both, cache, trainable):
+    """An unaligned head of few rows, which the kernels read in place: the bits that its aligned copy gives, which a
+    transposed head goes through, with and without the logits cache and with hidden rows that are unaligned themselves, and
+    the f32 gradients."""
+
+    shape = ct._lib.CutceShape(rows, width, vocab)
+    assert ct._lib.load().ct_cutce_head_in_place(shape) == both
+    case = _case(rows + vocab, rows, width, vocab)
+    hidden, head, targets, weights = (t.to(gpu) for t in case)
+    outcomes = []
+    shifted = torch.empty(rows * width + 1, dtype=torch.bfloat16, device=gpu)[1:].copy_(hidden.flatten())
+    for layout, source in (("dv", hidden), ("vd", hidden), ("dv", shifted)):
+        x = source.detach().view(1, rows, width).requires_grad_(True)
+        w = (head if layout == "dv" else head.t().contiguous()).requires_grad_(True)
+        nll, _ = ct.pallas_cut_linear_cross_entropy(x, w, targets.view(1, -1), weights.view(1, -1), logits_cache=cache,
+                                                    lm_head_trainable=trainable, head_layout=layout)
+        grads = torch.autograd.grad(nll, (x, w) if trainable else (x,), torch.tensor(0.37, device=gpu))
+        outcomes.append((nll.detach(), grads[0].view(rows, width), *(g if layout == "dv" else g.t() for g in grads[1:])))
+    assert all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(*outcomes))
+    x, w = hidden.float(), head.float()
+    logits = x @ w
+    lse = torch.logsumexp(logits, 1)
+    g = torch.softmax(logits, 1)
+    g[torch.arange(rows), targets.long().clamp(min=0)] -= 1
+    g *= (0.37 * weights)[:, None]
+    assert relative_l2(outcomes[0][1].cpu(), (g @ w.t()).cpu()) <= GRAD_RTOL
+    if trainable:
+        assert relative_l2(outcomes[0][2].cpu(), (x.t() @ g).cpu()) <= GRAD_RTOL
+    picked = logits[torch.arange(rows), targets.long().clamp(min=0)]
+    assert float(outcomes[0][0]) == pytest.approx(float((weights * (lse - picked)).double().sum()), rel=2e-5, abs=2e-3)
+
+
 @pytest.mark.parametrize("rows,cols,ld", [(7, 128, 256), (65, 64, 65), (1031, 200, 1280)])
 def test_transpose16_into_padded_rows(ct, gpu, rows, cols, ld):
     source = torch.randint(-2 ** 15, 2 ** 15, (rows, cols), dtype=torch.int16, device=gpu)
