@@ -536,7 +536,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
   int chunk, rb;
   bool more = next_unit(chunk, rb);
   McLoader<NB> A;
-  KcLoader<NB> B;
+  GemmB<NB, LOADS> B;
   GemmTiles<NB, LOADS, CACHE> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
@@ -793,7 +793,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
   int chunk, rb;
   bool more = units.next(chunk, rb, &unit_s);
   McLoader<NB> A;
-  KcLoader<NB> B;
+  GemmB<NB, LOADS> B;
   GemmTiles<NB, LOADS, true> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
@@ -1009,26 +1009,16 @@ CT_DEVICE void dhidden_unit(const CutceParams& p, const CutceSlab& sl, const Cut
   // (rows of B interleaved: lane j owns the NB consecutive columns c0 + wn + NB j + nb; rows past d
   // are copies of the first, their columns are not stored)
   const bf16* head = p.head.base + (sl.first - p.head.col0);
+  GemmB<NB, LOADS> B;
   if constexpr (LOADS == GemmLoads::kGuarded) {
-    KcLoader<NB> B;
     B.init(head, p.head.ld, nullptr, c0, p.d, k_width, true);
     gemm_tile<LOADS>(A, B, k_begin, with_tail ? k_width : k_mid, smem, acc);
   } else {
     const bf16* tail = p.head.tail + (sl.first - p.head.tail_first);
 #pragma nounroll
     for (int part = 0; part <= (int)with_tail; ++part) {
-      const bf16* from = part ? tail : head;
-      const long ld = part ? p.head.tail_cols : p.head.ld;
-      const int begin = part ? k_mid : k_begin, end = part ? k_mid + 128 : k_mid;
-      if constexpr (LOADS == GemmLoads::kThroughRegisters) {
-        KcPairLoader<NB> B;
-        B.init(from, ld, c0, p.d);
-        gemm_tile(A, B, begin, end, smem, acc);
-      } else {
-        KcLoader<NB> B;
-        B.init(from, ld, nullptr, c0, p.d, k_width, true);
-        gemm_tile<LOADS>(A, B, begin, end, smem, acc);
-      }
+      B.init(part ? tail : head, part ? p.head.tail_cols : p.head.ld, nullptr, c0, p.d, k_width, true);
+      gemm_tile<LOADS>(A, B, part ? k_mid : k_begin, part ? k_mid + 128 : k_mid, smem, acc);
     }
   }
   units.request();
@@ -1119,7 +1109,7 @@ CT_DEVICE void dhead_unit(const CutceParams& p, const CutceSlab& sl, const Cutce
   McLoader<NB> A;  // (columns past d are copies, their rows of dHead are not stored)
   A.init(sl.packed, p.d, m0, p.d, k_end);
   // (rows of B interleaved: lane j owns NB consecutive vocabulary ids)
-  KcLoader<NB> B;
+  GemmB<NB, LOADS> B;
   B.init(sl.G, p.n_pad, nullptr, v0, sl.width, k_end, true);
   GemmAcc<NB> acc;
   acc.clear();

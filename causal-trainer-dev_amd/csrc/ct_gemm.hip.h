@@ -7,8 +7,8 @@
 //
 // An operand comes in one of two memory layouts:
 //   KcLoader  "k-contiguous": matrix rows are the M (or N) index, the
-//             contraction index is contiguous. LDS tile [64 NB][BK], MFMA
-//             fragments read with ds_read_b128.
+//             contraction index is contiguous. LDS tile [64 NB][2 BK], two steps, MFMA
+//             fragments read with ds_read_b128 (KcStepLoader: one step, for the guarded loop).
 //   McLoader  "m-contiguous": matrix rows are the contraction index, the M
 //             (or N) index is contiguous. LDS tile [BK][64 NB], fragments read
 //             with transposed LDS reads.
@@ -27,6 +27,8 @@
 //   guarded    unaligned operands: element-wise guarded loads that zero fill, staged through
 //              registers, 2 LDS stages.
 #pragma once
+
+#include <type_traits>
 
 #include "ct_common.hip.h"
 #include "ct_gemm_asm.inc"
@@ -50,43 +52,42 @@ template <int NB>
 struct GemmShape {
   static constexpr int kTile = 64 * NB, kWave = 32 * NB;
   static constexpr int kTileBytes = kTile * kGemmBK * 2;  // NB = 4: 16 KB
-  static constexpr int kStageBytes = 2 * kTileBytes;      // A tile then B tile
+  static constexpr int kStageBytes = 2 * kTileBytes;      // of the guarded loop: A tile then B tile
   static constexpr int kStages = 4;
+  // of the others: four stages of A, a step each, then two of B, two steps each
+  static constexpr int kB = kStages * kTileBytes, kPairBytes = 2 * kTileBytes;
   static constexpr int kGroups = NB == 4 ? 1 : 2;         // workgroups per compute unit that registers are for
   static constexpr size_t kBytes = (size_t)kStages * kStageBytes;  // NB = 4: 128 KB
 };
 
-// In both loaders thread t owns the 16-byte LDS slots t + 256 n of the tile
-// (n < NB): slot P holds physical chunk P % CPR of row P / CPR, i.e. logical
-// chunk (P % CPR) ^ swizzle(row); voff[n] is the byte offset of that chunk
-// from `base` at k = 0 (32 bits: the host checks sizes and strides against it).
-template <int NB>
-struct KcLoader {
-  static constexpr int CPR = kGemmBK / 8;  // 4
-  static constexpr int NCH = NB;
+// In all loaders thread t owns the 16-byte LDS slots t + 256 n of the tile: slot P holds physical chunk P % CPR of
+// row P / CPR, i.e. logical chunk (P % CPR) ^ swizzle(row); voff[n] is the byte offset of that chunk from `base` at
+// k = 0 (32 bits: the host checks sizes and strides against it).
+template <int NB, int STEPS>
+struct KcRows {
+  static constexpr int CPR = STEPS * kGemmBK / 8;  // 4 a step
+  static constexpr int NCH = NB * STEPS;
+  static constexpr int kRowsPerPass = 256 / CPR;
   const char* base;    // uniform
   unsigned voff[NCH];
-  u32x4 regs[NCH];
-  int chunk, k_valid;
+  int chunk;
 
   // rows m0 .. of `base_` (leading dimension ld elements), optionally
   // gathered through row_index. Rows >= rows_valid are copies of the first row (callers discard
-  // what they get from them); the guarded loop reads k >= k_valid as zero.
+  // what they get from them).
   // With interleave_rows, row 32 nb + j of a wavefront's rows holds matrix row NB j + nb of them:
   // in the accumulator layout lane j of a wavefront then owns NB consecutive matrix rows (its
   // column blocks), which an epilogue can store with one access.
-  CT_DEVICE void init(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid,
-                      int k_valid_, bool interleave_rows = false) {
+  CT_DEVICE void init_rows(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid, bool interleave_rows) {
     const int t = threadIdx.x;
-    k_valid = k_valid_;
     const bool gathered = row_index != nullptr;
     base = reinterpret_cast<const char*>(gathered ? base_ : base_ + (size_t)m0 * ld);
     const int r0 = t / CPR;
-    chunk = (t % CPR) ^ swizzle<CPR>(r0);  // rows r0 + 64 n share the swizzle
+    chunk = (t % CPR) ^ swizzle<CPR>(r0);  // rows r0 + kRowsPerPass n share the swizzle
     int src[NCH];
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      const int tile_row = r0 + 64 * n;
+      const int tile_row = r0 + kRowsPerPass * n;
       constexpr int wave_rows = 32 * NB;
       const int r = interleave_rows ? ((tile_row & wave_rows) | ((tile_row & 31) * NB) | ((tile_row >> 5) % NB)) : tile_row;
       const bool ok = m0 + r < rows_valid;
@@ -99,23 +100,42 @@ struct KcLoader {
 #pragma unroll
     for (int n = 0; n < NCH; ++n) voff[n] = (unsigned)(((long)src[n] * ld + chunk * 8) * 2);
   }
-  // copies N0 .. N1-1 of the thread's NCH 16-byte slots
-  template <int N0 = 0, int N1 = NCH>
+};
+
+template <int NB>
+struct KcLoader : KcRows<NB, 2> {
+  typedef KcRows<NB, 2> Rows;
+  typedef RowFragOffsets<Rows::CPR> FragOffsets;
+  CT_DEVICE void init(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid, int, bool interleave_rows = false) {
+    this->init_rows(base_, ld, row_index, m0, rows_valid, interleave_rows);
+  }
+  // copies of the steps at k0 and behind
   CT_DEVICE void dma(int k0, lds_addr tile) const {
     const int wave = uniform(threadIdx.x >> 6);
-    const char* p = base + (size_t)k0 * 2;
+    const char* p = this->base + (size_t)k0 * 2;
 #pragma unroll
-    for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
+    for (int n = 0; n < Rows::NCH; ++n) dma16_s(p, this->voff[n], tile + (n * 256 + wave * 64) * 16);
+  }
+};
+
+// One step at a time, by loads that read k >= k_valid as zero.
+template <int NB>
+struct KcStepLoader : KcRows<NB, 1> {
+  static constexpr int NCH = NB, CPR = KcRows<NB, 1>::CPR;
+  u32x4 regs[NCH];
+  int k_valid;
+  CT_DEVICE void init(const bf16* base_, long ld, const int* row_index, int m0, int rows_valid,
+                      int k_valid_, bool interleave_rows = false) {
+    k_valid = k_valid_;
+    this->init_rows(base_, ld, row_index, m0, rows_valid, interleave_rows);
   }
   CT_DEVICE void fetch(int k0) {
-    const int k = k0 + chunk * 8;
+    const int k = k0 + this->chunk * 8;
     const int count = min(max(k_valid - k, 0), 8);
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      regs[n] = count ? load_chunk_guarded(reinterpret_cast<const bf16*>(
-                                                       base + (size_t)k0 * 2 + voff[n]),
-                                                   count)
-                              : u32x4{0u, 0u, 0u, 0u};
+      regs[n] = count ? load_chunk_guarded(reinterpret_cast<const bf16*>(this->base + (size_t)k0 * 2 + this->voff[n]), count)
+                      : u32x4{0u, 0u, 0u, 0u};
     }
   }
   CT_DEVICE void commit(lds_addr tile) const {
@@ -127,29 +147,6 @@ struct KcLoader {
   typedef RowFragOffsets<CPR> FragOffsets;
   static CT_DEVICE bf16x8 frag(int tile_off, const FragOffsets& fo, int ks, int wave_first, int i) {
     return fo.load(tile_off + (wave_first / 32) * FragOffsets::kRowBlockBytes, i, ks);
-  }
-};
-
-// The rows of a k-contiguous tile through registers, two steps (128 bytes of a row) at a time: thread t loads 16-byte
-// chunk t % 8 of the rows t / 8 + 32 n of the tile, n < 2 NB, and stores it to the stage of its step. Rows as in KcLoader
-// with interleave_rows, which may start at any multiple of 2 bytes.
-template <int NB>
-struct KcPairLoader {
-  static constexpr int CPR = kGemmBK / 8, NCH = 2 * NB;
-  const char* base;  // uniform
-  unsigned voff[NCH];
-  int lds;  // byte offset of the thread's first chunk from the B tile of an even stage
-
-  CT_DEVICE void init(const bf16* base_, long ld, int m0, int rows_valid) {
-    const int t = threadIdx.x, r0 = t / 8, chunk = t % 8;
-    base = reinterpret_cast<const char*>(base_ + (size_t)m0 * ld);
-    lds = (chunk / CPR) * GemmShape<NB>::kStageBytes + tile_byte_offset<CPR>(r0, chunk % CPR);
-#pragma unroll
-    for (int n = 0; n < NCH; ++n) {
-      const int tile_row = r0 + 32 * n;
-      const int r = (tile_row & (32 * NB)) | ((tile_row & 31) * NB) | ((tile_row >> 5) % NB);
-      voff[n] = (unsigned)(((long)(m0 + r < rows_valid ? r : 0) * ld + chunk * 8) * 2);
-    }
   }
 };
 
@@ -183,13 +180,11 @@ struct McLoader {
       voff[n] = (unsigned)(((long)r * ld + c) * 2);
     }
   }
-  // copies N0 .. N1-1 of the thread's NCH 16-byte slots (N0 even, N1 = N0 + 2 or NCH)
-  template <int N0 = 0, int N1 = NCH>
   CT_DEVICE void dma(int k0, lds_addr tile) const {
     const int wave = uniform(threadIdx.x >> 6);
     const char* p = base + (size_t)k0 * ld * 2;
 #pragma unroll
-    for (int n = N0; n < N1; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
+    for (int n = 0; n < NCH; ++n) dma16_s(p, voff[n], tile + (n * 256 + wave * 64) * 16);
   }
   CT_DEVICE void fetch(int k0) {
     const int r0 = (int)threadIdx.x / CPR;
@@ -213,6 +208,9 @@ struct McLoader {
     return fo.load(tile_off + (wave_first / 128) * 256, ks, i);
   }
 };
+
+template <int NB, GemmLoads LOADS>
+using GemmB = std::conditional_t<LOADS == GemmLoads::kGuarded, KcStepLoader<NB>, KcLoader<NB>>;
 
 template <int NB>
 struct GemmAcc {
@@ -264,11 +262,11 @@ struct GemmFrags {
 };
 
 CT_DEVICE void load_frags(GemmFrags& f, int stage_off, const McLoader<4>::FragOffsets& afo,
-                          const KcLoader<4>::FragOffsets& bfo, int ks, int wm, int wn) {
+                          const KcStepLoader<4>::FragOffsets& bfo, int ks, int wm, int wn) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     f.a[i] = McLoader<4>::frag(stage_off, afo, ks, wm, i);
-    f.b[i] = KcLoader<4>::frag(stage_off + GemmShape<4>::kTileBytes, bfo, ks, wn, i);
+    f.b[i] = KcStepLoader<4>::frag(stage_off + GemmShape<4>::kTileBytes, bfo, ks, wn, i);
   }
 }
 
@@ -286,10 +284,10 @@ CT_DEVICE void wait_vmcnt16() { __builtin_amdgcn_s_waitcnt(0x0F70 | (1 << 14)); 
 CT_DEVICE void workgroup_barrier() { __builtin_amdgcn_s_barrier(); }
 
 // The pipelined main loop with a fixed instruction order (see gen_gemm_asm.py), for an
-// m-contiguous A, a k-contiguous B and a step count that is a positive multiple of 4. Entered with the copies of steps 0..2 issued and step 0 landed for every
-// wavefront; returns with nothing in flight and the LDS tiles free. It adds to the accumulators (kAdd) or writes them
-// (kFresh; kFreshBehindStores: at least kStoresBehindCopies stores of every wavefront follow the copies of step 2, or
-// these have landed).
+// m-contiguous A, a k-contiguous B and a step count that is a positive multiple of 4. Entered with A's copies of steps 0..2
+// and B's of pairs 0 and 1 issued, those of step 0 landed for every wavefront; returns with nothing in flight and the LDS tiles free. It adds to the accumulators (kAdd) or writes them
+// (kFresh; kFreshBehindStores: at least kStoresBehindCopies stores of every wavefront follow these copies, or they
+// have landed).
 enum class GemmStart { kAdd, kFresh, kFreshBehindStores };
 CT_DEVICE unsigned long long uniform64(const void* p) {
   const unsigned long long b = (unsigned long long)(uintptr_t)p;
@@ -298,22 +296,25 @@ CT_DEVICE unsigned long long uniform64(const void* p) {
   return ((unsigned long long)hi << 32) | (unsigned long long)lo;
 }
 // Operands of the loops' asm statements. THROUGH: the operand that comes through registers (A: CT_GEMM_VIA_A_LOOP, from C = 0;
-// B: CT_GEMM_VIA_B_LOOP, adding), entered with the other one's copies of steps 0..2 issued and none of its own loads.
+// B: CT_GEMM_VIA_B_LOOP, adding), entered with the other one's copies issued and none of its own loads.
 enum class Through { kNone, kA, kB };
-template <GemmStart START, Through THROUGH = Through::kNone, class LoaderB = KcLoader<4>>
-CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const LoaderB& B, int k_begin, int steps,
+// Where the source of B's copies starts: at pair 2, or at the last pair.
+CT_DEVICE int first_pair(int k_begin, int steps) { return k_begin + min(4, steps - 2) * kGemmBK; }
+template <GemmStart START, Through THROUGH = Through::kNone>
+CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, int steps,
                                    lds_addr smem, const McLoader<4>::FragOffsets& afo,
                                    const KcLoader<4>::FragOffsets& bfo, int wm, int wn, GemmAcc<4>& acc) {
   const int wave = uniform(threadIdx.x >> 6);
   // sources of the copies of step 3, of the loads of step 0
-  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK), first_b = k_begin + (THROUGH == Through::kB ? 0 : 3 * kGemmBK);
+  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK);
+  const int first_b = THROUGH == Through::kB ? k_begin : first_pair(k_begin, steps);
   const unsigned long long src_a = uniform64(A.base + (size_t)first_a * (size_t)A.ld * 2);
   const unsigned long long src_b = uniform64(B.base + (size_t)first_b * 2);
   const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
   const unsigned steps_u = (unsigned)uniform(steps);
   const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + wave * 1024));
   const int a_off = (wm / 128) * 256;
-  const int b_off = GemmShape<4>::kTileBytes + (wn / 32) * KcLoader<4>::FragOffsets::kRowBlockBytes;
+  const int b_off = GemmShape<4>::kB + (wn / 32) * KcLoader<4>::FragOffsets::kRowBlockBytes;
 #define CT_GEMM_ACC(mode) \
   mode(acc.c[0][0]), mode(acc.c[0][1]), mode(acc.c[0][2]), mode(acc.c[0][3]), mode(acc.c[1][0]), mode(acc.c[1][1]), mode(acc.c[1][2]), mode(acc.c[1][3]), \
       mode(acc.c[2][0]), mode(acc.c[2][1]), mode(acc.c[2][2]), mode(acc.c[2][3]), mode(acc.c[3][0]), mode(acc.c[3][1]), mode(acc.c[3][2]), mode(acc.c[3][3])
@@ -321,20 +322,18 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const LoaderB& B, int k
   "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps_u), "s"(lds_wave), "v"(afo.ptr[0][0] + a_off), \
       "v"(afo.ptr[0][1] + a_off), "v"(afo.ptr[0][2] + a_off), "v"(afo.ptr[0][3] + a_off), "v"(afo.ptr[1][0] + a_off), \
       "v"(afo.ptr[1][1] + a_off), "v"(afo.ptr[1][2] + a_off), "v"(afo.ptr[1][3] + a_off), "v"(bfo.ptr[0] + b_off), \
-      "v"(bfo.ptr[1] + b_off), "v"(A.voff[0]), "v"(A.voff[1]), "v"(A.voff[2]), "v"(A.voff[3]), "v"(B.voff[0]), \
-      "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
+      "v"(bfo.ptr[1] + b_off), "v"(bfo.ptr[2] + b_off), "v"(bfo.ptr[3] + b_off), "v"(A.voff[0]), "v"(A.voff[1]), \
+      "v"(A.voff[2]), "v"(A.voff[3]), "v"(B.voff[0]), "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3]), "v"(B.voff[4]), \
+      "v"(B.voff[5]), "v"(B.voff[6]), "v"(B.voff[7])
   if constexpr (THROUGH != Through::kNone) {
     static_assert((THROUGH == Through::kA) == (START != GemmStart::kAdd), "the forms that there are");
-    if constexpr (THROUGH == Through::kA) {
-      const lds_addr thread = smem + (int)threadIdx.x * 16;
+    const lds_addr thread = smem + (THROUGH == Through::kB ? GemmShape<4>::kB : 0) + (int)threadIdx.x * 16;
+    if constexpr (THROUGH == Through::kA)
       asm volatile(CT_GEMM_VIA_A_LOOP : CT_GEMM_ACC("=&a") : CT_GEMM_IN, "v"(thread)
                    : "memory", "m0", "scc", CT_GEMM_VIA_LOOP_CLOBBERS);
-    } else {
-      const lds_addr thread = smem + B.lds;
-      asm volatile(CT_GEMM_VIA_B_LOOP : CT_GEMM_ACC("+a")
-                   : CT_GEMM_IN, "v"(B.voff[4]), "v"(B.voff[5]), "v"(B.voff[6]), "v"(B.voff[7]), "v"(thread)
+    else
+      asm volatile(CT_GEMM_VIA_B_LOOP : CT_GEMM_ACC("+a") : CT_GEMM_IN, "v"(thread)
                    : "memory", "m0", "scc", CT_GEMM_VIA_LOOP_CLOBBERS);
-    }
   } else if constexpr (START == GemmStart::kAdd)
     asm volatile(CT_GEMM_LOOP : CT_GEMM_ACC("+a") : CT_GEMM_IN : "memory", "m0", "scc", CT_GEMM_LOOP_CLOBBERS);
   else if constexpr (START == GemmStart::kFresh)
@@ -346,33 +345,35 @@ CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const LoaderB& B, int k
 #undef CT_GEMM_IN
 }
 
-// The copies of an operand's first three steps (four in the small tile).
-template <class Loader>
-CT_DEVICE void copy_first_steps(const Loader& loader, int k_begin, lds_addr tile) {
-  constexpr int kNb = Loader::NCH;
+// The copies that a loop is entered with: A's of steps STEP .. END - 1, B's of a pair.
+template <int STEP, int END, int NB>
+CT_DEVICE void copy_steps(const McLoader<NB>& A, int k_begin, lds_addr smem) {
 #pragma unroll
-  for (int i = 0; i < (kNb == 4 ? 3 : 4); ++i) loader.dma(k_begin + i * kGemmBK, tile + i * GemmShape<kNb>::kStageBytes);
+  for (int i = STEP; i < END; ++i) A.dma(k_begin + i * kGemmBK, smem + i * GemmShape<NB>::kTileBytes);
 }
-
-// The copies of a tile's first three steps, ahead of gemm_tile_fresh (nothing may be using the LDS stages).
-CT_DEVICE void gemm_copy_ahead(const McLoader<4>& A, const KcLoader<4>& B, lds_addr smem) {
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    A.dma(i * kGemmBK, smem + i * GemmShape<4>::kStageBytes);
-    B.dma(i * kGemmBK, smem + i * GemmShape<4>::kStageBytes + GemmShape<4>::kTileBytes);
-  }
+template <int NB>
+CT_DEVICE void copy_pair(const KcLoader<NB>& B, int pair, int k_begin, lds_addr smem) {
+  B.dma(k_begin + pair * 2 * kGemmBK, smem + GemmShape<NB>::kB + pair * GemmShape<NB>::kPairBytes);
+}
+// Those of step 0 first, then the rest: `behind step 0` many.
+constexpr int kCopiesBehindStep0 = 4 + 4 + 8;
+CT_DEVICE void gemm_copy_ahead(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, lds_addr smem) {
+  copy_steps<0, 1>(A, k_begin, smem);
+  copy_pair(B, 0, k_begin, smem);
+  copy_steps<1, 3>(A, k_begin, smem);
+  copy_pair(B, 1, k_begin, smem);
 }
 
 // acc = A[m-tile, 0:k_end] * B[n-tile, 0:k_end]^T behind gemm_copy_ahead, k_end a positive multiple of 128. STORES:
 // every wavefront has issued at least kStoresBehindCopies stores since, or it waits for all of the copies (`landed`).
-constexpr int kStoresBehindCopies = 51;  // what the waits of CT_GEMM_FRESH_LOOP_BEHIND_STORES need (gen_gemm_asm.py)
+constexpr int kStoresBehindCopies = 55;  // what the waits of CT_GEMM_FRESH_LOOP_BEHIND_STORES need (gen_gemm_asm.py)
 template <bool STORES>
 CT_DEVICE void gemm_tile_fresh(const McLoader<4>& A, const KcLoader<4>& B, int k_end, lds_addr smem, GemmAcc<4>& acc, bool landed) {
   constexpr GemmStart kStart = STORES ? GemmStart::kFreshBehindStores : GemmStart::kFresh;
   const int w = threadIdx.x >> 6;
   const McLoader<4>::FragOffsets afo(smem);
   const KcLoader<4>::FragOffsets bfo(smem);
-  // step 0's copies: at least 16 + 51 others behind them, or the 16 of steps 1 and 2
+  // step 0's copies: at least 16 + 55 others behind them, or the 16 of the other steps
   if (!STORES) wait_vmcnt16();
   else if (landed) dma_wait_all();
   else asm volatile("s_waitcnt vmcnt(63)" ::: "memory");
@@ -380,7 +381,7 @@ CT_DEVICE void gemm_tile_fresh(const McLoader<4>& A, const KcLoader<4>& B, int k
   gemm_loop_scheduled<kStart>(A, B, 0, k_end / kGemmBK, smem, afo, bfo, (w >> 1) * 128, (w & 1) * 128, acc);
 }
 
-// acc = the same product with A through registers, behind copy_first_steps of B.
+// acc = the same product with A through registers, behind B's two pairs of copies.
 CT_DEVICE void gemm_tile_through_a(const McLoader<4>& A, const KcLoader<4>& B, int k_end, lds_addr smem, GemmAcc<4>& acc) {
   const int w = threadIdx.x >> 6;
   const McLoader<4>::FragOffsets afo(smem);
@@ -389,27 +390,29 @@ CT_DEVICE void gemm_tile_through_a(const McLoader<4>& A, const KcLoader<4>& B, i
 }
 
 // acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T (k_end - k_begin a multiple of 128
-// unless kGuarded). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
+// unless kGuarded; kThroughRegisters: B comes through them). Must be called by all 256 threads; ends with the LDS tiles free for reuse.
 template <GemmLoads LOADS>
-CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
-  constexpr int BK = kGemmBK, kTile = GemmShape<4>::kTileBytes, kStage = GemmShape<4>::kStageBytes;
+CT_DEVICE void gemm_tile(McLoader<4>& A, GemmB<4, LOADS>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
   const int w = threadIdx.x >> 6;
   const int wm = (w >> 1) * 128, wn = (w & 1) * 128;
   if (k_begin >= k_end) return;
   const McLoader<4>::FragOffsets afo(smem);
-  const KcLoader<4>::FragOffsets bfo(smem);
-  if constexpr (LOADS == GemmLoads::kCopies) {
+  const typename GemmB<4, LOADS>::FragOffsets bfo(smem);
+  if constexpr (LOADS != GemmLoads::kGuarded) {
+    const int steps = (k_end - k_begin) / kGemmBK;
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      A.dma(k_begin + i * BK, smem + i * kStage);
-      B.dma(k_begin + i * BK, smem + i * kStage + kTile);
+    if constexpr (LOADS == GemmLoads::kCopies) {
+      gemm_copy_ahead(A, B, k_begin, smem);
+      static_assert(kCopiesBehindStep0 == 16, "the wait leaves the copies behind step 0's in flight");
+      wait_vmcnt16();
+      workgroup_barrier();
+      gemm_loop_scheduled<GemmStart::kAdd>(A, B, k_begin, steps, smem, afo, bfo, wm, wn, acc);
+    } else {
+      copy_steps<0, 3>(A, k_begin, smem);
+      gemm_loop_scheduled<GemmStart::kAdd, Through::kB>(A, B, k_begin, steps, smem, afo, bfo, wm, wn, acc);
     }
-    static_assert(McLoader<4>::NCH + KcLoader<4>::NCH == 8, "the wait leaves the copies of two steps in flight");
-    wait_vmcnt16();
-    workgroup_barrier();
-    gemm_loop_scheduled<GemmStart::kAdd>(A, B, k_begin, (k_end - k_begin) / BK, smem, afo, bfo, wm, wn, acc);
   } else {
+    constexpr int BK = kGemmBK, kTile = GemmShape<4>::kTileBytes, kStage = GemmShape<4>::kStageBytes;
     A.fetch(k_begin);
     B.fetch(k_begin);
     A.commit(smem);
@@ -441,25 +444,12 @@ CT_DEVICE void gemm_tile(McLoader<4>& A, KcLoader<4>& B, int k_begin, int k_end,
   }
 }
 
-// The same with B through registers.
-CT_DEVICE void gemm_tile(McLoader<4>& A, KcPairLoader<4>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<4>& acc) {
-  if (k_begin >= k_end) return;
-  const int w = threadIdx.x >> 6;
-  const McLoader<4>::FragOffsets afo(smem);
-  const KcLoader<4>::FragOffsets bfo(smem);
-  dma_wait_all();
-  copy_first_steps(A, k_begin, smem);
-  gemm_loop_scheduled<GemmStart::kAdd, Through::kB>(A, B, k_begin, (k_end - k_begin) / kGemmBK, smem, afo, bfo, (w >> 1) * 128,
-                                                    (w & 1) * 128, acc);
-}
-
 // The small tile (NB = 2: 128 x 128, 64 accumulator registers, two workgroups per compute unit), with a fixed order of its
 // own (gen_gemm_asm.py).
+// This lane's part of the wavefront's fragments of A, stage 0.
 struct SmallFrags {
-  lds_addr a[2][2];  // this lane's part of the wavefront's fragments, stage 0
-  RowFragOffsets<KcLoader<2>::CPR> b;
-  CT_DEVICE explicit SmallFrags(lds_addr smem)
-      : b(smem + GemmShape<2>::kTileBytes + (uniform(threadIdx.x >> 6) & 1) * 2 * RowFragOffsets<KcLoader<2>::CPR>::kRowBlockBytes) {
+  lds_addr a[2][2];
+  CT_DEVICE explicit SmallFrags(lds_addr smem) {
     const int wm = (uniform(threadIdx.x >> 6) >> 1) * GemmShape<2>::kWave, l = lane_id();
 #pragma unroll
     for (int second = 0; second < 2; ++second)
@@ -470,13 +460,17 @@ struct SmallFrags {
       }
   }
 };
+// The row block of B that a wavefront starts at.
+CT_DEVICE int small_first_block() { return (uniform(threadIdx.x >> 6) & 1) * 2; }
 
-// acc += the product, entered with the first four steps' copies issued (step 0's landed, for every wavefront), of an
-// operand through registers none.
-template <Through THROUGH, class LoaderB>
-CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const LoaderB& B, int k_begin, int k_end, lds_addr smem, const SmallFrags& f,
-                               GemmAcc<2>& acc) {
-  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK), first_b = k_begin + (THROUGH == Through::kB ? 0 : 3 * kGemmBK);
+// acc += the product, entered with A's copies of the first four steps and B's of two pairs issued (those of step 0
+// landed for every wavefront, this one's of A's step 1 too), of an operand through registers none.
+template <Through THROUGH>
+CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
+  const SmallFrags f(smem);
+  const KcLoader<2>::FragOffsets b(smem + GemmShape<2>::kB + small_first_block() * KcLoader<2>::FragOffsets::kRowBlockBytes);
+  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK);
+  const int first_b = THROUGH == Through::kB ? k_begin : first_pair(k_begin, (k_end - k_begin) / kGemmBK);
   const unsigned long long src_a = uniform64(A.base + (size_t)first_a * (size_t)A.ld * 2);
   const unsigned long long src_b = uniform64(B.base + (size_t)first_b * 2);
   const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
@@ -485,44 +479,53 @@ CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const LoaderB& B, int k_beg
 #define CT_GEMM_SMALL_ACC "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[1][0]), "+a"(acc.c[1][1])
 #define CT_GEMM_SMALL_IN \
   "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps), "s"(lds_wave), "v"(f.a[0][0]), "v"(f.a[0][1]), "v"(f.a[1][0]), \
-      "v"(f.a[1][1]), "v"(f.b.ptr[0]), "v"(f.b.ptr[1]), "v"(A.voff[0]), "v"(A.voff[1]), "v"(B.voff[0]), "v"(B.voff[1])
+      "v"(f.a[1][1]), "v"(b.ptr[0]), "v"(b.ptr[1]), "v"(b.ptr[2]), "v"(b.ptr[3]), "v"(A.voff[0]), "v"(A.voff[1]), \
+      "v"(B.voff[0]), "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
   if constexpr (THROUGH == Through::kNone) {
     asm volatile(CT_GEMM_SMALL_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN
                  : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
-  } else if constexpr (THROUGH == Through::kA) {
-    const lds_addr thread = smem + (int)threadIdx.x * 16;
-    asm volatile(CT_GEMM_SMALL_VIA_A_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
-                 : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
   } else {
-    const lds_addr thread = smem + B.lds;
-    asm volatile(CT_GEMM_SMALL_VIA_B_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(B.voff[2]), "v"(B.voff[3]), "v"(thread)
-                 : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
+    const lds_addr thread = smem + (THROUGH == Through::kB ? GemmShape<2>::kB : 0) + (int)threadIdx.x * 16;
+    if constexpr (THROUGH == Through::kA)
+      asm volatile(CT_GEMM_SMALL_VIA_A_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
+                   : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
+    else
+      asm volatile(CT_GEMM_SMALL_VIA_B_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
+                   : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
   }
 #undef CT_GEMM_SMALL_ACC
 #undef CT_GEMM_SMALL_IN
 }
 
-// acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T in the small tile; kThroughRegisters: A comes through them.
-template <GemmLoads LOADS>
-CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
-  constexpr int kTile = GemmShape<2>::kTileBytes;
+// acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T in the small tile; THROUGH: the operand of kThroughRegisters.
+template <GemmLoads LOADS, Through THROUGH = Through::kB>
+CT_DEVICE void gemm_tile(McLoader<2>& A, GemmB<2, LOADS>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
   if (k_begin >= k_end) return;
-  const SmallFrags frags(smem);
-  static_assert(McLoader<2>::NCH + KcLoader<2>::NCH == 4, "the waits count the copies of a step");
   if constexpr (LOADS == GemmLoads::kCopies) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      A.dma(k_begin + i * kGemmBK, smem + i * GemmShape<2>::kStageBytes);
-      B.dma(k_begin + i * kGemmBK, smem + i * GemmShape<2>::kStageBytes + kTile);
-    }
-    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // step 0 has landed
-    gemm_small_loop<Through::kNone>(A, B, k_begin, k_end, smem, frags, acc);
+    copy_steps<0, 1>(A, k_begin, smem);
+    copy_pair(B, 0, k_begin, smem);
+    copy_steps<1, 2>(A, k_begin, smem);
+    copy_pair(B, 1, k_begin, smem);
+    copy_steps<2, 4>(A, k_begin, smem);
+    // step 0 and A's step 1 have landed
+    static_assert(2 * McLoader<2>::NCH + KcLoader<2>::NCH == 8, "the wait leaves A's steps 2 and 3 and a pair in flight");
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    gemm_small_loop<Through::kNone>(A, B, k_begin, k_end, smem, acc);
   } else if constexpr (LOADS == GemmLoads::kThroughRegisters) {
     dma_wait_all();
-    copy_first_steps(B, k_begin, smem + kTile);
-    gemm_small_loop<Through::kA>(A, B, k_begin, k_end, smem, frags, acc);
+    if constexpr (THROUGH == Through::kA) {
+      copy_pair(B, 0, k_begin, smem);
+      copy_pair(B, 1, k_begin, smem);
+    } else {
+      copy_steps<0, 4>(A, k_begin, smem);
+    }
+    gemm_small_loop<THROUGH>(A, B, k_begin, k_end, smem, acc);
   } else {
+    constexpr int kTile = GemmShape<2>::kTileBytes;
+    typedef KcStepLoader<2>::FragOffsets StepOffsets;
+    const SmallFrags frags(smem);
+    const StepOffsets b_ptr(smem + kTile + small_first_block() * StepOffsets::kRowBlockBytes);
 #pragma nounroll
     for (int k0 = k_begin; k0 < k_end; k0 += kGemmBK) {
       A.fetch(k0);
@@ -538,7 +541,7 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
           const int off = ks * (16 * McLoader<2>::CPR * 16);
           const bf16x4_vs lo = lds_load_tr(frags.a[0][i] + off), hi = lds_load_tr(frags.a[1][i] + off);
           a[i] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          b[i] = frags.b.load(0, i, ks);
+          b[i] = b_ptr.load(0, i, ks);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -549,14 +552,6 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, KcLoader<2>& B, int k_begin, int k_end,
     }
     acc.settle();
   }
-}
-
-// The same with B through registers.
-CT_DEVICE void gemm_tile(McLoader<2>& A, KcPairLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
-  if (k_begin >= k_end) return;
-  dma_wait_all();
-  copy_first_steps(A, k_begin, smem);
-  gemm_small_loop<Through::kB>(A, B, k_begin, k_end, smem, SmallFrags(smem), acc);
 }
 
 // The rows of a wavefront's tile in the order of its accumulators (0..3, 8..11, ...; lanes of the other half
@@ -580,11 +575,16 @@ struct TileRows {
 // kThroughRegisters (A): only B's copies travel ahead.
 template <int NB, GemmLoads LOADS, bool STORES>
 struct GemmTiles {
+  typedef GemmB<NB, LOADS> LoaderB;
   static constexpr bool kAhead = NB == 4 && LOADS == GemmLoads::kCopies;
   int stores = 0;  // of this wavefront behind the copies of begin()
-  CT_DEVICE void begin(const McLoader<NB>& A, const KcLoader<NB>& B, lds_addr smem) {
-    if constexpr (kAhead) gemm_copy_ahead(A, B, smem);
-    else if constexpr (NB == 4 && LOADS == GemmLoads::kThroughRegisters) copy_first_steps(B, 0, smem + GemmShape<4>::kTileBytes);
+  CT_DEVICE void begin(const McLoader<NB>& A, const LoaderB& B, lds_addr smem) {
+    if constexpr (kAhead) {
+      gemm_copy_ahead(A, B, 0, smem);
+    } else if constexpr (NB == 4 && LOADS == GemmLoads::kThroughRegisters) {
+      copy_pair(B, 0, 0, smem);
+      copy_pair(B, 1, 0, smem);
+    }
   }
   // a lane's NB consecutive elements of accumulator row r of a block (wave-uniform control flow only)
   template <class Elements>
@@ -594,7 +594,7 @@ struct GemmTiles {
     rows.advance(r);
     if constexpr (kAhead) ++stores;
   }
-  CT_DEVICE void run(McLoader<NB>& A, KcLoader<NB>& B, int k_end, lds_addr smem, GemmAcc<NB>& acc) {
+  CT_DEVICE void run(McLoader<NB>& A, LoaderB& B, int k_end, lds_addr smem, GemmAcc<NB>& acc) {
     if constexpr (kAhead) {
       gemm_tile_fresh<STORES>(A, B, k_end, smem, acc, stores < kStoresBehindCopies);
       stores = 0;
@@ -602,7 +602,8 @@ struct GemmTiles {
       gemm_tile_through_a(A, B, k_end, smem, acc);
     } else {
       acc.clear();
-      gemm_tile<LOADS>(A, B, 0, k_end, smem, acc);
+      if constexpr (NB == 2) gemm_tile<LOADS, Through::kA>(A, B, 0, k_end, smem, acc);
+      else gemm_tile<LOADS>(A, B, 0, k_end, smem, acc);
     }
   }
 };

@@ -30,32 +30,41 @@ def gen():
 
 
 class Tile:
-    """What the operands of a loop's asm statement stand for, and the layout of its LDS stages."""
+    """What the operands of a loop's asm statement stand for, and the layout of its LDS stages: four of A, a step each, then
+    two of B, a pair of steps each."""
 
-    def __init__(self, small, via=None):
+    def __init__(self, small):
         self.blocks = 2 if small else 4                     # of a wavefront, in each direction
-        self.chunks = self.blocks                           # copies of a wavefront per operand and step
-        self.ahead = 4 if small else 3                      # steps copied in front of the loop
-        self.stage = 16384 if small else 32768
+        self.chunks = (self.blocks, 2 * self.blocks)        # copies of a wavefront per stage
+        # stages copied in front of the loop
+        self.ahead = ((0, 0), (1, 0), (0, 1), (1, 1), (0, 2), (0, 3)) if small else ((0, 0), (1, 0), (0, 1), (0, 2), (1, 1))
+        self.a_stage = 8192 if small else 16384
+        self.b_at, self.b_stage = 4 * self.a_stage, 2 * self.a_stage
         first = self.blocks ** 2                            # (the accumulators are operands 0 ..)
         self.src = {"%%%d" % first: 0, "%%%d" % (first + 1): 1}
         self.stride, self.steps, self.lds_wave = ("%%%d" % (first + k) for k in (2, 3, 4))
-        self.reads, self.copies = {}, {}                    # operand -> (matrix, second, block or k-step), (matrix, chunk)
+        self.reads, self.copies = {}, {}                    # operand -> (matrix, second, block or k-step of a pair), (matrix, chunk)
         at = first + 5
         for second in range(2):
             for block in range(self.blocks):
                 self.reads["%%%d" % at] = (0, second, block)
                 at += 1
-        for ks in range(2):
+        for ks in range(4):
             self.reads["%%%d" % at] = (1, None, ks)
             at += 1
-        self.pairs = via == 1                               # B through registers, two steps at a time
-        self.per_operand = (self.chunks, self.chunks * (2 if self.pairs else 1))
         for matrix in range(2):
-            for chunk in range(self.per_operand[matrix]):
+            for chunk in range(self.chunks[matrix]):
                 self.copies["%%%d" % at] = (matrix, chunk)
                 at += 1
         self.thread = "%%%d" % at
+
+    def place(self, offset):
+        """(matrix, stage, chunk) of 4 KB of LDS"""
+        matrix = int(offset >= self.b_at)
+        stage, rest = divmod(offset - matrix * self.b_at, self.b_stage if matrix else self.a_stage)
+        chunk, rest = divmod(rest, 4096)
+        assert rest == 0 and stage < (2 if matrix else 4)
+        return matrix, stage, chunk
 
 
 class Machine:
@@ -64,18 +73,19 @@ class Machine:
 
     # bytes from step to step of the two sources (the first carries into the upper half of the address), and between them
     STRIDE, HIGH = ((1 << 32) - 4096, 64), 1 << 40
+    # (a slot's step: A's, or the first of B's pair)
 
     def __init__(self, tile, steps, fresh, stores, start_wait, via=None):
         self.tile, self.steps, self.fresh, self.via = tile, steps, fresh, via
-        self.scalar, self.scc, self.address, self.fragment = {}, 0, {}, {}
+        self.scalar, self.scc, self.fragment = {}, 0, {}
         self.loaded, self.lds_stores = {}, []               # first register -> what a load puts there; on their way to LDS
         self.memory, self.lds_reads = [], []                # in flight, in the order of their issue
         self.slots, self.mfmas, self.started = {}, 0, set()
-        for step in range(tile.ahead):
-            for matrix in range(2):
-                for chunk in range(tile.chunks):
-                    if matrix != via:
-                        self._copy(matrix, chunk, step, step)
+        # (in the order of ct_gemm.hip.h)
+        for matrix, stage in tile.ahead:
+            for chunk in range(tile.chunks[matrix]):
+                if matrix != via:
+                    self._copy(matrix, chunk, stage * (1 + matrix), stage)
         self.memory += [None] * stores
         if start_wait is not None:
             self._wait_memory(start_wait)
@@ -98,14 +108,12 @@ class Machine:
         self.memory.append(held)
 
     def _store(self, registers, where, offset):
-        base, extra = self.address.get(where, (where, 0))
-        assert base == self.tile.thread
-        stage, rest = divmod(offset + extra, self.tile.stage)
+        assert where == self.tile.thread
         held = self.loaded[registers[0]]
         assert held["state"] == "landed", ("store of a chunk that has not landed", held)
-        assert rest == held["matrix"] * self.tile.stage // 2 + held["chunk"] * (2048 if self.tile.pairs else 4096)
-        for second in range(2 if self.tile.pairs else 1):   # (half of the lanes have the next step's chunk)
-            self._copy(held["matrix"], held["chunk"], held["step"] + second, stage + second, self.lds_stores)
+        matrix, stage, chunk = self.tile.place(offset + self.via * self.tile.b_at)
+        assert (matrix, chunk) == (held["matrix"], held["chunk"])
+        self._copy(matrix, chunk, held["step"], stage, self.lds_stores)
 
     def _wait_memory(self, most):
         assert most <= 63
@@ -132,18 +140,18 @@ class Machine:
             slot["readers"] = ["fenced" if reader in ("done", "fenced") else reader for reader in slot["readers"]]
 
     def _read(self, registers, operand, offset):
-        base, extra = self.address.get(operand, (operand, 0))
-        matrix, second, which = self.tile.reads[base]
-        stage, offset = divmod(offset + extra, self.tile.stage)
-        half = self.tile.stage // 4                         # of one operand's tile
+        matrix, second, which = self.tile.reads[operand]
         if matrix == 0:                                     # rows of the contraction: half of the tile per k-step
-            ks, rest = divmod(offset, half)
-            assert rest == 0, operand
-            block, chunks = which, range(ks * self.tile.chunks // 2, (ks + 1) * self.tile.chunks // 2)
+            stage, rest = divmod(offset, self.tile.a_stage)
+            ks, rest = divmod(rest, self.tile.a_stage // 2)
+            half = self.tile.chunks[0] // 2
+            block, parity, chunks = which, 0, range(ks * half, (ks + 1) * half)
         else:
-            ks, (block, rest) = which, divmod(offset, 2048)
-            assert rest == 0 and block < self.tile.blocks, operand
-            chunks = range(self.tile.per_operand[1])        # (half of them, by the wavefront)
+            stage, rest = divmod(offset, self.tile.b_stage)
+            block, rest = divmod(rest, 4096)
+            parity, ks = divmod(which, 2)
+            chunks = range(self.tile.chunks[1])             # (half of them, by the wavefront)
+        assert rest == 0 and block < self.tile.blocks, operand
         slots = []
         for chunk in chunks:
             assert (stage, matrix, chunk) in self.slots, ("LDS read of a place that nothing was copied to", stage, matrix, chunk)
@@ -155,6 +163,7 @@ class Machine:
                        for first, held in self.loaded.items() for register in registers)
         step = slots[0][0]["step"]
         assert all(slot["step"] == step for slot, _ in slots)
+        step += parity
         for k, register in enumerate(registers):
             assert self.fragment.get(register, [None, True])[1], ("register of a read in flight", register)
             self.fragment[register] = [(matrix, step, ks, block, second if matrix == 0 else k // 2), False]
@@ -180,7 +189,8 @@ class Machine:
     def _get(self, operand):
         if operand in self.tile.src:                        # address of the copies of step 3
             matrix = self.tile.src[operand]
-            return matrix * self.HIGH + (0 if matrix == self.via else 3) * self.STRIDE[matrix]
+            step = 0 if matrix == self.via else min(4, self.steps - 2) if matrix else 3
+            return matrix * self.HIGH + step * self.STRIDE[matrix]
         if operand == self.tile.stride:
             return self.STRIDE[0]
         if operand == self.tile.steps:
@@ -225,17 +235,15 @@ class Machine:
                 source = (self.scalar["s%d" % (low + 1)] << 32 | self.scalar["s%d" % low]) - matrix * self.HIGH
                 step, rest = divmod(source, self.STRIDE[matrix])
                 assert rest == 0 and 0 <= step < self.steps, ("copy from outside of the matrix", step)
-                assert target is None or not self.tile.pairs or step % 2 == 0 and step + 1 < self.steps
+                assert matrix == 0 or step % 2 == 0, ("half of a pair", step)
                 if target is not None:
                     self._load(matrix, chunk, step, _registers(target))
                     continue
-                stage, where = divmod(self.scalar["m0"], self.tile.stage)
-                assert where == matrix * self.tile.stage // 2 + chunk * 4096
-                self._copy(matrix, chunk, step, stage)
+                place = self.tile.place(self.scalar["m0"])
+                assert (place[0], place[2]) == (matrix, chunk)
+                self._copy(matrix, chunk, step, place[1])
             elif name == "v_mfma_f32_32x32x16_bf16":
                 self._mfma(*ops)
-            elif name == "v_add_u32":
-                self.address[ops[0]] = (ops[2], int(ops[1], 0))
             elif name == "s_mov_b64":
                 low, high = re.fullmatch(r"s\[(\d+):(\d+)\]", ops[0]).groups()
                 value = self._get(ops[1])
@@ -270,7 +278,7 @@ def _registers(operand):
 
 # loop -> (small tile, from C = 0, vmcnt in front of it, stores that may lie behind the first copies; as in ct_gemm.hip.h)
 LOOPS = {"CT_GEMM_LOOP": (False, False, 16, (0,)), "CT_GEMM_FRESH_LOOP": (False, True, 16, (0,)),
-         "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (51, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 12, (0,)),
+         "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (55, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 8, (0,)),
          "CT_GEMM_VIA_A_LOOP": (False, True, None, (0, 70)), "CT_GEMM_VIA_B_LOOP": (False, False, None, (0,)),
          "CT_GEMM_SMALL_VIA_A_LOOP": (True, False, None, (0, 70)), "CT_GEMM_SMALL_VIA_B_LOOP": (True, False, None, (0,))}
 VIA = {"CT_GEMM_VIA_A_LOOP": 0, "CT_GEMM_VIA_B_LOOP": 1, "CT_GEMM_SMALL_VIA_A_LOOP": 0, "CT_GEMM_SMALL_VIA_B_LOOP": 1}
@@ -286,7 +294,7 @@ def _lines(gen, name):
 
 def _run(lines, name, steps, stores, start_wait=None):
     small, fresh, wait, _ = LOOPS[name]
-    machine = Machine(Tile(small, VIA.get(name)), steps, fresh, stores, wait if start_wait is None else start_wait, VIA.get(name))
+    machine = Machine(Tile(small), steps, fresh, stores, wait if start_wait is None else start_wait, VIA.get(name))
     machine.run(lines)
 
 
@@ -301,7 +309,7 @@ def test_waits_and_fragments(gen, name):
 def test_copies_that_have_landed_need_no_stores(gen):
     """A kernel's first tile, and one behind an epilogue with too few stores, wait for all copies in front of the loop."""
 
-    for stores in (0, 7, 50):
+    for stores in (0, 7, 54):
         _run(_lines(gen, "CT_GEMM_FRESH_LOOP_BEHIND_STORES"), "CT_GEMM_FRESH_LOOP_BEHIND_STORES", 8, stores, start_wait=0)
 
 
@@ -341,11 +349,12 @@ def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
         if line in ("s_barrier", "s_waitcnt lgkmcnt(0)") and binds(at):
             broken(lambda lines: lines.__setitem__(at, "s_nop 0"))
     # a fragment read from the next stage, and a copy to it
+    tile = Tile(LOOPS[name][0])
     first = next(at for at, line in enumerate(good) if line.startswith("ds_read") and line.endswith("offset:0"))
-    broken(lambda lines: lines.__setitem__(first, good[first].replace("offset:0", "offset:%d" % Tile(LOOPS[name][0]).stage)))
+    broken(lambda lines: lines.__setitem__(first, good[first].replace("offset:0", "offset:%d" % tile.a_stage)))
     copy = next(at for at, line in enumerate(good) if line.startswith("s_add_u32 m0"))
     operand, offset = re.fullmatch(r"s_add_u32 m0, (\S+), (\d+)", good[copy]).groups()
-    other = (int(offset) + Tile(LOOPS[name][0]).stage) % (4 * Tile(LOOPS[name][0]).stage)
+    other = (int(offset) + tile.a_stage) % tile.b_at if int(offset) < tile.b_at else (int(offset) - tile.b_at) ^ tile.b_stage
     broken(lambda lines: lines.__setitem__(copy, "s_add_u32 m0, %s, %d" % (operand, other)))
     # a source that moves on past the last step
     for chosen in dict.fromkeys(line for line in good if line.startswith("s_cselect_b32")):
