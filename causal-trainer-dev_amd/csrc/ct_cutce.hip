@@ -511,8 +511,8 @@ CT_DEVICE void head_tile(McLoader<NB>& A, const CutceParams& p, int v0) {
 // latency, the cleared accumulators and a second reading of them in the epilogue took 116 us to 104 there, 67 to 65
 // at 900 x 32003, d = 1024, 175 to 162 at 1845 x 67203, d = 512. (Small tiles on two workgroups per compute unit, whose epilogues could
 // fall behind each other's products: 152, 81 and 196, bound by the bytes that reach LDS.)
-template <int NB, bool CACHE, GemmLoads LOADS>
-__global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
+template <int NB, bool CACHE, GemmLoads LOADS, int RING = 4>
+__global__ __launch_bounds__(256, (GemmShape<NB, RING>::kGroups)) void cutce_stats_kernel(CutceParams p, float* part, int chunk0, int chunks,
                                                                     int tiles_per_chunk, float* cache) {
   constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
   extern __shared__ __align__(16) char smem_raw[];
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_stats_kerne
   bool more = next_unit(chunk, rb);
   McLoader<NB> A;
   GemmB<NB, LOADS> B;
-  GemmTiles<NB, LOADS, CACHE> gemm;
+  GemmTiles<NB, LOADS, CACHE, RING> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots.
   typedef int LaneInts __attribute__((ext_vector_type(NB)));
@@ -771,8 +771,8 @@ CT_DEVICE float dlogit(float logit, float fac, float lse2, int tgt, int v) {
 // G^T[v - slab0][slot], logits recomputed (transposed tile as in the statistics kernel: rows =
 // vocabulary, lanes = row slots). Persistent like the statistics kernel and with its unit order:
 // a unit is tiles_per_chunk vocabulary tiles of the slab times one block of 256 active rows.
-template <int NB, GemmLoads LOADS>
-__global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
+template <int NB, GemmLoads LOADS, int RING = 4>
+__global__ __launch_bounds__(256, (GemmShape<NB, RING>::kGroups)) void cutce_dlogits_kernel(CutceParams p, CutceRowParams rp,
                                                                       int slab0, int slab_tiles, int tiles_per_chunk,
                                                                       bf16* G) {
   constexpr int kTile = GemmShape<NB>::kTile, kWave = GemmShape<NB>::kWave;
@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256, GemmShape<NB>::kGroups) void cutce_dlogits_ker
   bool more = units.next(chunk, rb, &unit_s);
   McLoader<NB> A;
   GemmB<NB, LOADS> B;
-  GemmTiles<NB, LOADS, true> gemm;
+  GemmTiles<NB, LOADS, true, RING> gemm;
   // Rows are interleaved in the tile (KcLoader): column block nb of lane j is row slot
   // n0 + wn + NB j + nb, so a lane owns NB consecutive slots of G^T and stores them together.
   LaneFloats next_fac, next_lse2;
@@ -1625,39 +1625,54 @@ static Kernel by_loads(GemmLoads loads, Kernel copies, Kernel through, Kernel gu
   return loads == kCopies ? copies : loads == kThrough ? through : guarded;
 }
 
-template <int NB>
+// Launches of no more small tiles than compute units: a workgroup has its compute unit to itself, its copies are its own
+// latency, and with twice the LDS they are on their way for six steps instead of two. Statistics kernel, four / eight stages,
+// us: 588 x 1248, d = 6400 (50 tiles) 48.5 / 42.0; 1393 x 704, d = 5504 (66) 43.9 / 36.8; 385 x 3120, d = 7296 (100)
+// 56.3 / 49.3; 69 x 5667, d = 1536 (45) 20.4 / 17.4; a contraction that is over in a few steps pays for the longer
+// start: 64 x 600, d = 256 7.9 / 8.6.
+static bool alone(int units, int hidden, GemmLoads loads) { return units <= device_cu_count() && hidden >= 768 && loads != kGuarded; }
+
+template <int NB, int RING = 4>
 static int launch_stats(const char* fn, hipStream_t stream, const CutceParams& p, GemmLoads loads, float* part, int chunk0,
                         int chunks, int tiles_per_chunk, float* cache) {
+  const int units = chunks * ((p.N + 64 * NB - 1) / (64 * NB));
+  if constexpr (NB == 2 && RING == 4)
+    if (alone(units, p.d, loads)) return launch_stats<2, 8>(fn, stream, p, loads, part, chunk0, chunks, tiles_per_chunk, cache);
+  constexpr GemmLoads kAny = RING == 4 ? kGuarded : kCopies;
   static std::atomic<unsigned> lds_allowed{0};
-  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<NB, false, kCopies>, cutce_stats_kernel<NB, true, kCopies>,
-                                cutce_stats_kernel<NB, false, kThrough>, cutce_stats_kernel<NB, true, kThrough>,
-                                cutce_stats_kernel<NB, false, kGuarded>, cutce_stats_kernel<NB, true, kGuarded>);
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_stats_kernel<NB, false, kCopies, RING>, cutce_stats_kernel<NB, true, kCopies, RING>,
+                                cutce_stats_kernel<NB, false, kThrough, RING>, cutce_stats_kernel<NB, true, kThrough, RING>,
+                                cutce_stats_kernel<NB, false, kAny, RING>, cutce_stats_kernel<NB, true, kAny, RING>);
   if (rc) return rc;
-  const auto kernel = cache ? by_loads(loads, cutce_stats_kernel<NB, true, kCopies>, cutce_stats_kernel<NB, true, kThrough>,
-                                       cutce_stats_kernel<NB, true, kGuarded>)
-                            : by_loads(loads, cutce_stats_kernel<NB, false, kCopies>, cutce_stats_kernel<NB, false, kThrough>,
-                                       cutce_stats_kernel<NB, false, kGuarded>);
-  const int slots = device_cu_count() * GemmShape<NB>::kGroups, units = chunks * ((p.N + 64 * NB - 1) / (64 * NB));
+  const auto kernel = cache ? by_loads(loads, cutce_stats_kernel<NB, true, kCopies, RING>, cutce_stats_kernel<NB, true, kThrough, RING>,
+                                       cutce_stats_kernel<NB, true, kAny, RING>)
+                            : by_loads(loads, cutce_stats_kernel<NB, false, kCopies, RING>, cutce_stats_kernel<NB, false, kThrough, RING>,
+                                       cutce_stats_kernel<NB, false, kAny, RING>);
+  typedef GemmShape<NB, RING> Shape;
   LaunchScope scope("cutce_stats_kernel", stream);
-  hipLaunchKernelGGL(kernel, dim3(min(slots, units)), dim3(256), GemmShape<NB>::kBytes, stream, p, part, chunk0, chunks,
-                     tiles_per_chunk, cache);
+  hipLaunchKernelGGL(kernel, dim3(min(device_cu_count() * Shape::kGroups, units)), dim3(256), Shape::kBytes, stream, p, part, chunk0,
+                     chunks, tiles_per_chunk, cache);
   return scope.done();
 }
 
 // slab_tiles: of the kernel's tile size
-template <int NB>
+template <int NB, int RING = 4>
 static int launch_dlogits(const char* fn, hipStream_t stream, const CutceParams& p, const CutceRowParams& rp, GemmLoads loads,
                           int slab0, int slab_tiles, int tiles_per_chunk, bf16* G) {
-  static std::atomic<unsigned> lds_allowed{0};
-  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_dlogits_kernel<NB, kCopies>, cutce_dlogits_kernel<NB, kThrough>,
-                                cutce_dlogits_kernel<NB, kGuarded>);
-  if (rc) return rc;
-  const int slots = device_cu_count() * GemmShape<NB>::kGroups;
   const int units = (slab_tiles + tiles_per_chunk - 1) / tiles_per_chunk * ((p.N + 64 * NB - 1) / (64 * NB));
+  if constexpr (NB == 2 && RING == 4)
+    if (alone(units, p.d, loads)) return launch_dlogits<2, 8>(fn, stream, p, rp, loads, slab0, slab_tiles, tiles_per_chunk, G);
+  constexpr GemmLoads kAny = RING == 4 ? kGuarded : kCopies;
+  static std::atomic<unsigned> lds_allowed{0};
+  const int rc = allow_gemm_lds(fn, lds_allowed, cutce_dlogits_kernel<NB, kCopies, RING>, cutce_dlogits_kernel<NB, kThrough, RING>,
+                                cutce_dlogits_kernel<NB, kAny, RING>);
+  if (rc) return rc;
+  typedef GemmShape<NB, RING> Shape;
   LaunchScope scope("cutce_dlogits_kernel", stream);
-  hipLaunchKernelGGL(by_loads(loads, cutce_dlogits_kernel<NB, kCopies>, cutce_dlogits_kernel<NB, kThrough>,
-                              cutce_dlogits_kernel<NB, kGuarded>), dim3(min(slots, units)),
-                     dim3(256), GemmShape<NB>::kBytes, stream, p, rp, slab0, slab_tiles, tiles_per_chunk, G);
+  hipLaunchKernelGGL(by_loads(loads, cutce_dlogits_kernel<NB, kCopies, RING>, cutce_dlogits_kernel<NB, kThrough, RING>,
+                              cutce_dlogits_kernel<NB, kAny, RING>),
+                     dim3(min(device_cu_count() * Shape::kGroups, units)), dim3(256), Shape::kBytes, stream, p, rp, slab0, slab_tiles,
+                     tiles_per_chunk, G);
   return scope.done();
 }
 
@@ -1762,7 +1777,7 @@ static int32_t cutce_fwd_on(void* stream_, const ct_cutce_fwd_args* a, void* ws_
     }
     const int list_blocks = chunk0 == 0 ? (p.N + 1023) / 1024 : 0;
     if ((rc = launch_prepare<false>(stream, p, CutceRowWork{}, copy, list_blocks, list_blocks == 0))) return rc;
-    const auto launch = units.tile == kGemmTile ? launch_stats<4> : launch_stats<2>;
+    const auto launch = units.tile == kGemmTile ? launch_stats<4, 4> : launch_stats<2, 4>;
     if ((rc = launch(fn, stream, p, loads, part, chunk0, pass_chunks, units.per_chunk, static_cast<float*>(a->logits_cache))))
       return rc;
   }

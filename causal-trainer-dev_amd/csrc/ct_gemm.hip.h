@@ -47,16 +47,17 @@ CT_DEVICE u32x4 load_chunk_guarded(const bf16* p, int count) {
   return as_u32x4(v);
 }
 
-// A workgroup's tile: 4 wavefronts of NB x NB accumulator blocks.
-template <int NB>
+// A workgroup's tile: 4 wavefronts of NB x NB accumulator blocks. RING: stages of A (8: the small tile for launches of
+// no more workgroups than compute units, whose copies nothing but their own number hides).
+template <int NB, int RING = 4>
 struct GemmShape {
   static constexpr int kTile = 64 * NB, kWave = 32 * NB;
   static constexpr int kTileBytes = kTile * kGemmBK * 2;  // NB = 4: 16 KB
   static constexpr int kStageBytes = 2 * kTileBytes;      // of the guarded loop: A tile then B tile
-  static constexpr int kStages = 4;
-  // of the others: four stages of A, a step each, then two of B, two steps each
+  static constexpr int kStages = RING;
+  // of the others: RING stages of A, a step each, then half as many of B, two steps each
   static constexpr int kB = kStages * kTileBytes, kPairBytes = 2 * kTileBytes;
-  static constexpr int kGroups = NB == 4 ? 1 : 2;         // workgroups per compute unit that registers are for
+  static constexpr int kGroups = NB == 4 || RING == 8 ? 1 : 2;         // workgroups per compute unit that registers are for
   static constexpr size_t kBytes = (size_t)kStages * kStageBytes;  // NB = 4: 128 KB
 };
 
@@ -298,8 +299,9 @@ CT_DEVICE unsigned long long uniform64(const void* p) {
 // Operands of the loops' asm statements. THROUGH: the operand that comes through registers (A: CT_GEMM_VIA_A_LOOP, from C = 0;
 // B: CT_GEMM_VIA_B_LOOP, adding), entered with the other one's copies issued and none of its own loads.
 enum class Through { kNone, kA, kB };
-// Where the source of B's copies starts: at pair 2, or at the last pair.
-CT_DEVICE int first_pair(int k_begin, int steps) { return k_begin + min(4, steps - 2) * kGemmBK; }
+// Where the source of B's copies starts: at the pair behind those that a loop is entered with, or at the last pair.
+template <int RING = 4>
+CT_DEVICE int first_pair(int k_begin, int steps) { return k_begin + min(RING, steps - 2) * kGemmBK; }
 template <GemmStart START, Through THROUGH = Through::kNone>
 CT_DEVICE void gemm_loop_scheduled(const McLoader<4>& A, const KcLoader<4>& B, int k_begin, int steps,
                                    lds_addr smem, const McLoader<4>::FragOffsets& afo,
@@ -351,9 +353,13 @@ CT_DEVICE void copy_steps(const McLoader<NB>& A, int k_begin, lds_addr smem) {
 #pragma unroll
   for (int i = STEP; i < END; ++i) A.dma(k_begin + i * kGemmBK, smem + i * GemmShape<NB>::kTileBytes);
 }
+template <int RING, int NB>
+CT_DEVICE void copy_pair_at(const KcLoader<NB>& B, int stage, int k0, lds_addr smem) {
+  B.dma(k0, smem + GemmShape<NB, RING>::kB + stage * GemmShape<NB, RING>::kPairBytes);
+}
 template <int NB>
 CT_DEVICE void copy_pair(const KcLoader<NB>& B, int pair, int k_begin, lds_addr smem) {
-  B.dma(k_begin + pair * 2 * kGemmBK, smem + GemmShape<NB>::kB + pair * GemmShape<NB>::kPairBytes);
+  copy_pair_at<4>(B, pair, k_begin + pair * 2 * kGemmBK, smem);
 }
 // Those of step 0 first, then the rest: `behind step 0` many.
 constexpr int kCopiesBehindStep0 = 4 + 4 + 8;
@@ -465,28 +471,36 @@ CT_DEVICE int small_first_block() { return (uniform(threadIdx.x >> 6) & 1) * 2; 
 
 // acc += the product, entered with A's copies of the first four steps and B's of two pairs issued (those of step 0
 // landed for every wavefront, this one's of A's step 1 too), of an operand through registers none.
-template <Through THROUGH>
+template <Through THROUGH, int RING = 4>
 CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const KcLoader<2>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
   const SmallFrags f(smem);
-  const KcLoader<2>::FragOffsets b(smem + GemmShape<2>::kB + small_first_block() * KcLoader<2>::FragOffsets::kRowBlockBytes);
-  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : 3 * kGemmBK);
-  const int first_b = THROUGH == Through::kB ? k_begin : first_pair(k_begin, (k_end - k_begin) / kGemmBK);
+  constexpr int kB = GemmShape<2, RING>::kB;
+  const int loop_steps = (k_end - k_begin) / kGemmBK;
+  const KcLoader<2>::FragOffsets b(smem + kB + small_first_block() * KcLoader<2>::FragOffsets::kRowBlockBytes);
+  const int first_a = k_begin + (THROUGH == Through::kA ? 0 : (RING == 4 ? 3 : min(RING, loop_steps) - 1) * kGemmBK);
+  const int first_b = THROUGH == Through::kB ? k_begin : first_pair<RING>(k_begin, loop_steps);
   const unsigned long long src_a = uniform64(A.base + (size_t)first_a * (size_t)A.ld * 2);
   const unsigned long long src_b = uniform64(B.base + (size_t)first_b * 2);
   const unsigned stride_a = (unsigned)uniform((int)(kGemmBK * A.ld * 2));
-  const unsigned steps = (unsigned)uniform((k_end - k_begin) / kGemmBK);
+  const unsigned steps = (unsigned)uniform(loop_steps);
   const unsigned lds_wave = (unsigned)uniform((int)(uintptr_t)(smem + uniform(threadIdx.x >> 6) * 1024));
 #define CT_GEMM_SMALL_ACC "+a"(acc.c[0][0]), "+a"(acc.c[0][1]), "+a"(acc.c[1][0]), "+a"(acc.c[1][1])
 #define CT_GEMM_SMALL_IN \
   "s"(src_a), "s"(src_b), "s"(stride_a), "s"(steps), "s"(lds_wave), "v"(f.a[0][0]), "v"(f.a[0][1]), "v"(f.a[1][0]), \
       "v"(f.a[1][1]), "v"(b.ptr[0]), "v"(b.ptr[1]), "v"(b.ptr[2]), "v"(b.ptr[3]), "v"(A.voff[0]), "v"(A.voff[1]), \
       "v"(B.voff[0]), "v"(B.voff[1]), "v"(B.voff[2]), "v"(B.voff[3])
-  if constexpr (THROUGH == Through::kNone) {
+  if constexpr (THROUGH == Through::kNone && RING == 8) {
+    asm volatile(CT_GEMM_SMALL_DEEP_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN
+                 : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
+  } else if constexpr (THROUGH == Through::kNone) {
     asm volatile(CT_GEMM_SMALL_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN
                  : "memory", "m0", "scc", CT_GEMM_SMALL_LOOP_CLOBBERS);
   } else {
-    const lds_addr thread = smem + (THROUGH == Through::kB ? GemmShape<2>::kB : 0) + (int)threadIdx.x * 16;
-    if constexpr (THROUGH == Through::kA)
+    const lds_addr thread = smem + (THROUGH == Through::kB ? kB : 0) + (int)threadIdx.x * 16;
+    if constexpr (RING == 8)
+      asm volatile(CT_GEMM_SMALL_DEEP_VIA_A_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
+                   : "memory", "m0", "scc", CT_GEMM_SMALL_DEEP_VIA_LOOP_CLOBBERS);
+    else if constexpr (THROUGH == Through::kA)
       asm volatile(CT_GEMM_SMALL_VIA_A_LOOP : CT_GEMM_SMALL_ACC : CT_GEMM_SMALL_IN, "v"(thread)
                    : "memory", "m0", "scc", CT_GEMM_SMALL_VIA_LOOP_CLOBBERS);
     else
@@ -498,10 +512,22 @@ CT_DEVICE void gemm_small_loop(const McLoader<2>& A, const KcLoader<2>& B, int k
 }
 
 // acc += A[m-tile, k_begin:k_end] * B[n-tile, k_begin:k_end]^T in the small tile; THROUGH: the operand of kThroughRegisters.
-template <GemmLoads LOADS, Through THROUGH = Through::kB>
+template <GemmLoads LOADS, Through THROUGH = Through::kB, int RING = 4>
 CT_DEVICE void gemm_tile(McLoader<2>& A, GemmB<2, LOADS>& B, int k_begin, int k_end, lds_addr smem, GemmAcc<2>& acc) {
   if (k_begin >= k_end) return;
-  if constexpr (LOADS == GemmLoads::kCopies) {
+  if constexpr (LOADS == GemmLoads::kCopies && RING == 8) {
+    // (past the end the last step and pair again: nobody reads them)
+    const int last = k_end - kGemmBK, last_pair = k_end - 2 * kGemmBK;
+    dma_wait_all();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (i % 2) copy_pair_at<8>(B, i / 2, min(k_begin + (i - 1) * kGemmBK, last_pair), smem);
+      A.dma(min(k_begin + i * kGemmBK, last), smem + i * GemmShape<2>::kTileBytes);
+    }
+    // (32 copies, the 6 of step 0 first)
+    asm volatile("s_waitcnt vmcnt(26)\n\ts_barrier" ::: "memory");
+    gemm_small_loop<Through::kNone, 8>(A, B, k_begin, k_end, smem, acc);
+  } else if constexpr (LOADS == GemmLoads::kCopies) {
     dma_wait_all();  // nothing of ours may still be in flight when counting copies below
     copy_steps<0, 1>(A, k_begin, smem);
     copy_pair(B, 0, k_begin, smem);
@@ -515,12 +541,13 @@ CT_DEVICE void gemm_tile(McLoader<2>& A, GemmB<2, LOADS>& B, int k_begin, int k_
   } else if constexpr (LOADS == GemmLoads::kThroughRegisters) {
     dma_wait_all();
     if constexpr (THROUGH == Through::kA) {
-      copy_pair(B, 0, k_begin, smem);
-      copy_pair(B, 1, k_begin, smem);
+#pragma unroll
+      for (int pair = 0; pair < RING / 2; ++pair)
+        copy_pair_at<RING>(B, pair, min(k_begin + pair * 2 * kGemmBK, k_end - 2 * kGemmBK), smem);
     } else {
       copy_steps<0, 4>(A, k_begin, smem);
     }
-    gemm_small_loop<THROUGH>(A, B, k_begin, k_end, smem, acc);
+    gemm_small_loop<THROUGH, RING>(A, B, k_begin, k_end, smem, acc);
   } else {
     constexpr int kTile = GemmShape<2>::kTileBytes;
     typedef KcStepLoader<2>::FragOffsets StepOffsets;
@@ -573,7 +600,7 @@ struct TileRows {
 // stores counted since begin() (a constant wherever an epilogue issues them on every path): where they are too
 // few for the counted waits, as on a kernel's first tile, it waits for all copies.
 // kThroughRegisters (A): only B's copies travel ahead.
-template <int NB, GemmLoads LOADS, bool STORES>
+template <int NB, GemmLoads LOADS, bool STORES, int RING = 4>
 struct GemmTiles {
   typedef GemmB<NB, LOADS> LoaderB;
   static constexpr bool kAhead = NB == 4 && LOADS == GemmLoads::kCopies;
@@ -602,7 +629,7 @@ struct GemmTiles {
       gemm_tile_through_a(A, B, k_end, smem, acc);
     } else {
       acc.clear();
-      if constexpr (NB == 2) gemm_tile<LOADS, Through::kA>(A, B, 0, k_end, smem, acc);
+      if constexpr (NB == 2) gemm_tile<LOADS, Through::kA, RING>(A, B, 0, k_end, smem, acc);
       else gemm_tile<LOADS>(A, B, 0, k_end, smem, acc);
     }
   }

@@ -182,7 +182,7 @@ def gemm_loop(fresh=False, behind_stores=False, via=None):
 
 
 # ---------------------------------------------------------------------------
-# The 128 x 128 tile (2 x 2 blocks per wavefront; four stages of A of 8 KB, two of B of 16 KB)
+# The 128 x 128 tile (2 x 2 blocks per wavefront; four stages of A of 8 KB, two of B of 16 KB; or eight and four)
 # ---------------------------------------------------------------------------
 # 8 MFMAs a step are too few to read a step's second half of fragments behind its first, so all fragments
 # of step k + 1 are read, into the other of two register sets, behind the MFMAs of step k:
@@ -194,15 +194,19 @@ def gemm_loop(fresh=False, behind_stores=False, via=None):
 #     reads of step k+1's fragments behind MFMA 1..6, in an odd step copies of the pair of steps k+3 and k+4 behind MFMA 1 to
 #       4, then those of A's step k+4 -> stage s behind MFMA 5, 7
 #
+# With eight stages of A and four of B (RING = 8, for a workgroup that has its compute unit to itself) the copies of A's
+# step k+8 and in odd steps of the pair of steps k+7 and k+8 take their places: six steps on their way instead of
+# two. A body of eight steps, with an end in the middle.
+#
 # An operand through registers (`via`): a chunk of step k+2, loaded in step k-2, goes to LDS behind MFMA 1 or 3, the load
 # of step k+4 into its registers follows. It is there in front of the next step's barrier, behind which step k+2's
 # fragments are read (an odd step's barrier has let it land already). Of B an even step k stores the chunks of the pair
-# k+2, k+3 and loads those of k+4, k+5. 16 registers.
+# k+2, k+3 and loads those of k+4, k+5. 16 registers; with eight stages 32, the load is that of step k+6.
 #
 # Fixed registers (clobbers): v[64:95], v[96:127] the two sets, s[40:41] / s[42:43], s44, s45-s46 as above. With an
 # operand through registers v[48:79], v[80:111], v[112:127] the loads': the compiler gives a kernel of two workgroups
 # 128 vector registers and 128 accumulation registers, and one more of the first would be one workgroup less.
-SMALL_A_STAGE, SMALL_B_AT, SMALL_B_STAGE = 8192, 32768, 16384
+SMALL_A_STAGE, SMALL_B_STAGE = 8192, 16384
 SMALL_SETS = {None: (64, 96), 0: (48, 80), 1: (48, 80)}
 SMALL_VIA = 112
 SMALL_ACC = lambda i, j: "%%%d" % (2 * i + j)
@@ -234,8 +238,8 @@ def small_voff(operand, n):
     return SMALL_IN["v%s%d" % ("ab"[operand], n)]
 
 
-def small_copy(operand, n, stage):
-    dst = (SMALL_B_AT + stage * SMALL_B_STAGE if operand else stage * SMALL_A_STAGE) + n * 4096
+def small_copy(operand, n, stage, ring):
+    dst = (ring * SMALL_A_STAGE + stage * SMALL_B_STAGE if operand else stage * SMALL_A_STAGE) + n * 4096
     return ["s_add_u32 m0, %s, %d" % (SMALL_IN["lds_wave"], dst), "s_nop 0",
             "global_load_lds_dwordx4 %s, %s" % (small_voff(operand, n), SRC[operand])]
 
@@ -253,37 +257,39 @@ def small_names(lines):
     return [line.replace(STRIDE_A, SMALL_IN["stride_a"]).replace(STEPS, SMALL_IN["steps"]) for line in lines]
 
 
-def small_step(u, via=None, behind_chunk=7):
-    stage, odd, current, other = u, u & 1, SMALL_SETS[via][u & 1], SMALL_SETS[via][(u + 1) & 1]
-    reads = small_reads((u + 1) & 3, other)
+def small_step(u, via=None, ring=4, behind_chunk=None):
+    odd, current, other = u & 1, SMALL_SETS[via][u & 1], SMALL_SETS[via][(u + 1) & 1]
+    reads = small_reads((u + 1) % ring, other)
     behind = {m: [] for m in range(8)}
-    # (sources: A's of step k + 4, in a step of B's copies that of the pair that begins with step k + 3 or k + 4)
-    pair = odd if via != 1 else not odd
-    behind[0] = (ADVANCE_A if via == 1 else []) + (ADVANCE_B if via == 1 and pair else [])
-    if via != 1:
-        behind[0] += ADVANCE_A
-    behind[0] = small_names(behind[0] + NEXT_STEP)
-    landed = 8 if via == 1 else (4, 2)[via == 0] if odd else 8 if via is None else None
+    # Sources: A's of step k + ring (k + 6 through registers with eight stages); B's of the pair that begins with step
+    # k + 4 through registers, else, behind its copies, with step k + ring + 1.
+    if via == 0 and ring == 8:
+        behind[0] = ["s_sub_u32 s45, s44, 2", "s_cmp_lt_u32 s45, " + STEPS] + ADVANCE_A[1:]
+    else:
+        behind[0] = list(ADVANCE_A)
+    behind[0] = small_names(behind[0] + (ADVANCE_B if via == 1 and not odd else []) + NEXT_STEP)
+    landed = {(None, 4): (8, 4), (None, 8): (24, 20), (0, 4): (None, 2), (0, 8): (None, None), (1, 4): (8, 8)}[via, ring][odd]
     if landed is not None:
         behind[0].append("s_waitcnt vmcnt(%d)" % landed)
     behind[0].append("s_barrier")
     for m in range(1, 7):
         behind[m] += reads[2 * m - 2:2 * m]
+    if behind_chunk is None:
+        behind_chunk = 15 if ring == 8 else 7
     chunk_wait = ["s_waitcnt vmcnt(%d)" % behind_chunk]
     if via == 1:
-        for n in range(4 if pair else 0):
+        for n in range(0 if odd else 4):
             behind[1 + n] += chunk_wait + [small_to_lds(1, n, SMALL_VIA, ((u + 2) & 3) >> 1), small_load(1, n, SMALL_VIA)]
         for n, m in enumerate((5, 7)):
-            behind[m] += small_copy(0, n, stage)
+            behind[m] += small_copy(0, n, u, ring)
     else:
-        through = SMALL_VIA + 8 * odd
+        through = SMALL_VIA + 8 * ((u + 2) % (ring // 2))
         for n, m in enumerate((5, 7) if via is None else (1, 3)):
-            behind[m] += small_copy(0, n, stage) if via is None else ([] if odd else chunk_wait) + [
-                small_to_lds(0, n, through, (u + 2) & 3), small_load(0, n, through)]
-        for n in range(4 if pair else 0):
-            behind[(1 if via is None else 4) + n] += small_copy(1, n, stage >> 1)
-        # (the pair behind the next one: s44 is k + 5)
-        behind[7] += small_names(ADVANCE_B) if pair else []
+            behind[m] += small_copy(0, n, u, ring) if via is None else ([] if odd and ring == 4 else chunk_wait) + [
+                small_to_lds(0, n, through, (u + 2) % ring), small_load(0, n, through)]
+        for n in range(4 if odd else 0):
+            behind[(1 if via is None else 4) + n] += small_copy(1, n, u >> 1, ring)
+        behind[7] += small_names(ADVANCE_B) if odd else []
     lines = ["s_waitcnt lgkmcnt(0)"]
     for m in range(8):
         ks, i, j = m >> 2, (m >> 1) & 1, m & 1
@@ -294,34 +300,43 @@ def small_step(u, via=None, behind_chunk=7):
     return lines
 
 
-def small_loop(via=None):
-    lines = ["s_mov_b64 s[40:41], " + SMALL_IN["src_a"], "s_mov_b64 s[42:43], " + SMALL_IN["src_b"], "s_mov_b32 s44, 4"]
+def small_loop(via=None, ring=4):
+    lines = ["s_mov_b64 s[40:41], " + SMALL_IN["src_a"], "s_mov_b64 s[42:43], " + SMALL_IN["src_b"], "s_mov_b32 s44, %d" % ring]
     if via is not None:     # (the source of an operand through registers is that of step 0)
         first = SMALL_SETS[via][1]
         if via == 0:
-            for k, registers in enumerate((first, first + 8, SMALL_VIA, SMALL_VIA + 8)):
-                lines += ["s_add_u32 s40, s40, " + SMALL_IN["stride_a"], "s_addc_u32 s41, s41, 0"] if k else []
+            # steps 0 and 1, then as many as there are sets (steps 4 and 5 only if there are any)
+            for k, registers in enumerate([first, first + 8] + [SMALL_VIA + 8 * ((k + 2) % (ring // 2)) for k in range(ring // 2)]):
+                if k > 3:
+                    lines += ["s_cmp_gt_u32 %s, 4" % SMALL_IN["steps"]] + small_names(ADVANCE_A[1:])
+                elif k:
+                    lines += ["s_add_u32 s40, s40, " + SMALL_IN["stride_a"], "s_addc_u32 s41, s41, 0"]
                 lines += [small_load(0, n, registers) for n in range(2)]
         else:
             lines += [small_load(1, n, first) for n in range(4)] + ["s_add_u32 s42, s42, 128", "s_addc_u32 s43, s43, 0"]
             lines += [small_load(1, n, SMALL_VIA) for n in range(4)]
         # steps 0 and 1 and all copies have landed
-        lines.append("s_waitcnt vmcnt(4)")
+        lines.append("s_waitcnt vmcnt(%d)" % ring)
         lines += [small_to_lds(1, n, first, 0) for n in range(4)] if via else [
             small_to_lds(0, n, first + 8 * k, k) for k in range(2) for n in range(2)]
         lines += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
     lines += small_reads(0, SMALL_SETS[via][0])
-    # (s44 has advanced by 4: the steps done are s44 - 4; the last one read fragments that nobody uses)
-    more = ["s_sub_u32 s45, s44, 4", "s_cmp_lt_u32 s45, " + SMALL_IN["steps"]]
+    # (s44 has advanced with the steps; the last one read fragments that nobody uses)
+    more = ["s_sub_u32 s45, s44, %d" % ring, "s_cmp_lt_u32 s45, " + SMALL_IN["steps"]]
+    done = more + ["s_cbranch_scc0 ct_gemm_small_done_%="]
+
+    def body(first_iteration=False):
+        out = []
+        for u in range(ring):
+            behind_chunk = {4: {0: 3}, 8: {0: 7, 1: 7, 2: 11, 3: 11}}[ring].get(u) if first_iteration else None
+            out += small_step(u, via, ring, behind_chunk) + (done if u == 3 and ring == 8 else [])
+        return out
+
     if via is not None:
-        for u in range(4):
-            lines += small_step(u, via, 3 if u == 0 else 7)
-        lines += more + ["s_cbranch_scc0 ct_gemm_small_done_%="]
+        lines += body(True) + done
     lines.append("ct_gemm_small_loop_%=:")
-    for u in range(4):
-        lines += small_step(u, via)
-    lines += more + ["s_cbranch_scc1 ct_gemm_small_loop_%="]
-    if via is not None:
+    lines += body() + more + ["s_cbranch_scc1 ct_gemm_small_loop_%="]
+    if via is not None or ring == 8:
         lines.append("ct_gemm_small_done_%=:")
     lines += ["s_waitcnt vmcnt(0)", "s_waitcnt lgkmcnt(0)", "s_barrier", "s_nop 15", "s_nop 7"]
     return lines
@@ -351,3 +366,6 @@ if __name__ == "__main__":
     print(emit(small_loop(via=0), "CT_GEMM_SMALL_VIA_A_LOOP"))
     print(emit(small_loop(via=1), "CT_GEMM_SMALL_VIA_B_LOOP"))
     print("#define CT_GEMM_SMALL_VIA_LOOP_CLOBBERS %s" % clobbers(SMALL_SETS[0][0], SMALL_VIA + 16))
+    print(emit(small_loop(ring=8), "CT_GEMM_SMALL_DEEP_LOOP"))
+    print(emit(small_loop(via=0, ring=8), "CT_GEMM_SMALL_DEEP_VIA_A_LOOP"))
+    print("#define CT_GEMM_SMALL_DEEP_VIA_LOOP_CLOBBERS %s" % clobbers(SMALL_SETS[0][0], SMALL_VIA + 32))

@@ -30,16 +30,18 @@ def gen():
 
 
 class Tile:
-    """What the operands of a loop's asm statement stand for, and the layout of its LDS stages: four of A, a step each, then
-    two of B, a pair of steps each."""
+    """What the operands of a loop's asm statement stand for, and the layout of its LDS stages: `ring` (four, or eight in
+    the small tile) of A, a step each, then half as many of B, a pair of steps each."""
 
-    def __init__(self, small):
+    def __init__(self, small, ring=4):
         self.blocks = 2 if small else 4                     # of a wavefront, in each direction
         self.chunks = (self.blocks, 2 * self.blocks)        # copies of a wavefront per stage
         # stages copied in front of the loop
         self.ahead = ((0, 0), (1, 0), (0, 1), (1, 1), (0, 2), (0, 3)) if small else ((0, 0), (1, 0), (0, 1), (0, 2), (1, 1))
-        self.a_stage = 8192 if small else 16384
-        self.b_at, self.b_stage = 4 * self.a_stage, 2 * self.a_stage
+        if ring == 8:
+            self.ahead = ((0, 0), (1, 0), (0, 1), (0, 2), (1, 1), (0, 3), (0, 4), (1, 2), (0, 5), (0, 6), (1, 3), (0, 7))
+        self.ring, self.a_stage = ring, 8192 if small else 16384
+        self.b_at, self.b_stage = ring * self.a_stage, 2 * self.a_stage
         first = self.blocks ** 2                            # (the accumulators are operands 0 ..)
         self.src = {"%%%d" % first: 0, "%%%d" % (first + 1): 1}
         self.stride, self.steps, self.lds_wave = ("%%%d" % (first + k) for k in (2, 3, 4))
@@ -63,7 +65,7 @@ class Tile:
         matrix = int(offset >= self.b_at)
         stage, rest = divmod(offset - matrix * self.b_at, self.b_stage if matrix else self.a_stage)
         chunk, rest = divmod(rest, 4096)
-        assert rest == 0 and stage < (2 if matrix else 4)
+        assert rest == 0 and stage < (self.ring // 2 if matrix else self.ring)
         return matrix, stage, chunk
 
 
@@ -84,7 +86,7 @@ class Machine:
         # (in the order of ct_gemm.hip.h)
         for matrix, stage in tile.ahead:
             for chunk in range(tile.chunks[matrix]):
-                if matrix != via:
+                if matrix != via:                           # (past the end the last step's again, which nobody reads)
                     self._copy(matrix, chunk, stage * (1 + matrix), stage)
         self.memory += [None] * stores
         if start_wait is not None:
@@ -189,7 +191,8 @@ class Machine:
     def _get(self, operand):
         if operand in self.tile.src:                        # address of the copies of step 3
             matrix = self.tile.src[operand]
-            step = 0 if matrix == self.via else min(4, self.steps - 2) if matrix else 3
+            ring = self.tile.ring
+            step = 0 if matrix == self.via else min(ring, self.steps - 2) if matrix else min(ring, self.steps) - 1
             return matrix * self.HIGH + step * self.STRIDE[matrix]
         if operand == self.tile.stride:
             return self.STRIDE[0]
@@ -258,6 +261,8 @@ class Machine:
                 self.scalar[ops[0]], self.scc = value & 0xffffffff, int(value < 0)
             elif name == "s_cmp_lt_u32":
                 self.scc = int(self._get(ops[0]) < self._get(ops[1]))
+            elif name == "s_cmp_gt_u32":
+                self.scc = int(self._get(ops[0]) > self._get(ops[1]))
             elif name == "s_cselect_b32":
                 self.scalar[ops[0]] = self._get(ops[1] if self.scc else ops[2])
             elif name in ("s_cbranch_scc0", "s_cbranch_scc1"):
@@ -281,7 +286,9 @@ LOOPS = {"CT_GEMM_LOOP": (False, False, 16, (0,)), "CT_GEMM_FRESH_LOOP": (False,
          "CT_GEMM_FRESH_LOOP_BEHIND_STORES": (False, True, 63, (55, 64, 300)), "CT_GEMM_SMALL_LOOP": (True, False, 8, (0,)),
          "CT_GEMM_VIA_A_LOOP": (False, True, None, (0, 70)), "CT_GEMM_VIA_B_LOOP": (False, False, None, (0,)),
          "CT_GEMM_SMALL_VIA_A_LOOP": (True, False, None, (0, 70)), "CT_GEMM_SMALL_VIA_B_LOOP": (True, False, None, (0,))}
-VIA = {"CT_GEMM_VIA_A_LOOP": 0, "CT_GEMM_VIA_B_LOOP": 1, "CT_GEMM_SMALL_VIA_A_LOOP": 0, "CT_GEMM_SMALL_VIA_B_LOOP": 1}
+RING = {"CT_GEMM_SMALL_DEEP_LOOP": 8, "CT_GEMM_SMALL_DEEP_VIA_A_LOOP": 8}
+LOOPS.update({"CT_GEMM_SMALL_DEEP_LOOP": (True, False, 26, (0,)), "CT_GEMM_SMALL_DEEP_VIA_A_LOOP": (True, False, None, (0, 70))})
+VIA = {"CT_GEMM_SMALL_DEEP_VIA_A_LOOP": 0, "CT_GEMM_VIA_A_LOOP": 0, "CT_GEMM_VIA_B_LOOP": 1, "CT_GEMM_SMALL_VIA_A_LOOP": 0, "CT_GEMM_SMALL_VIA_B_LOOP": 1}
 
 
 def _lines(gen, name):
@@ -289,19 +296,21 @@ def _lines(gen, name):
             "CT_GEMM_FRESH_LOOP_BEHIND_STORES": lambda: gen.gemm_loop(fresh=True, behind_stores=True),
             "CT_GEMM_SMALL_LOOP": lambda: gen.small_loop(), "CT_GEMM_VIA_A_LOOP": lambda: gen.gemm_loop(fresh=True, via=0),
             "CT_GEMM_VIA_B_LOOP": lambda: gen.gemm_loop(via=1), "CT_GEMM_SMALL_VIA_A_LOOP": lambda: gen.small_loop(via=0),
-            "CT_GEMM_SMALL_VIA_B_LOOP": lambda: gen.small_loop(via=1)}[name]()
+            "CT_GEMM_SMALL_VIA_B_LOOP": lambda: gen.small_loop(via=1),
+            "CT_GEMM_SMALL_DEEP_LOOP": lambda: gen.small_loop(ring=8),
+            "CT_GEMM_SMALL_DEEP_VIA_A_LOOP": lambda: gen.small_loop(via=0, ring=8)}[name]()
 
 
 def _run(lines, name, steps, stores, start_wait=None):
     small, fresh, wait, _ = LOOPS[name]
-    machine = Machine(Tile(small), steps, fresh, stores, wait if start_wait is None else start_wait, VIA.get(name))
+    machine = Machine(Tile(small, RING.get(name, 4)), steps, fresh, stores, wait if start_wait is None else start_wait, VIA.get(name))
     machine.run(lines)
 
 
 @pytest.mark.parametrize("name", LOOPS)
 def test_waits_and_fragments(gen, name):
     lines = _lines(gen, name)
-    for steps in (4, 8, 12, 20):
+    for steps in (4, 8, 12, 16, 20):
         for stores in LOOPS[name][3]:
             _run(lines, name, steps, stores)
 
@@ -331,7 +340,7 @@ def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
         lines = list(good)
         change(lines)
         with pytest.raises(AssertionError):
-            _run(lines, name, 12, stores)
+            _run(lines, name, 3 * RING.get(name, 4), stores)
 
     # every wait for copies, one copy weaker (63 is the largest there is)
     loop = next(at for at, line in enumerate(good) if "_loop_" in line)
@@ -349,7 +358,7 @@ def test_model_catches_the_mistakes_it_is_meant_for(gen, name):
         if line in ("s_barrier", "s_waitcnt lgkmcnt(0)") and binds(at):
             broken(lambda lines: lines.__setitem__(at, "s_nop 0"))
     # a fragment read from the next stage, and a copy to it
-    tile = Tile(LOOPS[name][0])
+    tile = Tile(LOOPS[name][0], RING.get(name, 4))
     first = next(at for at, line in enumerate(good) if line.startswith("ds_read") and line.endswith("offset:0"))
     broken(lambda lines: lines.__setitem__(first, good[first].replace("offset:0", "offset:%d" % tile.a_stage)))
     copy = next(at for at, line in enumerate(good) if line.startswith("s_add_u32 m0"))

@@ -501,6 +501,9 @@ def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
     (50, 4224, 520),      # rows longer than what is read ahead of the list
     (1024, 256, 6144),    # 8 x 48 small tiles, gradients in large ones
     (1025, 256, 5500),    # 9 x 43, unaligned rows
+    (1024, 768, 4096),    # 8 x 32 small tiles, the most that have a compute unit each, 24 steps
+    (1024, 768, 4104),    # 8 x 33
+    (130, 896, 700),      # 2 x 6: a last half of eight steps; d = 640 below is too short for them
     (1024, 256, 7680),    # 8 x 60 small tiles: the last projection that takes them
     (1025, 256, 6912),    # 9 x 54: the first in large tiles, 5 x 27 of them: a round that fills part of the device
     (897, 640, 1288),     # gradients in small tiles, the last 8 columns from the tail
