@@ -291,21 +291,29 @@ struct CutceRowWork {
   bf16* dhidden;
 };
 
-// Backward. A workgroup of 16 wavefronts places 16 * row_rounds(N) rows and does their row work, a wavefront per
-// row: packed[slot] = hidden[row], and zeros for the dHidden rows of ignored tokens. (The head gradient
+// Backward. A workgroup of 16 wavefronts places rows_per_group(N, d) rows and does their row work, one or
+// several per row: packed[slot] = hidden[row], and zeros for the dHidden rows of ignored tokens. (The head gradient
 // contracts over slots; with the rows packed its operand tiles are plain strided copies instead of a gather at
 // every step. The slots past the active rows up to the next multiple of 256 hold zeros; their G^T entries
 // are zero or not read.) Every workgroup counts all weights by itself, from L2, and no workgroup waits for
 // another; a wavefront's first row is on its way meanwhile. The list and the row work in two launches took
 // 4.5 + 4.8 us at N = 380, d = 1664, now 5.8, and 9.2 + 40 at N = 16384, d = 4096. One round everywhere makes
 // the counting the longer part (69 us there).
+// Few long rows are shared by several wavefronts each, for more workgroups: a compute unit moves about 50 GB/s (a wavefront
+// per row / four, us: 64 rows, d = 6400 13.4 / 8.4, 250 10.0 / 7.4, 1000 12.1 / 9.8; d = 2048 6.8 / 6.1, 6.0 / 6.1,
+// 6.8 / 6.9, and 1024 and less 0.2 longer; two, 2000 rows: d = 2048 9.0 / 8.2, 6400 13.3 / 12.5).
 constexpr int kMostRowRounds = 64;
 __host__ __device__ inline int row_rounds(int rows) { return min((rows + 4095) / 4096, kMostRowRounds); }
+__host__ __device__ inline int row_waves(int rows, int d) { return d < 2048 || rows > 2048 ? 1 : rows > 1024 ? 2 : 4; }
+__host__ __device__ inline int rows_per_group(int rows, int d) { return 16 * row_rounds(rows) / row_waves(rows, d); }
 constexpr int kAhead = 8;         // chunks of a row per lane that are read while the weights are counted
 CT_DEVICE void list_and_pack_rows(const CutceParams& p, const CutceRowWork& work, int block, int blocks) {
   __shared__ int wave_before[16], wave_total[16], wave_first[16], group_count[16], slot_of[16 * kMostRowRounds];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rounds = row_rounds(p.N), rows = 16 * rounds, begin = block * rows, row_chunks = p.d / 8;
+  const int rounds = row_rounds(p.N), waves = row_waves(p.N, p.d), rows = rows_per_group(p.N, p.d);
+  const int begin = block * rows, row_chunks = p.d / 8;
+  // the wavefront's row of a round, and its chunks of the row: lane0 + stride k
+  const int group_row = wave / waves, lane0 = wave % waves * 64 + lane, stride = 64 * waves;
   if (block == 0) {
     reset_unit_counters(p.header);
     reset_dlogits_counters(p.header);
@@ -317,7 +325,7 @@ CT_DEVICE void list_and_pack_rows(const CutceParams& p, const CutceRowWork& work
   };
   if (ahead) {
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(begin + wave, lane + 64 * k);
+    for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(begin + group_row, lane0 + stride * k);
   }
   int before = begin, total = p.N, filler = 0;
   if (p.compact) {
@@ -377,28 +385,28 @@ CT_DEVICE void list_and_pack_rows(const CutceParams& p, const CutceRowWork& work
   }
   __syncthreads();
   for (int round = 0; round < rounds; ++round) {
-    const int row = begin + 16 * round + wave;
+    const int in_group = 16 / waves * round + group_row, row = begin + in_group;
     if (row >= p.N) break;
     if (p.weights[row] == 0.f) {
       u32x4* dst = reinterpret_cast<u32x4*>(work.dhidden + (size_t)row * p.d);
-      for (int c = lane; c < row_chunks; c += 64) dst[c] = u32x4{0u, 0u, 0u, 0u};
+      for (int c = lane0; c < row_chunks; c += stride) dst[c] = u32x4{0u, 0u, 0u, 0u};
     }
-    const int slot = uniform(slot_of[16 * round + wave]);
+    const int slot = uniform(slot_of[in_group]);
     if (!work.packed || slot < 0) continue;
     u32x4* dst = reinterpret_cast<u32x4*>(work.packed + (size_t)slot * p.d);
     if (ahead) {
       if (round != 0) {
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(row, lane + 64 * k);
+        for (int k = 0; k < kAhead; ++k) chunk[k] = row_chunk(row, lane0 + stride * k);
       }
 #pragma unroll
       for (int k = 0; k < kAhead; ++k)
-        if (lane + 64 * k < row_chunks) dst[lane + 64 * k] = chunk[k];
+        if (lane0 + stride * k < row_chunks) dst[lane0 + stride * k] = chunk[k];
 #pragma unroll 4
-      for (int c = lane + 64 * kAhead; c < row_chunks; c += 64) dst[c] = row_chunk(row, c);
+      for (int c = lane0 + stride * kAhead; c < row_chunks; c += stride) dst[c] = row_chunk(row, c);
     } else {
       const bf16* from = p.hidden + (size_t)row * p.d;
-      for (int c = lane; c < p.d; c += 64) reinterpret_cast<bf16*>(dst)[c] = from[c];
+      for (int c = lane0; c < p.d; c += stride) reinterpret_cast<bf16*>(dst)[c] = from[c];
     }
   }
   if (work.packed) {
@@ -530,7 +538,7 @@ __global__ __launch_bounds__(256, (GemmShape<NB, RING>::kGroups)) void cutce_sta
   units.init(p.header->xcd_counter[0], chunks, active_blocks, UnitQueue::kSweep);
   const auto next_unit = [&](int& chunk, int& rb) {
     while (units.next(chunk, rb, &unit_s))
-      if (p.block_active[rb * kTile / kGemmTile]) return true;
+      if (p.compact || p.block_active[rb * kTile / kGemmTile]) return true;
     return false;
   };
   int chunk, rb;
@@ -1934,7 +1942,7 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
     } else if (s == 0) {
       copy = tail;
     }
-    const int list_blocks = s == 0 ? (p.N + 16 * row_rounds(p.N) - 1) / (16 * row_rounds(p.N)) : 0;
+    const int per_group = rows_per_group(p.N, p.d), list_blocks = s == 0 ? (p.N + per_group - 1) / per_group : 0;
     if ((list_blocks || panel) && (rc = launch_prepare<true>(stream, p, work, copy, list_blocks, false))) return rc;
     if (cache) {
       LaunchScope scope11("cutce_dlogits_cached_kernel", stream);

@@ -508,6 +508,8 @@ def test_ragged_sizes_and_cut_contractions(ct, gpu, rows, width, vocab):
     (1025, 256, 6912),    # 9 x 54: the first in large tiles, 5 x 27 of them: a round that fills part of the device
     (897, 640, 1288),     # gradients in small tiles, the last 8 columns from the tail
     (1025, 1152, 1288),   # small tiles for the projection, large ones for the gradients
+    (1023, 2048, 300),    # row lists: four wavefronts a row, the last workgroup ragged
+    (1030, 8192, 130),    # two, of rows longer than what is read ahead
     (4099, 128, 300),     # row lists: two rounds of 16 rows per workgroup, the last one ragged
     (70001, 128, 130),    # 18 rounds: five wavefronts list rows
 ])
