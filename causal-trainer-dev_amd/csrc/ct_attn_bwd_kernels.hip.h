@@ -357,41 +357,49 @@ struct QdoCursor {
   CT_DEVICE QueryBlockBounds query_bounds() const { return query_block_bounds(reinterpret_cast<const int*>(bounds), 0); }
 };
 
-// Fragment address structures of the dK/dV kernel: the register-lean ones where the tile is
-// wide enough for them (the kernel is at the register limit).
-template <int D>
-using DkvRowFrags = std::conditional_t<(D / 8 >= 16), RowFragCompact<D / 8>, RowFragOffsets<D / 8>>;
-template <int D>
-using DkvTrFrags = std::conditional_t<(D / 8 >= 16), TrFragCompact<D / 8, KSlots::kAccum>,
-                                      TrFragOffsets<D / 8, KSlots::kAccum>>;
+// What a step of the dK/dV kernel for D = 128 needs besides its sums, the same in every step.
+struct DkvFrame {
+  const RowFragOffsets<16>& ro;
+  const TrFragOffsets<16, KSlots::kAccum>& to;
+  const bf16x8* kf;     // K fragments
+  lds_addr stat_ptr;    // LDS base + 16 * (lane / 32)
+  float scale_log2e;
+  unsigned v_off;       // byte offset of this wavefront's V rows
+};
 
-// Hand-scheduled MFMA sequences of the dK/dV kernel for D = 128 (gen_attn_asm.py): the
-// compiler's own schedule issues each LDS fragment read directly in front of the MFMA that
-// consumes it, so with two wavefronts per SIMD every MFMA pays most of the LDS latency.
-// STAGE_OFF is the byte offset of the stage (Q tile, then dO tile) from the LDS base the
-// pointers were built on; v_off the byte offset of this wavefront's V rows.
-template <int STAGE_OFF>
-CT_DEVICE void dkv_sdp_sequence_128(const RowFragOffsets<16>& ro, const bf16x8* kf, unsigned v_off,
-                                    f32x16& s, f32x16& dp) {
-  asm volatile(CT_DKV_SDP_SEQUENCE
-               : "+v"(s), "+v"(dp)
-               : "v"(ro.ptr[0]), "v"(ro.ptr[1]), "v"(ro.ptr[2]), "v"(ro.ptr[3]), "v"(ro.ptr[4]),
-                 "v"(ro.ptr[5]), "v"(ro.ptr[6]), "v"(ro.ptr[7]), "v"(kf[0]), "v"(kf[1]), "v"(kf[2]),
-                 "v"(kf[3]), "v"(kf[4]), "v"(kf[5]), "v"(kf[6]), "v"(kf[7]), "s"(v_off), "i"(STAGE_OFF)
-               : "memory", CT_DKV_ASM_SCRATCH);
-}
-template <int STAGE_OFF>
-CT_DEVICE void dkv_acc_sequence_128(const TrFragOffsets<16, KSlots::kAccum>& to, const f32x16& prob,
-                                    const f32x16& ds, f32x16* dvacc, f32x16* dkacc) {
-  const bf16x8 p0 = pack_acc8(prob, 0), p1 = pack_acc8(prob, 1);
-  const bf16x8 d0 = pack_acc8(ds, 0), d1 = pack_acc8(ds, 1);
-  asm volatile(CT_DKV_ACC_SEQUENCE
-               : "+v"(dvacc[0]), "+v"(dvacc[1]), "+v"(dvacc[2]), "+v"(dvacc[3]), "+v"(dkacc[0]),
-                 "+v"(dkacc[1]), "+v"(dkacc[2]), "+v"(dkacc[3])
-               : "v"(to.ptr[0][0]), "v"(to.ptr[0][1]), "v"(to.ptr[0][2]), "v"(to.ptr[0][3]),
-                 "v"(to.ptr[1][0]), "v"(to.ptr[1][1]), "v"(to.ptr[1][2]), "v"(to.ptr[1][3]), "v"(p0),
-                 "v"(p1), "v"(d0), "v"(d1), "i"(STAGE_OFF)
-               : "memory", CT_DKV_ASM_SCRATCH);
+// Which pairs of a step are allowed: all, those with the key's id and a key not behind the row's visible end, or those with
+// its id and a key not behind the row itself.
+enum class DkvPairs { kAll, kToEnds, kToRows };
+
+// One step as one generated stream (gen_attn_asm.py). `key`: for kToRows relative to the first query row of the lane's
+// half. STORE: the dS block leaves to `block` as well, as the lanes hold it: two runs of 64 x 16 bytes.
+template <int STAGE_OFF, DkvPairs PAIRS, bool STORE>
+CT_DEVICE void dkv_step_128(const DkvFrame& f, float masked, int id, int key, char* block, unsigned lane16) {
+#define CT_DKV_STEP_OPERANDS                                                                                            \
+  "v"(f.kf[0]), "v"(f.kf[1]), "v"(f.kf[2]), "v"(f.kf[3]), "v"(f.kf[4]), "v"(f.kf[5]), "v"(f.kf[6]), "v"(f.kf[7]),       \
+      "v"(f.ro.ptr[0]), "v"(f.ro.ptr[1]), "v"(f.ro.ptr[2]), "v"(f.ro.ptr[3]), "v"(f.ro.ptr[4]), "v"(f.ro.ptr[5]),       \
+      "v"(f.ro.ptr[6]), "v"(f.ro.ptr[7]), "v"(f.to.ptr[0][0]), "v"(f.to.ptr[0][1]), "v"(f.to.ptr[0][2]),                \
+      "v"(f.to.ptr[0][3]), "v"(f.to.ptr[1][0]), "v"(f.to.ptr[1][1]), "v"(f.to.ptr[1][2]), "v"(f.to.ptr[1][3]),          \
+      "v"(f.stat_ptr), "s"(f.scale_log2e), "s"(f.v_off), "i"(STAGE_OFF)
+#define CT_DKV_STEP_CLOBBERS "memory", "vcc", "scc", "s96", "s97", CT_DKV_STEP_SCRATCH, CT_DKV_ACCUMULATORS
+#define CT_DKV_STEP(SEQUENCE, ...) asm volatile(SEQUENCE : : CT_DKV_STEP_OPERANDS, ##__VA_ARGS__ : CT_DKV_STEP_CLOBBERS)
+#define CT_DKV_MASK "s"(masked), "v"(id), "v"(key)
+#define CT_DKV_STORE "s"(block), "v"(lane16)
+  if constexpr (PAIRS == DkvPairs::kAll) {
+    if constexpr (STORE) CT_DKV_STEP(CT_DKV_STEP_STORE_SEQUENCE, CT_DKV_STORE);
+    else CT_DKV_STEP(CT_DKV_STEP_SEQUENCE);
+  } else if constexpr (PAIRS == DkvPairs::kToEnds) {
+    if constexpr (STORE) CT_DKV_STEP(CT_DKV_STEP_ENDS_STORE_SEQUENCE, CT_DKV_MASK, CT_DKV_STORE);
+    else CT_DKV_STEP(CT_DKV_STEP_ENDS_SEQUENCE, CT_DKV_MASK);
+  } else {
+    if constexpr (STORE) CT_DKV_STEP(CT_DKV_STEP_ROWS_STORE_SEQUENCE, CT_DKV_MASK, CT_DKV_STORE);
+    else CT_DKV_STEP(CT_DKV_STEP_ROWS_SEQUENCE, CT_DKV_MASK);
+  }
+#undef CT_DKV_STORE
+#undef CT_DKV_MASK
+#undef CT_DKV_STEP
+#undef CT_DKV_STEP_CLOBBERS
+#undef CT_DKV_STEP_OPERANDS
 }
 
 // Store a (32 rows x D) accumulator (lanes along D) as bf16 rows via an LDS patch.
@@ -417,6 +425,66 @@ CT_DEVICE void store_rows(const f32x16* acc, lds_addr patch, bf16* gbase, size_t
   }
 }
 
+
+// An accumulator that only the assembly statements name, a[16 INDEX : 16 INDEX + 15]. A store in front may still read the
+// registers that the statement writes, and the compiler does not wait for it here.
+template <int INDEX>
+CT_DEVICE f32x16 read_accumulator() {
+  float v[16];
+  asm volatile("s_nop 1\n\t" CT_DKVW_READ
+               : "=v"(v[0]), "=v"(v[1]), "=v"(v[2]), "=v"(v[3]), "=v"(v[4]), "=v"(v[5]), "=v"(v[6]), "=v"(v[7]),
+                 "=v"(v[8]), "=v"(v[9]), "=v"(v[10]), "=v"(v[11]), "=v"(v[12]), "=v"(v[13]), "=v"(v[14]), "=v"(v[15])
+               : "i"(16 * INDEX));
+  f32x16 out;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) out[e] = v[e];
+  return out;
+}
+
+// dK or dV of a wavefront's 32 keys of D = 128, accumulators FIRST to FIRST + 3, as bf16 rows (store_rows), or to `mine` as
+// the f32 sums of a chunk. One accumulator at a time, and the lane anew for each: what the compiler has no room for it would
+// put into accumulation registers.
+template <int FIRST, bool SCALED>
+CT_DEVICE void leave_accumulators(float scale, float* mine, lds_addr patch, bf16* gbase, size_t row_stride) {
+  constexpr int CPR = 16;
+  const auto each = [&](auto db_tag) {
+    constexpr int kDb = decltype(db_tag)::value;
+    f32x16 sum = read_accumulator<FIRST + kDb>();
+    if (SCALED) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sum[e] *= scale;
+    }
+    const int l = lane_id_here();
+    if (mine) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        f32x4 quad;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) quad[e] = sum[4 * q4 + e];
+        *reinterpret_cast<f32x4*>(mine + l * 4 + (kDb * 4 + q4) * 256) = quad;
+      }
+    } else {
+      const int col = kDb * 32 + (l & 31);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        lds_store<bf16>(patch + tile_byte_offset<CPR>(acc_row(r, l >> 5), col >> 3) + (col & 7) * 2, (bf16)sum[r]);
+    }
+  };
+  each(std::integral_constant<int, 0>{});
+  each(std::integral_constant<int, 1>{});
+  each(std::integral_constant<int, 2>{});
+  each(std::integral_constant<int, 3>{});
+  if (mine) return;
+  __builtin_amdgcn_wave_barrier();
+  const int l = lane_id_here();
+#pragma unroll
+  for (int n = 0; n < 32 * CPR / 64; ++n) {
+    const int e = l + 64 * n;
+    const u32x4 val = lds_load<u32x4>(patch + tile_byte_offset<CPR>(e / CPR, e % CPR));
+    store_global16(gbase + (size_t)(e / CPR) * row_stride + e % CPR * 8, val);
+  }
+  __builtin_amdgcn_wave_barrier();
+}
 
 // Number of (head, query block) items of 128-key tile `tile` (= batch row * tiles per row + kt).
 CT_DEVICE int dkv_tile_items(const int* meta, int nrb, int tile, int g, int* q_lo_out = nullptr) {
@@ -830,8 +898,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
   const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
   const int g = p.Hq / p.Hkv;
   const int* meta_b = p.meta + (size_t)b * nrb * kMetaW;
-  const DkvRowFrags<D> ro(lds0);
-  const DkvTrFrags<D> to(lds0);
+  const RowFragOffsets<D / 8> ro(lds0);
+  const TrFragOffsets<D / 8, KSlots::kAccum> to(lds0);
 
   int q_lo = INT_MAX, q_hi = -1;
 #pragma unroll
@@ -867,11 +935,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
     kf[ks] = as_bf16x8(load_global16(p.k + kv_off + 16 * ks + 8 * half));
     lds_store<u32x4>(ro.addr(vpatch_off, 0, ks), load_global16(p.v + kv_off + 16 * ks + 8 * half));
   }
-  f32x16 dkacc[D / 32], dvacc[D / 32];
+  f32x16 dkacc[D / 32], dvacc[D / 32];  // (D = 128: in accumulation registers until the end)
+  if constexpr (D == 128) {
+    asm volatile(CT_DKV_ZERO : : : CT_DKV_ACCUMULATORS);
+  } else {
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
-    dkacc[db] = zero16();
-    dvacc[db] = zero16();
+    for (int db = 0; db < D / 32; ++db) {
+      dkacc[db] = zero16();
+      dvacc[db] = zero16();
+    }
   }
 
   // Make the K fragment loads complete here. Left pending, their first use inside the item
@@ -915,7 +987,21 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
     QueryBlockBounds bounds_ahead;  // (behind the last item: the same bounds again)
     const bool visit = blocks_interact(q_min, q_max, q_end_max, my_min, my_max, my_rb * 32);
     if (D != 64 || !visit) bounds_ahead = next.query_bounds();
-    if (visit) {
+    if (!visit) {
+    } else if constexpr (D == 128) {
+      const bool interior = tile_is_interior(q_uni, q_end_min, my_uni, my_rb * 32 + 31);
+      const int seg_k_or_never = seg_k != 0 ? seg_k : -1;  // ids are >= 0
+      char* block = SPILL ? ds_block_address(p, head, b, my_ds_off, my_q_first, qb) : nullptr;
+      const unsigned lane16 = SPILL ? (unsigned)lane_id_here() * 16 : 0;
+      const DkvFrame f{ro, to, kf, lds0 + 16 * half, scale_log2e, (unsigned)vpatch_off};
+      if (interior)
+        dkv_step_128<CUR * kStage, DkvPairs::kAll, SPILL>(f, masked, 0, 0, block, lane16);
+      else if (has_end)
+        dkv_step_128<CUR * kStage, DkvPairs::kToEnds, SPILL>(f, masked, seg_k_or_never, key, block, lane16);
+      else
+        dkv_step_128<CUR * kStage, DkvPairs::kToRows, SPILL>(f, masked, seg_k_or_never, key - 4 * half - qb * kQueryTile, block,
+                                                             lane16);
+    } else {
       // The row offsets below depend on the lane only; hoisted out of the loop they become
       // spilled registers whose reloads wait for every copy in flight. Recompute them here.
       int half_here = half;
@@ -935,22 +1021,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
           dp[4 * qd + e] = del4[e];
         }
       }
-      if constexpr (D == 128) {
-        // (fragment pointers built here from the lane id: held across the loop they would
-        // push the kernel over its register budget)
-        const RowFragOffsets<16> rp = RowFragOffsets<16>::expand(RowFragCompact<16>(lds0, lane_id_here()));
-        dkv_sdp_sequence_128<CUR * kStage>(rp, kf, (unsigned)vpatch_off, s, dp);
-      } else {
-        constexpr int kSteps = D / 16, qOff = CUR * kStage + QdoStage<D>::kQ, doOff = CUR * kStage + QdoStage<D>::kDo;
-        fragments_ahead<kSteps, kSteps>([&](int i) { return ro.load(qOff, 0, i); },
-                                        [&](int i, bf16x8 queries) { s = mfma32(queries, kf[i], s); });
-        struct Pair {
-          bf16x8 dout, v;
-        };
-        fragments_ahead<kSteps, 2>([&](int i) { return Pair{ro.load(doOff, 0, i), ro.load(vpatch_off, 0, i)}; },
-                                   [&](int i, const Pair& rows) { dp = mfma32(rows.dout, rows.v, dp); });
-        bounds_ahead = next.query_bounds();  // (a wait for LDS reads is one for all scalar loads too)
-      }
+      constexpr int kSteps = D / 16, qOff = CUR * kStage + QdoStage<D>::kQ, doOff = CUR * kStage + QdoStage<D>::kDo;
+      fragments_ahead<kSteps, kSteps>([&](int i) { return ro.load(qOff, 0, i); },
+                                      [&](int i, bf16x8 queries) { s = mfma32(queries, kf[i], s); });
+      struct Pair {
+        bf16x8 dout, v;
+      };
+      fragments_ahead<kSteps, 2>([&](int i) { return Pair{ro.load(doOff, 0, i), ro.load(vpatch_off, 0, i)}; },
+                                 [&](int i, const Pair& rows) { dp = mfma32(rows.dout, rows.v, dp); });
+      bounds_ahead = next.query_bounds();  // (a wait for LDS reads is one for all scalar loads too)
       const bool interior = tile_is_interior(q_uni, q_end_min, my_uni, my_rb * 32 + 31);
       f32x16 prob;
       if (!interior) {
@@ -989,22 +1068,16 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
         store_global16_s<0>(block, lane_off, __builtin_bit_cast(f32x4, pack_acc8(dp, 0)));
         store_global16_s<1024>(block, lane_off, __builtin_bit_cast(f32x4, pack_acc8(dp, 1)));
       }
-      if constexpr (D == 128) {
-        const TrFragOffsets<16, KSlots::kAccum> tp =
-            TrFragOffsets<16, KSlots::kAccum>::expand(TrFragCompact<16, KSlots::kAccum>(lds0, lane_id_here()));
-        dkv_acc_sequence_128<CUR * kStage>(tp, prob, dp, dvacc, dkacc);
-      } else {
-        const bf16x8 keys[4] = {pack_acc8(prob, 0), pack_acc8(prob, 1), pack_acc8(dp, 0), pack_acc8(dp, 1)};
-        constexpr int kBlocks = D / 32;
-        fragments_ahead<4 * kBlocks, 4>(
-            [&](int i) {
-              return to.load(CUR * kStage + (i < 2 * kBlocks ? QdoStage<D>::kDo : QdoStage<D>::kQ), i / kBlocks % 2, i % kBlocks);
-            },
-            [&](int i, bf16x8 rows) {
-              f32x16& acc = (i < 2 * kBlocks ? dvacc : dkacc)[i % kBlocks];
-              acc = mfma32(keys[i / kBlocks], rows, acc);
-            });
-      }
+      const bf16x8 keys[4] = {pack_acc8(prob, 0), pack_acc8(prob, 1), pack_acc8(dp, 0), pack_acc8(dp, 1)};
+      constexpr int kBlocks = D / 32;
+      fragments_ahead<4 * kBlocks, 4>(
+          [&](int i) {
+            return to.load(CUR * kStage + (i < 2 * kBlocks ? QdoStage<D>::kDo : QdoStage<D>::kQ), i / kBlocks % 2, i % kBlocks);
+          },
+          [&](int i, bf16x8 rows) {
+            f32x16& acc = (i < 2 * kBlocks ? dvacc : dkacc)[i % kBlocks];
+            acc = mfma32(keys[i / kBlocks], rows, acc);
+          });
     }
     // The next block's bounds are waited for here, where the step has given them the time. Left to their first use
     // the wait stands in the next step behind the loads for the step after it, and as scalar loads return in any
@@ -1025,6 +1098,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
     step(std::integral_constant<int, 1>{});
   }
 
+  if constexpr (D == 128) {
+    // The last sums have left the matrix pipe after these wait states (the compiler does not see the MFMAs).
+    asm volatile("s_nop 15\n\ts_nop 7" : : : "memory");
+    float* mine = nsplit > 1 ? p.dkv_partials + dkv_partial_offset<D>(slot0 + chunk, p.Hkv, kvh, w) : nullptr;
+    const size_t out_off = (((size_t)b * p.S + my_rb * 32) * p.Hkv + kvh) * D;
+    leave_accumulators<4, true>(p.scale, mine, vpatch, p.dk + out_off, kv_row_stride);
+    leave_accumulators<0, false>(p.scale, mine ? mine + DkvPartial<D>::kPerTensor : nullptr, vpatch, p.dv + out_off, kv_row_stride);
+    return;
+  }
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll

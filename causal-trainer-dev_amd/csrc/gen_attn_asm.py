@@ -14,14 +14,6 @@ SCRATCH0 = 240
 # The compiler cannot see the MFMAs inside an asm statement, so it will not insert the wait
 # states that a vector ALU read of a fresh MFMA result needs; the sequences end with them.
 TAIL = ["s_nop 15", "s_nop 7"]
-# dK/dV: the wavefront drops to issue priority 0 for a sequence and returns to 1 after it, so
-# that the other wavefront of the SIMD, when it is in its exponent / dS arithmetic, issues
-# first: an MFMA sequence issues one instruction every 32 cycles and loses nothing by waiting a
-# few, while the arithmetic phase is issue-bound (measured: dK/dV kernel 3 % faster; the same
-# in the forward sequences, or with the levels swapped, is slower or neutral).
-DKV_HEAD = ["s_waitcnt lgkmcnt(0)", "s_setprio 0"]
-DKV_TAIL = ["s_setprio 1"] + TAIL
-
 
 def slot_regs(slot):
     lo = SCRATCH0 + 4 * slot
@@ -333,6 +325,8 @@ def fwd_private_clobbers():
                      ['"a%d"' % r for r in range(64)])
 
 
+# dK/dV, the products and the sums of a step as two plain sequences with the arithmetic between them: the order of the sums
+# that the stream below keeps.
 DKV_SLOTS = 5
 DKV_SCRATCH0 = 256 - 4 * DKV_SLOTS - 1  # one address temporary, then the fragment slots
 
@@ -355,7 +349,7 @@ def dkv_sdp_sequence():
     """
     steps = 8
     total = 3 * steps  # read r = 3 ks + which; which: 0 Q, 1 dO, 2 V
-    lines = list(DKV_HEAD)
+    lines = ["s_waitcnt lgkmcnt(0)"]
     state = {"issued": 0}
 
     def load_next():
@@ -384,7 +378,7 @@ def dkv_sdp_sequence():
                                                                                v_slot[1]))
         lines += load_next()
         lines += load_next()
-    return lines + DKV_TAIL
+    return lines + TAIL
 
 
 def dkv_acc_sequence(ahead=DKV_SLOTS, slots=DKV_SLOTS):
@@ -398,7 +392,7 @@ def dkv_acc_sequence(ahead=DKV_SLOTS, slots=DKV_SLOTS):
     """
     order = [(step, db, which) for step in range(2) for db in range(4) for which in range(2)]  # which: 0 dV, 1 dK
     n = len(order)
-    lines = list(DKV_HEAD)
+    lines = ["s_waitcnt lgkmcnt(0)"]
 
     def load(i):
         step, db, which = order[i]
@@ -419,7 +413,177 @@ def dkv_acc_sequence(ahead=DKV_SLOTS, slots=DKV_SLOTS):
         lines.append("v_mfma_f32_32x32x16_bf16 %%%d, %%%d, v[%d:%d], %%%d" % (acc, aop, lo, hi, acc))
         if i + ahead < n:
             lines += load(i + ahead)
-    return lines + DKV_TAIL
+    return lines + TAIL
+
+
+class Stream:
+    """Instruction list with in-order tracking of the LDS reads in flight (lgkmcnt)."""
+
+    def __init__(self, head=("s_waitcnt lgkmcnt(0)",)):
+        self.lines = list(head)
+        self.pending = []
+
+    def lds(self, text, tag):
+        self.lines.append(text)
+        self.pending.append(tag)
+        assert len(self.pending) <= 15, "lgkmcnt holds at most 15"
+
+    def wait(self, tag):
+        if tag not in self.pending:
+            return
+        i = len(self.pending) - 1 - self.pending[::-1].index(tag)
+        self.lines.append("s_waitcnt lgkmcnt(%d)" % (len(self.pending) - 1 - i))
+        self.pending = self.pending[i + 1:]
+
+    def wait_all(self):
+        self.lines.append("s_waitcnt lgkmcnt(0)")
+        self.pending = []
+
+    def emit(self, text):
+        self.lines.append(text)
+
+
+def w_acc(i):
+    """Accumulator i of the wide kernel: 0-3 dV of key block 0 (column block db), 4-7 dV of key
+    block 1, 8-11 dK of key block 0, 12-15 dK of key block 1. They live in fixed accumulation
+    registers for the whole kernel and are never handed to the compiler."""
+    return "a[%d:%d]" % (16 * i, 16 * i + 15)
+
+
+# dK/dV, a step as one stream: S first, then dP with the exponents of S behind its
+# MFMAs, then dV with the dS arithmetic behind its MFMAs, then dK. Fixed registers (declared as clobbers): a bit
+# per pair that is allowed, the bf16 P fragments, the address of a V fragment, S, dP (its first 8 registers later hold the bf16 dS fragments) and the ring; the
+# sums are a[0:127] for the whole kernel (w_acc: 0-3 dV, 4-7 dK) and never handed to the compiler, so a step does not end
+# with the wait states behind its last MFMA (1.5 % of the kernel): whoever reads the sums waits. Between its streams a
+# wavefront issues behind the other one of its SIMD (the other way round 0.5 to 1 % longer). The matrix pipe is busy 64 % of
+# the time with five fragment slots, 61.5 with the two sequences above and the arithmetic between them ([2, 8192, 16/16] whole
+# rows); [4, 4096, 32/8] documents of 64 to 4096 682 -> 642 us, [2, 8192, 16/16] of 64 to 2000 235 -> 224. Five slots instead
+# of six 0.2 % longer, seven 0.5 % shorter in launches of one round and 0.7 % longer in large ones.
+DKVS_SLOTS = 6
+DKVS_RING0 = 128 - 4 * DKVS_SLOTS
+DKVS_DP = DKVS_RING0 - 16
+DKVS_S = DKVS_DP - 16
+DKVS_ADDR = DKVS_S - 1
+DKVS_ALLOWED = DKVS_ADDR - 1
+DKVS_P = DKVS_ALLOWED - 8   # (register runs begin at even numbers)
+
+
+def dkv_step_sequence(mask, stores):
+    """operands: %0-%7 K fragments, %8-%15 row-fragment pointers, %16-%19 transposed fragments, lo, and %20-%23, hi, %24
+    pointer of this lane's statistics (LDS base + 16 * (lane / 32)), %25 scale * log2(e) and %26 byte offset of this
+    wavefront's V rows (scalar), %27 byte offset of the stage (Q tile, dO tile 8192 later, -lse / scale at 16384, -delta at
+    16512). With `mask` some pair is not allowed, and its sum becomes %28 (scalar): those with another id than %29 among the
+    ids of the query rows (at 16640 of the stage), and with "ends" those whose key %30 lies behind the row's visible end
+    (at 16768), with "rows" those where %30, the key less the number of the half's first row, is more than the row's own. With `stores` the dS block leaves as well: behind those its address (scalar pair)
+    and 16 * lane.
+
+    Scalar loads may be in flight where the stream begins: its first wait is for everything, and no other counts them.
+    """
+    st = Stream(head=[])
+    stage = "%27"
+    block = lambda base: "v[%d:%d]" % (base, base + 15)
+
+    def stats(base, offset):
+        for qd in range(4):
+            st.lds("ds_read_b128 v[%d:%d], %%24 offset:%s+%d" % (base + 4 * qd, base + 4 * qd + 3, stage, offset + 32 * qd), "stat")
+
+    def slot(r):
+        lo = DKVS_RING0 + 4 * (r % DKVS_SLOTS)
+        return lo, "v[%d:%d]" % (lo, lo + 3)
+
+    reads, mfmas = [], []
+    for ks in range(8):
+        reads.append(["ds_read_b128 {v4}, %%%d offset:%s" % (8 + ks, stage)])
+        mfmas.append(("v_mfma_f32_32x32x16_bf16 %s, {r0}, %%%d, %s" % (block(DKVS_S), ks, block(DKVS_S)), [ks]))
+    for ks in range(8):
+        base = len(reads)
+        reads.append(["ds_read_b128 {v4}, %%%d offset:%s+8192" % (8 + ks, stage)])
+        reads.append(["v_add_u32_e32 v%d, %%26, %%%d" % (DKVS_ADDR, 8 + ks), "ds_read_b128 {v4}, v%d" % DKVS_ADDR])
+        mfmas.append(("v_mfma_f32_32x32x16_bf16 %s, {r0}, {r1}, %s" % (block(DKVS_DP), block(DKVS_DP)), [base, base + 1]))
+    for which, source in ((0, DKVS_P), (1, DKVS_DP)):   # dV (P^T, dO), dK (dS^T, Q)
+        for step in range(2):
+            for db in range(4):
+                off = "%s+%d" % (stage, step * 4096 + (8192 if which == 0 else 0))
+                reads.append(["ds_read_b64_tr_b16 {v2lo}, %%%d offset:%s" % (16 + db, off),
+                              "ds_read_b64_tr_b16 {v2hi}, %%%d offset:%s" % (20 + db, off)])
+                a = w_acc(4 * which + db)
+                mfmas.append(("v_mfma_f32_32x32x16_bf16 %s, v[%d:%d], {r0}, %s" % (a, source + 4 * step, source + 4 * step + 3, a),
+                              [len(reads) - 1]))
+
+    # A product's sums are read two MFMAs after its last one at the earliest: they have left the matrix pipe by then.
+    fill = [[] for _ in range(len(mfmas) + 1)]
+    packed_at = {}
+    for e in range(16):
+        t = 9 + (e * 9) // 16
+        if mask:   # (the address register is free between the pairs of instructions that use it)
+            fill[t] += ["v_bfe_i32 v%d, v%d, %d, 1" % (DKVS_ADDR, DKVS_ALLOWED, 15 - e),
+                        "v_bfi_b32 v%d, v%d, v%d, %%28" % (DKVS_S + e, DKVS_ADDR, DKVS_S + e)]
+        fill[t] += ["v_mul_f32_e32 v%d, %%25, v%d" % (DKVS_S + e, DKVS_S + e), "v_exp_f32_e32 v%d, v%d" % (DKVS_S + e, DKVS_S + e)]
+        t_ds = 17 + (e * 9) // 16
+        fill[t_ds] += ["v_mul_f32_e32 v%d, v%d, v%d" % (DKVS_DP + e, DKVS_S + e, DKVS_DP + e)]
+        if e % 2 == 1:
+            k = e // 2
+            fill[t + 1] += ["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (DKVS_P + k, DKVS_S + 2 * k, DKVS_S + 2 * k + 1)]
+            fill[t_ds] += ["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (DKVS_DP + k, DKVS_DP + 2 * k, DKVS_DP + 2 * k + 1)]
+            packed_at[e] = (t + 1, t_ds)
+    assert packed_at[7][0] < 16 and packed_at[15][0] < 20 and packed_at[7][1] < 24 and packed_at[15][1] < 28
+    if stores:
+        address, lane = ("%31", "%32") if mask else ("%28", "%29")
+        for half, e in ((0, 7), (1, 15)):
+            fill[packed_at[e][1] + 2] += ["global_store_dwordx4 %s, v[%d:%d], %s offset:%d" % (
+                lane, DKVS_DP + 4 * half, DKVS_DP + 4 * half + 3, address, 1024 * half)]
+
+    # The bits of the pairs, four rows at a time behind two MFMAs of S: ids and ends go where the P fragments will be.
+    def mask_reads(qd):
+        st.lds("ds_read_b128 v[%d:%d], %%24 offset:%s+%d" % (DKVS_P, DKVS_P + 3, stage, 16640 + 32 * qd), "mask")
+        if mask == "ends":
+            st.lds("ds_read_b128 v[%d:%d], %%24 offset:%s+%d" % (DKVS_P + 4, DKVS_P + 7, stage, 16768 + 32 * qd), "mask")
+
+    def mask_bits(qd, e):
+        limit = "v_cmp_le_i32_e64 s[96:97], %%30, v%d" % (DKVS_P + 4 + e) if mask == "ends" else "v_cmp_ge_i32_e64 s[96:97], %d, %%30" % (8 * qd + e)
+        return ["v_cmp_eq_u32_e32 vcc, %%29, v%d" % (DKVS_P + e), limit, "s_and_b64 vcc, vcc, s[96:97]",
+                "v_addc_co_u32_e32 v%d, vcc, v%d, v%d, vcc" % (DKVS_ALLOWED, DKVS_ALLOWED, DKVS_ALLOWED)]
+
+    state = {"issued": 0}
+    consumed = [False] * len(reads)
+
+    def issue_reads():
+        while state["issued"] < len(reads):
+            r = state["issued"]
+            if r >= DKVS_SLOTS and not consumed[r - DKVS_SLOTS]:
+                break
+            lo, v4 = slot(r)
+            for text in reads[r]:
+                text = text.format(v4=v4, v2lo="v[%d:%d]" % (lo, lo + 1), v2hi="v[%d:%d]" % (lo + 2, lo + 3))
+                (st.lds(text, r) if text.startswith("ds_") else st.emit(text))
+            state["issued"] += 1
+
+    stats(DKVS_S, 16384)
+    issue_reads()
+    st.wait_all()
+    st.emit("s_setprio 1")
+    if mask:
+        st.emit("v_mov_b32_e32 v%d, 0" % DKVS_ALLOWED)
+    for i, (text, needs) in enumerate(mfmas):
+        st.wait(needs[-1])
+        st.emit(text.format(**{"r%d" % n: slot(r)[1] for n, r in enumerate(needs)}))
+        for r in needs:
+            consumed[r] = True
+        if i == 0:
+            stats(DKVS_DP, 16512)
+        if mask and i < 8:
+            if i % 2 == 0:
+                mask_reads(i // 2)
+            else:
+                st.wait("mask")
+                for e in range(4):
+                    for line in mask_bits(i // 2, e):
+                        st.emit(line)
+        issue_reads()
+        for line in fill[i]:
+            st.emit(line)
+    assert not fill[len(mfmas)] and state["issued"] == len(reads)
+    return st.lines + ["s_setprio 0"]
 
 
 # (Dropping the issue priority for these sequences, as the dK/dV ones do, measured neutral here.)
@@ -503,36 +667,6 @@ W_S = (W_RING0 - 64, W_RING0 - 32)      # S^T accumulators of key block 0 / 1 (1
 W_DP = (W_RING0 - 48, W_RING0 - 16)     # dP accumulators
 W_ADDR = W_RING0 - 65                   # address of a V fragment
 W_FIRST = W_ADDR
-
-
-class Stream:
-    """Instruction list with in-order tracking of the LDS reads in flight (lgkmcnt)."""
-
-    def __init__(self):
-        self.lines = ["s_waitcnt lgkmcnt(0)"]
-        self.pending = []
-
-    def lds(self, text, tag):
-        self.lines.append(text)
-        self.pending.append(tag)
-        assert len(self.pending) <= 15, "lgkmcnt holds at most 15"
-
-    def wait(self, tag):
-        if tag not in self.pending:
-            return
-        i = len(self.pending) - 1 - self.pending[::-1].index(tag)
-        self.lines.append("s_waitcnt lgkmcnt(%d)" % (len(self.pending) - 1 - i))
-        self.pending = self.pending[i + 1:]
-
-    def emit(self, text):
-        self.lines.append(text)
-
-
-def w_acc(i):
-    """Accumulator i of the wide kernel: 0-3 dV of key block 0 (column block db), 4-7 dV of key
-    block 1, 8-11 dK of key block 0, 12-15 dK of key block 1. They live in fixed accumulation
-    registers for the whole kernel and are never handed to the compiler."""
-    return "a[%d:%d]" % (16 * i, 16 * i + 15)
 
 
 class WideOperands:
@@ -725,8 +859,8 @@ def dkvw_run_sequence():
     return lines + TAIL
 
 
-def dkvw_zero():
-    return ["v_accvgpr_write_b32 a%d, 0" % r for r in range(256)]
+def dkv_zero(registers):
+    return ["v_accvgpr_write_b32 a%d, 0" % r for r in range(registers)]
 
 
 def dkvw_read():
@@ -736,11 +870,14 @@ def dkvw_read():
 
 def clobbers():
     regs = ", ".join('"v%d"' % r for r in range(SCRATCH0, SCRATCH0 + 16))
-    dkv = ", ".join('"v%d"' % r for r in range(DKV_SCRATCH0, 256))
+    step = ", ".join('"v%d"' % r for r in range(DKVS_P, 128))
+    step_accs = ", ".join('"a%d"' % r for r in range(128))
     wide = ", ".join('"v%d"' % r for r in range(W_FIRST, 256))
     accs = ", ".join('"a%d"' % r for r in range(256))
-    return ("#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DKV_ASM_SCRATCH %s\n\n#define CT_DKVW_ASM_SCRATCH %s\n\n"
-            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (regs, dkv, wide, accs,
+    return ("#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DKV_STEP_SCRATCH %s\n\n"
+            "#define CT_DKV_ACCUMULATORS %s\n\n"
+            "#define CT_DKVW_ASM_SCRATCH %s\n\n"
+            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (regs, step, step_accs, wide, accs,
                                                                              fwd_private_clobbers()))
 
 
@@ -755,11 +892,13 @@ if __name__ == "__main__":
         print(emit(lines, "CT_FWD_ACC_%s" % name))
     print(emit(dq_sdp_half_sequence(), "CT_DQ_SDP_HALF_SEQUENCE"))
     print(emit(dq_acc_half_sequence(), "CT_DQ_ACC_HALF_SEQUENCE"))
-    print(emit(dkv_sdp_sequence(), "CT_DKV_SDP_SEQUENCE"))
-    print(emit(dkv_acc_sequence(), "CT_DKV_ACC_SEQUENCE"))
+    for mask in ("", "ends", "rows"):
+        for stores in (False, True):
+            print(emit(dkv_step_sequence(mask, stores), "CT_DKV_STEP_%s%sSEQUENCE" % (mask.upper() + "_" * bool(mask), "STORE_" * stores)))
+    print(emit(dkv_zero(128), "CT_DKV_ZERO"))
     print(emit(dkvw_step_sequence(), "CT_DKVW_FAST_SEQUENCE"))
     print(emit(dkvw_step_sequence(masked=True), "CT_DKVW_MASKED_SEQUENCE"))
     print(emit(dkvw_run_sequence(), "CT_DKVW_RUN_SEQUENCE"))
-    print(emit(dkvw_zero(), "CT_DKVW_ZERO"))
+    print(emit(dkv_zero(256), "CT_DKVW_ZERO"))
     print(emit(dkvw_read(), "CT_DKVW_READ"))
     print(clobbers())

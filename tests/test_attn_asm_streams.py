@@ -106,6 +106,9 @@ def _sequences(gen):
         "dkvw_step": gen.dkvw_step_sequence(), "dkvw_masked": gen.dkvw_step_sequence(masked=True),
         "dkvw_run": gen.dkvw_run_sequence(),
     }
+    for mask in ("", "ends", "rows"):
+        for stores in (False, True):
+            sequences["dkv_step_%s_%s" % (mask, stores)] = gen.dkv_step_sequence(mask, stores)
     for cur in ("a", "b"):
         for name, lines in gen.fwd_statements(cur).items():
             sequences["fwd_%s_%s" % (name.lower(), cur)] = lines
@@ -177,6 +180,57 @@ def test_wide_stream_structure(gen):
     assert len(narrowed) == 2
     for i in narrowed:
         assert lines[i + 1].startswith("global_load_lds") and lines[i + 2] == "s_mov_b64 exec, -1"
+
+
+@pytest.mark.parametrize("mask", ["", "ends", "rows"])
+@pytest.mark.parametrize("stores", [False, True])
+def test_dkv_step_stream(gen, mask, stores):
+    """One step of the dK/dV kernel: the MFMAs of every sum in the order of the plain sequences, the arithmetic of every
+    element between the products and the sums that need it, the mask in front of it, the stores behind it."""
+
+    lines = gen.dkv_step_sequence(mask, stores)
+    mfmas = [(i, _split(line)[1]) for i, line in enumerate(lines) if line.startswith("v_mfma")]
+    assert len(mfmas) == 32
+    s0, dp0, p0 = gen.DKVS_S, gen.DKVS_DP, gen.DKVS_P
+    block = lambda base, n: "v[%d:%d]" % (base, base + n - 1)
+    products = {base: [i for i, ops in mfmas if ops[0] == block(base, 16)] for base in (s0, dp0)}
+    assert [len(v) for v in products.values()] == [8, 8]
+    assert [ops[2] for i, ops in mfmas if ops[0] == block(s0, 16)] == ["%%%d" % ks for ks in range(8)]
+    # every sum: its two k-steps in order, P or dS as their operand
+    for which, base in ((0, p0), (1, dp0)):
+        for db in range(4):
+            sum_ops = [ops for _, ops in mfmas if ops[0] == gen.w_acc(4 * which + db)]
+            assert [ops[1] for ops in sum_ops] == [block(base, 4), block(base + 4, 4)] and all(ops[3] == ops[0] for ops in sum_ops)
+    position = {line: i for i, line in enumerate(lines)}
+    first_use = lambda base: min(i for i, ops in mfmas if ops[1] == block(base, 4))
+    for e in range(16):
+        s, dp, k = s0 + e, dp0 + e, e // 2
+        scaled, exp2 = position["v_mul_f32_e32 v%d, %%25, v%d" % (s, s)], position["v_exp_f32_e32 v%d, v%d" % (s, s)]
+        ds = position["v_mul_f32_e32 v%d, v%d, v%d" % (dp, s, dp)]
+        pack_p = position["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (p0 + k, s0 + 2 * k, s0 + 2 * k + 1)]
+        pack_ds = position["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (dp0 + k, dp0 + 2 * k, dp0 + 2 * k + 1)]
+        assert max(products[s0]) < scaled < exp2 < pack_p - 1 and pack_p < first_use(p0 + 4 * (e // 8))
+        assert max(products[dp0]) < ds and exp2 < ds - 1 and ds < pack_ds < first_use(dp0 + 4 * (e // 8))
+        # (a pair's packing overwrites element k, whose own packing is done)
+        assert position["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (dp0 + k // 2, dp0 + 2 * (k // 2), dp0 + 2 * (k // 2) + 1)] <= pack_ds
+        if mask:
+            bit = position["v_bfe_i32 v%d, v%d, %d, 1" % (gen.DKVS_ADDR, gen.DKVS_ALLOWED, 15 - e)]
+            assert max(products[s0]) < bit and bit + 2 == scaled and lines[bit + 1] == "v_bfi_b32 v%d, v%d, v%d, %%28" % (s, gen.DKVS_ADDR, s)
+    if mask:   # 16 bits, shifted in element by element, each by the id of its row and its end or its number
+        bits = [i for i, line in enumerate(lines) if line.startswith("v_addc_co_u32")]
+        assert len(bits) == 16 and max(bits) < max(products[dp0])
+        for e, i in enumerate(bits):
+            assert lines[i - 3] == "v_cmp_eq_u32_e32 vcc, %%29, v%d" % (p0 + e % 4) and lines[i - 1] == "s_and_b64 vcc, vcc, s[96:97]"
+            assert lines[i - 2] == ("v_cmp_le_i32_e64 s[96:97], %%30, v%d" % (p0 + 4 + e % 4) if mask == "ends" else
+                                    "v_cmp_ge_i32_e64 s[96:97], %d, %%30" % (8 * (e // 4) + e % 4))
+            reads = [line for line in lines[:i] if line.startswith("ds_read_b128 v[%d:%d]" % (p0, p0 + 3))]
+            assert reads[-1].endswith("offset:%%27+%d" % (16640 + 32 * (e // 4)))
+    # scalar loads may be in flight at the beginning: the first wait is for everything
+    assert next(line for line in lines if "lgkmcnt" in line) == "s_waitcnt lgkmcnt(0)"
+    stored = [(i, _split(line)[1]) for i, line in enumerate(lines) if line.startswith("global_store")]
+    assert [ops[1] for _, ops in stored] == ([block(dp0, 4), block(dp0 + 4, 4)] if stores else [])
+    for n, (i, _) in enumerate(stored):
+        assert i > position["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (dp0 + 4 * n + 3, dp0 + 8 * n + 6, dp0 + 8 * n + 7)]
 
 
 def _vector_alu(lines):
