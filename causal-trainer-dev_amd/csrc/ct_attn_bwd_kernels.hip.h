@@ -402,11 +402,38 @@ CT_DEVICE void dkv_step_128(const DkvFrame& f, float masked, int id, int key, ch
 #undef CT_DKV_STEP_OPERANDS
 }
 
-// Store a (32 rows x D) accumulator (lanes along D) as bf16 rows via an LDS patch.
+// The rows of 32 keys of D = 128 on their way through a wavefront's patch (swizzled tile layout): element r of column block
+// db is row 8 (r / 4) + 4 half + r % 4, chunk 4 db + j / 8, and lies a constant behind one of two addresses. (Formed from row
+// and chunk numbers for each, they were much of the end of a tile: documents of 17 to 113 in [1, 2048, 8/8 heads], the kernel
+// 20.6 us with them, 19.5 without.)
+struct KeyRowsPatch {
+  lds_addr at[2];
+  CT_DEVICE KeyRowsPatch(lds_addr patch, int l) {
+    const int j = l & 31, half = l >> 5;
+#pragma unroll
+    for (int odd = 0; odd < 2; ++odd) at[odd] = patch + half * 1024 + (j & 7) * 2 + (((j >> 3) ^ half ^ (2 * odd)) << 4);
+  }
+  CT_DEVICE void store(int db, const f32x16& sum) const {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      lds_store<bf16>(at[r / 4 % 2] + (2048 * (r / 4) + 256 * (r % 4) + 64 * (db ^ (r % 4))), (bf16)sum[r]);
+  }
+};
+
+// Store a (32 rows x D) accumulator (lanes along D) as bf16 rows via an LDS patch. (Head dimension 64 with two addresses
+// as well: what the compiler then does with the item loop in front takes 1 to 2 % longer.)
 template <int D>
 CT_DEVICE void store_rows(const f32x16* acc, lds_addr patch, bf16* gbase, size_t row_stride) {
   constexpr int CPR = D / 8;
   const int l = lane_id(), j = l & 31, half = l >> 5;
+  if constexpr (D == 128) {
+    const KeyRowsPatch rows(patch, l);
+#pragma unroll
+    for (int db = 0; db < 4; ++db) rows.store(db, acc[db]);
+    __builtin_amdgcn_wave_barrier();
+    PatchRows<D>::to_global(patch, l, gbase, row_stride);
+    return;
+  }
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) {
     const int col = db * 32 + j;
@@ -425,7 +452,6 @@ CT_DEVICE void store_rows(const f32x16* acc, lds_addr patch, bf16* gbase, size_t
   }
 }
 
-
 // An accumulator that only the assembly statements name, a[16 INDEX : 16 INDEX + 15]. A store in front may still read the
 // registers that the statement writes, and the compiler does not wait for it here.
 template <int INDEX>
@@ -442,11 +468,12 @@ CT_DEVICE f32x16 read_accumulator() {
 }
 
 // dK or dV of a wavefront's 32 keys of D = 128, accumulators FIRST to FIRST + 3, as bf16 rows (store_rows), or to `mine` as
-// the f32 sums of a chunk. One accumulator at a time, and the lane anew for each: what the compiler has no room for it would
-// put into accumulation registers.
+// the f32 sums of a chunk. One accumulator at a time: what the compiler has no room for it would put into accumulation
+// registers.
 template <int FIRST, bool SCALED>
 CT_DEVICE void leave_accumulators(float scale, float* mine, lds_addr patch, bf16* gbase, size_t row_stride) {
-  constexpr int CPR = 16;
+  const int l = lane_id_here();
+  const KeyRowsPatch rows(patch, l);
   const auto each = [&](auto db_tag) {
     constexpr int kDb = decltype(db_tag)::value;
     f32x16 sum = read_accumulator<FIRST + kDb>();
@@ -454,7 +481,6 @@ CT_DEVICE void leave_accumulators(float scale, float* mine, lds_addr patch, bf16
 #pragma unroll
       for (int e = 0; e < 16; ++e) sum[e] *= scale;
     }
-    const int l = lane_id_here();
     if (mine) {
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
@@ -464,10 +490,7 @@ CT_DEVICE void leave_accumulators(float scale, float* mine, lds_addr patch, bf16
         *reinterpret_cast<f32x4*>(mine + l * 4 + (kDb * 4 + q4) * 256) = quad;
       }
     } else {
-      const int col = kDb * 32 + (l & 31);
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        lds_store<bf16>(patch + tile_byte_offset<CPR>(acc_row(r, l >> 5), col >> 3) + (col & 7) * 2, (bf16)sum[r]);
+      rows.store(kDb, sum);
     }
   };
   each(std::integral_constant<int, 0>{});
@@ -476,14 +499,8 @@ CT_DEVICE void leave_accumulators(float scale, float* mine, lds_addr patch, bf16
   each(std::integral_constant<int, 3>{});
   if (mine) return;
   __builtin_amdgcn_wave_barrier();
-  const int l = lane_id_here();
-#pragma unroll
-  for (int n = 0; n < 32 * CPR / 64; ++n) {
-    const int e = l + 64 * n;
-    const u32x4 val = lds_load<u32x4>(patch + tile_byte_offset<CPR>(e / CPR, e % CPR));
-    store_global16(gbase + (size_t)(e / CPR) * row_stride + e % CPR * 8, val);
-  }
-  __builtin_amdgcn_wave_barrier();
+  PatchRows<128>::to_global(patch, l, gbase, row_stride);
+  __builtin_amdgcn_wave_barrier();  // (the other tensor leaves through the same patch)
 }
 
 // Number of (head, query block) items of 128-key tile `tile` (= batch row * tiles per row + kt).
