@@ -21,14 +21,6 @@ namespace ct {
 // ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
-// Fragment address structures of the backward kernels: the register-lean ones where the tile
-// is wide enough for them (both kernels are at the register limit).
-template <int D>
-using LeanRowFrags = std::conditional_t<(D / 8 >= 16), RowFragCompact<D / 8>, RowFragOffsets<D / 8>>;
-template <int D>
-using LeanTrFrags = std::conditional_t<(D / 8 >= 16), TrFragCompact<D / 8, KSlots::kAccum>,
-                                       TrFragOffsets<D / 8, KSlots::kAccum>>;
-
 // The dK/dV kernels work on unscaled Q K^T and put the softmax scale into the exponent. Any finite
 // scale is legal (the operator only asks for a finite one): a scale too small for lse / scale to
 // stay finite (|scale| < 1e-30, zero included) is replaced there by 1e-30, for which scale * S
@@ -54,6 +46,49 @@ CT_DEVICE void dq_arith(f32x16& s, const f32x16& dp, float lse2) {
   for (int r = 0; r < 16; ++r) s[r] = exp2_fast(fmaf(s[r], kLog2e, -lse2)) * dp[r];
 }
 
+// What a key tile of the dQ kernel for D = 128 needs besides its sums, the same for every tile.
+struct DqFrame {
+  const RowFragOffsets<16>& ro;
+  const TrFragOffsets<16, KSlots::kAccum>& to;
+  const bf16x8* qf;     // Q and dO fragments
+  const bf16x8* dof;
+  float lse2, delta;    // of the lane's query row
+};
+
+// One key tile as one generated stream (gen_attn_asm.py). MASKED: bit e of `allowed` tells whether the pair of element e is
+// allowed (key 8 (e / 4) + 4 half + e % 4 of the tile).
+template <int STAGE_OFF, bool MASKED>
+CT_DEVICE void dq_step_128(const DqFrame& f, unsigned allowed) {
+#define CT_DQ_STEP_OPERANDS                                                                                             \
+  "v"(f.qf[0]), "v"(f.qf[1]), "v"(f.qf[2]), "v"(f.qf[3]), "v"(f.qf[4]), "v"(f.qf[5]), "v"(f.qf[6]), "v"(f.qf[7]),       \
+      "v"(f.dof[0]), "v"(f.dof[1]), "v"(f.dof[2]), "v"(f.dof[3]), "v"(f.dof[4]), "v"(f.dof[5]), "v"(f.dof[6]),          \
+      "v"(f.dof[7]), "v"(f.ro.ptr[0]), "v"(f.ro.ptr[1]), "v"(f.ro.ptr[2]), "v"(f.ro.ptr[3]), "v"(f.ro.ptr[4]),          \
+      "v"(f.ro.ptr[5]), "v"(f.ro.ptr[6]), "v"(f.ro.ptr[7]), "v"(f.to.ptr[0][0]), "v"(f.to.ptr[0][1]),                   \
+      "v"(f.to.ptr[0][2]), "v"(f.to.ptr[0][3]), "v"(f.to.ptr[1][0]), "v"(f.to.ptr[1][1]), "v"(f.to.ptr[1][2]),          \
+      "v"(f.to.ptr[1][3]), "v"(f.lse2), "v"(f.delta), "s"(kLog2e), "i"(STAGE_OFF)
+  if constexpr (MASKED)
+    asm volatile(CT_DQ_STEP_MASKED_SEQUENCE
+                 : : CT_DQ_STEP_OPERANDS, "v"(allowed), "s"(kNegInf)
+                 : "memory", CT_DQ_STEP_SCRATCH, CT_DQ_ACCUMULATORS);
+  else
+    asm volatile(CT_DQ_STEP_SEQUENCE : : CT_DQ_STEP_OPERANDS : "memory", CT_DQ_STEP_SCRATCH, CT_DQ_ACCUMULATORS);
+#undef CT_DQ_STEP_OPERANDS
+}
+
+// The pairs of a tile whose key has the row's id, and those whose key is not behind `last_rel` (of the lane's half).
+template <int STAGE_OFF>
+CT_DEVICE unsigned dq_pairs_of_id(lds_addr ids, int id) {
+  unsigned allowed;
+  asm volatile(CT_DQ_IDS_SEQUENCE
+               : "=&v"(allowed) : "v"(ids), "v"(id), "i"(STAGE_OFF)
+               : "memory", "vcc", CT_DQ_STEP_SCRATCH, CT_DQ_ACCUMULATORS);
+  return allowed;
+}
+CT_DEVICE unsigned dq_pairs_up_to(int last_rel) {
+  const int count = min(max(last_rel >> 3, -1) * 4 + min((last_rel & 7) + 1, 4), 32);
+  return count <= 0 ? 0u : ~0u >> (32 - count);
+}
+
 // One query tile (4 / HS row blocks x HS heads of one KV head), start to finish.
 template <int D, int HS, int PER_UNIT>
 CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int qt, const lds_addr lds_base) {
@@ -62,8 +97,14 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
   // they end up spilled and reloaded in the key-tile loop)
   lds_addr lds0 = lds_base;
   asm volatile("" : "+v"(lds0));
-  const LeanRowFrags<D> ro(lds0);
-  const LeanTrFrags<D> to(lds0);
+  // (and for D = 128, whose item loop has no room for their shares of the lane either, from an opaque lane)
+  RowFragOffsets<D / 8> ro(lds0);
+  TrFragOffsets<D / 8, KSlots::kAccum> to(lds0);
+  if constexpr (D == 128) {
+    const int lane = lane_id_here();
+    ro = RowFragOffsets<D / 8>(lds0, lane);
+    to = TrFragOffsets<D / 8, KSlots::kAccum>(lds0, lane);
+  }
 
   const QueryTileContext<D, HS> ctx(p, b, kvh, slice, qt);
   const int l = lane_id(), half = l >> 5, w = threadIdx.x >> 6;
@@ -97,9 +138,13 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) qf[ks] = scale_bf16x8(qf[ks], p.scale);
   }
-  f32x16 dqacc[D / 32];
+  f32x16 dqacc[D / 32];  // (D = 128: in accumulation registers)
+  if constexpr (D == 128) {
+    asm volatile(CT_DQ_ZERO : : : CT_DQ_ACCUMULATORS);
+  } else {
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) dqacc[db] = zero16();
+    for (int db = 0; db < D / 32; ++db) dqacc[db] = zero16();
+  }
   dma_wait_all();
   __syncthreads();
 
@@ -156,26 +201,14 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
       if (k_uniform != 0 && seg_cmp != k_uniform) last_rel = -1;
       constexpr int kOff = CUR * kStage + KvStage<D>::kK, vOff = CUR * kStage + KvStage<D>::kV;
       if constexpr (D == 128) {
-        // The tile is worked in its two 32-key halves, each start to finish (S and dP, the
-        // arithmetic, the half's share of dQ): 32 score registers are live at a time instead of
-        // 64, which is what leaves room for the fragment ring of the hand-scheduled sequences
-        // without spilling registers inside this loop.
-        const RowFragOffsets<16> rp = RowFragOffsets<16>::expand(ro);
-        const TrFragOffsets<16, KSlots::kAccum> tp =
-            TrFragOffsets<16, KSlots::kAccum>::expand(TrFragCompact<16, KSlots::kAccum>(lds_base, lane_id_here()));
-        auto half_tile = [&](auto kb_tag) {
-          constexpr int KB = decltype(kb_tag)::value;
-          f32x16 s, dp;
-          dq_sdp_half_128<kOff + KB * 8192, vOff + KB * 8192>(rp, qf, dof, s, dp);
-          if (need_seg || need_causal) {
-            if (k_uniform == 0) mask_block_t<true, true>(stage + KvStage<D>::kSeg, seg_cmp, last_rel, KB, s);
-            else mask_block_t<false, true>(stage, seg_cmp, last_rel, KB, s);
-          }
-          dq_arith(s, dp, lse2, delta_q);
-          dq_acc_half_128<kOff + KB * 8192>(tp, pack_acc8(s, 0), pack_acc8(s, 1), dqacc);
-        };
-        half_tile(std::integral_constant<int, 0>{});
-        half_tile(std::integral_constant<int, 1>{});
+        const DqFrame f{ro, to, qf, dof, lse2, delta_q};
+        if (need_seg || need_causal) {
+          unsigned allowed = dq_pairs_up_to(last_rel);
+          if (k_uniform == 0) allowed &= dq_pairs_of_id<CUR * kStage>(lds0 + KvStage<D>::kSeg + 16 * half, seg_cmp);
+          dq_step_128<CUR * kStage, true>(f, allowed);
+        } else {
+          dq_step_128<CUR * kStage, false>(f, 0);
+        }
       } else {
         // Both 32-key blocks at once, or one after the other where registers are for three workgroups on a compute unit.
         // (dP starts from -delta, a register block of its own, and needs no subtraction)
@@ -227,7 +260,12 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
   if (ctx.active) {
     const lds_addr patch = lds0 + w * 32 * D * 2;
     bf16* gbase = p.dq + (((size_t)ctx.work.b * p.S + ctx.work.rb * 32) * p.Hq + ctx.work.h) * D;
-    store_rows_t<D>(dqacc, p.scale, patch, gbase, q_row_stride);
+    if constexpr (D == 128) {
+      asm volatile("s_nop 15\n\ts_nop 7" : : : "memory");  // the last sums leave the matrix pipe
+      fwd_store_rows(p.scale, patch, gbase, q_row_stride);
+    } else {
+      store_rows_t<D>(dqacc, p.scale, patch, gbase, q_row_stride);
+    }
   }
   // the store patches overlap the stages of the next item: its copies may start once every
   // wavefront has read its patch back

@@ -463,30 +463,6 @@ CT_DEVICE f32x16 fwd_acc_read() {
   return out;
 }
 
-// dQ kernel, one 32-key half of a key tile (see gen_attn_asm.py): S^T and dP^T of the half, and
-// the half's contribution to dQ^T. K_OFF / V_OFF are the byte offsets of the half's K and V rows.
-template <int K_OFF, int V_OFF>
-CT_DEVICE void dq_sdp_half_128(const RowFragOffsets<16>& ro, const bf16x8* qf, const bf16x8* dof, f32x16& s,
-                               f32x16& dp) {
-  asm volatile(CT_DQ_SDP_HALF_SEQUENCE
-               : "=&v"(s), "=&v"(dp)
-               : "v"(ro.ptr[0]), "v"(ro.ptr[1]), "v"(ro.ptr[2]), "v"(ro.ptr[3]), "v"(ro.ptr[4]),
-                 "v"(ro.ptr[5]), "v"(ro.ptr[6]), "v"(ro.ptr[7]), "v"(qf[0]), "v"(qf[1]), "v"(qf[2]),
-                 "v"(qf[3]), "v"(qf[4]), "v"(qf[5]), "v"(qf[6]), "v"(qf[7]), "v"(dof[0]), "v"(dof[1]),
-                 "v"(dof[2]), "v"(dof[3]), "v"(dof[4]), "v"(dof[5]), "v"(dof[6]), "v"(dof[7]), "i"(K_OFF),
-                 "i"(V_OFF)
-               : "memory", CT_ATTN_ASM_SCRATCH);
-}
-template <int K_OFF>
-CT_DEVICE void dq_acc_half_128(const TrFragOffsets<16, KSlots::kAccum>& to, bf16x8 p0, bf16x8 p1, f32x16* acc) {
-  asm volatile(CT_DQ_ACC_HALF_SEQUENCE
-               : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
-               : "v"(to.ptr[0][0]), "v"(to.ptr[0][1]), "v"(to.ptr[0][2]), "v"(to.ptr[0][3]),
-                 "v"(to.ptr[1][0]), "v"(to.ptr[1][1]), "v"(to.ptr[1][2]), "v"(to.ptr[1][3]), "v"(p0), "v"(p1),
-                 "i"(K_OFF)
-               : "memory", CT_ATTN_ASM_SCRATCH);
-}
-
 // ---------------------------------------------------------------------------
 // Forward
 //

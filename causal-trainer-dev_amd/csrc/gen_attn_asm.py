@@ -586,7 +586,7 @@ def dkv_step_sequence(mask, stores):
     return st.lines + ["s_setprio 0"]
 
 
-# (Dropping the issue priority for these sequences, as the dK/dV ones do, measured neutral here.)
+# dQ, the two halves of a key tile as two plain sequences each: the order of the sums that the stream below keeps.
 DQ_HEAD = ["s_waitcnt lgkmcnt(0)"]
 DQ_TAIL = TAIL
 
@@ -648,6 +648,105 @@ def dq_acc_half_sequence(ahead=4, slots=4):
         if i + ahead < n:
             lines += load(i + ahead)
     return lines + DQ_TAIL
+
+
+# dQ, a key tile of 64 keys as one stream: S and dP of its first half, S of the second with the first half's dS behind its
+# MFMAs, dP of the second, the first half's share of dQ with the second's dS behind it, the second's share. Fixed registers
+# (declared as clobbers): one temporary, three score blocks (S0, later dP1; dP0; S1; the first 8 registers of a dP block
+# later hold its bf16 dS fragments) and the fragment ring; the sums are a[0:63] for the whole query tile. (With the two
+# halves one after the other, each as two sequences with the arithmetic between them: [2, 8192, 16/16], documents of 64 to
+# 2000, the kernel 191 us, now 178; [2, 10496, 64/8] of 248 to 3277 1214 and 1095; whole rows of 16384, 8/1, 769 and 703;
+# [1, 6144, 4/4] of 100 to 600 38.3 and 31.9. Five or seven fragment slots and a raised issue priority, as in dK/dV, change nothing.)
+DQS_SLOTS = 6
+DQS_RING0 = 192 - 4 * DQS_SLOTS
+DQS_S = (DQS_RING0 - 48, DQS_RING0 - 16)
+DQS_DP = (DQS_RING0 - 32, DQS_RING0 - 48)
+DQS_TMP = DQS_RING0 - 49
+DQS_FIRST = DQS_TMP
+
+
+def dq_step_sequence(masked):
+    """operands: %0-%7 Q and %8-%15 dO fragments, %16-%23 row-fragment pointers, %24-%27 transposed fragments, lo, and
+    %28-%31, hi, %32 lse * log2(e), %33 delta of the lane's query row, %34 log2(e) (scalar), %35 byte offset of the stage (64 K
+    rows, 64 V rows 16384 later). With `masked` bit e of %36 tells whether the pair of element e (second half: 16 + e) is
+    allowed, and the score of one that is not becomes %37 (scalar).
+
+    Scalar loads may be in flight where the stream begins: its first wait is for everything, and no other counts them.
+    """
+    st = Stream(head=[])
+    stage = "%35"
+    block = lambda base: "v[%d:%d]" % (base, base + 15)
+
+    def slot(r):
+        lo = DQS_RING0 + 4 * (r % DQS_SLOTS)
+        return lo, "v[%d:%d]" % (lo, lo + 3)
+
+    reads, mfmas = [], []
+    for half in range(2):
+        for which, base in ((0, DQS_S[half]), (1, DQS_DP[half])):
+            for ks in range(8):
+                reads.append(["ds_read_b128 {v4}, %%%d offset:%s+%d" % (16 + ks, stage, 16384 * which + 8192 * half)])
+                mfmas.append("v_mfma_f32_32x32x16_bf16 %s, {r0}, %%%d, %s" % (block(base), 8 * which + ks, block(base) if ks else "0"))
+    for half in range(2):
+        for step in range(2):
+            for db in range(4):
+                off = "%s+%d" % (stage, 8192 * half + 4096 * step)
+                reads.append(["ds_read_b64_tr_b16 {v2lo}, %%%d offset:%s" % (24 + db, off),
+                              "ds_read_b64_tr_b16 {v2hi}, %%%d offset:%s" % (28 + db, off)])
+                source = DQS_DP[half] + 4 * step
+                mfmas.append("v_mfma_f32_32x32x16_bf16 %s, {r0}, v[%d:%d], %s" % (w_acc(db), source, source + 3, w_acc(db)))
+
+    # A product's scores are read two MFMAs after its last one at the earliest: they have left the matrix pipe by then.
+    fill = [[] for _ in mfmas]
+    for half in range(2):
+        S, DP = DQS_S[half], DQS_DP[half]
+        for e in range(16):
+            t = 9 + 16 * half + (e * 7) // 16
+            t_ds = 17 + (e * 7) // 16 if half == 0 else 33 + (e * 11) // 16
+            if masked:
+                fill[t] += ["v_bfe_i32 v%d, %%36, %d, 1" % (DQS_TMP, 16 * half + e),
+                            "v_bfi_b32 v%d, v%d, v%d, %%37" % (S + e, DQS_TMP, S + e)]
+            fill[t] += ["v_fma_f32 v%d, v%d, %%34, -%%32" % (S + e, S + e), "v_exp_f32_e32 v%d, v%d" % (S + e, S + e)]
+            fill[t_ds] += ["v_sub_f32_e32 v%d, v%d, %%33" % (DP + e, DP + e), "v_mul_f32_e32 v%d, v%d, v%d" % (DP + e, S + e, DP + e)]
+            if e % 2 == 1:
+                k = e // 2
+                fill[t_ds] += ["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (DP + k, DP + 2 * k, DP + 2 * k + 1)]
+
+    state = {"issued": 0, "consumed": 0}
+
+    def issue_reads():
+        while state["issued"] < min(len(reads), state["consumed"] + DQS_SLOTS):
+            r = state["issued"]
+            lo, v4 = slot(r)
+            for text in reads[r]:
+                st.lds(text.format(v4=v4, v2lo="v[%d:%d]" % (lo, lo + 1), v2hi="v[%d:%d]" % (lo + 2, lo + 3)), r)
+            state["issued"] += 1
+
+    issue_reads()
+    st.wait_all()
+    for i, text in enumerate(mfmas):
+        st.wait(i)
+        st.emit(text.format(r0=slot(i)[1]))
+        state["consumed"] += 1
+        issue_reads()
+        for line in fill[i]:
+            st.emit(line)
+    return st.lines
+
+
+def dq_ids_sequence():
+    """%0: bit e tells whether the id of element e's key is %2 (elements as in the stream above); %1 pointer of the lane's ids
+    (LDS address of the ids + 16 * (lane / 32)), %3 byte offset of the stage."""
+    lines = ["s_waitcnt lgkmcnt(0)"]
+    base = DQS_DP[1]
+    for q in range(8):
+        lines.append("ds_read_b128 v[%d:%d], %%1 offset:%%3+%d" % (base + 4 * q, base + 4 * q + 3, 32 * (7 - q)))
+    lines.append("v_mov_b32_e32 %0, 0")
+    for q in range(8):
+        lines.append("s_waitcnt lgkmcnt(%d)" % (7 - q))
+        for e in (3, 2, 1, 0):
+            lines += ["v_cmp_eq_u32_e32 vcc, %%2, v%d" % (base + 4 * q + e), "v_addc_co_u32_e32 %0, vcc, %0, %0, vcc"]
+    return lines
 
 
 # ---------------------------------------------------------------------------
@@ -859,7 +958,7 @@ def dkvw_run_sequence():
     return lines + TAIL
 
 
-def dkv_zero(registers):
+def accumulators_zero(registers):
     return ["v_accvgpr_write_b32 a%d, 0" % r for r in range(registers)]
 
 
@@ -870,14 +969,17 @@ def dkvw_read():
 
 def clobbers():
     regs = ", ".join('"v%d"' % r for r in range(SCRATCH0, SCRATCH0 + 16))
+    dq = ", ".join('"v%d"' % r for r in range(DQS_FIRST, 192))
+    dq_accs = ", ".join('"a%d"' % r for r in range(64))
     step = ", ".join('"v%d"' % r for r in range(DKVS_P, 128))
     step_accs = ", ".join('"a%d"' % r for r in range(128))
     wide = ", ".join('"v%d"' % r for r in range(W_FIRST, 256))
     accs = ", ".join('"a%d"' % r for r in range(256))
-    return ("#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DKV_STEP_SCRATCH %s\n\n"
+    return ("#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DQ_STEP_SCRATCH %s\n\n#define CT_DQ_ACCUMULATORS %s\n\n"
+            "#define CT_DKV_STEP_SCRATCH %s\n\n"
             "#define CT_DKV_ACCUMULATORS %s\n\n"
             "#define CT_DKVW_ASM_SCRATCH %s\n\n"
-            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (regs, step, step_accs, wide, accs,
+            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (regs, dq, dq_accs, step, step_accs, wide, accs,
                                                                              fwd_private_clobbers()))
 
 
@@ -890,15 +992,17 @@ if __name__ == "__main__":
             print(emit(lines, "CT_FWD_%s_%s" % (name, cur.upper())))
     for name, lines in fwd_accumulator_statements().items():
         print(emit(lines, "CT_FWD_ACC_%s" % name))
-    print(emit(dq_sdp_half_sequence(), "CT_DQ_SDP_HALF_SEQUENCE"))
-    print(emit(dq_acc_half_sequence(), "CT_DQ_ACC_HALF_SEQUENCE"))
+    print(emit(dq_step_sequence(False), "CT_DQ_STEP_SEQUENCE"))
+    print(emit(dq_step_sequence(True), "CT_DQ_STEP_MASKED_SEQUENCE"))
+    print(emit(dq_ids_sequence(), "CT_DQ_IDS_SEQUENCE"))
+    print(emit(accumulators_zero(64), "CT_DQ_ZERO"))
     for mask in ("", "ends", "rows"):
         for stores in (False, True):
             print(emit(dkv_step_sequence(mask, stores), "CT_DKV_STEP_%s%sSEQUENCE" % (mask.upper() + "_" * bool(mask), "STORE_" * stores)))
-    print(emit(dkv_zero(128), "CT_DKV_ZERO"))
+    print(emit(accumulators_zero(128), "CT_DKV_ZERO"))
     print(emit(dkvw_step_sequence(), "CT_DKVW_FAST_SEQUENCE"))
     print(emit(dkvw_step_sequence(masked=True), "CT_DKVW_MASKED_SEQUENCE"))
     print(emit(dkvw_run_sequence(), "CT_DKVW_RUN_SEQUENCE"))
-    print(emit(dkv_zero(256), "CT_DKVW_ZERO"))
+    print(emit(accumulators_zero(256), "CT_DKVW_ZERO"))
     print(emit(dkvw_read(), "CT_DKVW_READ"))
     print(clobbers())

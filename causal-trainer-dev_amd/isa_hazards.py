@@ -109,7 +109,7 @@ def scan(assembly: str) -> list[str]:
 
 def private_accumulators(assembly: str, kernel: str) -> list[str]:
     """Checks a kernel that keeps values in accumulation registers across inline-assembly
-    statements without telling the compiler (attn_dkv_wide_kernel, attn_dkv_kernel of 128): outside those statements the
+    statements without telling the compiler (attn_dkv_wide_kernel, attn_dkv_kernel and attn_dq_kernel of 128): outside those statements the
     compiler must not touch an accumulation register (it would, to park a spilled vector register
     there), and no spilled register may be reloaded between the kernel's first and last workgroup
     barrier, i.e. inside its item loop, where the wait for the reload also waits for every
@@ -260,7 +260,8 @@ def scan_library() -> dict[str, list[str]]:
     findings = {path.name: scan(text) for path, text in zip(sources, texts)}
     for path, text in zip(sources, texts):
         if path.name == "ct_attn.hip":
-            for kernel in ("attn_dkv_wide_kernel", "attn_dkv_kernelILi128ELb0E", "attn_dkv_kernelILi128ELb1E"):
+            for kernel in ("attn_dkv_wide_kernel", "attn_dkv_kernelILi128ELb0E", "attn_dkv_kernelILi128ELb1E",
+                           "attn_dq_kernelILi128ELi1E", "attn_dq_kernelILi128ELi2E", "attn_dq_kernelILi128ELi4E"):
                 findings[path.name] += private_accumulators(text, kernel)
             for heads in (1, 2, 4):
                 findings[path.name] += private_registers(text, f"attn_fwd_kernelILi128ELi{heads}E", 112, 191)

@@ -109,6 +109,9 @@ def _sequences(gen):
     for mask in ("", "ends", "rows"):
         for stores in (False, True):
             sequences["dkv_step_%s_%s" % (mask, stores)] = gen.dkv_step_sequence(mask, stores)
+    for masked in (False, True):
+        sequences["dq_step_%s" % masked] = gen.dq_step_sequence(masked)
+    sequences["dq_ids"] = gen.dq_ids_sequence()
     for cur in ("a", "b"):
         for name, lines in gen.fwd_statements(cur).items():
             sequences["fwd_%s_%s" % (name.lower(), cur)] = lines
@@ -231,6 +234,69 @@ def test_dkv_step_stream(gen, mask, stores):
     assert [ops[1] for _, ops in stored] == ([block(dp0, 4), block(dp0 + 4, 4)] if stores else [])
     for n, (i, _) in enumerate(stored):
         assert i > position["v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (dp0 + 4 * n + 3, dp0 + 8 * n + 6, dp0 + 8 * n + 7)]
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_dq_step_stream(gen, masked):
+    """One key tile of the dQ kernel: the MFMAs of every sum in the order of the two half sequences, the arithmetic of every
+    element between its products and the sums that need it, no block written before its last reader."""
+
+    lines = gen.dq_step_sequence(masked)
+    block = lambda base, n: "v[%d:%d]" % (base, base + n - 1)
+    mfmas = [(i, _split(line)[1]) for i, line in enumerate(lines) if line.startswith("v_mfma")]
+    assert len(mfmas) == 48
+    for db in range(4):
+        sums = [ops for _, ops in mfmas if ops[0] == gen.w_acc(db)]
+        assert [ops[2] for ops in sums] == [block(gen.DQS_DP[half] + 4 * step, 4) for half in range(2) for step in range(2)]
+        assert all(ops[3] == ops[0] for ops in sums)
+    at = {}
+    for half in range(2):
+        for base, operands in ((gen.DQS_S[half], ["%%%d" % ks for ks in range(8)]), (gen.DQS_DP[half], ["%%%d" % (8 + ks) for ks in range(8)])):
+            chain = [(i, ops) for i, ops in mfmas if ops[0] == block(base, 16) and ops[2] in operands]
+            assert [ops[2] for _, ops in chain] == operands and [ops[3] for _, ops in chain] == ["0"] + [block(base, 16)] * 7
+            at[base, operands[0]] = (chain[0][0], chain[-1][0])
+    find = lambda line, first: next(i for i in range(first, len(lines)) if lines[i] == line)
+    for half in range(2):
+        S, DP = gen.DQS_S[half], gen.DQS_DP[half]
+        s_done, dp_first, dp_done = at[S, "%0"][1], at[DP, "%8"][0], at[DP, "%8"][1]
+        for e in range(16):
+            s, dp, k = S + e, DP + e, e // 2
+            scaled = find("v_fma_f32 v%d, v%d, %%34, -%%32" % (s, s), s_done)
+            exp2 = find("v_exp_f32_e32 v%d, v%d" % (s, s), scaled)
+            less = find("v_sub_f32_e32 v%d, v%d, %%33" % (dp, dp), dp_done)
+            ds = find("v_mul_f32_e32 v%d, v%d, v%d" % (dp, s, dp), less)
+            pack = find("v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (DP + k, DP + 2 * k, DP + 2 * k + 1), ds)
+            assert exp2 < less and pack < min(i for i, ops in mfmas if ops[2] == block(DP + 4 * (e // 8), 4) and i > dp_done)
+            # an even element packed by its pair's instruction overwrites nothing that is still to be read
+            assert find("v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (DP + k // 2, DP + 2 * (k // 2), DP + 2 * (k // 2) + 1), dp_done) <= pack
+            if masked:
+                bit = find("v_bfe_i32 v%d, %%36, %d, 1" % (gen.DQS_TMP, 16 * half + e), s_done)
+                assert bit + 2 == scaled and lines[bit + 1] == "v_bfi_b32 v%d, v%d, v%d, %%37" % (s, gen.DQS_TMP, s)
+            if half == 0:   # dP of the second half takes the place of S of the first
+                assert gen.DQS_DP[1] == gen.DQS_S[0] and ds < at[gen.DQS_DP[1], "%8"][0]
+    assert next(line for line in lines if "lgkmcnt" in line) == "s_waitcnt lgkmcnt(0)"
+
+
+def test_dq_bits_of_ids(gen):
+    """The statement on a model of the id ring: bit e is the comparison with the id of key 8 (e / 4) + 4 half + e % 4."""
+
+    for half in (0, 1):
+        registers, compared = {}, None
+        bits = []
+        for line in gen.dq_ids_sequence():
+            name, operands = _split(line)
+            if name == "ds_read_b128":
+                offset = int(line.split("offset:%3+")[1])
+                for e, register in enumerate(sorted(_registers(operands[0]))):
+                    registers[register] = 4 * half + offset // 4 + e
+            elif name == "v_cmp_eq_u32_e32":
+                assert operands[:2] == ["vcc", "%2"]
+                (register,) = _registers(operands[2])
+                compared = registers[register]
+            elif name == "v_addc_co_u32_e32":
+                assert operands == ["%0", "vcc", "%0", "%0", "vcc"]
+                bits.insert(0, compared)     # shifted in from below
+        assert bits == [8 * (e // 4) + 4 * half + e % 4 for e in range(32)]
 
 
 def _vector_alu(lines):
