@@ -755,8 +755,8 @@ static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduc
   CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_blocks_kernel<D, HS, KS>), smem);
   const int groups = p.Hq / p.Hkv / HS * p.kvh_count;
   const int grid = KS == 1 ? dq_grid(p, HS) : groups * p.B * bin_tiles_per_row(p.S / 32, kDqbWaves / KS / HS);
-  reduce = reduce && KS > 1;
-  const int reduce_groups = reduce ? 128 : 0;
+  reduce = reduce && (KS > 1 || p.ds_most_blocks);
+  const int reduce_groups = !reduce ? 0 : KS > 1 ? 128 : 512;
   LaunchScope scope("attn_dq_blocks_kernel", stream);
   hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS, KS>), dim3(grid + reduce_groups), dim3(kDqbWaves * 64), smem, stream, p, reduce_groups);
   return scope.done();
@@ -771,12 +771,15 @@ static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduc
 //   2880, D = 64: 34 / 19 / 29                 8928, D = 64: 248 / 248
 //   3744, D = 128: 124 / 102 / 127, but 2.5 us slower by two with short documents (a compute unit holds one of its
 //   workgroups, of the others two); 7680: 201 / 227
+// Stored blocks that were chosen for their small number (most_stored_blocks) are shared by two up to 10240 row blocks, as the
+// walks are short: the backward, D = 64, by one / two, [11, 384, 64/16], 8448, documents of 16 to 64, 92 / 84 us, of 128 to 192
+// 97 / 92; [22, 768, 16/4], 8448, 256 to 384, 109 / 110; [32, 768, 16/4], 12288, 145 / 149, 16 to 64 97 / 98; 24576: 193 / 208.
 template <int D>
 static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
   const long blocks = (long)p.B * p.kvh_count * (p.Hq / p.Hkv) * (p.S / 32);
   const int hs = heads_per_group(p.Hq, p.Hkv);
   if (blocks <= 768) return hs == 1 ? launch_dq_blocks<D, 1, 4>(stream, p, reduce) : launch_dq_blocks<D, 2, 4>(stream, p, reduce);
-  if (blocks <= (D == 64 ? 8192 : 3072))
+  if (blocks <= (D == 128 ? 3072 : p.ds_most_blocks ? 10240 : 8192))
     return hs == 4   ? launch_dq_blocks<D, 4, 2>(stream, p, reduce)
            : hs == 2 ? launch_dq_blocks<D, 2, 2>(stream, p, reduce)
                      : launch_dq_blocks<D, 1, 2>(stream, p, reduce);
@@ -805,6 +808,13 @@ static int launch_dkv(hipStream_t stream, const AttnParams& p, bool wide) {
     }
   }
   LaunchScope scope3("attn_dkv_kernel", stream);
+  if constexpr (D == 64) {
+    if (p.ds_most_blocks) {
+      CT_ENSURE_LDS("ct_attn_bwd", &attn_dkv_choice_kernel<D>, smem);
+      hipLaunchKernelGGL(attn_dkv_choice_kernel<D>, dim3(grid), dim3(256), smem, stream, p);
+      return scope3.done();
+    }
+  }
   if (p.ds) {
     CT_ENSURE_LDS("ct_attn_bwd", (&attn_dkv_kernel<D, true>), smem);
     hipLaunchKernelGGL((attn_dkv_kernel<D, true>), dim3(grid), dim3(256), smem, stream, p);
@@ -843,22 +853,42 @@ static int launch_schedule(hipStream_t stream, const AttnParams& p, int kvh_side
 // Recompute form: the work list; dQ per query tile (evaluates S and dP itself and computes delta
 // and -lse / scale for its rows on the way); dK/dV per key tile; the sum of split chunks.
 template <int D>
+static int dispatch_dq(hipStream_t stream, const AttnParams& p) {
+  switch (heads_per_group(p.Hq, p.Hkv)) {
+    case 4: return launch_dq<D, 4>(stream, p);
+    case 2: return launch_dq<D, 2>(stream, p);
+    default: return launch_dq<D, 1>(stream, p);
+  }
+}
+
+template <int D>
 static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool wide, bool list_kept) {
   int rc = list_kept ? 0 : launch_schedule<D>(stream, p, p.Hkv);
   if (rc) return rc;
-  switch (heads_per_group(p.Hq, p.Hkv)) {
-    case 4: rc = launch_dq<D, 4>(stream, p); break;
-    case 2: rc = launch_dq<D, 2>(stream, p); break;
-    default: rc = launch_dq<D, 1>(stream, p); break;
-  }
+  rc = dispatch_dq<D>(stream, p);
   if (rc) return rc;
   rc = launch_dkv<D>(stream, p, wide);
   if (rc) return rc;
   return launch_dkv_reduce<D>(stream, p);
 }
 
+// The most dS blocks per query head with which dQ comes from stored blocks, 0 where the form is settled (see kDqRecomputes).
+// Up to 8192 row blocks stored ones are ahead with all but the longest documents and the sums ride with their dQ already, so that
+// the recomputing kernel's launch would be lost. Beyond, recomputing is ahead from about 42000 blocks (of all heads) and 2.3 per
+// row block on, sooner per row block the larger the launch. Backward in us, stored / this / recomputing (head dimension 64):
+//   [3, 1536, 64/16]  9216 row blocks, documents of 16 to 64 93 / 90 / 103, of 512 to 768 165 / 152 / 149, whole rows 323 / 260 / 257
+//   [4, 4096, 64/16] 32768, 16 to 64 261 / 263 / 269, 1365 to 2048 875 / 690 / 702, whole rows 2475 / 1826 / 1826
+//   [12, 4096, 8/8] 12288, whole rows 1028 / 732 / 736, image blocks 596 / 445 / 473
+// Over 70 shapes of 8200 to 61000 row blocks: short documents 0.93 to 1.02 of the stored form's time, long ones 0.71 to 0.9.
+static int most_stored_blocks(const AttnParams& p, int head_dim) {
+  const long rows = (long)p.B * p.Hq * (p.S / 32);
+  if (head_dim != 64 || rows <= 8192 || p.Hq / heads_per_group(p.Hq, p.Hkv) > kChoiceCounters) return 0;
+  return (int)((42000 + 2.3 * rows) / p.Hq);
+}
+
 // Stored-dS form: row statistics and the work list; then per pass of KV heads the dK/dV kernel, which
-// leaves its dS blocks in the region, and dQ as a product over those blocks; the sum of split chunks.
+// leaves its dS blocks in the region, and dQ as a product over those blocks; the sum of split chunks. With p.ds_most_blocks the
+// recomputing dQ stands between the first two, and forms the statistics, where the header asks for it.
 template <int D>
 static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pass, bool wide, bool list_kept) {
   const long tiles = (long)p.B * p.Hq * (p.S / (D == 128 ? 64 : 128));
@@ -875,6 +905,10 @@ static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pas
     rc = scope.done();
   }
   if (rc) return rc;
+  if constexpr (D == 64) {
+    if (p.ds_most_blocks) rc = dispatch_dq<D>(stream, p);
+    if (rc) return rc;
+  }
   bool reduced = false;
   for (int base = 0; base < p.Hkv; base += kvh_per_pass) {
     p.kvh_base = base;
@@ -1111,6 +1145,7 @@ extern "C" int32_t ct_attn_bwd(void* stream, const ct_attn_bwd_args* a) {
   if (plan.spill) {
     p.ds = ws + plan.ds;
     p.ds_row_blocks = plan.row_blocks;
+    if (path_choice == 0) p.ds_most_blocks = most_stored_blocks(p, a->head_dim);
     return a->head_dim == 128 ? dispatch_bwd_blocks<128>(s, p, plan.kvh_per_pass, false, list_kept)
                               : dispatch_bwd_blocks<64>(s, p, plan.kvh_per_pass, false, list_kept);
   }

@@ -19,6 +19,21 @@
 namespace ct {
 
 // ---------------------------------------------------------------------------
+// The form of dQ by the number of dS blocks (kDqRecomputes)
+// ---------------------------------------------------------------------------
+// dS blocks of one query head, all batch rows. (Per row: where the last key block's start and how many it has.)
+CT_DEVICE int ds_blocks_per_head(const AttnParams& p) {
+  const int nrb = p.S / 32;
+  int blocks = 0;
+  for (int b = lane_id(); b < p.B; b += 64) {
+    const int* last = p.meta + ((size_t)b * nrb + nrb - 1) * kMetaW;
+    blocks += last[kDsOff] + max(last[kQLast] - last[kQFirst] + 1, 0);
+  }
+  return lane_value(wave_scan(blocks), 63);
+}
+CT_DEVICE bool dq_recomputes(const AttnParams& p) { return uniform(p.dkv_header[kDqRecomputes]) != 0; }
+
+// ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
 // The dK/dV kernels work on unscaled Q K^T and put the softmax scale into the exponent. Any finite
@@ -289,6 +304,7 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
 template <int D, int HS, int PER_UNIT>
 __global__ __launch_bounds__(256, PER_UNIT) void attn_dq_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
+  if (D == 64 && p.ds_most_blocks && !dq_recomputes(p)) return;
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
   constexpr int PB = 4 / HS;
@@ -773,11 +789,14 @@ __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, i
 // two costs nothing.
 template <int D>
 __global__ __launch_bounds__(1024) void attn_bwd_setup_kernel(AttnParams p, int kvh_side_by_side, float exponent_scale) {
+  const bool recompute = p.ds_most_blocks && ds_blocks_per_head(p) > p.ds_most_blocks;
   if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) p.dkv_header[kDqRecomputes] = recompute;
     dkv_schedule<D>(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
                  p.dkv_entries, p.dq_counters, kDqCounters);
     return;
   }
+  if (recompute) return;  // (that dQ kernel forms the statistics on its way)
   bwd_stats_tiles<D>(p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale,
                      (blockIdx.x - 1) * 4 + (threadIdx.x >> 8), (gridDim.x - 1) * 4, threadIdx.x & 255);
 }
@@ -821,7 +840,7 @@ CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceL
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
   if (group == 0)
-    for (int i = threadIdx.x; i < kDqCounters; i += 64 * WAVES) p.dq_counters[i] = 0;
+    for (int i = threadIdx.x; i < (p.ds_most_blocks ? kChoiceCounters : kDqCounters); i += 64 * WAVES) p.dq_counters[i] = 0;
   const int entries = uniform(p.dkv_header[0]);
   int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
   for (int base = 0; base < entries; base += 256 * WAVES) {
@@ -938,9 +957,7 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
 // [2, 15616, 12/2 heads of 64] 544 -> 445 us, [1, 7424, 6/1] 95 -> 80. Its fragments are read ahead of the products
 // (fragments_ahead): [1, 25472, 64/8], image blocks, 1800 -> 1690; the dQ kernel above likewise, 1280 -> 1190.
 template <int D, bool SPILL>
-__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnParams p) {
-  extern __shared__ __align__(16) char smem_raw[];
-  const lds_addr lds0 = lds_address_of(smem_raw);
+CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   constexpr int kStage = QdoStage<D>::kBytes;
 
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
@@ -1192,6 +1209,23 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
   store_rows<D>(dkacc, patch, p.dk + out_off, kv_row_stride);
   __builtin_amdgcn_wave_barrier();
   store_rows<D>(dvacc, patch, p.dv + out_off, kv_row_stride);
+}
+
+template <int D, bool SPILL>
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  dkv_entry<D, SPILL>(p, lds_address_of(smem_raw));
+}
+
+// With the stores or without them, as the header says. (Two kernels, one of them to exit at once, would be one more launch; with
+// both bodies in one a few scalar registers and 12 bytes of scratch a lane go to what the loops do not use.)
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_choice_kernel(AttnParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  if (blockIdx.x == 0)  // (dQ's own of the stored blocks, whose launch also ends the call)
+    for (int i = threadIdx.x; i < kChoiceCounters; i += 256) p.dq_counters[kChoiceCounters + i] = 0;
+  if (dq_recomputes(p)) dkv_entry<D, false>(p, lds_address_of(smem_raw));
+  else dkv_entry<D, true>(p, lds_address_of(smem_raw));
 }
 
 // ---------------------------------------------------------------------------
@@ -1475,10 +1509,13 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
 // dK/dV kernel left and write different tensors, and a workgroup per tile leaves room for the other one where its tiles
 // are light: a launch and, in small calls, most of the sums' time less. (The pulling form, KS = 1, fills the device to
 // the end; there the sums have the device to themselves afterwards.) It uses no work counters.
+// Under a choice of the form (kDqRecomputes) they ride with KS = 1 as well, by as many wavefronts as in a launch of their own: either
+// the tiles' workgroups exit at once, or the documents are short and few key tiles are split. That is the launch that the other
+// dQ kernel costs. The counters are another half there, for the sums clear the first one.
 template <int D, int HS, int KS>
 __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p, int reduce_groups) {
   extern __shared__ __align__(16) char smem_raw[];
-  if constexpr (KS > 1) {
+  if constexpr (KS > 1 || D == 64) {
     typedef DkvReduceLds<kDqbWaves> ReduceLds;
     static_assert(sizeof(ReduceLds) <= DsStage<D, KS>::kTotalBytes, "the sums' list and patches fit");
     const int group = (int)blockIdx.x - ((int)gridDim.x - reduce_groups);
@@ -1487,6 +1524,7 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
       return;
     }
   }
+  if (D == 64 && p.ds_most_blocks && dq_recomputes(p)) return;
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
   using Stage = DsStage<D, KS>;
@@ -1494,12 +1532,13 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
   const int nrb = p.S / 32;
   const int slices = (p.Hq / p.Hkv) / HS;
   const int groups = slices * p.kvh_count;
-  const int group = blockIdx.x % groups, member = blockIdx.x / groups, members = gridDim.x / groups;
+  const int group = blockIdx.x % groups, member = blockIdx.x / groups, members = (gridDim.x - reduce_groups) / groups;
   const int kvh = p.kvh_base + group % p.kvh_count, slice = group / p.kvh_count;
   const int tpr = bin_tiles_per_row(nrb, PB);
   const int total = p.B * tpr;
   const MetaPtr sched = meta_const(p.sched + query_schedule_offset(nrb, PB));
-  const bool dynamic = slices * p.Hkv <= kDqCounters;
+  const bool dynamic = slices * p.Hkv <= kDqCounters;  // (under a choice no more groups than kChoiceCounters)
+  int* counters = p.dq_counters + (D == 64 && p.ds_most_blocks ? kChoiceCounters : 0);
   const typename Stage::KDma kdma((size_t)p.Hkv * D * 2);
   const int w = threadIdx.x >> 6;
   const DsFragPtrs frags(lds0 + (Stage::kDs + w * Stage::kPatch), lane_id());
@@ -1511,7 +1550,7 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
   }
   for (int pull = member;; pull += members) {
     if (dynamic) {
-      if (threadIdx.x == 0) next_pull = atomicAdd(&p.dq_counters[slice * p.Hkv + kvh], 1);
+      if (threadIdx.x == 0) next_pull = atomicAdd(&counters[slice * p.Hkv + kvh], 1);
       __syncthreads();
       pull = uniform(next_pull);
       __syncthreads();

@@ -54,7 +54,8 @@ struct AttnParams {
   // dK/dV work list (backward only)
   int* dkv_header;
   int2* dkv_entries;
-  int* dq_counters;  // kDqCounters ints, zeroed by the work-list kernel and with the sums that end a call
+  int* dq_counters;  // kDqCounters ints, zeroed by the work-list kernel and with the sums that end a call (under a choice of
+                     // the form the second half, which the stored form's dQ uses, by the dK/dV kernel in front of it)
   float* dkv_partials;
   int dkv_max_entries, dkv_max_partials;
   // KV heads [kvh_base, kvh_base + kvh_count) are what a backward launch works on (all of them
@@ -62,7 +63,15 @@ struct AttnParams {
   int kvh_base, kvh_count;
   char* ds;              // dS region of the pass, null when dQ recomputes S and dP
   size_t ds_row_blocks;  // dS blocks reserved per (query head, batch row)
+  int ds_most_blocks;    // head dimension 64: with more dS blocks per query head than this dQ recomputes after all; 0: no such choice
 };
+
+// Whether dQ of head dimension 64 is the faster one from stored dS blocks or recomputed goes by how many blocks there are:
+// stored ones save launches and products and cost 4 KB of traffic each. The documents decide that, which the host does not
+// know, so where it matters (most_stored_blocks) the kernel that makes the work list counts the blocks and leaves the answer in
+// the list's header; both dQ kernels are launched, and the workgroups of the one that is not wanted exit at once.
+constexpr int kDqRecomputes = 2;  // place in the header
+constexpr int kChoiceCounters = kDqCounters / 2;  // work counters of each of the two dQ kernels
 
 // ---------------------------------------------------------------------------
 // K/V tile staging: global -> registers -> swizzled LDS.
@@ -1110,6 +1119,7 @@ CT_DEVICE void bwd_stats_tiles(const bf16* out, const bf16* dout, const float* l
 
 template <int D>
 __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(AttnParams p, float exponent_scale) {
+  if (D == 64 && p.ds_most_blocks && p.dkv_header[kDqRecomputes]) return;
   bwd_stats_tiles<D>(p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale, blockIdx.x, gridDim.x,
                      threadIdx.x);
 }

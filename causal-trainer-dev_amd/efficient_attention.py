@@ -203,7 +203,7 @@ def efficient_attention(query, key, value, metadata, *, mesh=None, profile=None,
     query ``[B, S, Hq, D]``, key / value ``[B, S, Hkv, D]``, all bf16 on a ROCm
     device; returns ``[B, S, Hq, D]`` bf16. Gradients flow to query, key, value.
     Its backward takes dQ from stored dS blocks (up to 4 GiB of scratch): rows of up to 4096 positions, longer ones at
-    head dimension 128 or with few query rows. Where the device has no room for the blocks it recomputes instead.
+    head dimension 128 or with few query rows; large calls at head dimension 64 only while the documents are short. Where the device has no room for the blocks it recomputes instead.
     ``backward_workspace`` (this build's addition, a :class:`BackwardWorkspace`) lets the layers of
     a model that share ``metadata`` share the scratch buffer of the backward and the work list in it.
     """
@@ -267,7 +267,8 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     kernel or a form of the backward for this call (``ct_attn_bwd_args.variant``); ``None`` leaves
     the choice to the library, which is what training code does (the dK/dV kernel goes by sequence
     length; dQ comes from stored dS blocks at rows of up to 4096 positions when their workspace is at
-    most 4 GiB, and from a recomputing kernel otherwise). ``workspace_bytes`` overrides the size of the scratch buffer (default: what
+    most 4 GiB, and from a recomputing kernel otherwise; from 8193 row blocks of head dimension 64 on, the
+    documents decide between the two on the device). ``workspace_bytes`` overrides the size of the scratch buffer (default: what
     the library asks for the chosen form); ``workspace`` (a :class:`BackwardWorkspace`) keeps the
     buffer, and with it the dK/dV work list, from one call to the next."""
 

@@ -151,15 +151,17 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * pair and head; needs ct_attn_bwd_workspace_bytes_from_ds. Left open (0): FROM_DS for
  * rows of at most CT_ATTN_FROM_DS_UP_TO_SEQ positions if the caller's workspace holds the dS blocks of all KV heads
  * (workspace_bytes >= ct_attn_bwd_workspace_bytes_from_ds and that size is the one-pass size),
- * else RECOMPUTE: a caller chooses by the workspace it offers. All give the same results within
+ * else RECOMPUTE: a caller chooses by the workspace it offers. At head dimension 64 that offer is taken up to 8192
+ * row blocks (32 query rows of one head); in larger launches the batch's number of dS blocks decides on the device
+ * between the two forms, in the same workspace. All give the same results within
  * the operator's tolerances (not bitwise: summation orders differ).
  * Measured, backward in us, RECOMPUTE / FROM_DS. Head dimension 128: [4, 4096, 32/8 heads] with documents of
  * 64..4096 positions 703 / 670, whole rows 1831 / 1731; 0.96 to 1.18 times over rows of 1024 to 4096; [1, 32768, 64/8]
  * 26405 / 26749 and whole rows 52877 / 61723 (eight passes), [1, 32768, 8/2] 3631 / 3082.
- * Head dimension 64 at up to 4096 positions: 0.98 to 1.14 times for launches of up to 2048 row blocks (32 query rows
- * of one head); beyond, ahead with short documents only ([4, 4096, 16/4], 8192 row blocks: documents of 16..128
- * positions 105 / 92, of 64..4096 246 / 276, whole rows 550 / 715). The line looks at the row length alone: a caller
- * with such launches offers the small workspace, or asks for RECOMPUTE. */
+ * Head dimension 64 at up to 4096 positions: FROM_DS is ahead up to 2048 row blocks, 1.0 to 1.5 times; from there to
+ * 8192 with short documents only ([4, 4096, 16/4], 8192 row blocks: documents of 16..64 positions 88 / 78, of
+ * 1365..2048 211 / 259, whole rows 510 / 693), and a caller with long ones offers the small workspace or asks for
+ * RECOMPUTE. */
 #define CT_ATTN_FROM_DS_UP_TO_SEQ 4096
 #define CT_ATTN_BWD_DKV_NARROW 1
 #define CT_ATTN_BWD_DKV_WIDE 2

@@ -394,6 +394,38 @@ def test_form_of_the_operators_backward(ct, gpu, shape, form):
         assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
 
 
+@pytest.mark.parametrize("shape,chooses", [
+    ((4, 1024, 64, 16), False), ((129, 128, 16, 8), True), ((4, 1152, 64, 16), True), ((3, 1536, 96, 96), True),
+    ((5, 1280, 64, 64), True), ((1, 1152, 256, 256), False)], ids=lambda v: "" if isinstance(v, bool) else "B%d_S%d_Hq%d_Hkv%d" % v)
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_form_by_the_number_of_blocks(ct, gpu, shape, chooses, with_ends):
+    """Head dimension 64, from 8193 row blocks on (and up to 224 groups of heads): few dS blocks are stored, many are not,
+    where the documents decide. The recomputing form shows by its bits; stored blocks may be added in another order, and
+    then differ from it and from the pinned form by bf16 roundings. The work list and the answer in it are kept."""
+
+    batch, seq, q_heads, kv_heads = shape
+    generator = torch.Generator(device=gpu).manual_seed(seq)
+    q, k, v, dout = (torch.randn((batch, seq, heads, 64), generator=generator, device=gpu).to(torch.bfloat16)
+                     for heads in (q_heads, kv_heads, kv_heads, q_heads))
+    kept = ct.BackwardWorkspace()
+    rng = np.random.default_rng(batch)
+    for longest in (24, None, 24):
+        ids = np.ones((batch, seq), np.int32) if longest is None else _layout(rng, batch, seq, holes=True, max_len=longest)
+        ends = torch.from_numpy(_random_ends(rng, ids)).to(gpu) if with_ends else None
+        profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=with_ends)
+        metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile, attention_end=ends)
+        out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+        call = lambda **form: ct.attention_backward(q, k, v, metadata, out, lse, dout, **form)  # noqa: E731
+        recomputed, stored, chosen = call(dq_form="recompute"), call(dq_form="from_ds"), call()
+        recomputes = chooses and longest is None and seq > 128
+        same = [torch.equal(a, b) for a, b in zip(chosen, recomputed if recomputes else stored)]
+        assert same[1] and same[2] and (same[0] or not recomputes)
+        assert torch.equal(chosen[0], recomputed[0]) == recomputes
+        assert float((chosen[0].float() - stored[0].float()).norm() / stored[0].float().norm()) <= 1e-2   # bf16 results of bf16 dS
+        for _ in range(2):                      # (the list is built, then kept)
+            assert all(torch.equal(a, b) for a, b in zip(call(workspace=kept), chosen))
+
+
 @pytest.mark.parametrize("seq,q_heads", [(8192, 8), (4096, 32)])
 def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     """The operator's own choice of the stored-dS form gives way to the recomputing form where the allocator has no room
