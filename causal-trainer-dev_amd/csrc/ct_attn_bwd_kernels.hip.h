@@ -963,15 +963,38 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
   const int kvh = p.kvh_base + blockIdx.x % p.kvh_count, entry = blockIdx.x / p.kvh_count;
-  if (entry >= uniform(p.dkv_header[0])) return;
+  // The way to the first products is a chain of memory round trips: the list's length and the entry (the grid is the list's
+  // room, so it can be read whatever the length is), the tile's bounds beside its K and V rows, the first copies beside their
+  // way into fragments. One after the other, and K and V by instructions that touch 32 rows each, the kernel took, us,
+  // [3, 640, 12/2 heads of 128] 20.9 for 19.5, [4, 1792, 4/4] 26.7 for 25.2, [2, 2432, 16/16] 65.3 for 64.2, [4, 4096, 32/8],
+  // documents of 64 to 300, 121.6 for 120.5, [8, 1152, 32/32 of 64], 16 to 64, 54.7 for 53.4.
   const int2 work_entry = p.dkv_entries[entry];
-  const int tile = uniform(work_entry.x), packed = uniform(work_entry.y);
+  int tile = uniform(work_entry.x), packed = uniform(work_entry.y);
+  asm volatile("" : "+s"(tile), "+s"(packed));
+  if (entry >= uniform(p.dkv_header[0])) return;
   const int chunk = packed & 255, nsplit = (packed >> 8) & 255, slot0 = (unsigned)packed >> 16;
   const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
   const int g = p.Hq / p.Hkv;
   const int* meta_b = p.meta + (size_t)b * nrb * kMetaW;
   const RowFragOffsets<D / 8> ro(lds0);
   const TrFragOffsets<D / 8, KSlots::kAccum> to(lds0);
+
+  const int my_rb = kt * 4 + w;
+  const int key = my_rb * 32 + j;
+  const int seg_k = p.seg[(size_t)b * p.S + key];
+  const bool has_end = p.end != nullptr;
+  const size_t kv_row_stride = (size_t)p.Hkv * D;
+  const size_t kv_off = (((size_t)b * p.S + my_rb * 32) * p.Hkv + kvh) * D;
+  // (V at D = 64 directly, for the addresses at which it is stored: they stay for the loop's reads. Without them the compiler
+  // forms them in every step, and the kernel is 4 % slower with long documents.)
+  RowBlockLoader<D> k_rows, v_rows;
+  k_rows.request(p.k + kv_off, kv_row_stride);
+  if constexpr (D == 128) {
+    v_rows.request(p.v + kv_off, kv_row_stride);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) v_rows.raw[ks] = load_global16(p.v + kv_off + j * kv_row_stride + 16 * ks + 8 * half);
+  }
 
   int q_lo = INT_MAX, q_hi = -1;
 #pragma unroll
@@ -983,30 +1006,17 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   // (the extremes of several come out of the vector unit, and what is selected and added by them would stay there)
   q_lo = uniform(q_lo);
   q_hi = uniform(q_hi);
-  const int my_rb = kt * 4 + w;
   const int my_min = uniform(meta_const(meta_b)[my_rb * kMetaW + kMinNz]);
   const int my_max = uniform(meta_const(meta_b)[my_rb * kMetaW + kMaxId]);
   const int my_uni = uniform(meta_const(meta_b)[my_rb * kMetaW + kUniform]);
   const int my_q_first = uniform(meta_const(meta_b)[my_rb * kMetaW + kQFirst]);
   const int my_ds_off = uniform(meta_const(meta_b)[my_rb * kMetaW + kDsOff]);
 
-  const int key = my_rb * 32 + j;
-  const int seg_k = p.seg[(size_t)b * p.S + key];
-  const bool has_end = p.end != nullptr;
-  const size_t kv_row_stride = (size_t)p.Hkv * D;
-  const size_t kv_off = (((size_t)b * p.S + key) * p.Hkv + kvh) * D;
-
   // K fragments stay in registers; V fragments are parked in LDS (this wavefront's
   // private 32-row patch) and re-read per block, which keeps the kernel under 256
   // registers so that two workgroups share a CU.
   const int vpatch_off = QdoStage<D>::kVResident + w * 32 * D * 2;
   const lds_addr vpatch = lds0 + vpatch_off;
-  bf16x8 kf[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    kf[ks] = as_bf16x8(load_global16(p.k + kv_off + 16 * ks + 8 * half));
-    lds_store<u32x4>(ro.addr(vpatch_off, 0, ks), load_global16(p.v + kv_off + 16 * ks + 8 * half));
-  }
   f32x16 dkacc[D / 32], dvacc[D / 32];  // (D = 128: in accumulation registers until the end)
   if constexpr (D == 128) {
     asm volatile(CT_DKV_ZERO : : : CT_DKV_ACCUMULATORS);
@@ -1017,12 +1027,6 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
       dvacc[db] = zero16();
     }
   }
-
-  // Make the K fragment loads complete here. Left pending, their first use inside the item
-  // loop gets an `s_waitcnt vmcnt(n)` whose count fits the first item only; on every later item
-  // the same wait stalls until the asynchronous copies of the next stage have landed.
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) asm volatile("" : "+v"(kf[ks]));
 
   // The Q tiles stay unscaled in LDS: the softmax scale enters the exponent in f32
   // (S = scale * (Q K^T); the forward rounded scale * Q to bf16 first, a difference of one
@@ -1038,10 +1042,21 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   const TileDma<kQueryTile, D / 8> dma((size_t)p.Hq * D * 2);
   // (a chunk without items: an address inside the arrays all the same)
   QdoCursor<D> next(p, b, uniform(kvh * g + (it < items ? it / nq : 0)), uniform(it < items ? q_lo + it % nq : 0), q_lo, q_hi, w);
-  if (it < items) {
-    next.fetch(dma, lds0, w);
-    dma_wait_all();
+  if (it < items) next.fetch(dma, lds0, w);
+  // Make the K fragment loads complete here. Left pending, their first use inside the item
+  // loop gets an `s_waitcnt vmcnt(n)` whose count fits the first item only; on every later item
+  // the same wait stalls until the asynchronous copies of the next stage have landed.
+  bf16x8 kf[D / 16];
+  k_rows.to_fragments(vpatch, kf);
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) asm volatile("" : "+v"(kf[ks]));
+  if constexpr (D == 128) {
+    v_rows.to_patch(vpatch);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) lds_store<u32x4>(ro.addr(vpatch_off, 0, ks), v_rows.raw[ks]);
   }
+  dma_wait_all();
   __syncthreads();
 
   QueryBlockBounds qb_bounds = next.query_bounds();

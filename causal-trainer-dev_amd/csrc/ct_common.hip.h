@@ -332,13 +332,17 @@ struct RowBlockLoader {
   }
   // (LDS operations of one wavefront complete in order: the reads see the writes, and the next
   // block's writes come after these reads)
-  template <class Fragment>
-  CT_DEVICE void to_fragments(lds_addr patch, Fragment* fragments) {
+  CT_DEVICE void to_patch(lds_addr patch) const {
     const int l = lane_id_here();
 #pragma unroll
     for (int n = 0; n < kLoads; ++n)
       lds_store<u32x4>(patch + tile_byte_offset<CPR>(l / CPR + n * kRowsPerLoad, l % CPR), raw[n]);
     __builtin_amdgcn_wave_barrier();
+  }
+  template <class Fragment>
+  CT_DEVICE void to_fragments(lds_addr patch, Fragment* fragments) {
+    const int l = lane_id_here();
+    to_patch(patch);
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks)
       fragments[ks] = lds_load<Fragment>(patch + tile_byte_offset<CPR>(l & 31, 2 * ks + (l >> 5)));
