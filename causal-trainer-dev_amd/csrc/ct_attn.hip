@@ -719,12 +719,16 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   }
 }
 
-// Workgroups of the persistent dQ kernels: 64 or 96 per (head slice, KV head) group, two or three per compute
-// unit when there are 8 groups; more per group when a pass has fewer groups than that.
+// Workgroups of the persistent dQ kernels: two or three per compute unit, the same number for every (head slice, KV head) group.
+// Where the groups do not share the places evenly some have a member less at first, and members behind the places go on with
+// those groups' tiles as places come free: up to twice as many, 64 or 96 a group at most. (That many for any number of groups were
+// up to 6144 workgroups, which still had to be started when all tiles were taken. dQ, us, so / now: [3, 5632, 24/8 heads of 64],
+// documents of 64 to 300, 79 / 72; [3, 1536, 64/64 of 64] whole rows 129 / 123; from stored blocks [2, 4096, 36/12 of 128], 16 to
+// 100, 42 / 36, [8, 768, 64/8 of 64] 53 / 48. No further members at all: [4, 5760, 48/16 of 128] 337 / 349, with them 344.)
 static int dq_grid(const AttnParams& p, int hs, int per_unit = 2) {
   const int groups = ((p.Hq / p.Hkv) / hs) * p.kvh_count;
-  const int members = groups >= 8 ? per_unit * kBins : (per_unit * kBins * 8 + groups - 1) / groups;
-  return groups * members;
+  const int places = per_unit * kBins * 8, members = (places + groups - 1) / groups;
+  return groups * (places % groups == 0 ? members : std::min(2 * members, std::max(members, per_unit * kBins)));
 }
 
 template <int D, int HS, int PER_UNIT>
