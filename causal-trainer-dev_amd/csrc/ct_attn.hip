@@ -747,19 +747,19 @@ static int launch_dq(hipStream_t stream, const AttnParams& p) {
   return launch_dq<D, HS, 2>(stream, p);
 }
 
-// `reduce`: the launch also adds the chunks of split key tiles, where its form can (KS > 1), by 128 workgroups of eight
-// wavefronts. There can be many more pieces than these 1024 wavefronts (17408 at [1, 3072, 32/32 of 128]), which then take several
-// each beside the tiles. A pass, us, with the sums in a launch of their own / by 128 / by 256: [2, 1024, 8/8 of 64], whole rows,
+// `reduce`: the launch also adds the chunks of split key tiles. Beside a workgroup per tile (KS > 1) by 128 workgroups of eight
+// wavefronts: there can be many more pieces than these 1024 wavefronts (17408 at [1, 3072, 32/32 of 128]), which then take several
+// each. A pass, us, with the sums in a launch of their own / by 128 / by 256: [2, 1024, 8/8 of 64], whole rows,
 // 40.7 / 38.0 / 37.5; [1, 2304, 6/1 of 64], documents of 256 to 900, 39.6 / 38.7 / 34.3; [1, 2688, 16/16 of 64], whole rows,
 // 91.6 / 87.4 / 88.0; [4, 1792, 16/8 of 64] 153.5 / 152.6 / 148.5; [1, 3072, 32/32 of 128] 311 / 306 / 301; [2, 1536, 8/2 of
 // 128], documents of 32 to 128, 46.1 / 41.4 / 42.3. Over 33 calls of 64 to 8192 row blocks 0.88 to 1.01 of their own launch.
+// Behind workgroups that pull tiles (KS = 1) by 512, as many wavefronts as a launch of their own has (attn_dq_blocks_kernel).
 template <int D, int HS, int KS>
-static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
+static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool reduce) {
   const size_t smem = DsStage<D, KS>::kTotalBytes;
   CT_ENSURE_LDS("ct_attn_bwd", (&attn_dq_blocks_kernel<D, HS, KS>), smem);
   const int groups = p.Hq / p.Hkv / HS * p.kvh_count;
   const int grid = KS == 1 ? dq_grid(p, HS) : groups * p.B * bin_tiles_per_row(p.S / 32, kDqbWaves / KS / HS);
-  reduce = reduce && (KS > 1 || p.ds_most_blocks);
   const int reduce_groups = !reduce ? 0 : KS > 1 ? 128 : 512;
   LaunchScope scope("attn_dq_blocks_kernel", stream);
   hipLaunchKernelGGL((attn_dq_blocks_kernel<D, HS, KS>), dim3(grid + reduce_groups), dim3(kDqbWaves * 64), smem, stream, p, reduce_groups);
@@ -779,7 +779,7 @@ static int launch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduc
 // walks are short: the backward, D = 64, by one / two, [11, 384, 64/16], 8448, documents of 16 to 64, 92 / 84 us, of 128 to 192
 // 97 / 92; [22, 768, 16/4], 8448, 256 to 384, 109 / 110; [32, 768, 16/4], 12288, 145 / 149, 16 to 64 97 / 98; 24576: 193 / 208.
 template <int D>
-static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool& reduce) {
+static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool reduce) {
   const long blocks = (long)p.B * p.kvh_count * (p.Hq / p.Hkv) * (p.S / 32);
   const int hs = heads_per_group(p.Hq, p.Hkv);
   if (blocks <= 768) return hs == 1 ? launch_dq_blocks<D, 1, 4>(stream, p, reduce) : launch_dq_blocks<D, 2, 4>(stream, p, reduce);
@@ -886,7 +886,7 @@ static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool 
 // Over 70 shapes of 8200 to 61000 row blocks: short documents 0.93 to 1.02 of the stored form's time, long ones 0.71 to 0.9.
 static int most_stored_blocks(const AttnParams& p, int head_dim) {
   const long rows = (long)p.B * p.Hq * (p.S / 32);
-  if (head_dim != 64 || rows <= 8192 || p.Hq / heads_per_group(p.Hq, p.Hkv) > kChoiceCounters) return 0;
+  if (head_dim != 64 || rows <= 8192) return 0;
   return (int)((42000 + 2.3 * rows) / p.Hq);
 }
 
@@ -913,17 +913,16 @@ static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pas
     if (p.ds_most_blocks) rc = dispatch_dq<D>(stream, p);
     if (rc) return rc;
   }
-  bool reduced = false;
   for (int base = 0; base < p.Hkv; base += kvh_per_pass) {
     p.kvh_base = base;
     p.kvh_count = min(kvh_per_pass, p.Hkv - base);
     rc = launch_dkv<D>(stream, p, wide);
     if (rc) return rc;
-    reduced = base + p.kvh_count == p.Hkv;  // with the last pass all chunks are there
-    rc = dispatch_dq_blocks<D>(stream, p, reduced);
+    // (with the last pass all chunks are there)
+    rc = dispatch_dq_blocks<D>(stream, p, base + p.kvh_count == p.Hkv);
     if (rc) return rc;
   }
-  return reduced ? CT_OK : launch_dkv_reduce<D>(stream, p);
+  return CT_OK;
 }
 
 }  // namespace ct

@@ -831,7 +831,7 @@ struct DkvReduceLds {
   __align__(16) bf16 patches[WAVES][32 * 32];
 };
 // Workgroup `group` of `groups`, WAVES wavefronts each (four or eight). Every backward call ends with a launch that does this, and
-// it leaves the dQ kernels' work counters at zero, so that a later call on the same workspace can keep the work list and skip
+// it leaves the recomputing dQ kernel's work counters at zero, so that a later call on the same workspace can keep the work list and skip
 // the kernel that builds it (and clears the counters). Nothing in such a launch uses them; an earlier pass of the call may have.
 template <int D, int WAVES>
 CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceLds<WAVES>& lds) {
@@ -840,7 +840,7 @@ CT_DEVICE void dkv_reduce(const AttnParams& p, int group, int groups, DkvReduceL
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
   const int nrb = p.S / 32;
   if (group == 0)
-    for (int i = threadIdx.x; i < (p.ds_most_blocks ? kChoiceCounters : kDqCounters); i += 64 * WAVES) p.dq_counters[i] = 0;
+    for (int i = threadIdx.x; i < kDqCounters; i += 64 * WAVES) p.dq_counters[i] = 0;
   const int entries = uniform(p.dkv_header[0]);
   int tiles = 0;  // split tiles found, in list order (the same in every workgroup)
   for (int base = 0; base < entries; base += 256 * WAVES) {
@@ -958,6 +958,8 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
 // (fragments_ahead): [1, 25472, 64/8], image blocks, 1800 -> 1690; the dQ kernel above likewise, 1280 -> 1190.
 template <int D, bool SPILL>
 CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
+  if (SPILL && blockIdx.x == 0)  // work counters of the dQ kernel that reads the blocks
+    for (int i = threadIdx.x; i < kDqCounters; i += 256) p.dq_counters[kDqCounters + i] = 0;
   constexpr int kStage = QdoStage<D>::kBytes;
 
   const int l = lane_id(), j = l & 31, half = l >> 5, w = uniform(threadIdx.x >> 6);
@@ -1237,8 +1239,6 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_choice_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
-  if (blockIdx.x == 0)  // (dQ's own of the stored blocks, whose launch also ends the call)
-    for (int i = threadIdx.x; i < kChoiceCounters; i += 256) p.dq_counters[kChoiceCounters + i] = 0;
   if (dq_recomputes(p)) dkv_entry<D, false>(p, lds_address_of(smem_raw));
   else dkv_entry<D, true>(p, lds_address_of(smem_raw));
 }
@@ -1520,17 +1520,16 @@ CT_DEVICE void attn_dq_blocks_item(const AttnParams& p, int b, int kvh, int slic
   }
 }
 
-// KS > 1: the last reduce_groups workgroups add the chunks of split key tiles (dkv_reduce). The two passes read what the
-// dK/dV kernel left and write different tensors, and a workgroup per tile leaves room for the other one where its tiles
-// are light: a launch and, in small calls, most of the sums' time less. (The pulling form, KS = 1, fills the device to
-// the end; there the sums have the device to themselves afterwards.) It uses no work counters.
-// Under a choice of the form (kDqRecomputes) they ride with KS = 1 as well, by as many wavefronts as in a launch of their own: either
-// the tiles' workgroups exit at once, or the documents are short and few key tiles are split. That is the launch that the other
-// dQ kernel costs. The counters are another half there, for the sums clear the first one.
+// The last reduce_groups workgroups add the chunks of split key tiles (dkv_reduce). The two passes read what the dK/dV kernel
+// left and write different tensors; the sums are few bytes a place and take the places that tiles leave free: where a workgroup
+// has one tile (KS > 1) beside them, where the workgroups pull tiles (KS = 1) when the first of those end. Both in launches of
+// their own / in this one, us: [4, 4096, 32/8 heads of 128], documents of 64 to 4096, 203 + 15 / 206, [2, 10496, 12/4], 248 to
+// 3277, 81 + 18 / 86, [4, 4096, 8/1] 90 + 19 / 93, [2, 8192, 16/16], 64 to 2000, 100 + 5 / 100. The sums clear the recomputing
+// kernel's work counters, so this kernel has counters of its own.
 template <int D, int HS, int KS>
 __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnParams p, int reduce_groups) {
   extern __shared__ __align__(16) char smem_raw[];
-  if constexpr (KS > 1 || D == 64) {
+  {
     typedef DkvReduceLds<kDqbWaves> ReduceLds;
     static_assert(sizeof(ReduceLds) <= DsStage<D, KS>::kTotalBytes, "the sums' list and patches fit");
     const int group = (int)blockIdx.x - ((int)gridDim.x - reduce_groups);
@@ -1552,8 +1551,8 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
   const int tpr = bin_tiles_per_row(nrb, PB);
   const int total = p.B * tpr;
   const MetaPtr sched = meta_const(p.sched + query_schedule_offset(nrb, PB));
-  const bool dynamic = slices * p.Hkv <= kDqCounters;  // (under a choice no more groups than kChoiceCounters)
-  int* counters = p.dq_counters + (D == 64 && p.ds_most_blocks ? kChoiceCounters : 0);
+  const bool dynamic = slices * p.Hkv <= kDqCounters;
+  int* counters = p.dq_counters + kDqCounters;
   const typename Stage::KDma kdma((size_t)p.Hkv * D * 2);
   const int w = threadIdx.x >> 6;
   const DsFragPtrs frags(lds0 + (Stage::kDs + w * Stage::kPatch), lane_id());

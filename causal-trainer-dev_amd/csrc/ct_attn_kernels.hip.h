@@ -54,8 +54,8 @@ struct AttnParams {
   // dK/dV work list (backward only)
   int* dkv_header;
   int2* dkv_entries;
-  int* dq_counters;  // kDqCounters ints, zeroed by the work-list kernel and with the sums that end a call (under a choice of
-                     // the form the second half, which the stored form's dQ uses, by the dK/dV kernel in front of it)
+  int* dq_counters;  // kDqCounters ints of the recomputing kernel, zeroed by the work-list kernel and with the sums that end a
+                     // call, then as many of the one from stored blocks, zeroed by the dK/dV kernel in front of it
   float* dkv_partials;
   int dkv_max_entries, dkv_max_partials;
   // KV heads [kvh_base, kvh_base + kvh_count) are what a backward launch works on (all of them
@@ -71,7 +71,6 @@ struct AttnParams {
 // know, so where it matters (most_stored_blocks) the kernel that makes the work list counts the blocks and leaves the answer in
 // the list's header; both dQ kernels are launched, and the workgroups of the one that is not wanted exit at once.
 constexpr int kDqRecomputes = 2;  // place in the header
-constexpr int kChoiceCounters = kDqCounters / 2;  // work counters of each of the two dQ kernels
 
 // ---------------------------------------------------------------------------
 // K/V tile staging: global -> registers -> swizzled LDS.

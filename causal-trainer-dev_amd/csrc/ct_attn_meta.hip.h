@@ -137,7 +137,7 @@ constexpr int kDkvMinChunk = 16;
 constexpr int kDkvMaxSplit = 32;
 constexpr int kDkvKeys = 128;      // keys per dK/dV tile
 
-constexpr int kDqCounters = 448;  // one per (head slice, KV head) group of the dQ kernel
+constexpr int kDqCounters = 448;  // of each of the two dQ kernels: one per (head slice, KV head) group
 
 struct DkvLayout {
   int max_entries, max_partials;
@@ -153,8 +153,8 @@ __host__ inline DkvLayout dkv_layout(int B, int S, int Hq, int Hkv, int D, int k
   L.max_entries = tiles + extra;
   L.max_partials = min(2 * extra, L.max_entries);
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-  L.header = 0;  // 64 ints of dK/dV list header, then kDqCounters work counters of the dQ kernel
-  L.entries = (64 + kDqCounters) * sizeof(int);
+  L.header = 0;  // 64 ints of dK/dV list header, then the work counters of the two dQ kernels
+  L.entries = (64 + 2 * kDqCounters) * sizeof(int);
   // -lse / scale, head-major [B, Hq, S] (the caller's delta scratch holds -delta the same way)
   L.lse2 = L.entries + up((size_t)L.max_entries * 2 * sizeof(int));
   L.partials = L.lse2 + up((size_t)B * S * Hq * sizeof(float));

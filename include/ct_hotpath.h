@@ -172,7 +172,7 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * (same tile_meta, shape, variant and workspace size) can keep the list. With this flag the call
  * does not build it: the head of `workspace` must be as the previous ct_attn_bwd call on this
  * workspace left it (every call leaves the list in place and, whatever the forms of its passes, the
- * work counters of the dQ kernels at zero). Saves a launch and 0.01 ms per call of the recomputing
+ * work counters of the dQ kernels as the next call needs them). Saves a launch and 0.01 ms per call of the recomputing
  * form, and in the stored-dS form the list's share of the launch that also forms the row statistics
  * (up to 7 us of small launches); anything else in the workspace may be overwritten between the calls. */
 #define CT_ATTN_BWD_WORK_LIST_KEPT 0x100

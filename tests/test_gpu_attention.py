@@ -396,11 +396,11 @@ def test_form_of_the_operators_backward(ct, gpu, shape, form):
 
 @pytest.mark.parametrize("shape,chooses", [
     ((4, 1024, 64, 16), False), ((129, 128, 16, 8), True), ((4, 1152, 64, 16), True), ((3, 1536, 96, 96), True),
-    ((5, 1280, 64, 64), True), ((1, 1152, 256, 256), False)], ids=lambda v: "" if isinstance(v, bool) else "B%d_S%d_Hq%d_Hkv%d" % v)
+    ((5, 1280, 64, 64), True), ((1, 1152, 480, 480), True)], ids=lambda v: "" if isinstance(v, bool) else "B%d_S%d_Hq%d_Hkv%d" % v)
 @pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
 def test_form_by_the_number_of_blocks(ct, gpu, shape, chooses, with_ends):
-    """Head dimension 64, from 8193 row blocks on (and up to 224 groups of heads): few dS blocks are stored, many are not,
-    where the documents decide. The recomputing form shows by its bits; stored blocks may be added in another order, and
+    """Head dimension 64, from 8193 row blocks on (the last shape has more groups of heads than work counters): few dS
+    blocks are stored, many are not, as the documents decide. The recomputing form shows by its bits; stored blocks may be added in another order, and
     then differ from it and from the pinned form by bf16 roundings. The work list and the answer in it are kept."""
 
     batch, seq, q_heads, kv_heads = shape
