@@ -274,11 +274,12 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_backward(const Tensor& q, c
 // that form where it is the faster one and its workspace is at most 4 GiB. It saves the two products that the
 // recomputing dQ kernel repeats and pays 2 KB written and read per block. Measured over rows of 4224 to 25600
 // positions with documents from 16 positions to the whole row, recomputing / stored:
-//   head dimension 128: 0.98 to 1.39, below 1 only by noise, at every length whose blocks fit
-//     ([1, 7424, 6/1 heads] 297 / 254 us, [2, 8192, 8/8] 107 / 90, [1, 16384, 8/8] 174 / 144, [1, 25600, 4/4] 448 / 389).
+//   head dimension 128: 0.95 to 1.2, below 1 with documents of thousands of positions at up to 8000 row blocks only
+//     ([3, 6144, 8/8 heads] documents of 16 to 64 112 / 95 us, of 64 to 6144 396 / 416, whole rows 728 / 734; [6, 10240, 8/8] 100 to
+//     400 428 / 377, whole rows 3749 / 3662).
 //   head dimension 64: a block's products are half as long and its traffic the same. Launches of few row blocks (32
-//     query rows of one head) gain, 0.99 to 1.18 up to 1400 of them ([1, 7424, 6/1] 189 / 167); with 2048 whole-row
-//     documents lose (0.84 at [1, 16384, 4/1]), with 4096 most long ones (0.75 to 0.91).
+//     query rows of one head) gain, up to 1400 of them ([1, 7424, 6/1], images, 159 / 115; [1, 5376, 6/2] 126 / 85); with 2048
+//     whole-row documents lose (0.84 at [1, 16384, 4/1]), with 4096 most long ones (0.75 to 0.91).
 int operator_form(const AttnShape& s, bool with_ends) {
   if (s.seq <= CT_ATTN_FROM_DS_UP_TO_SEQ) return 0;
   const bool pays = s.head_dim == 128 ? s.seq <= 32768

@@ -156,8 +156,9 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * between the two forms, in the same workspace. All give the same results within
  * the operator's tolerances (not bitwise: summation orders differ).
  * Measured, backward in us, RECOMPUTE / FROM_DS. Head dimension 128: [4, 4096, 32/8 heads] with documents of
- * 64..4096 positions 703 / 670, whole rows 1831 / 1731; 0.96 to 1.18 times over rows of 1024 to 4096; [1, 32768, 64/8]
- * 26405 / 26749 and whole rows 52877 / 61723 (eight passes), [1, 32768, 8/2] 3631 / 3082.
+ * 64..4096 positions 652 / 643, of 100..400 343 / 321, whole rows 1672 / 1685; over rows of 1536 to 10240 positions 1.0 to
+ * 1.4 times with documents of up to some hundred positions, 0.93 to 1.06 with long ones and whole rows; [1, 32768, 64/8],
+ * measured before both forms' kernels became faster, whole rows 52877 / 61723 (eight passes).
  * Head dimension 64 at up to 4096 positions: FROM_DS is ahead up to 2048 row blocks, 1.0 to 1.5 times; from there to
  * 8192 with short documents only ([4, 4096, 16/4], 8192 row blocks: documents of 16..64 positions 88 / 78, of
  * 1365..2048 211 / 259, whole rows 510 / 693), and a caller with long ones offers the small workspace or asks for
