@@ -702,7 +702,8 @@ def dq_step_sequence(masked):
         S, DP = DQS_S[half], DQS_DP[half]
         for e in range(16):
             t = 9 + 16 * half + (e * 7) // 16
-            t_ds = 17 + (e * 7) // 16 if half == 0 else 33 + (e * 11) // 16
+            # (the last pair is packed behind MFMA 42 and read by MFMA 44: what lies between are the two wait states that it takes)
+            t_ds = 17 + (e * 7) // 16 if half == 0 else 33 + (e * 10) // 16
             if masked:
                 fill[t] += ["v_bfe_i32 v%d, %%36, %d, 1" % (DQS_TMP, 16 * half + e),
                             "v_bfi_b32 v%d, v%d, v%d, %%37" % (S + e, DQS_TMP, S + e)]

@@ -1,4 +1,4 @@
-"""Static check of the compiled kernels for one hazard the compiler does not cover.
+"""Static check of the compiled kernels for hazards that the compiler does not cover in ``asm`` statements.
 
 On gfx9-family hardware a memory instruction that reads a scalar register needs 5 wait states
 after a vector instruction wrote that register (v_readfirstlane, v_readlane, carries, compares).
@@ -9,7 +9,9 @@ pair held before. ``scan`` walks device assembly (``hipcc -S --cuda-device-only`
 every memory instruction whose scalar operands were written by a vector instruction fewer than
 5 wait states earlier. It also reports the second hazard of that kind: a store of more than 8 bytes
 reads its data registers late, and a vector instruction that writes one of them within 2 wait
-states of the store replaces the data on its way out. ``python -m causal_trainer_dev_amd.isa_hazards`` compiles every source of
+states of the store replaces the data on its way out. And a third: an MFMA reads its operands without a look at vector
+instructions that are still under way, so 2 wait states lie between the write of a register and the MFMA that reads it
+(``fresh_operands``). ``python -m causal_trainer_dev_amd.isa_hazards`` compiles every source of
 the library and scans it; tests/test_isa_hazards.py runs the same on the CPU.
 """
 
@@ -24,6 +26,7 @@ from pathlib import Path
 
 WAIT_STATES = 5
 STORE_DATA_WAIT_STATES = 2
+MFMA_OPERAND_WAIT_STATES = 2
 _WIDE_STORE = re.compile(r"^\s*(global|buffer|flat|scratch)_store_dwordx[34]\s+(.*)")
 _VECTOR_ALU = re.compile(r"^\s*v_\w+\s+(.*)")
 _MEMORY = re.compile(r"^\s*(global_|buffer_|flat_|scratch_)")
@@ -51,6 +54,32 @@ def _vector_registers(text: str) -> set:
     for match in re.finditer(r"(?<![\w\[])v(\d+)\b", text):
         found.add(int(match.group(1)))
     return found
+
+
+def _registers(text: str) -> set:
+    """Vector, accumulation and scalar registers as ("v", 7), and "vcc"."""
+
+    found = {(kind, register) for kind, low, high in re.findall(r"\b([vas])\[(\d+):(\d+)\]", text)
+             for register in range(int(low), int(high) + 1)}
+    found.update((kind, int(register)) for kind, register in re.findall(r"(?<![\w\[])([vas])(\d+)\b", text))
+    if re.search(r"\bvcc\b", text):
+        found.add("vcc")
+    return found
+
+
+# (what a carry, a scaled division or an exchange writes besides its first operand is its second one)
+_TWO_RESULTS = re.compile(r"v_(add_co|sub_co|subrev_co|addc|subb|div_scale|mad_[ui]64|swap|permlane\d+_swap)")
+_RESULT_IS_OPERAND = re.compile(r"v_(fmac|mac|swap|permlane\d+_swap|dot\w*c_)")
+
+
+def _results_and_operands(text: str) -> tuple[set, set]:
+    """Registers that a vector instruction writes and reads."""
+
+    mnemonic, _, rest = text.partition(" ")
+    fields = rest.split(";")[0].split(",")
+    results = 2 if _TWO_RESULTS.match(mnemonic) else 1
+    written, read = _registers(",".join(fields[:results])), _registers(",".join(fields[results:]))
+    return written, read | written if _RESULT_IS_OPERAND.match(mnemonic) else read
 
 
 def _wait_states(line: str) -> int:
@@ -105,6 +134,48 @@ def scan(assembly: str) -> list[str]:
         if len(window) > 16:
             del window[0]
     return problems
+
+
+def fresh_operands(assembly: str) -> list[str]:
+    """One message per vector instruction that reads what another one wrote too few wait states before. Also takes the lines
+    of an asm statement with operands such as %3 in them, which count as registers that nothing writes."""
+
+    problems, window, kernel = [], [], "?"
+    for number, line in enumerate(assembly.splitlines(), start=1):
+        text = line.strip()
+        label = _LABEL.match(text)
+        if label:
+            if not text.startswith(".L"):
+                kernel = label.group(1)
+            continue
+        if not text or text.startswith((";", ".")):
+            continue
+        if text.startswith(("s_branch", "s_endpgm", "s_setpc")):
+            window = []        # what follows is reached from elsewhere
+            continue
+        if text.startswith("v_"):
+            written, read = _results_and_operands(text)
+            elapsed = 0
+            for earlier_number, earlier, results in reversed(window):
+                needed = _wait_states_between(earlier, results & read, text)
+                if elapsed < needed:
+                    problems.append(f"{kernel}: line {number} '{text}' reads what line {earlier_number} '{earlier}' wrote "
+                                    f"{elapsed} wait states earlier, needs {needed}")
+                    break
+                elapsed += _wait_states(earlier)
+        else:
+            written = set()
+        window = window[-7:] + [(number, text, written)]
+    return problems
+
+
+def _wait_states_between(writer: str, registers: set, reader: str) -> int:
+    """Wait states that the compiler keeps between two vector instructions, `registers` passing from one to the other."""
+
+    vectors = any(register[0] in "va" for register in registers if register != "vcc")
+    if vectors and reader.startswith("v_mfma") and not writer.startswith("v_mfma"):
+        return MFMA_OPERAND_WAIT_STATES
+    return 0
 
 
 def private_accumulators(assembly: str, kernel: str) -> list[str]:
@@ -257,7 +328,7 @@ def scan_library() -> dict[str, list[str]]:
     sources = [recipe.CSRC / name for name in recipe.SOURCES]
     with ThreadPoolExecutor(max_workers=4) as pool:
         texts = list(pool.map(lambda path: device_assembly(path, recipe.HIP_FLAGS), sources))
-    findings = {path.name: scan(text) for path, text in zip(sources, texts)}
+    findings = {path.name: scan(text) + fresh_operands(text) for path, text in zip(sources, texts)}
     for path, text in zip(sources, texts):
         if path.name == "ct_attn.hip":
             for kernel in ("attn_dkv_wide_kernel", "attn_dkv_kernelILi128ELb0E", "attn_dkv_kernelILi128ELb1E",

@@ -1,5 +1,6 @@
 """The compiled kernels must not read a scalar register in a memory instruction fewer than
-5 wait states after a vector instruction wrote it (the compiler does not pad inline asm)."""
+5 wait states after a vector instruction wrote it, nor an MFMA operand fewer than 2 after it was
+written (the compiler does not pad inline asm)."""
 
 import shutil
 
@@ -48,6 +49,26 @@ kernel_e:
     assert isa_hazards.scan(wide.replace("\tv_accvgpr", "\ts_nop 1\n\tv_accvgpr")) == []
     assert isa_hazards.scan(wide.replace("v3, a17", "v9, a17")) == []
     assert isa_hazards.scan(wide.replace("dwordx4 v252, v[2:5]", "dwordx2 v252, v[2:3]")) == []
+
+
+def test_scanner_flags_fresh_mfma_operands(ct):
+    from causal_trainer_dev_amd import isa_hazards
+
+    packed = """
+kernel_a:
+	v_cvt_pk_bf16_f32 v127, v134, v135
+	s_waitcnt lgkmcnt(6)
+	v_mfma_f32_32x32x16_bf16 a[0:15], v[176:179], v[124:127], a[0:15]
+"""
+    assert len(isa_hazards.fresh_operands(packed)) == 1
+    assert isa_hazards.fresh_operands(packed.replace("\tv_mfma", "\ts_nop 0\n\tv_mfma")) == []
+    assert isa_hazards.fresh_operands(packed.replace("\tv_mfma", "\ts_branch .LBB0_1\n.LBB0_2:\n\tv_mfma")) == []
+    assert isa_hazards.fresh_operands(packed.replace("v127, v134", "v123, v134")) == []
+    cleared = "kernel_b:\n\tv_accvgpr_write_b32 a3, 0\n\tv_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[8:11], a[0:15]\n"
+    assert len(isa_hazards.fresh_operands(cleared)) == 1
+    # (one MFMA into the next one's sums is the matrix pipe's own affair)
+    chained = "kernel_c:\n" + "\tv_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[8:11], a[0:15]\n" * 2
+    assert isa_hazards.fresh_operands(chained) == []
 
 
 def test_private_accumulator_check(ct):
