@@ -96,7 +96,7 @@ CT_DEVICE unsigned dq_pairs_of_id(lds_addr ids, int id) {
   unsigned allowed;
   asm volatile(CT_DQ_IDS_SEQUENCE
                : "=&v"(allowed) : "v"(ids), "v"(id), "i"(STAGE_OFF)
-               : "memory", "vcc", CT_DQ_STEP_SCRATCH, CT_DQ_ACCUMULATORS);
+               : "memory", CT_MASK_PAIRS, CT_DQ_STEP_SCRATCH, CT_DQ_ACCUMULATORS);
   return allowed;
 }
 CT_DEVICE unsigned dq_pairs_up_to(int last_rel) {

@@ -438,7 +438,7 @@ struct FwdCopies {
     asm volatile(CT_FWD_MASK_CAUSAL_##UPPER                                                                   \
                  :                                                                                            \
                  : [rel] "v"(rel), [ninf] "v"(kNegInf)                                                        \
-                 : "memory", "vcc", CT_FWD_PRIVATE);                                                          \
+                 : "memory", CT_MASK_PAIRS, CT_FWD_PRIVATE);                                                  \
   }                                                                                                           \
   /* -inf where the key's id differs from seg (per lane); ids: the lane's address of the id of key */        \
   /* 4 * (lane / 32) of the tile in the id ring                                                      */        \
@@ -446,7 +446,7 @@ struct FwdCopies {
     asm volatile(CT_FWD_MASK_IDS_##UPPER                                                                      \
                  :                                                                                            \
                  : [idp] "v"(ids), [segq] "v"(seg), [ninf] "v"(kNegInf)                                       \
-                 : "memory", "vcc", CT_FWD_PRIVATE);                                                          \
+                 : "memory", CT_MASK_PAIRS, CT_FWD_PRIVATE);                                                  \
   }
 CT_FWD_STATEMENTS(a, A)
 CT_FWD_STATEMENTS(b, B)

@@ -235,6 +235,22 @@ def fwd_max_ops(cur):
     return ops
 
 
+# Two wait states lie between a vector compare and the vector instruction that reads its bits: the bits of one are used
+# behind the next two compares, and three scalar pairs take turns.
+MASK_PAIRS = ("vcc", "s[96:97]", "s[98:99]")
+
+
+def compare_and_use(compare, use):
+    """One list of instructions per element: compare(e) and, two elements later, use(e); both give a mnemonic and its operands
+    with {} where the pair stands."""
+    def text(instruction, e):
+        pair = MASK_PAIRS[e % 3]     # (vcc has the short encoding)
+        return "%s_%s %s" % (instruction[0], "e32" if pair == "vcc" else "e64", instruction[1].format(pair))
+    groups = [[text(compare(e), e)] + ([text(use(e - 2), e - 2)] if e >= 2 else []) for e in range(32)]
+    groups[-1] += [text(use(e), e) for e in (30, 31)]
+    return groups
+
+
 def flatten(head, groups):
     return head + [ln for g in groups for ln in g]
 
@@ -246,10 +262,8 @@ def fwd_statements(cur):
     head_qk, qk = fwd_qk_groups(cur)
     key_offset = lambda i: 32 * (i // 16) + 8 * ((i % 16) // 4) + (i % 16) % 4
     s0 = FWD_S[cur]
-    causal = []
-    for i in range(32):
-        causal += ["v_cmp_le_i32_e32 vcc, %d, %%[rel]" % key_offset(i),
-                   "v_cndmask_b32_e32 v%d, %%[ninf], v%d, vcc" % (s0 + i, s0 + i)]
+    select = lambda i: ("v_cndmask_b32", "v%d, %%[ninf], v%d, {}" % (s0 + i, s0 + i))
+    causal = flatten([], compare_and_use(lambda i: ("v_cmp_le_i32", "{}, %d, %%[rel]" % key_offset(i)), select))
     # ids: the tile's 64 key ids sit in LDS in key order; %[idp] is this lane's address of key
     # 4 * (lane / 32), so the quad of registers 4 q .. 4 q + 3 of block kb is the 16 bytes at
     # offset 4 * (32 kb + 8 q). Quads go through the fragment ring (four in flight).
@@ -258,12 +272,10 @@ def fwd_statements(cur):
     quad_read = lambda q: "ds_read_b128 v[%d:%d], %%[idp] offset:%d" % (
         quad_regs(q), quad_regs(q) + 3, 4 * (32 * (q // 4) + 8 * (q % 4)))
     ids += [quad_read(q) for q in range(4)]
+    by_id = compare_and_use(lambda i: ("v_cmp_eq_u32", "{}, %%[segq], v%d" % (quad_regs(i // 4) + i % 4)), select)
     for q in range(8):
         ids.append("s_waitcnt lgkmcnt(%d)" % min(3, 7 - q))
-        for e in range(4):
-            i = 4 * q + e
-            ids += ["v_cmp_eq_u32_e32 vcc, %%[segq], v%d" % (quad_regs(q) + e),
-                    "v_cndmask_b32_e32 v%d, %%[ninf], v%d, vcc" % (s0 + i, s0 + i)]
+        ids += flatten([], by_id[4 * q:4 * q + 4])
         if q + 4 < 8:
             ids.append(quad_read(q + 4))
     return {
@@ -743,10 +755,12 @@ def dq_ids_sequence():
     for q in range(8):
         lines.append("ds_read_b128 v[%d:%d], %%1 offset:%%3+%d" % (base + 4 * q, base + 4 * q + 3, 32 * (7 - q)))
     lines.append("v_mov_b32_e32 %0, 0")
+    # (the last element first; what a carry leaves in its pair nothing reads)
+    bits = compare_and_use(lambda i: ("v_cmp_eq_u32", "{}, %%2, v%d" % (base + (i | 3) - i % 4)),
+                           lambda i: ("v_addc_co_u32", "%0, {0}, %0, %0, {0}"))
     for q in range(8):
         lines.append("s_waitcnt lgkmcnt(%d)" % (7 - q))
-        for e in (3, 2, 1, 0):
-            lines += ["v_cmp_eq_u32_e32 vcc, %%2, v%d" % (base + 4 * q + e), "v_addc_co_u32_e32 %0, vcc, %0, %0, vcc"]
+        lines += flatten([], bits[4 * q:4 * q + 4])
     return lines
 
 
@@ -976,11 +990,12 @@ def clobbers():
     step_accs = ", ".join('"a%d"' % r for r in range(128))
     wide = ", ".join('"v%d"' % r for r in range(W_FIRST, 256))
     accs = ", ".join('"a%d"' % r for r in range(256))
-    return ("#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DQ_STEP_SCRATCH %s\n\n#define CT_DQ_ACCUMULATORS %s\n\n"
+    pairs = '"vcc", "s96", "s97", "s98", "s99"'
+    return ("#define CT_MASK_PAIRS %s\n\n#define CT_ATTN_ASM_SCRATCH %s\n\n#define CT_DQ_STEP_SCRATCH %s\n\n#define CT_DQ_ACCUMULATORS %s\n\n"
             "#define CT_DKV_STEP_SCRATCH %s\n\n"
             "#define CT_DKV_ACCUMULATORS %s\n\n"
             "#define CT_DKVW_ASM_SCRATCH %s\n\n"
-            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (regs, dq, dq_accs, step, step_accs, wide, accs,
+            "#define CT_DKVW_ACCUMULATORS %s\n\n#define CT_FWD_PRIVATE %s\n" % (pairs, regs, dq, dq_accs, step, step_accs, wide, accs,
                                                                              fwd_private_clobbers()))
 
 

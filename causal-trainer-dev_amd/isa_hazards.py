@@ -10,7 +10,8 @@ every memory instruction whose scalar operands were written by a vector instruct
 5 wait states earlier. It also reports the second hazard of that kind: a store of more than 8 bytes
 reads its data registers late, and a vector instruction that writes one of them within 2 wait
 states of the store replaces the data on its way out. And a third: an MFMA reads its operands without a look at vector
-instructions that are still under way, so 2 wait states lie between the write of a register and the MFMA that reads it
+instructions that are still under way, so 2 wait states lie between the write of a register and the MFMA that reads it, and
+as many between a vector instruction that writes a scalar register (a compare's bits, a carry) and one that reads it
 (``fresh_operands``). ``python -m causal_trainer_dev_amd.isa_hazards`` compiles every source of
 the library and scans it; tests/test_isa_hazards.py runs the same on the CPU.
 """
@@ -27,6 +28,7 @@ from pathlib import Path
 WAIT_STATES = 5
 STORE_DATA_WAIT_STATES = 2
 MFMA_OPERAND_WAIT_STATES = 2
+SCALAR_OPERAND_WAIT_STATES = 2
 _WIDE_STORE = re.compile(r"^\s*(global|buffer|flat|scratch)_store_dwordx[34]\s+(.*)")
 _VECTOR_ALU = re.compile(r"^\s*v_\w+\s+(.*)")
 _MEMORY = re.compile(r"^\s*(global_|buffer_|flat_|scratch_)")
@@ -175,7 +177,7 @@ def _wait_states_between(writer: str, registers: set, reader: str) -> int:
     vectors = any(register[0] in "va" for register in registers if register != "vcc")
     if vectors and reader.startswith("v_mfma") and not writer.startswith("v_mfma"):
         return MFMA_OPERAND_WAIT_STATES
-    return 0
+    return SCALAR_OPERAND_WAIT_STATES if any(register == "vcc" or register[0] == "s" for register in registers) else 0
 
 
 def private_accumulators(assembly: str, kernel: str) -> list[str]:

@@ -281,7 +281,7 @@ def test_dq_bits_of_ids(gen):
     """The statement on a model of the id ring: bit e is the comparison with the id of key 8 (e / 4) + 4 half + e % 4."""
 
     for half in (0, 1):
-        registers, compared = {}, None
+        registers, compared = {}, {}
         bits = []
         for line in gen.dq_ids_sequence():
             name, operands = _split(line)
@@ -289,14 +289,27 @@ def test_dq_bits_of_ids(gen):
                 offset = int(line.split("offset:%3+")[1])
                 for e, register in enumerate(sorted(_registers(operands[0]))):
                     registers[register] = 4 * half + offset // 4 + e
-            elif name == "v_cmp_eq_u32_e32":
-                assert operands[:2] == ["vcc", "%2"]
+            elif name.startswith("v_cmp_eq_u32"):
+                assert operands[1] == "%2"
                 (register,) = _registers(operands[2])
-                compared = registers[register]
-            elif name == "v_addc_co_u32_e32":
-                assert operands == ["%0", "vcc", "%0", "%0", "vcc"]
-                bits.insert(0, compared)     # shifted in from below
-        assert bits == [8 * (e // 4) + 4 * half + e % 4 for e in range(32)]
+                compared[operands[0]] = registers[register]
+            elif name.startswith("v_addc_co_u32"):
+                assert operands == ["%0", operands[1], "%0", "%0", operands[1]]
+                bits.insert(0, compared.pop(operands[1]))     # shifted in from below
+        assert bits == [8 * (e // 4) + 4 * half + e % 4 for e in range(32)] and not compared
+
+
+def test_bits_of_compares_are_read_late_enough(gen):
+    """Two wait states between a compare and the vector instruction that reads its bits, in every statement."""
+
+    from causal_trainer_dev_amd import isa_hazards
+
+    for name, lines in _sequences(gen).items():
+        assert isa_hazards.fresh_operands("\n".join(lines)) == [], name
+    early = gen.dq_ids_sequence()
+    first = next(i for i, line in enumerate(early) if line.startswith("v_addc_co"))
+    early.insert(first - 1, early.pop(first))
+    assert isa_hazards.fresh_operands("\n".join(early))
 
 
 def _vector_alu(lines):
@@ -395,17 +408,25 @@ def test_forward_masks(gen):
         s0 = gen.FWD_S[cur]
         causal = gen.fwd_statements(cur)["MASK_CAUSAL"]
         assert len(causal) == 64
-        for i in range(32):
-            offset = 32 * (i // 16) + 8 * ((i % 16) // 4) + (i % 16) % 4
-            assert causal[2 * i] == "v_cmp_le_i32_e32 vcc, %d, %%[rel]" % offset
-            assert causal[2 * i + 1] == "v_cndmask_b32_e32 v%d, %%[ninf], v%d, vcc" % (s0 + i, s0 + i)
+        compared = {}
+        selected = []
+        for line in causal:
+            name, operands = _split(line)
+            if name.startswith("v_cmp_le_i32"):
+                assert operands[2] == "%[rel]"
+                compared[operands[0]] = int(operands[1])
+            else:
+                (score,) = _registers(operands[0])
+                assert name.startswith("v_cndmask_b32") and operands[1] == "%[ninf]" and _registers(operands[2]) == {score}
+                selected.append((score - s0, compared.pop(operands[3])))
+        assert selected == [(i, 32 * (i // 16) + 8 * ((i % 16) // 4) + (i % 16) % 4) for i in range(32)]
         # ids: run the statement on a model of the id ring (key k's id at byte 4 k; the lane's pointer
         # is the address of key 4 * half): every score must be compared with the id of its own key,
         # and no register may be read before the wait that covers its load
         for half in (0, 1):
             registers, landed, in_flight = {}, set(), []
             compared = {}
-            pending_compare = None
+            pending = {}
             for line in gen.fwd_statements(cur)["MASK_IDS"]:
                 name, operands = _split(line)
                 if name == "s_waitcnt":
@@ -420,16 +441,15 @@ def test_forward_masks(gen):
                         registers[register] = 4 * half + offset // 4 + e     # the key whose id it holds
                     landed -= set(quad)
                     in_flight.append(set(quad))
-                elif name == "v_cmp_eq_u32_e32":
-                    assert operands[:2] == ["vcc", "%[segq]"]
+                elif name.startswith("v_cmp_eq_u32"):
+                    assert operands[1] == "%[segq]"
                     (register,) = _registers(operands[2])
                     assert register in landed, line
-                    pending_compare = registers[register]
-                elif name == "v_cndmask_b32_e32":
+                    pending[operands[0]] = registers[register]
+                elif name.startswith("v_cndmask_b32"):
                     (score,) = _registers(operands[0])
-                    assert operands[1] == "%[ninf]" and _registers(operands[2]) == {score} and operands[3] == "vcc"
-                    compared[score - s0] = pending_compare
-                    pending_compare = None
+                    assert operands[1] == "%[ninf]" and _registers(operands[2]) == {score}
+                    compared[score - s0] = pending.pop(operands[3])
                 else:
                     raise AssertionError(line)
             assert compared == {i: 32 * (i // 16) + 8 * ((i % 16) // 4) + (i % 16) % 4 + 4 * half for i in range(32)}

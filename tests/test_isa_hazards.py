@@ -1,6 +1,6 @@
 """The compiled kernels must not read a scalar register in a memory instruction fewer than
-5 wait states after a vector instruction wrote it, nor an MFMA operand fewer than 2 after it was
-written (the compiler does not pad inline asm)."""
+5 wait states after a vector instruction wrote it, nor an MFMA operand, or a scalar register in a
+vector instruction, fewer than 2 after (the compiler does not pad inline asm)."""
 
 import shutil
 
@@ -69,6 +69,22 @@ kernel_a:
     # (one MFMA into the next one's sums is the matrix pipe's own affair)
     chained = "kernel_c:\n" + "\tv_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[8:11], a[0:15]\n" * 2
     assert isa_hazards.fresh_operands(chained) == []
+
+
+def test_scanner_flags_fresh_scalar_operands(ct):
+    from causal_trainer_dev_amd import isa_hazards
+
+    select = """
+kernel_a:
+	v_cmp_le_i32_e32 vcc, 3, v61
+	v_mov_b32_e32 v1, v2
+	v_cndmask_b32_e32 v144, v56, v144, vcc
+"""
+    assert len(isa_hazards.fresh_operands(select)) == 1
+    assert isa_hazards.fresh_operands(select.replace("\tv_mov", "\ts_nop 0\n\tv_mov")) == []
+    assert isa_hazards.fresh_operands(select.replace("vcc, 3", "s[96:97], 3")) == []
+    pair = select.replace("_e32 vcc", "_e64 s[96:97]").replace("vcc", "s[96:97]")
+    assert len(isa_hazards.fresh_operands(pair)) == 1
 
 
 def test_private_accumulator_check(ct):
