@@ -1341,8 +1341,14 @@ static bool backward_in_place(const ct_cutce_shape& s) {
   const long elements = (long)s.hidden * s.vocab;
   return needs_panel(s) && s.vocab >= 8192 && elements >= 12000000 && s.rows <= (elements <= 100000000 ? 1024 : 512);
 }
-// With a logits cache the forward leaves the backward panel or tail, with nothing kept each direction has its own.
-static bool both_in_place(const ct_cutce_shape& s) { return forward_in_place(s) && backward_in_place(s); }
+// With a logits cache or a kept panel one copy serves both directions, so it has to be paid for once only, and reading in place is
+// ahead of it for fewer calls. A pass with both buffers allowed, copy / in place: 64 x 32003, d = 4096 360 / 287; 512 x 16001, d = 1024
+// 117 / 115, x 100003 535 / 491, d = 512 331 / 312, x 150001 448 / 441; up to 35 million elements at 1024 rows too: x 50257, d = 256
+// 206 / 196, x 32003, d = 512 183 / 183, x 16001, d = 2048 252 / 234; not beyond: 1024 x 100003, d = 512 508 / 525, x 150001 712 / 756,
+// 640 x 100003, d = 768 521 / 551, x 32003, d = 2048 374 / 397.
+static bool both_in_place(const ct_cutce_shape& s) {
+  return forward_in_place(s) && backward_in_place(s) && (s.rows <= 512 || (long)s.hidden * s.vocab <= 35000000);
+}
 static size_t panel_tile_bytes(const ct_cutce_shape& s) { return (size_t)s.hidden * kGemmTile * sizeof(bf16); }
 // bytes of the panel of the whole vocabulary, 0 if none is needed
 static size_t full_panel_bytes(const ct_cutce_shape& s) {

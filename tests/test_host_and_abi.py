@@ -143,6 +143,17 @@ def test_cutce_panel_and_logits_cache_cannot_be_mixed_up(ct):
         assert b"workspace" in library.ct_last_error()
 
 
+@pytest.mark.parametrize("rows,hidden,vocab,both", [
+    (512, 512, 150001, 1), (513, 512, 150001, 0),       # many rows and a large head: one copy for both directions is faster
+    (640, 768, 100003, 0), (1000, 1024, 32003, 1),      # ... up to 35 million elements it is not
+    (1024, 2048, 16001, 1), (1024, 2048, 17091, 0),
+    (1025, 1024, 16001, 0), (64, 1024, 16000, 0),       # too many rows for the backward; a head that is aligned
+])
+def test_cutce_heads_that_both_directions_read_in_place(ct, rows, hidden, vocab, both):
+    shape = ct._lib.CutceShape(rows, hidden, vocab)
+    assert ct._lib.load().ct_cutce_head_in_place(ctypes.byref(shape)) == both
+
+
 @pytest.mark.parametrize("torch_side", ["absent", "broken", "there"])
 def test_library_is_linked_whatever_becomes_of_the_torch_side(monkeypatch, tmp_path, torch_side):
     """libct_hotpath.so needs hipcc only: it is linked without torch, and before a torch side that fails to compile
