@@ -1334,12 +1334,15 @@ static bool forward_in_place(const ct_cutce_shape& s) {
   return needs_panel(s) && s.rows <= 2048 && s.vocab >= 8l * s.rows && 2l * s.vocab >= s.hidden;
 }
 // Backward (copy, dlogits and gradients), where dHidden reads short rows: 64 x 150001, d = 4096 1466 / 1165, d = 256 163 / 132;
-// 250 x 50001, d = 1024 149 / 122; 500 x 16001, d = 1024 88 / 85, x 50001, d = 4096 790 / 723; 1000 x 50001, d = 1024 351 /
-// 335, 1000 x 16001, d = 4096 388 / 361, but x 150001, d = 1024 985 / 1004, x 50001, d = 4096 1265 / 1296; 2000 x 50001,
-// d = 1024 628 / 636. Small heads: 64 x 16001, d = 256 31.2 / 32.0, 500 x 5001, d = 1024 46.8 / 50.6.
+// 250 x 50001, d = 1024 149 / 122; 512 x 100003, d = 1024 418 / 391, x 50257, d = 4096 747 / 696. The larger the head, the fewer the
+// rows that it pays for: 640 x 50257, d = 2048 491 / 510, x 16001, d = 8192 646 / 720; 768 x 50257, d = 1024 273 / 264, x 16001, d = 4096
+// 316 / 301, x 100003, d = 512 296 / 303; 1024 x 150001, d = 256 340 / 353, x 50257, d = 1024 333 / 348, x 32003, d = 2048 382 / 393, but
+// x 16001, d = 2048 213 / 194, x 32003, d = 512 129 / 126; 1280 x 16001, d = 1024 147 / 155, d = 2048 268 / 264; 2048 x 16001, d = 1024
+// 190 / 202, x 150001, d = 256 605 / 656. Small heads: 64 x 16001, d = 256 31.2 / 32.0, 500 x 5001, d = 1024 46.8 / 50.6.
 static bool backward_in_place(const ct_cutce_shape& s) {
   const long elements = (long)s.hidden * s.vocab;
-  return needs_panel(s) && s.vocab >= 8192 && elements >= 12000000 && s.rows <= (elements <= 100000000 ? 1024 : 512);
+  const int most_rows = elements <= 35000000 ? 1024 : elements <= 100000000 ? 768 : 512;
+  return needs_panel(s) && s.vocab >= 8192 && elements >= 12000000 && s.rows <= most_rows;
 }
 // With a logits cache or a kept panel one copy serves both directions, so it has to be paid for once only, and reading in place is
 // ahead of it for fewer calls. A pass with both buffers allowed, copy / in place: 64 x 32003, d = 4096 360 / 287; 512 x 16001, d = 1024
