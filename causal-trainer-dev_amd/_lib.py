@@ -155,6 +155,9 @@ SYMBOLS = {
     "ct_cutce_bwd_workspace_min_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_bwd_workspace_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_logits_cache_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_fwd_workspace_used_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_bwd_workspace_used_bytes": (c_size_t, [POINTER(CutceShape)]),
+    "ct_cutce_logits_cache_used_bytes": (c_size_t, [POINTER(CutceShape)]),
     "ct_cutce_fwd": (c_int32, [c_void_p, POINTER(CutceFwdArgs)]),
     "ct_cutce_bwd": (c_int32, [c_void_p, POINTER(CutceBwdArgs)]),
     "ct_cutce_panel_bytes": (c_size_t, [POINTER(CutceShape)]),

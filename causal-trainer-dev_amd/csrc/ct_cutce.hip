@@ -1357,8 +1357,10 @@ static size_t panel_tile_bytes(const ct_cutce_shape& s) { return (size_t)s.hidde
 static size_t full_panel_bytes(const ct_cutce_shape& s) {
   return needs_panel(s) ? panel_tile_bytes(s) * vocab_tile_count(s.vocab) : 0;
 }
+// What a direction makes of an unaligned head: read in place, the tail only.
+static size_t copy_bytes(const ct_cutce_shape& s, bool in_place) { return in_place ? panel_tile_bytes(s) : full_panel_bytes(s); }
 
-// Workspace of the forward: `base` bytes it cannot do without, then as much of the panel as fits.
+// Workspace of the forward: `base` bytes it cannot do without, then as much of the panel as fits, or the tail.
 struct FwdLayout {
   size_t header, idx, target, active, part, sums, base, total;
 };
@@ -1417,16 +1419,23 @@ static size_t bwd_fixed_bytes(int n_pad, int d) {
   return align_up(sizeof(CutceHeader), 256) + 4 * align_up((size_t)n_pad * sizeof(int), 256) +
          align_up((size_t)n_pad * d * sizeof(bf16), 256) + (size_t)d * 128 * sizeof(bf16);
 }
-// What one tile column of a slab takes: its part of G^T, without a panel in the logits cache of the
-// panel, and the partial sums of dHead if that is cut.
+// What one tile column of a slab takes: its part of G^T, its columns of a head that is copied here, and the partial
+// sums of dHead if that is cut.
 struct BwdTileBytes {
   size_t g, panel, head_sums;
   size_t all() const { return g + panel + head_sums; }
 };
-static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, bool panel_elsewhere, bool with_head) {
+// What the workspace of the backward holds of an unaligned head: copies of the slabs' columns, the tail, or nothing (the panel is lent
+// or in the logits cache). With the tail the copies' bytes go to wider slabs and more parts. A bounded call that copies slab by
+// slab / reads in place, us of a pass: 144 x 30159, d = 2432 in chunks of 24 rows 494 / 237, 64 x 50257, d = 1024 by 4 568 / 269,
+// 512 x 32003, d = 4096 by 85 955 / 575, 999 x 32003, d = 1024 by 166 506 / 441, 900 x 50257, d = 256 by 450 211 / 219.
+enum class HeadPart { kPanel, kTail, kNothing };
+static HeadPart bwd_head_part(const ct_cutce_shape& s, bool panel_elsewhere) {
+  return !needs_panel(s) || panel_elsewhere ? HeadPart::kNothing : backward_in_place(s) ? HeadPart::kTail : HeadPart::kPanel;
+}
+static BwdTileBytes bwd_tile_bytes(const ct_cutce_shape& s, HeadPart part, bool with_head) {
   const int parts = with_head ? most_head_parts(s) : 1;
-  return BwdTileBytes{(size_t)padded_rows(s.rows) * kGemmTile * sizeof(bf16),
-                      needs_panel(s) && !panel_elsewhere ? panel_tile_bytes(s) : 0,
+  return BwdTileBytes{(size_t)padded_rows(s.rows) * kGemmTile * sizeof(bf16), part == HeadPart::kPanel ? panel_tile_bytes(s) : 0,
                       parts > 1 ? (size_t)parts * s.hidden * kGemmTile * sizeof(float) : 0};
 }
 static size_t bwd_acc_bytes(const ct_cutce_shape& s) {
@@ -1464,6 +1473,7 @@ static float slabs_time(const ct_cutce_shape& s, int slab_tiles, size_t spare, b
 // 84 x 2432 x 132192 by 22, 4, 3516 / 913, 290 x 768 x 141343 by 32, frozen head, 12, 2420 / 732, 456 x 256 x 24749 by 23, 14,
 // 432 / 388, 5058 x 1024 x 108442 by 125, 39, 5105 / 5100.
 static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_elsewhere, bool with_head) {
+  const HeadPart part = bwd_head_part(s, panel_elsewhere);
   const int n_pad = padded_rows(s.rows);
   const int tiles = vocab_tile_count(s.vocab);
   BwdLayout L = {};
@@ -1473,16 +1483,17 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_el
   L.packed = L.rowparams + 3 * align_up((size_t)n_pad * sizeof(int), 256);
   L.panel = bwd_fixed_bytes(n_pad, s.hidden);
   L.tail = L.panel - (size_t)s.hidden * 128 * sizeof(bf16);
-  const BwdTileBytes tile = bwd_tile_bytes(s, panel_elsewhere, with_head);
+  const BwdTileBytes tile = bwd_tile_bytes(s, part, with_head);
   const size_t per_tile = tile.all(), acc_bytes = bwd_acc_bytes(s);
+  const size_t slab = L.panel + (part == HeadPart::kTail ? panel_tile_bytes(s) : 0);  // where a slab's part begins
   size_t fit = tiles, room;
   L.head_most = with_head ? most_head_parts(s) : 1;
-  const bool whole = bytes >= L.panel + per_tile * tiles;
-  room = whole ? bytes - L.panel : 0;
+  const bool whole = bytes >= slab + per_tile * tiles;
+  room = whole ? bytes - slab : 0;
   const size_t all_sums = std::min(hidden_sums_bytes(s, tiles, with_head), most_hidden_sums_bytes(s, tiles));
   if (!whole || room - per_tile * tiles < all_sums) {
     float least = whole ? slabs_time(s, tiles, room - per_tile * tiles, with_head) : __builtin_inff();
-    const size_t slabs_room = bytes < L.panel + acc_bytes ? 0 : bytes - L.panel - acc_bytes;
+    const size_t slabs_room = bytes < slab + acc_bytes ? 0 : bytes - slab - acc_bytes;
     const size_t most = slabs_room / per_tile;
     if (!whole && most == 0) return L;
     for (size_t fewer = most < (size_t)tiles ? most : (size_t)tiles - 1; fewer > 0; fewer -= (fewer + 7) / 8) {
@@ -1497,7 +1508,7 @@ static BwdLayout bwd_layout(const ct_cutce_shape& s, size_t bytes, bool panel_el
   L.hidden_sums_bytes = want < spare ? want : spare;
   L.slab_cols = (int)fit * kGemmTile;
   L.slabs = (tiles + (int)fit - 1) / (int)fit;
-  L.g = L.panel + tile.panel * fit;
+  L.g = slab + tile.panel * fit;
   L.head_sums = L.g + tile.g * fit;
   L.acc = L.head_sums + tile.head_sums * fit;
   L.hidden_sums = L.acc + (L.slabs > 1 ? acc_bytes : 0);
@@ -1566,6 +1577,10 @@ extern "C" size_t ct_cutce_fwd_workspace_bytes(const ct_cutce_shape* shape) {
   return valid_sizes(shape) ? fwd_layout(*shape).total : 0;
 }
 
+extern "C" size_t ct_cutce_fwd_workspace_used_bytes(const ct_cutce_shape* shape) {
+  return valid_sizes(shape) ? fwd_layout(*shape).base + copy_bytes(*shape, forward_in_place(*shape)) : 0;
+}
+
 extern "C" size_t ct_cutce_fwd_workspace_min_bytes(const ct_cutce_shape* shape) {
   return valid_sizes(shape) ? fwd_layout(*shape).base : 0;
 }
@@ -1580,17 +1595,27 @@ extern "C" size_t ct_cutce_logits_cache_bytes(const ct_cutce_shape* shape) {
   return valid_sizes(shape) ? logits_bytes(*shape) + full_panel_bytes(*shape) : 0;
 }
 
-extern "C" size_t ct_cutce_bwd_workspace_bytes(const ct_cutce_shape* shape) {
+extern "C" size_t ct_cutce_logits_cache_used_bytes(const ct_cutce_shape* shape) {
+  return valid_sizes(shape) ? logits_bytes(*shape) + copy_bytes(*shape, both_in_place(*shape)) : 0;
+}
+
+extern "C" size_t ct_cutce_bwd_workspace_used_bytes(const ct_cutce_shape* shape) {
   if (!valid_sizes(shape)) return 0;
   const size_t trained = bwd_layout(*shape, ~(size_t)0, false, true).total;
   const size_t frozen = bwd_layout(*shape, ~(size_t)0, false, false).total;
   return trained > frozen ? trained : frozen;
 }
 
+extern "C" size_t ct_cutce_bwd_workspace_bytes(const ct_cutce_shape* shape) {
+  if (!valid_sizes(shape)) return 0;
+  return ct_cutce_bwd_workspace_used_bytes(shape) + full_panel_bytes(*shape) - copy_bytes(*shape, backward_in_place(*shape));
+}
+
 extern "C" size_t ct_cutce_bwd_workspace_min_bytes(const ct_cutce_shape* shape) {
   if (!valid_sizes(shape)) return 0;
   const size_t fixed =
-      bwd_fixed_bytes(padded_rows(shape->rows), shape->hidden) + bwd_tile_bytes(*shape, false, true).all();
+      bwd_fixed_bytes(padded_rows(shape->rows), shape->hidden) + bwd_tile_bytes(*shape, HeadPart::kNothing, true).all() +
+      (needs_panel(*shape) ? panel_tile_bytes(*shape) : 0);  // (one column of the panel, or the tail)
   return vocab_tile_count(shape->vocab) == 1 ? fixed : fixed + bwd_acc_bytes(*shape);
 }
 
@@ -1711,7 +1736,7 @@ static int launch_grads(const char* fn, hipStream_t stream, const CutceParams& p
   return scope.done();
 }
 
-// The panel and the logits cache that a caller lends. A cache has room for a panel behind its logits, which a
+// The panel and the logits cache that a caller lends. A cache has room for a panel (or a tail) behind its logits, which a
 // forward with a lent panel would leave unwritten, so with one the cache ends behind the logits: the entries
 // without a panel refuse it as too small.
 static int validate_lent(const char* fn, const ct_cutce_shape& s, const void* panel, size_t panel_bytes, const void* cache,
@@ -1722,7 +1747,7 @@ static int validate_lent(const char* fn, const ct_cutce_shape& s, const void* pa
     return fail(CT_WORKSPACE_TOO_SMALL, "%s: panel %zu < %zu bytes", fn, panel_bytes, full_panel_bytes(s));
   if (!cache) return CT_OK;
   CT_REQUIRE(is_aligned16(cache), "%s: logits cache must be 16-byte aligned", fn);
-  const size_t need = logits_bytes(s) + (lent ? 0 : full_panel_bytes(s));
+  const size_t need = logits_bytes(s) + (lent ? 0 : copy_bytes(s, both_in_place(s)));
   if (cache_bytes < need) return fail(CT_WORKSPACE_TOO_SMALL, "%s: logits cache %zu < %zu bytes", fn, cache_bytes, need);
   CT_REQUIRE(!lent || cache_bytes == need, "%s: beside a panel the logits cache is %zu bytes, without room for one, not %zu", fn,
              need, cache_bytes);
@@ -1918,7 +1943,7 @@ extern "C" int32_t ct_cutce_bwd_panel(void* stream_, const ct_cutce_bwd_args* a,
   const bf16* head = p.head.base;
   bf16* panel = nullptr;
   HeadCopy tail = {};
-  const bool in_place = !lent && (cache ? both_in_place(a->shape) : L.slabs == 1 && backward_in_place(a->shape));
+  const bool in_place = !lent && (cache ? both_in_place(a->shape) : backward_in_place(a->shape));
   if (head_aligned && p.V % 128) {
     p.head = tail_view(p, reinterpret_cast<const bf16*>(ws + L.tail), 128);
     tail = tail_copy(p.head);

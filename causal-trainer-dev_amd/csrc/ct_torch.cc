@@ -533,7 +533,7 @@ std::tuple<Tensor, Tensor, Tensor> cutce_forward_on(const ct_cutce_shape& shape,
   // (with a logits cache the aligned copy of an unaligned head goes there)
   const bool cached = cache && cache->defined();
   const size_t bytes = cached || panel ? ct_cutce_fwd_workspace_min_bytes(&shape)
-                       : workspace_bytes >= 0 ? (size_t)workspace_bytes : ct_cutce_fwd_workspace_bytes(&shape);
+                       : workspace_bytes >= 0 ? (size_t)workspace_bytes : ct_cutce_fwd_workspace_used_bytes(&shape);
   Tensor workspace = scratch(bytes, hidden);
   Tensor nll = floats({}, hidden), weight_sum = floats({}, hidden), lse = floats({shape.rows}, hidden);
   ct_cutce_fwd_args a = {};
@@ -565,12 +565,13 @@ std::tuple<Tensor, MaybeTensor> cutce_backward_on(const ct_cutce_shape& shape, c
                                                   const Tensor& dy, bool compaction, bool with_head, int64_t workspace_bytes,
                                                   const MaybeTensor& cache, const MaybeTensor& panel) {
   const c10::DeviceGuard guard(hidden.device());
+  const bool cached = cache && cache->defined();
   const size_t bytes = workspace_bytes >= 0 ? (size_t)workspace_bytes
-                                            : ct_cutce_bwd_workspace_bytes(&shape) - (panel ? ct_cutce_panel_bytes(&shape) : 0);
+                       : cached || panel    ? ct_cutce_bwd_workspace_bytes(&shape) - ct_cutce_panel_bytes(&shape)
+                                            : ct_cutce_bwd_workspace_used_bytes(&shape);
   Tensor workspace = scratch(bytes, hidden), dhidden = fresh(hidden);
   MaybeTensor dhead;
   if (with_head) dhead = at::empty({shape.hidden, shape.vocab}, hidden.options().requires_grad(false));
-  const bool cached = cache && cache->defined();
   ct_cutce_bwd_args a = {};
   a.hidden = bits(hidden);
   a.head = bits(head);
@@ -666,7 +667,7 @@ std::optional<std::tuple<Tensor, Tensor>> cut_ce(const Tensor& hidden, const Ten
   }
   MaybeTensor cache, panel;
   if (use_cache && graph) {
-    const size_t bytes = ct_cutce_logits_cache_bytes(&shape) - (head_is_panel ? panel_bytes : 0);
+    const size_t bytes = head_is_panel ? ct_cutce_logits_cache_bytes(&shape) - panel_bytes : ct_cutce_logits_cache_used_bytes(&shape);
     if ((int64_t)bytes <= cache_limit && cache_pays(shape)) cache = scratch(bytes, hidden);
   }
   // An unaligned head is copied once for both directions only where the caller lets a buffer be kept between them, like

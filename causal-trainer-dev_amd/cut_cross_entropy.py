@@ -29,10 +29,11 @@ is no saved tensor (hooks do not see it) and goes with the first backward. With
 ``local_chunk_size`` (:697-825). The reference's chunk loop bounds what one TPU core holds at
 a time: it walks the rows in chunks, compacts inside the chunk and accumulates the head
 gradient in f32 across chunks. What the option buys is a bound on transient memory, and that
-is what it selects here: with ``local_chunk_size = C > 0`` the backward's dlogits slab is no
-larger than the dlogits of C rows over the whole vocabulary would be (``backward_workspace_bytes``;
-never below the kernels' minimum of one 256-wide vocabulary tile), the vocabulary is walked in
-slabs of that size with dHidden accumulated in f32 across slabs and rounded once, and no logits
+is what it selects here: with ``local_chunk_size = C > 0`` the backward's workspace is the share
+C / rows of what a single slab over the whole vocabulary takes with the aligned copy of an unaligned
+head (``backward_workspace_bytes``; never below the kernels' minimum of one 256-wide vocabulary tile,
+and where the head is read in place no more than the slab without the copy), the vocabulary is walked in
+slabs that fit with dHidden accumulated in f32 across slabs and rounded once, and no logits
 cache is kept. A row's statistics and gradients do not depend on which slab or slot it sits in;
 only the order of f32 additions differs, inside the operator's tolerances. ``0`` (the default)
 keeps the single full-vocabulary slab.
@@ -59,19 +60,20 @@ def _shape_struct(rows: int, hidden: int, vocab: int) -> _lib.CutceShape:
 def logits_cache_bytes(rows: int, hidden: int, vocab: int) -> int:
     """Size of the optional f32 logits cache for this problem."""
 
-    return int(_lib.load().ct_cutce_logits_cache_bytes(_shape_struct(rows, hidden, vocab)))
+    return int(_lib.load().ct_cutce_logits_cache_used_bytes(_shape_struct(rows, hidden, vocab)))
 
 
 def backward_workspace_bytes(rows: int, hidden: int, vocab: int, local_chunk_size: int = 0) -> int:
-    """Workspace of the backward: the full-vocabulary slab, or with ``local_chunk_size`` rows per
-    chunk a slab as large as the dlogits of one chunk of rows (at least the kernels' minimum)."""
+    """Workspace of the backward: what the full-vocabulary slab uses, or with ``local_chunk_size`` rows per chunk their
+    share of that slab and a copy of the head (at least the kernels' minimum)."""
 
     lib = _lib.load()
     shape = _shape_struct(rows, hidden, vocab)
-    full, least = int(lib.ct_cutce_bwd_workspace_bytes(shape)), int(lib.ct_cutce_bwd_workspace_min_bytes(shape))
+    most, least = int(lib.ct_cutce_bwd_workspace_used_bytes(shape)), int(lib.ct_cutce_bwd_workspace_min_bytes(shape))
     if local_chunk_size <= 0 or local_chunk_size >= rows:
-        return full
-    return max(least, min(full, least + (full - least) * local_chunk_size // rows))
+        return most
+    full = int(lib.ct_cutce_bwd_workspace_bytes(shape))
+    return max(least, min(most, least + (full - least) * local_chunk_size // rows))
 
 
 def cutce_forward(hidden, head, targets, weights, *, sparse_compaction: bool = False,
@@ -110,7 +112,7 @@ def _workspaces(rows: int, hidden: int, vocab: int, local_chunk_size: int):
     backward = backward_workspace_bytes(rows, hidden, vocab, local_chunk_size)
     lib, shape = _lib.load(), _shape_struct(rows, hidden, vocab)
     # (the forward's part that may be smaller, an aligned copy of the head, keeps to the same bound)
-    forward = max(lib.ct_cutce_fwd_workspace_min_bytes(shape), min(lib.ct_cutce_fwd_workspace_bytes(shape), backward))
+    forward = max(lib.ct_cutce_fwd_workspace_min_bytes(shape), min(lib.ct_cutce_fwd_workspace_used_bytes(shape), backward))
     return int(forward), int(backward)
 
 

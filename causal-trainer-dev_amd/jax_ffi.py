@@ -321,15 +321,16 @@ def _cutce_shape(rows: int, hidden: int, vocab: int):
 
 def backward_workspace_bytes(rows: int, hidden: int, vocab: int, local_chunk_size: int) -> int:
     """Workspace of the backward. Without chunking the dlogits slab spans the vocabulary; with
-    ``local_chunk_size`` rows per chunk the slab is as large as the dlogits of one chunk of rows
-    would be (never below the kernels' minimum), and the vocabulary is walked in slabs."""
+    ``local_chunk_size`` rows per chunk the workspace is their share of that slab and a copy of the head
+    (never below the kernels' minimum), and the vocabulary is walked in slabs."""
 
     lib = _lib.load()
     shape = _cutce_shape(rows, hidden, vocab)
-    full, least = int(lib.ct_cutce_bwd_workspace_bytes(shape)), int(lib.ct_cutce_bwd_workspace_min_bytes(shape))
+    most, least = int(lib.ct_cutce_bwd_workspace_used_bytes(shape)), int(lib.ct_cutce_bwd_workspace_min_bytes(shape))
     if local_chunk_size <= 0 or local_chunk_size >= rows:
-        return full
-    return max(least, min(full, least + (full - least) * local_chunk_size // rows))
+        return most
+    full = int(lib.ct_cutce_bwd_workspace_bytes(shape))
+    return max(least, min(most, least + (full - least) * local_chunk_size // rows))
 
 
 @functools.lru_cache(maxsize=1)
@@ -341,7 +342,7 @@ def _cut_ce_impl():
         rows, width = hidden.shape
         lib = _lib.load()
         scalar = _struct((1,), jnp.float32)
-        workspace = int(lib.ct_cutce_fwd_workspace_bytes(_cutce_shape(rows, width, head.shape[1])))
+        workspace = int(lib.ct_cutce_fwd_workspace_used_bytes(_cutce_shape(rows, width, head.shape[1])))
         nll, weight_sum, lse, _, cache = _call(
             "ct_ffi_cutce_fwd",
             [scalar, scalar, _struct((rows,), jnp.float32), _struct((workspace,), jnp.uint8),
@@ -357,7 +358,7 @@ def _cut_ce_impl():
     def cut_ce_fwd(hidden, head, targets, weights, lm_head_trainable, sparse_compaction, local_chunk_size):
         cache_bytes = 0
         if not local_chunk_size:            # a chunked call asks for bounded memory: no logits cache
-            size = int(_lib.load().ct_cutce_logits_cache_bytes(_cutce_shape(*hidden.shape, head.shape[1])))
+            size = int(_lib.load().ct_cutce_logits_cache_used_bytes(_cutce_shape(*hidden.shape, head.shape[1])))
             cache_bytes = size if size <= LOGITS_CACHE_LIMIT_BYTES else 0
         nll, weight_sum, lse, cache = forward(hidden, head, targets, weights, sparse_compaction, cache_bytes)
         return (nll, weight_sum), (hidden, head, targets, weights, lse, cache)

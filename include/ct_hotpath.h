@@ -441,6 +441,14 @@ size_t ct_cutce_fwd_workspace_min_bytes(const ct_cutce_shape* shape);
 size_t ct_cutce_bwd_workspace_min_bytes(const ct_cutce_shape* shape);
 size_t ct_cutce_bwd_workspace_bytes(const ct_cutce_shape* shape);
 /*
+ * What a call without a lent panel (see ct_cutce_fwd_panel) uses of the preferred sizes and of the logits cache below. Less than
+ * those where the head is read in place, which takes the copy of 256 columns instead of all (64 rows x 150001, hidden 4096: 2 MB
+ * for 1.2 GB), the same otherwise. Either size will do.
+ */
+size_t ct_cutce_fwd_workspace_used_bytes(const ct_cutce_shape* shape);
+size_t ct_cutce_bwd_workspace_used_bytes(const ct_cutce_shape* shape);
+size_t ct_cutce_logits_cache_used_bytes(const ct_cutce_shape* shape);
+/*
  * Bytes of the optional logits cache (f32, vocabulary-major, rows and
  * vocabulary padded to 256; where vocab is no multiple of 8 also the aligned copy
  * of the head that both directions read). When the caller lends one to ct_cutce_fwd and
@@ -468,7 +476,7 @@ typedef struct ct_cutce_fwd_args {
   ct_cutce_shape shape;
   int32_t sparse_compaction; /* gather active rows first (same results; rows of a hidden tensor of
                               * more than 4 GiB stay in place, where the gather does not reach) */
-  void* logits_cache;        /* NULL, or ct_cutce_logits_cache_bytes() of device memory to fill */
+  void* logits_cache;        /* NULL, or at least ct_cutce_logits_cache_used_bytes() of device memory to fill */
   size_t logits_cache_bytes;
 } ct_cutce_fwd_args;
 

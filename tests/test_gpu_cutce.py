@@ -620,6 +620,33 @@ def test_head_read_in_place(ct, gpu, rows, width, vocab, both, cache, trainable)
     assert float(outcomes[0][0]) == pytest.approx(float((weights * (lse - picked)).double().sum()), rel=2e-5, abs=2e-3)
 
 
+@pytest.mark.parametrize("rows,width,vocab,columns", [
+    (64, 1536, 8209, 1),    # a slab for each tile column, the last one the tail's first half
+    (300, 1024, 12543, 3),  # a last slab of one column
+    (513, 768, 32021, 40),  # parts of dHidden that end inside of a slab
+])
+@pytest.mark.parametrize("trainable", [True, False])
+def test_head_read_in_place_in_slabs(ct, gpu, rows, width, vocab, columns, trainable):
+    """A bounded workspace: the vocabulary in slabs, the head in place all the same (no copy is made for a slab)."""
+
+    import ctypes
+
+    lib, shape = ct._lib.load(), ct._lib.CutceShape(rows, width, vocab)
+    case = _case(rows + vocab, rows, width, vocab)
+    least = lib.ct_cutce_bwd_workspace_min_bytes(ctypes.byref(shape))
+    size = least + (columns - 1) * ((rows + 255) // 256 * 256) * 256 * 2
+    assert size < lib.ct_cutce_bwd_workspace_used_bytes(ctypes.byref(shape))
+    whole = _gpu(ct, gpu, *case, 0.37, compaction=True, trainable=trainable)
+    with ct.profiling.KernelTimer() as timer:
+        slabs = _gpu(ct, gpu, *case, 0.37, compaction=True, trainable=trainable, workspace=size)
+    launches = timer.durations_ms()
+    assert len(launches["cutce_dlogits_kernel"]) > 1 and len(launches["cutce_prepare_kernel"]) == 2  # (one a direction)
+    assert relative_l2(slabs[3], whole[3]) <= 2.0 ** -8     # (f32 sums in another order, rounded to bf16 once)
+    assert not trainable or torch.equal(slabs[4], whole[4])
+    if trainable:
+        _check(slabs, *case, 0.37)
+
+
 @pytest.mark.parametrize("rows,cols,ld", [(7, 128, 256), (65, 64, 65), (1031, 200, 1280)])
 def test_transpose16_into_padded_rows(ct, gpu, rows, cols, ld):
     source = torch.randint(-2 ** 15, 2 ** 15, (rows, cols), dtype=torch.int16, device=gpu)

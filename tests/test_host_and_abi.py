@@ -154,6 +154,32 @@ def test_cutce_heads_that_both_directions_read_in_place(ct, rows, hidden, vocab,
     assert ct._lib.load().ct_cutce_head_in_place(ctypes.byref(shape)) == both
 
 
+@pytest.mark.parametrize("rows,hidden,vocab,forward,backward,both", [
+    (64, 4096, 150001, True, True, True), (768, 1024, 50257, True, True, False), (769, 1024, 50257, True, False, False),
+    (700, 512, 5001, False, False, False), (64, 1024, 16000, False, False, False)])
+def test_cutce_sizes_leave_out_a_copy_that_nobody_makes(ct, rows, hidden, vocab, forward, backward, both):
+    """A direction that reads the head in place uses the copy of 256 columns; whoever lends a panel still finds its bytes
+    in the sizes that the panel's are to be taken from."""
+
+    library, shape = ct._lib.load(), ct._lib.CutceShape(rows, hidden, vocab)
+    query = lambda name: int(getattr(library, name)(ctypes.byref(shape)))  # noqa: E731
+    panel, tail = query("ct_cutce_panel_bytes"), hidden * 256 * 2
+    least = query("ct_cutce_fwd_workspace_min_bytes")
+    logits = (rows + 255) // 256 * 256 * ((vocab + 255) // 256 * 256) * 4
+    assert query("ct_cutce_fwd_workspace_bytes") - least == panel and query("ct_cutce_logits_cache_bytes") - logits == panel
+    assert query("ct_cutce_fwd_workspace_used_bytes") - least == (tail if forward else panel)
+    assert query("ct_cutce_logits_cache_used_bytes") - logits == (tail if both else panel)
+    spared = query("ct_cutce_bwd_workspace_bytes") - query("ct_cutce_bwd_workspace_used_bytes")
+    assert spared == (panel - tail if backward else 0) and query("ct_cutce_bwd_workspace_bytes") > panel
+    # what the operators allocate
+    assert ct.cut_cross_entropy.logits_cache_bytes(rows, hidden, vocab) == query("ct_cutce_logits_cache_used_bytes")
+    assert ct.cut_cross_entropy.backward_workspace_bytes(rows, hidden, vocab) == query("ct_cutce_bwd_workspace_used_bytes")
+    bounded = ct.cut_cross_entropy.backward_workspace_bytes(rows, hidden, vocab, 16)
+    floor, share = query("ct_cutce_bwd_workspace_min_bytes"), query("ct_cutce_bwd_workspace_bytes")
+    # (a bound is the share of the whole that it has always been, and no more than is used)
+    assert bounded == min(floor + (share - floor) * 16 // rows, query("ct_cutce_bwd_workspace_used_bytes"))
+
+
 @pytest.mark.parametrize("torch_side", ["absent", "broken", "there"])
 def test_library_is_linked_whatever_becomes_of_the_torch_side(monkeypatch, tmp_path, torch_side):
     """libct_hotpath.so needs hipcc only: it is linked without torch, and before a torch side that fails to compile
