@@ -337,97 +337,6 @@ def fwd_private_clobbers():
                      ['"a%d"' % r for r in range(64)])
 
 
-# dK/dV, the products and the sums of a step as two plain sequences with the arithmetic between them: the order of the sums
-# that the stream below keeps.
-DKV_SLOTS = 5
-DKV_SCRATCH0 = 256 - 4 * DKV_SLOTS - 1  # one address temporary, then the fragment slots
-
-
-def dkv_slot(slot):
-    lo = DKV_SCRATCH0 + 1 + 4 * slot
-    return lo, lo + 3
-
-
-def dkv_sdp_sequence():
-    """S = Q K^T and dP = dO V^T of one (32 query rows x 32 keys) block, interleaved: per k-step
-    one MFMA of each chain. The fragment reads (Q, dO, V per k-step) run through a ring of
-    DKV_SLOTS registers quads: a read is issued as soon as the MFMA that used its slot has been
-    issued, so reads stay DKV_SLOTS fragments in front of their MFMAs.
-
-    operands: %0 S, %1 dP (read and written: the chains start from what the caller put there, the
-    per-row terms -lse / scale and -delta), %2-%9 row-fragment pointers (k-step), %10-%17 K
-    fragments (registers), %18 byte offset of this wavefront's V rows (scalar), %19 byte offset of
-    the stage (Q tile; the dO tile follows 8192 bytes later).
-    """
-    steps = 8
-    total = 3 * steps  # read r = 3 ks + which; which: 0 Q, 1 dO, 2 V
-    lines = ["s_waitcnt lgkmcnt(0)"]
-    state = {"issued": 0}
-
-    def load_next():
-        r = state["issued"]
-        if r >= total:
-            return []
-        state["issued"] += 1
-        ks, which = divmod(r, 3)
-        lo, hi = dkv_slot(r % DKV_SLOTS)
-        if which == 2:
-            return ["v_add_u32_e32 v%d, %%18, %%%d" % (DKV_SCRATCH0, 2 + ks),
-                    "ds_read_b128 v[%d:%d], v%d" % (lo, hi, DKV_SCRATCH0)]
-        return ["ds_read_b128 v[%d:%d], %%%d offset:%%19+%d" % (lo, hi, 2 + ks, which * 8192)]
-
-    for _ in range(DKV_SLOTS):
-        lines += load_next()
-    for ks in range(steps):
-        q_slot = dkv_slot((3 * ks) % DKV_SLOTS)
-        do_slot = dkv_slot((3 * ks + 1) % DKV_SLOTS)
-        v_slot = dkv_slot((3 * ks + 2) % DKV_SLOTS)
-        lines.append("s_waitcnt lgkmcnt(%d)" % (state["issued"] - (3 * ks + 1)))
-        lines.append("v_mfma_f32_32x32x16_bf16 %%0, v[%d:%d], %%%d, %%0" % (q_slot[0], q_slot[1], 10 + ks))
-        lines += load_next()
-        lines.append("s_waitcnt lgkmcnt(%d)" % (state["issued"] - (3 * ks + 3)))
-        lines.append("v_mfma_f32_32x32x16_bf16 %%1, v[%d:%d], v[%d:%d], %%1" % (do_slot[0], do_slot[1], v_slot[0],
-                                                                               v_slot[1]))
-        lines += load_next()
-        lines += load_next()
-    return lines + TAIL
-
-
-def dkv_acc_sequence(ahead=DKV_SLOTS, slots=DKV_SLOTS):
-    """dV[db] += P^T[step] dO(step, db) and dK[db] += dS^T[step] Q(step, db), interleaved: 16
-    MFMAs, each with one transposed fragment (2 ds_read_b64_tr_b16) read `ahead` fragments in
-    front of it.
-
-    operands: %0-%3 dV accumulators, %4-%7 dK accumulators, %8-%11 lo pointers (column block db),
-    %12-%15 hi pointers, %16-%17 P^T (k-step), %18-%19 dS^T (k-step), %20 byte offset of the
-    stage (Q tile; the dO tile follows 8192 bytes later).
-    """
-    order = [(step, db, which) for step in range(2) for db in range(4) for which in range(2)]  # which: 0 dV, 1 dK
-    n = len(order)
-    lines = ["s_waitcnt lgkmcnt(0)"]
-
-    def load(i):
-        step, db, which = order[i]
-        lo, _ = dkv_slot(i % slots)
-        off = "%%20+%d" % (step * 4096 + (8192 if which == 0 else 0))
-        return ["ds_read_b64_tr_b16 v[%d:%d], %%%d offset:%s" % (lo, lo + 1, 8 + db, off),
-                "ds_read_b64_tr_b16 v[%d:%d], %%%d offset:%s" % (lo + 2, lo + 3, 12 + db, off)]
-
-    for i in range(min(ahead, n)):
-        lines += load(i)
-    for i in range(n):
-        later = min(ahead - 1, n - 1 - i)
-        lines.append("s_waitcnt lgkmcnt(%d)" % (2 * later))
-        step, db, which = order[i]
-        lo, hi = dkv_slot(i % slots)
-        acc = db if which == 0 else 4 + db
-        aop = (16 if which == 0 else 18) + step
-        lines.append("v_mfma_f32_32x32x16_bf16 %%%d, %%%d, v[%d:%d], %%%d" % (acc, aop, lo, hi, acc))
-        if i + ahead < n:
-            lines += load(i + ahead)
-    return lines + TAIL
-
-
 class Stream:
     """Instruction list with in-order tracking of the LDS reads in flight (lgkmcnt)."""
 
@@ -468,7 +377,7 @@ def w_acc(i):
 # sums are a[0:127] for the whole kernel (w_acc: 0-3 dV, 4-7 dK) and never handed to the compiler, so a step does not end
 # with the wait states behind its last MFMA (1.5 % of the kernel): whoever reads the sums waits. Between its streams a
 # wavefront issues behind the other one of its SIMD (the other way round 0.5 to 1 % longer). The matrix pipe is busy 64 % of
-# the time with five fragment slots, 61.5 with the two sequences above and the arithmetic between them ([2, 8192, 16/16] whole
+# the time with five fragment slots, 61.5 as two sequences (products, sums) with the arithmetic between them ([2, 8192, 16/16] whole
 # rows); [4, 4096, 32/8] documents of 64 to 4096 682 -> 642 us, [2, 8192, 16/16] of 64 to 2000 235 -> 224. Five slots instead
 # of six 0.2 % longer, seven 0.5 % shorter in launches of one round and 0.7 % longer in large ones.
 DKVS_SLOTS = 6
@@ -596,70 +505,6 @@ def dkv_step_sequence(mask, stores):
             st.emit(line)
     assert not fill[len(mfmas)] and state["issued"] == len(reads)
     return st.lines + ["s_setprio 0"]
-
-
-# dQ, the two halves of a key tile as two plain sequences each: the order of the sums that the stream below keeps.
-DQ_HEAD = ["s_waitcnt lgkmcnt(0)"]
-DQ_TAIL = TAIL
-
-
-def dq_sdp_half_sequence(ahead=4, slots=4):
-    """dQ kernel, one 32-key half of a key tile: S^T = K_half Q^T and dP^T = V_half dO^T, the two
-    chains alternating (16 MFMAs, one ds_read_b128 fragment each, read `ahead` fragments in front).
-
-    operands: %0 S^T, %1 dP^T (written), %2-%9 row-fragment pointers (k-step), %10-%17 Q fragments,
-    %18-%25 dO fragments, %26 byte offset of the half's K rows, %27 that of its V rows.
-    """
-    n = 16
-    lines = list(DQ_HEAD)
-
-    def load(i):
-        ks, which = divmod(i, 2)
-        lo, hi = slot_regs(i % slots)
-        return ["ds_read_b128 v[%d:%d], %%%d offset:%%%d" % (lo, hi, 2 + ks, 26 + which)]
-
-    for i in range(min(ahead, n)):
-        lines += load(i)
-    for i in range(n):
-        later = min(ahead - 1, n - 1 - i)
-        lines.append("s_waitcnt lgkmcnt(%d)" % later)
-        ks, which = divmod(i, 2)
-        lo, hi = slot_regs(i % slots)
-        src_c = "0" if ks == 0 else "%%%d" % which
-        lines.append("v_mfma_f32_32x32x16_bf16 %%%d, v[%d:%d], %%%d, %s" % (which, lo, hi, (18 if which else 10) + ks, src_c))
-        if i + ahead < n:
-            lines += load(i + ahead)
-    return lines + DQ_TAIL
-
-
-def dq_acc_half_sequence(ahead=4, slots=4):
-    """dQ kernel, one 32-key half: dQ^T[db] += K_half^T frag(step, db) * dS^T[step], 8 MFMAs, each
-    fragment = 2 ds_read_b64_tr_b16.
-
-    operands: %0-%3 accumulators, %4-%7 lo pointers (column block db), %8-%11 hi pointers,
-    %12-%13 dS fragments (k-step), %14 byte offset of the half's K rows.
-    """
-    n = 8
-    lines = list(DQ_HEAD)
-
-    def load(i):
-        step, db = divmod(i, 4)
-        lo, _ = slot_regs(i % slots)
-        off = "%%14+%d" % (step * 4096)
-        return ["ds_read_b64_tr_b16 v[%d:%d], %%%d offset:%s" % (lo, lo + 1, 4 + db, off),
-                "ds_read_b64_tr_b16 v[%d:%d], %%%d offset:%s" % (lo + 2, lo + 3, 8 + db, off)]
-
-    for i in range(min(ahead, n)):
-        lines += load(i)
-    for i in range(n):
-        later = min(ahead - 1, n - 1 - i)
-        lines.append("s_waitcnt lgkmcnt(%d)" % (2 * later))
-        step, db = divmod(i, 4)
-        lo, hi = slot_regs(i % slots)
-        lines.append("v_mfma_f32_32x32x16_bf16 %%%d, v[%d:%d], %%%d, %%%d" % (db, lo, hi, 12 + step, db))
-        if i + ahead < n:
-            lines += load(i + ahead)
-    return lines + DQ_TAIL
 
 
 # dQ, a key tile of 64 keys as one stream: S and dP of its first half, S of the second with the first half's dS behind its

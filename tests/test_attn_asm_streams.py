@@ -101,9 +101,7 @@ class Model:
 
 def _sequences(gen):
     sequences = {
-        "pv": gen.pv_sequence(4, 4), "qk": gen.qk_sequence(4, 4), "dq_sdp_half": gen.dq_sdp_half_sequence(),
-        "dq_acc_half": gen.dq_acc_half_sequence(), "dkv_sdp": gen.dkv_sdp_sequence(), "dkv_acc": gen.dkv_acc_sequence(),
-        "dkvw_step": gen.dkvw_step_sequence(), "dkvw_masked": gen.dkvw_step_sequence(masked=True),
+        "pv": gen.pv_sequence(4, 4), "qk": gen.qk_sequence(4, 4), "dkvw_step": gen.dkvw_step_sequence(), "dkvw_masked": gen.dkvw_step_sequence(masked=True),
         "dkvw_run": gen.dkvw_run_sequence(),
     }
     for mask in ("", "ends", "rows"):
@@ -188,7 +186,7 @@ def test_wide_stream_structure(gen):
 @pytest.mark.parametrize("mask", ["", "ends", "rows"])
 @pytest.mark.parametrize("stores", [False, True])
 def test_dkv_step_stream(gen, mask, stores):
-    """One step of the dK/dV kernel: the MFMAs of every sum in the order of the plain sequences, the arithmetic of every
+    """One step of the dK/dV kernel: the MFMAs of every sum in the order of their k-steps, the arithmetic of every
     element between the products and the sums that need it, the mask in front of it, the stores behind it."""
 
     lines = gen.dkv_step_sequence(mask, stores)
@@ -238,7 +236,7 @@ def test_dkv_step_stream(gen, mask, stores):
 
 @pytest.mark.parametrize("masked", [False, True])
 def test_dq_step_stream(gen, masked):
-    """One key tile of the dQ kernel: the MFMAs of every sum in the order of the two half sequences, the arithmetic of every
+    """One key tile of the dQ kernel: the MFMAs of every sum in the order of the keys, the arithmetic of every
     element between its products and the sums that need it, no block written before its last reader."""
 
     lines = gen.dq_step_sequence(masked)
