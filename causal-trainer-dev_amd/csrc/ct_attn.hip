@@ -793,9 +793,11 @@ static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool redu
 }
 
 // Which dK/dV kernel runs for head dimension 128 when the caller leaves the choice open: the wide
-// kernel's streams pay off where runs of all-allowed steps are long, which needs long segments;
-// measured 8 % faster at S = 32768 with segments up to the whole row and 3 % slower at S = 4096
-// with segments of 64 to 4096 positions.
+// kernel's streams pay off where runs of all-allowed steps are long, which needs long segments. The line is of a
+// narrow kernel whose steps were not streams yet (the wide one 8 % faster at S = 32768 with segments up to the whole row). With
+// the present one, recomputing backward, us, narrow / wide: [1, 16384, 32/8 heads] whole rows 6576 / 6335, 512 to 2048 607 / 690;
+// [1, 65536, 8/2] whole rows 25939 / 24721, images 1502 / 1773; [1, 32768, 64/8] whole rows 50492 / 50925, 512 to 32768
+// 23413 / 25354, 64 to 300 1021 / 1164; [2, 8192, 32/8] whole rows 3338 / 3242, 512 to 2048 648 / 702.
 constexpr int kWideDkvFromSeq = 16384;
 
 // One pass of the dK/dV kernel over the KV heads p.kvh_base ... (all of them unless dS is stored).
@@ -854,8 +856,7 @@ static int launch_schedule(hipStream_t stream, const AttnParams& p, int kvh_side
   return scope7.done();
 }
 
-// Recompute form: the work list; dQ per query tile (evaluates S and dP itself and computes delta
-// and -lse / scale for its rows on the way); dK/dV per key tile; the sum of split chunks.
+// dQ per query tile: evaluates S and dP itself and computes delta and -lse / scale for its rows on the way.
 template <int D>
 static int dispatch_dq(hipStream_t stream, const AttnParams& p) {
   switch (heads_per_group(p.Hq, p.Hkv)) {
@@ -865,6 +866,7 @@ static int dispatch_dq(hipStream_t stream, const AttnParams& p) {
   }
 }
 
+// Recompute form: the work list; dQ; dK/dV per key tile; the sum of split chunks.
 template <int D>
 static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool wide, bool list_kept) {
   int rc = list_kept ? 0 : launch_schedule<D>(stream, p, p.Hkv);

@@ -301,7 +301,8 @@ struct CutceRowWork {
 // the counting the longer part (69 us there).
 // Few long rows are shared by several wavefronts each, for more workgroups: a compute unit moves about 50 GB/s (a wavefront
 // per row / four, us: 64 rows, d = 6400 13.4 / 8.4, 250 10.0 / 7.4, 1000 12.1 / 9.8; d = 2048 6.8 / 6.1, 6.0 / 6.1,
-// 6.8 / 6.9, and 1024 and less 0.2 longer; two, 2000 rows: d = 2048 9.0 / 8.2, 6400 13.3 / 12.5).
+// 6.8 / 6.9, and 1024 and less 0.2 longer, d = 1280 to 1792 0.8 less to 0.7 longer; two, 2000 rows: d = 2048 9.0 / 8.2, 6400
+// 13.3 / 12.5).
 constexpr int kMostRowRounds = 64;
 __host__ __device__ inline int row_rounds(int rows) { return min((rows + 4095) / 4096, kMostRowRounds); }
 __host__ __device__ inline int row_waves(int rows, int d) { return d < 2048 || rows > 2048 ? 1 : rows > 1024 ? 2 : 4; }

@@ -12,7 +12,8 @@ Run ``python gen_attn_asm.py > ct_attn_asm.inc`` after editing; the output is co
 
 SCRATCH0 = 240
 # The compiler cannot see the MFMAs inside an asm statement, so it will not insert the wait
-# states that a vector ALU read of a fresh MFMA result needs; the sequences end with them.
+# states that a vector ALU read of a fresh MFMA result needs; the sequences end with them (the steps of dQ and dK/dV, whose sums
+# stay in accumulation registers, leave them to whoever reads those).
 TAIL = ["s_nop 15", "s_nop 7"]
 
 def slot_regs(slot):
