@@ -792,13 +792,21 @@ static int dispatch_dq_blocks(hipStream_t stream, const AttnParams& p, bool redu
                    : launch_dq_blocks<D, 1, 1>(stream, p, reduce);
 }
 
-// Which dK/dV kernel runs for head dimension 128 when the caller leaves the choice open: the wide
-// kernel's streams pay off where runs of all-allowed steps are long, which needs long segments. The line is of a
-// narrow kernel whose steps were not streams yet (the wide one 8 % faster at S = 32768 with segments up to the whole row). With
-// the present one, recomputing backward, us, narrow / wide: [1, 16384, 32/8 heads] whole rows 6576 / 6335, 512 to 2048 607 / 690;
-// [1, 65536, 8/2] whole rows 25939 / 24721, images 1502 / 1773; [1, 32768, 64/8] whole rows 50492 / 50925, 512 to 32768
-// 23413 / 25354, 64 to 300 1021 / 1164; [2, 8192, 32/8] whole rows 3338 / 3242, 512 to 2048 648 / 702.
+// Which dK/dV kernel runs for head dimension 128 when the caller leaves the choice open: the wide one's streams, of one wavefront
+// per SIMD, are ahead only where nearly every step of a long walk is all-allowed (whole rows) and every compute unit has key tiles
+// to the end. Recomputing backward of [B, S, heads / KV heads], us, narrow / wide, 50 calls:
+//   whole rows, (key tile, KV head) pairs beyond the places: [1, 16384, 32/8] 6779 / 6548, [2, 16384, 16/4] 6710 / 6475; where KV
+//     heads have no group or one of eight 3275 / 3294 ([1, 16384, 16/16]), 53789 / 54627 ([1, 32768, 64/8])
+//   up to 320 pairs: [1, 16384, 2/1] 677 / 724, 8/2 1844 / 1950, [1, 32768, 8/1] 7256 / 7698, [1, 20480, 6/2] 2118 / 2220
+//   packed documents, of 512 to the whole row: 0.80 to 0.98 of the wide one's time ([1, 32768, 64/8] 25121 / 26978), of 512 to 2048
+//     0.82 to 0.94, of 64 to 300 0.78 to 0.87, image blocks 0.84 to 0.94.
+// The documents are the device's to see: long rows launch both kernels, the wide one first, and count the visited blocks.
 constexpr int kWideDkvFromSeq = 16384;
+static int wide_least_blocks(const AttnParams& p) {
+  const long nrb = p.S / 32, pairs = (long)p.B * (p.S / kDkvKeys) * p.Hkv;
+  const long whole = p.B * (nrb * (nrb + 1) / 2);
+  return pairs <= kDkvSlots ? INT_MAX : (int)std::min(whole * 9 / 10, (long)INT_MAX);
+}
 
 // One pass of the dK/dV kernel over the KV heads p.kvh_base ... (all of them unless dS is stored).
 template <int D>
@@ -810,6 +818,10 @@ static int launch_dkv(hipStream_t stream, const AttnParams& p, bool wide) {
       CT_ENSURE_LDS("ct_attn_bwd", &attn_dkv_wide_kernel, DkvWideLds::kTotalBytes);
       LaunchScope scope("attn_dkv_wide_kernel", stream);
       hipLaunchKernelGGL(attn_dkv_wide_kernel, dim3(grid), dim3(128), DkvWideLds::kTotalBytes, stream, p);
+      if (p.dkv_by_blocks) {  // (timed with it: one of the two exits at once)
+        CT_ENSURE_LDS("ct_attn_bwd", (&attn_dkv_kernel<D, false>), smem);
+        hipLaunchKernelGGL((attn_dkv_kernel<D, false>), dim3(grid), dim3(256), smem, stream, p);
+      }
       return scope.done();
     }
   }
@@ -1146,6 +1158,7 @@ extern "C" int32_t ct_attn_bwd(void* stream, const ct_attn_bwd_args* a) {
   p.dkv_max_partials = L.max_partials;
   p.kvh_base = 0;
   p.kvh_count = a->kv_heads;
+  if (a->head_dim == 128 && a->seq >= kWideDkvFromSeq) p.wide_least_blocks = wide_least_blocks(p);
   hipStream_t s = (hipStream_t)stream;
   if (plan.spill) {
     p.ds = ws + plan.ds;
@@ -1154,8 +1167,8 @@ extern "C" int32_t ct_attn_bwd(void* stream, const ct_attn_bwd_args* a) {
     return a->head_dim == 128 ? dispatch_bwd_blocks<128>(s, p, plan.kvh_per_pass, false, list_kept)
                               : dispatch_bwd_blocks<64>(s, p, plan.kvh_per_pass, false, list_kept);
   }
-  const bool wide = a->head_dim == 128 &&
-                    (wide_forced || (kernel_choice == 0 && a->seq >= kWideDkvFromSeq));
+  p.dkv_by_blocks = kernel_choice == 0 && p.wide_least_blocks;
+  const bool wide = wide_forced || p.dkv_by_blocks;
   return a->head_dim == 128 ? dispatch_bwd_recompute<128>(s, p, wide, list_kept)
                             : dispatch_bwd_recompute<64>(s, p, wide, list_kept);
 }

@@ -32,6 +32,15 @@ CT_DEVICE int ds_blocks_per_head(const AttnParams& p) {
   return lane_value(wave_scan(blocks), 63);
 }
 CT_DEVICE bool dq_recomputes(const AttnParams& p) { return uniform(p.dkv_header[kDqRecomputes]) != 0; }
+CT_DEVICE void leave_dkv_choice(const AttnParams& p) {
+  if (!p.wide_least_blocks || threadIdx.x >= 64) return;
+  const int blocks = ds_blocks_per_head(p);
+  if (threadIdx.x == 0) p.dkv_header[kDkvWide] = blocks >= p.wide_least_blocks;
+}
+// Whether this launch's dK/dV kernel is not the one that the documents call for.
+CT_DEVICE bool other_dkv_kernel(const AttnParams& p, bool wide) {
+  return p.dkv_by_blocks && (uniform(p.dkv_header[kDkvWide]) != 0) != wide;
+}
 
 // ---------------------------------------------------------------------------
 // dQ
@@ -780,6 +789,7 @@ CT_DEVICE void dkv_schedule(const int* meta, int B, int S, int Hkv, int g, int m
 
 template <int D>
 __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, int kvh_side_by_side) {
+  if (D == 128) leave_dkv_choice(p);
   dkv_schedule<D>(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
                p.dkv_entries, p.dq_counters, kDqCounters);
 }
@@ -792,6 +802,7 @@ __global__ __launch_bounds__(1024) void attn_bwd_setup_kernel(AttnParams p, int 
   const bool recompute = p.ds_most_blocks && ds_blocks_per_head(p) > p.ds_most_blocks;
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) p.dkv_header[kDqRecomputes] = recompute;
+    if (D == 128) leave_dkv_choice(p);
     dkv_schedule<D>(p.meta, p.B, p.S, kvh_side_by_side, p.Hq / p.Hkv, p.dkv_max_entries, p.dkv_max_partials, p.dkv_header,
                  p.dkv_entries, p.dq_counters, kDqCounters);
     return;
@@ -973,7 +984,7 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   const int2 work_entry = p.dkv_entries[entry];
   int tile = uniform(work_entry.x), packed = uniform(work_entry.y);
   asm volatile("" : "+s"(tile), "+s"(packed));
-  if (entry >= uniform(p.dkv_header[0])) return;
+  if (entry >= uniform(p.dkv_header[0]) || (D == 128 && !SPILL && other_dkv_kernel(p, false))) return;
   const int chunk = packed & 255, nsplit = (packed >> 8) & 255, slot0 = (unsigned)packed >> 16;
   const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
   const int g = p.Hq / p.Hkv;

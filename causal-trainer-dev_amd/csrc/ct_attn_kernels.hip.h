@@ -64,6 +64,8 @@ struct AttnParams {
   char* ds;              // dS region of the pass, null when dQ recomputes S and dP
   size_t ds_row_blocks;  // dS blocks reserved per (query head, batch row)
   int ds_most_blocks;    // head dimension 64: with more dS blocks per query head than this dQ recomputes after all; 0: no such choice
+  int wide_least_blocks; // head dimension 128, long rows: from as many blocks per query head on dK/dV is the wide kernel's, ...
+  bool dkv_by_blocks;    // ... where the call leaves that open
 };
 
 // Whether dQ of head dimension 64 is the faster one from stored dS blocks or recomputed goes by how many blocks there are:
@@ -71,6 +73,8 @@ struct AttnParams {
 // know, so where it matters (most_stored_blocks) the kernel that makes the work list counts the blocks and leaves the answer in
 // the list's header; both dQ kernels are launched, and the workgroups of the one that is not wanted exit at once.
 constexpr int kDqRecomputes = 2;  // place in the header
+// Likewise for the two dK/dV kernels of head dimension 128 in long rows (wide_least_blocks); every list has that answer.
+constexpr int kDkvWide = 3;
 
 // ---------------------------------------------------------------------------
 // K/V tile staging: global -> registers -> swizzled LDS.

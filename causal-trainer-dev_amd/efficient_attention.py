@@ -266,7 +266,7 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     ``dkv_kernel`` (``"narrow"`` / ``"wide"``) and ``dq_form`` (``"recompute"`` / ``"from_ds"``) pin a
     kernel or a form of the backward for this call (``ct_attn_bwd_args.variant``); ``None`` leaves
     the choice to the library, which is what training code does (the dK/dV kernel goes by sequence
-    length; dQ comes from stored dS blocks at rows of up to 4096 positions when their workspace is at
+    length, and in long rows by the documents, on the device; dQ comes from stored dS blocks at rows of up to 4096 positions when their workspace is at
     most 4 GiB, and from a recomputing kernel otherwise; from 8193 row blocks of head dimension 64 on, the
     documents decide between the two on the device). ``workspace_bytes`` overrides the size of the scratch buffer (default: what
     the library asks for the chosen form); ``workspace`` (a :class:`BackwardWorkspace`) keeps the

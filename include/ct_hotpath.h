@@ -143,7 +143,8 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * per call, nothing is process-wide. Low 4 bits, the dK/dV kernel at head dimension 128:
  * NARROW = two wavefronts per SIMD with 32 keys each, WIDE = one wavefront per SIMD with 64
  * keys, the (dK, dV) sums in the accumulation registers and each step one generated
- * instruction stream (left open: WIDE from 16384 positions on, NARROW below). Bits 4-7, how dQ
+ * instruction stream (left open: NARROW below 16384 positions; from there on the batch's number of visited blocks decides on
+ * the device, WIDE for whole rows on a full device, and both are launched, one to exit at once). Bits 4-7, how dQ
  * is formed: RECOMPUTE = a query-stationary kernel evaluates S and dP a second time (the
  * reference's _local_attention_dq, src/kernels/efficient_attention.py:985-1267); FROM_DS = the
  * dK/dV kernel (NARROW) stores its bf16 dS blocks in the workspace and dQ is the product of those

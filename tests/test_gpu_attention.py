@@ -225,6 +225,33 @@ def test_default_choices_of_the_backward(ct, gpu, seq, expected):
         _run_gpu(ct, gpu, q, k, v, dout, ids, None, 128 ** -0.5, dq_form="from_ds", dkv_kernel="wide")
 
 
+@pytest.mark.parametrize("heads,max_len", [((5, 5), 16384), ((5, 5), 3000), ((4, 4), 16384), ((5, 1), 700)], ids=str)
+def test_documents_choose_the_dkv_kernel_of_long_rows(ct, gpu, heads, max_len):
+    """From 16384 positions on both dK/dV kernels are launched and one of them works: the wide one for whole rows with more key
+    tiles than places (5 KV heads), the narrow one for the others. Both give the same bits; the results' memory holds NaN
+    before the call, so that a tile nobody worked on shows."""
+
+    q_heads, kv_heads = heads
+    rng = np.random.default_rng(max_len + q_heads)
+    seq = 16384
+    ids = np.ones((1, seq), np.int32) if max_len == seq else _layout(rng, 1, seq, max_len=max_len)
+    profile = ct.resolve_attention_profile((1, seq, q_heads, 128), (1, seq, kv_heads, 128), None, has_attention_end=False)
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile)
+    generator = torch.Generator().manual_seed(max_len)
+    q, k, v, dout = (torch.randn((1, seq, n, 128), generator=generator).to(torch.bfloat16).to(gpu)
+                     for n in (q_heads, kv_heads, kv_heads, q_heads))
+    out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+    print(heads, max_len, flush=True)
+    pinned = ct.attention_backward(q, k, v, metadata, out, lse, dout, dkv_kernel="narrow", dq_form="recompute")
+    kept = ct.BackwardWorkspace()
+    for workspace in (None, kept, kept):
+        stale = [torch.full_like(t, float("nan")) for t in pinned]    # (what the results' memory holds)
+        del stale
+        got = ct.attention_backward(q, k, v, metadata, out, lse, dout, dq_form="recompute", workspace=workspace)
+        for a, b in zip(pinned, got):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("form", ["recompute", "from_ds"])
 def test_kept_work_list(ct, gpu, form):
     """Layers that share a packing can share the backward's scratch buffer and the dK/dV work list
