@@ -4,9 +4,10 @@
 // One workgroup of NW wavefronts per query tile, launched heaviest tile first and dealt by the
 // hardware. Nothing runs in step across workgroups: what one of them spends on its prologue, its row
 // maxima and its stores is another one's time on the matrix pipe, and no hand-written interleaving is
-// needed. At head dimension 64 the loop is bound by the vector ALU (about 140 instructions, 32 of them
-// exponentials, against 16 MFMAs per 64 keys), and 4 wavefronts per SIMD at 103 registers keep it
-// busy; the 8-wavefront workgroup in two half-step-shifted groups that this replaces had 2. The forms:
+// needed. At head dimension 64 the loop is bound by the vector ALU (57 instructions, 16 of them exponentials, against 8 MFMAs
+// per 32 keys of whole rows: 365 clocks for that mix by four wavefronts on end, 480 here; the matrix pipe is busy half of the
+// time), and 4 wavefronts per SIMD at 104 registers keep it busy; the 8-wavefront workgroup in two half-step-shifted groups
+// that this replaces had 2. The forms:
 //
 //   KS = 1  a wavefront takes all keys of its 32 query rows
 //   KS = 2  two wavefronts share them, 32 keys each per step: half the chain of steps per row
@@ -20,6 +21,10 @@
 //   (2, 4096, 8/8, 64, 4.2)        37.3 -> 20.4  KS = 2     (3, 2944, 24/8, 64, 5.7) 72.7 -> 45.4  KS = 2
 //   (3, 4224, 48/8, 64, 2.3)      121.2 -> 68.9  KS = 1     (8, 4096, 32/8, 64, 32)   796 -> 660   KS = 1
 //   (3, 2560, 8/8, 128, 7.8)       55.3 -> 42.0  KS = 2     (6, 1280, 32/16, 128, 0.4) 61.1 -> 46.2  KS = 1
+// The maximum of a piece formed before its exponents / only where their sum asks for it, and padded row blocks through the loop / by
+// themselves, us:
+//   (8, 4096, 32/8, 64; rows) 608 / 590     (3, 2944, 24/8, 64; 40-2944) 39.5 / 38.7      (2, 1024, 8/8, 64; 32-512) 7.6 / 7.6
+//   (3, 3072, 6/2, 128; images) 50.9 / 46.4 (4, 1024, 12/4, 128; 172-914) 21.4 / 20.5     (8, 640, 6/2, 64; 319-424) 9.0 / 9.1
 #pragma once
 
 #include "ct_attn_kernels.hip.h"
@@ -87,6 +92,17 @@ attn_fwd_split_kernel(AttnParams p) {
   int t = any ? first_tile * 64 / Stage::kKeys : 0;
   const int last = any ? (last_tile * 64 + 63) / Stage::kKeys : -1;
 
+  // Row blocks of padding (a quarter of the workgroups at (3, 2944, 24/8, 64), 6000 clocks each on the way below): zeros.
+  if (!any) {
+    if (share != 0) return;
+    bf16* rows = p.out + (((size_t)b * p.S + rb * 32) * p.Hq + h) * D;
+    constexpr int kPerRow = D / 8;
+#pragma unroll
+    for (int i = 0; i < 32 * kPerRow / 64; ++i)
+      store_global16(rows + (size_t)(i * (64 / kPerRow) + l / kPerRow) * p.Hq * D + l % kPerRow * 8, u32x4{0, 0, 0, 0});
+    if (l < 32) p.lse[((size_t)b * p.S + rb * 32 + l) * p.Hq + h] = 0.f;
+    return;
+  }
   const TileDma<Stage::kKeys, D / 8, NW * 64> dma((size_t)p.Hkv * D * 2);
   const char* kbase = reinterpret_cast<const char*>(p.k + ((size_t)b * p.S * p.Hkv + kvh) * D);
   const char* vbase = reinterpret_cast<const char*>(p.v + ((size_t)b * p.S * p.Hkv + kvh) * D);
@@ -121,11 +137,9 @@ attn_fwd_split_kernel(AttnParams p) {
   f32x16 oacc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) oacc[db] = zero16();
-  float m_run = kNegInf;  // softmax reference (a recent running max), log2 domain
-  // What a piece takes of it: the score that moves it and the term of its exponents (0 as long as nothing is visible).
-  // Kept where registers are to spare: at head dimension 64, whose loop the vector ALU bounds, with the addresses below 12 of
-  // the 90 instructions of a piece (1 to 4 % of the kernel; at 128, where 256 registers are in use, 0.7 % slower).
-  float moves_at = kNegInf, minus_m = 0.f;
+  // softmax reference (a recent running max, log2 domain) and the term of the exponents that it makes
+  float m_run = kNegInf, minus_m = kUnseen;
+  bool fresh = true;      // no piece yet
   float l_run = 0.f;      // this lane's share of the running sum
   const int own = share * SUB * KB * RowFragOffsets<D / 8>::kRowBlockBytes;  // this wavefront's keys in a stage
   RowFragOffsets<D / 8> ro(lds0 + own);
@@ -150,17 +164,26 @@ attn_fwd_split_kernel(AttnParams p) {
     } else {
 #pragma unroll
       for (int i = 0; i < KB; ++i) s[i] = zero16();
+      if constexpr (KB == 1) {
+        fragments_ahead<D / 16, 4>([&](int kk) { return ro.load(OFF + Stage::kK, 0, kk); },
+                                   [&](int kk, bf16x8 k) { s[0] = mfma32(k, qf[kk], s[0]); });
+      } else {
 #pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk)
+        for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
-        for (int i = 0; i < KB; ++i) s[i] = mfma32(ro.load(OFF + Stage::kK, i, kk), qf[kk], s[i]);
+          for (int i = 0; i < KB; ++i) s[i] = mfma32(ro.load(OFF + Stage::kK, i, kk), qf[kk], s[i]);
+      }
     }
     // (a piece with one shared id turns the id test into a per-query predicate)
     const int k_uniform = uniform(keys.uniform);
-    if (mine.uniform == 0 || mine.uniform != k_uniform || key0 + KB * 32 - 1 > mine.end_min) {
+    const bool masked = mine.uniform == 0 || mine.uniform != k_uniform || key0 + KB * 32 - 1 > mine.end_min;
+    if (masked) {
       const int seg_cmp = seg_q != 0 ? seg_q : -1;
       int last_rel = end_q - key0 - 4 * half;
-      if (k_uniform == 0) {
+      if (k_uniform == 0 && key0 + KB * 32 - 1 <= mine.end_min) {
+#pragma unroll
+        for (int i = 0; i < KB; ++i) mask_block_t<true, false>(ids, seg_cmp, last_rel, i, s[i]);
+      } else if (k_uniform == 0) {
 #pragma unroll
         for (int i = 0; i < KB; ++i) mask_block_t<true, true>(ids, seg_cmp, last_rel, i, s[i]);
       } else {
@@ -169,37 +192,52 @@ attn_fwd_split_kernel(AttnParams p) {
         for (int i = 0; i < KB; ++i) mask_block_t<false, true>(ids, seg_cmp, last_rel, i, s[i]);
       }
     }
-    float mx = kNegInf;
+    f32x16 e[KB];
+    auto exponents = [&] {
+      float sum = -0.f;  // (the neutral element, so that the first addition falls away)
 #pragma unroll
-    for (int i = 0; i < KB; ++i)
+      for (int i = 0; i < KB; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[i][r]);
-    mx = pair_max(mx) * kLog2e;
-    if (__any(mx > (D == 64 ? moves_at : m_run + kRescaleSlack))) {  // (lazily, as attn_fwd_item)
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = exp2_fast(m_run - (m_new == kNegInf ? 0.f : m_new));
-      l_run *= alpha;
-#pragma unroll
-      for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
-      m_run = m_new;
-      moves_at = m_new + kRescaleSlack;
-      minus_m = m_new == kNegInf ? 0.f : -m_new;
+        for (int r = 0; r < 16; ++r) {
+          e[i][r] = exp2_fast(fmaf(s[i][r], kLog2e, minus_m));
+          sum += e[i][r];
+        }
+      return sum;
+    };
+    // Where the rows have a reference the sum of a piece says whether it has to move, and the maximum, 15 of 72 vector
+    // instructions and a chain in front of the exponents, is formed only then; where rows are likely to see their first key (a
+    // masked piece, or the first) it is formed at once. A sum that is infinite or no number asks for the maximum as well.
+    float psum = 0.f;
+    bool settled = !(masked || fresh);
+    fresh = false;
+    if (settled) {
+      psum = exponents();
+      settled = __builtin_amdgcn_ballot_w64(!(psum <= kMostSum)) == 0;
     }
-    const float minus = D == 64 ? minus_m : m_run == kNegInf ? 0.f : -m_run;
-    float psum = D == 64 ? -0.f : 0.f;  // (the neutral element, so that the first addition falls away)
+    if (!settled) {
+      float mx = kNegInf;
 #pragma unroll
-    for (int i = 0; i < KB; ++i)
+      for (int i = 0; i < KB; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[i][r] = exp2_fast(fmaf(s[i][r], kLog2e, minus));
-        psum += s[i][r];
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[i][r]);
+      mx = pair_max(mx) * kLog2e;
+      if (__any(mx > m_run + kMovesBy)) {
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = exp2_fast(m_run - (m_new == kNegInf ? 0.f : m_new));
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+        m_run = m_new;
+        minus_m = m_new == kNegInf ? kUnseen : -m_new;
       }
+      psum = exponents();
+    }
     l_run += psum;
     bf16x8 pf[2 * KB];
 #pragma unroll
-    for (int i = 0; i < 2 * KB; ++i) pf[i] = pack_acc8(s[i >> 1], i & 1);
+    for (int i = 0; i < 2 * KB; ++i) pf[i] = pack_acc8(e[i >> 1], i & 1);
     if constexpr (kSequences) {
       pv_sequence_128<OFF + Stage::kV>(to, pf, oacc);
     } else {

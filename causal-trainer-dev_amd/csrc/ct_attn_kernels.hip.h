@@ -497,6 +497,12 @@ CT_DEVICE f32x16 fwd_acc_read() {
 // ---------------------------------------------------------------------------
 constexpr int kFwdWaves = 8;
 constexpr float kRescaleSlack = 8.f;
+// Where the maximum is formed only once a lane's sum of 16 or 32 probabilities says that the reference has to move: that sum
+// (probabilities stay below 2^8, as above); how far the maximum then lies above the reference at least (log2 of kMostSum / 32);
+// and the term of the exponents in a row that has seen no key: so large that any finite score makes the sum infinite.
+constexpr float kMostSum = 256.f;
+constexpr float kMovesBy = 2.9f;
+constexpr float kUnseen = 3.402823466e38f;
 
 template <int D>
 struct VkStage {

@@ -1226,3 +1226,40 @@ def test_forms_of_dq_from_stored_blocks(ct, gpu, shape, with_ends):
     assert (stored[0][0][torch.from_numpy(ids).to(gpu) == 0] == 0).all()
     for a, b in zip(stored[0], expected):
         assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
+
+
+@pytest.mark.parametrize("shape", [(1, 1024, 28, 4, 64), (8, 1024, 28, 4, 64), (1, 1024, 20, 4, 128), (3, 1024, 24, 4, 128),
+                                   (1, 1024, 4, 4, 64), (1, 1024, 4, 4, 128), (2, 2048, 32, 8, 128)], ids=str)
+def test_scores_that_rise_and_fall_by_hundreds(ct, gpu, shape):
+    """The forward's reference of the softmax follows scores that jump from one piece of 32 keys to the next, in rows whose
+    first visited blocks hold ids around theirs but none of them, and in rows of padding, in every form of the forward."""
+
+    batch, seq, q_heads, kv_heads, dim = shape
+    rng = np.random.default_rng(5)
+    scale, pieces = 0.125, seq // 32
+    ids = np.full((batch, seq), 2, np.int32)
+    ids[:, :64] = np.where(np.arange(64) % 2, 3, 1)      # around 2, without it
+    ids[:, 512:528], ids[:, 528:700], ids[:, seq - 160:] = 5, 6, 0
+    q = 0.3 * rng.standard_normal((batch, seq, q_heads, dim))
+    k = 0.3 * rng.standard_normal((batch, seq, kv_heads, dim))
+    v = rng.standard_normal((batch, seq, kv_heads, dim))
+    q[..., 0] = 16.0                                     # a score is about twice the key's first element
+    levels = rng.choice([-250.0, -150.0, -40.0, 0.0, 30.0, 100.0, 200.0], (batch, pieces, kv_heads))
+    levels[:, 2:4] = -250.0
+    k[..., 0] = np.repeat(levels, 32, axis=1)
+    q, k, v = _bf16(q), _bf16(k), _bf16(v)
+    profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=False)
+    metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile)
+    out, lse = (t.cpu() for t in ct.attention_forward_with_lse(q.to(gpu), k.to(gpu), v.to(gpu), metadata, scale=scale))
+    assert torch.isfinite(out.float()).all() and torch.isfinite(lse).all()
+    assert (out[torch.from_numpy(ids == 0)] == 0).all() and (lse[torch.from_numpy(ids == 0)] == 0).all()
+    position = torch.arange(seq)
+    for row, head in ((0, 0), (batch - 1, q_heads - 1)):
+        kv = head // (q_heads // kv_heads)
+        segment = torch.from_numpy(ids[row])
+        allowed = (segment[:, None] == segment[None]) & (position[None] <= position[:, None]) & (segment[:, None] != 0)
+        scores = scale * q[row, :, head].double() @ k[row, :, kv].double().T
+        scores = scores.masked_fill(~allowed, -torch.inf)[segment != 0]
+        want = torch.softmax(scores, dim=1) @ v[row, :, kv].double()
+        assert float((out[row, segment != 0, head].double() - want).abs().max()) <= O_ATOL
+        assert float((lse[row, segment != 0, head].double() - torch.logsumexp(scores, dim=1)).abs().max()) <= LSE_ATOL
