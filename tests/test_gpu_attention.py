@@ -1263,3 +1263,10 @@ def test_scores_that_rise_and_fall_by_hundreds(ct, gpu, shape):
         want = torch.softmax(scores, dim=1) @ v[row, :, kv].double()
         assert float((out[row, segment != 0, head].double() - want).abs().max()) <= O_ATOL
         assert float((lse[row, segment != 0, head].double() - torch.logsumexp(scores, dim=1)).abs().max()) <= LSE_ATOL
+
+
+@pytest.mark.parametrize("shape,max_len", [((2, 2304, 15, 15), 1500), ((1, 2048, 66, 33), 700), ((8, 384, 44, 22), 384)], ids=str)
+def test_chunk_length_of_lists_beyond_the_slots(ct, gpu, bwd_variant, shape, max_len):
+    """The same with 528 to 540 (key tile, KV head) pairs, whose chunks are longer than a slot's share where that is short."""
+
+    test_chunk_length_by_the_lists_end(ct, gpu, bwd_variant, shape, max_len)
