@@ -8,6 +8,7 @@
 #include "ct_attn_dkv_wide.hip.h"
 #include "ct_attn_fwd_shares.hip.h"
 #include "ct_attn_fwd_split.hip.h"
+#include "ct_attn_fwd_tile.hip.h"
 #include "ct_attn_kernels.hip.h"
 #include "ct_error.h"
 #include "ct_lanes.hip.h"
@@ -621,6 +622,15 @@ static int launch_fwd(hipStream_t stream, const AttnParams& p) {
   return scope1.done();
 }
 
+template <int HS>
+static int launch_fwd_tile(hipStream_t stream, const AttnParams& p) {
+  CT_ENSURE_LDS("ct_attn_fwd", (&attn_fwd_tile_kernel<HS>), FwdTileStage::kTotalBytes);
+  const int grid = (p.Hq / HS) * p.B * (p.S / 32 / (kTileWaves / HS));
+  LaunchScope scope("attn_fwd_tile_kernel", stream);
+  hipLaunchKernelGGL(attn_fwd_tile_kernel<HS>, dim3(grid), dim3(kTileWaves * 64), FwdTileStage::kTotalBytes, stream, p);
+  return scope.done();
+}
+
 template <int D, int NW>
 static int launch_fwd_shares(hipStream_t stream, const AttnParams& p) {
   const size_t smem = NW * ShareRegion<D>::kBytes;
@@ -678,21 +688,18 @@ static int launch_fwd_split(hipStream_t stream, const AttnParams& p) {
 //     to 4 % in 7, the second none. Shared keys lose with short documents (they are staged for every head: [1, 2304, 8/2], 576,
 //     8.2 -> 8.7, though 14.7 -> 12.0 and 37 -> 29 with longer ones), and so does a second round (832, 10.8 -> 12.5).
 //   head dimension 64: sharing by two wins up to between 6144 (62 against 77 us with a long document) and 8192 (52 against 47).
-//   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920); from there to 2304 the longest row's
-//     chain still counts in long rows (large launch / by two: [1, 4096, 16/16] with documents up to the row 58.5 / 42.0),
-//     but whole rows and short ones lose (44.0 / 48.9 at [2, 1536, 24/8], and [4, 768, 24/8] 26.4 by four-wavefront workgroups /
-//     33.3). Above, the large launch's interleaved loop is ahead where rows see 8 key tiles or more
-//     (229 against 242 us), and is behind where they see few (61 against 46 us), which is certain
-//     only for short rows: the line at 20 key tiles per row is where whole-row documents cost 4 %.
-//     The large launch walks 8 row blocks in step: with 4 heads per slice 64 rows, but with 2 heads 128 and with 1 head 256,
-//     most of which do not see most of what they wait for. There the four-wavefront workgroups are ahead in longer rows
-//     too, whatever the documents, where KV heads come in eights (each XCD then has its own heads' K and V in its L2), row
-//     blocks are enough for every place (3072) and not too many (9216): up to 26 key tiles per row with 2 heads, 46 with 1, 40
-//     with 8 heads in all. 112 shapes inside these lines (large / here): whole rows 1.07 times in the geometric mean and 0.995
-//     at least, documents up to the row 1.23 and 1.05, up to 100 positions 1.37 and 1.15. Past each line whole rows lose (us):
-//     [8, 2944, 8/8] 148 / 152, [4, 4096, 16/16] 260 / 271, [8, 2048, 32/16] 296 / 314; 12 KV heads, [16, 2560, 12/12] 360 /
-//     396; 2560 row blocks, [2, 2560, 16/16] 68 / 71; 22528, [8, 1408, 64/64] 392 / 417; image blocks in a call with ends,
-//     [8, 2304, 8/8] 88 / 103.
+//   head dimension 128: sharing by two wins below 2048 (42 against 55 us at 1920) where rows see many keys; short documents lose
+//     there (four heads that share keys, 1536 row blocks, documents of up to 128 13.9 / 10.2 by whole row blocks, [3, 4608, 4/4]
+//     images 58 / 93), and the host does not know them. A little over one round of tiles in long rows of image blocks (a call with
+//     ends says so) still waits for the longest rows' chains: by two / a tile each [1, 4224, 16/4] 57 / 70 us, [1, 17152, 4/1] 86 /
+//     109, [2, 5504, 6/2] 77 / 91, [4, 4992, 4/4] 111 / 99; 19 shapes 1.08 times. Shorter rows lose ([1, 3200, 24/8] 58 / 50), and
+//     so do more blocks ([3, 4864, 8/2] alike, [1, 30208, 4/4] 160 / 130) and whole rows without ends ([1, 9216, 8/2] 203 / 177).
+//     Rows of up to 20 key tiles: pieces of 64 keys on their own ([8, 768, 24/4], documents of 61 to 122, 29 us, by query tiles
+//     32; whole rows of 1280, [4, 1280, 32/8], 65 / 63). Longer ones: a query tile per workgroup of four wavefronts
+//     (attn_fwd_tile_kernel). Workgroups of eight that walk the metadata's bins are ahead only where the tiles of four heads that
+//     share keys fill the places exactly twice, so that nothing evens out what the pairs leave: 3841 to 4096 row blocks, us
+//     so / a tile each, [1, 8192, 16/4] whole rows 242 / 249, [1, 16384, 8/2] 466 / 484, [2, 4096, 16/4] 128.7 / 132.3, [6, 2688,
+//     8/1] images 92 / 95; [1, 6144, 32/8], 6144 blocks, whole rows 287 / 277.
 template <int D>
 static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
   const long blocks = (long)p.B * p.Hq * (p.S / 32);
@@ -706,15 +713,12 @@ static int dispatch_fwd(hipStream_t stream, const AttnParams& p) {
     if (blocks <= 512) return launch_fwd_shares<D, 4>(stream, p);
     if (p.Hq == p.Hkv && p.S >= 1024 && blocks > 536 && blocks <= (p.Hq % 4 == 0 ? 768 : 592))
       return launch_fwd_shares<D, 3>(stream, p);
-    if (blocks < 2048) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
-    const int hs = heads_per_group(p.Hq, p.Hkv);
-    const bool local = !p.end && p.Hkv % 8 == 0 && blocks >= 3072 && blocks <= 9216;
-    const int short_row = !local || hs == 4 ? 20 : hs == 2 ? 26 : p.Hq < 16 ? 40 : 46;
-    if (p.S <= short_row * kKeyTile) return launch_fwd_split<D, 4, 1, 2, 1>(stream, p);
-    switch (hs) {
-      case 4: return launch_fwd<D, 4>(stream, p);
-      case 2: return launch_fwd<D, 2>(stream, p);
-      default: return launch_fwd<D, 1>(stream, p);
+    if (blocks < 2048 || (p.end && blocks < 2560 && p.S >= 56 * kKeyTile)) return launch_fwd_split<D, 4, 2, 1, 1>(stream, p);
+    if (p.S <= 20 * kKeyTile) return launch_fwd_split<D, 4, 1, 2, 1>(stream, p);
+    switch (heads_per_group(p.Hq, p.Hkv)) {
+      case 4: return blocks > 3840 && blocks <= 4096 ? launch_fwd<D, 4>(stream, p) : launch_fwd_tile<4>(stream, p);
+      case 2: return launch_fwd_tile<2>(stream, p);
+      default: return launch_fwd_tile<1>(stream, p);
     }
   }
 }

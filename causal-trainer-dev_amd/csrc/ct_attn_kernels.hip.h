@@ -389,6 +389,38 @@ struct FwdCopies {
                  : "memory", "m0", CT_FWD_PRIVATE);                                                           \
     return mx;                                                                                                \
   }                                                                                                           \
+  template <int V_OFF>                                                                                        \
+  CT_DEVICE float fwd_max_4_##NAME(const TrFragOffsets<16, KSlots::kAccum>& to, unsigned long long vsrc, unsigned long long ksrc, \
+                                   const unsigned* off, unsigned v_dst, unsigned k_dst) {                     \
+    float mx, tmp;                                                                                            \
+    asm volatile(CT_FWD_MAX_4_##UPPER                                                                         \
+                 : [mx] "=&v"(mx), [tmp] "=&v"(tmp)                                                           \
+                 : CT_FWD_TR_PTRS(to), [c] "s"(kLog2e), [voff] "i"(V_OFF), [vsrc] "s"(vsrc), [ksrc] "s"(ksrc), \
+                   [off0] "v"(off[0]), [off1] "v"(off[1]), [off2] "v"(off[2]), [off3] "v"(off[3]),            \
+                   [d0] "s"(v_dst), [d1] "s"(v_dst + 4096), [d2] "s"(v_dst + 8192), [d3] "s"(v_dst + 12288),  \
+                   [d4] "s"(k_dst), [d5] "s"(k_dst + 4096), [d6] "s"(k_dst + 8192), [d7] "s"(k_dst + 12288)   \
+                 : "memory", "m0", CT_FWD_PRIVATE);                                                           \
+    return mx;                                                                                                \
+  }                                                                                                           \
+  /* the whole PV product and the copies | first exponentials, against a reference that stays as it is */    \
+  template <int V_OFF>                                                                                        \
+  CT_DEVICE void fwd_free_pv_##NAME(const TrFragOffsets<16, KSlots::kAccum>& to, unsigned long long vsrc, unsigned long long ksrc, \
+                                    const unsigned* off, unsigned v_dst, unsigned k_dst, float m, float& psum) { \
+    asm volatile(CT_FWD_FREE_PV_##UPPER                                                                       \
+                 : [psum] "+v"(psum)                                                                          \
+                 : CT_FWD_TR_PTRS(to), [m] "v"(m), [c] "s"(kLog2e), [voff] "i"(V_OFF), [vsrc] "s"(vsrc), [ksrc] "s"(ksrc), \
+                   [off0] "v"(off[0]), [off1] "v"(off[1]), [off2] "v"(off[2]), [off3] "v"(off[3]),            \
+                   [d0] "s"(v_dst), [d1] "s"(v_dst + 4096), [d2] "s"(v_dst + 8192), [d3] "s"(v_dst + 12288),  \
+                   [d4] "s"(k_dst), [d5] "s"(k_dst + 4096), [d6] "s"(k_dst + 8192), [d7] "s"(k_dst + 12288)   \
+                 : "memory", "m0", CT_FWD_PRIVATE);                                                           \
+  }                                                                                                           \
+  template <int K_OFF>                                                                                        \
+  CT_DEVICE void fwd_free_qk_##NAME(const RowFragOffsets<16>& ro, const bf16x8* qf, float m, float& psum) {  \
+    asm volatile(CT_FWD_FREE_QK_##UPPER                                                                       \
+                 : [psum] "+v"(psum)                                                                          \
+                 : CT_FWD_ROW_PTRS(ro, qf), [m] "v"(m), [c] "s"(kLog2e), [koff] "i"(K_OFF)                    \
+                 : "memory", CT_FWD_PRIVATE);                                                                 \
+  }                                                                                                           \
   /* second half of the PV product | first exponentials */                                                    \
   template <int V_OFF>                                                                                        \
   CT_DEVICE void fwd_exp_a_##NAME(const TrFragOffsets<16, KSlots::kAccum>& to, float m, float& psum) {       \
@@ -478,7 +510,8 @@ CT_DEVICE f32x16 fwd_acc_read() {
 // ---------------------------------------------------------------------------
 // Forward
 //
-// Head dimension 128, large launches (the others: ct_attn_fwd_split.hip.h). One workgroup of 8
+// Head dimension 128, four heads that share keys, launches whose query tiles would fill the chip exactly twice (dispatch_fwd
+// says why; other large launches: ct_attn_fwd_tile.hip.h, the rest: ct_attn_fwd_split.hip.h). One workgroup of 8
 // wavefronts per compute unit (wavefronts w and w + 4 share a SIMD), each with 32 query rows of one
 // head. Per key tile t a wavefront has three pieces of work: the
 // softmax arithmetic of tile t (vector ALU), O += V(t-1)^T P(t-1)^T and S(t+1)^T = K(t+1) Q^T

@@ -104,7 +104,11 @@ def qk_sequence(ahead, slots):
 #   exp_a: second half of the PV product (k-steps 2, 3)  | exponentials of scores 0..FWD_SPLIT-1
 #   exp_b: S(t+1)                                        | exponentials of the other scores
 # (an asm statement takes at most 30 operands, and the decision to move the running maximum sits
-# between the first two). Otherwise the same arithmetic and the same products as statements of
+# between the first two). Workgroups of four wavefronts have twice the copies in the first one (max_4), and in stretches that
+# need no masks a step of two statements, whose exponentials stay with the reference that there is:
+#   free_pv: the whole PV product (16 MFMAs, 8 copies)   | exponentials of scores 0..FWD_FREE_SPLIT-1
+#   free_qk: S(t+1)                                      | exponentials of the other scores
+# Otherwise the same arithmetic and the same products as statements of
 # their own (FWD_*_ONLY, FWD_QK, FWD_PV, FWD_PV_LATE), which give the same bits.
 # ---------------------------------------------------------------------------
 FWD_S = {"a": 112, "b": 144}
@@ -112,6 +116,7 @@ FWD_FIRST_PRIVATE = 112
 FWD_RING0 = 176          # four fragment slots of four registers
 FWD_LAST_PRIVATE = 191
 FWD_SPLIT = 10
+FWD_FREE_SPLIT = 16
 
 
 def other(cur):
@@ -282,6 +287,11 @@ def fwd_statements(cur):
     return {
         # the three interleaved statements
         "MAX": head_pv01 + weave(fwd_with_copies(pv01, 2), fwd_max_ops(cur)),
+        # with twice the copies, for workgroups of four wavefronts
+        "MAX_4": head_pv01 + weave(fwd_with_copies(pv01, 4), fwd_max_ops(cur)),
+        # the step in two statements, without the maximum: the exponentials against the reference as it is
+        "FREE_PV": head_pv + weave(fwd_with_copies(pv, 4), fwd_exp_ops(cur, 0, FWD_FREE_SPLIT)),
+        "FREE_QK": head_qk + weave(qk, fwd_exp_ops(cur, FWD_FREE_SPLIT, 32), lead=6) + TAIL,
         "EXP_A": head_pv23 + weave(pv23, fwd_exp_ops(cur, 0, FWD_SPLIT)),
         "EXP_B": head_qk + weave(qk, fwd_exp_ops(cur, FWD_SPLIT, 32), lead=6) + TAIL,
         # the same pieces on their own

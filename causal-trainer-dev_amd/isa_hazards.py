@@ -336,8 +336,8 @@ def scan_library() -> dict[str, list[str]]:
             for kernel in ("attn_dkv_wide_kernel", "attn_dkv_kernelILi128ELb0E", "attn_dkv_kernelILi128ELb1E",
                            "attn_dq_kernelILi128ELi1E", "attn_dq_kernelILi128ELi2E", "attn_dq_kernelILi128ELi4E"):
                 findings[path.name] += private_accumulators(text, kernel)
-            for heads in (1, 2, 4):
-                findings[path.name] += private_registers(text, f"attn_fwd_kernelILi128ELi{heads}E", 112, 191)
+            for kernel in ("attn_fwd_kernelILi128ELi4E", *(f"attn_fwd_tile_kernelILi{heads}E" for heads in (1, 2, 4))):
+                findings[path.name] += private_registers(text, kernel, 112, 191)
     return findings
 
 

@@ -27,7 +27,7 @@ import os
 from .rocprof_traffic import _short
 
 # resident wavefronts per SIMD of the kernels reported (launch bounds and register use fix them)
-WAVES_PER_SIMD = {"attn_fwd_kernel": 2, "attn_dq_kernel": 2, "attn_dkv_kernel": 2, "attn_dkv_wide_kernel": 1,
+WAVES_PER_SIMD = {"attn_fwd_kernel": 2, "attn_fwd_tile_kernel": 2, "attn_dq_kernel": 2, "attn_dkv_kernel": 2, "attn_dkv_wide_kernel": 1,
                   "attn_dq_blocks_kernel": 4, "cutce_stats_kernel": 1, "cutce_dlogits_kernel": 1,
                   "cutce_grads_kernel": 1, "cutce_dhidden_kernel": 1, "cutce_dhead_kernel": 1}
 

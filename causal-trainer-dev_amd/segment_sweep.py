@@ -21,7 +21,7 @@ import dataclasses
 import numpy as np
 import torch
 
-KERNELS = ("attn_fwd_kernel", "attn_dq_kernel", "attn_dkv_kernel", "attn_dkv_reduce_kernel")
+KERNELS = ("attn_fwd_tile_kernel", "attn_dq_kernel", "attn_dkv_kernel", "attn_dkv_reduce_kernel")
 
 
 def kernel_times(ct, config, steps):
@@ -80,7 +80,7 @@ def main() -> None:
     lines += ["", "least-squares fit time = fixed + slope * pairs over the runs above, and what it says about the shape's",
               "own packing (%d pairs): measured time, fixed share, the rate the slope corresponds to" % own_pairs]
     unit = base.head_dim * base.q_heads
-    executed = {"attn_fwd_kernel": 4, "attn_dq_kernel": 6, "attn_dkv_kernel": 8}
+    executed = {"attn_fwd_tile_kernel": 4, "attn_dq_kernel": 6, "attn_dkv_kernel": 8}
     for name in KERNELS[:3]:
         x = np.array([pairs for _, pairs, _ in rows], dtype=np.float64)
         y = np.array([times[name] for _, _, times in rows], dtype=np.float64)

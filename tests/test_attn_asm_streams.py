@@ -397,6 +397,33 @@ def test_forward_interleaved_statements(gen, cur):
         assert not any("m0" in line or line.startswith("global_") for line in statements[name]), name
 
 
+@pytest.mark.parametrize("cur", ["a", "b"])
+def test_forward_statements_of_four_wavefronts(gen, cur):
+    """A step with eight copies: with the maximum, and in two statements without it. The same products and the same vector
+    instructions as the pieces on their own; the copies V rows first, each with its m0 in front."""
+
+    statements = gen.fwd_statements(cur)
+    mfmas = {name: [line for line in lines if line.startswith("v_mfma")] for name, lines in statements.items()}
+    assert mfmas["MAX_4"] == mfmas["MAX"] and _vector_alu(statements["MAX_4"]) == _vector_alu(statements["MAX"])
+    assert mfmas["FREE_PV"] == mfmas["PV"] and mfmas["FREE_QK"] == mfmas["QK"]
+    split = _vector_alu(statements["FREE_PV"]) + _vector_alu(statements["FREE_QK"])
+    assert sorted(split) == sorted(_vector_alu(statements["EXP_ONLY"])) and len(split) / 32 <= 3.5
+    additions = lambda lines: [line for line in lines if line.startswith("v_add_f32")]
+    assert additions(split) == additions(_vector_alu(statements["EXP_ONLY"]))
+    for name in ("MAX_4", "FREE_PV"):
+        lines = statements[name]
+        copies = [i for i, line in enumerate(lines) if line.startswith("global_load_lds")]
+        settings = [i for i, line in enumerate(lines) if line.startswith("s_mov_b32 m0")]
+        assert [lines[i] for i in copies] == ["global_load_lds_dwordx4 %%[off%d], %%[%s]" % (g % 4, "vsrc" if g < 4 else "ksrc")
+                                              for g in range(8)]
+        assert [lines[i] for i in settings] == ["s_mov_b32 m0, %%[d%d]" % g for g in range(8)]
+        assert all(settings[g] + 1 < copies[g] and (g == 7 or copies[g] < settings[g + 1]) for g in range(8))
+    for line in statements["FREE_PV"]:
+        if line.startswith(("v_", "ds_read")):
+            other = gen.FWD_S[gen.other(cur)]
+            assert not _registers(_split(line)[1][0]) & set(range(other, other + 32)), line
+
+
 def test_forward_masks(gen):
     """The mask statements: one compare and one select per score, the key offset of a score register
     as the accumulator layout has it (block 32 kb, then 8 (r / 4) + r % 4, plus 4 for the lanes of

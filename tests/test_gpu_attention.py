@@ -1228,11 +1228,14 @@ def test_forms_of_dq_from_stored_blocks(ct, gpu, shape, with_ends):
         assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2   # bf16 results of bf16 dS
 
 
+@pytest.mark.parametrize("levels", [(-250.0, -150.0, -40.0, 0.0, 30.0, 100.0, 200.0), (-30.0, 0.0, 6.0, 12.0, 20.0)], ids=["far", "near"])
 @pytest.mark.parametrize("shape", [(1, 1024, 28, 4, 64), (8, 1024, 28, 4, 64), (1, 1024, 20, 4, 128), (3, 1024, 24, 4, 128),
-                                   (1, 1024, 4, 4, 64), (1, 1024, 4, 4, 128), (2, 2048, 32, 8, 128)], ids=str)
-def test_scores_that_rise_and_fall_by_hundreds(ct, gpu, shape):
-    """The forward's reference of the softmax follows scores that jump from one piece of 32 keys to the next, in rows whose
-    first visited blocks hold ids around theirs but none of them, and in rows of padding, in every form of the forward."""
+                                   (1, 1024, 4, 4, 64), (1, 1024, 4, 4, 128), (2, 2048, 32, 8, 128), (2, 2304, 16, 4, 128),
+                                   (2, 2304, 16, 8, 128), (2, 2304, 16, 16, 128)], ids=str)
+def test_scores_that_rise_and_fall(ct, gpu, shape, levels):
+    """The forward's reference of the softmax follows scores that jump from one piece of 32 keys to the next (by hundreds, or by
+    so much that sums reach 2^30 to 2^60 against it), in rows whose first visited blocks hold ids around theirs but none of
+    them, and in rows of padding, in every form of the forward; a row of no numbers stays alone with them."""
 
     batch, seq, q_heads, kv_heads, dim = shape
     rng = np.random.default_rng(5)
@@ -1244,25 +1247,42 @@ def test_scores_that_rise_and_fall_by_hundreds(ct, gpu, shape):
     k = 0.3 * rng.standard_normal((batch, seq, kv_heads, dim))
     v = rng.standard_normal((batch, seq, kv_heads, dim))
     q[..., 0] = 16.0                                     # a score is about twice the key's first element
-    levels = rng.choice([-250.0, -150.0, -40.0, 0.0, 30.0, 100.0, 200.0], (batch, pieces, kv_heads))
-    levels[:, 2:4] = -250.0
-    k[..., 0] = np.repeat(levels, 32, axis=1)
+    steps = rng.choice(levels, (batch, pieces, kv_heads))
+    steps[:, 2:4] = min(levels)
+    k[..., 0] = np.repeat(steps, 32, axis=1)
+    q[0, 800, 0] = np.nan
     q, k, v = _bf16(q), _bf16(k), _bf16(v)
     profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=False)
     metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile)
     out, lse = (t.cpu() for t in ct.attention_forward_with_lse(q.to(gpu), k.to(gpu), v.to(gpu), metadata, scale=scale))
+    assert torch.isnan(out[0, 800, 0]).all()
+    out[0, 800, 0] = 0
     assert torch.isfinite(out.float()).all() and torch.isfinite(lse).all()
     assert (out[torch.from_numpy(ids == 0)] == 0).all() and (lse[torch.from_numpy(ids == 0)] == 0).all()
     position = torch.arange(seq)
     for row, head in ((0, 0), (batch - 1, q_heads - 1)):
         kv = head // (q_heads // kv_heads)
         segment = torch.from_numpy(ids[row])
-        allowed = (segment[:, None] == segment[None]) & (position[None] <= position[:, None]) & (segment[:, None] != 0)
+        rows = (segment != 0) & ~torch.isnan(q[row, :, head].float()).any(dim=1)
+        allowed = (segment[:, None] == segment[None]) & (position[None] <= position[:, None])
         scores = scale * q[row, :, head].double() @ k[row, :, kv].double().T
-        scores = scores.masked_fill(~allowed, -torch.inf)[segment != 0]
+        scores = scores.masked_fill(~allowed, -torch.inf)[rows]
         want = torch.softmax(scores, dim=1) @ v[row, :, kv].double()
-        assert float((out[row, segment != 0, head].double() - want).abs().max()) <= O_ATOL
-        assert float((lse[row, segment != 0, head].double() - torch.logsumexp(scores, dim=1)).abs().max()) <= LSE_ATOL
+        assert float((out[row, rows, head].double() - want).abs().max()) <= O_ATOL
+        assert float((lse[row, rows, head].double() - torch.logsumexp(scores, dim=1)).abs().max()) <= LSE_ATOL
+
+
+@pytest.mark.parametrize("shape", [
+    # D = 128, rows beyond 20 key tiles: the first launch of a query tile per workgroup with four, two and one heads, two batch
+    # rows of eight groups, the sides of the two filled rounds, and launches whose rows go out sixteen tiles at a time, with a rest
+    (1, 2048, 32, 8, 128), (1, 2048, 32, 16, 128), (1, 2048, 32, 32, 128), (2, 2304, 32, 8, 128), (1, 3840, 32, 4, 128),
+    (1, 4096, 32, 8, 128), (1, 4224, 16, 4, 128), (1, 4224, 32, 8, 128), (3, 4224, 32, 8, 128), (6, 2176, 32, 16, 128), (6, 2176, 32, 32, 128)],
+    ids=lambda c: "B%d_S%d_Hq%d_Hkv%d_D%d" % c)
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_a_query_tile_per_workgroup(ct, gpu, shape, with_ends):
+    """O and LSE at the sizes where the large launches at head dimension 128 change."""
+
+    test_forms_of_the_forward(ct, gpu, shape, with_ends)
 
 
 @pytest.mark.parametrize("shape,max_len", [((2, 2304, 15, 15), 1500), ((1, 2048, 66, 33), 700), ((8, 384, 44, 22), 384)], ids=str)
