@@ -133,6 +133,9 @@ SYMBOLS = {
     "ct_rms_norm_fwd": (c_int32, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int64, c_int32,
                                   c_void_p, c_void_p]),
     "ct_rms_norm_bwd_workspace_bytes": (c_size_t, [c_int32]),
+    "ct_rms_norm_keeps_rstd": (c_int32, [c_int64, c_int32]),
+    "ct_rms_norm_bwd_saved": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                        c_int32, c_void_p, c_void_p]),
     "ct_rms_norm_bwd": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int64,
                                   c_int32, c_void_p, c_void_p, c_void_p, c_size_t]),
     "ct_rms_norm_bwd_rounded": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int64,

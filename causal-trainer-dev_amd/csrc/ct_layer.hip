@@ -402,6 +402,83 @@ __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const uint16_t* x, co
     }
 }
 
+// The same with the forward's r of every row, for few of them: dx and dscale then have nothing to wait for in each other and
+// are one launch. Workgroups before column_groups add 32 columns of dscale over all rows (8 columns of every 64th row a
+// thread, the 16 rows of a wavefront, the wavefronts, in that order), the others form dx of 4 / WAVES rows.
+// Bound by latency: us of the two kernels above and below without the wait between them / of this one, [260, 1024] 6.2 / 4.8,
+// [4, 512] 4.2 / 3.6, [1024, 512] 6.1 / 6.8, [512, 4096] 10.8 / 6.6, [1024, 8192] 21.7 / 18.4; the launch saved is 2 us of a
+// host that does not keep ahead (norm and rotary on [2, 130, 1024], both directions, 90.6 / 88.8; on [4, 128, 4096] 90.8 / 88.4). More rows lose: [2048, 512]
+// 7.6 / 10.0, [2048, 2048] 13.3 / 17.8, [4096, 1024] 12.0 / 29.4. (Every column group forming r by itself: [260, 1024] 14.9.)
+template <int WAVES, int NCH>
+__global__ __launch_bounds__(256) void rms_norm_bwd_saved_kernel(const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
+                                                                 const float* rstd, int rows, int d, int column_groups, uint16_t* dx,
+                                                                 bf16* dscale) {
+  __shared__ float exch[4][32];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if ((int)blockIdx.x < column_groups) {
+    const int col = (int)blockIdx.x * 32 + (threadIdx.x & 3) * 8;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    if (col < d) {
+#pragma unroll 4
+      for (int row = threadIdx.x >> 2; row < rows; row += 64) {
+        const bf16x8 xv = as_bf16x8(*reinterpret_cast<const u32x4*>(x + (size_t)row * d + col));
+        const bf16x8 gv = as_bf16x8(*reinterpret_cast<const u32x4*>(dy + (size_t)row * d + col));
+        const float r = rstd[row];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += (float)gv[e] * (float)(bf16)((float)xv[e] * r);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int off = 32; off >= 4; off >>= 1) acc[e] += __shfl_xor(acc[e], off, 64);
+      if (lane < 4) exch[wave][lane * 8 + e] = acc[e];
+    }
+    __syncthreads();
+    const int out = (int)blockIdx.x * 32 + threadIdx.x;
+    if (threadIdx.x < 32 && out < d)
+      dscale[out] = (bf16)((exch[0][threadIdx.x] + exch[1][threadIdx.x]) + (exch[2][threadIdx.x] + exch[3][threadIdx.x]));
+    return;
+  }
+  const int part = wave % WAVES, chunks = d / 8, row = ((int)blockIdx.x - column_groups) * (4 / WAVES) + wave / WAVES;
+  u32x4 w[NCH], xv[NCH], gv[NCH];
+  float dot = 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = lane + 64 * (part + WAVES * i);
+    const bool in = row < rows && c < chunks;
+    w[i] = in ? *reinterpret_cast<const u32x4*>(scale + c * 8) : u32x4{0, 0, 0, 0};
+    xv[i] = in ? *reinterpret_cast<const u32x4*>(x + (size_t)row * d + c * 8) : u32x4{0, 0, 0, 0};
+    gv[i] = in ? *reinterpret_cast<const u32x4*>(dy + (size_t)row * d + c * 8) : u32x4{0, 0, 0, 0};
+  }
+  const float r = row < rows ? rstd[row] : 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot += (float)as_bf16x8(gv[i])[e] * (float)as_bf16x8(w[i])[e] * (float)as_bf16x8(xv[i])[e];
+  dot = wave_sum(dot);
+  if constexpr (WAVES > 1) {
+    if (lane == 0) exch[wave][0] = dot;
+    __syncthreads();
+    dot = 0.f;
+#pragma unroll
+    for (int k = 0; k < WAVES; ++k) dot += exch[wave / WAVES * WAVES + k][0];
+  }
+  const float mean = dot * r / (float)d;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = lane + 64 * (part + WAVES * i);
+    if (row >= rows || c >= chunks) continue;
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      o[e] = (bf16)(r * ((float)as_bf16x8(gv[i])[e] * (float)as_bf16x8(w[i])[e] - (float)as_bf16x8(xv[i])[e] * r * mean));
+    *reinterpret_cast<u32x4*>(dx + (size_t)row * d + c * 8) = as_u32x4(o);
+  }
+}
+
 // Hidden sizes past 8192: the row is walked three times (sum of squares, the
 // dot product, dx; the repeats are served from cache) and the wavefront's dscale sums live in its
 // row of `partial` instead of registers (a lane only ever touches its own columns of it).
@@ -486,6 +563,8 @@ __global__ __launch_bounds__(1024) void rms_norm_dscale_kernel(const float* part
 // leave room for (the walking kernel writes one per wavefront).
 constexpr int kNormBwdBlocks = 768;
 constexpr int kNormBwdAnyBlocks = 512;
+// The line: the threads of a column group walk rows / 64 rows each, and x and dy are read twice (figures at the kernel).
+constexpr long kNormSavedRows = 1024;
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -602,6 +681,9 @@ extern "C" size_t ct_rms_norm_bwd_workspace_bytes(int32_t hidden) {
   return (size_t)(hidden <= 8192 ? kNormBwdBlocks : kNormBwdAnyBlocks * 4) * hidden * sizeof(float);
 }
 
+// Wavefronts that share a row of up to 8192: the fewest that keep a lane at 2 chunks (3 or 4 past 4096).
+static int norm_bwd_waves(int hidden) { return hidden <= 1024 ? 1 : hidden <= 2048 ? 2 : 4; }
+
 static int32_t rms_norm_bwd_on(void* stream_, const uint16_t* x, const uint16_t* scale, const uint16_t* dy, float eps,
                                int64_t rows, int32_t hidden, uint16_t* dx, float* dscale, uint16_t* dscale_rounded,
                                void* workspace, size_t workspace_bytes) {
@@ -622,8 +704,7 @@ static int32_t rms_norm_bwd_on(void* stream_, const uint16_t* x, const uint16_t*
                        hidden, dx, partial);
     count = kNormBwdAnyBlocks * 4;
   } else {
-    // wavefronts that share a row: the fewest that keep a lane at 2 chunks (3 or 4 past 4096)
-    const int waves = hidden <= 1024 ? 1 : hidden <= 2048 ? 2 : 4, at_a_time = 4 / waves;
+    const int waves = norm_bwd_waves(hidden), at_a_time = 4 / waves;
     const int64_t groups = (rows + at_a_time - 1) / at_a_time;
     count = groups < kNormBwdBlocks ? (int)groups : kNormBwdBlocks;
     const size_t smem = (size_t)(at_a_time - 1) * hidden * sizeof(float);
@@ -645,6 +726,35 @@ static int32_t rms_norm_bwd_on(void* stream_, const uint16_t* x, const uint16_t*
   hipLaunchKernelGGL(rms_norm_dscale_kernel, dim3((hidden + 31) / 32), dim3(1024), 0, stream, partial, count, hidden, dscale,
                      reinterpret_cast<bf16*>(dscale_rounded));
   return scope2.done();
+}
+
+extern "C" int32_t ct_rms_norm_keeps_rstd(int64_t rows, int32_t hidden) {
+  return rows > 0 && rows <= kNormSavedRows && hidden > 0 && hidden <= 8192 && hidden % 8 == 0;
+}
+
+extern "C" int32_t ct_rms_norm_bwd_saved(void* stream_, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
+                                         const float* rstd, int64_t rows, int32_t hidden, uint16_t* dx, uint16_t* dscale) {
+  CT_REQUIRE(x && scale && dy && rstd && dx && dscale, "ct_rms_norm_bwd_saved: null pointer");
+  CT_REQUIRE(ct_rms_norm_keeps_rstd(rows, hidden), "ct_rms_norm_bwd_saved: not a size that keeps rstd, got [%lld, %d]",
+             (long long)rows, hidden);
+  CT_REQUIRE(aligned16(x) && aligned16(scale) && aligned16(dy) && aligned16(dx), "ct_rms_norm_bwd_saved: pointers must be 16-byte aligned");
+  hipStream_t stream = (hipStream_t)stream_;
+  LaunchScope scope("rms_norm_bwd_saved_kernel", stream);
+  const int waves = norm_bwd_waves(hidden), column_groups = (hidden + 31) / 32;
+  const int row_groups = ((int)rows + 4 / waves - 1) / (4 / waves);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(column_groups + row_groups), dim3(256), 0, stream, x, scale, dy, rstd, (int)rows, hidden,
+                       column_groups, dx, reinterpret_cast<bf16*>(dscale));
+  };
+  switch (int chunks = (hidden + 512 * waves - 1) / (512 * waves); 8 * waves + chunks) {
+    case 9: launch(rms_norm_bwd_saved_kernel<1, 1>); break;
+    case 10: launch(rms_norm_bwd_saved_kernel<1, 2>); break;
+    case 18: launch(rms_norm_bwd_saved_kernel<2, 2>); break;
+    case 34: launch(rms_norm_bwd_saved_kernel<4, 2>); break;
+    case 35: launch(rms_norm_bwd_saved_kernel<4, 3>); break;
+    default: launch(rms_norm_bwd_saved_kernel<4, 4>); break;
+  }
+  return scope.done();
 }
 
 extern "C" int32_t ct_rms_norm_bwd(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy, float eps,

@@ -359,6 +359,7 @@ MaybeTensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
 // ---------------------------------------------------------------------------------------------
 struct RmsNormNode : OperatorNode {
   SavedVariable x, scale;
+  Tensor rstd;  // of few rows
   double eps = 0;
   variable_list differentiate(variable_list&& grads) override {
     const Tensor X = x.unpack(), W = scale.unpack();
@@ -366,6 +367,11 @@ struct RmsNormNode : OperatorNode {
     const int64_t hidden = X.size(-1), rows = X.numel() / hidden;
     const Tensor dy = gradient(grads[0], X.sizes(), at::kBFloat16, X);
     Tensor dx = fresh(X), dscale = fresh(W);
+    if (rstd.defined()) {
+      check(ct_rms_norm_bwd_saved(current_stream(), bits(X), bits(W), bits(dy), ptr<float>(rstd), rows, (int32_t)hidden, bits(dx),
+                                  bits(dscale)));
+      return {dx, dscale};
+    }
     const size_t bytes = ct_rms_norm_bwd_workspace_bytes((int32_t)hidden);
     Tensor workspace = scratch(bytes, X);
     check(ct_rms_norm_bwd_rounded(current_stream(), bits(X), bits(W), bits(dy), (float)eps, rows, (int32_t)hidden, bits(dx),
@@ -375,6 +381,7 @@ struct RmsNormNode : OperatorNode {
   void release_variables() override {
     x.reset_data();
     scale.reset_data();
+    rstd.reset();
   }
   std::string name() const override { return "RmsNormBackward"; }
 };
@@ -384,14 +391,17 @@ MaybeTensor rms_norm(const Tensor& x, const Tensor& scale, double eps) {
       scale.size(0) != x.size(-1) || x.numel() == 0)
     return std::nullopt;
   const c10::DeviceGuard guard(x.device());
-  const int64_t hidden = x.size(-1);
-  Tensor y = fresh(x);
-  check(ct_rms_norm_fwd(current_stream(), bits(x), bits(scale), (float)eps, x.numel() / hidden, (int32_t)hidden, bits(y),
-                        nullptr));
-  if (needs_graph({x, scale})) {
+  const int64_t hidden = x.size(-1), rows = x.numel() / hidden;
+  const bool graph = needs_graph({x, scale});
+  Tensor y = fresh(x), rstd;
+  if (graph && ct_rms_norm_keeps_rstd(rows, (int32_t)hidden)) rstd = floats({rows}, x);
+  check(ct_rms_norm_fwd(current_stream(), bits(x), bits(scale), (float)eps, rows, (int32_t)hidden, bits(y),
+                        rstd.defined() ? ptr<float>(rstd) : nullptr));
+  if (graph) {
     auto node = graph_node<RmsNormNode>({x, scale});
     node->x = SavedVariable(x, false);
     node->scale = SavedVariable(scale, false);
+    node->rstd = rstd;
     node->eps = eps;
     torch::autograd::set_history(y, node);
   }

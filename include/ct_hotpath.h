@@ -358,6 +358,9 @@ int32_t ct_rms_norm_fwd(void* stream, const uint16_t* x, const uint16_t* scale, 
 
 size_t ct_rms_norm_bwd_workspace_bytes(int32_t hidden);
 
+/* 1 where a forward whose gradients will be wanted should keep rstd: ct_rms_norm_bwd_saved takes these sizes. */
+int32_t ct_rms_norm_keeps_rstd(int64_t rows, int32_t hidden);
+
 /*
  * Gradients of ct_rms_norm_fwd: dx bf16 [rows, hidden], dscale f32 [hidden]
  * (summed over rows in a fixed order). hidden % 8 == 0 (up to 8192 the row is
@@ -372,6 +375,10 @@ int32_t ct_rms_norm_bwd(void* stream, const uint16_t* x, const uint16_t* scale, 
 int32_t ct_rms_norm_bwd_rounded(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
                                 float eps, int64_t rows, int32_t hidden, uint16_t* dx, uint16_t* dscale,
                                 void* workspace, size_t workspace_bytes);
+
+/* The same in one launch, for few rows, from the rstd that ct_rms_norm_fwd wrote. */
+int32_t ct_rms_norm_bwd_saved(void* stream, const uint16_t* x, const uint16_t* scale, const uint16_t* dy,
+                              const float* rstd, int64_t rows, int32_t hidden, uint16_t* dx, uint16_t* dscale);
 
 /* ------------------------------------------------------------------------
  * Sparse cross-entropy on materialised logits (the non-fused loss backend)

@@ -230,6 +230,28 @@ def test_rms_norm_rows_shared_by_wavefronts(ct, gpu, rows, hidden):
     test_rms_norm_gradients_match_oracle(ct, gpu, rows, hidden)
 
 
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (63, 40), (64, 1024), (65, 1032), (130, 2056), (9, 8192), (1024, 512), (1025, 512)])
+def test_rms_norm_gradients_of_few_rows(ct, gpu, rows, hidden):
+    """Up to 1024 rows the forward keeps what one launch forms both gradients from: the sides of that line, and column and row
+    counts that leave places of its workgroups empty. A second pass over a kept graph gives the same bits, and so does one whose
+    saved tensors went through the host."""
+
+    test_rms_norm_gradients_match_oracle(ct, gpu, rows, hidden)
+    generator = torch.Generator().manual_seed(rows + hidden)
+    x, dy = (torch.randn((rows, hidden), generator=generator).to(torch.bfloat16).to(gpu) for _ in range(2))
+    scale = torch.randn(hidden, generator=generator).to(torch.bfloat16).to(gpu)
+    x.requires_grad_(True)
+    scale.requires_grad_(True)
+    y = ct.rms_norm(x, scale, 1e-5)
+    first = torch.autograd.grad(y, (x, scale), dy, retain_graph=True)
+    again = torch.autograd.grad(y, (x, scale), dy)
+    with torch.autograd.graph.save_on_cpu():
+        hooked = ct.rms_norm(x, scale, 1e-5)
+    through_host = torch.autograd.grad(hooked, (x, scale), dy)
+    for a, b, c in zip(first, again, through_host):
+        assert torch.equal(a, b) and torch.equal(a, c)
+
+
 @pytest.mark.parametrize("style", ["gpt-j", "gpt-neox"])
 def test_rotary_of_two_tokens_per_workgroup(ct, gpu, style):
     """Many tokens, an odd number of them: the last workgroup has one."""
