@@ -831,6 +831,16 @@ static int launch_dkv(hipStream_t stream, const AttnParams& p, bool wide) {
   }
   LaunchScope scope3("attn_dkv_kernel", stream);
   if constexpr (D == 64) {
+    if (p.dq_rides) {
+      const int hs = heads_per_group(p.Hq, p.Hkv);
+      const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), std::max(smem, (size_t)2 * KvStage<D>::kBytes), stream, p);
+      };
+      if (hs == 4) launch(attn_dkv_then_dq_kernel<4>);
+      else if (hs == 2) launch(attn_dkv_then_dq_kernel<2>);
+      else launch(attn_dkv_then_dq_kernel<1>);
+      return scope3.done();
+    }
     if (p.ds_most_blocks) {
       CT_ENSURE_LDS("ct_attn_bwd", &attn_dkv_choice_kernel<D>, smem);
       hipLaunchKernelGGL(attn_dkv_choice_kernel<D>, dim3(grid), dim3(256), smem, stream, p);
@@ -895,22 +905,26 @@ static int dispatch_bwd_recompute(hipStream_t stream, const AttnParams& p, bool 
 }
 
 // The most dS blocks per query head with which dQ comes from stored blocks, 0 where the form is settled (see kDqRecomputes).
-// Up to 8192 row blocks stored ones are ahead with all but the longest documents and the sums ride with their dQ already, so that
-// the recomputing kernel's launch would be lost. Beyond, recomputing is ahead from about 42000 blocks (of all heads) and 2.3 per
-// row block on, sooner per row block the larger the launch. Backward in us, stored / this / recomputing (head dimension 64):
+// Recomputing is ahead from about 42000 blocks (of all heads) and 2.3 per row block on, sooner per row block the larger the launch.
+// At 8192 row blocks stored ones are what a call gets (their bits are part of what callers hold this size to), below the recomputing
+// tiles ride with dK/dV (dq_rides); under 3072 row blocks those end unevenly: backward kernels, us, stored / so, [2, 2816, 16/16 of
+// 64], documents of 1408 to 2816, 110 / 124, [2, 3200, 12/4], images, 107 / 116, though [2, 4096, 10/2], whole rows, 227 / 190.
+// 36 drawn calls from 3072 on 0.985 to 1.43, 1.048 in the geometric mean.
+// Backward beyond 8192, in us, stored / this / recomputing (head dimension 64):
 //   [3, 1536, 64/16]  9216 row blocks, documents of 16 to 64 93 / 90 / 103, of 512 to 768 165 / 152 / 149, whole rows 323 / 260 / 257
 //   [4, 4096, 64/16] 32768, 16 to 64 261 / 263 / 269, 1365 to 2048 875 / 690 / 702, whole rows 2475 / 1826 / 1826
 //   [12, 4096, 8/8] 12288, whole rows 1028 / 732 / 736, image blocks 596 / 445 / 473
 // Over 70 shapes of 8200 to 61000 row blocks: short documents 0.93 to 1.02 of the stored form's time, long ones 0.71 to 0.9.
+constexpr long kStoredRowBlocks = 8192;
 static int most_stored_blocks(const AttnParams& p, int head_dim) {
   const long rows = (long)p.B * p.Hq * (p.S / 32);
-  if (head_dim != 64 || rows <= 8192) return 0;
+  if (head_dim != 64 || rows < 3072 || rows == kStoredRowBlocks) return 0;
   return (int)((42000 + 2.3 * rows) / p.Hq);
 }
 
 // Stored-dS form: row statistics and the work list; then per pass of KV heads the dK/dV kernel, which
 // leaves its dS blocks in the region, and dQ as a product over those blocks; the sum of split chunks. With p.ds_most_blocks the
-// recomputing dQ stands between the first two, and forms the statistics, where the header asks for it.
+// recomputing dQ stands between the first two, and forms the statistics, where the header asks for it, or rides with the second.
 template <int D>
 static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pass, bool wide, bool list_kept) {
   const long tiles = (long)p.B * p.Hq * (p.S / (D == 128 ? 64 : 128));
@@ -928,7 +942,7 @@ static int dispatch_bwd_blocks(hipStream_t stream, AttnParams p, int kvh_per_pas
   }
   if (rc) return rc;
   if constexpr (D == 64) {
-    if (p.ds_most_blocks) rc = dispatch_dq<D>(stream, p);
+    if (p.ds_most_blocks && !p.dq_rides) rc = dispatch_dq<D>(stream, p);
     if (rc) return rc;
   }
   for (int base = 0; base < p.Hkv; base += kvh_per_pass) {
@@ -1168,6 +1182,9 @@ extern "C" int32_t ct_attn_bwd(void* stream, const ct_attn_bwd_args* a) {
     p.ds = ws + plan.ds;
     p.ds_row_blocks = plan.row_blocks;
     if (path_choice == 0) p.ds_most_blocks = most_stored_blocks(p, a->head_dim);
+    p.dq_rides = p.ds_most_blocks && (long)p.B * p.Hq * (p.S / 32) < kStoredRowBlocks;
+    // (every group of heads needs a workgroup of that launch)
+    if (p.dq_rides && p.Hq / heads_per_group(p.Hq, p.Hkv) > p.dkv_max_entries * p.Hkv) p.ds_most_blocks = p.dq_rides = 0;
     return a->head_dim == 128 ? dispatch_bwd_blocks<128>(s, p, plan.kvh_per_pass, false, list_kept)
                               : dispatch_bwd_blocks<64>(s, p, plan.kvh_per_pass, false, list_kept);
   }

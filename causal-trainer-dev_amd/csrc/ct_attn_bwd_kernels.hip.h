@@ -31,7 +31,7 @@ CT_DEVICE int ds_blocks_per_head(const AttnParams& p) {
   }
   return lane_value(wave_scan(blocks), 63);
 }
-CT_DEVICE bool dq_recomputes(const AttnParams& p) { return uniform(p.dkv_header[kDqRecomputes]) != 0; }
+CT_DEVICE bool dq_recomputes(const AttnParams& p) { return uniform(meta_const(p.dkv_header)[kDqRecomputes]) != 0; }
 CT_DEVICE void leave_dkv_choice(const AttnParams& p) {
   if (!p.wide_least_blocks || threadIdx.x >= 64) return;
   const int blocks = ds_blocks_per_head(p);
@@ -113,8 +113,9 @@ CT_DEVICE unsigned dq_pairs_up_to(int last_rel) {
   return count <= 0 ? 0u : ~0u >> (32 - count);
 }
 
-// One query tile (4 / HS row blocks x HS heads of one KV head), start to finish.
-template <int D, int HS, int PER_UNIT>
+// One query tile (4 / HS row blocks x HS heads of one KV head), start to finish. STATS: with the rows' statistics, which are
+// there already otherwise.
+template <int D, int HS, int PER_UNIT, bool STATS>
 CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int qt, const lds_addr lds_base) {
   constexpr int kStage = KvStage<D>::kBytes;
   // (the fragment pointers are rebuilt per item from an opaque base: kept across the item loop
@@ -136,6 +137,7 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
   const size_t kv_row_stride = (size_t)p.Hkv * D;
   const size_t stat_t = ((size_t)ctx.work.b * p.Hq + ctx.work.h) * p.S + ctx.pos;  // head-major
   const float lse2 = p.lse[ctx.stat_off] * kLog2e;
+  float minus_delta_q = STATS ? 0.f : p.delta[stat_t];
 
   // The first key tile's copies go first (stage 0), the rows of Q, dO and O behind them; their
   // way into fragments leads through this wavefront's patch in stage 1, which nothing uses yet.
@@ -155,10 +157,10 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
     RowBlockLoader<D> q_rows, do_rows, o_rows;
     q_rows.request(p.q + block_off, q_row_stride);
     do_rows.request(p.dout + block_off, q_row_stride);
-    o_rows.request(p.out + block_off, q_row_stride);
+    if constexpr (STATS) o_rows.request(p.out + block_off, q_row_stride);
     q_rows.to_fragments(patch, qf);
     do_rows.to_fragments(patch, dof);
-    o_rows.to_fragments(patch, of);
+    if constexpr (STATS) o_rows.to_fragments(patch, of);
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) qf[ks] = scale_bf16x8(qf[ks], p.scale);
   }
@@ -175,27 +177,30 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
   // delta = sum_d out[row, d] * dout[row, d], after the wait above so that the first key tile's
   // copies are not held back behind these loads; the dK/dV kernel, launched after this one, reads
   // delta and lse * log2(e) head-major
-  float delta_part = 0.f;
+  if constexpr (STATS) {
+    float delta_part = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    u32x4 o_bits = of[ks];
-    asm volatile("" : "+v"(o_bits));
-    const u32x4 do_bits = __builtin_bit_cast(u32x4, dof[ks]);
+    for (int ks = 0; ks < D / 16; ++ks) {
+      u32x4 o_bits = of[ks];
+      asm volatile("" : "+v"(o_bits));
+      const u32x4 do_bits = __builtin_bit_cast(u32x4, dof[ks]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      delta_part = fmaf(__uint_as_float(o_bits[e] << 16), __uint_as_float(do_bits[e] << 16), delta_part);
-      delta_part = fmaf(__uint_as_float(o_bits[e] & 0xffff0000u), __uint_as_float(do_bits[e] & 0xffff0000u),
-                        delta_part);
+      for (int e = 0; e < 4; ++e) {
+        delta_part = fmaf(__uint_as_float(o_bits[e] << 16), __uint_as_float(do_bits[e] << 16), delta_part);
+        delta_part = fmaf(__uint_as_float(o_bits[e] & 0xffff0000u), __uint_as_float(do_bits[e] & 0xffff0000u),
+                          delta_part);
+      }
     }
+    minus_delta_q = -pair_sum(delta_part);
   }
-  const float delta_q = pair_sum(delta_part);
+  const float delta_q = -minus_delta_q;
   f32x16 minus_delta;
   if constexpr (D == 64) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) minus_delta[r] = -delta_q;
     asm volatile("" : "+v"(minus_delta));
   }
-  if (ctx.active && half == 0) {
+  if (STATS && ctx.active && half == 0) {
     // for the dK/dV kernel: the values it adds to its S and dP blocks, P = exp2((S - lse / scale) *
     // scale * log2(e)) and dS = P (dP - delta)
     p.delta[stat_t] = -delta_q;
@@ -310,34 +315,38 @@ CT_DEVICE void attn_dq_item(const AttnParams& p, int b, int kvh, int slice, int 
 // query tile). dQ, us, two / three: [1, 25472, 64/8 heads of 64], images, 1289 / 1186; [6, 2816, 64/16], images, 692 / 642; [4, 4096, 64/8]
 // 374 / 342; [4, 4992, 48/8], documents of 99 to 152, 160 / 151. Below 12288 row blocks short documents lose more than long ones
 // gain: [4, 5376, 16/16], 10752, 45 to 111, 74 / 81, [1, 17280, 12/4], 6480, 121 to 236, 49 / 55, [1, 16384, 16/2], whole rows, 813 / 752.
-template <int D, int HS, int PER_UNIT>
-__global__ __launch_bounds__(256, PER_UNIT) void attn_dq_kernel(AttnParams p) {
-  extern __shared__ __align__(16) char smem_raw[];
-  if (D == 64 && p.ds_most_blocks && !dq_recomputes(p)) return;
-  const lds_addr lds0 = lds_address_of(smem_raw);
-  __shared__ int next_pull;
+template <int D, int HS, int PER_UNIT, bool STATS>
+CT_DEVICE void attn_dq_tiles(const AttnParams& p, int index, int workgroups, const lds_addr lds0, int* next_pull) {
   constexpr int PB = 4 / HS;
   const int nrb = p.S / 32;
   const int slices = (p.Hq / p.Hkv) / HS;
   const int groups = slices * p.kvh_count;
-  const int group = blockIdx.x % groups, member = blockIdx.x / groups, members = gridDim.x / groups;
+  const int group = index % groups, member = index / groups, members = workgroups / groups;
   const int kvh = p.kvh_base + group % p.kvh_count, slice = group / p.kvh_count;
   const int tpr = bin_tiles_per_row(nrb, PB);
   const int total = p.B * tpr;
   const MetaPtr sched = meta_const(p.sched + query_schedule_offset(nrb, PB));
   const bool dynamic = slices * p.Hkv <= kDqCounters;
+  if (!dynamic && member >= members) return;
   for (int pull = member;; pull += members) {
     if (dynamic) {
-      if (threadIdx.x == 0) next_pull = atomicAdd(&p.dq_counters[slice * p.Hkv + kvh], 1);
+      if (threadIdx.x == 0) *next_pull = atomicAdd(&p.dq_counters[slice * p.Hkv + kvh], 1);
       __syncthreads();
-      pull = uniform(next_pull);
+      pull = uniform(*next_pull);
       __syncthreads();
     }
     if (pull >= total) break;
     const int b = pull % p.B, rank = pull / p.B;
     const int qt = uniform(sched[(size_t)b * schedule_ints(nrb) + rank]);
-    attn_dq_item<D, HS, PER_UNIT>(p, b, kvh, slice, qt, lds0);
+    attn_dq_item<D, HS, PER_UNIT, STATS>(p, b, kvh, slice, qt, lds0);
   }
+}
+template <int D, int HS, int PER_UNIT>
+__global__ __launch_bounds__(256, PER_UNIT) void attn_dq_kernel(AttnParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  if (D == 64 && p.ds_most_blocks && !dq_recomputes(p)) return;
+  __shared__ int next_pull;
+  attn_dq_tiles<D, HS, PER_UNIT, true>(p, blockIdx.x, gridDim.x, lds_address_of(smem_raw), &next_pull);
 }
 
 // ---------------------------------------------------------------------------
@@ -807,7 +816,8 @@ __global__ __launch_bounds__(1024) void attn_dkv_schedule_kernel(AttnParams p, i
 // two costs nothing.
 template <int D>
 __global__ __launch_bounds__(1024) void attn_bwd_setup_kernel(AttnParams p, int kvh_side_by_side, float exponent_scale) {
-  const bool recompute = p.ds_most_blocks && ds_blocks_per_head(p) > p.ds_most_blocks;
+  const bool asked = p.ds_most_blocks && (blockIdx.x == 0 || !p.dq_rides);
+  const bool recompute = asked && ds_blocks_per_head(p) > p.ds_most_blocks;
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) p.dkv_header[kDqRecomputes] = recompute;
     if (D == 128) leave_dkv_choice(p);
@@ -968,6 +978,17 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
   return p.ds + block * kDsBlockBytes;
 }
 
+// A workgroup's place in the work list, by scalar loads that do not wait for one another.
+struct DkvEntry {
+  int tile, packed, entries;  // (how many the list has)
+  CT_DEVICE explicit DkvEntry(const AttnParams& p) {
+    const MetaPtr entry = meta_const(reinterpret_cast<const int*>(p.dkv_entries)) + 2 * (blockIdx.x / p.kvh_count);
+    tile = entry[0];
+    packed = entry[1];
+    entries = meta_const(p.dkv_header)[0];
+  }
+};
+
 // SPILL: every (key block, query block) step also stores its bf16 dS block to the dS region, for
 // attn_dq_blocks_kernel.
 //
@@ -976,7 +997,7 @@ CT_DEVICE char* ds_block_address(const AttnParams& p, int head, int b, int ds_of
 // [2, 15616, 12/2 heads of 64] 544 -> 445 us, [1, 7424, 6/1] 95 -> 80. Its fragments are read ahead of the products
 // (fragments_ahead): [1, 25472, 64/8], image blocks, 1800 -> 1690; the dQ kernel above likewise, 1280 -> 1190.
 template <int D, bool SPILL>
-CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
+CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0, const DkvEntry& work) {
   if (SPILL && blockIdx.x == 0)  // work counters of the dQ kernel that reads the blocks
     for (int i = threadIdx.x; i < kDqCounters; i += 256) p.dq_counters[kDqCounters + i] = 0;
   constexpr int kStage = QdoStage<D>::kBytes;
@@ -989,10 +1010,9 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
   // way into fragments. One after the other, and K and V by instructions that touch 32 rows each, the kernel took, us,
   // [3, 640, 12/2 heads of 128] 20.9 for 19.5, [4, 1792, 4/4] 26.7 for 25.2, [2, 2432, 16/16] 65.3 for 64.2, [4, 4096, 32/8],
   // documents of 64 to 300, 121.6 for 120.5, [8, 1152, 32/32 of 64], 16 to 64, 54.7 for 53.4.
-  const int2 work_entry = p.dkv_entries[entry];
-  int tile = uniform(work_entry.x), packed = uniform(work_entry.y);
+  int tile = uniform(work.tile), packed = uniform(work.packed);
   asm volatile("" : "+s"(tile), "+s"(packed));
-  if (entry >= uniform(p.dkv_header[0]) || (D == 128 && !SPILL && other_dkv_kernel(p, false))) return;
+  if (entry >= uniform(work.entries) || (D == 128 && !SPILL && other_dkv_kernel(p, false))) return;
   const int chunk = packed & 255, nsplit = (packed >> 8) & 255, slot0 = (unsigned)packed >> 16;
   const int b = tile / (nrb / 4), kt = tile % (nrb / 4);
   const int g = p.Hq / p.Hkv;
@@ -1250,7 +1270,7 @@ CT_DEVICE void dkv_entry(const AttnParams& p, const lds_addr lds0) {
 template <int D, bool SPILL>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
-  dkv_entry<D, SPILL>(p, lds_address_of(smem_raw));
+  dkv_entry<D, SPILL>(p, lds_address_of(smem_raw), DkvEntry(p));
 }
 
 // With the stores or without them, as the header says. (Two kernels, one of them to exit at once, would be one more launch; with
@@ -1258,8 +1278,31 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_kernel(AttnPara
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_dkv_choice_kernel(AttnParams p) {
   extern __shared__ __align__(16) char smem_raw[];
-  if (dq_recomputes(p)) dkv_entry<D, false>(p, lds_address_of(smem_raw));
-  else dkv_entry<D, true>(p, lds_address_of(smem_raw));
+  const DkvEntry entry(p);
+  if (dq_recomputes(p)) dkv_entry<D, false>(p, lds_address_of(smem_raw), entry);
+  else dkv_entry<D, true>(p, lds_address_of(smem_raw), entry);
+}
+
+// The same for launches in which the recomputing dQ has none of its own: where the header asks for it the workgroups, as many as
+// the list has room, go on with query tiles when they have left their key tile, and the tiles fill what the list leaves at its
+// end. (Workgroups of their own behind the list's: 768 more to start for nothing, 1 us of 19 with short documents. The answer read
+// by a vector load, a round trip in front of the entry's: 0.98 of the time then; three scalar loads side by side: 0.997.)
+// Backward kernels, us, stored blocks / so: [1, 4096, 24/8 heads of 64], documents of 2048 to 4096 225 / 188, whole rows 263 / 212;
+// [3, 2048, 32/8] whole rows 272 / 212, of 16 to 64 72.0 / 71.9; [1, 3456, 48/8], images, 385 / 278; [7, 1024, 32/32], of 512 to 1024
+// 136 / 119, of 100 to 200 88.9 / 89.4.
+template <int HS>
+__global__ __launch_bounds__(256, 3) void attn_dkv_then_dq_kernel(AttnParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  __shared__ int next_pull;
+  const lds_addr lds0 = lds_address_of(smem_raw);
+  const DkvEntry entry(p);
+  if (!dq_recomputes(p)) {
+    dkv_entry<64, true>(p, lds0, entry);
+    return;
+  }
+  dkv_entry<64, false>(p, lds0, entry);
+  __syncthreads();  // the store patches become stages
+  attn_dq_tiles<64, HS, 3, false>(p, blockIdx.x, gridDim.x, lds0, &next_pull);
 }
 
 // ---------------------------------------------------------------------------
@@ -1557,7 +1600,9 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
       return;
     }
   }
-  if (D == 64 && p.ds_most_blocks && dq_recomputes(p)) return;
+  // (beside the first reads of the schedule for a workgroup per tile, whose time this round trip would be part of)
+  const int recomputes = D == 64 && p.ds_most_blocks ? meta_const(p.dkv_header)[kDqRecomputes] : 0;
+  if (KS == 1 && uniform(recomputes) != 0) return;
   const lds_addr lds0 = lds_address_of(smem_raw);
   __shared__ int next_pull;
   using Stage = DsStage<D, KS>;
@@ -1577,7 +1622,9 @@ __global__ __launch_bounds__(kDqbWaves * 64, 2) void attn_dq_blocks_kernel(AttnP
   const DsFragPtrs frags(lds0 + (Stage::kDs + w * Stage::kPatch), lane_id());
   const TrFragOffsets<D / 8, KSlots::kAccum> tp(lds0 + w / (kDqbWaves / KS) * Stage::kKBytes);
   if constexpr (KS > 1) {  // a workgroup per tile, heaviest first
-    const int b = member % p.B, qt = uniform(sched[(size_t)b * schedule_ints(nrb) + member / p.B]);
+    const int b = member % p.B, tile = sched[(size_t)b * schedule_ints(nrb) + member / p.B];
+    if (uniform(recomputes) != 0) return;
+    const int qt = uniform(tile);
     attn_dq_blocks_item<D, HS, KS>(p, b, kvh, slice, qt, lds0, kdma, frags, tp);
     return;
   }

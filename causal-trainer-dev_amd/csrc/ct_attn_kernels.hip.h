@@ -64,6 +64,7 @@ struct AttnParams {
   char* ds;              // dS region of the pass, null when dQ recomputes S and dP
   size_t ds_row_blocks;  // dS blocks reserved per (query head, batch row)
   int ds_most_blocks;    // head dimension 64: with more dS blocks per query head than this dQ recomputes after all; 0: no such choice
+  bool dq_rides;         // ... behind the key tiles of the dK/dV kernel, with statistics formed in front of it in either form
   int wide_least_blocks; // head dimension 128, long rows: from as many blocks per query head on dK/dV is the wide kernel's, ...
   bool dkv_by_blocks;    // ... where the call leaves that open
 };
@@ -71,7 +72,9 @@ struct AttnParams {
 // Whether dQ of head dimension 64 is the faster one from stored dS blocks or recomputed goes by how many blocks there are:
 // stored ones save launches and products and cost 4 KB of traffic each. The documents decide that, which the host does not
 // know, so where it matters (most_stored_blocks) the kernel that makes the work list counts the blocks and leaves the answer in
-// the list's header; both dQ kernels are launched, and the workgroups of the one that is not wanted exit at once.
+// the list's header; both dQ kernels are launched, and the workgroups of the one that is not wanted exit at once. In smaller launches
+// such a launch for nothing costs short documents more than long ones gain: there the recomputing tiles are the second half of the
+// dK/dV kernel's work (dq_rides).
 constexpr int kDqRecomputes = 2;  // place in the header
 // Likewise for the two dK/dV kernels of head dimension 128 in long rows (wide_least_blocks); every list has that answer.
 constexpr int kDkvWide = 3;
@@ -1161,7 +1164,7 @@ CT_DEVICE void bwd_stats_tiles(const bf16* out, const bf16* dout, const float* l
 
 template <int D>
 __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(AttnParams p, float exponent_scale) {
-  if (D == 64 && p.ds_most_blocks && p.dkv_header[kDqRecomputes]) return;
+  if (D == 64 && p.ds_most_blocks && !p.dq_rides && p.dkv_header[kDqRecomputes]) return;
   bwd_stats_tiles<D>(p.out, p.dout, p.lse, p.delta, p.lse2, p.B, p.S, p.Hq, exponent_scale, blockIdx.x, gridDim.x,
                      threadIdx.x);
 }

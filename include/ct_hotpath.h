@@ -152,8 +152,8 @@ int32_t ct_attn_fwd(void* stream, const ct_attn_fwd_args* args);
  * pair and head; needs ct_attn_bwd_workspace_bytes_from_ds. Left open (0): FROM_DS for
  * rows of at most CT_ATTN_FROM_DS_UP_TO_SEQ positions if the caller's workspace holds the dS blocks of all KV heads
  * (workspace_bytes >= ct_attn_bwd_workspace_bytes_from_ds and that size is the one-pass size),
- * else RECOMPUTE: a caller chooses by the workspace it offers. At head dimension 64 that offer is taken up to 8192
- * row blocks (32 query rows of one head); in larger launches the batch's number of dS blocks decides on the device
+ * else RECOMPUTE: a caller chooses by the workspace it offers. At head dimension 64 that offer is taken below 3072
+ * row blocks (32 query rows of one head) and at 8192; in other launches the batch's number of dS blocks decides on the device
  * between the two forms, in the same workspace. All give the same results within
  * the operator's tolerances (not bitwise: summation orders differ).
  * Measured, backward in us, RECOMPUTE / FROM_DS. Head dimension 128: [4, 4096, 32/8 heads] with documents of

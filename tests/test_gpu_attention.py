@@ -453,6 +453,37 @@ def test_form_by_the_number_of_blocks(ct, gpu, shape, chooses, with_ends):
             assert all(torch.equal(a, b) for a, b in zip(call(workspace=kept), chosen))
 
 
+@pytest.mark.parametrize("shape,chooses", [
+    ((1, 3968, 24, 8), False), ((2, 1536, 32, 8), True), ((3, 1024, 32, 32), True), ((5, 640, 66, 11), True), ((1, 512, 450, 450), True),
+    ((3, 1408, 62, 31), True), ((1, 384, 677, 1), False)], ids=lambda v: "" if isinstance(v, bool) else "B%d_S%d_Hq%d_Hkv%d" % v)
+@pytest.mark.parametrize("with_ends", [False, True], ids=["causal", "ends"])
+def test_form_by_the_number_of_blocks_behind_the_key_tiles(ct, gpu, shape, chooses, with_ends):
+    """Head dimension 64, from 3072 to 8191 row blocks: many dS blocks are recomputed by the launch that forms dK and dV. One
+    of the shapes has more groups of heads than work counters, the last one more than that launch has workgroups. The statistics have a pass of their own in either form, so dK
+    and dV are the stored form's; dQ is too where it comes from stored blocks, and has other bits where not: the same
+    sums in another order, a rounding of bf16 (2^-9) an element at most in either case."""
+
+    batch, seq, q_heads, kv_heads = shape
+    generator = torch.Generator(device=gpu).manual_seed(seq)
+    q, k, v, dout = (torch.randn((batch, seq, heads, 64), generator=generator, device=gpu).to(torch.bfloat16)
+                     for heads in (q_heads, kv_heads, kv_heads, q_heads))
+    kept = ct.BackwardWorkspace()
+    rng = np.random.default_rng(batch)
+    for longest in (24, None, 24):
+        ids = np.ones((batch, seq), np.int32) if longest is None else _layout(rng, batch, seq, holes=True, max_len=longest)
+        ends = torch.from_numpy(_random_ends(rng, ids)).to(gpu) if with_ends else None
+        profile = ct.resolve_attention_profile(q.shape, k.shape, None, has_attention_end=with_ends)
+        metadata = ct.prepare_attention_metadata(torch.from_numpy(ids).to(gpu), mesh=None, profile=profile, attention_end=ends)
+        out, lse = ct.attention_forward_with_lse(q, k, v, metadata)
+        call = lambda **form: ct.attention_backward(q, k, v, metadata, out, lse, dout, **form)  # noqa: E731
+        recomputed, stored, chosen = call(dq_form="recompute"), call(dq_form="from_ds"), call()
+        assert torch.equal(chosen[1], stored[1]) and torch.equal(chosen[2], stored[2])
+        assert torch.equal(chosen[0], stored[0]) == (not (chooses and longest is None))
+        assert float((chosen[0].float() - recomputed[0].float()).norm() / recomputed[0].float().norm()) <= 2.0 ** -9
+        for _ in range(3):                      # (the list is built, then kept)
+            assert all(torch.equal(a, b) for a, b in zip(call(workspace=kept), chosen))
+
+
 @pytest.mark.parametrize("seq,q_heads", [(8192, 8), (4096, 32)])
 def test_backward_without_room_for_stored_blocks(ct, gpu, seq, q_heads):
     """The operator's own choice of the stored-dS form gives way to the recomputing form where the allocator has no room
