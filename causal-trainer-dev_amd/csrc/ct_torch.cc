@@ -359,7 +359,9 @@ MaybeTensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
 // ---------------------------------------------------------------------------------------------
 struct RmsNormNode : OperatorNode {
   SavedVariable x, scale;
-  Tensor rstd;  // of few rows
+  // Of few rows, 4 KB at most. Beside the residuals: what saved-tensor hooks are given stays x and scale, for any number of rows
+  // (x is unpacked first, so that a graph that was released or an x that was overwritten is refused as before).
+  Tensor rstd;
   double eps = 0;
   variable_list differentiate(variable_list&& grads) override {
     const Tensor X = x.unpack(), W = scale.unpack();

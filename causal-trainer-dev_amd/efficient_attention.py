@@ -267,7 +267,7 @@ def attention_backward(query, key, value, metadata, out, lse, dout, *, scale=Non
     kernel or a form of the backward for this call (``ct_attn_bwd_args.variant``); ``None`` leaves
     the choice to the library, which is what training code does (the dK/dV kernel goes by sequence
     length, and in long rows by the documents, on the device; dQ comes from stored dS blocks at rows of up to 4096 positions when their workspace is at
-    most 4 GiB, and from a recomputing kernel otherwise; from 8193 row blocks of head dimension 64 on, the
+    most 4 GiB, and from a recomputing kernel otherwise; from 3072 row blocks of head dimension 64 on (8192 apart), the
     documents decide between the two on the device). ``workspace_bytes`` overrides the size of the scratch buffer (default: what
     the library asks for the chosen form); ``workspace`` (a :class:`BackwardWorkspace`) keeps the
     buffer, and with it the dK/dV work list, from one call to the next."""
